@@ -322,8 +322,22 @@ size_t decode_buffers(const QmkHybridArgs* a, void* base, DecodeBuffers* b) {
 
 inline size_t values_cap(const QmkHybridArgs* a) { return (static_cast<size_t>(a->max_positions) + 31) & ~size_t(31); }
 
+// Parts of products that are cut along K: the head of every prefill workspace, so that a workspace that serves launches of
+// different sizes keeps its tickets, zero between products, in one place.
+struct SplitBuffers {
+  int32_t* tickets;
+  f32x4* partial;
+};
+inline SplitBuffers split_buffers(Carver& c) {
+  SplitBuffers b;
+  b.tickets = c.take<int32_t>(kMaxTickets);
+  b.partial = c.take<f32x4>(kPartialUnits);
+  return b;
+}
+
 template <class T>
 struct PlainBuffers {
+  SplitBuffers split;
   float *x, *branch, *qkv, *values, *decay, *beta, *o, *chunks;
   T *h, *q, *low, *gate, *mix, *vt;
 };
@@ -358,6 +372,7 @@ size_t plain_buffers(const QmkHybridArgs* a, void* base, PlainBuffers<T>* b) {
   Carver c{static_cast<char*>(base)};
   PlainBuffers<T> local;
   if (b == nullptr) b = &local;
+  b->split = split_buffers(c);
   b->x = c.take<float>(P * D);
   b->branch = c.take<float>(branch);
   b->qkv = c.take<float>(qkv);
@@ -379,6 +394,7 @@ inline int keys_cap(const QmkHybridArgs* a, const QmkHybridLayer& l) { return (s
 
 template <class T>
 struct PrefillBuffers {
+  SplitBuffers split;
   float *x, *u, *fa, *fb, *raw;
   T *h, *p0, *p1, *p2, *mix, *rows, *kn, *vt;
 };
@@ -415,6 +431,7 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
     }
   }
   Carver c{static_cast<char*>(base)};
+  b->split = split_buffers(c);
   b->x = c.take<float>(P * a->streams * D);
   b->u = c.take<float>(P * D);
   b->fa = c.take<float>(fa);
@@ -431,22 +448,99 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
   return c.used;
 }
 
-// Large tiles where they fill the chip, small ones otherwise.
+// The tiles of a product.  A workgroup of the Turns kernels has a CU for itself, so a product takes as many rounds as its
+// tiles fill the chip, each about `step` us for 2048 columns and `fixed` us besides; of the others several share a CU, their
+// fixed part overlaps and `slots` of them make a round.  Cut along K into parts it takes `meet` us more for the first part and
+// `each` for every part.  All figures measured with weights that come from memory (us, M x N x K, the kernels this replaced ->
+// now): 2048 x 16384 x 2048 160 -> 138, 1531 x 16384 x 2048 115 -> 113, 2048 x 6144 x 2048 77 -> 64, 1531 x 5696 x 2048 63 -> 54,
+// 2048 x 2048 x 8192 107 -> 75, 1531 x 2048 x 8192 with the residual's streams 141 -> 83, 1531 x 2048 x 2048 with them 71 -> 41,
+// 512 x 2048 x 8192 73 -> 37, 43 x 2048 x 6144 38 -> 15, 43 x 12288 x 2048 23 -> 13.
+struct TileCost {
+  int bm, bn, slots;
+  double step, fixed, overlapped, meet, each;
+};
+constexpr int kTileKinds = 7;
+constexpr TileCost kTileCosts[kTileKinds] = {
+    {64, 64, 256, 9.0, 0.0, 5.0, 1.0, 0.6},     // Tiles64
+    {128, 128, 512, 36.0, 8.0, 0.0, 0.0, 0.0},  // Tiles128
+    {64, 128, 256, 12.0, 6.5, 0.0, 3.0, 1.5},   // Turns64
+    {96, 128, 256, 14.5, 6.5, 0.0, 3.0, 1.5},   // Turns96
+    {128, 128, 256, 17.0, 9.0, 0.0, 3.0, 2.0},  // Turns128
+    {192, 256, 256, 47.0, 10.0, 0.0, 0.0, 0.0},  // Turns192
+    {256, 256, 256, 60.0, 9.0, 0.0, 0.0, 0.0},   // Turns256
+};
+struct TileChoice {
+  int kind = 0, splits = 1;
+};
+inline TileChoice choose_tiles(int M, int N, int K, int groups) {
+  TileChoice best;
+  double least = 0.;
+  for (int kind = 0; kind < kTileKinds; ++kind) {
+    const TileCost& t = kTileCosts[kind];
+    const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * groups;
+    for (int splits = 1; splits <= 8; splits *= 2) {
+      if (splits > 1 && (t.each == 0. || K / splits < 256 || tiles > kMaxTickets || tiles * splits * t.bm * t.bn / 4 > kPartialUnits)) break;
+      const double rounds = static_cast<double>((tiles * splits + t.slots - 1) / t.slots);
+      const double us = rounds * (t.step * K / 2048. / splits + t.fixed) + t.overlapped + (splits > 1 ? t.meet + t.each * splits : 0.);
+      if ((kind == 0 && splits == 1) || us < least) {
+        least = us;
+        best = TileChoice{kind, splits};
+      }
+    }
+  }
+  return best;
+}
+
+// The same for products with an fp32 side, or of columns that are no multiple of 64: tiles of 64 x 64 cut along K until they
+// fill the chip four times over, of 128 x 128 where a part of them fills it already.
+inline TileChoice choose_register_tiles(int M, int N, int K, int groups) {
+  TileChoice c;
+  const long long large = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128) * groups, small = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) * groups;
+  if (large >= 256) {
+    c.kind = 1;
+    return c;
+  }
+  while (c.splits < 8 && small * c.splits < 512 && K / c.splits >= 512 && small <= kMaxTickets && small * c.splits * 2 * 64 * 64 / 4 <= kPartialUnits) c.splits *= 2;
+  return c;
+}
+
 template <class TA, class TW, class T>
-void launch_gemm(const GemmArgs& g, hipStream_t st) {
+void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   const int n = std::max(g.N, g.last_n);
-  auto grid = [&](int bm, int bn) { return dim3((n + bn - 1) / bn, (g.M + bm - 1) / bm, g.groups); };
-  const dim3 large = grid(128, 128), block(kPfThreads);
-  const bool fills = static_cast<long long>(large.x) * large.y * large.z >= 192;
+  g.tickets = split.tickets;
+  g.partial = reinterpret_cast<float*>(split.partial);
+  auto launch = [&](auto kernel, int bm, int bn, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((n + bn - 1) / bn * ((g.M + bm - 1) / bm) * g.splits), 1, g.groups), dim3(threads), 0, st, g);
+  };
   if constexpr (sizeof(TA) == 2 && sizeof(TW) == 2) {
     if (g.K % 64 == 0) {
-      if (fills) hipLaunchKernelGGL((gemm_direct<T, 128, 128, 2>), large, block, 0, st, g);
-      else hipLaunchKernelGGL((gemm_direct<T, 64, 64, 4>), grid(64, 64), block, 0, st, g);
+      const TileChoice c = choose_tiles(g.M, n, g.K, g.groups);
+      g.splits = c.splits;
+      auto direct = [&](auto s) { using S = decltype(s); launch(gemm_direct<T, S>, S::BM, S::BN, S::kThreadCount); };
+      auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S>, S::BM, S::BN, S::kThreadCount); };
+      switch (c.kind) {
+        case 0: direct(Tiles64{}); break;
+        case 1: direct(Tiles128{}); break;
+        case 2: turns(Turns64{}); break;
+        case 3: turns(Turns96{}); break;
+        case 4: turns(Turns128{}); break;
+        case 5: turns(Turns192{}); break;
+        default: turns(Turns256{}); break;
+      }
       return;
     }
   }
-  if (fills) hipLaunchKernelGGL((gemm<TA, TW, T, 128, 128>), large, block, 0, st, g);
-  else hipLaunchKernelGGL((gemm<TA, TW, T, 64, 64>), grid(64, 64), block, 0, st, g);
+  if constexpr (sizeof(TA) == 4 || sizeof(TW) == 4) {
+    if (g.K <= 64) {
+      g.splits = 1;
+      launch(gemm_short<TA, TW, T>, 64, 64, kPfThreads);
+      return;
+    }
+  }
+  const TileChoice c = choose_register_tiles(g.M, n, g.K, g.groups);
+  g.splits = c.splits;
+  if (c.kind == 1) launch(gemm<TA, TW, T, 128, 128, 2>, 128, 128, kPfThreads);
+  else launch(gemm<TA, TW, T, 64, 64, 1>, 64, 64, kPfThreads);
 }
 
 // rows: where the rotated part of a latent attention's keys is, behind the latent.
@@ -483,7 +577,7 @@ int prefill(const QmkHybridArgs* a) {
   auto residual = [&](const u16* w, int K, const QmkHybridLayer& l, bool down) {
     GemmArgs g = gemm_args(b.mix, K, w, D, K, l, EPI_RESIDUAL);
     g.f0 = b.x; g.f1 = b.u; g.down = down; g.next = down ? l.next2 : l.next1;
-    launch_gemm<T, u16, T>(g, st);
+    launch_gemm<T, u16, T>(g, b.split, st);
   };
   for (int i = 0; i < a->num_layers; ++i) {
     const QmkHybridLayer& l = a->layers[i];
@@ -493,26 +587,26 @@ int prefill(const QmkHybridArgs* a) {
     if (l.type == QMK_MIXER_RGLRU) {
       GemmArgs g = gemm_args(b.h, D, l.in_w, l.in_rows, D, l, EPI_RGLRU_IN);
       g.out = b.p0; g.out2 = b.p1;
-      launch_gemm<T, u16, T>(g, st);
+      launch_gemm<T, u16, T>(g, b.split, st);
       const long long quads = static_cast<long long>(M) * (W / 4);
       hipLaunchKernelGGL(causal_conv<T>, dim3(static_cast<unsigned>((quads + kPfThreads - 1) / kPfThreads)), block, 0, st, b.p1, l, a->slot, a->flip, M, b.p2);
       GemmArgs e = gemm_args(b.p2, W, l.mid_w, 2 * l.block_dim, l.block_dim, l, EPI_LRU_GATES);
       e.groups = l.blocks; e.a_step = l.block_dim; e.w_step = 2LL * l.block_dim * l.block_dim;
       e.src = b.p2; e.f0 = b.fa; e.f1 = b.fb;
-      launch_gemm<T, u16, T>(e, st);
+      launch_gemm<T, u16, T>(e, b.split, st);
       hipLaunchKernelGGL(lru_scan<T>, dim3(W / kScanChannels), dim3(kScanChannels * kScanRuns), 0, st, b.fa, b.fb, b.p0, l, a->slot, M, b.mix);
     } else if (l.type == QMK_MIXER_LATENT) {
       GemmArgs g = gemm_args(b.h, D, l.in_w, l.in_rows, D, l, EPI_LATENT_IN);
       g.out = b.p0; g.out2 = b.p1; g.f0 = b.raw;
-      launch_gemm<T, u16, T>(g, st);
+      launch_gemm<T, u16, T>(g, b.split, st);
       const int first = std::max(0, a->position + 1 - l.window), keys = a->position + M - first, cap = keys_cap(a, l), width = l.rank + l.rot_dim;
       hipLaunchKernelGGL(latent_rows<T>, dim3(keys), block, 0, st, b.raw, l, a->slot, first, a->position, a->eps, b.rows);
       GemmArgs k = gemm_args(b.rows, width, l.uk_w, l.heads * l.head_dim, l.rank, l, EPI_STORE);
       k.M = keys; k.out = b.kn; k.ldo = l.heads * l.head_dim;
-      launch_gemm<T, u16, T>(k, st);
+      launch_gemm<T, u16, T>(k, b.split, st);
       GemmArgs v = gemm_args(nullptr, l.rank, nullptr, keys, l.rank, l, EPI_STORE);   // transposed: W_uv rows x keys
       v.a = l.uv_w; v.w = b.rows; v.ldw = width; v.M = l.heads * l.v_dim; v.out = b.vt; v.ldo = cap;
-      launch_gemm<u16, T, T>(v, st);
+      launch_gemm<u16, T, T>(v, b.split, st);
       const Keys<T> expanded{b.kn, l.heads * l.head_dim, l.head_dim, 1};
       launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix, st);
     } else {
@@ -521,10 +615,10 @@ int prefill(const QmkHybridArgs* a) {
       GemmArgs g = gemm_args(b.h, D, l.in_w, N, D, l, EPI_WKV_IN);
       g.groups = 5; g.last_n = l.rank; g.a_step = static_cast<long long>(P) * D; g.w_step = static_cast<long long>(N) * D;
       g.f0 = b.fa; g.out = b.p0; g.out2 = b.p1;
-      launch_gemm<T, u16, T>(g, st);
+      launch_gemm<T, u16, T>(g, b.split, st);
       GemmArgs d = gemm_args(b.p1, l.rank, l.mid_w, N, l.rank, l, EPI_WKV_DECAY);
       d.f0 = b.fb; d.ldo = N;
-      launch_gemm<T, u16, T>(d, st);
+      launch_gemm<T, u16, T>(d, b.split, st);
       const size_t step = static_cast<size_t>(P) * N;
       const dim3 grid(n / kWkvColumns, l.heads), lanes(kWkvThreads);
       const float *r = b.fa, *k = b.fa + step, *v = b.fa + 2 * step;
@@ -538,7 +632,7 @@ int prefill(const QmkHybridArgs* a) {
       hipLaunchKernelGGL(norm_rows<T>, dim3(M), block, 0, st, b.u, l.norm2, nullptr, M, D, a->width_true, a->eps, b.h);
       GemmArgs g = gemm_args(b.h, D, l.mlp_w, 2 * l.ff, D, l, EPI_GEGLU);
       g.out = b.mix;
-      launch_gemm<T, u16, T>(g, st);
+      launch_gemm<T, u16, T>(g, b.split, st);
       residual(l.down_w, l.ff, l, true);
     }
     if (a->layer_out != nullptr)
@@ -548,7 +642,7 @@ int prefill(const QmkHybridArgs* a) {
     hipLaunchKernelGGL(norm_rows<T>, dim3(a->num_want), block, 0, st, b.u, a->final_norm, a->want, M, D, a->width_true, a->eps, b.h);
     GemmArgs g = gemm_args(b.h, D, a->head, a->vocab_rows, D, a->layers[0], EPI_LOGITS);
     g.M = a->num_want; g.f0 = a->logits; g.ldo = a->vocab_rows;
-    launch_gemm<T, u16, T>(g, st);
+    launch_gemm<T, u16, T>(g, b.split, st);
   }
   return hipGetLastError() == hipSuccess ? QMK_OK : QMK_ERR_LAUNCH;
 }
@@ -606,7 +700,7 @@ int prefill_plain(const QmkHybridArgs* a) {
         residual(l, a->want, a->num_want, dump == nullptr, nullptr);
         GemmArgs g = gemm_args(b.h, a->head, a->vocab_rows, D, l, EPI_CAPPED_LOGITS);
         g.M = a->num_want; g.f0 = a->logits; g.ldo = a->vocab_rows;
-        launch_gemm<T, u16, T>(g, st);
+        launch_gemm<T, u16, T>(g, b.split, st);
       }
       break;
     }
@@ -614,13 +708,13 @@ int prefill_plain(const QmkHybridArgs* a) {
     if (l.type == QMK_ENTRY_JOIN) {
       GemmArgs g = gemm_args(b.h, l.in_w, D, 2 * D, l, EPI_LOGITS);
       g.f0 = b.x;
-      launch_gemm<T, u16, T>(g, st);
+      launch_gemm<T, u16, T>(g, b.split, st);
       continue;
     }
     if (l.type == QMK_MIXER_ATTENTION) {
       GemmArgs g = gemm_args(b.h, l.in_w, l.in_rows, D, l, EPI_ATTENTION_IN);
       g.out = b.q; g.out2 = b.gate;
-      launch_gemm<T, u16, T>(g, st);
+      launch_gemm<T, u16, T>(g, b.split, st);
       const int row = l.head_dim + l.v_dim, pitch = l.kv_heads * row, keys = a->position + M, cap = static_cast<int>(values_cap(a));
       const T* cache = static_cast<const T*>(l.cache) + static_cast<size_t>(a->slot) * l.ring * pitch;
       hipLaunchKernelGGL(transpose_values<T>, dim3((keys + 63) / 64, (l.v_dim + 63) / 64, l.kv_heads), block, 0, st, cache, pitch, row, l.head_dim, l.v_dim, keys, cap, b.vt);
@@ -632,14 +726,14 @@ int prefill_plain(const QmkHybridArgs* a) {
         const int channels = conv_channels(l), ranks = l.rank + l.gate_rank, beta_ld = (l.heads + 15) / 16 * 16;
         GemmArgs g = gemm_args(b.h, l.in_w, l.in_rows, D, l, EPI_DELTA_IN);
         g.f1 = b.qkv; g.out2 = b.low; g.f0 = b.beta; g.ldo = beta_ld;
-        launch_gemm<T, u16, T>(g, st);
+        launch_gemm<T, u16, T>(g, b.split, st);
         const int keys = l.heads * l.head_dim;
         GemmArgs e = gemm_args(b.low, l.mid_w, keys, l.rank, l, EPI_DELTA_DECAY);
         e.lda = ranks; e.f0 = b.decay; e.ldo = keys;
-        launch_gemm<T, u16, T>(e, st);
+        launch_gemm<T, u16, T>(e, b.split, st);
         GemmArgs f = gemm_args(b.low + l.rank, l.gate_w, W, l.gate_rank, l, EPI_SIGMOID);
         f.lda = ranks; f.out = b.gate; f.ldo = W;
-        launch_gemm<T, u16, T>(f, st);
+        launch_gemm<T, u16, T>(f, b.split, st);
         c.qkv = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = W;
         run_chunks<true>(a, c, st);
         if (l.taps > 1)
@@ -648,10 +742,10 @@ int prefill_plain(const QmkHybridArgs* a) {
         const int keys = l.heads * l.head_dim;
         GemmArgs g = gemm_args(b.h, l.in_w, l.in_rows, D, l, EPI_GLA_IN);
         g.f0 = b.qkv; g.out = b.gate; g.out2 = b.low;
-        launch_gemm<T, u16, T>(g, st);
+        launch_gemm<T, u16, T>(g, b.split, st);
         GemmArgs e = gemm_args(b.low, l.mid_w, keys, l.rank, l, EPI_GLA_DECAY);
         e.f0 = b.decay; e.ldo = keys;
-        launch_gemm<T, u16, T>(e, st);
+        launch_gemm<T, u16, T>(e, b.split, st);
         c.qkv = b.qkv; c.values = b.qkv; c.value_ld = 2 * keys + W; c.value_at = 2 * keys;
         run_chunks<false>(a, c, st);
       }
@@ -659,16 +753,16 @@ int prefill_plain(const QmkHybridArgs* a) {
     }
     GemmArgs o = gemm_args(b.mix, l.o_w, D, W, l, l.branches > 1 ? EPI_LOGITS : EPI_ADD);
     o.f0 = l.branches > 1 ? b.branch + l.branch * rows : b.x;
-    launch_gemm<T, u16, T>(o, st);
+    launch_gemm<T, u16, T>(o, b.split, st);
     if (l.branch + 1 == l.branches) {
       const QmkHybridLayer& head = a->layers[i - l.branch];
       if (head.has_mlp) {
         GemmArgs g = gemm_args(b.h, head.mlp_w, 2 * head.ff, D, head, EPI_GEGLU);
         g.out = b.mix;
-        launch_gemm<T, u16, T>(g, st);
+        launch_gemm<T, u16, T>(g, b.split, st);
         GemmArgs d = gemm_args(b.mix, head.down_w, D, head.ff, head, EPI_ADD);
         d.f0 = b.x;
-        launch_gemm<T, u16, T>(d, st);
+        launch_gemm<T, u16, T>(d, b.split, st);
       }
     }
   }

@@ -1,0 +1,775 @@
+// Matrix products of the hybrid route's prefill: out[m][n] = sum_k a[m][k] w[n][k], tokens x weight rows, with everything
+// element-wise done in the epilogue.
+#pragma once
+
+#include "qmk_hybrid_ops.h"
+
+namespace qmk {
+namespace hybrid {
+
+constexpr int kPfThreads = 256;
+
+enum : int {
+  EPI_STORE = 0,        // out T [m][ldo]
+  EPI_RGLRU_IN,         // gelu of the y half, bias on both
+  EPI_LRU_GATES,        // (r, i) pairs -> decay a and input b of the recurrence
+  EPI_LATENT_IN,        // rotation of q, sigmoid of the gate, raw latent
+  EPI_RESIDUAL,         // all streams of the residual and the next sublayer's input (residual_quads)
+  EPI_GEGLU,            // (gate, up) pairs
+  EPI_WKV_IN,           // r, k, v fp32; silu gate; tanh
+  EPI_WKV_DECAY,        // exp(-exp(. + w0))
+  EPI_LOGITS,
+  EPI_CAPPED_LOGITS,    // logits times a constant, softly capped
+  EPI_ADD,              // onto the fp32 residual
+  EPI_ATTENTION_IN,     // rotation of q and k, k and v into the cache, sigmoid of the gate
+  EPI_DELTA_IN,         // q, k, v fp32; raw ranks; sigmoid of the step sizes
+  EPI_DELTA_DECAY,
+  EPI_SIGMOID,
+  EPI_GLA_IN,           // q, k, v fp32; silu gate; raw rank
+  EPI_GLA_DECAY,
+};
+
+struct GemmArgs {
+  const void* a;         // TA [M][lda]
+  const void* w;         // TW [N][ldw]
+  int M, N, K, lda, ldw, groups, last_n;   // group g: a + g a_step, w + g w_step, N rows (the last: last_n)
+  long long a_step, w_step;
+  int epi;
+  void* out;             // meaning by epilogue
+  void* out2;
+  float* f0;
+  float* f1;
+  const void* src;
+  int ldo;
+  QmkHybridLayer layer;
+  int down, first, position, streams, width, rows_cap, slot;
+  float logit_scale, logit_softcap;
+  const float* next;
+  float* partial;        // sums of the parts of a product that is cut along K, and a zero per tile
+  int32_t* tickets;
+  int splits;
+};
+
+template <class T>
+__device__ __forceinline__ void store4(T* at, f32x4 v) {
+  if constexpr (sizeof(T) == 2) {
+    *reinterpret_cast<uint2*>(at) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+  } else {
+    *reinterpret_cast<f32x4*>(at) = v;
+  }
+}
+template <class T>
+__device__ __forceinline__ f32x4 read4(const T* at) {
+  if constexpr (sizeof(T) == 2) {
+    const uint2 t = *reinterpret_cast<const uint2*>(at);
+    return f32x4{bf_lo(t.x), bf_hi(t.x), bf_lo(t.y), bf_hi(t.y)};
+  } else {
+    return *reinterpret_cast<const f32x4*>(at);
+  }
+}
+
+// Four consecutive outputs n .. n+3 of token m.
+template <class T>
+__device__ __forceinline__ void epilogue(const GemmArgs& g, int group, int m, int n, f32x4 v) {
+  const QmkHybridLayer& l = g.layer;
+  switch (g.epi) {
+    case EPI_STORE: store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + n, v); break;
+    case EPI_RGLRU_IN: {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(l.in_b + n);
+      v += b;
+      if (n < l.mix_width) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = gelu_tanh(v[i]);
+        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * l.mix_width + n, v);
+      } else {
+        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.mix_width + n - l.mix_width, v);
+      }
+      break;
+    }
+    case EPI_LRU_GATES: {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + static_cast<size_t>(group) * 2 * l.block_dim + n);
+      v += b;
+      const int c = group * l.block_dim + n / 2;
+      const size_t at = static_cast<size_t>(m) * l.mix_width + c;
+      const T* u = static_cast<const T*>(g.src) + at;
+      float2 a2, b2;
+      {
+        const float la = sigmoid(v[0]) * l.vec0[c];
+        a2.x = expf(la);
+        b2.x = sqrtf(-expm1f(2.f * la)) * sigmoid(v[1]) * to_f32(u[0]);
+      }
+      {
+        const float la = sigmoid(v[2]) * l.vec0[c + 1];
+        a2.y = expf(la);
+        b2.y = sqrtf(-expm1f(2.f * la)) * sigmoid(v[3]) * to_f32(u[1]);
+      }
+      *reinterpret_cast<float2*>(g.f0 + at) = a2;
+      *reinterpret_cast<float2*>(g.f1 + at) = b2;
+      break;
+    }
+    case EPI_LATENT_IN: {
+      const int q_rows = l.heads * l.q_stride, g_rows = l.heads * l.v_dim;
+      if (n < q_rows) {
+        const int d = n % l.q_stride - l.head_dim;
+        if (d >= 0) {
+          float e[4] = {v[0], v[1], v[2], v[3]};
+          rotate(l, g.position + m, d, e[0], e[1]);
+          rotate(l, g.position + m, d + 2, e[2], e[3]);
+          v = f32x4{e[0], e[1], e[2], e[3]};
+        }
+        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * q_rows + n, v);
+      } else if (n < q_rows + g_rows) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
+        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * g_rows + n - q_rows, v);
+      } else {
+        store4(g.f0 + static_cast<size_t>(m) * (l.rank + l.rot_dim) + n - q_rows - g_rows, v);
+      }
+      break;
+    }
+    case EPI_GEGLU: {
+      T* o = static_cast<T*>(g.out) + static_cast<size_t>(m) * l.ff + n / 2;
+      const bool silu = l.act == QMK_ACT_SILU;
+      const float a = (silu ? v[0] * sigmoid(v[0]) : gelu_tanh(v[0])) * v[1], b = (silu ? v[2] * sigmoid(v[2]) : gelu_tanh(v[2])) * v[3];
+      if constexpr (sizeof(T) == 2) *reinterpret_cast<uint32_t*>(o) = f2bf2(a, b);
+      else *reinterpret_cast<float2*>(o) = make_float2(a, b);
+      break;
+    }
+    case EPI_WKV_IN: {
+      const int N = l.heads * l.head_dim;
+      if (group < 3) {
+        store4(g.f0 + (static_cast<size_t>(group) * g.rows_cap + m) * N + n, v);
+      } else if (group == 3) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] *= sigmoid(v[i]);
+        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * N + n, v);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = tanhf(v[i]);
+        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.rank + n, v);
+      }
+      break;
+    }
+    case EPI_WKV_DECAY: {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = expf(-expf(v[i] + b[i]));
+      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
+      break;
+    }
+    case EPI_CAPPED_LOGITS: {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = soft_cap(v[i] * g.logit_scale, g.logit_softcap);
+      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
+      break;
+    }
+    case EPI_ADD: {
+      float* x = g.f0 + static_cast<size_t>(m) * g.ldo + n;
+      store4(x, read4(x) + v);
+      break;
+    }
+    case EPI_ATTENTION_IN: {
+      const int q_rows = l.heads * l.q_stride, k_rows = l.kv_heads * l.head_dim, v_rows = l.kv_heads * l.v_dim, row = l.head_dim + l.v_dim, pos = g.position + m;
+      T* cache = static_cast<T*>(l.cache) + (static_cast<size_t>(g.slot) * l.ring + pos % l.ring) * l.kv_heads * row;
+      if (n < q_rows + k_rows) {
+        const int d = n < q_rows ? n % l.q_stride : (n - q_rows) % l.head_dim;
+        float e[4] = {v[0], v[1], v[2], v[3]};
+        rotate(l, pos, d, e[0], e[1]);
+        rotate(l, pos, d + 2, e[2], e[3]);
+        v = f32x4{e[0], e[1], e[2], e[3]};
+        store4(n < q_rows ? static_cast<T*>(g.out) + static_cast<size_t>(m) * q_rows + n : cache + (n - q_rows) / l.head_dim * row + d, v);
+      } else if (n < q_rows + k_rows + v_rows) {
+        const int c = n - q_rows - k_rows;
+        store4(cache + c / l.v_dim * row + l.head_dim + c % l.v_dim, v);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
+        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.mix_width + n - q_rows - k_rows - v_rows, v);
+      }
+      break;
+    }
+    case EPI_DELTA_IN: {
+      const int channels = conv_channels(l), ranks = l.rank + l.gate_rank;
+      if (n < channels) {
+        store4(g.f1 + static_cast<size_t>(m) * channels + n, v);
+      } else if (n < channels + ranks) {
+        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * ranks + n - channels, v);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
+        store4(g.f0 + static_cast<size_t>(m) * g.ldo + n - channels - ranks, v);
+      }
+      break;
+    }
+    case EPI_DELTA_DECAY: {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = delta_decay(l, n / l.head_dim, v[i] + b[i]);
+      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
+      break;
+    }
+    case EPI_SIGMOID: {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
+      store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + n, v);
+      break;
+    }
+    case EPI_GLA_IN: {
+      const int qkv = 2 * l.heads * l.head_dim + l.mix_width;
+      if (n < qkv) {
+        store4(g.f0 + static_cast<size_t>(m) * qkv + n, v);
+      } else if (n < qkv + l.mix_width) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] *= sigmoid(v[i]);
+        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * l.mix_width + n - qkv, v);
+      } else {
+        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.rank + n - qkv - l.mix_width, v);
+      }
+      break;
+    }
+    case EPI_GLA_DECAY: {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = gla_decay(l, v[i] + b[i]);
+      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
+      break;
+    }
+    default: store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v); break;
+  }
+}
+
+// ---- tiles ----
+// A tile is BM tokens x BN weight rows, BK columns a step; a wave owns WM x WN of it.  Where fewer waves than there are cover
+// the tile, two groups of them take a half of a step's columns each and are summed at the end.
+template <int BM_, int BN_, int BK_, int WM_, int WN_, int WAVES_, int STAGES_>
+struct Tile {
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, kStages = STAGES_, kThreadCount = WAVES_ * 64;
+  static constexpr int kWavesM = BM / WM, kWavesN = BN / WN, kCover = kWavesM * kWavesN, kGroups = WAVES_ / kCover;
+  static constexpr int kTm = WM / 16, kTn = WN / 16, kKept = kTn / kGroups;   // a wave's fragments; of those a thread sums up
+  static constexpr int kRow = BK / 8;                                           // a row of a step: units of 16 bytes
+  static constexpr int kUnits = (BM + BN) * kRow, kLoads = (kUnits + kThreadCount - 1) / kThreadCount;
+  static constexpr int kLastWaves = (kUnits - (kLoads - 1) * kThreadCount) / 64;   // waves that take part in a stage's last load
+  static constexpr bool kSplits = kKept * kTm <= 8;                             // may be cut along K
+  static constexpr int kSteps = BK / 32 / kGroups;                              // matrix steps a wave takes of a step
+  static constexpr int kOutUnits = BM * BN / 4, kPasses = kOutUnits > kStages * kUnits ? 2 : 1;
+  static constexpr int kLds = kStages * kUnits > kOutUnits / kPasses ? kStages * kUnits : kOutUnits / kPasses;
+  static_assert(kUnits % 64 == 0 && kSteps >= 1 && kTm % kPasses == 0 && kLds * 16 < 160 * 1024, "a tile's sizes");
+  static_assert(kGroups == 1 || (kGroups == 2 && kTn % 2 == 0), "groups of waves along K");
+};
+
+// Workgroups go to the XCDs in turn; here an XCD gets a run of neighbouring tiles, which share rows through its L2.
+__device__ __forceinline__ int xcd_order(int id, int total) {
+  const int per = total >> 3, rest = total & 7, xcd = id & 7;
+  return xcd * per + min(xcd, rest) + (id >> 3);
+}
+
+// Of a product cut along K every part leaves its sums; the part that arrives last adds them up in their order and goes on
+// (true), the others are done.  `sums`: COUNT quads a thread.
+template <int COUNT, int THREADS>
+__device__ __forceinline__ bool sum_parts(const GemmArgs& g, int tile, int part, f32x4 (&sums)[COUNT], int* last) {
+  const int tid = threadIdx.x;
+  float* all = g.partial + static_cast<size_t>(tile) * g.splits * COUNT * THREADS * 4 + tid * 4;
+  auto at = [&](int p, int i) { return all + (static_cast<size_t>(p) * COUNT + i) * THREADS * 4; };
+#pragma unroll
+  for (int i = 0; i < COUNT; ++i) {
+    uint64_t* to = reinterpret_cast<uint64_t*>(at(part, i));
+    __hip_atomic_store(to, __builtin_bit_cast(uint64_t, f32x2_t{sums[i][0], sums[i][1]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(to + 1, __builtin_bit_cast(uint64_t, f32x2_t{sums[i][2], sums[i][3]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  release_stores();
+  __syncthreads();
+  if (tid == 0) {
+    const int before = __hip_atomic_fetch_add(g.tickets + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *last = before == g.splits - 1;
+    if (before == g.splits - 1) st_shared32(g.tickets + tile, 0);       // for the next product
+  }
+  __syncthreads();
+  if (!*last) return false;
+#pragma unroll
+  for (int i = 0; i < COUNT; ++i) sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int kBatch = COUNT <= 4 ? 4 : 2;      // parts asked for together
+  for (int p = 0; p < g.splits; p += kBatch) {
+    v4u r[kBatch][COUNT];
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b)
+#pragma unroll
+      for (int i = 0; i < COUNT; ++i) r[b][i] = ld_shared128(at(min(p + b, g.splits - 1), i));
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b)
+      if (p + b < g.splits)
+#pragma unroll
+        for (int i = 0; i < COUNT; ++i) sums[i] += __builtin_bit_cast(f32x4, r[b][i]);
+  }
+  return true;
+}
+
+// All streams of the residual for quads id, id + step, .. of a tile: the next quad's streams are asked for before this one's
+// are mixed.
+template <class At, class Value>
+__device__ __forceinline__ void residual_quads(const GemmArgs& g, int id, int total, int step, At&& at, Value&& value) {
+  const QmkHybridLayer& l = g.layer;
+  const int S = g.streams, D = g.width;
+  const float* hc = l.hc + (g.down ? S * (S + 2) : 0);
+  f32x4 old[kMaxStreams] = {}, ahead[kMaxStreams] = {};
+  auto load = [&](f32x4(&to)[kMaxStreams], int i) {
+    int m, n;
+    if (i >= total || !at(i, m, n)) return;
+    const float* x = g.f0 + static_cast<size_t>(m) * S * D + n;
+#pragma unroll
+    for (int s = 0; s < kMaxStreams; ++s)
+      if (s < S) to[s] = read4(x + static_cast<size_t>(s) * D);
+  };
+  load(old, id);
+#pragma unroll 1
+  for (; id < total; id += step) {
+    load(ahead, id + step);
+    int m, n;
+    if (at(id, m, n)) {
+      const f32x4 v = value(id);
+      float* x = g.f0 + static_cast<size_t>(m) * S * D + n;
+      f32x4 u = {};
+#pragma unroll
+      for (int t = 0; t < kMaxStreams; ++t) {
+        if (t < S) {
+          f32x4 now = v * hc[S + t];
+#pragma unroll
+          for (int s = 0; s < kMaxStreams; ++s)
+            if (s < S) now += old[s] * hc[2 * S + s * S + t];
+          store4(x + static_cast<size_t>(t) * D, now);
+          u += now * g.next[t];
+        }
+      }
+      store4(g.f1 + static_cast<size_t>(m) * D + n, u);
+    }
+#pragma unroll
+    for (int s = 0; s < kMaxStreams; ++s) old[s] = ahead[s];
+  }
+}
+
+// A workgroup's accumulators -> epilogue, through LDS (quads of a row exchanged by its number): the lanes of a row then
+// write neighbouring outputs of one token.  Unit LDS of the array is one word beside it.  (A kernel has one LDS array: with two,
+// this compiler waits for all requests before every read of the main loop, which costs half of the rate.)
+template <class T, class S, int LDS>
+__device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int tile, int part, int m0, int n0, int N, v4u* lds, f32x4 (&acc)[S::kTn][S::kTm]) {
+  constexpr int kQuads = S::BN / 4, kPassM = S::WM / S::kPasses, kRows = S::BM / S::kPasses, kTm = S::kTm;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave / S::kCover, wt = wave % S::kCover, wm = wt % S::kWavesM, wn = wt / S::kWavesM;
+  f32x4* out = reinterpret_cast<f32x4*>(lds);
+  f32x4 sums[S::kKept * kTm];
+  __syncthreads();
+  if constexpr (S::kGroups == 2) {      // each group keeps a half of the rows of weights and gives away the other
+    f32x4* box = out + wt * S::kKept * kTm * 64 + lane;
+    f32x4 *give = box + (1 - kg) * S::kCover * S::kKept * kTm * 64, *take = box + kg * S::kCover * S::kKept * kTm * 64;
+    static_assert(2 * S::kCover * S::kKept * kTm * 64 <= S::kLds, "both groups' halves");
+#pragma unroll
+    for (int j = 0; j < S::kKept; ++j)
+#pragma unroll
+      for (int i = 0; i < kTm; ++i) {
+        sums[j * kTm + i] = kg == 0 ? acc[j][i] : acc[S::kKept + j][i];
+        give[(j * kTm + i) * 64] = kg == 0 ? acc[S::kKept + j][i] : acc[j][i];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < S::kKept * kTm; ++c) sums[c] += take[c * 64];
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int c = 0; c < S::kKept * kTm; ++c) sums[c] = acc[c / kTm][c % kTm];
+  }
+  if constexpr (S::kSplits)
+    if (g.splits > 1 && !sum_parts<S::kKept * kTm, S::kThreadCount>(g, tile, part, sums, reinterpret_cast<int*>(lds + LDS))) return;
+#pragma unroll
+  for (int pass = 0; pass < S::kPasses; ++pass) {
+    if (pass > 0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTm / S::kPasses; ++i)
+#pragma unroll
+      for (int j = 0; j < S::kKept; ++j) {
+        const int r = wm * kPassM + i * 16 + (lane & 15), quad = wn * (S::WN / 4) + (kg * S::kKept + j) * 4 + (lane >> 4);
+        out[r * kQuads + (quad ^ (r & 15))] = sums[j * kTm + pass * (kTm / S::kPasses) + i];
+      }
+    __syncthreads();
+    auto at = [&](int id, int& m, int& n) {
+      const int r = id / kQuads;
+      m = m0 + r / kPassM * S::WM + pass * kPassM + r % kPassM;
+      n = n0 + id % kQuads * 4;
+      return m < g.M && n < N;
+    };
+    auto value = [&](int id) {
+      const int r = id / kQuads;
+      return out[r * kQuads + (id % kQuads ^ (r & 15))];
+    };
+    if (g.epi == EPI_RESIDUAL) {
+      residual_quads(g, tid, kRows * kQuads, S::kThreadCount, at, value);
+    } else {
+#pragma unroll 1
+      for (int id = tid; id < kRows * kQuads; id += S::kThreadCount) {
+        int m, n;
+        if (at(id, m, n)) epilogue<T>(g, group, m, n, value(id));
+      }
+    }
+  }
+}
+
+// Which part of the product a workgroup takes.
+struct Place {
+  int group, tile, part, m0, n0, N, first, steps;
+};
+template <class S>
+__device__ __forceinline__ Place place_of(const GemmArgs& g) {
+  Place p;
+  p.group = blockIdx.z;
+  p.N = p.group == g.groups - 1 ? g.last_n : g.N;
+  const int id = xcd_order(blockIdx.x, gridDim.x), tiles_m = (g.M + S::BM - 1) / S::BM, tile = id / g.splits;
+  p.part = id % g.splits;
+  p.m0 = tile % tiles_m * S::BM;
+  p.n0 = tile / tiles_m * S::BN;
+  p.tile = p.group * (gridDim.x / g.splits) + tile;
+  const int all = (g.K + S::BK - 1) / S::BK;
+  p.first = all * p.part / g.splits;
+  p.steps = all * (p.part + 1) / g.splits - p.first;
+  return p;
+}
+
+// Until at most `n` of this wave's vector-memory requests are outstanding and none of its LDS reads.
+template <int n>
+__device__ __forceinline__ void wait_outstanding() {
+  static_assert(n >= 0 && n < 64, "six bits");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(n) : "memory");
+}
+
+// The tiles of a step, bf16: memory -> LDS without passing through registers, kStages buffers deep.  A row's units are exchanged
+// by its number on the memory side (the LDS side of such a load is one run of 64 units per wave), so that fragment reads do
+// not conflict.
+template <class S>
+struct Stages {
+  using Lds = __attribute__((address_space(3))) v4u;      // said outright: a pointer kept in a struct may become a generic one
+  const u16* from[S::kLoads];      // this thread's places in a stage: unit i * threads + tid, tokens first
+  Lds* lds;
+  int wave;
+
+  static __device__ __forceinline__ int exchange(int r) { return S::kRow == 4 ? (r >> 1) & 3 : r & 7; }
+  __device__ __forceinline__ Stages(const GemmArgs& g, const Place& p, v4u* buffers, int wave_number) : lds((Lds*)buffers), wave(wave_number) {
+    const u16* a = static_cast<const u16*>(g.a) + p.group * g.a_step + p.first * S::BK;
+    const u16* w = static_cast<const u16*>(g.w) + p.group * g.w_step + p.first * S::BK;
+#pragma unroll
+    for (int i = 0; i < S::kLoads; ++i) {
+      const int u = i * S::kThreadCount + threadIdx.x, r = u / S::kRow, c = ((u % S::kRow) ^ exchange(r)) * 8;
+      from[i] = r < S::BM ? a + static_cast<size_t>(min(p.m0 + r, g.M - 1)) * g.lda + c : w + static_cast<size_t>(min(p.n0 + r - S::BM, p.N - 1)) * g.ldw + c;
+    }
+  }
+  __device__ __forceinline__ void issue(int buf) {
+#pragma unroll
+    for (int i = 0; i < S::kLoads; ++i) {
+      if (i == S::kLoads - 1 && S::kLastWaves * 64 < S::kThreadCount && wave >= S::kLastWaves) continue;
+      const auto* src = (const __attribute__((address_space(1))) uint32_t*)from[i];
+      auto* dst = (__attribute__((address_space(3))) uint32_t*)(lds + buf * S::kUnits + i * S::kThreadCount + wave * 64);
+      __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+      from[i] += S::BK;
+    }
+  }
+  // Until at most `stages` stages of this wave's are outstanding.
+  template <int stages>
+  __device__ __forceinline__ void wait() const {
+    if (S::kLastWaves * 64 == S::kThreadCount || wave < S::kLastWaves) wait_outstanding<stages * S::kLoads>();
+    else wait_outstanding<stages * (S::kLoads - 1)>();
+  }
+  __device__ __forceinline__ void fragments(int buf, int q, int wm, int wn, Frag<u16> (&fa)[S::kTm], Frag<u16> (&fw)[S::kTn]) const {
+    const Lds *la = lds + buf * S::kUnits, *lw = la + S::BM * S::kRow;
+    const int row = threadIdx.x & 15;
+    auto frag = [](const Lds* at) { return Frag<u16>{__builtin_bit_cast(bf16x8_t, *at)}; };
+#pragma unroll
+    for (int j = 0; j < S::kTn; ++j) {
+      const int r = wn * S::WN + j * 16 + row;
+      fw[j] = frag(lw + r * S::kRow + (q ^ exchange(r)));
+    }
+#pragma unroll
+    for (int i = 0; i < S::kTm; ++i) {
+      const int r = wm * S::WM + i * 16 + row;
+      fa[i] = frag(la + r * S::kRow + (q ^ exchange(r)));
+    }
+  }
+};
+
+template <class S>
+__device__ __forceinline__ void multiply(const Frag<u16> (&fa)[S::kTm], const Frag<u16> (&fw)[S::kTn], f32x4 (&acc)[S::kTn][S::kTm]) {
+#pragma unroll
+  for (int i = 0; i < S::kTm; ++i)
+#pragma unroll
+    for (int j = 0; j < S::kTn; ++j) acc[j][i] = mma(fw[j], fa[i], acc[j][i]);
+}
+
+// out[m][n] = sum_k a[m][k] w[n][k], bf16 x bf16, K a multiple of BK.  The weights are the matrix instruction's first operand,
+// so a lane ends up with four consecutive outputs of one token.  Four waves; several workgroups share a CU.
+template <class T, class S>
+__global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g) {
+  constexpr int kAhead = S::kStages - 1;
+  __shared__ __align__(16) v4u lds[S::kLds + 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % S::kWavesM, wn = wave / S::kWavesM;
+  const Place p = place_of<S>(g);
+  if (p.n0 >= p.N) return;
+  Stages<S> stages(g, p, lds, wave);
+  f32x4 acc[S::kTn][S::kTm] = {};
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s)
+    if (s < p.steps) stages.issue(s);
+  int buf = 0;
+  for (int s = 0; s < p.steps; ++s) {
+    // Everything up to this step's stage has landed; the barrier makes that true of every wave's part, and says that the
+    // buffer filled next is no longer read.
+    if (s + kAhead - 1 < p.steps) stages.template wait<kAhead - 1>();
+    else wait_outstanding<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + kAhead < p.steps) stages.issue(buf == 0 ? S::kStages - 1 : buf - 1);
+#pragma unroll
+    for (int kk = 0; kk < S::kSteps; ++kk) {
+      Frag<u16> fa[S::kTm], fw[S::kTn];
+      stages.fragments(buf, kk * 4 + (lane >> 4), wm, wn, fa, fw);
+      multiply<S>(fa, fw, acc);
+    }
+    buf = buf + 1 == S::kStages ? 0 : buf + 1;
+  }
+  finish_tile<T, S, S::kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+}
+
+// The same with eight waves, one workgroup a CU.  Two waves share a SIMD's matrix unit, and the halves of the workgroup take
+// turns: while one multiplies, the other reads its next fragments; a barrier ends each turn, and the second half starts one
+// turn late.
+template <class T, class S>
+__global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
+  static_assert(S::kThreadCount == 512 && S::kSteps == 1 && S::kStages == 4, "one turn a step, three stages ahead");
+  constexpr int kAhead = S::kStages - 1;
+  __shared__ __align__(16) v4u lds[S::kLds + 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = wave / S::kCover, wt = wave % S::kCover, wm = wt % S::kWavesM, wn = wt / S::kWavesM;
+  const Place p = place_of<S>(g);
+  if (p.n0 >= p.N) return;
+  Stages<S> stages(g, p, lds, wave);
+  auto barrier = [] {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  };
+  f32x4 acc[S::kTn][S::kTm] = {};
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s)
+    if (s < p.steps) stages.issue(s);
+  if (kAhead - 1 < p.steps) stages.template wait<kAhead - 1>();
+  else wait_outstanding<0>();
+  barrier();                       // stage 0 is there
+  if (wave >= 4) barrier();
+  int buf = 0;
+  for (int s = 0; s < p.steps; ++s) {
+    // The buffer filled here was read in step s - 1: by this half a turn ago, by the other one before the last barrier.
+    if (s + kAhead < p.steps) stages.issue(buf == 0 ? S::kStages - 1 : buf - 1);
+    Frag<u16> fa[S::kTm], fw[S::kTn];
+    stages.fragments(buf, kg * 4 + (lane >> 4), wm, wn, fa, fw);
+    // Stage s + 1 has landed: a barrier lies between this wait and either half's reads of it.
+    if (s + kAhead < p.steps) stages.template wait<kAhead - 1>();
+    else wait_outstanding<0>();
+    barrier();
+    __builtin_amdgcn_s_setprio(1);
+    multiply<S>(fa, fw, acc);
+    __builtin_amdgcn_s_setprio(0);
+    barrier();
+    buf = buf + 1 == S::kStages ? 0 : buf + 1;
+  }
+  if (wave < 4) barrier();
+  finish_tile<T, S, S::kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+}
+
+// ---- products with an fp32 side, and bf16 ones of any K ----
+// An fp32 value is the sum of three bf16 values that take its significand's bits 23..16, 15..8 and 7..0 (exactly: every
+// remainder is exact, and the exponents are the same), and a product of two bf16 values is exact in fp32: three bf16 instructions
+// add up the same products as the eight fp32 ones of the same columns, in a fifth of their time.  Values that are not finite
+// stay whole in the first part.
+template <class T>
+constexpr int kPlanes = sizeof(T) == 2 ? 1 : 3;
+__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+__device__ __forceinline__ float behind_upper_half(float v) { return v - __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
+__device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+// Eight values -> their planes.
+__device__ __forceinline__ void split8(const v4u& lo, const v4u& hi, v4u (&plane)[3]) {
+  const uint32_t bits[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  bool odd = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float x = __uint_as_float(bits[2 * e]), y = __uint_as_float(bits[2 * e + 1]);
+    odd |= not_finite(x) | not_finite(y);
+    plane[0][e] = upper_halves(x, y);
+    const float x1 = behind_upper_half(x), y1 = behind_upper_half(y);
+    plane[1][e] = upper_halves(x1, y1);
+    plane[2][e] = upper_halves(behind_upper_half(x1), behind_upper_half(y1));
+  }
+  if (__builtin_expect(odd, 0)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = __uint_as_float(bits[e]);
+      if (not_finite(x)) {
+        const uint32_t keep = e & 1 ? 0x0000ffffu : 0xffff0000u, top = x != x ? 0x7fc0u : bits[e] >> 16;
+        plane[0][e >> 1] = (plane[0][e >> 1] & keep) | (e & 1 ? top << 16 : top);
+        plane[1][e >> 1] &= keep;
+        plane[2][e >> 1] &= keep;
+      }
+    }
+  }
+}
+
+// BN weight rows x BM tokens a workgroup, four waves as 2 x 2, 64 columns a step, through registers.  LDS holds
+// 16-byte units of bf16, planes one after the other, a row's units exchanged by its number.
+template <class TA, class TW, class T, int BM_, int BN_, int BUFFERS>
+__global__ __launch_bounds__(kPfThreads) void gemm(const GemmArgs g) {
+  using S = Tile<BM_, BN_, 64, BM_ / 2, BN_ / 2, 4, 2>;
+  constexpr int BM = S::BM, BN = S::BN, kBK = S::BK, kTm = S::kTm, kTn = S::kTn;
+  constexpr int kPa = kPlanes<TA>, kPw = kPlanes<TW>, kUnitsA = BM * 8, kUnitsW = BN * 8;
+  constexpr int kRunsA = kUnitsA / kPfThreads, kRunsW = kUnitsW / kPfThreads;       // runs of eight columns a thread stages
+  constexpr int kStage = kPa * kUnitsA + kPw * kUnitsW, kLds = BUFFERS * kStage > S::kOutUnits ? BUFFERS * kStage : S::kOutUnits;
+  __shared__ __align__(16) v4u lds[kLds + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+  const Place p = place_of<S>(g);
+  if (p.n0 >= p.N) return;
+  const TA* a = static_cast<const TA*>(g.a) + p.group * g.a_step;
+  const TW* w = static_cast<const TW*>(g.w) + p.group * g.w_step;
+
+  v4u ra[kRunsA][sizeof(TA) / 2], rw[kRunsW][sizeof(TW) / 2];
+  auto fetch = [&](int k0) {
+    auto side = [&](auto* base, auto& r, int runs, int row0, int rows, long long ld) {
+      constexpr int kUnit = 16 / sizeof(*base), kEach = 8 / kUnit;
+#pragma unroll
+      for (int i = 0; i < runs; ++i) {
+        const int id = i * kPfThreads + tid, k = k0 + id % 8 * 8;
+        const auto* from = base + static_cast<size_t>(min(row0 + id / 8, rows - 1)) * ld + k;
+#pragma unroll
+        for (int e = 0; e < kEach; ++e)
+          r[i][e] = k + e * kUnit < g.K ? *reinterpret_cast<const v4u*>(from + e * kUnit) : v4u{0u, 0u, 0u, 0u};
+      }
+    };
+    side(a, ra, kRunsA, p.m0, g.M, g.lda);
+    side(w, rw, kRunsW, p.n0, p.N, g.ldw);
+  };
+  auto stash = [&](int buf) {
+    auto side = [&](auto tag, auto& r, int runs, v4u* to, int units) {
+      using E = decltype(tag);
+#pragma unroll
+      for (int i = 0; i < runs; ++i) {
+        const int id = i * kPfThreads + tid, row = id / 8, place = row * 8 + (id % 8 ^ (row & 7));
+        if constexpr (sizeof(E) == 2) {
+          to[place] = r[i][0];
+        } else {
+          v4u plane[3];
+          split8(r[i][0], r[i][1], plane);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) to[q * units + place] = plane[q];
+        }
+      }
+    };
+    side(TA{}, ra, kRunsA, lds + buf * kStage, kUnitsA);
+    side(TW{}, rw, kRunsW, lds + buf * kStage + kPa * kUnitsA, kUnitsW);
+  };
+  f32x4 acc[kTn][kTm] = {};
+  if (p.steps > 0) {
+    fetch(p.first * kBK);
+    stash(0);
+  }
+  __syncthreads();
+  for (int s = 0; s < p.steps; ++s) {
+    const v4u *la = lds + (BUFFERS == 2 ? s & 1 : 0) * kStage, *lw = la + kPa * kUnitsA;
+    if (s + 1 < p.steps) fetch((p.first + s + 1) * kBK);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int q = kk * 4 + (lane >> 4);
+      Frag<u16> fa[kPa][kTm], fw[kPw][kTn];
+#pragma unroll
+      for (int pl = 0; pl < kPa; ++pl)
+#pragma unroll
+        for (int i = 0; i < kTm; ++i) {
+          const int r = wm * S::WM + i * 16 + (lane & 15);
+          fa[pl][i] = load_frag(reinterpret_cast<const u16*>(la + pl * kUnitsA + r * 8 + (q ^ (r & 7))));
+        }
+#pragma unroll
+      for (int pl = 0; pl < kPw; ++pl)
+#pragma unroll
+        for (int j = 0; j < kTn; ++j) {
+          const int r = wn * S::WN + j * 16 + (lane & 15);
+          fw[pl][j] = load_frag(reinterpret_cast<const u16*>(lw + pl * kUnitsW + r * 8 + (q ^ (r & 7))));
+        }
+      static_assert(kPa == 1 || kPw == 1, "one side is bf16");
+#pragma unroll
+      for (int j = 0; j < kTn; ++j)
+#pragma unroll
+        for (int i = 0; i < kTm; ++i) {
+          if constexpr (kPa * kPw == 1) {
+            acc[j][i] = mma(fw[0][j], fa[0][i], acc[j][i]);
+          } else {      // 32 columns by themselves, small parts first, then one rounded addition
+            f32x4 t = {};
+#pragma unroll
+            for (int pl = 2; pl >= 0; --pl) t = mma(fw[kPw == 1 ? 0 : pl][j], fa[kPa == 1 ? 0 : pl][i], t);
+            acc[j][i] += t;
+          }
+        }
+    }
+    if (BUFFERS == 1) __syncthreads();
+    if (s + 1 < p.steps) stash(BUFFERS == 2 ? (s + 1) & 1 : 0);
+    __syncthreads();
+  }
+  finish_tile<T, S, kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+}
+
+// At most 64 columns with an fp32 side: one step, where the fp32 instruction is no slower than three parts (5.1 us against 5.6 for
+// 64 x 64 x 64; both are a launch and its loads).
+template <class TA, class TW, class T>
+__global__ __launch_bounds__(kPfThreads) void gemm_short(const GemmArgs g) {
+  using S = Tile<64, 64, 64, 32, 32, 4, 4>;
+  constexpr int kUnitA = 16 / sizeof(TA), kUnitW = 16 / sizeof(TW), kRowA = 64 / kUnitA, kRowW = 64 / kUnitW;
+  __shared__ __align__(16) v4u lds[S::kLds + 1];
+  static_assert(64 * (kRowA + kRowW) <= S::kLds, "both tiles");
+  v4u *la = lds, *lw = lds + 64 * kRowA;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+  const Place p = place_of<S>(g);
+  if (p.n0 >= p.N) return;
+  auto place = [](int r, int unit, int row_units) { return r * row_units + (unit ^ ((r & 7) * (row_units / 8))); };
+  auto stage = [&](auto* from, v4u* to, int row_units, int unit, int row0, int rows, long long ld) {
+    for (int id = tid; id < 64 * row_units; id += kPfThreads) {
+      const int r = id / row_units, k = id % row_units * unit;
+      to[place(r, id % row_units, row_units)] =
+          k < g.K ? *reinterpret_cast<const v4u*>(from + static_cast<size_t>(min(row0 + r, rows - 1)) * ld + k) : v4u{0u, 0u, 0u, 0u};
+    }
+  };
+  stage(static_cast<const TA*>(g.a) + p.group * g.a_step, la, kRowA, kUnitA, p.m0, g.M, g.lda);
+  stage(static_cast<const TW*>(g.w) + p.group * g.w_step, lw, kRowW, kUnitW, p.n0, p.N, g.ldw);
+  __syncthreads();
+  f32x4 acc[S::kTn][S::kTm] = {};
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int q = kk * 4 + (lane >> 4);
+    Frag<TA> fa[S::kTm];
+#pragma unroll
+    for (int i = 0; i < S::kTm; ++i) fa[i] = load_frag(reinterpret_cast<const TA*>(&la[place(wm * S::WM + i * 16 + (lane & 15), q * (kRowA / 8), kRowA)]));
+#pragma unroll
+    for (int j = 0; j < S::kTn; ++j) {
+      const Frag<TW> fw = load_frag(reinterpret_cast<const TW*>(&lw[place(wn * S::WN + j * 16 + (lane & 15), q * (kRowW / 8), kRowW)]));
+#pragma unroll
+      for (int i = 0; i < S::kTm; ++i) acc[j][i] = mma(fw, fa[i], acc[j][i]);
+    }
+  }
+  finish_tile<T, S, S::kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+}
+
+// ---- which tiles ----
+using Tiles64 = Tile<64, 64, 64, 32, 32, 4, 4>;
+using Tiles128 = Tile<128, 128, 64, 64, 64, 4, 2>;
+using Turns64 = Tile<64, 128, 64, 32, 64, 8, 4>;
+using Turns96 = Tile<96, 128, 64, 48, 64, 8, 4>;
+using Turns128 = Tile<128, 128, 64, 64, 64, 8, 4>;
+using Turns192 = Tile<192, 256, 32, 96, 64, 8, 4>;
+using Turns256 = Tile<256, 256, 32, 128, 64, 8, 4>;
+
+constexpr int kMaxTickets = 512;                       // tiles of a product that is cut along K
+constexpr int kPartialUnits = 256 * 128 * 128 / 4;     // quads its parts leave: 256 of 128 x 128, or as many values
+
+}  // namespace hybrid
+}  // namespace qmk

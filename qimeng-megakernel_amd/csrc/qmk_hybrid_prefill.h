@@ -1,446 +1,15 @@
 // Prefill kernels of the hybrid route: a portion of M tokens, one launch per fused operation.
 //
 // Element type T (bf16 or fp32) is that of the activations between kernels; sums, norms, angles, scores, gates,
-// recurrences and the residual streams are fp32 in both.  Weights are bf16 in memory in both: in fp32 mode they are
-// widened in registers and multiplied by the fp32 matrix instructions.
+// recurrences and the residual streams are fp32 in both.  Weights are bf16 in memory in both; in fp32 mode a product's
+// activations are cut into three bf16 parts on their way to the matrix instructions (qmk_hybrid_gemm.h), and attention and the
+// recurrences use the fp32 ones.
 #pragma once
 
-#include "qmk_hybrid_ops.h"
+#include "qmk_hybrid_gemm.h"
 
 namespace qmk {
 namespace hybrid {
-
-constexpr int kPfThreads = 256;
-
-enum : int {
-  EPI_STORE = 0,        // out T [m][ldo]
-  EPI_RGLRU_IN,         // gelu of the y half, bias on both
-  EPI_LRU_GATES,        // (r, i) pairs -> decay a and input b of the recurrence
-  EPI_LATENT_IN,        // rotation of q, sigmoid of the gate, raw latent
-  EPI_RESIDUAL,         // all streams of the residual and the next sublayer's input
-  EPI_GEGLU,            // (gate, up) pairs
-  EPI_WKV_IN,           // r, k, v fp32; silu gate; tanh
-  EPI_WKV_DECAY,        // exp(-exp(. + w0))
-  EPI_LOGITS,
-  EPI_CAPPED_LOGITS,    // logits times a constant, softly capped
-  EPI_ADD,              // onto the fp32 residual
-  EPI_ATTENTION_IN,     // rotation of q and k, k and v into the cache, sigmoid of the gate
-  EPI_DELTA_IN,         // q, k, v fp32; raw ranks; sigmoid of the step sizes
-  EPI_DELTA_DECAY,
-  EPI_SIGMOID,
-  EPI_GLA_IN,           // q, k, v fp32; silu gate; raw rank
-  EPI_GLA_DECAY,
-};
-
-struct GemmArgs {
-  const void* a;         // TA [M][lda]
-  const void* w;         // TW [N][ldw]
-  int M, N, K, lda, ldw, groups, last_n;   // group g: a + g a_step, w + g w_step, N rows (the last: last_n)
-  long long a_step, w_step;
-  int epi;
-  void* out;             // meaning by epilogue
-  void* out2;
-  float* f0;
-  float* f1;
-  const void* src;
-  int ldo;
-  QmkHybridLayer layer;
-  int down, first, position, streams, width, rows_cap, slot;
-  float logit_scale, logit_softcap;
-  const float* next;
-};
-
-template <class T>
-__device__ __forceinline__ void store4(T* at, f32x4 v) {
-  if constexpr (sizeof(T) == 2) {
-    *reinterpret_cast<uint2*>(at) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
-  } else {
-    *reinterpret_cast<f32x4*>(at) = v;
-  }
-}
-template <class T>
-__device__ __forceinline__ f32x4 read4(const T* at) {
-  if constexpr (sizeof(T) == 2) {
-    const uint2 t = *reinterpret_cast<const uint2*>(at);
-    return f32x4{bf_lo(t.x), bf_hi(t.x), bf_lo(t.y), bf_hi(t.y)};
-  } else {
-    return *reinterpret_cast<const f32x4*>(at);
-  }
-}
-
-// Four consecutive outputs n .. n+3 of token m.
-template <class T>
-__device__ __forceinline__ void epilogue(const GemmArgs& g, int group, int m, int n, f32x4 v) {
-  const QmkHybridLayer& l = g.layer;
-  switch (g.epi) {
-    case EPI_STORE: store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + n, v); break;
-    case EPI_RGLRU_IN: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.in_b + n);
-      v += b;
-      if (n < l.mix_width) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = gelu_tanh(v[i]);
-        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * l.mix_width + n, v);
-      } else {
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.mix_width + n - l.mix_width, v);
-      }
-      break;
-    }
-    case EPI_LRU_GATES: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + static_cast<size_t>(group) * 2 * l.block_dim + n);
-      v += b;
-      const int c = group * l.block_dim + n / 2;
-      const size_t at = static_cast<size_t>(m) * l.mix_width + c;
-      const T* u = static_cast<const T*>(g.src) + at;
-      float2 a2, b2;
-      {
-        const float la = sigmoid(v[0]) * l.vec0[c];
-        a2.x = expf(la);
-        b2.x = sqrtf(-expm1f(2.f * la)) * sigmoid(v[1]) * to_f32(u[0]);
-      }
-      {
-        const float la = sigmoid(v[2]) * l.vec0[c + 1];
-        a2.y = expf(la);
-        b2.y = sqrtf(-expm1f(2.f * la)) * sigmoid(v[3]) * to_f32(u[1]);
-      }
-      *reinterpret_cast<float2*>(g.f0 + at) = a2;
-      *reinterpret_cast<float2*>(g.f1 + at) = b2;
-      break;
-    }
-    case EPI_LATENT_IN: {
-      const int q_rows = l.heads * l.q_stride, g_rows = l.heads * l.v_dim;
-      if (n < q_rows) {
-        const int d = n % l.q_stride - l.head_dim;
-        if (d >= 0) {
-          float e[4] = {v[0], v[1], v[2], v[3]};
-          rotate(l, g.position + m, d, e[0], e[1]);
-          rotate(l, g.position + m, d + 2, e[2], e[3]);
-          v = f32x4{e[0], e[1], e[2], e[3]};
-        }
-        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * q_rows + n, v);
-      } else if (n < q_rows + g_rows) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * g_rows + n - q_rows, v);
-      } else {
-        store4(g.f0 + static_cast<size_t>(m) * (l.rank + l.rot_dim) + n - q_rows - g_rows, v);
-      }
-      break;
-    }
-    case EPI_RESIDUAL: {
-      const int S = g.streams, D = g.width;
-      const float* hc = l.hc + (g.down ? S * (S + 2) : 0);
-      float* x = g.f0 + static_cast<size_t>(m) * S * D + n;
-      f32x4 old[kMaxStreams];
-#pragma unroll
-      for (int s = 0; s < kMaxStreams; ++s)
-        if (s < S) old[s] = *reinterpret_cast<const f32x4*>(x + static_cast<size_t>(s) * D);
-      f32x4 u = {};
-#pragma unroll
-      for (int t = 0; t < kMaxStreams; ++t) {
-        if (t < S) {
-          f32x4 now = v * hc[S + t];
-#pragma unroll
-          for (int s = 0; s < kMaxStreams; ++s)
-            if (s < S) now += old[s] * hc[2 * S + s * S + t];
-          *reinterpret_cast<f32x4*>(x + static_cast<size_t>(t) * D) = now;
-          u += now * g.next[t];
-        }
-      }
-      *reinterpret_cast<f32x4*>(g.f1 + static_cast<size_t>(m) * D + n) = u;
-      break;
-    }
-    case EPI_GEGLU: {
-      T* o = static_cast<T*>(g.out) + static_cast<size_t>(m) * l.ff + n / 2;
-      const bool silu = l.act == QMK_ACT_SILU;
-      const float a = (silu ? v[0] * sigmoid(v[0]) : gelu_tanh(v[0])) * v[1], b = (silu ? v[2] * sigmoid(v[2]) : gelu_tanh(v[2])) * v[3];
-      if constexpr (sizeof(T) == 2) *reinterpret_cast<uint32_t*>(o) = f2bf2(a, b);
-      else *reinterpret_cast<float2*>(o) = make_float2(a, b);
-      break;
-    }
-    case EPI_WKV_IN: {
-      const int N = l.heads * l.head_dim;
-      if (group < 3) {
-        store4(g.f0 + (static_cast<size_t>(group) * g.rows_cap + m) * N + n, v);
-      } else if (group == 3) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= sigmoid(v[i]);
-        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * N + n, v);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = tanhf(v[i]);
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.rank + n, v);
-      }
-      break;
-    }
-    case EPI_WKV_DECAY: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = expf(-expf(v[i] + b[i]));
-      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    case EPI_CAPPED_LOGITS: {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = soft_cap(v[i] * g.logit_scale, g.logit_softcap);
-      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    case EPI_ADD: {
-      float* x = g.f0 + static_cast<size_t>(m) * g.ldo + n;
-      store4(x, read4(x) + v);
-      break;
-    }
-    case EPI_ATTENTION_IN: {
-      const int q_rows = l.heads * l.q_stride, k_rows = l.kv_heads * l.head_dim, v_rows = l.kv_heads * l.v_dim, row = l.head_dim + l.v_dim, pos = g.position + m;
-      T* cache = static_cast<T*>(l.cache) + (static_cast<size_t>(g.slot) * l.ring + pos % l.ring) * l.kv_heads * row;
-      if (n < q_rows + k_rows) {
-        const int d = n < q_rows ? n % l.q_stride : (n - q_rows) % l.head_dim;
-        float e[4] = {v[0], v[1], v[2], v[3]};
-        rotate(l, pos, d, e[0], e[1]);
-        rotate(l, pos, d + 2, e[2], e[3]);
-        v = f32x4{e[0], e[1], e[2], e[3]};
-        store4(n < q_rows ? static_cast<T*>(g.out) + static_cast<size_t>(m) * q_rows + n : cache + (n - q_rows) / l.head_dim * row + d, v);
-      } else if (n < q_rows + k_rows + v_rows) {
-        const int c = n - q_rows - k_rows;
-        store4(cache + c / l.v_dim * row + l.head_dim + c % l.v_dim, v);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.mix_width + n - q_rows - k_rows - v_rows, v);
-      }
-      break;
-    }
-    case EPI_DELTA_IN: {
-      const int channels = conv_channels(l), ranks = l.rank + l.gate_rank;
-      if (n < channels) {
-        store4(g.f1 + static_cast<size_t>(m) * channels + n, v);
-      } else if (n < channels + ranks) {
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * ranks + n - channels, v);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
-        store4(g.f0 + static_cast<size_t>(m) * g.ldo + n - channels - ranks, v);
-      }
-      break;
-    }
-    case EPI_DELTA_DECAY: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = delta_decay(l, n / l.head_dim, v[i] + b[i]);
-      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    case EPI_SIGMOID: {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
-      store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    case EPI_GLA_IN: {
-      const int qkv = 2 * l.heads * l.head_dim + l.mix_width;
-      if (n < qkv) {
-        store4(g.f0 + static_cast<size_t>(m) * qkv + n, v);
-      } else if (n < qkv + l.mix_width) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= sigmoid(v[i]);
-        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * l.mix_width + n - qkv, v);
-      } else {
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.rank + n - qkv - l.mix_width, v);
-      }
-      break;
-    }
-    case EPI_GLA_DECAY: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = gla_decay(l, v[i] + b[i]);
-      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    default: store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v); break;
-  }
-}
-
-// A workgroup's accumulators -> epilogue, through LDS (a wave's own part, quads of a row exchanged by its number): a lane's
-// accumulators are then read back in a loop, and the lanes of a row write neighbouring outputs of one token.
-template <class T, int BM, int BN, int kTn, int kTm>
-__device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int m0, int n0, int N, v4u* lds, const f32x4 (&acc)[kTn][kTm]) {
-  constexpr int kWm = BM / 2, kWn = BN / 2, kQuads = kWn / 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave & 1, wn = wave >> 1;
-  f32x4* out = reinterpret_cast<f32x4*>(lds) + wave * kWm * kQuads;
-#pragma unroll
-  for (int i = 0; i < kTm; ++i)
-#pragma unroll
-    for (int j = 0; j < kTn; ++j) {
-      const int m = i * 16 + (lane & 15), quad = j * 4 + (lane >> 4);
-      out[m * kQuads + (quad ^ (m & (kQuads - 1)))] = acc[j][i];
-    }
-#pragma unroll 1
-  for (int id = lane; id < kWm * kQuads; id += 64) {
-    const int r = id / kQuads, quad = id % kQuads, m = m0 + wm * kWm + r, n = n0 + wn * kWn + quad * 4;
-    if (m < g.M && n < N) epilogue<T>(g, group, m, n, out[r * kQuads + (quad ^ (r & (kQuads - 1)))]);
-  }
-}
-
-// Until at most `n` of this wave's vector-memory requests are outstanding and none of its LDS reads.
-template <int n>
-__device__ __forceinline__ void wait_outstanding() {
-  static_assert(n >= 0 && n < 64, "six bits");
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(n) : "memory");
-}
-
-// out[m][n] = sum_k a[m][k] w[n][k]: BN weight rows x BM tokens per workgroup, four waves as 2 x 2, 64 columns a step.
-// The weights are the matrix instruction's first operand, so a lane ends up with four consecutive outputs of one token.
-// LDS tiles hold 16-byte units, a row's units rotated by the row number (conflict-free fragment reads).
-template <class TA, class TW, class T, int BM, int BN>
-__global__ __launch_bounds__(kPfThreads) void gemm(const GemmArgs g) {
-  constexpr int kBK = 64;
-  constexpr int kUnitA = 16 / sizeof(TA), kUnitW = 16 / sizeof(TW);       // elements of a unit
-  constexpr int kRowA = kBK / kUnitA, kRowW = kBK / kUnitW;                // units of a row
-  constexpr int kLoadsA = BM * kRowA / kPfThreads, kLoadsW = BN * kRowW / kPfThreads;
-  constexpr int kTm = BM / 2 / 16, kTn = BN / 2 / 16;
-  constexpr int kTileUnits = 2 * (BM * kRowA + BN * kRowW), kOutUnits = BM * BN / 4;
-  __shared__ v4u lds[kTileUnits > kOutUnits ? kTileUnits : kOutUnits];
-  v4u(*la)[BM * kRowA] = reinterpret_cast<v4u(*)[BM * kRowA]>(lds);
-  v4u(*lw)[BN * kRowW] = reinterpret_cast<v4u(*)[BN * kRowW]>(lds + 2 * BM * kRowA);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 1, wn = wave >> 1;
-  const int group = blockIdx.z;
-  const int N = group == g.groups - 1 ? g.last_n : g.N;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  if (n0 >= N) return;
-  const TA* a = static_cast<const TA*>(g.a) + group * g.a_step;
-  const TW* w = static_cast<const TW*>(g.w) + group * g.w_step;
-
-  v4u ra[kLoadsA], rw[kLoadsW];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < kLoadsA; ++i) {
-      const int id = i * kPfThreads + tid, r = id / kRowA, c = id % kRowA, k = k0 + c * kUnitA;
-      v4u z = {0u, 0u, 0u, 0u};
-      ra[i] = k < g.K ? *reinterpret_cast<const v4u*>(a + static_cast<size_t>(min(m0 + r, g.M - 1)) * g.lda + k) : z;
-    }
-#pragma unroll
-    for (int i = 0; i < kLoadsW; ++i) {
-      const int id = i * kPfThreads + tid, r = id / kRowW, c = id % kRowW, k = k0 + c * kUnitW;
-      v4u z = {0u, 0u, 0u, 0u};
-      rw[i] = k < g.K ? *reinterpret_cast<const v4u*>(w + static_cast<size_t>(min(n0 + r, N - 1)) * g.ldw + k) : z;
-    }
-  };
-  auto place = [](int r, int unit, int row_units) { return r * row_units + (unit ^ ((r & 7) * (row_units / 8))); };
-  auto stash = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < kLoadsA; ++i) {
-      const int id = i * kPfThreads + tid;
-      la[buf][place(id / kRowA, id % kRowA, kRowA)] = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < kLoadsW; ++i) {
-      const int id = i * kPfThreads + tid;
-      lw[buf][place(id / kRowW, id % kRowW, kRowW)] = rw[i];
-    }
-  };
-  f32x4 acc[kTn][kTm] = {};
-  const int steps = (g.K + kBK - 1) / kBK;
-  fetch(0);
-  stash(0);
-  __syncthreads();
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s & 1;
-    if (s + 1 < steps) fetch((s + 1) * kBK);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      Frag<TA> fa[kTm];
-      const int q = kk * 4 + (lane >> 4);      // which run of eight columns
-#pragma unroll
-      for (int i = 0; i < kTm; ++i) {
-        const int r = wm * (BM / 2) + i * 16 + (lane & 15);
-        fa[i] = load_frag(reinterpret_cast<const TA*>(&la[buf][place(r, q * (kRowA / 8), kRowA)]));
-      }
-#pragma unroll
-      for (int j = 0; j < kTn; ++j) {
-        const int r = wn * (BN / 2) + j * 16 + (lane & 15);
-        const Frag<TW> fw = load_frag(reinterpret_cast<const TW*>(&lw[buf][place(r, q * (kRowW / 8), kRowW)]));
-#pragma unroll
-        for (int i = 0; i < kTm; ++i) acc[j][i] = mma(fw, fa[i], acc[j][i]);
-      }
-    }
-    if (s + 1 < steps) stash(buf ^ 1);
-    __syncthreads();
-  }
-  finish_tile<T, BM, BN>(g, group, m0, n0, N, lds, acc);
-}
-
-// The same for bf16 x bf16 with K a multiple of 64: tiles go from memory to LDS without passing through registers, STAGES
-// buffers deep, so that STAGES - 1 steps are in flight while one is multiplied.
-template <class T, int BM, int BN, int STAGES>
-__global__ __launch_bounds__(kPfThreads) void gemm_direct(const GemmArgs g) {
-  constexpr int kBK = 64, kRow = kBK / 8;                                   // a row: eight units of 16 bytes
-  constexpr int kLoads = (BM + BN) * kRow / kPfThreads, kStageUnits = (BM + BN) * kRow;
-  constexpr int kTm = BM / 2 / 16, kTn = BN / 2 / 16, kOutUnits = BM * BN / 4, kAhead = STAGES - 1;
-  __shared__ __align__(16) v4u lds[STAGES * kStageUnits > kOutUnits ? STAGES * kStageUnits : kOutUnits];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
-  const int group = blockIdx.z;
-  const int N = group == g.groups - 1 ? g.last_n : g.N;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  if (n0 >= N) return;
-  const u16* a = static_cast<const u16*>(g.a) + group * g.a_step;
-  const u16* w = static_cast<const u16*>(g.w) + group * g.w_step;
-
-  // This thread's places in a stage: unit i * 256 + tid, tokens first.  A row's units are exchanged by its number, here on
-  // the memory side: the LDS side of such a load is one run of 64 units per wave.
-  const u16* from[kLoads];
-#pragma unroll
-  for (int i = 0; i < kLoads; ++i) {
-    const int id = i * kPfThreads + tid, r = id / kRow, c = ((id % kRow) ^ (r & 7)) * 8;
-    from[i] = r < BM ? a + static_cast<size_t>(min(m0 + r, g.M - 1)) * g.lda + c : w + static_cast<size_t>(min(n0 + r - BM, N - 1)) * g.ldw + c;
-  }
-  auto issue = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      const auto* src = (const __attribute__((address_space(1))) uint32_t*)from[i];
-      auto* dst = (__attribute__((address_space(3))) uint32_t*)(lds + buf * kStageUnits + i * kPfThreads + wave * 64);
-      __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
-      from[i] += kBK;
-    }
-  };
-  f32x4 acc[kTn][kTm] = {};
-  const int steps = g.K / kBK;
-#pragma unroll
-  for (int s = 0; s < kAhead; ++s)
-    if (s < steps) issue(s);
-  int buf = 0;
-  for (int s = 0; s < steps; ++s) {
-    // Everything up to this step's stage has landed; the barrier makes that true of every wave's part, and says that the
-    // buffer filled next is no longer read.
-    if (s + kAhead - 1 < steps) wait_outstanding<(kAhead - 1) * kLoads>();
-    else wait_outstanding<0>();
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (s + kAhead < steps) issue(buf == 0 ? STAGES - 1 : buf - 1);
-    const v4u* la = lds + buf * kStageUnits;
-    const v4u* lw = la + BM * kRow;
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const int q = kk * 4 + (lane >> 4);
-      Frag<u16> fa[kTm];
-#pragma unroll
-      for (int i = 0; i < kTm; ++i) {
-        const int r = wm * (BM / 2) + i * 16 + (lane & 15);
-        fa[i] = load_frag(reinterpret_cast<const u16*>(la + r * kRow + (q ^ (r & 7))));
-      }
-#pragma unroll
-      for (int j = 0; j < kTn; ++j) {
-        const int r = wn * (BN / 2) + j * 16 + (lane & 15);
-        const Frag<u16> fw = load_frag(reinterpret_cast<const u16*>(lw + r * kRow + (q ^ (r & 7))));
-#pragma unroll
-        for (int i = 0; i < kTm; ++i) acc[j][i] = mma(fw, fa[i], acc[j][i]);
-      }
-    }
-    buf = buf + 1 == STAGES ? 0 : buf + 1;
-  }
-  __syncthreads();
-  finish_tile<T, BM, BN>(g, group, m0, n0, N, lds, acc);
-}
 
 __device__ __forceinline__ float pf_block_sum(float v, float* scratch) {
   v = wave_sum(v);

@@ -1,0 +1,63 @@
+"""The prefill's matrix products over the sizes at which their tiles change (csrc/qmk_hybrid_gemm.h, ``choose_tiles``): one
+layer of each mixer at a width where every kind of tile is taken, cut along K or not, against the plain implementation in 64 bits.
+
+Tolerances as in test_gpu_hybrid.py: fp32 at rounding level, bf16 at bf16's."""
+import functools
+
+import pytest
+import torch
+
+import hybrid_oracle as O
+from qimeng_megakernel_amd import decode_hybrid, synthetic
+from qimeng_megakernel_amd.decode_schedule_hybrid import mk_kernel, weights
+from qimeng_megakernel_amd.decode_schedule_hybrid.globs import build_globals
+from qimeng_megakernel_amd.decode_schedule_hybrid.state import RequestTable
+
+pytestmark = pytest.mark.gpu
+
+DEVICE = "cuda:0"
+TOL = {torch.float32: 2e-5, torch.bfloat16: 4e-2}
+MOST = 1540
+#: feed-forwards of a size that fills the large tiles, and of one no tile divides
+SHAPES = {
+    "large": synthetic.hybrid_shape("a", width=2048, vocab=640, streams=2, ff={"a": 4096}, heads=8, dim=128, rot_dim=64, v_dim=128, rank=256, window=512),
+    "ragged": synthetic.hybrid_shape("a", width=1104, vocab=336, streams=3, ff={"a": 1744}, heads=3, dim=80, rot_dim=32, v_dim=112, rank=144, window=77),
+}
+
+
+@functools.lru_cache(maxsize=None)
+def expected(name):
+    shape = SHAPES[name]
+    w = synthetic.random_hybrid_weights(shape, 3, DEVICE)
+    tokens = torch.randint(0, shape.vocab, (MOST,), generator=torch.Generator().manual_seed(5))
+    with torch.device(DEVICE):
+        return w, tokens, O.forward(shape.to_config(), w, tokens.to(DEVICE), dtype=torch.float64)     # causal: a prefix's logits are its rows
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("n", [2, 16, 63, 65, 129, 200, 520, 1024, MOST])
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_products_at_the_edges_of_tiles(name, n, dtype):
+    shape = SHAPES[name]
+    w, tokens, want = expected(name)
+    g = build_globals(shape, weights.pack(shape, w, DEVICE), dtype=dtype, max_positions=MOST, portion_rows=MOST)
+    got = decode_hybrid.run_tokens(g, mk_kernel.get_mk(), RequestTable(g).open(0), tokens[:n], range(n)).double()
+    d = got - want[:n]
+    d = d - d.mean(-1, keepdim=True)
+    err = float((d.pow(2).mean(-1).sqrt() / want[:n].pow(2).mean().sqrt()).max())
+    assert err < TOL[dtype], f"{err:.3g}"
+
+
+def test_values_that_are_not_finite_stay_so_in_fp32():
+    """An infinite or undefined embedding reaches the logits of its token as such, and none of a token before it.  (A
+    recurrence: an attention's weight of zero times an undefined value is undefined.)"""
+    shape = synthetic.hybrid_shape("r", width=208, vocab=96, streams=2, ff={"r": 176}, lru_width=160, blocks=1, taps=3)
+    w = synthetic.random_hybrid_weights(shape, 6, DEVICE)
+    w["embed"][7, 3] = float("inf")
+    w["embed"][8, 5] = float("nan")
+    ids = torch.arange(40) % 6
+    ids[20], ids[30] = 7, 8
+    g = build_globals(shape, weights.pack(shape, w, DEVICE), dtype=torch.float32, max_positions=64, portion_rows=64)
+    got = decode_hybrid.run_tokens(g, mk_kernel.get_mk(), RequestTable(g).open(0), ids, range(40))
+    assert torch.isfinite(got[:20]).all()
+    assert not torch.isfinite(got[20]).any() and not torch.isfinite(got[30]).any()
