@@ -500,6 +500,80 @@ __device__ __forceinline__ void merge_partials(const Params& p, int head0, int n
   }
 }
 
+// Four neighbouring dims of one head, `item` of NQ * D / 4, over the slices of the context: running maximum, weights and sums in
+// the log2 domain.
+struct SliceMerge {
+  const float *lse, *part;
+  float mx, den, n0, n1, n2, n3;
+
+  template <class M>
+  __device__ __forceinline__ void start(const Params& p, int item) {
+    const int h = item / (M::D / 4), d0 = 4 * (item % (M::D / 4));
+    lse = p.attn_lse + static_cast<size_t>(h) * p.max_splits;
+    part = p.attn_partial + static_cast<size_t>(h) * p.max_splits * M::D + d0;
+    mx = -INFINITY;
+    den = n0 = n1 = n2 = n3 = 0.f;
+  }
+  __device__ __forceinline__ void add(const float (&e)[4], const v4u (&o)[4]) {
+    float mn = mx;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) mn = fmaxf(mn, e[q]);
+    const float rescale = (mx == -INFINITY) ? 0.f : exp2_fast(mx - mn);
+    den *= rescale; n0 *= rescale; n1 *= rescale; n2 *= rescale; n3 *= rescale;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float f = (e[q] == -INFINITY) ? 0.f : exp2_fast(e[q] - mn);
+      den += f;
+      n0 = __builtin_fmaf(__uint_as_float(o[q].x), f, n0);
+      n1 = __builtin_fmaf(__uint_as_float(o[q].y), f, n1);
+      n2 = __builtin_fmaf(__uint_as_float(o[q].z), f, n2);
+      n3 = __builtin_fmaf(__uint_as_float(o[q].w), f, n3);
+    }
+    mx = mn;
+  }
+  __device__ __forceinline__ uint2 result() const {
+    const float inv = den > 0.f ? 1.0f / den : 0.f;
+    return make_uint2(f2bf2(n0 * inv, n1 * inv), f2bf2(n2 * inv, n3 * inv));
+  }
+};
+
+// P slices into `m`, four at a time; FOURS fours are asked for together (one trip to memory), all loads first.
+template <class M, int ITEMS, int FOURS>
+__device__ __forceinline__ void merge_slices(SliceMerge (&m)[ITEMS], int P) {
+  for (int j0 = 0; j0 < P; j0 += 4 * FOURS) {
+    float e[ITEMS][FOURS][4];
+    v4u o[ITEMS][FOURS][4];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+#pragma unroll
+      for (int f = 0; f < FOURS; ++f)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int i = j0 + 4 * f + q, j = min(i, P - 1);
+          e[k][f][q] = i < P ? ld_shared_f32(m[k].lse + j) : -INFINITY;
+          o[k][f][q] = ld_shared128(m[k].part + static_cast<size_t>(j) * M::D);
+        }
+#pragma unroll
+    for (int f = 0; f < FOURS; ++f)
+      if (f == 0 || j0 + 4 * f < P)
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) m[k].add(e[k][f], o[k][f]);
+  }
+}
+
+// Slices per KV head up to which every O-projection workgroup of a tagged launch merges all heads for itself (merge mode 2).
+// It spares a hand-over, but reads NQ * P * D floats in each of 256 workgroups, P / 4 trips to memory one after the other: at
+// 32 slices of the Llama shape 262 KB a workgroup, 67 MB a layer.  Beyond it the slice that arrives last on a KV head merges that
+// head's group, with the same operations in the same order, sixteen slices a trip, and the O-projection reads the finished 4 KB.
+// Step time (us) by merging everywhere -> in the last slice: Llama shape 7 slices (context 2048) 542 -> 541, 10 (3000) 562 -> 546,
+// 32 (8192) 673 -> 616, 32 (16384) 754 -> 684; Qwen3-1.7B shape 12 (900) 849 -> 844, 32 (8000) 1393 -> 1218.  Up to four are one trip
+// either way.
+constexpr int kMostSelfMerged = 4;
+template <class M>
+__device__ __forceinline__ bool last_slice_merges(const Params& p, int P) {
+  return (std::is_same_v<M, Llama1B> || std::is_same_v<M, Qwen3_1p7B>) && P > kMostSelfMerged && tagged(p);
+}
+
 // One role of the Qwen3 op set's attention prologue, run by one wave on the staged vectors (`words`: q heads
 // from 0, then the new K row, then the new V row; lane l owns the rotation pair (2l, 2l+1)).  Roles 0..GQA-1:
 // a query head; GQA: the K row — per-head RMSNorm, n = bf16(w * (x * rsqrt(mean(x^2) + eps))) in fp32 with one
@@ -899,13 +973,32 @@ __device__ bool op_attn_splitkv(const Params& p, Smem<M>& s, const Ctx& c) {
   __syncthreads();
   QMK_STAMP(3);  // stores acknowledged
   if (merge_mode == 2) {  // one arrival per partial on the attention -> O-proj edge
+    int arrivals = 1;
+    if (__builtin_expect(last_slice_merges<M>(p, P), 0)) {     // ... or all of a KV head's at once, by whoever sees P - 1 earlier ones
+      if (c.tid == 0)
+        s.ctl[3] = __hip_atomic_fetch_add(counter_ptr(p, layer, ROW_SPLITKV, kvh * GQA), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == P - 1;
+      __syncthreads();
+      if (!s.ctl[3]) return true;
+      constexpr int kGroup = GQA * D / 4;
+      if (c.tid < kGroup) {
+        SliceMerge m[1];
+        m[0].template start<M>(p, kvh * kGroup + c.tid);
+        merge_slices<M, 1, 4>(m, P);
+        const uint2 o = m[0].result();
+        st_shared32(p.attn_out + (kvh * kGroup + c.tid) * 4, o.x);
+        st_shared32(p.attn_out + (kvh * kGroup + c.tid) * 4 + 2, o.y);
+      }
+      release_stores();
+      __syncthreads();
+      arrivals = P;
+    }
     // (an arrival on every XCD's line where the launch has such lines: Llama shape 1 911 -> 1 931 tok/s)
     if (xcd_counters(p)) {
-      if (c.tid < kXcds) publish(sub_counter(p, layer, ROW_REDUCE, c.tid), 1);
+      if (c.tid < kXcds) publish(sub_counter(p, layer, ROW_REDUCE, c.tid), arrivals);
     } else if (p.flags & kFlagAttentionRows2To5) {
-      if (c.tid < kXcds) publish(counter_ptr(p, layer, ROW_REDUCE, c.tid * kLineInts), 1);
+      if (c.tid < kXcds) publish(counter_ptr(p, layer, ROW_REDUCE, c.tid * kLineInts), arrivals);
     } else if (c.tid == 0) {
-      publish(counter_ptr(p, layer, ROW_REDUCE, 0), 1);
+      publish(counter_ptr(p, layer, ROW_REDUCE, 0), arrivals);
     }
     return true;
   }
@@ -1052,8 +1145,13 @@ __device__ bool op_oproj_residual(const Params& p, Smem<M>& s, const Ctx& c, Car
   parked = parked && carried && M::PARK_ROWS > 0;
   if (parked) park_upgate_rows<M>(p, s, s.next, layer, lane, c.tid >> 6);
   const int self_merge = s.inst[5];  // reduction_block_idx: 0, or the split-KV fan-out P when this op merges
-  if (self_merge == 0) {
-    if (!wg_wait(p, s, c, 1, [&](int) { return counter_ptr(p, layer, ROW_REDUCE, 0); }, M::NQ)) return false;
+  const bool merged = self_merge > 0 && self_merge <= kMaxSelfMerge && last_slice_merges<M>(p, self_merge);
+  if (__builtin_expect(self_merge == 0 || merged, 0)) {
+    if (merged) {
+      if (!wg_wait_all(p, s, c, layer, ROW_REDUCE, 0, M::NKV * self_merge)) return false;
+    } else if (!wg_wait(p, s, c, 1, [&](int) { return counter_ptr(p, layer, ROW_REDUCE, 0); }, M::NQ)) {
+      return false;
+    }
 #pragma unroll
     for (int k = 0; k < AW / (kThreads * 4); ++k)
       *reinterpret_cast<uint64_t*>(s.x + (c.tid + k * kThreads) * 4) = ld_shared64(p.attn_out + (c.tid + k * kThreads) * 4);
@@ -1061,62 +1159,22 @@ __device__ bool op_oproj_residual(const Params& p, Smem<M>& s, const Ctx& c, Car
     // Every O-proj workgroup merges the split-KV partials itself (python_vm.py:439-488 for all heads):
     // no merging workgroup, no attn_out round trip, one synchronisation hop less.  Item t (one or two
     // per thread) is dims 4*(t % (D/4)).. of head t / (D/4).
-    const int P = self_merge;
+    const int P = self_merge;   // no more than kMostSelfMerged of them in a tagged launch
     if (P < 1 || P > kMaxSelfMerge || P > p.max_splits) return bad_operand(p, s, c, 5);  // no list to fit: any fan-out the workspaces hold
     if (!wg_wait_all(p, s, c, layer, ROW_REDUCE, 0, M::NKV * P)) return false;
     constexpr int kItems = AW / (kThreads * 4);
-    const float* lse[kItems];
-    const float* part[kItems];
-    float mx[kItems], den[kItems], n0[kItems], n1[kItems], n2[kItems], n3[kItems];
+    SliceMerge m[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) m[k].template start<M>(p, c.tid + k * kThreads);
+    merge_slices<M, kItems, 1>(m, P);
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
       const int item = c.tid + k * kThreads;
-      const int h = item / (M::D / 4), d0 = 4 * (item % (M::D / 4));
-      lse[k] = p.attn_lse + static_cast<size_t>(h) * p.max_splits;
-      part[k] = p.attn_partial + static_cast<size_t>(h) * p.max_splits * M::D + d0;
-      mx[k] = -INFINITY;
-      den[k] = n0[k] = n1[k] = n2[k] = n3[k] = 0.f;
-    }
-    for (int j0 = 0; j0 < P; j0 += 4) {   // four partials of every item per round, all loads first
-      float e[kItems][4];
-      v4u o[kItems][4];
-#pragma unroll
-      for (int k = 0; k < kItems; ++k)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int j = min(j0 + q, P - 1);
-          e[k][q] = (j0 + q < P) ? ld_shared_f32(lse[k] + j) : -INFINITY;
-          o[k][q] = ld_shared128(part[k] + static_cast<size_t>(j) * M::D);
-        }
-#pragma unroll
-      for (int k = 0; k < kItems; ++k) {
-        float mn = mx[k];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) mn = fmaxf(mn, e[k][q]);
-        const float rescale = (mx[k] == -INFINITY) ? 0.f : exp2_fast(mx[k] - mn);
-        den[k] *= rescale; n0[k] *= rescale; n1[k] *= rescale; n2[k] *= rescale; n3[k] *= rescale;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float f = (e[k][q] == -INFINITY) ? 0.f : exp2_fast(e[k][q] - mn);
-          den[k] += f;
-          n0[k] = __builtin_fmaf(__uint_as_float(o[k][q].x), f, n0[k]);
-          n1[k] = __builtin_fmaf(__uint_as_float(o[k][q].y), f, n1[k]);
-          n2[k] = __builtin_fmaf(__uint_as_float(o[k][q].z), f, n2[k]);
-          n3[k] = __builtin_fmaf(__uint_as_float(o[k][q].w), f, n3[k]);
-        }
-        mx[k] = mn;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-      const int item = c.tid + k * kThreads;
-      const float inv = den[k] > 0.f ? 1.0f / den[k] : 0.f;
-      const uint32_t lo = f2bf2(n0[k] * inv, n1[k] * inv);
-      const uint32_t hi = f2bf2(n2[k] * inv, n3[k] * inv);
-      *reinterpret_cast<uint2*>(s.x + item * 4) = make_uint2(lo, hi);
+      const uint2 o = m[k].result();
+      *reinterpret_cast<uint2*>(s.x + item * 4) = o;
       if (nstart == 0) {  // one workgroup also leaves attn_out in memory, as the reference does
-        st_shared32(p.attn_out + item * 4, lo);
-        st_shared32(p.attn_out + item * 4 + 2, hi);
+        st_shared32(p.attn_out + item * 4, o.x);
+        st_shared32(p.attn_out + item * 4 + 2, o.y);
       }
     }
   }
