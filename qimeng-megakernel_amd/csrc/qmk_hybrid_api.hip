@@ -492,11 +492,12 @@ inline TileChoice choose_tiles(int M, int N, int K, int groups) {
 }
 
 // The same for products with an fp32 side, or of columns that are no multiple of 64: tiles of 64 x 64 cut along K until they
-// fill the chip four times over, of 128 x 128 where a part of them fills it already.
+// fill the chip four times over, of 128 x 128 where there are tokens for them and they fill it already (us, 64 -> 128: 1 x 65536 x 2048
+// 94 -> 150, 200 x 12288 x 2048 62 -> 76, 2048 x 16384 x 2048 829 -> 589).
 inline TileChoice choose_register_tiles(int M, int N, int K, int groups) {
   TileChoice c;
   const long long large = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128) * groups, small = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) * groups;
-  if (large >= 256) {
+  if (M >= 512 && large >= 256) {
     c.kind = 1;
     return c;
   }
