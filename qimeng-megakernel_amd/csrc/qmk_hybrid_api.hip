@@ -454,20 +454,24 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
 // `each` for every part.  All figures measured with weights that come from memory (us, M x N x K, the kernels this replaced ->
 // now): 2048 x 16384 x 2048 160 -> 138, 1531 x 16384 x 2048 115 -> 113, 2048 x 6144 x 2048 77 -> 64, 1531 x 5696 x 2048 63 -> 54,
 // 2048 x 2048 x 8192 107 -> 75, 1531 x 2048 x 8192 with the residual's streams 141 -> 83, 1531 x 2048 x 2048 with them 71 -> 41,
-// 512 x 2048 x 8192 73 -> 37, 43 x 2048 x 6144 38 -> 15, 43 x 12288 x 2048 23 -> 13.
+// 512 x 2048 x 8192 73 -> 37.  Up to 64 tokens a product is a stream of weights, and narrow tiles put more workgroups on it and
+// leave less to add up: 43 x 2048 x 6144 with the streams 38 -> 20 on 64 rows of weights -> 14 on 16, 43 x 2048 x 2048 with them
+// 21 -> 16 -> 10, 43 x 12288 x 2048 23 -> 13.5 -> 13 on 32.
 struct TileCost {
-  int bm, bn, slots;
+  int most_tokens, bm, bn, slots;
   double step, fixed, overlapped, meet, each;
 };
-constexpr int kTileKinds = 7;
+constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 9;
 constexpr TileCost kTileCosts[kTileKinds] = {
-    {64, 64, 256, 9.0, 0.0, 5.0, 1.0, 0.6},     // Tiles64
-    {128, 128, 512, 36.0, 8.0, 0.0, 0.0, 0.0},  // Tiles128
-    {64, 128, 256, 12.0, 6.5, 0.0, 3.0, 1.5},   // Turns64
-    {96, 128, 256, 14.5, 6.5, 0.0, 3.0, 1.5},   // Turns96
-    {128, 128, 256, 17.0, 9.0, 0.0, 3.0, 2.0},  // Turns128
-    {192, 256, 256, 47.0, 10.0, 0.0, 0.0, 0.0},  // Turns192
-    {256, 256, 256, 60.0, 9.0, 0.0, 0.0, 0.0},   // Turns256
+    {kAnyTokens, 64, 64, 256, 9.0, 0.0, 5.0, 1.0, 0.6},      // Tiles64
+    {kAnyTokens, 128, 128, 512, 36.0, 8.0, 0.0, 0.0, 0.0},   // Tiles128
+    {kAnyTokens, 64, 128, 256, 12.0, 6.5, 0.0, 3.0, 1.5},    // Turns64
+    {kAnyTokens, 96, 128, 256, 14.5, 6.5, 0.0, 3.0, 1.5},    // Turns96
+    {kAnyTokens, 128, 128, 256, 17.0, 9.0, 0.0, 3.0, 2.0},   // Turns128
+    {kAnyTokens, 192, 256, 256, 47.0, 10.0, 0.0, 0.0, 0.0},  // Turns192
+    {kAnyTokens, 256, 256, 256, 60.0, 9.0, 0.0, 0.0, 0.0},   // Turns256
+    {64, 64, 32, 512, 6.5, 0.0, 4.5, 0.5, 0.35},             // Tiles32
+    {64, 64, 16, 512, 6.5, 0.0, 4.0, 0.5, 0.3},              // Tiles16
 };
 struct TileChoice {
   int kind = 0, splits = 1;
@@ -477,6 +481,7 @@ inline TileChoice choose_tiles(int M, int N, int K, int groups) {
   double least = 0.;
   for (int kind = 0; kind < kTileKinds; ++kind) {
     const TileCost& t = kTileCosts[kind];
+    if (M > t.most_tokens) continue;
     const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * groups;
     for (int splits = 1; splits <= 8; splits *= 2) {
       if (splits > 1 && (t.each == 0. || K / splits < 256 || tiles > kMaxTickets || tiles * splits * t.bm * t.bn / 4 > kPartialUnits)) break;
@@ -526,7 +531,9 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
         case 3: turns(Turns96{}); break;
         case 4: turns(Turns128{}); break;
         case 5: turns(Turns192{}); break;
-        default: turns(Turns256{}); break;
+        case 6: turns(Turns256{}); break;
+        case 7: direct(Tiles32{}); break;
+        default: direct(Tiles16{}); break;
       }
       return;
     }

@@ -386,7 +386,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
 #pragma unroll
       for (int j = 0; j < S::kKept; ++j) {
         const int r = wm * kPassM + i * 16 + (lane & 15), quad = wn * (S::WN / 4) + (kg * S::kKept + j) * 4 + (lane >> 4);
-        out[r * kQuads + (quad ^ (r & 15))] = sums[j * kTm + pass * (kTm / S::kPasses) + i];
+        out[r * kQuads + (quad ^ (r & (kQuads - 1) & 15))] = sums[j * kTm + pass * (kTm / S::kPasses) + i];
       }
     __syncthreads();
     auto at = [&](int id, int& m, int& n) {
@@ -397,7 +397,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
     };
     auto value = [&](int id) {
       const int r = id / kQuads;
-      return out[r * kQuads + (id % kQuads ^ (r & 15))];
+      return out[r * kQuads + (id % kQuads ^ (r & (kQuads - 1) & 15))];
     };
     if (g.epi == EPI_RESIDUAL) {
       residual_quads(g, tid, kRows * kQuads, S::kThreadCount, at, value);
@@ -760,6 +760,8 @@ __global__ __launch_bounds__(kPfThreads) void gemm_short(const GemmArgs g) {
 }
 
 // ---- which tiles ----
+using Tiles16 = Tile<64, 16, 64, 16, 16, 4, 4>;        // few tokens: weight rows of a workgroup
+using Tiles32 = Tile<64, 32, 64, 32, 16, 4, 4>;
 using Tiles64 = Tile<64, 64, 64, 32, 32, 4, 4>;
 using Tiles128 = Tile<128, 128, 64, 64, 64, 4, 2>;
 using Turns64 = Tile<64, 128, 64, 32, 64, 8, 4>;
