@@ -659,12 +659,14 @@ int prefill(const QmkHybridArgs* a) {
 template <bool DELTA>
 void run_chunks(const QmkHybridArgs* a, const ChunkArgs& g, hipStream_t st) {
   const QmkHybridLayer& l = g.layer;
-  const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens, tiles = wave_tiles(l.head_dim);
+  const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens, waves = scan_waves(l.head_dim, DELTA);
   hipLaunchKernelGGL(chunk_prepare<DELTA>, dim3(chunks, l.heads), dim3(kPfThreads), 0, st, g);
-  const dim3 grid(l.heads, l.v_dim / 16), block(kChunkWaves * 64);
-  if (tiles == 1) hipLaunchKernelGGL((chunk_scan<1, DELTA>), grid, block, 0, st, g);
-  else if (tiles == 2) hipLaunchKernelGGL((chunk_scan<2, DELTA>), grid, block, 0, st, g);
-  else hipLaunchKernelGGL((chunk_scan<4, DELTA>), grid, block, 0, st, g);
+  const dim3 grid(l.heads, l.v_dim / 16), block(waves * 64);
+  switch (chunk_tiles(l.head_dim)) {
+    case 4: hipLaunchKernelGGL((chunk_scan<1, 4, DELTA>), grid, block, 0, st, g); break;
+    case 8: hipLaunchKernelGGL((chunk_scan<8 / scan_waves(128, DELTA), scan_waves(128, DELTA), DELTA>), grid, block, 0, st, g); break;
+    default: hipLaunchKernelGGL((chunk_scan<16 / scan_waves(256, DELTA), scan_waves(256, DELTA), DELTA>), grid, block, 0, st, g); break;
+  }
 }
 
 template <class T>

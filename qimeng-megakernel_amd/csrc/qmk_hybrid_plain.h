@@ -124,11 +124,11 @@ __global__ __launch_bounds__(kPfThreads) void transpose_values(const T* cache, i
 }
 
 constexpr int kChunkTokens = 16;
-constexpr int kChunkWaves = 4;
+constexpr int kChunkWaves = 4;      // of chunk_prepare
 
-// Tiles of sixteen key channels a wave of chunk_scan holds, and those of a head, the last ones zeros.
-__host__ __device__ constexpr int wave_tiles(int head_dim) { return head_dim <= 64 ? 1 : head_dim <= 128 ? 2 : 4; }
-__host__ __device__ constexpr int chunk_tiles(int head_dim) { return wave_tiles(head_dim) * kChunkWaves; }
+// Tiles of sixteen key channels of a head, the last ones zeros, and the waves of chunk_scan that share them.
+__host__ __device__ constexpr int chunk_tiles(int head_dim) { return head_dim <= 64 ? 4 : head_dim <= 128 ? 8 : 16; }
+__host__ __device__ constexpr int scan_waves(int head_dim, bool delta) { return head_dim <= 64 || delta ? 4 : 8; }
 // Floats of one (chunk, head): per tile the fragments of G q, G k and D k and the decays G over the whole chunk, then B and
 // T.  A fragment is in the order the matrix instruction takes it: [lane][4].
 __host__ __device__ constexpr int chunk_floats(int head_dim) { return chunk_tiles(head_dim) * (3 * 256 + 16) + 2 * 256; }
@@ -328,20 +328,28 @@ __global__ __launch_bounds__(kPfThreads) void keep_inputs(const float* x, QmkHyb
 // tile's last product and the first use of its result on the path that skips the next tile.  Loads have no branches either,
 // so that kAhead chunks are in flight: a chunk, or token, behind the last one is the last one again, and its value is either
 // not used or multiplied by zero.
-template <int TILES, bool DELTA>
-__global__ __launch_bounds__(kChunkWaves * 64) void chunk_scan(const ChunkArgs g) {
+// What bounds it is the chain of a chunk: products of the state with the keys (four dependent instructions of 32 cycles a tile), the
+// waves' sums through LDS, T (v - X), the state's update.  So the waves hold one tile each where a head has no more than
+// eight, and what only the output needs is off the chain: G q S is taken while the sums are on their way, and a chunk's outputs
+// are added up and stored behind the next chunk's barrier.
+template <int TILES, int WAVES, bool DELTA>
+__global__ __launch_bounds__(WAVES * 64) void chunk_scan(const ChunkArgs g) {
   constexpr int kAhead = TILES <= 2 ? 4 : 2;      // chunks in flight
-  __shared__ f32x4 px[2][kChunkWaves][64], po[2][kChunkWaves][64];
+  __shared__ f32x4 px[2][WAVES][64], po[2][WAVES][64];
   const QmkHybridLayer& l = g.layer;
   const int dim = l.head_dim, n = l.v_dim, head = blockIdx.x, v0 = blockIdx.y * 16;
-  constexpr int tiles = TILES * kChunkWaves;
+  constexpr int tiles = TILES * WAVES;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, quad = lane >> 4;
   const int tile0 = wave * TILES, mine = min(max(dim / 16 - tile0, 0), TILES);
   const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens;
   const size_t step = static_cast<size_t>(l.heads) * chunk_floats(dim);
   const float* rec = g.chunks + static_cast<size_t>(head) * chunk_floats(dim);
   float* state = l.state + (static_cast<size_t>(g.slot) * l.heads + head) * dim * n + v0 + col;
-  const float* values = g.values + g.value_at + head * n + v0 + col;
+  // Values: one base per chunk for the whole wave, four fixed offsets per lane, cut off at the portion's last token.
+  const float* values = g.values + g.value_at + head * n + v0;
+  uint32_t value_at[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) value_at[i] = (quad * 4 + i) * g.value_ld + col;
   f32x4 s[TILES];
 #pragma unroll
   for (int j = 0; j < TILES; ++j)
@@ -364,44 +372,51 @@ __global__ __launch_bounds__(kChunkWaves * 64) void chunk_scan(const ChunkArgs g
     }
     f.b = read4(r + tiles * 784 + lane * 4);
     if constexpr (DELTA) f.t = read4(r + tiles * 784 + 256 + lane * 4);
+    const float* v = values + static_cast<size_t>(chunk) * kChunkTokens * g.value_ld;
+    const uint32_t most = min(g.M - 1 - chunk * kChunkTokens, kChunkTokens - 1) * g.value_ld + col;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) f.v[i] = values[static_cast<size_t>(min(chunk * kChunkTokens + quad * 4 + i, g.M - 1)) * g.value_ld];
+    for (int i = 0; i < 4; ++i) f.v[i] = v[min(value_at[i], most)];
   };
   auto product = [](f32x4 a, f32x4 b, f32x4 c) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
     return c;
   };
+  f32x4 inner = {};       // B u of the last chunk whose outputs are this wave's
+  auto outputs = [&](int chunk) {
+    if (chunk < 0 || wave != (chunk & (WAVES - 1))) return;
+    f32x4 o = inner;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) o += po[chunk & 1][w][lane];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = chunk * kChunkTokens + quad * 4 + i;
+      if (m < g.M) g.out[static_cast<size_t>(m) * l.heads * n + head * n + v0 + col] = o[i];
+    }
+  };
   auto advance = [&](const Fragments& f, int chunk) {
     const int buf = chunk & 1;
-    f32x4 x = {}, o = {};
     if constexpr (DELTA) {
+      f32x4 x = {};
 #pragma unroll
       for (int j = 0; j < TILES; ++j) x = product(f.k[j], s[j], x);
       px[buf][wave][lane] = x;
     }
-#pragma unroll
-    for (int j = 0; j < TILES; ++j) o = product(f.q[j], s[j], o);
-    po[buf][wave][lane] = o;
-    __syncthreads();
+    __syncthreads();      // everybody's X; the chunk before's G q S
     f32x4 u = f.v;
     if constexpr (DELTA) {
 #pragma unroll
-      for (int w = 0; w < kChunkWaves; ++w) u -= px[buf][w][lane];
-      u = product(f.t, u, f32x4{0.f, 0.f, 0.f, 0.f});
+      for (int w = 0; w < WAVES; ++w) u -= px[buf][w][lane];
     }
+    f32x4 o = {};
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) o = product(f.q[j], s[j], o);
+    po[buf][wave][lane] = o;
+    if constexpr (DELTA) u = product(f.t, u, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
     for (int j = 0; j < TILES; ++j) s[j] = product(f.d[j], u, s[j] * f.g[j]);
-    if (wave == (chunk & (kChunkWaves - 1))) {
-      o = product(f.b, u, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-      for (int w = 0; w < kChunkWaves; ++w) o += po[buf][w][lane];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = chunk * kChunkTokens + quad * 4 + i;
-        if (m < g.M) g.out[static_cast<size_t>(m) * l.heads * n + head * n + v0 + col] = o[i];
-      }
-    }
+    outputs(chunk - 1);
+    if (wave == (chunk & (WAVES - 1))) inner = product(f.b, u, f32x4{0.f, 0.f, 0.f, 0.f});
   };
   Fragments f[kAhead];
 #pragma unroll
@@ -417,6 +432,8 @@ __global__ __launch_bounds__(kChunkWaves * 64) void chunk_scan(const ChunkArgs g
 #pragma unroll
   for (int a = 0; a < kAhead - 1; ++a)
     if (chunk + a < chunks) advance(f[a], chunk + a);
+  __syncthreads();
+  outputs(chunks - 1);
 #pragma unroll
   for (int j = 0; j < TILES; ++j)
     if (j < mine)
