@@ -556,7 +556,7 @@ template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, T* out,
                       hipStream_t st) {
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
+    hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * kAttendGroups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
   };
   if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4>);
   else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8>);

@@ -181,14 +181,25 @@ struct Keys {
 // Windowed attention over expanded keys: 64 queries of one head a workgroup (16 a wave), 32 keys a step.
 // Scores are computed transposed (keys x queries), so a lane holds eight weights of ONE query in exactly the shape the
 // value product's second operand wants, with keys in the order 4g..4g+3, 16+4g..16+4g+3.
+// Two groups of four waves take the 32-key steps in turn, for the same queries, and meet at the end: a step is a chain (keys into LDS,
+// scores, maximum over the lanes, weights, values), and a CU that holds one or two workgroups of four waves mostly waits for it
+// (us, one group -> two: 2048 queries of 16 heads of 128 behind 0 and 2048 keys, mean 156 -> 99; 1531 of 192 | 128 in a window of 1024
+// 70 -> 66; 43 behind 400 29 -> 19; 200 in fp32 34 -> 29.  Four groups: 121, 84, 24.)
+constexpr int kAttendGroups = 2;
 template <class T, int QT, int VT>   // most 32-column steps of a query, most 16-row tiles of a value
-__global__ __launch_bounds__(kPfThreads) void window_attention(const T* q, Keys<T> keys, const T* rows, const T* v_t, const T* gate, QmkHybridLayer l,
+__global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(const T* q, Keys<T> keys, const T* rows, const T* v_t, const T* gate, QmkHybridLayer l,
                                                                int first, int position, int M, int keys_cap, T* out) {
   constexpr int kKeys = 32;
   constexpr int kPadK = 16 / sizeof(T), kPadV = 16 / sizeof(T);
-  __shared__ __align__(16) T sk[kKeys][QT * 32 + kPadK];
-  __shared__ __align__(16) T sv[VT * 16][kKeys + kPadV];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, col = lane & 15;
+  struct Step {
+    T k[kKeys][QT * 32 + kPadK];
+    T v[VT * 16][kKeys + kPadV];
+  };
+  __shared__ __align__(16) Step stage[kAttendGroups];
+  const int tid = threadIdx.x % kPfThreads, lane = tid & 63, wave = tid >> 6, g = lane >> 4, col = lane & 15;
+  const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kPfThreads);
+  auto& sk = stage[part].k;
+  auto& sv = stage[part].v;
   // Later queries see more keys where no window ends.  Workgroups 256 apart share a CU: every other such run of heads takes
   // its queries from the far end, so that a CU gets long and short ones.
   const bool mirrored = (blockIdx.y * gridDim.x >> 8 & 1) == 0;
@@ -209,7 +220,7 @@ __global__ __launch_bounds__(kPfThreads) void window_attention(const T* q, Keys<
   // this one is used.
   constexpr int kKLoads = kKeys * QT * 32 / kU / kPfThreads, kVLoads = VT * 16 * kKeys / kU / kPfThreads;
   static_assert(kKLoads * kPfThreads * kU == kKeys * QT * 32 && kVLoads * kPfThreads * kU == VT * 16 * kKeys, "every thread stages the same number of units");
-  const int base0 = first + ((lo - first) & ~(kKeys - 1));
+  const int begin = first + ((lo - first) & ~(kKeys - 1)), base0 = begin + part * kKeys;
   const T* k_at[kKLoads];
   int k_step[kKLoads];
   v4u rk[kKLoads], rv[kVLoads];
@@ -220,10 +231,10 @@ __global__ __launch_bounds__(kPfThreads) void window_attention(const T* q, Keys<
     k_step[i] = 0;
     if (c < l.head_dim) {
       k_at[i] = keys.at + static_cast<size_t>(row) * keys.pitch + kv * keys.head + c;
-      k_step[i] = kKeys * keys.pitch;
+      k_step[i] = kAttendGroups * kKeys * keys.pitch;
     } else if (c < l.head_dim + l.rot_dim) {
       k_at[i] = rows + static_cast<size_t>(row) * width + l.rank + c - l.head_dim;
-      k_step[i] = kKeys * width;
+      k_step[i] = kAttendGroups * kKeys * width;
     }
   }
   auto fetch = [&](int base) {
@@ -249,7 +260,7 @@ __global__ __launch_bounds__(kPfThreads) void window_attention(const T* q, Keys<
   };
   fetch(base0);
   const int first_pos = position + q0 + wave * 16;       // this wave's queries: first_pos .. first_pos + 15
-  for (int base = base0; base < hi; base += kKeys) {
+  for (int base = base0; base - part * kKeys < hi; base += kAttendGroups * kKeys) {      // (the groups share the barriers)
 #pragma unroll
     for (int i = 0; i < kKLoads; ++i) {
       const int id = i * kPfThreads + tid;
@@ -261,57 +272,80 @@ __global__ __launch_bounds__(kPfThreads) void window_attention(const T* q, Keys<
       *reinterpret_cast<v4u*>(&sv[id / (kKeys / kU)][id % (kKeys / kU) * kU]) = rv[i];
     }
     __syncthreads();
-    if (base + kKeys < hi) fetch(base + kKeys);
-    f32x4 d[2] = {};
+    if (base + kAttendGroups * kKeys < hi) fetch(base + kAttendGroups * kKeys);
+    if (base < hi) {
+      f32x4 d[2] = {};
 #pragma unroll
-    for (int s = 0; s < QT; ++s)
-      if (s < steps) {
+      for (int s = 0; s < QT; ++s)
+        if (s < steps) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) d[t] = mma(load_frag(&sk[t * 16 + col][s * 32 + g * 8]), fq[s], d[t]);
+          for (int t = 0; t < 2; ++t) d[t] = mma(load_frag(&sk[t * 16 + col][s * 32 + g * 8]), fq[s], d[t]);
+        }
+      float w[8];
+      float best = top;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w[j] = d[j >> 2][j & 3] * scale;
+      if (base + kKeys - 1 > first_pos || first_pos + 15 - base >= l.window) {   // some query does not see some key
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int key = base + (j >> 2) * 16 + g * 4 + (j & 3), dist = pos - key;
+          if (dist < 0 || dist >= l.window) w[j] = -INFINITY;
+        }
       }
-    float w[8];
-    float best = top;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) w[j] = d[j >> 2][j & 3] * scale;
-    if (base + kKeys - 1 > first_pos || first_pos + 15 - base >= l.window) {   // some query does not see some key
+      for (int j = 0; j < 8; ++j) best = fmaxf(best, w[j]);
+      best = fmaxf(best, __shfl_xor(best, 16));
+      best = fmaxf(best, __shfl_xor(best, 32));
+      const float ref = best == -INFINITY ? 0.f : best;      // no key of this query yet
+      const float shrink = exp2_fast(top - ref);
+      float part = 0.f;
+      Frag<T> fp;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int key = base + (j >> 2) * 16 + g * 4 + (j & 3), dist = pos - key;
-        if (dist < 0 || dist >= l.window) w[j] = -INFINITY;
+        w[j] = exp2_fast(w[j] - ref);
+        part += w[j];
+        fp.set(j, from_f32<T>(w[j]));
       }
-    }
+      sum = sum * shrink + part;
+      top = best;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) best = fmaxf(best, w[j]);
-    best = fmaxf(best, __shfl_xor(best, 16));
-    best = fmaxf(best, __shfl_xor(best, 32));
-    const float ref = best == -INFINITY ? 0.f : best;      // no key of this query yet
-    const float shrink = exp2_fast(top - ref);
-    float part = 0.f;
-    Frag<T> fp;
+      for (int t = 0; t < VT; ++t)
+        if (t < vt) {
+          Frag<T> fv;
+          const T* r = &sv[t * 16 + col][0];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      w[j] = exp2_fast(w[j] - ref);
-      part += w[j];
-      fp.set(j, from_f32<T>(w[j]));
-    }
-    sum = sum * shrink + part;
-    top = best;
-#pragma unroll
-    for (int t = 0; t < VT; ++t)
-      if (t < vt) {
-        Frag<T> fv;
-        const T* r = &sv[t * 16 + col][0];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          fv.set(j, r[g * 4 + j]);
-          fv.set(4 + j, r[16 + g * 4 + j]);
+          for (int j = 0; j < 4; ++j) {
+            fv.set(j, r[g * 4 + j]);
+            fv.set(4 + j, r[16 + g * 4 + j]);
+          }
+          acc[t] = mma(fv, fp, acc[t] * shrink);
         }
-        acc[t] = mma(fv, fp, acc[t] * shrink);
-      }
+    }
     __syncthreads();
   }
   sum += __shfl_xor(sum, 16);
   sum += __shfl_xor(sum, 32);
+  // The second group's maximum, sum and values of every lane's query onto the first one's.
+  float* box = reinterpret_cast<float*>(stage) + tid;
+  static_assert(kAttendGroups == 2 && sizeof(stage) >= sizeof(float) * (VT * 4 + 2) * kPfThreads, "the giving group's states");
+  if (part == 1) {
+    box[0] = top;
+    box[kPfThreads] = sum;
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) box[(2 + t * 4 + i) * kPfThreads] = acc[t][i];
+  }
+  __syncthreads();
+  if (part == 1) return;
+  {
+    const float other = box[0], most = fmaxf(top, other), ref = most == -INFINITY ? 0.f : most, mine = exp2_fast(top - ref), theirs = exp2_fast(other - ref);
+    sum = sum * mine + box[kPfThreads] * theirs;
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[t][i] = acc[t][i] * mine + box[(2 + t * 4 + i) * kPfThreads] * theirs;
+  }
   if (m >= M) return;
   const float inv = 1.f / sum;
   const size_t at = static_cast<size_t>(m) * l.heads * l.v_dim + head * l.v_dim;
