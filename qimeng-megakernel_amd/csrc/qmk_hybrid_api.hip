@@ -335,11 +335,26 @@ inline SplitBuffers split_buffers(Carver& c) {
   return b;
 }
 
+// Rows that products read: `count` elements, in fp32 mode whole or as three bf16 parts.  They are in parts where the kernels that
+// stage tiles straight to LDS take their product: a multiple of 64 columns, and more than 64 (shorter products keep the fp32
+// instruction).  us, split by the workgroups that read them -> by the kernel that makes them: 200 x 2048 x 2048 and x 6144 with the
+// residual's streams 45 -> 36 on the average, 200 x 5696 x 2048 41 -> 33, five of 200 x 2048 x 2048 60 -> 36, 200 x 12288 x 2048 63 -> 63,
+// 1 x 151936 x 2048 429 -> 147; the kernels that make them take as long as before.
+template <class T>
+struct OperandRows {
+  T* at = nullptr;
+  size_t count = 0;
+  OperandRows() = default;
+  OperandRows(Carver& c, size_t n) : at(c.take<T>(sizeof(T) == 4 ? n / 2 * 3 : n)), count(n) {}
+  Operand<T> of(int columns) const { return Operand<T>{at, sizeof(T) == 4 && columns > 64 && columns % 64 == 0 ? count : 0}; }
+};
+
 template <class T>
 struct PlainBuffers {
   SplitBuffers split;
   float *x, *branch, *qkv, *values, *decay, *beta, *o, *chunks;
-  T *h, *q, *low, *gate, *mix, *vt;
+  T *q, *low, *gate, *vt;
+  OperandRows<T> h, mix;
 };
 template <class T>
 size_t plain_buffers(const QmkHybridArgs* a, void* base, PlainBuffers<T>* b) {
@@ -381,11 +396,11 @@ size_t plain_buffers(const QmkHybridArgs* a, void* base, PlainBuffers<T>* b) {
   b->beta = c.take<float>(beta);
   b->o = c.take<float>(o);
   b->chunks = c.take<float>(chunks);
-  b->h = c.take<T>(h);
+  b->h = OperandRows<T>(c, h);
   b->q = c.take<T>(q);
   b->low = c.take<T>(low);
   b->gate = c.take<T>(gate);
-  b->mix = c.take<T>(mix);
+  b->mix = OperandRows<T>(c, mix);
   b->vt = c.take<T>(vt);
   return c.used;
 }
@@ -396,7 +411,8 @@ template <class T>
 struct PrefillBuffers {
   SplitBuffers split;
   float *x, *u, *fa, *fb, *raw;
-  T *h, *p0, *p1, *p2, *mix, *rows, *kn, *vt;
+  T *p0, *p1, *p2, *rows, *kn, *vt;
+  OperandRows<T> h, mix;
 };
 template <class T>
 size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b) {
@@ -437,11 +453,11 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
   b->fa = c.take<float>(fa);
   b->fb = c.take<float>(fb);
   b->raw = c.take<float>(raw);
-  b->h = c.take<T>(h);
+  b->h = OperandRows<T>(c, h);
   b->p0 = c.take<T>(p0);
   b->p1 = c.take<T>(p1);
   b->p2 = c.take<T>(p2);
-  b->mix = c.take<T>(mix);
+  b->mix = OperandRows<T>(c, mix);
   b->rows = c.take<T>(rows);
   b->kn = c.take<T>(kn);
   b->vt = c.take<T>(vt);
@@ -510,6 +526,15 @@ inline TileChoice choose_register_tiles(int M, int N, int K, int groups) {
   return c;
 }
 
+// Products whose tokens' side is in parts, cut along K until every CU has a workgroup (us, in 1, 2, 4, 8: 200 x 2048 x 6144 75, 44, 32, 42;
+// 200 x 5696 x 2048, 315 tiles 31, 39, 42; 20 x 12288 x 2048 24, 19, 18, 25).
+inline int choose_part_splits(long long tiles, int K) {
+  int splits = 1;
+  while (splits < 8 && tiles * splits < 256 && K / splits >= 512) splits *= 2;
+  return splits;
+}
+static_assert(256LL * 2 * TilesParts::BM * TilesParts::BN / 4 <= kPartialUnits && 256 <= kMaxTickets, "room for what is cut along K");
+
 template <class TA, class TW, class T>
 void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   const int n = std::max(g.N, g.last_n);
@@ -538,6 +563,14 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
       return;
     }
   }
+  if constexpr (sizeof(TA) == 4 && sizeof(TW) == 2) {
+    if (g.a_part != 0) {
+      using S = TilesParts;
+      g.splits = choose_part_splits(static_cast<long long>((g.M + S::BM - 1) / S::BM) * ((n + S::BN - 1) / S::BN) * g.groups, g.K);
+      launch(gemm_direct<T, S, 3>, S::BM, S::BN, S::kThreadCount);
+      return;
+    }
+  }
   if constexpr (sizeof(TA) == 4 || sizeof(TW) == 4) {
     if (g.K <= 64) {
       g.splits = 1;
@@ -553,7 +586,7 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
 
 // rows: where the rotated part of a latent attention's keys is, behind the latent.
 template <class T>
-void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, T* out,
+void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
                       hipStream_t st) {
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * kAttendGroups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
@@ -576,14 +609,15 @@ int prefill(const QmkHybridArgs* a) {
   const int M = a->tokens, D = a->width, S = a->streams, P = a->portion_rows;
   const dim3 block(kPfThreads);
   hipLaunchKernelGGL(embed_tokens, dim3(M), block, 0, st, a->embed, a->token_in, a->vocab, a->layers[0].hc, S, D, b.x, b.u);
-  auto gemm_args = [&](const T* in, int lda, const u16* w, int N, int K, const QmkHybridLayer& l, int epi) {
+  auto gemm_args = [&](Operand<T> in, int lda, const u16* w, int N, int K, const QmkHybridLayer& l, int epi) {
     GemmArgs g{};
-    g.a = in; g.lda = lda; g.w = w; g.ldw = K; g.M = M; g.N = g.last_n = N; g.K = K; g.groups = 1;
+    g.a = in.at; g.a_part = in.part; g.lda = lda; g.w = w; g.ldw = K; g.M = M; g.N = g.last_n = N; g.K = K; g.groups = 1;
     g.layer = l; g.epi = epi; g.position = a->position; g.streams = S; g.width = D; g.rows_cap = P;
     return g;
   };
+  auto whole = [](T* rows) { return Operand<T>{rows, 0}; };
   auto residual = [&](const u16* w, int K, const QmkHybridLayer& l, bool down) {
-    GemmArgs g = gemm_args(b.mix, K, w, D, K, l, EPI_RESIDUAL);
+    GemmArgs g = gemm_args(b.mix.of(K), K, w, D, K, l, EPI_RESIDUAL);
     g.f0 = b.x; g.f1 = b.u; g.down = down; g.next = down ? l.next2 : l.next1;
     launch_gemm<T, u16, T>(g, b.split, st);
   };
@@ -591,40 +625,40 @@ int prefill(const QmkHybridArgs* a) {
     const QmkHybridLayer& l = a->layers[i];
     const int W = l.mix_width;
     if (l.type != QMK_MIXER_WKV)
-      hipLaunchKernelGGL(norm_rows<T>, dim3(M), block, 0, st, b.u, l.norm1, nullptr, M, D, a->width_true, a->eps, b.h);
+      hipLaunchKernelGGL(norm_rows<T>, dim3(M), block, 0, st, b.u, l.norm1, nullptr, M, D, a->width_true, a->eps, b.h.of(D));
     if (l.type == QMK_MIXER_RGLRU) {
-      GemmArgs g = gemm_args(b.h, D, l.in_w, l.in_rows, D, l, EPI_RGLRU_IN);
+      GemmArgs g = gemm_args(b.h.of(D), D, l.in_w, l.in_rows, D, l, EPI_RGLRU_IN);
       g.out = b.p0; g.out2 = b.p1;
       launch_gemm<T, u16, T>(g, b.split, st);
       const long long quads = static_cast<long long>(M) * (W / 4);
       hipLaunchKernelGGL(causal_conv<T>, dim3(static_cast<unsigned>((quads + kPfThreads - 1) / kPfThreads)), block, 0, st, b.p1, l, a->slot, a->flip, M, b.p2);
-      GemmArgs e = gemm_args(b.p2, W, l.mid_w, 2 * l.block_dim, l.block_dim, l, EPI_LRU_GATES);
+      GemmArgs e = gemm_args(whole(b.p2), W, l.mid_w, 2 * l.block_dim, l.block_dim, l, EPI_LRU_GATES);
       e.groups = l.blocks; e.a_step = l.block_dim; e.w_step = 2LL * l.block_dim * l.block_dim;
       e.src = b.p2; e.f0 = b.fa; e.f1 = b.fb;
       launch_gemm<T, u16, T>(e, b.split, st);
-      hipLaunchKernelGGL(lru_scan<T>, dim3(W / kScanChannels), dim3(kScanChannels * kScanRuns), 0, st, b.fa, b.fb, b.p0, l, a->slot, M, b.mix);
+      hipLaunchKernelGGL(lru_scan<T>, dim3(W / kScanChannels), dim3(kScanChannels * kScanRuns), 0, st, b.fa, b.fb, b.p0, l, a->slot, M, b.mix.of(W));
     } else if (l.type == QMK_MIXER_LATENT) {
-      GemmArgs g = gemm_args(b.h, D, l.in_w, l.in_rows, D, l, EPI_LATENT_IN);
+      GemmArgs g = gemm_args(b.h.of(D), D, l.in_w, l.in_rows, D, l, EPI_LATENT_IN);
       g.out = b.p0; g.out2 = b.p1; g.f0 = b.raw;
       launch_gemm<T, u16, T>(g, b.split, st);
       const int first = std::max(0, a->position + 1 - l.window), keys = a->position + M - first, cap = keys_cap(a, l), width = l.rank + l.rot_dim;
       hipLaunchKernelGGL(latent_rows<T>, dim3(keys), block, 0, st, b.raw, l, a->slot, first, a->position, a->eps, b.rows);
-      GemmArgs k = gemm_args(b.rows, width, l.uk_w, l.heads * l.head_dim, l.rank, l, EPI_STORE);
+      GemmArgs k = gemm_args(whole(b.rows), width, l.uk_w, l.heads * l.head_dim, l.rank, l, EPI_STORE);
       k.M = keys; k.out = b.kn; k.ldo = l.heads * l.head_dim;
       launch_gemm<T, u16, T>(k, b.split, st);
-      GemmArgs v = gemm_args(nullptr, l.rank, nullptr, keys, l.rank, l, EPI_STORE);   // transposed: W_uv rows x keys
+      GemmArgs v = gemm_args(whole(nullptr), l.rank, nullptr, keys, l.rank, l, EPI_STORE);   // transposed: W_uv rows x keys
       v.a = l.uv_w; v.w = b.rows; v.ldw = width; v.M = l.heads * l.v_dim; v.out = b.vt; v.ldo = cap;
       launch_gemm<u16, T, T>(v, b.split, st);
       const Keys<T> expanded{b.kn, l.heads * l.head_dim, l.head_dim, 1};
-      launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix, st);
+      launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), st);
     } else {
       const int N = W, n = l.head_dim;
-      hipLaunchKernelGGL(shift_mix<T>, dim3(M), block, 0, st, b.u, l, a->slot, a->flip, M, P, D, a->width_true, a->eps, b.h);
-      GemmArgs g = gemm_args(b.h, D, l.in_w, N, D, l, EPI_WKV_IN);
+      hipLaunchKernelGGL(shift_mix<T>, dim3(M), block, 0, st, b.u, l, a->slot, a->flip, M, P, D, a->width_true, a->eps, b.h.of(D));
+      GemmArgs g = gemm_args(b.h.of(D), D, l.in_w, N, D, l, EPI_WKV_IN);
       g.groups = 5; g.last_n = l.rank; g.a_step = static_cast<long long>(P) * D; g.w_step = static_cast<long long>(N) * D;
       g.f0 = b.fa; g.out = b.p0; g.out2 = b.p1;
       launch_gemm<T, u16, T>(g, b.split, st);
-      GemmArgs d = gemm_args(b.p1, l.rank, l.mid_w, N, l.rank, l, EPI_WKV_DECAY);
+      GemmArgs d = gemm_args(whole(b.p1), l.rank, l.mid_w, N, l.rank, l, EPI_WKV_DECAY);
       d.f0 = b.fb; d.ldo = N;
       launch_gemm<T, u16, T>(d, b.split, st);
       const size_t step = static_cast<size_t>(P) * N;
@@ -633,13 +667,13 @@ int prefill(const QmkHybridArgs* a) {
       if (n <= 64) hipLaunchKernelGGL((wkv_scan<4, 32>), grid, lanes, 0, st, r, k, v, b.fb, l, a->slot, M, b.raw);
       else if (n <= 128) hipLaunchKernelGGL((wkv_scan<8, 16>), grid, lanes, 0, st, r, k, v, b.fb, l, a->slot, M, b.raw);
       else hipLaunchKernelGGL((wkv_scan<16, 8>), grid, lanes, 0, st, r, k, v, b.fb, l, a->slot, M, b.raw);
-      hipLaunchKernelGGL(wkv_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.raw, b.p0, l, M, a->eps, b.mix);
+      hipLaunchKernelGGL(wkv_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.raw, b.p0, l, M, a->eps, b.mix.of(W));
     }
     residual(l.o_w, W, l, false);
     if (l.has_mlp) {
-      hipLaunchKernelGGL(norm_rows<T>, dim3(M), block, 0, st, b.u, l.norm2, nullptr, M, D, a->width_true, a->eps, b.h);
-      GemmArgs g = gemm_args(b.h, D, l.mlp_w, 2 * l.ff, D, l, EPI_GEGLU);
-      g.out = b.mix;
+      hipLaunchKernelGGL(norm_rows<T>, dim3(M), block, 0, st, b.u, l.norm2, nullptr, M, D, a->width_true, a->eps, b.h.of(D));
+      GemmArgs g = gemm_args(b.h.of(D), D, l.mlp_w, 2 * l.ff, D, l, EPI_GEGLU);
+      g.out = b.mix.at; g.out_part = b.mix.of(l.ff).part;
       launch_gemm<T, u16, T>(g, b.split, st);
       residual(l.down_w, l.ff, l, true);
     }
@@ -647,8 +681,8 @@ int prefill(const QmkHybridArgs* a) {
       hipLaunchKernelGGL(sum_streams, dim3(M), block, 0, st, b.x, S, D, a->layer_out + static_cast<size_t>(i) * M * D);
   }
   if (a->num_want > 0) {
-    hipLaunchKernelGGL(norm_rows<T>, dim3(a->num_want), block, 0, st, b.u, a->final_norm, a->want, M, D, a->width_true, a->eps, b.h);
-    GemmArgs g = gemm_args(b.h, D, a->head, a->vocab_rows, D, a->layers[0], EPI_LOGITS);
+    hipLaunchKernelGGL(norm_rows<T>, dim3(a->num_want), block, 0, st, b.u, a->final_norm, a->want, M, D, a->width_true, a->eps, b.h.of(D));
+    GemmArgs g = gemm_args(b.h.of(D), D, a->head, a->vocab_rows, D, a->layers[0], EPI_LOGITS);
     g.M = a->num_want; g.f0 = a->logits; g.ldo = a->vocab_rows;
     launch_gemm<T, u16, T>(g, b.split, st);
   }
@@ -677,13 +711,14 @@ int prefill_plain(const QmkHybridArgs* a) {
   const int M = a->tokens, D = a->width;
   const size_t rows = static_cast<size_t>(a->portion_rows) * D;
   const dim3 block(kPfThreads);
-  auto gemm_args = [&](const T* in, const u16* w, int N, int K, const QmkHybridLayer& l, int epi) {
+  auto gemm_args = [&](Operand<T> in, const u16* w, int N, int K, const QmkHybridLayer& l, int epi) {
     GemmArgs g{};
-    g.a = in; g.lda = K; g.w = w; g.ldw = K; g.M = M; g.N = g.last_n = N; g.K = K; g.groups = 1;
+    g.a = in.at; g.a_part = in.part; g.lda = K; g.w = w; g.ldw = K; g.M = M; g.N = g.last_n = N; g.K = K; g.groups = 1;
     g.layer = l; g.epi = epi; g.position = a->position; g.slot = a->slot; g.width = D; g.ldo = D;
     g.logit_scale = a->logit_scale; g.logit_softcap = a->logit_softcap;
     return g;
   };
+  auto whole = [](T* rows) { return Operand<T>{rows, 0}; };
   int runs_done = 0;
   // x as entry l reads it: its norm (or [x; embedding]) -> h; `want`: of those rows alone, x stays.
   auto residual = [&](const QmkHybridLayer& l, const int32_t* want, int count, bool added, float* dump) {
@@ -695,7 +730,7 @@ int prefill_plain(const QmkHybridArgs* a) {
       const QmkHybridLayer* before = a->layers + l.prev;
       g.a = b.branch; g.b = b.branch + rows; g.wa = before[0].out_norm; g.wb = before[1].out_norm; g.scale = before[0].out_scale;
     }
-    hipLaunchKernelGGL(residual_rows<T>, dim3(count), block, 0, st, g, b.h);
+    hipLaunchKernelGGL(residual_rows<T>, dim3(count), block, 0, st, g, b.h.of(l.type == QMK_ENTRY_JOIN ? 2 * D : D));
   };
   auto dump_of = [&](const QmkHybridLayer& l) {   // where the run before this entry is asked for
     return a->layer_out != nullptr && l.prev >= 0 ? a->layer_out + static_cast<size_t>(runs_done++) * M * D : nullptr;
@@ -708,7 +743,7 @@ int prefill_plain(const QmkHybridArgs* a) {
       if (dump != nullptr) residual(l, nullptr, M, true, dump);     // (and x is complete)
       if (a->num_want > 0) {
         residual(l, a->want, a->num_want, dump == nullptr, nullptr);
-        GemmArgs g = gemm_args(b.h, a->head, a->vocab_rows, D, l, EPI_CAPPED_LOGITS);
+        GemmArgs g = gemm_args(b.h.of(D), a->head, a->vocab_rows, D, l, EPI_CAPPED_LOGITS);
         g.M = a->num_want; g.f0 = a->logits; g.ldo = a->vocab_rows;
         launch_gemm<T, u16, T>(g, b.split, st);
       }
@@ -716,32 +751,32 @@ int prefill_plain(const QmkHybridArgs* a) {
     }
     if (l.branch == 0) residual(l, nullptr, M, true, dump_of(l));
     if (l.type == QMK_ENTRY_JOIN) {
-      GemmArgs g = gemm_args(b.h, l.in_w, D, 2 * D, l, EPI_LOGITS);
+      GemmArgs g = gemm_args(b.h.of(2 * D), l.in_w, D, 2 * D, l, EPI_LOGITS);
       g.f0 = b.x;
       launch_gemm<T, u16, T>(g, b.split, st);
       continue;
     }
     if (l.type == QMK_MIXER_ATTENTION) {
-      GemmArgs g = gemm_args(b.h, l.in_w, l.in_rows, D, l, EPI_ATTENTION_IN);
+      GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_ATTENTION_IN);
       g.out = b.q; g.out2 = b.gate;
       launch_gemm<T, u16, T>(g, b.split, st);
       const int row = l.head_dim + l.v_dim, pitch = l.kv_heads * row, keys = a->position + M, cap = static_cast<int>(values_cap(a));
       const T* cache = static_cast<const T*>(l.cache) + static_cast<size_t>(a->slot) * l.ring * pitch;
       hipLaunchKernelGGL(transpose_values<T>, dim3((keys + 63) / 64, (l.v_dim + 63) / 64, l.kv_heads), block, 0, st, cache, pitch, row, l.head_dim, l.v_dim, keys, cap, b.vt);
-      launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix, st);
+      launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix.of(W), st);
     } else {
       ChunkArgs c{};
       c.layer = l; c.decay = b.decay; c.chunks = b.chunks; c.out = b.o; c.M = M; c.slot = a->slot; c.flip = a->flip;
       if (l.type == QMK_MIXER_DELTA) {
         const int channels = conv_channels(l), ranks = l.rank + l.gate_rank, beta_ld = (l.heads + 15) / 16 * 16;
-        GemmArgs g = gemm_args(b.h, l.in_w, l.in_rows, D, l, EPI_DELTA_IN);
+        GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_DELTA_IN);
         g.f1 = b.qkv; g.out2 = b.low; g.f0 = b.beta; g.ldo = beta_ld;
         launch_gemm<T, u16, T>(g, b.split, st);
         const int keys = l.heads * l.head_dim;
-        GemmArgs e = gemm_args(b.low, l.mid_w, keys, l.rank, l, EPI_DELTA_DECAY);
+        GemmArgs e = gemm_args(whole(b.low), l.mid_w, keys, l.rank, l, EPI_DELTA_DECAY);
         e.lda = ranks; e.f0 = b.decay; e.ldo = keys;
         launch_gemm<T, u16, T>(e, b.split, st);
-        GemmArgs f = gemm_args(b.low + l.rank, l.gate_w, W, l.gate_rank, l, EPI_SIGMOID);
+        GemmArgs f = gemm_args(whole(b.low + l.rank), l.gate_w, W, l.gate_rank, l, EPI_SIGMOID);
         f.lda = ranks; f.out = b.gate; f.ldo = W;
         launch_gemm<T, u16, T>(f, b.split, st);
         c.qkv = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = W;
@@ -750,27 +785,27 @@ int prefill_plain(const QmkHybridArgs* a) {
           hipLaunchKernelGGL(keep_inputs, dim3((channels + kPfThreads - 1) / kPfThreads), block, 0, st, b.qkv, l, channels, a->slot, a->flip, M);
       } else {
         const int keys = l.heads * l.head_dim;
-        GemmArgs g = gemm_args(b.h, l.in_w, l.in_rows, D, l, EPI_GLA_IN);
+        GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_GLA_IN);
         g.f0 = b.qkv; g.out = b.gate; g.out2 = b.low;
         launch_gemm<T, u16, T>(g, b.split, st);
-        GemmArgs e = gemm_args(b.low, l.mid_w, keys, l.rank, l, EPI_GLA_DECAY);
+        GemmArgs e = gemm_args(whole(b.low), l.mid_w, keys, l.rank, l, EPI_GLA_DECAY);
         e.f0 = b.decay; e.ldo = keys;
         launch_gemm<T, u16, T>(e, b.split, st);
         c.qkv = b.qkv; c.values = b.qkv; c.value_ld = 2 * keys + W; c.value_at = 2 * keys;
         run_chunks<false>(a, c, st);
       }
-      hipLaunchKernelGGL(state_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.o, b.gate, l, M, a->eps, b.mix);
+      hipLaunchKernelGGL(state_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.o, b.gate, l, M, a->eps, b.mix.of(W));
     }
-    GemmArgs o = gemm_args(b.mix, l.o_w, D, W, l, l.branches > 1 ? EPI_LOGITS : EPI_ADD);
+    GemmArgs o = gemm_args(b.mix.of(W), l.o_w, D, W, l, l.branches > 1 ? EPI_LOGITS : EPI_ADD);
     o.f0 = l.branches > 1 ? b.branch + l.branch * rows : b.x;
     launch_gemm<T, u16, T>(o, b.split, st);
     if (l.branch + 1 == l.branches) {
       const QmkHybridLayer& head = a->layers[i - l.branch];
       if (head.has_mlp) {
-        GemmArgs g = gemm_args(b.h, head.mlp_w, 2 * head.ff, D, head, EPI_GEGLU);
-        g.out = b.mix;
+        GemmArgs g = gemm_args(b.h.of(D), head.mlp_w, 2 * head.ff, D, head, EPI_GEGLU);
+        g.out = b.mix.at; g.out_part = b.mix.of(head.ff).part;
         launch_gemm<T, u16, T>(g, b.split, st);
-        GemmArgs d = gemm_args(b.mix, head.down_w, D, head.ff, head, EPI_ADD);
+        GemmArgs d = gemm_args(b.mix.of(head.ff), head.down_w, D, head.ff, head, EPI_ADD);
         d.f0 = b.x;
         launch_gemm<T, u16, T>(d, b.split, st);
       }

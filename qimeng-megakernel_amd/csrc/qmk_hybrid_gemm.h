@@ -29,6 +29,89 @@ enum : int {
   EPI_GLA_DECAY,
 };
 
+// An fp32 value is the sum of three bf16 values that take its significand's bits 23..16, 15..8 and 7..0 (exactly: every
+// remainder is exact, and the exponents are the same), and a product of two bf16 values is exact in fp32: three bf16 instructions
+// add up the same products as the eight fp32 ones of the same columns, in a fifth of their time.  Values that are not finite
+// stay whole in the first part.
+__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+__device__ __forceinline__ float behind_upper_half(float v) { return v - __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
+__device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+// Two neighbouring values -> their parts.
+__device__ __forceinline__ void split2(float x, float y, uint32_t (&part)[3]) {
+  part[0] = upper_halves(x, y);
+  const float x1 = behind_upper_half(x), y1 = behind_upper_half(y);
+  part[1] = upper_halves(x1, y1);
+  part[2] = upper_halves(behind_upper_half(x1), behind_upper_half(y1));
+  if (__builtin_expect(not_finite(x) | not_finite(y), 0)) {
+    const float v[2] = {x, y};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (not_finite(v[e])) {
+        const uint32_t keep = e ? 0x0000ffffu : 0xffff0000u, top = v[e] != v[e] ? 0x7fc0u : __float_as_uint(v[e]) >> 16;
+        part[0] = (part[0] & keep) | (e ? top << 16 : top);
+        part[1] &= keep;
+        part[2] &= keep;
+      }
+    }
+  }
+}
+
+// fp32 mode: the rows a projection reads next (normed input, mixed heads, gated rows) are left as three bf16 parts, `part`
+// elements from one to the next, by the kernel that makes them, so that their tiles go from memory to LDS as they are and by
+// themselves, instead of through the registers of the workgroups that read them.  part = 0: they stay whole.
+template <class T>
+struct Operand {
+  T* at;
+  size_t part;
+  __device__ __forceinline__ u16* parts() const { return reinterpret_cast<u16*>(at); }
+};
+template <class T>
+__device__ __forceinline__ void store4(T* at, f32x4 v);
+template <class T>
+__device__ __forceinline__ void put4(const Operand<T>& to, size_t i, f32x4 v) {
+  if constexpr (sizeof(T) == 4) {
+    if (to.part != 0) {
+      uint32_t a[3], b[3];
+      split2(v[0], v[1], a);
+      split2(v[2], v[3], b);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(to.parts() + q * to.part + i) = make_uint2(a[q], b[q]);
+      return;
+    }
+  }
+  store4(to.at + i, v);
+}
+template <class T>
+__device__ __forceinline__ void put2(const Operand<T>& to, size_t i, float x, float y) {
+  if constexpr (sizeof(T) == 4) {
+    if (to.part != 0) {
+      uint32_t a[3];
+      split2(x, y, a);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32_t*>(to.parts() + q * to.part + i) = a[q];
+      return;
+    }
+    *reinterpret_cast<float2*>(to.at + i) = make_float2(x, y);
+  } else {
+    *reinterpret_cast<uint32_t*>(to.at + i) = f2bf2(x, y);
+  }
+}
+template <class T>
+__device__ __forceinline__ void put1(const Operand<T>& to, size_t i, float x) {
+  if constexpr (sizeof(T) == 4) {
+    if (to.part != 0) {
+      uint32_t a[3];
+      split2(x, 0.f, a);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) to.parts()[q * to.part + i] = static_cast<u16>(a[q]);
+      return;
+    }
+  }
+  to.at[i] = from_f32<T>(x);
+}
+
 struct GemmArgs {
   const void* a;         // TA [M][lda]
   const void* w;         // TW [N][ldw]
@@ -48,6 +131,8 @@ struct GemmArgs {
   float* partial;        // sums of the parts of a product that is cut along K, and a zero per tile
   int32_t* tickets;
   int splits;
+  size_t a_part;         // Operand::part of a (last: the bf16 mode reads neither, and its first cache lines stay as they are)
+  size_t out_part;       // EPI_GEGLU: Operand::part of out
 };
 
 template <class T>
@@ -128,11 +213,9 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, int group, int m, in
       break;
     }
     case EPI_GEGLU: {
-      T* o = static_cast<T*>(g.out) + static_cast<size_t>(m) * l.ff + n / 2;
       const bool silu = l.act == QMK_ACT_SILU;
       const float a = (silu ? v[0] * sigmoid(v[0]) : gelu_tanh(v[0])) * v[1], b = (silu ? v[2] * sigmoid(v[2]) : gelu_tanh(v[2])) * v[3];
-      if constexpr (sizeof(T) == 2) *reinterpret_cast<uint32_t*>(o) = f2bf2(a, b);
-      else *reinterpret_cast<float2*>(o) = make_float2(a, b);
+      put2(Operand<T>{static_cast<T*>(g.out), g.out_part}, static_cast<size_t>(m) * l.ff + n / 2, a, b);
       break;
     }
     case EPI_WKV_IN: {
@@ -247,8 +330,7 @@ struct Tile {
   static constexpr int kWavesM = BM / WM, kWavesN = BN / WN, kCover = kWavesM * kWavesN, kGroups = WAVES_ / kCover;
   static constexpr int kTm = WM / 16, kTn = WN / 16, kKept = kTn / kGroups;   // a wave's fragments; of those a thread sums up
   static constexpr int kRow = BK / 8;                                           // a row of a step: units of 16 bytes
-  static constexpr int kUnits = (BM + BN) * kRow, kLoads = (kUnits + kThreadCount - 1) / kThreadCount;
-  static constexpr int kLastWaves = (kUnits - (kLoads - 1) * kThreadCount) / 64;   // waves that take part in a stage's last load
+  static constexpr int kUnits = (BM + BN) * kRow;
   static constexpr bool kSplits = kKept * kTm <= 8;                             // may be cut along K
   static constexpr int kSteps = BK / 32 / kGroups;                              // matrix steps a wave takes of a step
   static constexpr int kOutUnits = BM * BN / 4, kPasses = kOutUnits > kStages * kUnits ? 2 : 1;
@@ -441,10 +523,13 @@ __device__ __forceinline__ void wait_outstanding() {
 // The tiles of a step, bf16: memory -> LDS without passing through registers, kStages buffers deep.  A row's units are exchanged
 // by its number on the memory side (the LDS side of such a load is one run of 64 units per wave), so that fragment reads do
 // not conflict.
-template <class S>
+template <class S, int PARTS = 1>      // of the tokens' side
 struct Stages {
+  static constexpr int kRowsA = S::BM * PARTS, kUnits = (kRowsA + S::BN) * S::kRow, kLoads = (kUnits + S::kThreadCount - 1) / S::kThreadCount;
+  static constexpr int kLastWaves = (kUnits - (kLoads - 1) * S::kThreadCount) / 64;      // waves that take part in a stage's last load
+  static_assert(kUnits % 64 == 0, "a wave's loads are whole");
   using Lds = __attribute__((address_space(3))) v4u;      // said outright: a pointer kept in a struct may become a generic one
-  const u16* from[S::kLoads];      // this thread's places in a stage: unit i * threads + tid, tokens first
+  const u16* from[kLoads];      // this thread's places in a stage: unit i * threads + tid, tokens first
   Lds* lds;
   int wave;
 
@@ -453,17 +538,19 @@ struct Stages {
     const u16* a = static_cast<const u16*>(g.a) + p.group * g.a_step + p.first * S::BK;
     const u16* w = static_cast<const u16*>(g.w) + p.group * g.w_step + p.first * S::BK;
 #pragma unroll
-    for (int i = 0; i < S::kLoads; ++i) {
+    for (int i = 0; i < kLoads; ++i) {
       const int u = i * S::kThreadCount + threadIdx.x, r = u / S::kRow, c = ((u % S::kRow) ^ exchange(r)) * 8;
-      from[i] = r < S::BM ? a + static_cast<size_t>(min(p.m0 + r, g.M - 1)) * g.lda + c : w + static_cast<size_t>(min(p.n0 + r - S::BM, p.N - 1)) * g.ldw + c;
+      from[i] = r < kRowsA ? a + static_cast<size_t>(min(p.m0 + (PARTS == 1 ? r : r % S::BM), g.M - 1)) * g.lda + c
+                           : w + static_cast<size_t>(min(p.n0 + r - kRowsA, p.N - 1)) * g.ldw + c;
+      if constexpr (PARTS > 1) from[i] += r < kRowsA ? r / S::BM * g.a_part : 0;
     }
   }
   __device__ __forceinline__ void issue(int buf) {
 #pragma unroll
-    for (int i = 0; i < S::kLoads; ++i) {
-      if (i == S::kLoads - 1 && S::kLastWaves * 64 < S::kThreadCount && wave >= S::kLastWaves) continue;
+    for (int i = 0; i < kLoads; ++i) {
+      if (i == kLoads - 1 && kLastWaves * 64 < S::kThreadCount && wave >= kLastWaves) continue;
       const auto* src = (const __attribute__((address_space(1))) uint32_t*)from[i];
-      auto* dst = (__attribute__((address_space(3))) uint32_t*)(lds + buf * S::kUnits + i * S::kThreadCount + wave * 64);
+      auto* dst = (__attribute__((address_space(3))) uint32_t*)(lds + buf * kUnits + i * S::kThreadCount + wave * 64);
       __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
       from[i] += S::BK;
     }
@@ -471,11 +558,11 @@ struct Stages {
   // Until at most `stages` stages of this wave's are outstanding.
   template <int stages>
   __device__ __forceinline__ void wait() const {
-    if (S::kLastWaves * 64 == S::kThreadCount || wave < S::kLastWaves) wait_outstanding<stages * S::kLoads>();
-    else wait_outstanding<stages * (S::kLoads - 1)>();
+    if (kLastWaves * 64 == S::kThreadCount || wave < kLastWaves) wait_outstanding<stages * kLoads>();
+    else wait_outstanding<stages * (kLoads - 1)>();
   }
-  __device__ __forceinline__ void fragments(int buf, int q, int wm, int wn, Frag<u16> (&fa)[S::kTm], Frag<u16> (&fw)[S::kTn]) const {
-    const Lds *la = lds + buf * S::kUnits, *lw = la + S::BM * S::kRow;
+  __device__ __forceinline__ void fragments(int buf, int q, int wm, int wn, Frag<u16> (&fa)[PARTS][S::kTm], Frag<u16> (&fw)[S::kTn]) const {
+    const Lds *la = lds + buf * kUnits, *lw = la + kRowsA * S::kRow;
     const int row = threadIdx.x & 15;
     auto frag = [](const Lds* at) { return Frag<u16>{__builtin_bit_cast(bf16x8_t, *at)}; };
 #pragma unroll
@@ -483,32 +570,44 @@ struct Stages {
       const int r = wn * S::WN + j * 16 + row;
       fw[j] = frag(lw + r * S::kRow + (q ^ exchange(r)));
     }
+    static_assert(PARTS == 1 || S::BM % 16 == 0, "rows of every part are exchanged alike");
 #pragma unroll
-    for (int i = 0; i < S::kTm; ++i) {
-      const int r = wm * S::WM + i * 16 + row;
-      fa[i] = frag(la + r * S::kRow + (q ^ exchange(r)));
-    }
+    for (int part = 0; part < PARTS; ++part)
+#pragma unroll
+      for (int i = 0; i < S::kTm; ++i) {
+        const int r = part * S::BM + wm * S::WM + i * 16 + row;
+        fa[part][i] = frag(la + r * S::kRow + (q ^ exchange(r)));
+      }
   }
 };
 
-template <class S>
-__device__ __forceinline__ void multiply(const Frag<u16> (&fa)[S::kTm], const Frag<u16> (&fw)[S::kTn], f32x4 (&acc)[S::kTn][S::kTm]) {
+template <class S, int PARTS>
+__device__ __forceinline__ void multiply(const Frag<u16> (&fa)[PARTS][S::kTm], const Frag<u16> (&fw)[S::kTn], f32x4 (&acc)[S::kTn][S::kTm]) {
 #pragma unroll
   for (int i = 0; i < S::kTm; ++i)
 #pragma unroll
-    for (int j = 0; j < S::kTn; ++j) acc[j][i] = mma(fw[j], fa[i], acc[j][i]);
+    for (int j = 0; j < S::kTn; ++j) {
+      if constexpr (PARTS == 1) {
+        acc[j][i] = mma(fw[j], fa[0][i], acc[j][i]);
+      } else {      // 32 columns by themselves, small parts first, then one rounded addition
+        f32x4 t = {};
+#pragma unroll
+        for (int part = PARTS - 1; part >= 0; --part) t = mma(fw[j], fa[part][i], t);
+        acc[j][i] += t;
+      }
+    }
 }
 
-// out[m][n] = sum_k a[m][k] w[n][k], bf16 x bf16, K a multiple of BK.  The weights are the matrix instruction's first operand,
+// out[m][n] = sum_k a[m][k] w[n][k], bf16 x bf16 or the tokens' side in three parts, K a multiple of BK.  The weights are the matrix instruction's first operand,
 // so a lane ends up with four consecutive outputs of one token.  Four waves; several workgroups share a CU.
-template <class T, class S>
+template <class T, class S, int PARTS = 1>
 __global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g) {
-  constexpr int kAhead = S::kStages - 1;
-  __shared__ __align__(16) v4u lds[S::kLds + 1];
+  constexpr int kAhead = S::kStages - 1, kStageUnits = S::kStages * Stages<S, PARTS>::kUnits, kLds = kStageUnits > S::kLds ? kStageUnits : S::kLds;
+  __shared__ __align__(16) v4u lds[kLds + 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % S::kWavesM, wn = wave / S::kWavesM;
   const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
-  Stages<S> stages(g, p, lds, wave);
+  Stages<S, PARTS> stages(g, p, lds, wave);
   f32x4 acc[S::kTn][S::kTm] = {};
 #pragma unroll
   for (int s = 0; s < kAhead; ++s)
@@ -524,13 +623,13 @@ __global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g)
     if (s + kAhead < p.steps) stages.issue(buf == 0 ? S::kStages - 1 : buf - 1);
 #pragma unroll
     for (int kk = 0; kk < S::kSteps; ++kk) {
-      Frag<u16> fa[S::kTm], fw[S::kTn];
+      Frag<u16> fa[PARTS][S::kTm], fw[S::kTn];
       stages.fragments(buf, kk * 4 + (lane >> 4), wm, wn, fa, fw);
-      multiply<S>(fa, fw, acc);
+      multiply<S, PARTS>(fa, fw, acc);
     }
     buf = buf + 1 == S::kStages ? 0 : buf + 1;
   }
-  finish_tile<T, S, S::kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+  finish_tile<T, S, kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
 
 // The same with eight waves, one workgroup a CU.  Two waves share a SIMD's matrix unit, and the halves of the workgroup take
@@ -564,14 +663,14 @@ __global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
   for (int s = 0; s < p.steps; ++s) {
     // The buffer filled here was read in step s - 1: by this half a turn ago, by the other one before the last barrier.
     if (s + kAhead < p.steps) stages.issue(buf == 0 ? S::kStages - 1 : buf - 1);
-    Frag<u16> fa[S::kTm], fw[S::kTn];
+    Frag<u16> fa[1][S::kTm], fw[S::kTn];
     stages.fragments(buf, kg * 4 + (lane >> 4), wm, wn, fa, fw);
     // Stage s + 1 has landed: a barrier lies between this wait and either half's reads of it.
     if (s + kAhead < p.steps) stages.template wait<kAhead - 1>();
     else wait_outstanding<0>();
     barrier();
     __builtin_amdgcn_s_setprio(1);
-    multiply<S>(fa, fw, acc);
+    multiply<S, 1>(fa, fw, acc);
     __builtin_amdgcn_s_setprio(0);
     barrier();
     buf = buf + 1 == S::kStages ? 0 : buf + 1;
@@ -581,43 +680,8 @@ __global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
 }
 
 // ---- products with an fp32 side, and bf16 ones of any K ----
-// An fp32 value is the sum of three bf16 values that take its significand's bits 23..16, 15..8 and 7..0 (exactly: every
-// remainder is exact, and the exponents are the same), and a product of two bf16 values is exact in fp32: three bf16 instructions
-// add up the same products as the eight fp32 ones of the same columns, in a fifth of their time.  Values that are not finite
-// stay whole in the first part.
 template <class T>
 constexpr int kPlanes = sizeof(T) == 2 ? 1 : 3;
-__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
-  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-__device__ __forceinline__ float behind_upper_half(float v) { return v - __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
-__device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
-// Eight values -> their planes.
-__device__ __forceinline__ void split8(const v4u& lo, const v4u& hi, v4u (&plane)[3]) {
-  const uint32_t bits[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-  bool odd = false;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float x = __uint_as_float(bits[2 * e]), y = __uint_as_float(bits[2 * e + 1]);
-    odd |= not_finite(x) | not_finite(y);
-    plane[0][e] = upper_halves(x, y);
-    const float x1 = behind_upper_half(x), y1 = behind_upper_half(y);
-    plane[1][e] = upper_halves(x1, y1);
-    plane[2][e] = upper_halves(behind_upper_half(x1), behind_upper_half(y1));
-  }
-  if (__builtin_expect(odd, 0)) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = __uint_as_float(bits[e]);
-      if (not_finite(x)) {
-        const uint32_t keep = e & 1 ? 0x0000ffffu : 0xffff0000u, top = x != x ? 0x7fc0u : bits[e] >> 16;
-        plane[0][e >> 1] = (plane[0][e >> 1] & keep) | (e & 1 ? top << 16 : top);
-        plane[1][e >> 1] &= keep;
-        plane[2][e >> 1] &= keep;
-      }
-    }
-  }
-}
 
 // BN weight rows x BM tokens a workgroup, four waves as 2 x 2, 64 columns a step, through registers.  LDS holds
 // 16-byte units of bf16, planes one after the other, a row's units exchanged by its number.
@@ -661,7 +725,14 @@ __global__ __launch_bounds__(kPfThreads) void gemm(const GemmArgs g) {
           to[place] = r[i][0];
         } else {
           v4u plane[3];
-          split8(r[i][0], r[i][1], plane);
+          const uint32_t bits[8] = {r[i][0].x, r[i][0].y, r[i][0].z, r[i][0].w, r[i][1].x, r[i][1].y, r[i][1].z, r[i][1].w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            uint32_t t[3];
+            split2(__uint_as_float(bits[2 * e]), __uint_as_float(bits[2 * e + 1]), t);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) plane[q][e] = t[q];
+          }
 #pragma unroll
           for (int q = 0; q < 3; ++q) to[q * units + place] = plane[q];
         }
@@ -764,6 +835,9 @@ using Tiles16 = Tile<64, 16, 64, 16, 16, 4, 4>;        // few tokens: weight row
 using Tiles32 = Tile<64, 32, 64, 32, 16, 4, 4>;
 using Tiles64 = Tile<64, 64, 64, 32, 32, 4, 4>;
 using Tiles128 = Tile<128, 128, 64, 64, 64, 4, 2>;
+// The tokens' side in three parts: it is what fills LDS, so few tokens a tile (us, 32 x 128 and 64 x 64 and 64 x 128 and 128 x 128: 200 x 2048 x 6144
+// 32, 35, 54, 169; 200 x 12288 x 2048 52, 58, 52, 63; 2048 x 2048 x 8192 260, 420, 291, 280).
+using TilesParts = Tile<32, 128, 64, 16, 64, 4, 2>;
 using Turns64 = Tile<64, 128, 64, 32, 64, 8, 4>;
 using Turns96 = Tile<96, 128, 64, 48, 64, 8, 4>;
 using Turns128 = Tile<128, 128, 64, 64, 64, 8, 4>;

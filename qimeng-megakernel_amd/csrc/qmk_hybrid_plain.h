@@ -30,7 +30,7 @@ struct ResidualArgs {
   float scale, eps;
 };
 template <class T>
-__global__ __launch_bounds__(kPfThreads) void residual_rows(const ResidualArgs g, T* h) {
+__global__ __launch_bounds__(kPfThreads) void residual_rows(const ResidualArgs g, Operand<T> h) {
   __shared__ float scratch[4];
   const int D = g.D;
   int m = g.want != nullptr ? g.want[blockIdx.x] : blockIdx.x;
@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kPfThreads) void residual_rows(const ResidualArgs g
     if (i < D) take(i, held[j] = value(i));
   }
   for (int i = (kHeld * kPfThreads + threadIdx.x) * 4; i < D; i += kPfThreads * 4) take(i, value(i));
-  T* out = h + static_cast<size_t>(blockIdx.x) * D * (g.weight == nullptr ? 2 : 1);
+  const size_t out = static_cast<size_t>(blockIdx.x) * D * (g.weight == nullptr ? 2 : 1);
   float mean = 0.f, inv = 0.f;
   auto centred = [&](int i, f32x4 v) {
 #pragma unroll
@@ -93,10 +93,10 @@ __global__ __launch_bounds__(kPfThreads) void residual_rows(const ResidualArgs g
   auto put = [&](int i, f32x4 v) {
     if (keep) store4(x + i, v);
     if (g.weight != nullptr) {
-      store4(out + i, centred(i, v) * inv * read4(g.weight + i));
+      put4(h, out + i, centred(i, v) * inv * read4(g.weight + i));
     } else {
-      store4(out + i, v);
-      store4(out + D + i, read4(e + i));
+      put4(h, out + i, v);
+      put4(h, out + D + i, read4(e + i));
     }
   };
 #pragma unroll
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(WAVES * 64) void chunk_scan(const ChunkArgs g) {
 
 // Per-head norm, weight and gate behind the recurrence: one wave per (token, head).
 template <class T>
-__global__ __launch_bounds__(kPfThreads) void state_out(const float* o, const T* gate, QmkHybridLayer l, int M, float eps, T* out) {
+__global__ __launch_bounds__(kPfThreads) void state_out(const float* o, const T* gate, QmkHybridLayer l, int M, float eps, Operand<T> out) {
   const int id = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (id >= M * l.heads) return;
   const int n = l.v_dim;
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(kPfThreads) void state_out(const float* o, const T*
   float sq = 0.f;
   for (int i = lane; i < n; i += 64) sq = fmaf(o[at + i], o[at + i], sq);
   const float inv = 1.f / sqrtf(wave_sum(sq) / l.v_true + eps);
-  for (int i = lane; i < n; i += 64) out[at + i] = from_f32<T>(o[at + i] * inv * l.vec0[i] * to_f32(gate[at + i]));
+  for (int i = lane; i < n; i += 64) put1(out, at + i, o[at + i] * inv * l.vec0[i] * to_f32(gate[at + i]));
 }
 
 }  // namespace hybrid

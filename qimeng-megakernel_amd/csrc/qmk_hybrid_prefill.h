@@ -35,7 +35,7 @@ __global__ __launch_bounds__(kPfThreads) void embed_tokens(const u16* table, con
 
 // h = norm(u[row]); row = want[blockIdx.x] where given
 template <class T>
-__global__ __launch_bounds__(kPfThreads) void norm_rows(const float* u, const float* weight, const int32_t* want, int limit, int D, int true_width, float eps, T* h) {
+__global__ __launch_bounds__(kPfThreads) void norm_rows(const float* u, const float* weight, const int32_t* want, int limit, int D, int true_width, float eps, Operand<T> h) {
   __shared__ float scratch[4];
   const int m = blockIdx.x;
   int from = want != nullptr ? want[m] : m;
@@ -48,12 +48,12 @@ __global__ __launch_bounds__(kPfThreads) void norm_rows(const float* u, const fl
   }
   const float inv = 1.f / sqrtf(pf_block_sum(sq, scratch) / true_width + eps);
   for (int i = threadIdx.x * 4; i < D; i += kPfThreads * 4)
-    store4(h + static_cast<size_t>(m) * D + i, *reinterpret_cast<const f32x4*>(row + i) * inv * *reinterpret_cast<const f32x4*>(weight + i));
+    put4(h, static_cast<size_t>(m) * D + i, *reinterpret_cast<const f32x4*>(row + i) * inv * *reinterpret_cast<const f32x4*>(weight + i));
 }
 
 // The five mixes of a token's normed input with the previous token's; the last token leaves its own for the next portion.
 template <class T>
-__global__ __launch_bounds__(kPfThreads) void shift_mix(const float* u, QmkHybridLayer l, int slot, int flip, int M, int rows_cap, int D, int true_width, float eps, T* out) {
+__global__ __launch_bounds__(kPfThreads) void shift_mix(const float* u, QmkHybridLayer l, int slot, int flip, int M, int rows_cap, int D, int true_width, float eps, Operand<T> out) {
   __shared__ float scratch[4];
   const int m = blockIdx.x;
   const float* row = u + static_cast<size_t>(m) * D;
@@ -78,9 +78,7 @@ __global__ __launch_bounds__(kPfThreads) void shift_mix(const float* u, QmkHybri
 #pragma unroll
     for (int q = 0; q < 5; ++q) {
       const float a = h[0] + d[0] * l.vec2[q * D + i], b = h[1] + d[1] * l.vec2[q * D + i + 1];
-      T* o = out + (static_cast<size_t>(q) * rows_cap + m) * D + i;
-      if constexpr (sizeof(T) == 2) *reinterpret_cast<uint32_t*>(o) = f2bf2(a, b);
-      else *reinterpret_cast<float2*>(o) = make_float2(a, b);
+      put2(out, (static_cast<size_t>(q) * rows_cap + m) * D + i, a, b);
     }
   }
 }
@@ -107,7 +105,7 @@ __global__ __launch_bounds__(kPfThreads) void causal_conv(const T* x, QmkHybridL
 // S_t = a_t S_{t-1} + b_t, out = S y: sixteen channels a workgroup, the portion cut into 64 runs of tokens.
 constexpr int kScanChannels = 16, kScanRuns = 64;
 template <class T>
-__global__ __launch_bounds__(kScanChannels * kScanRuns) void lru_scan(const float* a, const float* b, const T* y, QmkHybridLayer l, int slot, int M, T* out) {
+__global__ __launch_bounds__(kScanChannels * kScanRuns) void lru_scan(const float* a, const float* b, const T* y, QmkHybridLayer l, int slot, int M, Operand<T> out) {
   __shared__ float sa[kScanRuns][kScanChannels], sb[kScanRuns][kScanChannels];
   const int W = l.mix_width, ch = threadIdx.x % kScanChannels, run = threadIdx.x / kScanChannels;
   const int c = blockIdx.x * kScanChannels + ch;
@@ -139,7 +137,7 @@ __global__ __launch_bounds__(kScanChannels * kScanRuns) void lru_scan(const floa
   for (int t = lo; t < hi; ++t) {
     const size_t at = static_cast<size_t>(t) * W + c;
     s = fmaf(a[at], s, b[at]);
-    out[at] = from_f32<T>(s * to_f32(y[at]));
+    put1(out, at, s * to_f32(y[at]));
   }
 }
 
@@ -188,7 +186,7 @@ struct Keys {
 constexpr int kAttendGroups = 2;
 template <class T, int QT, int VT>   // most 32-column steps of a query, most 16-row tiles of a value
 __global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(const T* q, Keys<T> keys, const T* rows, const T* v_t, const T* gate, QmkHybridLayer l,
-                                                               int first, int position, int M, int keys_cap, T* out) {
+                                                               int first, int position, int M, int keys_cap, Operand<T> out) {
   constexpr int kKeys = 32;
   constexpr int kPadK = 16 / sizeof(T), kPadV = 16 / sizeof(T);
   struct Step {
@@ -351,7 +349,7 @@ __global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(c
   const size_t at = static_cast<size_t>(m) * l.heads * l.v_dim + head * l.v_dim;
 #pragma unroll
   for (int t = 0; t < VT; ++t)
-    if (t < vt) store4(out + at + t * 16 + g * 4, acc[t] * inv * read4(gate + at + t * 16 + g * 4));
+    if (t < vt) put4(out, at + t * 16 + g * 4, acc[t] * inv * read4(gate + at + t * 16 + g * 4));
 }
 
 // The wkv recurrence: one head and eight value columns a workgroup; sixteen lanes share a column, KPL neighbouring key
@@ -450,7 +448,7 @@ __global__ __launch_bounds__(kWkvThreads) void wkv_scan(const float* r, const fl
 
 // Per-head norm, weight and gate behind the recurrence: one wave per (token, head).
 template <class T>
-__global__ __launch_bounds__(kPfThreads) void wkv_out(const float* o, const T* gate, QmkHybridLayer l, int M, float eps, T* out) {
+__global__ __launch_bounds__(kPfThreads) void wkv_out(const float* o, const T* gate, QmkHybridLayer l, int M, float eps, Operand<T> out) {
   const int id = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (id >= M * l.heads) return;
   const int n = l.head_dim, m = id / l.heads, head = id % l.heads;
@@ -458,7 +456,7 @@ __global__ __launch_bounds__(kPfThreads) void wkv_out(const float* o, const T* g
   float sq = 0.f;
   for (int i = lane; i < n; i += 64) sq = fmaf(o[at + i], o[at + i], sq);
   const float inv = 1.f / sqrtf(wave_sum(sq) / l.head_dim_true + eps);
-  for (int i = lane; i < n; i += 64) out[at + i] = from_f32<T>(o[at + i] * inv * l.vec0[head * n + i] * to_f32(gate[at + i]));
+  for (int i = lane; i < n; i += 64) put1(out, at + i, o[at + i] * inv * l.vec0[head * n + i] * to_f32(gate[at + i]));
 }
 
 __global__ __launch_bounds__(kPfThreads) void sum_streams(const float* x, int S, int D, float* out) {

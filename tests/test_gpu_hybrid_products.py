@@ -48,10 +48,11 @@ def test_products_at_the_edges_of_tiles(name, n, dtype):
     assert err < TOL[dtype], f"{err:.3g}"
 
 
-def test_values_that_are_not_finite_stay_so_in_fp32():
+@pytest.mark.parametrize("width,channels", [(208, 160), (256, 192)], ids=["whole", "parts"])
+def test_values_that_are_not_finite_stay_so_in_fp32(width, channels):
     """An infinite or undefined embedding reaches the logits of its token as such, and none of a token before it.  (A
     recurrence: an attention's weight of zero times an undefined value is undefined.)"""
-    shape = synthetic.hybrid_shape("r", width=208, vocab=96, streams=2, ff={"r": 176}, lru_width=160, blocks=1, taps=3)
+    shape = synthetic.hybrid_shape("r", width=width, vocab=96, streams=2, ff={"r": channels + 16 * (width == 208)}, lru_width=channels, blocks=1, taps=3)
     w = synthetic.random_hybrid_weights(shape, 6, DEVICE)
     w["embed"][7, 3] = float("inf")
     w["embed"][8, 5] = float("nan")
