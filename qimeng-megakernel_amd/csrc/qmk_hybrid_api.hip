@@ -470,24 +470,26 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
 // `each` for every part.  All figures measured with weights that come from memory (us, M x N x K, the kernels this replaced ->
 // now): 2048 x 16384 x 2048 160 -> 138, 1531 x 16384 x 2048 115 -> 113, 2048 x 6144 x 2048 77 -> 64, 1531 x 5696 x 2048 63 -> 54,
 // 2048 x 2048 x 8192 107 -> 75, 1531 x 2048 x 8192 with the residual's streams 141 -> 83, 1531 x 2048 x 2048 with them 71 -> 41,
-// 512 x 2048 x 8192 73 -> 37.  Up to 64 tokens a product is a stream of weights, and narrow tiles put more workgroups on it and
-// leave less to add up: 43 x 2048 x 6144 with the streams 38 -> 20 on 64 rows of weights -> 14 on 16, 43 x 2048 x 2048 with them
-// 21 -> 16 -> 10, 43 x 12288 x 2048 23 -> 13.5 -> 13 on 32.
+// 512 x 2048 x 8192 73 -> 37.  With few tokens a product is a stream of weights, and narrow tiles put more workgroups on it and
+// leave less to add up: 43 x 2048 x 6144 with the streams 38 -> 20 on 64 rows of weights -> 15 on 16, in four parts (19 on 32, in
+// eight), 43 x 2048 x 2048 with them 21 -> 16 -> 11, 43 x 12288 x 2048 23 -> 13.5 -> 13 on 32.  Beyond 64 tokens their several
+// token tiles share the weights in L2: whole prompts on the 64 rows before -> narrow tiles, 70 tokens 3491 -> 3143, 130 3939 -> 3636,
+// 200 4192 -> 3908; the line is at 256, since 300 tokens take 5085 -> 5202.
 struct TileCost {
   int most_tokens, bm, bn, slots;
   double step, fixed, overlapped, meet, each;
 };
 constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 9;
 constexpr TileCost kTileCosts[kTileKinds] = {
-    {kAnyTokens, 64, 64, 256, 9.0, 0.0, 5.0, 1.0, 0.6},      // Tiles64
+    {kAnyTokens, 64, 64, 256, 9.0, 0.0, 5.0, 1.3, 1.1},      // Tiles64
     {kAnyTokens, 128, 128, 512, 36.0, 8.0, 0.0, 0.0, 0.0},   // Tiles128
     {kAnyTokens, 64, 128, 256, 12.0, 6.5, 0.0, 3.0, 1.5},    // Turns64
     {kAnyTokens, 96, 128, 256, 14.5, 6.5, 0.0, 3.0, 1.5},    // Turns96
     {kAnyTokens, 128, 128, 256, 17.0, 9.0, 0.0, 3.0, 2.0},   // Turns128
     {kAnyTokens, 192, 256, 256, 47.0, 10.0, 0.0, 0.0, 0.0},  // Turns192
     {kAnyTokens, 256, 256, 256, 60.0, 9.0, 0.0, 0.0, 0.0},   // Turns256
-    {64, 64, 32, 512, 6.5, 0.0, 4.5, 0.5, 0.35},             // Tiles32
-    {64, 64, 16, 512, 6.5, 0.0, 4.0, 0.5, 0.3},              // Tiles16
+    {256, 64, 32, 512, 8.0, 0.0, 4.5, 1.2, 1.0},             // Tiles32
+    {256, 64, 16, 512, 6.5, 0.0, 4.0, 0.5, 0.7},             // Tiles16
 };
 struct TileChoice {
   int kind = 0, splits = 1;
