@@ -327,6 +327,7 @@ inline size_t values_cap(const QmkHybridArgs* a) { return (static_cast<size_t>(a
 struct SplitBuffers {
   int32_t* tickets;
   f32x4* partial;
+  bool one_order = false;      // of the portion: kOneOrderTokens
 };
 inline SplitBuffers split_buffers(Carver& c) {
   SplitBuffers b;
@@ -464,66 +465,68 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
   return c.used;
 }
 
-// The tiles of a product.  A workgroup of the Turns kernels has a CU for itself, so a product takes as many rounds as its
-// tiles fill the chip, each about `step` us for 2048 columns and `fixed` us besides; of the others several share a CU, their
-// fixed part overlaps and `slots` of them make a round.  Cut along K into parts it takes `meet` us more for the first part and
-// `each` for every part.  All figures measured with weights that come from memory (us, M x N x K, the kernels this replaced ->
-// now): 2048 x 16384 x 2048 160 -> 138, 1531 x 16384 x 2048 115 -> 113, 2048 x 6144 x 2048 77 -> 64, 1531 x 5696 x 2048 63 -> 54,
-// 2048 x 2048 x 8192 107 -> 75, 1531 x 2048 x 8192 with the residual's streams 141 -> 83, 1531 x 2048 x 2048 with them 71 -> 41,
-// 512 x 2048 x 8192 73 -> 37.  With few tokens a product is a stream of weights, and narrow tiles put more workgroups on it and
-// leave less to add up: 43 x 2048 x 6144 with the streams 38 -> 20 on 64 rows of weights -> 15 on 16, in four parts (19 on 32, in
-// eight), 43 x 2048 x 2048 with them 21 -> 16 -> 11, 43 x 12288 x 2048 23 -> 13.5 -> 13 on 32.  Beyond 64 tokens their several
-// token tiles share the weights in L2: whole prompts on the 64 rows before -> narrow tiles, 70 tokens 3491 -> 3143, 130 3939 -> 3636,
-// 200 4192 -> 3908; the line is at 256, since 300 tokens take 5085 -> 5202.
+// A portion of so many tokens in bf16, or fewer, is computed in one order, whatever its tiles: the columns of a product one after the other (no
+// group of waves takes half of them, no workgroup a part), an attention's keys by one group of waves, a head's key channels by four waves.  Some tokens
+// are ill-conditioned (the norm over a recurrence's first output leaves little but the sign of a sum that may be close to zero, and some later tokens
+// come close to that), so that a sum taken in another order is enough to change what they leave in the states; a long portion averages that out.  Largest
+// relative difference of a state, cache or logits between two orders, 24 sets of weights of each of four shapes (width 2048): 2 tokens 0.31, 34
+// 0.065, 100 0.077, 256 0.050, 512 0.038, 700 0.033, 1000 0.026, 1531 0.024; the median is 0.008 to 0.024 at every length.
+constexpr int kOneOrderTokens = 1024;
+
+// The tiles of a bf16 product.  It takes as many rounds as its tiles fill the chip, `slots` at a time, each about `step` us for 2048 columns and `fixed` us
+// besides, and `overlapped` us once.  Fitted to measurements of every kind at 20 to 2048 tokens and 11 of the N x K of the four shapes (weights from
+// memory); the kind that comes out cheapest takes 1.1 % longer than the best one on the average up to 1024 tokens, 1.6 % beyond.  us, M x N x K,
+// the kinds around the line: 43 x 2048 x 2048 with the residual's streams Few32 9.3, Few64 10.0, Tiles32 14.1; 128 x 2048 x 4096 Few64 14, Tiles64 23; 300 x 5696 x 2048
+// Tiles64 18.5, Wide64 17; 1024 x 2048 x 6144 with the streams Wide64 55, Tiles128 116; 2048 x 16384 x 2048 Turns256 137, Tiles128 155; 2048 x 2048 x 8192 Turns128 76,
+// Wide64 100; 4096 x 2048 x 8192 Tiles128 159, Turns192 186, Turns128 189 (with the streams 192, 216, 214), 4096 x 2048 x 2048 with them 99, 117, 103.  Epilogues are not
+// priced, they are the same for all kinds; nor is memory, which bounds all of them alike where there are many rows for few tokens (1 x 128256 x 2048 Tiles32 95, Tiles64
+// 99, Tiles128 124).
 struct TileCost {
-  int most_tokens, bm, bn, slots;
-  double step, fixed, overlapped, meet, each;
+  int most_tokens, bm, bn, bk, slots;
+  double step, fixed, overlapped;
+  bool one_order;
 };
-constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 9;
+constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 10;
 constexpr TileCost kTileCosts[kTileKinds] = {
-    {kAnyTokens, 64, 64, 256, 9.0, 0.0, 5.0, 1.3, 1.1},      // Tiles64
-    {kAnyTokens, 128, 128, 512, 36.0, 8.0, 0.0, 0.0, 0.0},   // Tiles128
-    {kAnyTokens, 64, 128, 256, 12.0, 6.5, 0.0, 3.0, 1.5},    // Turns64
-    {kAnyTokens, 96, 128, 256, 14.5, 6.5, 0.0, 3.0, 1.5},    // Turns96
-    {kAnyTokens, 128, 128, 256, 17.0, 9.0, 0.0, 3.0, 2.0},   // Turns128
-    {kAnyTokens, 192, 256, 256, 47.0, 10.0, 0.0, 0.0, 0.0},  // Turns192
-    {kAnyTokens, 256, 256, 256, 60.0, 9.0, 0.0, 0.0, 0.0},   // Turns256
-    {256, 64, 32, 512, 8.0, 0.0, 4.5, 1.2, 1.0},             // Tiles32
-    {256, 64, 16, 512, 6.5, 0.0, 4.0, 0.5, 0.7},             // Tiles16
+    {kAnyTokens, 64, 64, 64, 256, 8.0, 0.0, 6.1, true},        // Tiles64
+    {kAnyTokens, 128, 128, 64, 512, 27.0, 8.0, 0.0, true},     // Tiles128
+    {kAnyTokens, 128, 64, 64, 256, 11.3, 0.0, 6.5, true},      // Wide64
+    {kAnyTokens, 96, 128, 64, 256, 14.7, 5.4, 3.0, false},     // Turns96
+    {kAnyTokens, 128, 128, 64, 256, 16.9, 6.2, 3.0, false},    // Turns128
+    {kAnyTokens, 192, 256, 32, 256, 38.3, 13.1, 0.0, true},    // Turns192
+    {kAnyTokens, 256, 256, 32, 256, 43.0, 14.2, 0.0, true},    // Turns256
+    {128, 64, 32, 64, 512, 7.3, 0.7, 4.3, true},               // Tiles32
+    {256, 64, 16, 128, 512, 5.8, 2.0, 2.3, true},              // Few64
+    {64, 32, 16, 256, 256, 3.9, 1.3, 3.6, true},               // Few32
 };
-struct TileChoice {
-  int kind = 0, splits = 1;
-};
-inline TileChoice choose_tiles(int M, int N, int K, int groups) {
-  TileChoice best;
+inline int choose_tiles(int M, int N, int K, int groups, bool one_order) {
+  int best = 0;
   double least = 0.;
   for (int kind = 0; kind < kTileKinds; ++kind) {
     const TileCost& t = kTileCosts[kind];
-    if (M > t.most_tokens) continue;
+    if (M > t.most_tokens || K % t.bk != 0 || (one_order && !t.one_order)) continue;
     const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * groups;
-    for (int splits = 1; splits <= 8; splits *= 2) {
-      if (splits > 1 && (t.each == 0. || K / splits < 256 || tiles > kMaxTickets || tiles * splits * t.bm * t.bn / 4 > kPartialUnits)) break;
-      const double rounds = static_cast<double>((tiles * splits + t.slots - 1) / t.slots);
-      const double us = rounds * (t.step * K / 2048. / splits + t.fixed) + t.overlapped + (splits > 1 ? t.meet + t.each * splits : 0.);
-      if ((kind == 0 && splits == 1) || us < least) {
-        least = us;
-        best = TileChoice{kind, splits};
-      }
+    const double us = static_cast<double>((tiles + t.slots - 1) / t.slots) * (t.step * K / 2048. + t.fixed) + t.overlapped;
+    if (kind == 0 || us < least) {
+      least = us;
+      best = kind;
     }
   }
   return best;
 }
 
-// The same for products with an fp32 side, or of columns that are no multiple of 64: tiles of 64 x 64 cut along K until they
-// fill the chip four times over, of 128 x 128 where there are tokens for them and they fill it already (us, 64 -> 128: 1 x 65536 x 2048
+// The same for products with an fp32 side, or of columns that are no multiple of 64: tiles of 128 x 128 where there are tokens for them and they
+// fill the chip already, else of 64 x 64, with an fp32 side cut along K until they fill it four times over (us, 64 -> 128: 1 x 65536 x 2048
 // 94 -> 150, 200 x 12288 x 2048 62 -> 76, 2048 x 16384 x 2048 829 -> 589).
-inline TileChoice choose_register_tiles(int M, int N, int K, int groups) {
-  TileChoice c;
+struct RegisterTiles {
+  bool large = false;
+  int splits = 1;
+};
+inline RegisterTiles choose_register_tiles(int M, int N, int K, int groups, bool cut) {
+  RegisterTiles c;
   const long long large = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128) * groups, small = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) * groups;
-  if (M >= 512 && large >= 256) {
-    c.kind = 1;
-    return c;
-  }
+  c.large = M >= 512 && large >= 256;
+  if (c.large || !cut) return c;
   while (c.splits < 8 && small * c.splits < 512 && K / c.splits >= 512 && small <= kMaxTickets && small * c.splits * 2 * 64 * 64 / 4 <= kPartialUnits) c.splits *= 2;
   return c;
 }
@@ -545,22 +548,22 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   auto launch = [&](auto kernel, int bm, int bn, int threads) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((n + bn - 1) / bn * ((g.M + bm - 1) / bm) * g.splits), 1, g.groups), dim3(threads), 0, st, g);
   };
+  g.splits = 1;
   if constexpr (sizeof(TA) == 2 && sizeof(TW) == 2) {
     if (g.K % 64 == 0) {
-      const TileChoice c = choose_tiles(g.M, n, g.K, g.groups);
-      g.splits = c.splits;
       auto direct = [&](auto s) { using S = decltype(s); launch(gemm_direct<T, S>, S::BM, S::BN, S::kThreadCount); };
       auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S>, S::BM, S::BN, S::kThreadCount); };
-      switch (c.kind) {
+      switch (choose_tiles(g.M, n, g.K, g.groups, split.one_order)) {
         case 0: direct(Tiles64{}); break;
         case 1: direct(Tiles128{}); break;
-        case 2: turns(Turns64{}); break;
+        case 2: direct(Wide64{}); break;
         case 3: turns(Turns96{}); break;
         case 4: turns(Turns128{}); break;
         case 5: turns(Turns192{}); break;
         case 6: turns(Turns256{}); break;
         case 7: direct(Tiles32{}); break;
-        default: direct(Tiles16{}); break;
+        case 8: direct(Few64{}); break;
+        default: direct(Few32{}); break;
       }
       return;
     }
@@ -575,28 +578,34 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   }
   if constexpr (sizeof(TA) == 4 || sizeof(TW) == 4) {
     if (g.K <= 64) {
-      g.splits = 1;
       launch(gemm_short<TA, TW, T>, 64, 64, kPfThreads);
       return;
     }
   }
-  const TileChoice c = choose_register_tiles(g.M, n, g.K, g.groups);
+  const RegisterTiles c = choose_register_tiles(g.M, n, g.K, g.groups, sizeof(TA) == 4 || sizeof(TW) == 4);
   g.splits = c.splits;
-  if (c.kind == 1) launch(gemm<TA, TW, T, 128, 128, 2>, 128, 128, kPfThreads);
+  if (c.large) launch(gemm<TA, TW, T, 128, 128, 2>, 128, 128, kPfThreads);
   else launch(gemm<TA, TW, T, 64, 64, 1>, 64, 64, kPfThreads);
 }
 
-// rows: where the rotated part of a latent attention's keys is, behind the latent.
+// rows: where the rotated part of a latent attention's keys is, behind the latent.  Two groups of waves share a workgroup's queries, except where the order
+// counts (kOneOrderTokens).
 template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
-                      hipStream_t st) {
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * kAttendGroups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
+                      bool one_order, hipStream_t st) {
+  auto launch = [&](auto kernel, int groups) {
+    hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
   };
-  if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4>);
-  else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8>);
-  else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<T, 6, 8>);
-  else launch(window_attention<T, 8, 16>);
+  auto sized = [&](auto groups) {
+    constexpr int G = decltype(groups)::value;
+    if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4, G>, G);
+    else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8, G>, G);
+    else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<T, 6, 8, G>, G);
+    else launch(window_attention<T, 8, 16, G>, G);
+  };
+  if constexpr (sizeof(T) == 2)
+    if (one_order) return sized(std::integral_constant<int, 1>{});
+  sized(std::integral_constant<int, 2>{});
 }
 
 template <class T>
@@ -607,6 +616,7 @@ int prefill(const QmkHybridArgs* a) {
   if (a->streams == 0) return prefill_plain<T>(a);
   PrefillBuffers<T> b;
   if (prefill_buffers<T>(a, a->workspace, &b) > a->workspace_bytes) return QMK_ERR_SCRATCH;
+  b.split.one_order = sizeof(T) == 2 && a->tokens <= kOneOrderTokens;
   const hipStream_t st = static_cast<hipStream_t>(a->stream);
   const int M = a->tokens, D = a->width, S = a->streams, P = a->portion_rows;
   const dim3 block(kPfThreads);
@@ -652,7 +662,7 @@ int prefill(const QmkHybridArgs* a) {
       v.a = l.uv_w; v.w = b.rows; v.ldw = width; v.M = l.heads * l.v_dim; v.out = b.vt; v.ldo = cap;
       launch_gemm<u16, T, T>(v, b.split, st);
       const Keys<T> expanded{b.kn, l.heads * l.head_dim, l.head_dim, 1};
-      launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), st);
+      launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), b.split.one_order, st);
     } else {
       const int N = W, n = l.head_dim;
       hipLaunchKernelGGL(shift_mix<T>, dim3(M), block, 0, st, b.u, l, a->slot, a->flip, M, P, D, a->width_true, a->eps, b.h.of(D));
@@ -693,15 +703,21 @@ int prefill(const QmkHybridArgs* a) {
 
 // The recurrence of a gla or delta entry over the portion, from its projections to what its output projection reads.
 template <bool DELTA>
-void run_chunks(const QmkHybridArgs* a, const ChunkArgs& g, hipStream_t st) {
+void run_chunks(const QmkHybridArgs* a, const ChunkArgs& g, bool one_order, hipStream_t st) {
   const QmkHybridLayer& l = g.layer;
-  const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens, waves = scan_waves(l.head_dim, DELTA);
+  const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens;
   hipLaunchKernelGGL(chunk_prepare<DELTA>, dim3(chunks, l.heads), dim3(kPfThreads), 0, st, g);
-  const dim3 grid(l.heads, l.v_dim / 16), block(waves * 64);
+  auto launch = [&](auto kernel, int waves) { hipLaunchKernelGGL(kernel, dim3(l.heads, l.v_dim / 16), dim3(waves * 64), 0, st, g); };
   switch (chunk_tiles(l.head_dim)) {
-    case 4: hipLaunchKernelGGL((chunk_scan<1, 4, DELTA>), grid, block, 0, st, g); break;
-    case 8: hipLaunchKernelGGL((chunk_scan<8 / scan_waves(128, DELTA), scan_waves(128, DELTA), DELTA>), grid, block, 0, st, g); break;
-    default: hipLaunchKernelGGL((chunk_scan<16 / scan_waves(256, DELTA), scan_waves(256, DELTA), DELTA>), grid, block, 0, st, g); break;
+    case 4: return launch(chunk_scan<1, 4, DELTA>, 4);
+    case 8:
+      if constexpr (!DELTA)
+        if (!one_order) return launch(chunk_scan<1, 8, DELTA>, 8);
+      return launch(chunk_scan<2, 4, DELTA>, 4);
+    default:
+      if constexpr (!DELTA)
+        if (!one_order) return launch(chunk_scan<2, 8, DELTA>, 8);
+      return launch(chunk_scan<4, 4, DELTA>, 4);
   }
 }
 
@@ -709,6 +725,7 @@ template <class T>
 int prefill_plain(const QmkHybridArgs* a) {
   PlainBuffers<T> b;
   if (plain_buffers<T>(a, a->workspace, &b) > a->workspace_bytes) return QMK_ERR_SCRATCH;
+  b.split.one_order = sizeof(T) == 2 && a->tokens <= kOneOrderTokens;
   const hipStream_t st = static_cast<hipStream_t>(a->stream);
   const int M = a->tokens, D = a->width;
   const size_t rows = static_cast<size_t>(a->portion_rows) * D;
@@ -765,7 +782,7 @@ int prefill_plain(const QmkHybridArgs* a) {
       const int row = l.head_dim + l.v_dim, pitch = l.kv_heads * row, keys = a->position + M, cap = static_cast<int>(values_cap(a));
       const T* cache = static_cast<const T*>(l.cache) + static_cast<size_t>(a->slot) * l.ring * pitch;
       hipLaunchKernelGGL(transpose_values<T>, dim3((keys + 63) / 64, (l.v_dim + 63) / 64, l.kv_heads), block, 0, st, cache, pitch, row, l.head_dim, l.v_dim, keys, cap, b.vt);
-      launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix.of(W), st);
+      launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix.of(W), b.split.one_order, st);
     } else {
       ChunkArgs c{};
       c.layer = l; c.decay = b.decay; c.chunks = b.chunks; c.out = b.o; c.M = M; c.slot = a->slot; c.flip = a->flip;
@@ -782,7 +799,7 @@ int prefill_plain(const QmkHybridArgs* a) {
         f.lda = ranks; f.out = b.gate; f.ldo = W;
         launch_gemm<T, u16, T>(f, b.split, st);
         c.qkv = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = W;
-        run_chunks<true>(a, c, st);
+        run_chunks<true>(a, c, b.split.one_order, st);
         if (l.taps > 1)
           hipLaunchKernelGGL(keep_inputs, dim3((channels + kPfThreads - 1) / kPfThreads), block, 0, st, b.qkv, l, channels, a->slot, a->flip, M);
       } else {
@@ -794,7 +811,7 @@ int prefill_plain(const QmkHybridArgs* a) {
         e.f0 = b.decay; e.ldo = keys;
         launch_gemm<T, u16, T>(e, b.split, st);
         c.qkv = b.qkv; c.values = b.qkv; c.value_ld = 2 * keys + W; c.value_at = 2 * keys;
-        run_chunks<false>(a, c, st);
+        run_chunks<false>(a, c, b.split.one_order, st);
       }
       hipLaunchKernelGGL(state_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.o, b.gate, l, M, a->eps, b.mix.of(W));
     }

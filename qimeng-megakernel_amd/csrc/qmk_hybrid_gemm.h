@@ -599,7 +599,7 @@ __device__ __forceinline__ void multiply(const Frag<u16> (&fa)[PARTS][S::kTm], c
 }
 
 // out[m][n] = sum_k a[m][k] w[n][k], bf16 x bf16 or the tokens' side in three parts, K a multiple of BK.  The weights are the matrix instruction's first operand,
-// so a lane ends up with four consecutive outputs of one token.  Four waves; several workgroups share a CU.
+// so a lane ends up with four consecutive outputs of one token.  Two to eight waves; several workgroups share a CU where LDS has room.
 template <class T, class S, int PARTS = 1>
 __global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g) {
   constexpr int kAhead = S::kStages - 1, kStageUnits = S::kStages * Stages<S, PARTS>::kUnits, kLds = kStageUnits > S::kLds ? kStageUnits : S::kLds;
@@ -831,14 +831,17 @@ __global__ __launch_bounds__(kPfThreads) void gemm_short(const GemmArgs g) {
 }
 
 // ---- which tiles ----
-using Tiles16 = Tile<64, 16, 64, 16, 16, 4, 4>;        // few tokens: weight rows of a workgroup
+// Few tokens: weight rows of a workgroup, deep steps, since a step's barrier and reads are most of its time (us, M x N x K, 64 x 16 in steps of 64 columns, of
+// 128, 32 x 16 in steps of 256: 43 x 2048 x 2048 with the residual's streams 12.2, 10.1, 9.5; 43 x 2048 x 6144 with them 26.4, 19.9, 17.3).
+using Few32 = Tile<32, 16, 256, 16, 16, 2, 4>;
+using Few64 = Tile<64, 16, 128, 16, 16, 4, 3>;
 using Tiles32 = Tile<64, 32, 64, 32, 16, 4, 4>;
 using Tiles64 = Tile<64, 64, 64, 32, 32, 4, 4>;
+using Wide64 = Tile<128, 64, 64, 32, 32, 8, 3>;
 using Tiles128 = Tile<128, 128, 64, 64, 64, 4, 2>;
 // The tokens' side in three parts: it is what fills LDS, so few tokens a tile (us, 32 x 128 and 64 x 64 and 64 x 128 and 128 x 128: 200 x 2048 x 6144
 // 32, 35, 54, 169; 200 x 12288 x 2048 52, 58, 52, 63; 2048 x 2048 x 8192 260, 420, 291, 280).
 using TilesParts = Tile<32, 128, 64, 16, 64, 4, 2>;
-using Turns64 = Tile<64, 128, 64, 32, 64, 8, 4>;
 using Turns96 = Tile<96, 128, 64, 48, 64, 8, 4>;
 using Turns128 = Tile<128, 128, 64, 64, 64, 8, 4>;
 using Turns192 = Tile<192, 256, 32, 96, 64, 8, 4>;

@@ -126,9 +126,8 @@ __global__ __launch_bounds__(kPfThreads) void transpose_values(const T* cache, i
 constexpr int kChunkTokens = 16;
 constexpr int kChunkWaves = 4;      // of chunk_prepare
 
-// Tiles of sixteen key channels of a head, the last ones zeros, and the waves of chunk_scan that share them.
+// Tiles of sixteen key channels of a head, the last ones zeros.
 __host__ __device__ constexpr int chunk_tiles(int head_dim) { return head_dim <= 64 ? 4 : head_dim <= 128 ? 8 : 16; }
-__host__ __device__ constexpr int scan_waves(int head_dim, bool delta) { return head_dim <= 64 || delta ? 4 : 8; }
 // Floats of one (chunk, head): per tile the fragments of G q, G k and D k and the decays G over the whole chunk, then B and
 // T.  A fragment is in the order the matrix instruction takes it: [lane][4].
 __host__ __device__ constexpr int chunk_floats(int head_dim) { return chunk_tiles(head_dim) * (3 * 256 + 16) + 2 * 256; }
@@ -329,8 +328,8 @@ __global__ __launch_bounds__(kPfThreads) void keep_inputs(const float* x, QmkHyb
 // so that kAhead chunks are in flight: a chunk, or token, behind the last one is the last one again, and its value is either
 // not used or multiplied by zero.
 // What bounds it is the chain of a chunk: products of the state with the keys (four dependent instructions of 32 cycles a tile), the
-// waves' sums through LDS, T (v - X), the state's update.  So the waves hold one tile each where a head has no more than
-// eight, and what only the output needs is off the chain: G q S is taken while the sums are on their way, and a chunk's outputs
+// waves' sums through LDS, T (v - X), the state's update.  So eight waves hold the tiles of a gated linear attention's heads of more than 64 channels,
+// where the order does not count (kOneOrderTokens); and what only the output needs is off the chain: G q S is taken while the sums are on their way, and a chunk's outputs
 // are added up and stored behind the next chunk's barrier.
 template <int TILES, int WAVES, bool DELTA>
 __global__ __launch_bounds__(WAVES * 64) void chunk_scan(const ChunkArgs g) {

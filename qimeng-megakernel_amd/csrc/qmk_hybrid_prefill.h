@@ -179,13 +179,12 @@ struct Keys {
 // Windowed attention over expanded keys: 64 queries of one head a workgroup (16 a wave), 32 keys a step.
 // Scores are computed transposed (keys x queries), so a lane holds eight weights of ONE query in exactly the shape the
 // value product's second operand wants, with keys in the order 4g..4g+3, 16+4g..16+4g+3.
-// Two groups of four waves take the 32-key steps in turn, for the same queries, and meet at the end: a step is a chain (keys into LDS,
+// GROUPS = 2: two groups of four waves take the 32-key steps in turn, for the same queries, and meet at the end: a step is a chain (keys into LDS,
 // scores, maximum over the lanes, weights, values), and a CU that holds one or two workgroups of four waves mostly waits for it
 // (us, one group -> two: 2048 queries of 16 heads of 128 behind 0 and 2048 keys, mean 156 -> 99; 1531 of 192 | 128 in a window of 1024
-// 70 -> 66; 43 behind 400 29 -> 19; 200 in fp32 34 -> 29.  Four groups: 121, 84, 24.)
-constexpr int kAttendGroups = 2;
-template <class T, int QT, int VT>   // most 32-column steps of a query, most 16-row tiles of a value
-__global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(const T* q, Keys<T> keys, const T* rows, const T* v_t, const T* gate, QmkHybridLayer l,
+// 70 -> 66; 43 behind 400 29 -> 19; 200 in fp32 34 -> 29.  Four groups: 121, 84, 24.)  GROUPS = 1 takes the keys in their order.
+template <class T, int QT, int VT, int GROUPS>   // most 32-column steps of a query, most 16-row tiles of a value
+__global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const T* q, Keys<T> keys, const T* rows, const T* v_t, const T* gate, QmkHybridLayer l,
                                                                int first, int position, int M, int keys_cap, Operand<T> out) {
   constexpr int kKeys = 32;
   constexpr int kPadK = 16 / sizeof(T), kPadV = 16 / sizeof(T);
@@ -193,9 +192,9 @@ __global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(c
     T k[kKeys][QT * 32 + kPadK];
     T v[VT * 16][kKeys + kPadV];
   };
-  __shared__ __align__(16) Step stage[kAttendGroups];
+  __shared__ __align__(16) Step stage[GROUPS];
   const int tid = threadIdx.x % kPfThreads, lane = tid & 63, wave = tid >> 6, g = lane >> 4, col = lane & 15;
-  const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kPfThreads);
+  const int part = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kPfThreads);
   auto& sk = stage[part].k;
   auto& sv = stage[part].v;
   // Later queries see more keys where no window ends.  Workgroups 256 apart share a CU: every other such run of heads takes
@@ -229,10 +228,10 @@ __global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(c
     k_step[i] = 0;
     if (c < l.head_dim) {
       k_at[i] = keys.at + static_cast<size_t>(row) * keys.pitch + kv * keys.head + c;
-      k_step[i] = kAttendGroups * kKeys * keys.pitch;
+      k_step[i] = GROUPS * kKeys * keys.pitch;
     } else if (c < l.head_dim + l.rot_dim) {
       k_at[i] = rows + static_cast<size_t>(row) * width + l.rank + c - l.head_dim;
-      k_step[i] = kAttendGroups * kKeys * width;
+      k_step[i] = GROUPS * kKeys * width;
     }
   }
   auto fetch = [&](int base) {
@@ -258,7 +257,7 @@ __global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(c
   };
   fetch(base0);
   const int first_pos = position + q0 + wave * 16;       // this wave's queries: first_pos .. first_pos + 15
-  for (int base = base0; base - part * kKeys < hi; base += kAttendGroups * kKeys) {      // (the groups share the barriers)
+  for (int base = base0; base - part * kKeys < hi; base += GROUPS * kKeys) {      // (the groups share the barriers)
 #pragma unroll
     for (int i = 0; i < kKLoads; ++i) {
       const int id = i * kPfThreads + tid;
@@ -270,7 +269,7 @@ __global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(c
       *reinterpret_cast<v4u*>(&sv[id / (kKeys / kU)][id % (kKeys / kU) * kU]) = rv[i];
     }
     __syncthreads();
-    if (base + kAttendGroups * kKeys < hi) fetch(base + kAttendGroups * kKeys);
+    if (base + GROUPS * kKeys < hi) fetch(base + GROUPS * kKeys);
     if (base < hi) {
       f32x4 d[2] = {};
 #pragma unroll
@@ -296,15 +295,15 @@ __global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(c
       best = fmaxf(best, __shfl_xor(best, 32));
       const float ref = best == -INFINITY ? 0.f : best;      // no key of this query yet
       const float shrink = exp2_fast(top - ref);
-      float part = 0.f;
+      float step_sum = 0.f;
       Frag<T> fp;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         w[j] = exp2_fast(w[j] - ref);
-        part += w[j];
+        step_sum += w[j];
         fp.set(j, from_f32<T>(w[j]));
       }
-      sum = sum * shrink + part;
+      sum = sum * shrink + step_sum;
       top = best;
 #pragma unroll
       for (int t = 0; t < VT; ++t)
@@ -323,20 +322,19 @@ __global__ __launch_bounds__(kPfThreads * kAttendGroups) void window_attention(c
   }
   sum += __shfl_xor(sum, 16);
   sum += __shfl_xor(sum, 32);
-  // The second group's maximum, sum and values of every lane's query onto the first one's.
-  float* box = reinterpret_cast<float*>(stage) + tid;
-  static_assert(kAttendGroups == 2 && sizeof(stage) >= sizeof(float) * (VT * 4 + 2) * kPfThreads, "the giving group's states");
-  if (part == 1) {
-    box[0] = top;
-    box[kPfThreads] = sum;
+  if constexpr (GROUPS == 2) {      // the second group's maximum, sum and values of every lane's query onto the first one's
+    float* box = reinterpret_cast<float*>(stage) + tid;
+    static_assert(sizeof(stage) >= sizeof(float) * (VT * 4 + 2) * kPfThreads, "the giving group's states");
+    if (part == 1) {
+      box[0] = top;
+      box[kPfThreads] = sum;
 #pragma unroll
-    for (int t = 0; t < VT; ++t)
+      for (int t = 0; t < VT; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) box[(2 + t * 4 + i) * kPfThreads] = acc[t][i];
-  }
-  __syncthreads();
-  if (part == 1) return;
-  {
+        for (int i = 0; i < 4; ++i) box[(2 + t * 4 + i) * kPfThreads] = acc[t][i];
+    }
+    __syncthreads();
+    if (part == 1) return;
     const float other = box[0], most = fmaxf(top, other), ref = most == -INFINITY ? 0.f : most, mine = exp2_fast(top - ref), theirs = exp2_fast(other - ref);
     sum = sum * mine + box[kPfThreads] * theirs;
 #pragma unroll
