@@ -151,7 +151,8 @@ typedef struct QmkHybridArgs {
   float* logits;                /* decode [vocab_rows]; prefill [num_want][vocab_rows] */
   float* layer_out;             /* prefill: sum of the streams behind each layer [num_layers][tokens][D], or the plain residual
                                    behind each layer run [runs][tokens][D], or NULL */
-  void* workspace;              /* qmk_hybrid_decode_bytes / qmk_hybrid_prefill_bytes, 256-byte aligned, zeroed once */
+  void* workspace;              /* qmk_hybrid_decode_bytes / qmk_hybrid_prefill_bytes, 256-byte aligned, zeroed once; nothing in it
+                                   is kept between launches, so that launches one after the other may share it */
   uint64_t workspace_bytes;
   /* decode only */
   const int32_t* instructions;  /* [num_queues][num_insts][32] */

@@ -322,8 +322,7 @@ size_t decode_buffers(const QmkHybridArgs* a, void* base, DecodeBuffers* b) {
 
 inline size_t values_cap(const QmkHybridArgs* a) { return (static_cast<size_t>(a->max_positions) + 31) & ~size_t(31); }
 
-// Parts of products that are cut along K: the head of every prefill workspace, so that a workspace that serves launches of
-// different sizes keeps its tickets, zero between products, in one place.
+// Parts of products that are cut along K (fp32 mode).  The tickets are zero at a portion's start (begin_portion) and after every product.
 struct SplitBuffers {
   int32_t* tickets;
   f32x4* partial;
@@ -588,6 +587,13 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   else launch(gemm<TA, TW, T, 64, 64, 1>, 64, 64, kPfThreads);
 }
 
+// Ahead of a portion's other launches.
+template <class T>
+void begin_portion(const QmkHybridArgs* a, SplitBuffers& split, hipStream_t st) {
+  split.one_order = sizeof(T) == 2 && a->tokens <= kOneOrderTokens;
+  if constexpr (sizeof(T) == 4) hipLaunchKernelGGL(clear_tickets, dim3(1), dim3(kPfThreads), 0, st, split.tickets, kMaxTickets);
+}
+
 // rows: where the rotated part of a latent attention's keys is, behind the latent.  Two groups of waves share a workgroup's queries, except where the order
 // counts (kOneOrderTokens).
 template <class T>
@@ -616,8 +622,8 @@ int prefill(const QmkHybridArgs* a) {
   if (a->streams == 0) return prefill_plain<T>(a);
   PrefillBuffers<T> b;
   if (prefill_buffers<T>(a, a->workspace, &b) > a->workspace_bytes) return QMK_ERR_SCRATCH;
-  b.split.one_order = sizeof(T) == 2 && a->tokens <= kOneOrderTokens;
   const hipStream_t st = static_cast<hipStream_t>(a->stream);
+  begin_portion<T>(a, b.split, st);
   const int M = a->tokens, D = a->width, S = a->streams, P = a->portion_rows;
   const dim3 block(kPfThreads);
   hipLaunchKernelGGL(embed_tokens, dim3(M), block, 0, st, a->embed, a->token_in, a->vocab, a->layers[0].hc, S, D, b.x, b.u);
@@ -725,8 +731,8 @@ template <class T>
 int prefill_plain(const QmkHybridArgs* a) {
   PlainBuffers<T> b;
   if (plain_buffers<T>(a, a->workspace, &b) > a->workspace_bytes) return QMK_ERR_SCRATCH;
-  b.split.one_order = sizeof(T) == 2 && a->tokens <= kOneOrderTokens;
   const hipStream_t st = static_cast<hipStream_t>(a->stream);
+  begin_portion<T>(a, b.split, st);
   const int M = a->tokens, D = a->width;
   const size_t rows = static_cast<size_t>(a->portion_rows) * D;
   const dim3 block(kPfThreads);

@@ -385,6 +385,12 @@ __device__ __forceinline__ bool sum_parts(const GemmArgs& g, int tile, int part,
   return true;
 }
 
+// The first launch of a portion whose products are cut: a workspace may have held something else since the one before, and a ticket that is not
+// zero would leave a product without its last part.
+__global__ __launch_bounds__(kPfThreads) void clear_tickets(int32_t* tickets, int count) {
+  for (int i = threadIdx.x; i < count; i += kPfThreads) tickets[i] = 0;
+}
+
 // All streams of the residual for quads id, id + step, .. of a tile: the next quad's streams are asked for before this one's
 // are mixed.
 template <class At, class Value>

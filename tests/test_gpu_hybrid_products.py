@@ -62,3 +62,24 @@ def test_values_that_are_not_finite_stay_so_in_fp32(width, channels):
     got = decode_hybrid.run_tokens(g, mk_kernel.get_mk(), RequestTable(g).open(0), ids, range(40))
     assert torch.isfinite(got[:20]).all()
     assert not torch.isfinite(got[20]).any() and not torch.isfinite(got[30]).any()
+
+
+@pytest.mark.parametrize("byte", [0x01, 0xFF], ids=["ones", "undefined values"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("shape", [SHAPES["large"], synthetic.looped_shape("pg", width=2048, vocab=96, ff={"p": 2048}, heads=2, kv_heads=1, delta_heads=2,
+                                                                          delta_kv_heads=1, gla_heads=2)], ids=["streams", "plain"])
+def test_a_workspace_that_has_held_something_else(shape, dtype, byte):
+    """Decode and prefill launches may share a buffer: nothing a launch finds in it counts."""
+    g = build_globals(shape, weights.pack(shape, synthetic.random_hybrid_weights(shape, 4, DEVICE), DEVICE), dtype=dtype, max_positions=64, portion_rows=64)
+    mk, tokens, got = mk_kernel.get_mk(), torch.arange(40) % shape.vocab, []
+    for fill in (0, byte):
+        table = RequestTable(g)
+        request, parts = table.open(0), []
+        for part in tokens.split([20, 1, 18, 1]):
+            if got:
+                mk._prefill_ws.fill_(fill)
+                mk._decode_ws.fill_(fill)
+            parts.append(decode_hybrid.run_tokens(g, mk, request, part, range(len(part))))
+        mk.check()
+        got.append(torch.cat(parts))
+    assert torch.isfinite(got[0]).all() and torch.equal(got[0], got[1])
