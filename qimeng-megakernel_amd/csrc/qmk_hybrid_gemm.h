@@ -29,10 +29,10 @@ enum : int {
   EPI_GLA_DECAY,
 };
 
-// An fp32 value is the sum of three bf16 values that take its significand's bits 23..16, 15..8 and 7..0 (exactly: every
-// remainder is exact, and the exponents are the same), and a product of two bf16 values is exact in fp32: three bf16 instructions
-// add up the same products as the eight fp32 ones of the same columns, in a fifth of their time.  Values that are not finite
-// stay whole in the first part.
+// An fp32 value is the sum of three bf16 values of its sign: its upper half, the upper half of what that leaves, and the rest, which has eight
+// bits at most.  Both remainders are exact, so the sum is, from 2^-110 on (below, what is smaller than bf16's smallest value, 2^-133, is cut off).  A
+// product of two bf16 values is exact in fp32: three bf16 instructions add up the same products as the eight fp32 ones of the same
+// columns, in a fifth of their time.  Values that are not finite stay whole in the first part; infinite values on the other side: resolve_undefined.
 __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
   return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
@@ -604,6 +604,27 @@ __device__ __forceinline__ void multiply(const Frag<u16> (&fa)[PARTS][S::kTm], c
     }
 }
 
+// An infinite value on the bf16 side makes products with those parts of a finite value that are zero undefined, where the product with the whole
+// value is infinite.  A sum that came out undefined is therefore taken again, of first parts alone, which are zero or not finite where the
+// values are; nothing else can have made it so that does not make it so again.  `a`, `w`: fragments of first parts, tile i and 32 columns from k.
+template <class S, class A, class W>
+__device__ __forceinline__ void resolve_undefined(const Place& p, f32x4 (&acc)[S::kTn][S::kTm], A&& a, W&& w) {
+  static_assert(S::kGroups == 1, "a wave takes all columns");
+#pragma unroll
+  for (int j = 0; j < S::kTn; ++j)
+#pragma unroll
+    for (int i = 0; i < S::kTm; ++i) {
+      f32x4& v = acc[j][i];
+      if (__builtin_expect(__any(v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]), 0)) {
+        f32x4 t = {};
+#pragma unroll 1
+        for (int k = p.first * S::BK; k < (p.first + p.steps) * S::BK; k += 32) t = mma(w(j, k), a(i, k), t);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = v[e] != v[e] ? t[e] : v[e];
+      }
+    }
+}
+
 // out[m][n] = sum_k a[m][k] w[n][k], bf16 x bf16 or the tokens' side in three parts, K a multiple of BK.  The weights are the matrix instruction's first operand,
 // so a lane ends up with four consecutive outputs of one token.  Two to eight waves; several workgroups share a CU where LDS has room.
 template <class T, class S, int PARTS = 1>
@@ -634,6 +655,12 @@ __global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g)
       multiply<S, PARTS>(fa, fw, acc);
     }
     buf = buf + 1 == S::kStages ? 0 : buf + 1;
+  }
+  if constexpr (PARTS > 1) {
+    const u16 *a = static_cast<const u16*>(g.a) + p.group * g.a_step + (lane >> 4) * 8, *w = static_cast<const u16*>(g.w) + p.group * g.w_step + (lane >> 4) * 8;
+    resolve_undefined<S>(
+        p, acc, [&](int i, int k) { return load_frag(a + static_cast<size_t>(min(p.m0 + wm * S::WM + i * 16 + (lane & 15), g.M - 1)) * g.lda + k); },
+        [&](int j, int k) { return load_frag(w + static_cast<size_t>(min(p.n0 + wn * S::WN + j * 16 + (lane & 15), p.N - 1)) * g.ldw + k); });
   }
   finish_tile<T, S, kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
@@ -792,6 +819,32 @@ __global__ __launch_bounds__(kPfThreads) void gemm(const GemmArgs g) {
     if (BUFFERS == 1) __syncthreads();
     if (s + 1 < p.steps) stash(BUFFERS == 2 ? (s + 1) & 1 : 0);
     __syncthreads();
+  }
+  if constexpr (kPa * kPw > 1) {
+    auto first_part = [&](auto* base, int row, int rows, long long ld, int k) {      // (K is a multiple of the units a row is read in)
+      constexpr int kUnit = 16 / sizeof(*base);
+      const auto* from = base + static_cast<size_t>(min(row, rows - 1)) * ld;
+      k += (lane >> 4) * 8;
+      v4u unit = {0u, 0u, 0u, 0u};
+      if constexpr (kUnit == 8) {
+        if (k < g.K) unit = *reinterpret_cast<const v4u*>(from + k);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          if (k + e * kUnit < g.K) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(from + k + e * kUnit);
+            uint32_t lo[3], hi[3];
+            split2(x[0], x[1], lo);
+            split2(x[2], x[3], hi);
+            unit[2 * e] = lo[0];
+            unit[2 * e + 1] = hi[0];
+          }
+      }
+      return Frag<u16>{__builtin_bit_cast(bf16x8_t, unit)};
+    };
+    resolve_undefined<S>(
+        p, acc, [&](int i, int k) { return first_part(a, p.m0 + wm * S::WM + i * 16 + (lane & 15), g.M, g.lda, k); },
+        [&](int j, int k) { return first_part(w, p.n0 + wn * S::WN + j * 16 + (lane & 15), p.N, g.ldw, k); });
   }
   finish_tile<T, S, kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }

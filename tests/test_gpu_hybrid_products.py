@@ -64,6 +64,20 @@ def test_values_that_are_not_finite_stay_so_in_fp32(width, channels):
     assert not torch.isfinite(got[20]).any() and not torch.isfinite(got[30]).any()
 
 
+@pytest.mark.parametrize("width", [208, 256, 704], ids=["whole", "parts", "parts, cut"])
+def test_infinite_weights_in_fp32(width):
+    """A finite value times an infinite weight is infinite, also where some of the value's three parts are zero."""
+    shape = synthetic.hybrid_shape("r", width=width, vocab=160, streams=2, lru_width=96, blocks=1, taps=3)
+    w = synthetic.random_hybrid_weights(shape, 6)
+    for i in range(shape.vocab):
+        w["head"][i, i] = float("inf") if i % 3 else -float("inf")
+    ids = torch.randint(0, shape.vocab, (130,), generator=torch.Generator().manual_seed(2))
+    g = build_globals(shape, weights.pack(shape, w, DEVICE), dtype=torch.float32, max_positions=160, portion_rows=160)
+    got = decode_hybrid.run_tokens(g, mk_kernel.get_mk(), RequestTable(g).open(0), ids, range(130)).cpu()
+    want = O.forward(shape.to_config(), w, ids, dtype=torch.float64)
+    assert torch.isinf(want).all() and torch.equal(got.double(), want)
+
+
 @pytest.mark.parametrize("byte", [0x01, 0xFF], ids=["ones", "undefined values"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("shape", [SHAPES["large"], synthetic.looped_shape("pg", width=2048, vocab=96, ff={"p": 2048}, heads=2, kv_heads=1, delta_heads=2,
