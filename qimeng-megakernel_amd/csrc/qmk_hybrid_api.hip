@@ -595,7 +595,8 @@ void begin_portion(const QmkHybridArgs* a, SplitBuffers& split, hipStream_t st) 
 }
 
 // rows: where the rotated part of a latent attention's keys is, behind the latent.  Two groups of waves share a workgroup's queries, except where the order
-// counts (kOneOrderTokens).
+// counts (kOneOrderTokens) and in fp32 with the largest heads, whose two groups take 140 KB of LDS and more registers than there are (us a portion of one
+// layer, 16 heads of 256 | 256, one group -> two: fp32 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508; bf16 1141 -> 728, 194 -> 156).
 template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
                       bool one_order, hipStream_t st) {
@@ -603,11 +604,11 @@ void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* 
     hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
   };
   auto sized = [&](auto groups) {
-    constexpr int G = decltype(groups)::value;
+    constexpr int G = decltype(groups)::value, kLargest = sizeof(T) == 4 ? 1 : G;
     if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4, G>, G);
     else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8, G>, G);
     else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<T, 6, 8, G>, G);
-    else launch(window_attention<T, 8, 16, G>, G);
+    else launch(window_attention<T, 8, 16, kLargest>, kLargest);
   };
   if constexpr (sizeof(T) == 2)
     if (one_order) return sized(std::integral_constant<int, 1>{});
