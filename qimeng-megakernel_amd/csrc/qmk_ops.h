@@ -1145,7 +1145,7 @@ __device__ bool op_oproj_residual(const Params& p, Smem<M>& s, const Ctx& c, Car
   parked = parked && carried && M::PARK_ROWS > 0;
   if (parked) park_upgate_rows<M>(p, s, s.next, layer, lane, c.tid >> 6);
   const int self_merge = s.inst[5];  // reduction_block_idx: 0, or the split-KV fan-out P when this op merges
-  const bool merged = self_merge > 0 && self_merge <= kMaxSelfMerge && last_slice_merges<M>(p, self_merge);
+  const bool merged = self_merge > 0 && self_merge <= min(kMaxSelfMerge, p.max_splits) && last_slice_merges<M>(p, self_merge);
   if (__builtin_expect(self_merge == 0 || merged, 0)) {
     if (merged) {
       if (!wg_wait_all(p, s, c, layer, ROW_REDUCE, 0, M::NKV * self_merge)) return false;

@@ -44,3 +44,21 @@ def test_last_slice_merges_to_the_same_bits(model, slices, position, xcd):
         done.append(g)
     for name in BUFFERS:
         assert torch.equal(getattr(done[0], name), getattr(done[1], name)), name
+
+
+def test_a_fan_out_beyond_the_workspace_is_rejected():
+    """As where the O-projection reads the partials itself: an operand error, not a wait that runs out."""
+    shape = dataclasses.replace(LLAMA_3_2_1B, num_hidden_layers=1, vocab_size=512)
+    LlamaConfig.set_shape(shape)
+    g = synthetic.build_globals(synthetic.random_weights(shape, 5, 64), shape, 64, "cuda:0")
+    mk = mk_kernel.get_mk(tagged=True, spin_limit=20000)
+    S.tensorize_instructions(g, S.mi355x_scheduler(shape, num_partials=8).queues())
+    oproj = g.instructions[:, :, 0] == 4
+    assert set(g.instructions[..., 5][oproj].tolist()) == {8} and (splits := g.attn_lse_intermediates.shape[1]) < 64
+    g.instructions[..., 5][oproj] = splits + 1
+    g.position_id = 40
+    mk_kernel.call_mk(g, mk)
+    assert mk._tagged
+    with pytest.raises(RuntimeError, match="operand out of bounds") as err:
+        mk.check()
+    assert "opcode=4" in str(err.value) and "operand=5" in str(err.value)
