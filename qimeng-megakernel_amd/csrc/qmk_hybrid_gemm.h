@@ -3,6 +3,7 @@
 #pragma once
 
 #include "qmk_hybrid_ops.h"
+#include "qmk_hybrid_tiles.h"
 
 namespace qmk {
 namespace hybrid {
@@ -905,9 +906,6 @@ using Turns96 = Tile<96, 128, 64, 48, 64, 8, 4>;
 using Turns128 = Tile<128, 128, 64, 64, 64, 8, 4>;
 using Turns192 = Tile<192, 256, 32, 96, 64, 8, 4>;
 using Turns256 = Tile<256, 256, 32, 128, 64, 8, 4>;
-
-constexpr int kMaxTickets = 512;                       // tiles of a product that is cut along K
-constexpr int kPartialUnits = 256 * 128 * 128 / 4;     // quads its parts leave: 256 of 128 x 128, or as many values
 
 }  // namespace hybrid
 }  // namespace qmk

@@ -1,0 +1,87 @@
+// Which tiles a product of the hybrid route's prefill takes: rules of the host, over sizes alone.
+#pragma once
+
+namespace qmk {
+namespace hybrid {
+
+constexpr int kMaxTickets = 512;                       // tiles of a product that is cut along K
+constexpr int kPartialUnits = 256 * 128 * 128 / 4;     // quads its parts leave: 256 of 128 x 128, or as many values
+
+// A portion of so many tokens in bf16, or fewer, is computed in one order, whatever its tiles: the columns of a product one after the other (no
+// group of waves takes half of them, no workgroup a part), an attention's keys by one group of waves, a head's key channels by four waves.  Some tokens
+// are ill-conditioned (the norm over a recurrence's first output leaves little but the sign of a sum that may be close to zero, and some later tokens
+// come close to that), so that a sum taken in another order is enough to change what they leave in the states; a long portion averages that out.  Largest
+// relative difference of a state, cache or logits between two orders, 24 sets of weights of each of four shapes (width 2048): 2 tokens 0.31, 34
+// 0.065, 100 0.077, 256 0.050, 512 0.038, 700 0.033, 1000 0.026, 1531 0.024; the median is 0.008 to 0.024 at every length.
+constexpr int kOneOrderTokens = 1024;
+
+// The tiles of a bf16 product.  It takes as many rounds as its tiles fill the chip, `slots` at a time, each about `step` us for 2048 columns and `fixed` us
+// besides, and `overlapped` us once.  Fitted to measurements of every kind at 20 to 2048 tokens and 11 of the N x K of the four shapes (weights from
+// memory); the kind that comes out cheapest takes 1.1 % longer than the best one on the average up to 1024 tokens, 1.6 % beyond.  us, M x N x K,
+// the kinds around the line: 43 x 2048 x 2048 with the residual's streams Few32 9.3, Few64 10.0, Tiles32 14.1; 128 x 2048 x 4096 Few64 14, Tiles64 23; 300 x 5696 x 2048
+// Tiles64 18.5, Wide64 17; 1024 x 2048 x 6144 with the streams Wide64 55, Tiles128 116; 2048 x 16384 x 2048 Turns256 137, Tiles128 155; 2048 x 2048 x 8192 Turns128 76,
+// Wide64 100; 4096 x 2048 x 8192 Tiles128 159, Turns192 186, Turns128 189 (with the streams 192, 216, 214), 4096 x 2048 x 2048 with them 99, 117, 103.  Epilogues are not
+// priced, they are the same for all kinds; nor is memory, which bounds all of them alike where there are many rows for few tokens (1 x 128256 x 2048 Tiles32 95, Tiles64
+// 99, Tiles128 124).
+struct TileCost {
+  int most_tokens, bm, bn, bk, slots;
+  double step, fixed, overlapped;
+  bool one_order;
+};
+constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 10;
+constexpr TileCost kTileCosts[kTileKinds] = {
+    {kAnyTokens, 64, 64, 64, 256, 8.0, 0.0, 6.1, true},        // Tiles64
+    {kAnyTokens, 128, 128, 64, 512, 27.0, 8.0, 0.0, true},     // Tiles128
+    {kAnyTokens, 128, 64, 64, 256, 11.3, 0.0, 6.5, true},      // Wide64
+    {kAnyTokens, 96, 128, 64, 256, 14.7, 5.4, 3.0, false},     // Turns96
+    {kAnyTokens, 128, 128, 64, 256, 16.9, 6.2, 3.0, false},    // Turns128
+    {kAnyTokens, 192, 256, 32, 256, 38.3, 13.1, 0.0, true},    // Turns192
+    {kAnyTokens, 256, 256, 32, 256, 43.0, 14.2, 0.0, true},    // Turns256
+    {128, 64, 32, 64, 512, 7.3, 0.7, 4.3, true},               // Tiles32
+    {256, 64, 16, 128, 512, 5.8, 2.0, 2.3, true},              // Few64
+    {64, 32, 16, 256, 256, 3.9, 1.3, 3.6, true},               // Few32
+};
+inline int choose_tiles(int M, int N, int K, int groups, bool one_order) {
+  int best = 0;
+  double least = 0.;
+  for (int kind = 0; kind < kTileKinds; ++kind) {
+    const TileCost& t = kTileCosts[kind];
+    if (M > t.most_tokens || K % t.bk != 0 || (one_order && !t.one_order)) continue;
+    const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * groups;
+    const double us = static_cast<double>((tiles + t.slots - 1) / t.slots) * (t.step * K / 2048. + t.fixed) + t.overlapped;
+    if (kind == 0 || us < least) {
+      least = us;
+      best = kind;
+    }
+  }
+  return best;
+}
+
+// The same for products with an fp32 side, or of columns that are no multiple of 64: tiles of 128 x 128 where there are tokens for them and they
+// fill the chip already, else of 64 x 64, with an fp32 side cut along K until they fill it four times over (us, 64 -> 128: 1 x 65536 x 2048
+// 94 -> 150, 200 x 12288 x 2048 62 -> 76, 2048 x 16384 x 2048 829 -> 589).
+struct RegisterTiles {
+  bool large = false;
+  int splits = 1;
+};
+inline RegisterTiles choose_register_tiles(int M, int N, int K, int groups, bool cut) {
+  RegisterTiles c;
+  const long long large = static_cast<long long>((M + 127) / 128) * ((N + 127) / 128) * groups, small = static_cast<long long>((M + 63) / 64) * ((N + 63) / 64) * groups;
+  c.large = M >= 512 && large >= 256;
+  if (c.large || !cut) return c;
+  while (c.splits < 8 && small * c.splits < 512 && K / c.splits >= 512 && small <= kMaxTickets && small * c.splits * 2 * 64 * 64 / 4 <= kPartialUnits) c.splits *= 2;
+  return c;
+}
+
+// Products whose tokens' side is in parts, cut along K until every CU has a workgroup (us, in 1, 2, 4, 8: 200 x 2048 x 6144 75, 44, 32, 42;
+// 200 x 5696 x 2048, 315 tiles 31, 39, 42; 20 x 12288 x 2048 24, 19, 18, 25).
+constexpr int kPartTileTokens = 32, kPartTileRows = 128;
+inline int choose_part_splits(int M, int N, int K, int groups) {
+  const long long tiles = static_cast<long long>((M + kPartTileTokens - 1) / kPartTileTokens) * ((N + kPartTileRows - 1) / kPartTileRows) * groups;
+  int splits = 1;
+  while (splits < 8 && tiles * splits < 256 && K / splits >= 512) splits *= 2;
+  return splits;
+}
+
+}  // namespace hybrid
+}  // namespace qmk

@@ -1,12 +1,14 @@
-"""The prefill's matrix products over the sizes at which their tiles change (csrc/qmk_hybrid_gemm.h, ``choose_tiles``): one
-layer of each mixer at a width where every kind of tile is taken, cut along K or not, against the plain implementation in 64 bits.
+"""The prefill's matrix products over the sizes at which their tiles change (csrc/qmk_hybrid_tiles.h): layers of every mixer at widths and
+lengths where every kind of tile is taken, with tokens and rows of weights it does not divide, cut along K or not (test_hybrid_tiles.py
+holds that list against the rules), against the plain implementation in 64 bits.
 
-Tolerances as in test_gpu_hybrid.py: fp32 at rounding level, bf16 at bf16's."""
+Tolerances as in test_gpu_hybrid.py and, on a plain residual, test_gpu_looped.py: fp32 at rounding level, bf16 at bf16's."""
 import functools
 
 import pytest
 import torch
 
+import givopel_oracle
 import hybrid_oracle as O
 from qimeng_megakernel_amd import decode_hybrid, synthetic
 from qimeng_megakernel_amd.decode_schedule_hybrid import mk_kernel, weights
@@ -17,11 +19,17 @@ pytestmark = pytest.mark.gpu
 
 DEVICE = "cuda:0"
 TOL = {torch.float32: 2e-5, torch.bfloat16: 4e-2}
+TOL_PLAIN = {torch.float32: 4e-5, torch.bfloat16: 8e-2}
 MOST = 1540
-#: feed-forwards of a size that fills the large tiles, and of one no tile divides
+#: lengths at which some product of some shape changes its tiles, and odd ones
+LENGTHS = (2, 16, 40, 63, 65, 129, 200, 257, 520, 1024, 1100, 1531, MOST)
+#: feed-forwards of a size that fills the large tiles, and of one no tile divides; every mixer, with columns in multiples of 64 and not
 SHAPES = {
     "large": synthetic.hybrid_shape("a", width=2048, vocab=640, streams=2, ff={"a": 4096}, heads=8, dim=128, rot_dim=64, v_dim=128, rank=256, window=512),
     "ragged": synthetic.hybrid_shape("a", width=1104, vocab=336, streams=3, ff={"a": 1744}, heads=3, dim=80, rot_dim=32, v_dim=112, rank=144, window=77),
+    "recurrent": synthetic.hybrid_shape("rw", width=1088, vocab=336, streams=2, ff={"r": 2872, "w": 1936}, lru_width=1280, blocks=5, taps=4, wkv_heads=17, wkv_dim=64, wkv_rank=96),
+    "plain": synthetic.looped_shape("pgp", width=2048, vocab=336, ff={"p": 4040, "g": 2856}, loop=(1, 2, 2), heads=4, kv_heads=2, delta_heads=4, delta_kv_heads=2,
+                                    delta_rank=144, gate_rank=72, gla_heads=2, gla_rank=80),
 }
 
 
@@ -31,11 +39,12 @@ def expected(name):
     w = synthetic.random_hybrid_weights(shape, 3, DEVICE)
     tokens = torch.randint(0, shape.vocab, (MOST,), generator=torch.Generator().manual_seed(5))
     with torch.device(DEVICE):
-        return w, tokens, O.forward(shape.to_config(), w, tokens.to(DEVICE), dtype=torch.float64)     # causal: a prefix's logits are its rows
+        oracle = givopel_oracle if shape.plain else O
+        return w, tokens, oracle.forward(shape.to_config(), w, tokens.to(DEVICE), dtype=torch.float64)     # causal: a prefix's logits are its rows
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("n", [2, 16, 63, 65, 129, 200, 520, 1024, MOST])
+@pytest.mark.parametrize("n", LENGTHS)
 @pytest.mark.parametrize("name", sorted(SHAPES))
 def test_products_at_the_edges_of_tiles(name, n, dtype):
     shape = SHAPES[name]
@@ -45,7 +54,7 @@ def test_products_at_the_edges_of_tiles(name, n, dtype):
     d = got - want[:n]
     d = d - d.mean(-1, keepdim=True)
     err = float((d.pow(2).mean(-1).sqrt() / want[:n].pow(2).mean().sqrt()).max())
-    assert err < TOL[dtype], f"{err:.3g}"
+    assert err < (TOL_PLAIN if shape.plain else TOL)[dtype], f"{err:.3g}"
 
 
 @pytest.mark.parametrize("width,channels", [(208, 160), (256, 192)], ids=["whole", "parts"])

@@ -1,0 +1,103 @@
+"""The rules that choose a prefill product's tiles (csrc/qmk_hybrid_tiles.h, compiled for the host): what the GPU tests of the products reach, and properties that
+hold for any size."""
+import random
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+from test_gpu_hybrid_products import LENGTHS, SHAPES
+
+KINDS = ("Tiles64", "Tiles128", "Wide64", "Turns96", "Turns128", "Turns192", "Turns256", "Tiles32", "Few64", "Few32")
+IN_ORDER = set(KINDS) - {"Turns96", "Turns128"}
+MOST_IN_ORDER = 1024
+DRIVER = """
+#include <stdio.h>
+#include "qmk_hybrid_tiles.h"
+using namespace qmk::hybrid;
+int main() {
+  int M, N, K, groups, flag;
+  while (scanf("%d %d %d %d %d", &M, &N, &K, &groups, &flag) == 5) {
+    const RegisterTiles r = choose_register_tiles(M, N, K, groups, flag);
+    const int kind = K % 64 ? -1 : choose_tiles(M, N, K, groups, flag);
+    printf("%d %d %d %d %d %d %d\\n", kind, kind < 0 ? 1 : kTileCosts[kind].bm, kind < 0 ? 1 : kTileCosts[kind].bn, kind < 0 ? 1 : kTileCosts[kind].bk, choose_part_splits(M, N, K, groups),
+           r.large, r.splits);
+  }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def choose(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("tiles")
+    (folder / "driver.cpp").write_text(DRIVER)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", f"-I{ROOT / 'qimeng-megakernel_amd' / 'csrc'}", "-o", str(folder / "driver"), str(folder / "driver.cpp")], check=True)
+
+    def run(sizes):
+        """(kind, its rows of tokens, of weights, its columns, cuts of parts, whether register tiles are large, their cuts) of (M, N, K, groups, flag); the flag: in
+        one order, and for register tiles whether there is an fp32 side."""
+        text = "".join("%d %d %d %d %d\n" % s for s in sizes)
+        out = subprocess.run([str(folder / "driver")], input=text, capture_output=True, text=True, check=True).stdout
+        return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+    return run
+
+
+def products(shape, n):
+    """(M, N, K, groups, whether its tokens' side may be in parts) of every product of a portion of n tokens from a request's start."""
+    D, found = shape.width_s, []
+    for e in shape.entries:
+        l = e.shape
+        if e.type == "join":
+            found.append((n, D, 2 * D, 1, True))
+        if e.type in ("join", "final"):
+            continue
+        if e.type == "wkv":
+            found += [(n, max(l.mix_width, l.rank_s), D, 5, True), (n, l.mix_width, l.rank_s, 1, False)]
+        else:
+            found.append((n, l.in_rows, D, 1, True))
+        if e.type == "rglru":
+            found.append((n, 2 * l.block_s, l.block_s, l.blocks, False))
+        elif e.type == "latent_attention":
+            found += [(n, l.heads * l.dim_s, l.rank_s, 1, False), (l.heads * l.v_s, n, l.rank_s, 1, False)]
+        elif e.type in ("delta", "gla"):
+            found.append((n, l.heads * l.dim_s, l.rank_s, 1, False))
+            if e.type == "delta":
+                found.append((n, l.mix_width, l.gate_rank_s, 1, False))
+        found.append((n, D, l.mix_width, 1, True))
+        ff = (16 * -(-e.ff // 16)) if e.ff else 0
+        if ff:
+            found += [(n, 2 * ff, D, 1, True), (n, D, ff, 1, True)]
+    return found + [(n, shape.vocab_s, D, 1, True)]
+
+
+def test_the_gpu_tests_reach_every_kind_of_tile(choose):
+    tiles, parts, register = {}, set(), set()
+    for name, shape in SHAPES.items():
+        for n in LENGTHS:
+            sizes = products(shape, n)
+            for (M, N, K, groups, _), (kind, bm, bn, *_) in zip(sizes, choose([s[:4] + (n <= MOST_IN_ORDER,) for s in sizes])):
+                if kind >= 0:
+                    tiles.setdefault(KINDS[kind], set()).update(side for side, over in (("tokens", M % bm), ("rows", N % bn)) if over)
+            for (M, N, K, groups, may), (*_, cuts, large, small_cuts) in zip(sizes, choose([s[:4] + (1,) for s in sizes])):
+                if may and K > 64 and K % 64 == 0:
+                    parts.add(cuts)
+                elif K > 64:
+                    register.add("large" if large else small_cuts)
+    # with tokens and rows of weights that they do not divide (rows come in sixteens, which Few32 and Few64 always divide)
+    assert tiles == {kind: {"tokens", "rows"} if "Few" not in kind else {"tokens"} for kind in KINDS}
+    assert parts == {1, 2, 4, 8} and register == {"large", 1, 2, 4, 8}
+
+
+def test_rules_hold_for_any_size(choose):
+    rng = random.Random(1)
+    sizes = [(int(2 ** rng.uniform(0, 13)), 16 * int(2 ** rng.uniform(0, 14)), 16 * int(2 ** rng.uniform(0, 10.5)), rng.choice((1, 1, 5, 10)), rng.randint(0, 1)) for _ in range(4000)]
+    for (M, N, K, groups, flag), (kind, bm, bn, bk, cuts, large, small_cuts) in zip(sizes, choose(sizes)):
+        if kind >= 0:
+            assert K % bk == 0 and (not flag or KINDS[kind] in IN_ORDER)
+        # what is cut has room for its tickets and sums, and every part has columns of its own
+        for tiles, per, c in ((-(-M // 32) * -(-N // 128) * groups, 32 * 128, cuts), (-(-M // 64) * -(-N // 64) * groups, 64 * 64, small_cuts)):
+            if c > 1:
+                assert tiles <= 512 and tiles * c * per // 4 <= 256 * 128 * 128 // 4 and K // c >= 256
+        assert flag or small_cuts == 1
+        assert not large or small_cuts == 1
