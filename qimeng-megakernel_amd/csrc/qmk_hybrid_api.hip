@@ -484,7 +484,7 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
     if (g.K % 64 == 0) {
       auto direct = [&](auto s) { using S = decltype(s); launch(gemm_direct<T, S>, S::BM, S::BN, S::kThreadCount); };
       auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S>, S::BM, S::BN, S::kThreadCount); };
-      switch (choose_tiles(g.M, n, g.K, g.groups, split.one_order)) {
+      switch (choose_tiles(g.M, n, g.K, g.groups, g.epi == EPI_RESIDUAL, split.one_order)) {
         case 0: direct(Tiles64{}); break;
         case 1: direct(Tiles128{}); break;
         case 2: direct(Wide64{}); break;

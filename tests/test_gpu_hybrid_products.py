@@ -27,9 +27,9 @@ LENGTHS = (2, 16, 40, 63, 65, 129, 200, 257, 520, 1024, 1100, 1531, MOST)
 SHAPES = {
     "large": synthetic.hybrid_shape("a", width=2048, vocab=640, streams=2, ff={"a": 4096}, heads=8, dim=128, rot_dim=64, v_dim=128, rank=256, window=512),
     "ragged": synthetic.hybrid_shape("a", width=1104, vocab=336, streams=3, ff={"a": 1744}, heads=3, dim=80, rot_dim=32, v_dim=112, rank=144, window=77),
-    "recurrent": synthetic.hybrid_shape("rw", width=1088, vocab=336, streams=2, ff={"r": 2872, "w": 1936}, lru_width=1280, blocks=5, taps=4, wkv_heads=17, wkv_dim=64, wkv_rank=96),
+    "recurrent": synthetic.hybrid_shape("rw", width=2112, vocab=336, streams=2, ff={"r": 4096, "w": 1936}, lru_width=1280, blocks=5, taps=4, wkv_heads=17, wkv_dim=64, wkv_rank=96),
     "plain": synthetic.looped_shape("pgp", width=2048, vocab=336, ff={"p": 4040, "g": 2856}, loop=(1, 2, 2), heads=4, kv_heads=2, delta_heads=4, delta_kv_heads=2,
-                                    delta_rank=144, gate_rank=72, gla_heads=2, gla_rank=80),
+                                    delta_rank=144, gate_rank=72, gla_heads=11, gla_rank=80),
 }
 
 

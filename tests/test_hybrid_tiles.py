@@ -16,10 +16,10 @@ DRIVER = """
 #include "qmk_hybrid_tiles.h"
 using namespace qmk::hybrid;
 int main() {
-  int M, N, K, groups, flag;
-  while (scanf("%d %d %d %d %d", &M, &N, &K, &groups, &flag) == 5) {
+  int M, N, K, groups, streams, flag;
+  while (scanf("%d %d %d %d %d %d", &M, &N, &K, &groups, &streams, &flag) == 6) {
     const RegisterTiles r = choose_register_tiles(M, N, K, groups, flag);
-    const int kind = K % 64 ? -1 : choose_tiles(M, N, K, groups, flag);
+    const int kind = K % 64 ? -1 : choose_tiles(M, N, K, groups, streams, flag);
     printf("%d %d %d %d %d %d %d\\n", kind, kind < 0 ? 1 : kTileCosts[kind].bm, kind < 0 ? 1 : kTileCosts[kind].bn, kind < 0 ? 1 : kTileCosts[kind].bk, choose_part_splits(M, N, K, groups),
            r.large, r.splits);
   }
@@ -34,9 +34,9 @@ def choose(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", f"-I{ROOT / 'qimeng-megakernel_amd' / 'csrc'}", "-o", str(folder / "driver"), str(folder / "driver.cpp")], check=True)
 
     def run(sizes):
-        """(kind, its rows of tokens, of weights, its columns, cuts of parts, whether register tiles are large, their cuts) of (M, N, K, groups, flag); the flag: in
-        one order, and for register tiles whether there is an fp32 side."""
-        text = "".join("%d %d %d %d %d\n" % s for s in sizes)
+        """(kind, its rows of tokens, of weights, its columns, cuts of parts, whether register tiles are large, their cuts) of (M, N, K, groups, whether the
+        epilogue moves the residual's streams, flag); the flag: in one order, and for register tiles whether there is an fp32 side."""
+        text = "".join("%d %d %d %d %d %d\n" % s for s in sizes)
         out = subprocess.run([str(folder / "driver")], input=text, capture_output=True, text=True, check=True).stdout
         return [tuple(map(int, line.split())) for line in out.splitlines()]
 
@@ -44,31 +44,32 @@ def choose(tmp_path_factory):
 
 
 def products(shape, n):
-    """(M, N, K, groups, whether its tokens' side may be in parts) of every product of a portion of n tokens from a request's start."""
-    D, found = shape.width_s, []
+    """(M, N, K, groups, whether the epilogue moves the residual's streams, whether its tokens' side may be in parts) of every product of a portion of n
+    tokens from a request's start."""
+    D, S, found = shape.width_s, int(not shape.plain), []
     for e in shape.entries:
         l = e.shape
         if e.type == "join":
-            found.append((n, D, 2 * D, 1, True))
+            found.append((n, D, 2 * D, 1, 0, True))
         if e.type in ("join", "final"):
             continue
         if e.type == "wkv":
-            found += [(n, max(l.mix_width, l.rank_s), D, 5, True), (n, l.mix_width, l.rank_s, 1, False)]
+            found += [(n, max(l.mix_width, l.rank_s), D, 5, 0, True), (n, l.mix_width, l.rank_s, 1, 0, False)]
         else:
-            found.append((n, l.in_rows, D, 1, True))
+            found.append((n, l.in_rows, D, 1, 0, True))
         if e.type == "rglru":
-            found.append((n, 2 * l.block_s, l.block_s, l.blocks, False))
+            found.append((n, 2 * l.block_s, l.block_s, l.blocks, 0, False))
         elif e.type == "latent_attention":
-            found += [(n, l.heads * l.dim_s, l.rank_s, 1, False), (l.heads * l.v_s, n, l.rank_s, 1, False)]
+            found += [(n, l.heads * l.dim_s, l.rank_s, 1, 0, False), (l.heads * l.v_s, n, l.rank_s, 1, 0, False)]
         elif e.type in ("delta", "gla"):
-            found.append((n, l.heads * l.dim_s, l.rank_s, 1, False))
+            found.append((n, l.heads * l.dim_s, l.rank_s, 1, 0, False))
             if e.type == "delta":
-                found.append((n, l.mix_width, l.gate_rank_s, 1, False))
-        found.append((n, D, l.mix_width, 1, True))
+                found.append((n, l.mix_width, l.gate_rank_s, 1, 0, False))
+        found.append((n, D, l.mix_width, 1, S, True))
         ff = (16 * -(-e.ff // 16)) if e.ff else 0
         if ff:
-            found += [(n, 2 * ff, D, 1, True), (n, D, ff, 1, True)]
-    return found + [(n, shape.vocab_s, D, 1, True)]
+            found += [(n, 2 * ff, D, 1, 0, True), (n, D, ff, 1, S, True)]
+    return found + [(n, shape.vocab_s, D, 1, 0, True)]
 
 
 def test_the_gpu_tests_reach_every_kind_of_tile(choose):
@@ -76,10 +77,10 @@ def test_the_gpu_tests_reach_every_kind_of_tile(choose):
     for name, shape in SHAPES.items():
         for n in LENGTHS:
             sizes = products(shape, n)
-            for (M, N, K, groups, _), (kind, bm, bn, *_) in zip(sizes, choose([s[:4] + (n <= MOST_IN_ORDER,) for s in sizes])):
+            for (M, N, K, *_), (kind, bm, bn, *_) in zip(sizes, choose([s[:5] + (n <= MOST_IN_ORDER,) for s in sizes])):
                 if kind >= 0:
                     tiles.setdefault(KINDS[kind], set()).update(side for side, over in (("tokens", M % bm), ("rows", N % bn)) if over)
-            for (M, N, K, groups, may), (*_, cuts, large, small_cuts) in zip(sizes, choose([s[:4] + (1,) for s in sizes])):
+            for (M, N, K, *_, may), (*_, cuts, large, small_cuts) in zip(sizes, choose([s[:5] + (1,) for s in sizes])):
                 if may and K > 64 and K % 64 == 0:
                     parts.add(cuts)
                 elif K > 64:
@@ -91,8 +92,8 @@ def test_the_gpu_tests_reach_every_kind_of_tile(choose):
 
 def test_rules_hold_for_any_size(choose):
     rng = random.Random(1)
-    sizes = [(int(2 ** rng.uniform(0, 13)), 16 * int(2 ** rng.uniform(0, 14)), 16 * int(2 ** rng.uniform(0, 10.5)), rng.choice((1, 1, 5, 10)), rng.randint(0, 1)) for _ in range(4000)]
-    for (M, N, K, groups, flag), (kind, bm, bn, bk, cuts, large, small_cuts) in zip(sizes, choose(sizes)):
+    sizes = [(int(2 ** rng.uniform(0, 13)), 16 * int(2 ** rng.uniform(0, 14)), 16 * int(2 ** rng.uniform(0, 10.5)), rng.choice((1, 1, 5, 10)), rng.randint(0, 1), rng.randint(0, 1)) for _ in range(4000)]
+    for (M, N, K, groups, _, flag), (kind, bm, bn, bk, cuts, large, small_cuts) in zip(sizes, choose(sizes)):
         if kind >= 0:
             assert K % bk == 0 and (not flag or KINDS[kind] in IN_ORDER)
         # what is cut has room for its tickets and sums, and every part has columns of its own
@@ -101,3 +102,23 @@ def test_rules_hold_for_any_size(choose):
                 assert tiles <= 512 and tiles * c * per // 4 <= 256 * 128 * 128 // 4 and K // c >= 256
         assert flag or small_cuts == 1
         assert not large or small_cuts == 1
+
+
+#: us by kind where kinds are far apart or an epilogue decides between them (weights from memory, one MI355X)
+MEASURED = [
+    ((1700, 2048, 2048, 1), {"Wide64": 39.7, "Turns128": 50.1}),
+    ((2500, 2048, 2048, 1), {"Wide64": 64.7, "Turns96": 72.8, "Tiles128": 79.5}),
+    ((2500, 2048, 6144, 1), {"Turns96": 131.7, "Tiles128": 138.2}),
+    ((3000, 2048, 8192, 0), {"Tiles128": 130.3, "Turns96": 143.2, "Turns128": 150.2}),
+    ((4096, 2048, 8192, 0), {"Tiles128": 158.5, "Turns192": 186.1, "Turns128": 189.1}),
+    ((4096, 2048, 8192, 1), {"Tiles128": 191.8, "Turns128": 214.4, "Turns192": 216.0}),
+    ((4096, 16384, 2048, 0), {"Turns256": 270.5, "Turns192": 317.1, "Tiles128": 339.2}),
+    ((2048, 2048, 8192, 1), {"Turns128": 98.5, "Wide64": 120.1, "Tiles128": 142.4}),
+    ((1024, 2048, 6144, 1), {"Wide64": 54.7, "Tiles64": 63.1, "Tiles128": 116.0}),
+    ((43, 2048, 6144, 1), {"Few32": 17.3, "Few64": 19.9, "Tiles32": 27.2}),
+]
+
+
+def test_choices_where_kinds_are_far_apart(choose):
+    got = choose([(M, N, K, 1, streams, M <= MOST_IN_ORDER) for (M, N, K, streams), _ in MEASURED])
+    assert [KINDS[kind] for kind, *_ in got] == [min(us, key=us.get) for _, us in MEASURED]
