@@ -326,7 +326,6 @@ inline size_t values_cap(const QmkHybridArgs* a) { return (static_cast<size_t>(a
 struct SplitBuffers {
   int32_t* tickets;
   f32x4* partial;
-  bool one_order = false;      // of the portion: kOneOrderTokens
 };
 inline SplitBuffers split_buffers(Carver& c) {
   SplitBuffers b;
@@ -465,9 +464,9 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
 }
 
 template <class S, int KIND>
-constexpr bool priced_as = kTileCosts[KIND].bm == S::BM && kTileCosts[KIND].bn == S::BN && kTileCosts[KIND].bk == S::BK && (S::kGroups == 1 || !kTileCosts[KIND].one_order);
-static_assert(priced_as<Tiles64, 0> && priced_as<Tiles128, 1> && priced_as<Wide64, 2> && priced_as<Turns96, 3> && priced_as<Turns128, 4>, "tiles and their prices");
-static_assert(priced_as<Turns192, 5> && priced_as<Turns256, 6> && priced_as<Tiles32, 7> && priced_as<Few64, 8> && priced_as<Few32, 9>, "tiles and their prices");
+constexpr bool priced_as = kTileCosts[KIND].bm == S::BM && kTileCosts[KIND].bn == S::BN && kTileCosts[KIND].bk == S::BK;
+static_assert(priced_as<Tiles64, 0> && priced_as<Tiles128, 1> && priced_as<Wide64, 2> && priced_as<Turns192, 3> && priced_as<Turns256, 4>, "tiles and their prices");
+static_assert(priced_as<Tiles32, 5> && priced_as<Few64, 6> && priced_as<Few32, 7>, "tiles and their prices");
 static_assert(kPartTileTokens == TilesParts::BM && kPartTileRows == TilesParts::BN, "tiles of operands in parts");
 static_assert(256LL * 2 * kPartTileTokens * kPartTileRows / 4 <= kPartialUnits && 256 <= kMaxTickets, "room for what is cut along K");
 
@@ -484,16 +483,14 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
     if (g.K % 64 == 0) {
       auto direct = [&](auto s) { using S = decltype(s); launch(gemm_direct<T, S>, S::BM, S::BN, S::kThreadCount); };
       auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S>, S::BM, S::BN, S::kThreadCount); };
-      switch (choose_tiles(g.M, n, g.K, g.groups, g.epi == EPI_RESIDUAL, split.one_order)) {
+      switch (choose_tiles(g.M, n, g.K, g.groups, g.epi == EPI_RESIDUAL)) {
         case 0: direct(Tiles64{}); break;
         case 1: direct(Tiles128{}); break;
         case 2: direct(Wide64{}); break;
-        case 3: turns(Turns96{}); break;
-        case 4: turns(Turns128{}); break;
-        case 5: turns(Turns192{}); break;
-        case 6: turns(Turns256{}); break;
-        case 7: direct(Tiles32{}); break;
-        case 8: direct(Few64{}); break;
+        case 3: turns(Turns192{}); break;
+        case 4: turns(Turns256{}); break;
+        case 5: direct(Tiles32{}); break;
+        case 6: direct(Few64{}); break;
         default: direct(Few32{}); break;
       }
       return;
@@ -521,30 +518,24 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
 
 // Ahead of a portion's other launches.
 template <class T>
-void begin_portion(const QmkHybridArgs* a, SplitBuffers& split, hipStream_t st) {
-  split.one_order = sizeof(T) == 2 && a->tokens <= kOneOrderTokens;
+void begin_portion(const SplitBuffers& split, hipStream_t st) {
   if constexpr (sizeof(T) == 4) hipLaunchKernelGGL(clear_tickets, dim3(1), dim3(kPfThreads), 0, st, split.tickets, kMaxTickets);
 }
 
-// rows: where the rotated part of a latent attention's keys is, behind the latent.  Two groups of waves share a workgroup's queries, except where the order
-// counts (kOneOrderTokens) and in fp32 with the largest heads, whose two groups take 140 KB of LDS and more registers than there are (us a portion of one
-// layer, 16 heads of 256 | 256, one group -> two: fp32 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508; bf16 1141 -> 728, 194 -> 156).
+// rows: where the rotated part of a latent attention's keys is, behind the latent.  In fp32 two groups of waves share a workgroup's queries, except for
+// the largest heads, where they take 140 KB of LDS and more registers than there are (us a portion of one layer, 16 heads of 256 | 256, one group -> two:
+// 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508).
 template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
-                      bool one_order, hipStream_t st) {
+                      hipStream_t st) {
+  constexpr int G = sizeof(T) == 4 ? 2 : 1;
   auto launch = [&](auto kernel, int groups) {
     hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
   };
-  auto sized = [&](auto groups) {
-    constexpr int G = decltype(groups)::value, kLargest = sizeof(T) == 4 ? 1 : G;
-    if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4, G>, G);
-    else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8, G>, G);
-    else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<T, 6, 8, G>, G);
-    else launch(window_attention<T, 8, 16, kLargest>, kLargest);
-  };
-  if constexpr (sizeof(T) == 2)
-    if (one_order) return sized(std::integral_constant<int, 1>{});
-  sized(std::integral_constant<int, 2>{});
+  if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4, G>, G);
+  else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8, G>, G);
+  else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<T, 6, 8, G>, G);
+  else launch(window_attention<T, 8, 16, 1>, 1);
 }
 
 template <class T>
@@ -556,7 +547,7 @@ int prefill(const QmkHybridArgs* a) {
   PrefillBuffers<T> b;
   if (prefill_buffers<T>(a, a->workspace, &b) > a->workspace_bytes) return QMK_ERR_SCRATCH;
   const hipStream_t st = static_cast<hipStream_t>(a->stream);
-  begin_portion<T>(a, b.split, st);
+  begin_portion<T>(b.split, st);
   const int M = a->tokens, D = a->width, S = a->streams, P = a->portion_rows;
   const dim3 block(kPfThreads);
   hipLaunchKernelGGL(embed_tokens, dim3(M), block, 0, st, a->embed, a->token_in, a->vocab, a->layers[0].hc, S, D, b.x, b.u);
@@ -601,7 +592,7 @@ int prefill(const QmkHybridArgs* a) {
       v.a = l.uv_w; v.w = b.rows; v.ldw = width; v.M = l.heads * l.v_dim; v.out = b.vt; v.ldo = cap;
       launch_gemm<u16, T, T>(v, b.split, st);
       const Keys<T> expanded{b.kn, l.heads * l.head_dim, l.head_dim, 1};
-      launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), b.split.one_order, st);
+      launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), st);
     } else {
       const int N = W, n = l.head_dim;
       hipLaunchKernelGGL(shift_mix<T>, dim3(M), block, 0, st, b.u, l, a->slot, a->flip, M, P, D, a->width_true, a->eps, b.h.of(D));
@@ -641,22 +632,17 @@ int prefill(const QmkHybridArgs* a) {
 }
 
 // The recurrence of a gla or delta entry over the portion, from its projections to what its output projection reads.
-template <bool DELTA>
-void run_chunks(const QmkHybridArgs* a, const ChunkArgs& g, bool one_order, hipStream_t st) {
+template <class T, bool DELTA>
+void run_chunks(const ChunkArgs& g, hipStream_t st) {
+  constexpr bool kEight = sizeof(T) == 4 && !DELTA;
   const QmkHybridLayer& l = g.layer;
   const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens;
   hipLaunchKernelGGL(chunk_prepare<DELTA>, dim3(chunks, l.heads), dim3(kPfThreads), 0, st, g);
   auto launch = [&](auto kernel, int waves) { hipLaunchKernelGGL(kernel, dim3(l.heads, l.v_dim / 16), dim3(waves * 64), 0, st, g); };
   switch (chunk_tiles(l.head_dim)) {
     case 4: return launch(chunk_scan<1, 4, DELTA>, 4);
-    case 8:
-      if constexpr (!DELTA)
-        if (!one_order) return launch(chunk_scan<1, 8, DELTA>, 8);
-      return launch(chunk_scan<2, 4, DELTA>, 4);
-    default:
-      if constexpr (!DELTA)
-        if (!one_order) return launch(chunk_scan<2, 8, DELTA>, 8);
-      return launch(chunk_scan<4, 4, DELTA>, 4);
+    case 8: return launch(chunk_scan<kEight ? 1 : 2, kEight ? 8 : 4, DELTA>, kEight ? 8 : 4);
+    default: return launch(chunk_scan<kEight ? 2 : 4, kEight ? 8 : 4, DELTA>, kEight ? 8 : 4);
   }
 }
 
@@ -665,7 +651,7 @@ int prefill_plain(const QmkHybridArgs* a) {
   PlainBuffers<T> b;
   if (plain_buffers<T>(a, a->workspace, &b) > a->workspace_bytes) return QMK_ERR_SCRATCH;
   const hipStream_t st = static_cast<hipStream_t>(a->stream);
-  begin_portion<T>(a, b.split, st);
+  begin_portion<T>(b.split, st);
   const int M = a->tokens, D = a->width;
   const size_t rows = static_cast<size_t>(a->portion_rows) * D;
   const dim3 block(kPfThreads);
@@ -721,7 +707,7 @@ int prefill_plain(const QmkHybridArgs* a) {
       const int row = l.head_dim + l.v_dim, pitch = l.kv_heads * row, keys = a->position + M, cap = static_cast<int>(values_cap(a));
       const T* cache = static_cast<const T*>(l.cache) + static_cast<size_t>(a->slot) * l.ring * pitch;
       hipLaunchKernelGGL(transpose_values<T>, dim3((keys + 63) / 64, (l.v_dim + 63) / 64, l.kv_heads), block, 0, st, cache, pitch, row, l.head_dim, l.v_dim, keys, cap, b.vt);
-      launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix.of(W), b.split.one_order, st);
+      launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix.of(W), st);
     } else {
       ChunkArgs c{};
       c.layer = l; c.decay = b.decay; c.chunks = b.chunks; c.out = b.o; c.M = M; c.slot = a->slot; c.flip = a->flip;
@@ -738,7 +724,7 @@ int prefill_plain(const QmkHybridArgs* a) {
         f.lda = ranks; f.out = b.gate; f.ldo = W;
         launch_gemm<T, u16, T>(f, b.split, st);
         c.qkv = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = W;
-        run_chunks<true>(a, c, b.split.one_order, st);
+        run_chunks<T, true>(c, st);
         if (l.taps > 1)
           hipLaunchKernelGGL(keep_inputs, dim3((channels + kPfThreads - 1) / kPfThreads), block, 0, st, b.qkv, l, channels, a->slot, a->flip, M);
       } else {
@@ -750,7 +736,7 @@ int prefill_plain(const QmkHybridArgs* a) {
         e.f0 = b.decay; e.ldo = keys;
         launch_gemm<T, u16, T>(e, b.split, st);
         c.qkv = b.qkv; c.values = b.qkv; c.value_ld = 2 * keys + W; c.value_at = 2 * keys;
-        run_chunks<false>(a, c, b.split.one_order, st);
+        run_chunks<T, false>(c, st);
       }
       hipLaunchKernelGGL(state_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.o, b.gate, l, M, a->eps, b.mix.of(W));
     }

@@ -323,21 +323,20 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, int group, int m, in
 }
 
 // ---- tiles ----
-// A tile is BM tokens x BN weight rows, BK columns a step; a wave owns WM x WN of it.  Where fewer waves than there are cover
-// the tile, two groups of them take a half of a step's columns each and are summed at the end.
+// A tile is BM tokens x BN weight rows, BK columns a step; a wave owns WM x WN of it and takes all columns, one after the other.
 template <int BM_, int BN_, int BK_, int WM_, int WN_, int WAVES_, int STAGES_>
 struct Tile {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, kStages = STAGES_, kThreadCount = WAVES_ * 64;
-  static constexpr int kWavesM = BM / WM, kWavesN = BN / WN, kCover = kWavesM * kWavesN, kGroups = WAVES_ / kCover;
-  static constexpr int kTm = WM / 16, kTn = WN / 16, kKept = kTn / kGroups;   // a wave's fragments; of those a thread sums up
+  static constexpr int kWavesM = BM / WM, kWavesN = BN / WN;
+  static constexpr int kTm = WM / 16, kTn = WN / 16;     // a wave's fragments
   static constexpr int kRow = BK / 8;                                           // a row of a step: units of 16 bytes
   static constexpr int kUnits = (BM + BN) * kRow;
-  static constexpr bool kSplits = kKept * kTm <= 8;                             // may be cut along K
-  static constexpr int kSteps = BK / 32 / kGroups;                              // matrix steps a wave takes of a step
+  static constexpr bool kSplits = kTn * kTm <= 8;                               // may be cut along K
+  static constexpr int kSteps = BK / 32;                                        // matrix steps of a step
   static constexpr int kOutUnits = BM * BN / 4, kPasses = kOutUnits > kStages * kUnits ? 2 : 1;
   static constexpr int kLds = kStages * kUnits > kOutUnits / kPasses ? kStages * kUnits : kOutUnits / kPasses;
   static_assert(kUnits % 64 == 0 && kSteps >= 1 && kTm % kPasses == 0 && kLds * 16 < 160 * 1024, "a tile's sizes");
-  static_assert(kGroups == 1 || (kGroups == 2 && kTn % 2 == 0), "groups of waves along K");
+  static_assert(kWavesM * kWavesN == WAVES_, "the waves cover the tile");
 };
 
 // Workgroups go to the XCDs in turn; here an XCD gets a run of neighbouring tiles, which share rows through its L2.
@@ -442,39 +441,22 @@ template <class T, class S, int LDS>
 __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int tile, int part, int m0, int n0, int N, v4u* lds, f32x4 (&acc)[S::kTn][S::kTm]) {
   constexpr int kQuads = S::BN / 4, kPassM = S::WM / S::kPasses, kRows = S::BM / S::kPasses, kTm = S::kTm;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kg = wave / S::kCover, wt = wave % S::kCover, wm = wt % S::kWavesM, wn = wt / S::kWavesM;
+  const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
   f32x4* out = reinterpret_cast<f32x4*>(lds);
-  f32x4 sums[S::kKept * kTm];
+  f32x4 sums[S::kTn * kTm];
   __syncthreads();
-  if constexpr (S::kGroups == 2) {      // each group keeps a half of the rows of weights and gives away the other
-    f32x4* box = out + wt * S::kKept * kTm * 64 + lane;
-    f32x4 *give = box + (1 - kg) * S::kCover * S::kKept * kTm * 64, *take = box + kg * S::kCover * S::kKept * kTm * 64;
-    static_assert(2 * S::kCover * S::kKept * kTm * 64 <= S::kLds, "both groups' halves");
 #pragma unroll
-    for (int j = 0; j < S::kKept; ++j)
-#pragma unroll
-      for (int i = 0; i < kTm; ++i) {
-        sums[j * kTm + i] = kg == 0 ? acc[j][i] : acc[S::kKept + j][i];
-        give[(j * kTm + i) * 64] = kg == 0 ? acc[S::kKept + j][i] : acc[j][i];
-      }
-    __syncthreads();
-#pragma unroll
-    for (int c = 0; c < S::kKept * kTm; ++c) sums[c] += take[c * 64];
-    __syncthreads();
-  } else {
-#pragma unroll
-    for (int c = 0; c < S::kKept * kTm; ++c) sums[c] = acc[c / kTm][c % kTm];
-  }
+  for (int c = 0; c < S::kTn * kTm; ++c) sums[c] = acc[c / kTm][c % kTm];
   if constexpr (S::kSplits)
-    if (g.splits > 1 && !sum_parts<S::kKept * kTm, S::kThreadCount>(g, tile, part, sums, reinterpret_cast<int*>(lds + LDS))) return;
+    if (g.splits > 1 && !sum_parts<S::kTn * kTm, S::kThreadCount>(g, tile, part, sums, reinterpret_cast<int*>(lds + LDS))) return;
 #pragma unroll
   for (int pass = 0; pass < S::kPasses; ++pass) {
     if (pass > 0) __syncthreads();
 #pragma unroll
     for (int i = 0; i < kTm / S::kPasses; ++i)
 #pragma unroll
-      for (int j = 0; j < S::kKept; ++j) {
-        const int r = wm * kPassM + i * 16 + (lane & 15), quad = wn * (S::WN / 4) + (kg * S::kKept + j) * 4 + (lane >> 4);
+      for (int j = 0; j < S::kTn; ++j) {
+        const int r = wm * kPassM + i * 16 + (lane & 15), quad = wn * (S::WN / 4) + j * 4 + (lane >> 4);
         out[r * kQuads + (quad ^ (r & (kQuads - 1) & 15))] = sums[j * kTm + pass * (kTm / S::kPasses) + i];
       }
     __syncthreads();
@@ -610,7 +592,6 @@ __device__ __forceinline__ void multiply(const Frag<u16> (&fa)[PARTS][S::kTm], c
 // values are; nothing else can have made it so that does not make it so again.  `a`, `w`: fragments of first parts, tile i and 32 columns from k.
 template <class S, class A, class W>
 __device__ __forceinline__ void resolve_undefined(const Place& p, f32x4 (&acc)[S::kTn][S::kTm], A&& a, W&& w) {
-  static_assert(S::kGroups == 1, "a wave takes all columns");
 #pragma unroll
   for (int j = 0; j < S::kTn; ++j)
 #pragma unroll
@@ -675,7 +656,7 @@ __global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
   constexpr int kAhead = S::kStages - 1;
   __shared__ __align__(16) v4u lds[S::kLds + 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kg = wave / S::kCover, wt = wave % S::kCover, wm = wt % S::kWavesM, wn = wt / S::kWavesM;
+  const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
   const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
   Stages<S> stages(g, p, lds, wave);
@@ -698,7 +679,7 @@ __global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
     // The buffer filled here was read in step s - 1: by this half a turn ago, by the other one before the last barrier.
     if (s + kAhead < p.steps) stages.issue(buf == 0 ? S::kStages - 1 : buf - 1);
     Frag<u16> fa[1][S::kTm], fw[S::kTn];
-    stages.fragments(buf, kg * 4 + (lane >> 4), wm, wn, fa, fw);
+    stages.fragments(buf, lane >> 4, wm, wn, fa, fw);
     // Stage s + 1 has landed: a barrier lies between this wait and either half's reads of it.
     if (s + kAhead < p.steps) stages.template wait<kAhead - 1>();
     else wait_outstanding<0>();
@@ -902,8 +883,6 @@ using Tiles128 = Tile<128, 128, 64, 64, 64, 4, 2>;
 // The tokens' side in three parts: it is what fills LDS, so few tokens a tile (us, 32 x 128 and 64 x 64 and 64 x 128 and 128 x 128: 200 x 2048 x 6144
 // 32, 35, 54, 169; 200 x 12288 x 2048 52, 58, 52, 63; 2048 x 2048 x 8192 260, 420, 291, 280).
 using TilesParts = Tile<32, 128, 64, 16, 64, 4, 2>;
-using Turns96 = Tile<96, 128, 64, 48, 64, 8, 4>;
-using Turns128 = Tile<128, 128, 64, 64, 64, 8, 4>;
 using Turns192 = Tile<192, 256, 32, 96, 64, 8, 4>;
 using Turns256 = Tile<256, 256, 32, 128, 64, 8, 4>;
 

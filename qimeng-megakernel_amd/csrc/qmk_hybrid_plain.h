@@ -328,8 +328,8 @@ __global__ __launch_bounds__(kPfThreads) void keep_inputs(const float* x, QmkHyb
 // so that kAhead chunks are in flight: a chunk, or token, behind the last one is the last one again, and its value is either
 // not used or multiplied by zero.
 // What bounds it is the chain of a chunk: products of the state with the keys (four dependent instructions of 32 cycles a tile), the
-// waves' sums through LDS, T (v - X), the state's update.  So eight waves hold the tiles of a gated linear attention's heads of more than 64 channels,
-// where the order does not count (kOneOrderTokens); and what only the output needs is off the chain: G q S is taken while the sums are on their way, and a chunk's outputs
+// waves' sums through LDS, T (v - X), the state's update.  So in fp32 eight waves hold the tiles of a gated linear attention's heads of more than
+// 64 channels (bf16 portions keep one order, four waves, qmk_hybrid_tiles.h); and what only the output needs is off the chain: G q S is taken while the sums are on their way, and a chunk's outputs
 // are added up and stored behind the next chunk's barrier.
 template <int TILES, int WAVES, bool DELTA>
 __global__ __launch_bounds__(WAVES * 64) void chunk_scan(const ChunkArgs g) {

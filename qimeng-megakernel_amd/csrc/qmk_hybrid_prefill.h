@@ -179,10 +179,9 @@ struct Keys {
 // Windowed attention over expanded keys: 64 queries of one head a workgroup (16 a wave), 32 keys a step.
 // Scores are computed transposed (keys x queries), so a lane holds eight weights of ONE query in exactly the shape the
 // value product's second operand wants, with keys in the order 4g..4g+3, 16+4g..16+4g+3.
-// GROUPS = 2: two groups of four waves take the 32-key steps in turn, for the same queries, and meet at the end: a step is a chain (keys into LDS,
-// scores, maximum over the lanes, weights, values), and a CU that holds one or two workgroups of four waves mostly waits for it
-// (us, one group -> two: 2048 queries of 16 heads of 128 behind 0 and 2048 keys, mean 156 -> 99; 1531 of 192 | 128 in a window of 1024
-// 70 -> 66; 43 behind 400 29 -> 19; 200 in fp32 34 -> 29.  Four groups: 121, 84, 24.)  GROUPS = 1 takes the keys in their order.
+// GROUPS = 1 takes the keys in their order, as bf16 portions have to (qmk_hybrid_tiles.h).  GROUPS = 2, fp32: two groups of four waves take the 32-key steps in
+// turn, for the same queries, and meet at the end: a step is a chain (keys into LDS, scores, maximum over the lanes, weights, values), and a CU
+// that holds one or two workgroups of four waves mostly waits for it (us, one group -> two: 200 queries of 16 heads of 192 | 128 34 -> 29).
 template <class T, int QT, int VT, int GROUPS>   // most 32-column steps of a query, most 16-row tiles of a value
 __global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const T* q, Keys<T> keys, const T* rows, const T* v_t, const T* gate, QmkHybridLayer l,
                                                                int first, int position, int M, int keys_cap, Operand<T> out) {

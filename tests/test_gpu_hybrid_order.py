@@ -1,5 +1,5 @@
-"""bf16 portions of up to 1024 tokens are computed in one order whatever their length: a token's logits are the same bits in a portion of
-any length that starts at the same place.  (Lengths at which the tiles of the products change; no recurrence whose scan is cut by the length.)"""
+"""bf16 portions are computed in one order whatever their length: a token's logits are the same bits in a portion of any length that starts at the
+same place.  (Lengths at which the tiles of the products change; no recurrence whose scan is cut by the length.)"""
 import pytest
 import torch
 
@@ -10,7 +10,8 @@ from qimeng_megakernel_amd.decode_schedule_hybrid.state import RequestTable
 
 pytestmark = pytest.mark.gpu
 
-MOST = 1024
+MOST = 2100
+LENGTHS = (2, 33, 64, 65, 129, 200, 257, 520, 1023, 1025, 1531, 2049)
 SHAPES = {
     "streams": synthetic.hybrid_shape("aw", width=2048, vocab=512, streams=2, ff={"a": 4096, "w": 2816}, heads=8, dim=128, rot_dim=64, v_dim=128, rank=256, window=300,
                                       wkv_heads=16, wkv_dim=64, wkv_rank=64),
@@ -36,6 +37,6 @@ def test_a_tokens_bits_do_not_depend_on_its_portions_length(name):
         return got
 
     whole = logits(MOST)
-    for n in (2, 33, 64, 65, 129, 200, 257, 520, 1023):
+    for n in LENGTHS:
         differing = int((logits(n) != whole[:n]).any(-1).sum())
         assert differing == 0, f"{differing} of {n} tokens"

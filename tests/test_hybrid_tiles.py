@@ -8,18 +8,16 @@ import pytest
 from conftest import ROOT
 from test_gpu_hybrid_products import LENGTHS, SHAPES
 
-KINDS = ("Tiles64", "Tiles128", "Wide64", "Turns96", "Turns128", "Turns192", "Turns256", "Tiles32", "Few64", "Few32")
-IN_ORDER = set(KINDS) - {"Turns96", "Turns128"}
-MOST_IN_ORDER = 1024
+KINDS = ("Tiles64", "Tiles128", "Wide64", "Turns192", "Turns256", "Tiles32", "Few64", "Few32")
 DRIVER = """
 #include <stdio.h>
 #include "qmk_hybrid_tiles.h"
 using namespace qmk::hybrid;
 int main() {
-  int M, N, K, groups, streams, flag;
-  while (scanf("%d %d %d %d %d %d", &M, &N, &K, &groups, &streams, &flag) == 6) {
-    const RegisterTiles r = choose_register_tiles(M, N, K, groups, flag);
-    const int kind = K % 64 ? -1 : choose_tiles(M, N, K, groups, streams, flag);
+  int M, N, K, groups, streams, cut;
+  while (scanf("%d %d %d %d %d %d", &M, &N, &K, &groups, &streams, &cut) == 6) {
+    const RegisterTiles r = choose_register_tiles(M, N, K, groups, cut);
+    const int kind = K % 64 ? -1 : choose_tiles(M, N, K, groups, streams);
     printf("%d %d %d %d %d %d %d\\n", kind, kind < 0 ? 1 : kTileCosts[kind].bm, kind < 0 ? 1 : kTileCosts[kind].bn, kind < 0 ? 1 : kTileCosts[kind].bk, choose_part_splits(M, N, K, groups),
            r.large, r.splits);
   }
@@ -35,7 +33,7 @@ def choose(tmp_path_factory):
 
     def run(sizes):
         """(kind, its rows of tokens, of weights, its columns, cuts of parts, whether register tiles are large, their cuts) of (M, N, K, groups, whether the
-        epilogue moves the residual's streams, flag); the flag: in one order, and for register tiles whether there is an fp32 side."""
+        epilogue moves the residual's streams, whether there is an fp32 side)."""
         text = "".join("%d %d %d %d %d %d\n" % s for s in sizes)
         out = subprocess.run([str(folder / "driver")], input=text, capture_output=True, text=True, check=True).stdout
         return [tuple(map(int, line.split())) for line in out.splitlines()]
@@ -77,7 +75,7 @@ def test_the_gpu_tests_reach_every_kind_of_tile(choose):
     for name, shape in SHAPES.items():
         for n in LENGTHS:
             sizes = products(shape, n)
-            for (M, N, K, *_), (kind, bm, bn, *_) in zip(sizes, choose([s[:5] + (n <= MOST_IN_ORDER,) for s in sizes])):
+            for (M, N, K, *_), (kind, bm, bn, *_) in zip(sizes, choose([s[:5] + (0,) for s in sizes])):
                 if kind >= 0:
                     tiles.setdefault(KINDS[kind], set()).update(side for side, over in (("tokens", M % bm), ("rows", N % bn)) if over)
             for (M, N, K, *_, may), (*_, cuts, large, small_cuts) in zip(sizes, choose([s[:5] + (1,) for s in sizes])):
@@ -93,32 +91,29 @@ def test_the_gpu_tests_reach_every_kind_of_tile(choose):
 def test_rules_hold_for_any_size(choose):
     rng = random.Random(1)
     sizes = [(int(2 ** rng.uniform(0, 13)), 16 * int(2 ** rng.uniform(0, 14)), 16 * int(2 ** rng.uniform(0, 10.5)), rng.choice((1, 1, 5, 10)), rng.randint(0, 1), rng.randint(0, 1)) for _ in range(4000)]
-    for (M, N, K, groups, _, flag), (kind, bm, bn, bk, cuts, large, small_cuts) in zip(sizes, choose(sizes)):
+    for (M, N, K, groups, _, fp32), (kind, bm, bn, bk, cuts, large, small_cuts) in zip(sizes, choose(sizes)):
         if kind >= 0:
-            assert K % bk == 0 and (not flag or KINDS[kind] in IN_ORDER)
+            assert K % bk == 0
         # what is cut has room for its tickets and sums, and every part has columns of its own
         for tiles, per, c in ((-(-M // 32) * -(-N // 128) * groups, 32 * 128, cuts), (-(-M // 64) * -(-N // 64) * groups, 64 * 64, small_cuts)):
             if c > 1:
                 assert tiles <= 512 and tiles * c * per // 4 <= 256 * 128 * 128 // 4 and K // c >= 256
-        assert flag or small_cuts == 1
+        assert fp32 or small_cuts == 1
         assert not large or small_cuts == 1
 
 
 #: us by kind where kinds are far apart or an epilogue decides between them (weights from memory, one MI355X)
 MEASURED = [
-    ((1700, 2048, 2048, 1), {"Wide64": 39.7, "Turns128": 50.1}),
-    ((2500, 2048, 2048, 1), {"Wide64": 64.7, "Turns96": 72.8, "Tiles128": 79.5}),
-    ((2500, 2048, 6144, 1), {"Turns96": 131.7, "Tiles128": 138.2}),
-    ((3000, 2048, 8192, 0), {"Tiles128": 130.3, "Turns96": 143.2, "Turns128": 150.2}),
-    ((4096, 2048, 8192, 0), {"Tiles128": 158.5, "Turns192": 186.1, "Turns128": 189.1}),
-    ((4096, 2048, 8192, 1), {"Tiles128": 191.8, "Turns128": 214.4, "Turns192": 216.0}),
+    ((2500, 2048, 2048, 1), {"Wide64": 64.7, "Tiles128": 79.5}),
+    ((4096, 2048, 8192, 0), {"Tiles128": 158.5, "Turns192": 186.1}),
+    ((4096, 2048, 8192, 1), {"Tiles128": 191.8, "Turns192": 216.0}),
     ((4096, 16384, 2048, 0), {"Turns256": 270.5, "Turns192": 317.1, "Tiles128": 339.2}),
-    ((2048, 2048, 8192, 1), {"Turns128": 98.5, "Wide64": 120.1, "Tiles128": 142.4}),
+    ((2048, 2048, 8192, 1), {"Wide64": 120.1, "Tiles128": 142.4}),
     ((1024, 2048, 6144, 1), {"Wide64": 54.7, "Tiles64": 63.1, "Tiles128": 116.0}),
     ((43, 2048, 6144, 1), {"Few32": 17.3, "Few64": 19.9, "Tiles32": 27.2}),
 ]
 
 
 def test_choices_where_kinds_are_far_apart(choose):
-    got = choose([(M, N, K, 1, streams, M <= MOST_IN_ORDER) for (M, N, K, streams), _ in MEASURED])
+    got = choose([(M, N, K, 1, streams, 0) for (M, N, K, streams), _ in MEASURED])
     assert [KINDS[kind] for kind, *_ in got] == [min(us, key=us.get) for _, us in MEASURED]
