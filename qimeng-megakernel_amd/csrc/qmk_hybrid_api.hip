@@ -465,8 +465,8 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
 
 template <class S, int KIND>
 constexpr bool priced_as = kTileCosts[KIND].bm == S::BM && kTileCosts[KIND].bn == S::BN && kTileCosts[KIND].bk == S::BK;
-static_assert(priced_as<Tiles64, 0> && priced_as<Tiles128, 1> && priced_as<Wide64, 2> && priced_as<Turns192, 3> && priced_as<Turns256, 4>, "tiles and their prices");
-static_assert(priced_as<Tiles32, 5> && priced_as<Few64, 6> && priced_as<Few32, 7>, "tiles and their prices");
+static_assert(priced_as<Tiles64, 0> && priced_as<Tiles128, 1> && priced_as<Wide64, 2> && priced_as<Turns96, 3> && priced_as<Turns128, 4>, "tiles and their prices");
+static_assert(priced_as<Turns192, 5> && priced_as<Turns256, 6> && priced_as<Tiles32, 7> && priced_as<Few64, 8> && priced_as<Few32, 9>, "tiles and their prices");
 static_assert(kPartTileTokens == TilesParts::BM && kPartTileRows == TilesParts::BN, "tiles of operands in parts");
 static_assert(256LL * 2 * kPartTileTokens * kPartTileRows / 4 <= kPartialUnits && 256 <= kMaxTickets, "room for what is cut along K");
 
@@ -487,10 +487,12 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
         case 0: direct(Tiles64{}); break;
         case 1: direct(Tiles128{}); break;
         case 2: direct(Wide64{}); break;
-        case 3: turns(Turns192{}); break;
-        case 4: turns(Turns256{}); break;
-        case 5: direct(Tiles32{}); break;
-        case 6: direct(Few64{}); break;
+        case 3: turns(Turns96{}); break;
+        case 4: turns(Turns128{}); break;
+        case 5: turns(Turns192{}); break;
+        case 6: turns(Turns256{}); break;
+        case 7: direct(Tiles32{}); break;
+        case 8: direct(Few64{}); break;
         default: direct(Few32{}); break;
       }
       return;

@@ -652,7 +652,7 @@ __global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g)
 // turn late.
 template <class T, class S>
 __global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
-  static_assert(S::kThreadCount == 512 && S::kSteps == 1 && S::kStages == 4, "one turn a step, three stages ahead");
+  static_assert(S::kThreadCount == 512 && S::kStages == 4, "one turn a step, three stages ahead");
   constexpr int kAhead = S::kStages - 1;
   __shared__ __align__(16) v4u lds[S::kLds + 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -678,14 +678,16 @@ __global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
   for (int s = 0; s < p.steps; ++s) {
     // The buffer filled here was read in step s - 1: by this half a turn ago, by the other one before the last barrier.
     if (s + kAhead < p.steps) stages.issue(buf == 0 ? S::kStages - 1 : buf - 1);
-    Frag<u16> fa[1][S::kTm], fw[S::kTn];
-    stages.fragments(buf, lane >> 4, wm, wn, fa, fw);
+    Frag<u16> fa[S::kSteps][1][S::kTm], fw[S::kSteps][S::kTn];
+#pragma unroll
+    for (int kk = 0; kk < S::kSteps; ++kk) stages.fragments(buf, kk * 4 + (lane >> 4), wm, wn, fa[kk], fw[kk]);
     // Stage s + 1 has landed: a barrier lies between this wait and either half's reads of it.
     if (s + kAhead < p.steps) stages.template wait<kAhead - 1>();
     else wait_outstanding<0>();
     barrier();
     __builtin_amdgcn_s_setprio(1);
-    multiply<S, 1>(fa, fw, acc);
+#pragma unroll
+    for (int kk = 0; kk < S::kSteps; ++kk) multiply<S, 1>(fa[kk], fw[kk], acc);
     __builtin_amdgcn_s_setprio(0);
     barrier();
     buf = buf + 1 == S::kStages ? 0 : buf + 1;
@@ -883,6 +885,10 @@ using Tiles128 = Tile<128, 128, 64, 64, 64, 4, 2>;
 // The tokens' side in three parts: it is what fills LDS, so few tokens a tile (us, 32 x 128 and 64 x 64 and 64 x 128 and 128 x 128: 200 x 2048 x 6144
 // 32, 35, 54, 169; 200 x 12288 x 2048 52, 58, 52, 63; 2048 x 2048 x 8192 260, 420, 291, 280).
 using TilesParts = Tile<32, 128, 64, 16, 64, 4, 2>;
+// Two matrix steps a turn where a wave's part is small: a turn's reads and products then outlast its barriers (us, M x N x K: 1531 x 2048 x 8192 with the residual's
+// streams Turns96 76, Wide64 109; 2048 x 2048 x 6144 Turns128 60, Wide64 75, 128 x 128 in steps of 32 columns 78).
+using Turns96 = Tile<96, 128, 64, 48, 32, 8, 4>;
+using Turns128 = Tile<128, 128, 64, 32, 64, 8, 4>;
 using Turns192 = Tile<192, 256, 32, 96, 64, 8, 4>;
 using Turns256 = Tile<256, 256, 32, 128, 64, 8, 4>;
 

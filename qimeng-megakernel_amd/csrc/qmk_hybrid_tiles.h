@@ -13,26 +13,28 @@ constexpr int kPartialUnits = 256 * 128 * 128 / 4;     // quads its parts leave:
 // in another order is enough to change what they leave in the states.  Largest relative difference of a state, cache or logits between two orders, 24 sets of weights of
 // each of four shapes (width 2048): 2 tokens 0.31, 34 0.065, 100 0.077, 256 0.050, 512 0.038, 1000 0.026, 1531 0.024; 192 prompts of 1025 to 3900 tokens:
 // 0.053, and in one cache a value that differs by twice its root mean square.  The median is 0.008 to 0.024 at every length.  (Two groups of waves along K, two groups
-// in the attention and eight waves in the scan took 6.15 ms instead of 6.62 for 1531 tokens of the 1b shape, 14.3 instead of 15.5 for 2 x 2048 of the looped one.)
+// in the attention and eight waves in the scan took 6.18 ms instead of 6.26 for 1531 tokens of the 1b shape, 14.5 instead of 15.4 for 2 x 2048 of the looped one.)
 
 // The tiles of a bf16 product.  It takes as many rounds as its tiles fill the chip, `slots` at a time, each about `step` us for 2048 columns and `fixed` us
 // besides, `streams` us more where the epilogue moves the residual's streams, and `overlapped` us once.  Fitted to measurements of every kind at 20 to
-// 4096 tokens and 14 of the N x K of the four shapes (weights from memory): the kind that comes out cheapest takes 0.2 % longer than the fastest one it may
-// take on the average up to 1024 tokens, 0.3 % up to 2048 and 0.2 % beyond, at most 8 %.  Tiles32 ends at 128 tokens: beyond, its price is off by up to 30 %
+// 4096 tokens and 14 of the N x K of the four shapes (weights from memory): the kind that comes out cheapest takes 0.5 % longer than the fastest one
+// on the average up to 1024 tokens, 0.8 % up to 2048 and 0.3 % beyond, at most 9 %.  Tiles32 ends at 128 tokens: beyond, its price is off by up to 30 %
 // for many rows of weights (192 x 8256 x 2048 24.0, Tiles64 18.3), at what it would save for few (300 x 2048 x 2048 with the streams 17.9, Tiles64 21.7).
 // us, M x N x K, the kinds around the line: 43 x 2048 x 2048 with the streams Few32 9.3, Few64 10.0, Tiles32 14.1; 128 x 5696 x 2048 Tiles32 12.3, Tiles64 13.2; 1024 x 2048 x
-// 6144 with the streams Wide64 55, Tiles64 63, Tiles128 116; 2048 x 16384 x 2048 Turns256 137, Tiles128 155, Turns192 164; 2048 x 2048 x 8192 Wide64 100, with
-// the streams 120, Tiles128 142; 4096 x 2048 x 8192 Tiles128 159, Turns192 186, with them 192, 216.  Memory is not priced: it bounds
+// 6144 with the streams Wide64 55, Tiles64 63, Tiles128 116; 2048 x 16384 x 2048 Turns256 137, Tiles128 155, Turns192 164; 2048 x 2048 x 8192 with
+// the streams Turns128 92, Wide64 105, Tiles128 126; 1531 x 2048 x 2048 with them Wide64 29, Turns96 32; 4096 x 2048 x 8192 Tiles128 159, Turns192 186, with them 192, 216.  Memory is not priced: it bounds
 // all kinds alike where there are many rows for few tokens (1 x 128256 x 2048 Tiles32 95, Tiles64 99, Wide64 108, Tiles128 124).
 struct TileCost {
   int most_tokens, bm, bn, bk, slots;
   double step, fixed, overlapped, streams;
 };
-constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 8;
+constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 10;
 constexpr TileCost kTileCosts[kTileKinds] = {
     {kAnyTokens, 64, 64, 64, 256, 7.9, 0.0, 3.5, 7.0},         // Tiles64
     {kAnyTokens, 128, 128, 64, 512, 25.9, 9.4, 0.0, 38.3},     // Tiles128
     {kAnyTokens, 128, 64, 64, 256, 11.7, 0.9, 1.4, 8.4},       // Wide64
+    {kAnyTokens, 96, 128, 64, 256, 13.2, 11.9, 0.5, 20.7},     // Turns96
+    {kAnyTokens, 128, 128, 64, 256, 13.6, 10.8, 1.2, 24.6},    // Turns128
     {kAnyTokens, 192, 256, 32, 256, 32.3, 14.7, 0.0, 53.5},    // Turns192
     {kAnyTokens, 256, 256, 32, 256, 39.7, 16.8, 0.0, 64.4},    // Turns256
     {128, 64, 32, 64, 512, 7.1, 1.5, 2.8, 3.6},                // Tiles32

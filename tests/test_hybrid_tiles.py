@@ -8,7 +8,7 @@ import pytest
 from conftest import ROOT
 from test_gpu_hybrid_products import LENGTHS, SHAPES
 
-KINDS = ("Tiles64", "Tiles128", "Wide64", "Turns192", "Turns256", "Tiles32", "Few64", "Few32")
+KINDS = ("Tiles64", "Tiles128", "Wide64", "Turns96", "Turns128", "Turns192", "Turns256", "Tiles32", "Few64", "Few32")
 DRIVER = """
 #include <stdio.h>
 #include "qmk_hybrid_tiles.h"
@@ -104,11 +104,13 @@ def test_rules_hold_for_any_size(choose):
 
 #: us by kind where kinds are far apart or an epilogue decides between them (weights from memory, one MI355X)
 MEASURED = [
-    ((2500, 2048, 2048, 1), {"Wide64": 64.7, "Tiles128": 79.5}),
+    ((1531, 2048, 8192, 1), {"Turns96": 80.3, "Turns128": 90.4, "Wide64": 109.0}),
+    ((1700, 2048, 2048, 1), {"Wide64": 29.8, "Turns128": 37.6}),
+    ((3000, 2048, 8192, 0), {"Tiles128": 117.3, "Turns96": 136.0, "Turns128": 145.2}),
     ((4096, 2048, 8192, 0), {"Tiles128": 158.5, "Turns192": 186.1}),
-    ((4096, 2048, 8192, 1), {"Tiles128": 191.8, "Turns192": 216.0}),
+    ((4096, 2048, 8192, 1), {"Tiles128": 160.0, "Turns192": 180.8, "Turns128": 188.5}),
     ((4096, 16384, 2048, 0), {"Turns256": 270.5, "Turns192": 317.1, "Tiles128": 339.2}),
-    ((2048, 2048, 8192, 1), {"Wide64": 120.1, "Tiles128": 142.4}),
+    ((2048, 2048, 8192, 1), {"Turns128": 92.3, "Wide64": 105.0, "Tiles128": 125.6}),
     ((1024, 2048, 6144, 1), {"Wide64": 54.7, "Tiles64": 63.1, "Tiles128": 116.0}),
     ((43, 2048, 6144, 1), {"Few32": 17.3, "Few64": 19.9, "Tiles32": 27.2}),
 ]
