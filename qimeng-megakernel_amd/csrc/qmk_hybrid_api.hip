@@ -465,8 +465,8 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
 
 template <class S, int KIND>
 constexpr bool priced_as = kTileCosts[KIND].bm == S::BM && kTileCosts[KIND].bn == S::BN && kTileCosts[KIND].bk == S::BK;
-static_assert(priced_as<Tiles64, 0> && priced_as<Tiles128, 1> && priced_as<Wide64, 2> && priced_as<Turns96, 3> && priced_as<Turns128, 4>, "tiles and their prices");
-static_assert(priced_as<Turns192, 5> && priced_as<Turns256, 6> && priced_as<Tiles32, 7> && priced_as<Few64, 8> && priced_as<Few32, 9>, "tiles and their prices");
+static_assert(priced_as<Tiles64, 0> && priced_as<Wide256, 1> && priced_as<Wide64, 2> && priced_as<Turns96, 3> && priced_as<Turns128, 4> && priced_as<Tall192, 5>, "tiles and their prices");
+static_assert(priced_as<Tall256, 6> && priced_as<Turns192, 7> && priced_as<Turns256, 8> && priced_as<Tiles32, 9> && priced_as<Few64, 10> && priced_as<Few32, 11>, "tiles and their prices");
 static_assert(kPartTileTokens == TilesParts::BM && kPartTileRows == TilesParts::BN, "tiles of operands in parts");
 static_assert(256LL * 2 * kPartTileTokens * kPartTileRows / 4 <= kPartialUnits && 256 <= kMaxTickets, "room for what is cut along K");
 
@@ -485,14 +485,16 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
       auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S>, S::BM, S::BN, S::kThreadCount); };
       switch (choose_tiles(g.M, n, g.K, g.groups, g.epi == EPI_RESIDUAL)) {
         case 0: direct(Tiles64{}); break;
-        case 1: direct(Tiles128{}); break;
+        case 1: turns(Wide256{}); break;
         case 2: direct(Wide64{}); break;
         case 3: turns(Turns96{}); break;
         case 4: turns(Turns128{}); break;
-        case 5: turns(Turns192{}); break;
-        case 6: turns(Turns256{}); break;
-        case 7: direct(Tiles32{}); break;
-        case 8: direct(Few64{}); break;
+        case 5: turns(Tall192{}); break;
+        case 6: turns(Tall256{}); break;
+        case 7: turns(Turns192{}); break;
+        case 8: turns(Turns256{}); break;
+        case 9: direct(Tiles32{}); break;
+        case 10: direct(Few64{}); break;
         default: direct(Few32{}); break;
       }
       return;

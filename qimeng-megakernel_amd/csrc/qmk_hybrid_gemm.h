@@ -652,7 +652,7 @@ __global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g)
 // turn late.
 template <class T, class S>
 __global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
-  static_assert(S::kThreadCount == 512 && S::kStages == 4, "one turn a step, three stages ahead");
+  static_assert(S::kThreadCount == 512 && S::kStages >= 3, "one turn a step, the next stage has landed before it");
   constexpr int kAhead = S::kStages - 1;
   __shared__ __align__(16) v4u lds[S::kLds + 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -881,14 +881,18 @@ using Few64 = Tile<64, 16, 128, 16, 16, 4, 3>;
 using Tiles32 = Tile<64, 32, 64, 32, 16, 4, 4>;
 using Tiles64 = Tile<64, 64, 64, 32, 32, 4, 4>;
 using Wide64 = Tile<128, 64, 64, 32, 32, 8, 3>;
-using Tiles128 = Tile<128, 128, 64, 64, 64, 4, 2>;
 // The tokens' side in three parts: it is what fills LDS, so few tokens a tile (us, 32 x 128 and 64 x 64 and 64 x 128 and 128 x 128: 200 x 2048 x 6144
 // 32, 35, 54, 169; 200 x 12288 x 2048 52, 58, 52, 63; 2048 x 2048 x 8192 260, 420, 291, 280).
 using TilesParts = Tile<32, 128, 64, 16, 64, 4, 2>;
 // Two matrix steps a turn where a wave's part is small: a turn's reads and products then outlast its barriers (us, M x N x K: 1531 x 2048 x 8192 with the residual's
-// streams Turns96 76, Wide64 109; 2048 x 2048 x 6144 Turns128 60, Wide64 75, 128 x 128 in steps of 32 columns 78).
+// streams Turns96 90, Wide64 120; 2048 x 2048 x 6144 Turns128 60, Wide64 75, 128 x 128 in steps of 32 columns 78).
 using Turns96 = Tile<96, 128, 64, 48, 32, 8, 4>;
 using Turns128 = Tile<128, 128, 64, 32, 64, 8, 4>;
+// Three stages where four do not fit (two workgroups of 128 x 128 on four waves a CU, which these replace: 4096 x 2048 x 8192 with the streams 188, Tall256 173; 3000 x
+// 2048 x 8192 with them 162, Tall192 133; 1900 x 8256 x 2048 76, Wide256 72).
+using Tall192 = Tile<192, 128, 64, 96, 32, 8, 3>;
+using Tall256 = Tile<256, 128, 64, 64, 64, 8, 3>;
+using Wide256 = Tile<128, 256, 64, 64, 64, 8, 3>;
 using Turns192 = Tile<192, 256, 32, 96, 64, 8, 4>;
 using Turns256 = Tile<256, 256, 32, 128, 64, 8, 4>;
 

@@ -22,7 +22,7 @@ TOL = {torch.float32: 2e-5, torch.bfloat16: 4e-2}
 TOL_PLAIN = {torch.float32: 4e-5, torch.bfloat16: 8e-2}
 MOST = 1540
 #: lengths at which some product of some shape changes its tiles, and odd ones
-LENGTHS = (2, 16, 40, 63, 65, 129, 200, 257, 520, 1024, 1100, 1531, MOST)
+LENGTHS = (2, 16, 40, 63, 65, 129, 200, 257, 520, 1024, 1100, 1290, 1531, MOST)
 #: feed-forwards of a size that fills the large tiles, and of one no tile divides; every mixer, with columns in multiples of 64 and not
 SHAPES = {
     "large": synthetic.hybrid_shape("a", width=2048, vocab=640, streams=2, ff={"a": 4096}, heads=8, dim=128, rot_dim=64, v_dim=128, rank=256, window=512),

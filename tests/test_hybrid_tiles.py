@@ -8,7 +8,7 @@ import pytest
 from conftest import ROOT
 from test_gpu_hybrid_products import LENGTHS, SHAPES
 
-KINDS = ("Tiles64", "Tiles128", "Wide64", "Turns96", "Turns128", "Turns192", "Turns256", "Tiles32", "Few64", "Few32")
+KINDS = ("Tiles64", "Wide256", "Wide64", "Turns96", "Turns128", "Tall192", "Tall256", "Turns192", "Turns256", "Tiles32", "Few64", "Few32")
 DRIVER = """
 #include <stdio.h>
 #include "qmk_hybrid_tiles.h"
@@ -104,14 +104,17 @@ def test_rules_hold_for_any_size(choose):
 
 #: us by kind where kinds are far apart or an epilogue decides between them (weights from memory, one MI355X)
 MEASURED = [
-    ((1531, 2048, 8192, 1), {"Turns96": 80.3, "Turns128": 90.4, "Wide64": 109.0}),
-    ((1700, 2048, 2048, 1), {"Wide64": 29.8, "Turns128": 37.6}),
-    ((3000, 2048, 8192, 0), {"Tiles128": 117.3, "Turns96": 136.0, "Turns128": 145.2}),
-    ((4096, 2048, 8192, 0), {"Tiles128": 158.5, "Turns192": 186.1}),
-    ((4096, 2048, 8192, 1), {"Tiles128": 160.0, "Turns192": 180.8, "Turns128": 188.5}),
-    ((4096, 16384, 2048, 0), {"Turns256": 270.5, "Turns192": 317.1, "Tiles128": 339.2}),
-    ((2048, 2048, 8192, 1), {"Turns128": 92.3, "Wide64": 105.0, "Tiles128": 125.6}),
-    ((1024, 2048, 6144, 1), {"Wide64": 54.7, "Tiles64": 63.1, "Tiles128": 116.0}),
+    ((1531, 2048, 2048, 1), {"Wide64": 38.0, "Turns96": 41.9, "Turns128": 49.9}),
+    ((1531, 2048, 8192, 1), {"Turns96": 89.6, "Turns128": 103.6, "Wide64": 119.8}),
+    ((3000, 2048, 2048, 1), {"Tall192": 68.9, "Turns96": 77.4, "Wide64": 79.3}),
+    ((3000, 2048, 8192, 0), {"Tall192": 102.8, "Tall256": 118.3, "Turns96": 137.2}),
+    ((4096, 2048, 8192, 0), {"Tall256": 123.4, "Turns192": 154.3, "Turns128": 166.5}),
+    ((4096, 2048, 8192, 1), {"Tall256": 173.4, "Turns128": 213.8, "Turns192": 216.4}),
+    ((4096, 16384, 2048, 0), {"Turns256": 262.5, "Tall256": 285.1, "Turns192": 303.7}),
+    ((2048, 2048, 8192, 1), {"Turns128": 103.7, "Wide64": 120.1, "Tall192": 126.2}),
+    ((2048, 12288, 2048, 0), {"Tall256": 107.0, "Turns256": 121.7}),
+    ((520, 12288, 2048, 0), {"Wide256": 35.5, "Turns128": 46.0, "Wide64": 49.0}),
+    ((1024, 2048, 6144, 1), {"Wide64": 57.9, "Tiles64": 64.5, "Turns96": 70.1}),
     ((43, 2048, 6144, 1), {"Few32": 17.3, "Few64": 19.9, "Tiles32": 27.2}),
 ]
 
