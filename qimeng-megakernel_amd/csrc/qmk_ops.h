@@ -567,7 +567,7 @@ __device__ __forceinline__ void merge_slices(SliceMerge (&m)[ITEMS], int P) {
 // head's group, with the same operations in the same order, sixteen slices a trip, and the O-projection reads the finished 4 KB.
 // Step time (us) by merging everywhere -> in the last slice: Llama shape 7 slices (context 2048) 542 -> 541, 10 (3000) 562 -> 546,
 // 32 (8192) 673 -> 616, 32 (16384) 754 -> 684; Qwen3-1.7B shape 12 (900) 849 -> 844, 32 (8000) 1393 -> 1218.  Up to four are one trip
-// either way.
+// either way.  The shapes with experts have not been timed with it and merge everywhere, as do launches without tags.
 constexpr int kMostSelfMerged = 4;
 template <class M>
 __device__ __forceinline__ bool last_slice_merges(const Params& p, int P) {
