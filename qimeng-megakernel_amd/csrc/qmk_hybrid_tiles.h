@@ -12,8 +12,8 @@ constexpr int kPartialUnits = 256 * 128 * 128 / 4;     // quads its parts leave:
 // a recurrence's first output leaves little but the sign of a sum that may be close to zero, and some later tokens come close to that), so that a sum taken
 // in another order is enough to change what they leave in the states.  Largest relative difference of a state, cache or logits between two orders, 24 sets of weights of
 // each of four shapes (width 2048): 2 tokens 0.31, 34 0.065, 100 0.077, 256 0.050, 512 0.038, 1000 0.026, 1531 0.024; 192 prompts of 1025 to 3900 tokens:
-// 0.053, and in one cache a value that differs by twice its root mean square.  The median is 0.008 to 0.024 at every length.  (Two groups of waves along K, two groups
-// in the attention and eight waves in the scan took 6.18 ms instead of 6.26 for 1531 tokens of the 1b shape, 14.5 instead of 15.4 for 2 x 2048 of the looped one.)
+// 0.053, and in one cache a value that differs by twice its root mean square.  The median is 0.008 to 0.024 at every length.  (With cuts along K, two groups
+// in the attention and eight waves in the scan 43 tokens of the 2b shape took 2.72 ms instead of 2.98, 2 x 2048 of the looped 1b shape 14.4 instead of 15.1.)
 
 // The tiles of a bf16 product.  It takes as many rounds as its tiles fill the chip, `slots` at a time, each about `step` us for 2048 columns and `fixed` us
 // besides, `streams` us more where the epilogue moves the residual's streams, and `overlapped` us once.  Fitted to measurements of every kind at 20 to
