@@ -528,18 +528,28 @@ void begin_portion(const SplitBuffers& split, hipStream_t st) {
 
 // rows: where the rotated part of a latent attention's keys is, behind the latent.  In fp32 two groups of waves share a workgroup's queries, except for
 // the largest heads, where they take 140 KB of LDS and more registers than there are (us a portion of one layer, 16 heads of 256 | 256, one group -> two:
-// 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508).
+// 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508).  In bf16 the largest heads leave no registers for a second wave a SIMD, and take stages of 32 keys.
 template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
                       hipStream_t st) {
-  constexpr int G = sizeof(T) == 4 ? 2 : 1;
-  auto launch = [&](auto kernel, int groups) {
-    hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
-  };
-  if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4, G>, G);
-  else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8, G>, G);
-  else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<T, 6, 8, G>, G);
-  else launch(window_attention<T, 8, 16, 1>, 1);
+  const int runs = (a->tokens + 63) / 64;
+  if constexpr (sizeof(T) == 2) {
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(runs * l.heads), dim3(kPfThreads), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out.at);
+    };
+    if (l.q_stride <= 128 && l.v_dim <= 64) launch(attention_rows<4, 4, 64, 2, 2>);
+    else if (l.q_stride <= 128 && l.v_dim <= 128) launch(attention_rows<4, 8, 64, 2, 2>);
+    else if (l.q_stride <= 192 && l.v_dim <= 128) launch(attention_rows<6, 8, 64, 2, 2>);
+    else launch(attention_rows<8, 16, 32, 3, 1>);
+  } else {
+    auto launch = [&](auto kernel, int groups) {
+      hipLaunchKernelGGL(kernel, dim3(runs, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
+    };
+    if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4, 2>, 2);
+    else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8, 2>, 2);
+    else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<T, 6, 8, 2>, 2);
+    else launch(window_attention<T, 8, 16, 1>, 1);
+  }
 }
 
 template <class T>
@@ -592,7 +602,7 @@ int prefill(const QmkHybridArgs* a) {
       GemmArgs k = gemm_args(whole(b.rows), width, l.uk_w, l.heads * l.head_dim, l.rank, l, EPI_STORE);
       k.M = keys; k.out = b.kn; k.ldo = l.heads * l.head_dim;
       launch_gemm<T, u16, T>(k, b.split, st);
-      GemmArgs v = gemm_args(whole(nullptr), l.rank, nullptr, keys, l.rank, l, EPI_STORE);   // transposed: W_uv rows x keys
+      GemmArgs v = gemm_args(whole(nullptr), l.rank, nullptr, keys, l.rank, l, sizeof(T) == 2 ? EPI_STORE_VALUES : EPI_STORE);   // transposed: W_uv rows x keys
       v.a = l.uv_w; v.w = b.rows; v.ldw = width; v.M = l.heads * l.v_dim; v.out = b.vt; v.ldo = cap;
       launch_gemm<u16, T, T>(v, b.split, st);
       const Keys<T> expanded{b.kn, l.heads * l.head_dim, l.head_dim, 1};

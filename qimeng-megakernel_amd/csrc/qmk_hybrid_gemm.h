@@ -12,6 +12,7 @@ constexpr int kPfThreads = 256;
 
 enum : int {
   EPI_STORE = 0,        // out T [m][ldo]
+  EPI_STORE_VALUES,     // the same, columns where value_place puts them
   EPI_RGLRU_IN,         // gelu of the y half, bias on both
   EPI_LRU_GATES,        // (r, i) pairs -> decay a and input b of the recurrence
   EPI_LATENT_IN,        // rotation of q, sigmoid of the gate, raw latent
@@ -113,6 +114,10 @@ __device__ __forceinline__ void put1(const Operand<T>& to, size_t i, float x) {
   to.at[i] = from_f32<T>(x);
 }
 
+// Where key k lies in a row of transposed values of a bf16 portion: of every 32 keys, the eight that a lane of the value product takes (4g .. 4g+3 and
+// 16+4g .. 16+4g+3) side by side, one read of 16 bytes.
+__host__ __device__ constexpr int value_place(int k) { return (k & ~31) | ((k & 12) << 1) | ((k & 16) >> 2) | (k & 3); }
+
 struct GemmArgs {
   const void* a;         // TA [M][lda]
   const void* w;         // TW [N][ldw]
@@ -160,6 +165,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, int group, int m, in
   const QmkHybridLayer& l = g.layer;
   switch (g.epi) {
     case EPI_STORE: store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + n, v); break;
+    case EPI_STORE_VALUES: store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + value_place(n), v); break;
     case EPI_RGLRU_IN: {
       const f32x4 b = *reinterpret_cast<const f32x4*>(l.in_b + n);
       v += b;

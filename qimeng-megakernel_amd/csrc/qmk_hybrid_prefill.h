@@ -6,7 +6,7 @@
 // recurrences use the fp32 ones.
 #pragma once
 
-#include "qmk_hybrid_gemm.h"
+#include "qmk_hybrid_attention.h"
 
 namespace qmk {
 namespace hybrid {
@@ -169,17 +169,8 @@ __global__ __launch_bounds__(kPfThreads) void latent_rows(const float* raw, QmkH
   }
 }
 
-// Keys of an attention: key j of key head h at at[j * pitch + h * head]; heads_per query heads share a key head.
-template <class T>
-struct Keys {
-  const T* at;
-  int pitch, head, heads_per;
-};
-
-// Windowed attention over expanded keys: 64 queries of one head a workgroup (16 a wave), 32 keys a step.
-// Scores are computed transposed (keys x queries), so a lane holds eight weights of ONE query in exactly the shape the
-// value product's second operand wants, with keys in the order 4g..4g+3, 16+4g..16+4g+3.
-// GROUPS = 1 takes the keys in their order, as bf16 portions have to (qmk_hybrid_tiles.h).  GROUPS = 2, fp32: two groups of four waves take the 32-key steps in
+// The same as attention_rows for fp32 portions, values in the order of their keys, 32 keys a step through registers.
+// GROUPS = 2: two groups of four waves take the 32-key steps in
 // turn, for the same queries, and meet at the end: a step is a chain (keys into LDS, scores, maximum over the lanes, weights, values), and a CU
 // that holds one or two workgroups of four waves mostly waits for it (us, one group -> two: 200 queries of 16 heads of 192 | 128 34 -> 29).
 template <class T, int QT, int VT, int GROUPS>   // most 32-column steps of a query, most 16-row tiles of a value

@@ -39,7 +39,7 @@ def test_no_prefill_kernel_spills(tmp_path):
         for entry in notes.split(".agpr_count:")[1:]:
             field = dict(re.findall(r"\.(\w+):\s+(\S+)", entry))
             kernels[field["symbol"]] = field
-    assert any("gemm_direct" in name for name in kernels) and any("window_attention" in name for name in kernels)
+    assert any("gemm_direct" in name for name in kernels) and any("window_attention" in name for name in kernels) and any("attention_rows" in name for name in kernels)
     prefill = {name: k for name, k in kernels.items() if "decode_megakernel" not in name}
     spilled = {name: k["vgpr_spill_count"] for name, k in prefill.items() if int(k["vgpr_spill_count"])}
     assert not spilled, spilled
