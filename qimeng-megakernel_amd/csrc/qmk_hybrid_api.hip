@@ -467,8 +467,9 @@ template <class S, int KIND>
 constexpr bool priced_as = kTileCosts[KIND].bm == S::BM && kTileCosts[KIND].bn == S::BN && kTileCosts[KIND].bk == S::BK;
 static_assert(priced_as<Tiles64, 0> && priced_as<Wide256, 1> && priced_as<Wide64, 2> && priced_as<Turns96, 3> && priced_as<Turns128, 4> && priced_as<Tall192, 5>, "tiles and their prices");
 static_assert(priced_as<Tall256, 6> && priced_as<Turns192, 7> && priced_as<Turns256, 8> && priced_as<Tiles32, 9> && priced_as<Few64, 10> && priced_as<Few32, 11>, "tiles and their prices");
-static_assert(kPartTileTokens == TilesParts::BM && kPartTileRows == TilesParts::BN, "tiles of operands in parts");
-static_assert(256LL * 2 * kPartTileTokens * kPartTileRows / 4 <= kPartialUnits && 256 <= kMaxTickets, "room for what is cut along K");
+template <class S, int KIND>
+constexpr bool priced_as_parts = kPartCosts[KIND].bm == S::BM && kPartCosts[KIND].bn == S::BN && S::kSplits;
+static_assert(priced_as_parts<Parts32, 0> && priced_as_parts<Parts64, 1> && priced_as_parts<PartsWide, 2>, "tiles of operands in parts and their prices");
 
 template <class TA, class TW, class T>
 void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
@@ -482,15 +483,16 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   if constexpr (sizeof(TA) == 2 && sizeof(TW) == 2) {
     if (g.K % 64 == 0) {
       auto direct = [&](auto s) { using S = decltype(s); launch(gemm_direct<T, S>, S::BM, S::BN, S::kThreadCount); };
+      auto pipe = [&](auto s) { using S = decltype(s); launch(gemm_pipe<T, S>, S::BM, S::BN, S::kThreadCount); };
       auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S>, S::BM, S::BN, S::kThreadCount); };
       switch (choose_tiles(g.M, n, g.K, g.groups, g.epi == EPI_RESIDUAL)) {
-        case 0: direct(Tiles64{}); break;
-        case 1: turns(Wide256{}); break;
+        case 0: pipe(Tiles64{}); break;
+        case 1: pipe(Wide256{}); break;
         case 2: direct(Wide64{}); break;
-        case 3: turns(Turns96{}); break;
-        case 4: turns(Turns128{}); break;
-        case 5: turns(Tall192{}); break;
-        case 6: turns(Tall256{}); break;
+        case 3: pipe(Turns96{}); break;
+        case 4: pipe(Turns128{}); break;
+        case 5: pipe(Tall192{}); break;
+        case 6: pipe(Tall256{}); break;
         case 7: turns(Turns192{}); break;
         case 8: turns(Turns256{}); break;
         case 9: direct(Tiles32{}); break;
@@ -502,9 +504,13 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   }
   if constexpr (sizeof(TA) == 4 && sizeof(TW) == 2) {
     if (g.a_part != 0) {
-      using S = TilesParts;
       g.splits = choose_part_splits(g.M, n, g.K, g.groups);
-      launch(gemm_direct<T, S, 3>, S::BM, S::BN, S::kThreadCount);
+      auto parts = [&](auto s) { using S = decltype(s); launch(gemm_pipe<T, S, 3>, S::BM, S::BN, S::kThreadCount); };
+      switch (choose_part_tiles(g.M, n, g.K, g.groups).kind) {
+        case 0: parts(Parts32{}); break;
+        case 1: parts(Parts64{}); break;
+        default: parts(PartsWide{}); break;
+      }
       return;
     }
   }

@@ -2,6 +2,8 @@
 // element-wise done in the epilogue.
 #pragma once
 
+#include <type_traits>
+
 #include "qmk_hybrid_ops.h"
 #include "qmk_hybrid_tiles.h"
 
@@ -159,174 +161,148 @@ __device__ __forceinline__ f32x4 read4(const T* at) {
   }
 }
 
-// Four consecutive outputs n .. n+3 of token m.
+// Eight values side by side.
 template <class T>
-__device__ __forceinline__ void epilogue(const GemmArgs& g, int group, int m, int n, f32x4 v) {
-  const QmkHybridLayer& l = g.layer;
-  switch (g.epi) {
-    case EPI_STORE: store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + n, v); break;
-    case EPI_STORE_VALUES: store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + value_place(n), v); break;
-    case EPI_RGLRU_IN: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.in_b + n);
-      v += b;
-      if (n < l.mix_width) {
+__device__ __forceinline__ void store8(T* at, f32x4 lo, f32x4 hi) {
+  if constexpr (sizeof(T) == 2) {
+    *reinterpret_cast<v4u*>(at) = v4u{f2bf2(lo[0], lo[1]), f2bf2(lo[2], lo[3]), f2bf2(hi[0], hi[1]), f2bf2(hi[2], hi[3])};
+  } else {
+    store4(at, lo);
+    store4(at + 4, hi);
+  }
+}
+template <class F>
+__device__ __forceinline__ f32x4 each(f32x4 v, F&& f) { return f32x4{f(v[0]), f(v[1]), f(v[2]), f(v[3])}; }
+
+// Eight consecutive outputs n .. n+7 of a token (sizes of storage are multiples of sixteen, so they are of one kind).  What depends on the columns alone
+// is read once, ahead of the tokens.
+template <class T, int EPI>
+struct Epilogue {
+  const GemmArgs& g;
+  const int group, n;
+  f32x4 b[2] = {};       // constants of the eight outputs
+
+  __device__ __forceinline__ Epilogue(const GemmArgs& args, int group_, int n_) : g(args), group(group_), n(n_) {
+    const QmkHybridLayer& l = g.layer;
+    const float* from = EPI == EPI_RGLRU_IN ? l.in_b + n
+                        : EPI == EPI_LRU_GATES ? l.mid_b + static_cast<size_t>(group) * 2 * l.block_dim + n
+                        : EPI == EPI_WKV_DECAY || EPI == EPI_DELTA_DECAY || EPI == EPI_GLA_DECAY ? l.mid_b + n : nullptr;
+    if constexpr (EPI == EPI_RGLRU_IN || EPI == EPI_LRU_GATES || EPI == EPI_WKV_DECAY || EPI == EPI_DELTA_DECAY || EPI == EPI_GLA_DECAY) {
+      b[0] = read4(from);
+      b[1] = read4(from + 4);
+    }
+  }
+
+  // Pairs (d, d+1) .. (d+6, d+7) of a head turned to their position.
+  __device__ __forceinline__ void turn(int position, int d, f32x4& lo, f32x4& hi) const {
+    float e[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = gelu_tanh(v[i]);
-        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * l.mix_width + n, v);
-      } else {
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.mix_width + n - l.mix_width, v);
-      }
-      break;
-    }
-    case EPI_LRU_GATES: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + static_cast<size_t>(group) * 2 * l.block_dim + n);
-      v += b;
+    for (int i = 0; i < 8; i += 2) rotate(g.layer, position, d + i, e[i], e[i + 1]);
+    lo = f32x4{e[0], e[1], e[2], e[3]};
+    hi = f32x4{e[4], e[5], e[6], e[7]};
+  }
+
+  __device__ __forceinline__ void operator()(int m, f32x4 lo, f32x4 hi) const {
+    const QmkHybridLayer& l = g.layer;
+    T *out = static_cast<T*>(g.out), *out2 = static_cast<T*>(g.out2);
+    const auto gate = [](float x) { return sigmoid(x); };
+    const auto silu = [](float x) { return x * sigmoid(x); };
+    const auto gelu = [](float x) { return gelu_tanh(x); };
+    const size_t row = static_cast<size_t>(m);
+    if constexpr (EPI == EPI_STORE) {
+      store8(out + row * g.ldo + n, lo, hi);
+    } else if constexpr (EPI == EPI_STORE_VALUES) {
+      store4(out + row * g.ldo + value_place(n), lo);
+      store4(out + row * g.ldo + value_place(n + 4), hi);
+    } else if constexpr (EPI == EPI_RGLRU_IN) {
+      lo += b[0];
+      hi += b[1];
+      if (n < l.mix_width) store8(out + row * l.mix_width + n, each(lo, gelu), each(hi, gelu));
+      else store8(out2 + row * l.mix_width + n - l.mix_width, lo, hi);
+    } else if constexpr (EPI == EPI_LRU_GATES) {
       const int c = group * l.block_dim + n / 2;
-      const size_t at = static_cast<size_t>(m) * l.mix_width + c;
-      const T* u = static_cast<const T*>(g.src) + at;
-      float2 a2, b2;
-      {
-        const float la = sigmoid(v[0]) * l.vec0[c];
-        a2.x = expf(la);
-        b2.x = sqrtf(-expm1f(2.f * la)) * sigmoid(v[1]) * to_f32(u[0]);
+      const size_t at = row * l.mix_width + c;
+      const f32x4 v[2] = {lo + b[0], hi + b[1]}, u = read4(static_cast<const T*>(g.src) + at), rate = read4(l.vec0 + c);
+      f32x4 decay, input;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float la = sigmoid(v[i >> 1][i * 2 & 3]) * rate[i];
+        decay[i] = expf(la);
+        input[i] = sqrtf(-expm1f(2.f * la)) * sigmoid(v[i >> 1][(i * 2 & 3) + 1]) * u[i];
       }
-      {
-        const float la = sigmoid(v[2]) * l.vec0[c + 1];
-        a2.y = expf(la);
-        b2.y = sqrtf(-expm1f(2.f * la)) * sigmoid(v[3]) * to_f32(u[1]);
-      }
-      *reinterpret_cast<float2*>(g.f0 + at) = a2;
-      *reinterpret_cast<float2*>(g.f1 + at) = b2;
-      break;
-    }
-    case EPI_LATENT_IN: {
+      store4(g.f0 + at, decay);
+      store4(g.f1 + at, input);
+    } else if constexpr (EPI == EPI_LATENT_IN) {
       const int q_rows = l.heads * l.q_stride, g_rows = l.heads * l.v_dim;
       if (n < q_rows) {
         const int d = n % l.q_stride - l.head_dim;
-        if (d >= 0) {
-          float e[4] = {v[0], v[1], v[2], v[3]};
-          rotate(l, g.position + m, d, e[0], e[1]);
-          rotate(l, g.position + m, d + 2, e[2], e[3]);
-          v = f32x4{e[0], e[1], e[2], e[3]};
-        }
-        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * q_rows + n, v);
+        if (d >= 0) turn(g.position + m, d, lo, hi);
+        store8(out + row * q_rows + n, lo, hi);
       } else if (n < q_rows + g_rows) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * g_rows + n - q_rows, v);
+        store8(out2 + row * g_rows + n - q_rows, each(lo, gate), each(hi, gate));
       } else {
-        store4(g.f0 + static_cast<size_t>(m) * (l.rank + l.rot_dim) + n - q_rows - g_rows, v);
+        store8(g.f0 + row * (l.rank + l.rot_dim) + n - q_rows - g_rows, lo, hi);
       }
-      break;
-    }
-    case EPI_GEGLU: {
-      const bool silu = l.act == QMK_ACT_SILU;
-      const float a = (silu ? v[0] * sigmoid(v[0]) : gelu_tanh(v[0])) * v[1], b = (silu ? v[2] * sigmoid(v[2]) : gelu_tanh(v[2])) * v[3];
-      put2(Operand<T>{static_cast<T*>(g.out), g.out_part}, static_cast<size_t>(m) * l.ff + n / 2, a, b);
-      break;
-    }
-    case EPI_WKV_IN: {
+    } else if constexpr (EPI == EPI_GEGLU) {
+      const f32x4 a = {lo[0], lo[2], hi[0], hi[2]}, up = {lo[1], lo[3], hi[1], hi[3]};
+      put4(Operand<T>{out, g.out_part}, row * l.ff + n / 2, (l.act == QMK_ACT_SILU ? each(a, silu) : each(a, gelu)) * up);
+    } else if constexpr (EPI == EPI_WKV_IN) {
       const int N = l.heads * l.head_dim;
       if (group < 3) {
-        store4(g.f0 + (static_cast<size_t>(group) * g.rows_cap + m) * N + n, v);
+        store8(g.f0 + (static_cast<size_t>(group) * g.rows_cap + m) * N + n, lo, hi);
       } else if (group == 3) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= sigmoid(v[i]);
-        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * N + n, v);
+        store8(out + row * N + n, each(lo, silu), each(hi, silu));
       } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = tanhf(v[i]);
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.rank + n, v);
+        const auto bound = [](float x) { return tanhf(x); };
+        store8(out2 + row * l.rank + n, each(lo, bound), each(hi, bound));
       }
-      break;
-    }
-    case EPI_WKV_DECAY: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = expf(-expf(v[i] + b[i]));
-      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    case EPI_CAPPED_LOGITS: {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = soft_cap(v[i] * g.logit_scale, g.logit_softcap);
-      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    case EPI_ADD: {
-      float* x = g.f0 + static_cast<size_t>(m) * g.ldo + n;
-      store4(x, read4(x) + v);
-      break;
-    }
-    case EPI_ATTENTION_IN: {
-      const int q_rows = l.heads * l.q_stride, k_rows = l.kv_heads * l.head_dim, v_rows = l.kv_heads * l.v_dim, row = l.head_dim + l.v_dim, pos = g.position + m;
-      T* cache = static_cast<T*>(l.cache) + (static_cast<size_t>(g.slot) * l.ring + pos % l.ring) * l.kv_heads * row;
+    } else if constexpr (EPI == EPI_WKV_DECAY) {
+      const auto decay = [](float x) { return expf(-expf(x)); };
+      store8(g.f0 + row * g.ldo + n, each(lo + b[0], decay), each(hi + b[1], decay));
+    } else if constexpr (EPI == EPI_CAPPED_LOGITS) {
+      const auto cap = [&](float x) { return soft_cap(x * g.logit_scale, g.logit_softcap); };
+      store8(g.f0 + row * g.ldo + n, each(lo, cap), each(hi, cap));
+    } else if constexpr (EPI == EPI_ADD) {
+      float* x = g.f0 + row * g.ldo + n;
+      store8(x, read4(x) + lo, read4(x + 4) + hi);
+    } else if constexpr (EPI == EPI_ATTENTION_IN) {
+      const int q_rows = l.heads * l.q_stride, k_rows = l.kv_heads * l.head_dim, v_rows = l.kv_heads * l.v_dim, width = l.head_dim + l.v_dim, pos = g.position + m;
+      T* cache = static_cast<T*>(l.cache) + (static_cast<size_t>(g.slot) * l.ring + pos % l.ring) * l.kv_heads * width;
       if (n < q_rows + k_rows) {
         const int d = n < q_rows ? n % l.q_stride : (n - q_rows) % l.head_dim;
-        float e[4] = {v[0], v[1], v[2], v[3]};
-        rotate(l, pos, d, e[0], e[1]);
-        rotate(l, pos, d + 2, e[2], e[3]);
-        v = f32x4{e[0], e[1], e[2], e[3]};
-        store4(n < q_rows ? static_cast<T*>(g.out) + static_cast<size_t>(m) * q_rows + n : cache + (n - q_rows) / l.head_dim * row + d, v);
+        turn(pos, d, lo, hi);
+        store8(n < q_rows ? out + row * q_rows + n : cache + (n - q_rows) / l.head_dim * width + d, lo, hi);
       } else if (n < q_rows + k_rows + v_rows) {
         const int c = n - q_rows - k_rows;
-        store4(cache + c / l.v_dim * row + l.head_dim + c % l.v_dim, v);
+        store8(cache + c / l.v_dim * width + l.head_dim + c % l.v_dim, lo, hi);
       } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.mix_width + n - q_rows - k_rows - v_rows, v);
+        store8(out2 + row * l.mix_width + n - q_rows - k_rows - v_rows, each(lo, gate), each(hi, gate));
       }
-      break;
-    }
-    case EPI_DELTA_IN: {
+    } else if constexpr (EPI == EPI_DELTA_IN) {
       const int channels = conv_channels(l), ranks = l.rank + l.gate_rank;
-      if (n < channels) {
-        store4(g.f1 + static_cast<size_t>(m) * channels + n, v);
-      } else if (n < channels + ranks) {
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * ranks + n - channels, v);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
-        store4(g.f0 + static_cast<size_t>(m) * g.ldo + n - channels - ranks, v);
-      }
-      break;
-    }
-    case EPI_DELTA_DECAY: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = delta_decay(l, n / l.head_dim, v[i] + b[i]);
-      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    case EPI_SIGMOID: {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = sigmoid(v[i]);
-      store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    case EPI_GLA_IN: {
+      if (n < channels) store8(g.f1 + row * channels + n, lo, hi);
+      else if (n < channels + ranks) store8(out2 + row * ranks + n - channels, lo, hi);
+      else store8(g.f0 + row * g.ldo + n - channels - ranks, each(lo, gate), each(hi, gate));
+    } else if constexpr (EPI == EPI_DELTA_DECAY) {
+      const int head = n / l.head_dim;
+      const auto decay = [&](float x) { return delta_decay(l, head, x); };
+      store8(g.f0 + row * g.ldo + n, each(lo + b[0], decay), each(hi + b[1], decay));
+    } else if constexpr (EPI == EPI_SIGMOID) {
+      store8(out + row * g.ldo + n, each(lo, gate), each(hi, gate));
+    } else if constexpr (EPI == EPI_GLA_IN) {
       const int qkv = 2 * l.heads * l.head_dim + l.mix_width;
-      if (n < qkv) {
-        store4(g.f0 + static_cast<size_t>(m) * qkv + n, v);
-      } else if (n < qkv + l.mix_width) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= sigmoid(v[i]);
-        store4(static_cast<T*>(g.out) + static_cast<size_t>(m) * l.mix_width + n - qkv, v);
-      } else {
-        store4(static_cast<T*>(g.out2) + static_cast<size_t>(m) * l.rank + n - qkv - l.mix_width, v);
-      }
-      break;
+      if (n < qkv) store8(g.f0 + row * qkv + n, lo, hi);
+      else if (n < qkv + l.mix_width) store8(out + row * l.mix_width + n - qkv, each(lo, silu), each(hi, silu));
+      else store8(out2 + row * l.rank + n - qkv - l.mix_width, lo, hi);
+    } else if constexpr (EPI == EPI_GLA_DECAY) {
+      const auto decay = [&](float x) { return gla_decay(l, x); };
+      store8(g.f0 + row * g.ldo + n, each(lo + b[0], decay), each(hi + b[1], decay));
+    } else {
+      static_assert(EPI == EPI_LOGITS, "every epilogue has its place");
+      store8(g.f0 + row * g.ldo + n, lo, hi);
     }
-    case EPI_GLA_DECAY: {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(l.mid_b + n);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = gla_decay(l, v[i] + b[i]);
-      store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v);
-      break;
-    }
-    default: store4(g.f0 + static_cast<size_t>(m) * g.ldo + n, v); break;
   }
-}
+};
 
 // ---- tiles ----
 // A tile is BM tokens x BN weight rows, BK columns a step; a wave owns WM x WN of it and takes all columns, one after the other.
@@ -337,7 +313,7 @@ struct Tile {
   static constexpr int kTm = WM / 16, kTn = WN / 16;     // a wave's fragments
   static constexpr int kRow = BK / 8;                                           // a row of a step: units of 16 bytes
   static constexpr int kUnits = (BM + BN) * kRow;
-  static constexpr bool kSplits = kTn * kTm <= 8;                               // may be cut along K
+  static constexpr bool kSplits = kTn * kTm <= 12;                              // may be cut along K, with an fp32 side
   static constexpr int kSteps = BK / 32;                                        // matrix steps of a step
   static constexpr int kOutUnits = BM * BN / 4, kPasses = kOutUnits > kStages * kUnits ? 2 : 1;
   static constexpr int kLds = kStages * kUnits > kOutUnits / kPasses ? kStages * kUnits : kOutUnits / kPasses;
@@ -356,14 +332,13 @@ __device__ __forceinline__ int xcd_order(int id, int total) {
 template <int COUNT, int THREADS>
 __device__ __forceinline__ bool sum_parts(const GemmArgs& g, int tile, int part, f32x4 (&sums)[COUNT], int* last) {
   const int tid = threadIdx.x;
-  float* all = g.partial + static_cast<size_t>(tile) * g.splits * COUNT * THREADS * 4 + tid * 4;
-  auto at = [&](int p, int i) { return all + (static_cast<size_t>(p) * COUNT + i) * THREADS * 4; };
+  // Device-coherent units of 16 bytes (sc1); a line is read once in a launch, behind its writer's ticket.
+  constexpr int kCoherent = 16;
+  float* all = g.partial + static_cast<size_t>(tile) * g.splits * COUNT * THREADS * 4;
+  const auto unit = __builtin_amdgcn_make_buffer_rsrc(all, 0, -1, 0x00027000);
+  auto at = [&](int p, int i) { return ((p * COUNT + i) * THREADS + tid) * 16; };
 #pragma unroll
-  for (int i = 0; i < COUNT; ++i) {
-    uint64_t* to = reinterpret_cast<uint64_t*>(at(part, i));
-    __hip_atomic_store(to, __builtin_bit_cast(uint64_t, f32x2_t{sums[i][0], sums[i][1]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(to + 1, __builtin_bit_cast(uint64_t, f32x2_t{sums[i][2], sums[i][3]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  for (int i = 0; i < COUNT; ++i) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, sums[i]), unit, at(part, i), 0, kCoherent);
   release_stores();
   __syncthreads();
   if (tid == 0) {
@@ -375,13 +350,13 @@ __device__ __forceinline__ bool sum_parts(const GemmArgs& g, int tile, int part,
   if (!*last) return false;
 #pragma unroll
   for (int i = 0; i < COUNT; ++i) sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int kBatch = COUNT <= 4 ? 4 : 2;      // parts asked for together
+  constexpr int kBatch = COUNT <= 8 ? 4 : 2;      // parts asked for together
   for (int p = 0; p < g.splits; p += kBatch) {
     v4u r[kBatch][COUNT];
 #pragma unroll
     for (int b = 0; b < kBatch; ++b)
 #pragma unroll
-      for (int i = 0; i < COUNT; ++i) r[b][i] = ld_shared128(at(min(p + b, g.splits - 1), i));
+      for (int i = 0; i < COUNT; ++i) r[b][i] = __builtin_amdgcn_raw_buffer_load_b128(unit, at(min(p + b, g.splits - 1), i), 0, kCoherent);
 #pragma unroll
     for (int b = 0; b < kBatch; ++b)
       if (p + b < g.splits)
@@ -397,94 +372,165 @@ __global__ __launch_bounds__(kPfThreads) void clear_tickets(int32_t* tickets, in
   for (int i = threadIdx.x; i < count; i += kPfThreads) tickets[i] = 0;
 }
 
-// All streams of the residual for quads id, id + step, .. of a tile: the next quad's streams are asked for before this one's
-// are mixed.
-template <class At, class Value>
-__device__ __forceinline__ void residual_quads(const GemmArgs& g, int id, int total, int step, At&& at, Value&& value) {
-  const QmkHybridLayer& l = g.layer;
-  const int S = g.streams, D = g.width;
-  const float* hc = l.hc + (g.down ? S * (S + 2) : 0);
-  f32x4 old[kMaxStreams] = {}, ahead[kMaxStreams] = {};
-  auto load = [&](f32x4(&to)[kMaxStreams], int i) {
-    int m, n;
-    if (i >= total || !at(i, m, n)) return;
-    const float* x = g.f0 + static_cast<size_t>(m) * S * D + n;
+// All streams of the residual for quads id, id + step, .. of a tile, `BATCH` at a time: the next batch's streams are asked for before this one's are mixed, the first
+// one's (`begin`) ahead of the products' exchange where registers allow.  Few workgroups make it a chain of trips to memory, many are bound by its bytes (us, one
+// quad at a time with coefficients read among the stores -> now: 200 x 2048 x 64 on tiles of 64 x 128 in fp32 22.5 -> 14.9; 1531 x 2048 x 2048 on Turns96 45 -> 34).
+template <int BATCH, int STREAMS>
+struct ResidualQuads {
+  const GemmArgs& g;
+  f32x4 old[BATCH][STREAMS];
+
+  template <class At>
+  __device__ __forceinline__ void load(f32x4 (&to)[BATCH][STREAMS], int id, int total, int step, At&& at) const {
+    const int S = g.streams, D = g.width;
 #pragma unroll
-    for (int s = 0; s < kMaxStreams; ++s)
-      if (s < S) to[s] = read4(x + static_cast<size_t>(s) * D);
-  };
-  load(old, id);
+    for (int b = 0; b < BATCH; ++b) {
+      int m, n;
+      if (id + b * step >= total || !at(id + b * step, m, n)) continue;
+      const float* x = g.f0 + static_cast<size_t>(m) * S * D + n;
+#pragma unroll
+      for (int s = 0; s < STREAMS; ++s)
+        if (s < S) to[b][s] = read4(x + static_cast<size_t>(s) * D);
+    }
+  }
+  template <class At>
+  __device__ __forceinline__ void begin(int id, int total, int step, At&& at) { load(old, id, total, step, at); }
+  template <class At, class Value>
+  __device__ __forceinline__ void run(int id, int total, int step, At&& at, Value&& value) {
+    const QmkHybridLayer& l = g.layer;
+    const int S = g.streams, D = g.width;
+    // (Said to be constant: read among the stores, a coefficient would wait for all stores before it.)
+    ConstFloat *hc = (ConstFloat*)(l.hc + (g.down ? S * (S + 2) : 0)), *next = (ConstFloat*)g.next;
 #pragma unroll 1
-  for (; id < total; id += step) {
-    load(ahead, id + step);
-    int m, n;
-    if (at(id, m, n)) {
-      const f32x4 v = value(id);
-      float* x = g.f0 + static_cast<size_t>(m) * S * D + n;
-      f32x4 u = {};
+    for (; id < total; id += BATCH * step) {
+      f32x4 ahead[BATCH][STREAMS];
+      load(ahead, id + BATCH * step, total, step, at);
 #pragma unroll
-      for (int t = 0; t < kMaxStreams; ++t) {
-        if (t < S) {
-          f32x4 now = v * hc[S + t];
+      for (int b = 0; b < BATCH; ++b) {
+        int m, n;
+        if (id + b * step < total && at(id + b * step, m, n)) {
+          const f32x4 v = value(id + b * step);
+          float* x = g.f0 + static_cast<size_t>(m) * S * D + n;
+          f32x4 u = {};
 #pragma unroll
-          for (int s = 0; s < kMaxStreams; ++s)
-            if (s < S) now += old[s] * hc[2 * S + s * S + t];
-          store4(x + static_cast<size_t>(t) * D, now);
-          u += now * g.next[t];
+          for (int t = 0; t < STREAMS; ++t) {
+            if (t < S) {
+              f32x4 now = v * hc[S + t];
+#pragma unroll
+              for (int s = 0; s < STREAMS; ++s)
+                if (s < S) now += old[b][s] * hc[2 * S + s * S + t];
+              store4(x + static_cast<size_t>(t) * D, now);
+              u += now * next[t];
+            }
+          }
+          store4(g.f1 + static_cast<size_t>(m) * D + n, u);
         }
       }
-      store4(g.f1 + static_cast<size_t>(m) * D + n, u);
-    }
 #pragma unroll
-    for (int s = 0; s < kMaxStreams; ++s) old[s] = ahead[s];
+      for (int b = 0; b < BATCH; ++b)
+#pragma unroll
+        for (int s = 0; s < STREAMS; ++s) old[b][s] = ahead[b][s];
+    }
   }
-}
+};
 
-// A workgroup's accumulators -> epilogue, through LDS (quads of a row exchanged by its number): the lanes of a row then
-// write neighbouring outputs of one token.  Unit LDS of the array is one word beside it.  (A kernel has one LDS array: with two,
-// this compiler waits for all requests before every read of the main loop, which costs half of the rate.)
-template <class T, class S, int LDS>
+// A wave's accumulators -> epilogue, through its own part of LDS (quads of a row exchanged by its number): a lane then has eight neighbouring outputs of one
+// token, the same eight of every token it takes, and the lanes of a token write side by side (us, four outputs at a time with their columns worked out for each, by the whole
+// workgroup -> so: 2048 x 16384 x 2048 with gate and up 151 -> 141, 1531 x 16384 x 2048 129 -> 119).  Unit LDS of the array is one word beside it.  (A kernel has one LDS
+// array: with two, this compiler waits for all requests before every read of the main loop, which costs half of the rate.)
+template <class T, class S, int LDS, int BATCH = 1>
 __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int tile, int part, int m0, int n0, int N, v4u* lds, f32x4 (&acc)[S::kTn][S::kTm]) {
-  constexpr int kQuads = S::BN / 4, kPassM = S::WM / S::kPasses, kRows = S::BM / S::kPasses, kTm = S::kTm;
+  constexpr int kQuads = S::WN / 4, kPassM = S::WM / S::kPasses, kTm = S::kTm, kGroups = S::WN / 8;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
-  f32x4* out = reinterpret_cast<f32x4*>(lds);
   f32x4 sums[S::kTn * kTm];
+  constexpr int kRowQuads = S::BN / 4, kRows = S::BM / S::kPasses, kFewStreams = BATCH == 1 ? kMaxStreams : 4;
+  auto residual_at = [&](int pass) {
+    return [=, &g](int id, int& m, int& n) {
+      const int r = id / kRowQuads;
+      m = m0 + r / kPassM * S::WM + pass * kPassM + r % kPassM;
+      n = n0 + id % kRowQuads * 4;
+      return m < g.M && n < N;
+    };
+  };
+  // (The first batch ahead of the sums, where registers allow.)
+  constexpr bool kEarly = BATCH >= 4;
+  ResidualQuads<BATCH, kFewStreams> early{g};
+  const bool few_streams = g.epi == EPI_RESIDUAL && g.streams <= kFewStreams;
+  if (kEarly && few_streams) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(0));
   __syncthreads();
 #pragma unroll
   for (int c = 0; c < S::kTn * kTm; ++c) sums[c] = acc[c / kTm][c % kTm];
-  if constexpr (S::kSplits)
+  if constexpr (S::kSplits && sizeof(T) == 4)
     if (g.splits > 1 && !sum_parts<S::kTn * kTm, S::kThreadCount>(g, tile, part, sums, reinterpret_cast<int*>(lds + LDS))) return;
+  f32x4 *all = reinterpret_cast<f32x4*>(lds), *out = all + wave * kPassM * kQuads;
+  auto place = [](int r, int quad) { return r * kQuads + (quad ^ (r & (kQuads - 1) & 15)); };
+  const int column = n0 + wn * S::WN;
 #pragma unroll
   for (int pass = 0; pass < S::kPasses; ++pass) {
-    if (pass > 0) __syncthreads();
+    const int first = m0 + wm * S::WM + pass * kPassM;
 #pragma unroll
     for (int i = 0; i < kTm / S::kPasses; ++i)
 #pragma unroll
       for (int j = 0; j < S::kTn; ++j) {
-        const int r = wm * kPassM + i * 16 + (lane & 15), quad = wn * (S::WN / 4) + j * 4 + (lane >> 4);
-        out[r * kQuads + (quad ^ (r & (kQuads - 1) & 15))] = sums[j * kTm + pass * (kTm / S::kPasses) + i];
+        const int r = i * 16 + (lane & 15), quad = j * 4 + (lane >> 4);
+        out[place(r, quad)] = sums[j * kTm + pass * (kTm / S::kPasses) + i];
       }
-    __syncthreads();
-    auto at = [&](int id, int& m, int& n) {
-      const int r = id / kQuads;
-      m = m0 + r / kPassM * S::WM + pass * kPassM + r % kPassM;
-      n = n0 + id % kQuads * 4;
-      return m < g.M && n < N;
+    __builtin_amdgcn_wave_barrier();
+    auto rows = [&](auto epi) {
+      constexpr int kEachTime = 64 / kGroups;      // tokens (of 96 columns five, by 60 lanes)
+      const int n = column + lane % kGroups * 8;
+      if (n >= N || lane >= kEachTime * kGroups) return;
+      const Epilogue<T, decltype(epi)::value> put(g, group, n);
+      const int end = min(kPassM, g.M - first);
+#pragma unroll 2
+      for (int r = lane / kGroups; r < end; r += kEachTime) put(first + r, out[place(r, lane % kGroups * 2)], out[place(r, lane % kGroups * 2 + 1)]);
     };
-    auto value = [&](int id) {
-      const int r = id / kQuads;
-      return out[r * kQuads + (id % kQuads ^ (r & (kQuads - 1) & 15))];
-    };
-    if (g.epi == EPI_RESIDUAL) {
-      residual_quads(g, tid, kRows * kQuads, S::kThreadCount, at, value);
-    } else {
-#pragma unroll 1
-      for (int id = tid; id < kRows * kQuads; id += S::kThreadCount) {
-        int m, n;
-        if (at(id, m, n)) epilogue<T>(g, group, m, n, value(id));
+    switch (g.epi) {
+      case EPI_RESIDUAL: {      // the streams of a token are long runs: all waves take rows of the whole tile
+        auto product = [&](int id) {
+          const int r = id / kRowQuads, q = id % kRowQuads, owner = q / kQuads * S::kWavesM + r / kPassM;
+          return all[owner * kPassM * kQuads + place(r % kPassM, q % kQuads)];
+        };
+        __syncthreads();
+        if (few_streams) {
+          if constexpr (kEarly) {
+            if (pass > 0) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
+            early.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
+          } else {
+            ResidualQuads<BATCH, kFewStreams> few{g};
+            few.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
+            few.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
+          }
+        } else if constexpr (kFewStreams < kMaxStreams) {
+          ResidualQuads<1, kMaxStreams> many{g};
+          many.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
+          many.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
+        }
+        __syncthreads();
+        break;
       }
+#define QMK_EPILOGUE(EPI) case EPI: rows(std::integral_constant<int, EPI>{}); break;
+      QMK_EPILOGUE(EPI_STORE)
+      QMK_EPILOGUE(EPI_STORE_VALUES)
+      QMK_EPILOGUE(EPI_RGLRU_IN)
+      QMK_EPILOGUE(EPI_LRU_GATES)
+      QMK_EPILOGUE(EPI_LATENT_IN)
+      QMK_EPILOGUE(EPI_GEGLU)
+      QMK_EPILOGUE(EPI_WKV_IN)
+      QMK_EPILOGUE(EPI_WKV_DECAY)
+      QMK_EPILOGUE(EPI_LOGITS)
+      QMK_EPILOGUE(EPI_CAPPED_LOGITS)
+      QMK_EPILOGUE(EPI_ADD)
+      QMK_EPILOGUE(EPI_ATTENTION_IN)
+      QMK_EPILOGUE(EPI_DELTA_IN)
+      QMK_EPILOGUE(EPI_DELTA_DECAY)
+      QMK_EPILOGUE(EPI_SIGMOID)
+      QMK_EPILOGUE(EPI_GLA_IN)
+      QMK_EPILOGUE(EPI_GLA_DECAY)
+#undef QMK_EPILOGUE
     }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -515,46 +561,60 @@ __device__ __forceinline__ void wait_outstanding() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(n) : "memory");
 }
 
+// Until at most `n` of this wave's vector-memory requests are outstanding and none of its LDS reads, said with the builtin: the compiler's own waits take account of it.
+template <int n>
+__device__ __forceinline__ void wait_known() {
+  static_assert(n >= 0 && n < 64, "six bits");
+  __builtin_amdgcn_s_waitcnt((n & 15) | 7 << 4 | (n >> 4) << 14);
+}
+
 // The tiles of a step, bf16: memory -> LDS without passing through registers, kStages buffers deep.  A row's units are exchanged
 // by its number on the memory side (the LDS side of such a load is one run of 64 units per wave), so that fragment reads do
-// not conflict.
+// not conflict.  A lane's places are offsets of 32 bits that stay, and one scalar moves on, so that a request is one instruction (with pointers that move on
+// it is two more).
 template <class S, int PARTS = 1>      // of the tokens' side
 struct Stages {
-  static constexpr int kRowsA = S::BM * PARTS, kUnits = (kRowsA + S::BN) * S::kRow, kLoads = (kUnits + S::kThreadCount - 1) / S::kThreadCount;
+  static constexpr int kRowsA = S::BM * PARTS, kUnitsA = kRowsA * S::kRow, kUnits = (kRowsA + S::BN) * S::kRow, kLoads = (kUnits + S::kThreadCount - 1) / S::kThreadCount;
   static constexpr int kLastWaves = (kUnits - (kLoads - 1) * S::kThreadCount) / 64;      // waves that take part in a stage's last load
-  static_assert(kUnits % 64 == 0, "a wave's loads are whole");
+  static_assert(kUnits % 64 == 0 && kUnitsA % 64 == 0, "a wave's loads are whole, and of one side");
+  static_assert(PARTS == 1 || S::BM * S::kRow % S::kThreadCount == 0, "a load is of one part");
   using Lds = __attribute__((address_space(3))) v4u;      // said outright: a pointer kept in a struct may become a generic one
-  const u16* from[kLoads];      // this thread's places in a stage: unit i * threads + tid, tokens first
+  __amdgpu_buffer_rsrc_t a[PARTS], w;      // from the tile's first rows on: they are far less than 4 GB
+  uint32_t from[kLoads], at = 0;           // this thread's places in a stage: unit i * threads + tid, tokens first; columns of the stage
   Lds* lds;
   int wave;
 
   static __device__ __forceinline__ int exchange(int r) { return S::kRow == 4 ? (r >> 1) & 3 : r & 7; }
   __device__ __forceinline__ Stages(const GemmArgs& g, const Place& p, v4u* buffers, int wave_number) : lds((Lds*)buffers), wave(wave_number) {
-    const u16* a = static_cast<const u16*>(g.a) + p.group * g.a_step + p.first * S::BK;
-    const u16* w = static_cast<const u16*>(g.w) + p.group * g.w_step + p.first * S::BK;
+    auto rows = [&](const void* base, long long skip, int row, int ld) {
+      const u16* first = static_cast<const u16*>(base) + skip + static_cast<size_t>(row) * ld + p.first * S::BK;
+      return __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(first), 0, -1, 0x00027000);
+    };
+#pragma unroll
+    for (int part = 0; part < PARTS; ++part) a[part] = rows(g.a, p.group * g.a_step + (PARTS == 1 ? 0 : part * g.a_part), p.m0, g.lda);
+    w = rows(g.w, p.group * g.w_step, p.n0, g.ldw);
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int u = i * S::kThreadCount + threadIdx.x, r = u / S::kRow, c = ((u % S::kRow) ^ exchange(r)) * 8;
-      from[i] = r < kRowsA ? a + static_cast<size_t>(min(p.m0 + (PARTS == 1 ? r : r % S::BM), g.M - 1)) * g.lda + c
-                           : w + static_cast<size_t>(min(p.n0 + r - kRowsA, p.N - 1)) * g.ldw + c;
-      if constexpr (PARTS > 1) from[i] += r < kRowsA ? r / S::BM * g.a_part : 0;
+      from[i] = (r < kRowsA ? min(PARTS == 1 ? r : r % S::BM, g.M - 1 - p.m0) * g.lda + c : min(r - kRowsA, p.N - 1 - p.n0) * g.ldw + c) * 2;
     }
   }
   __device__ __forceinline__ void issue(int buf) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       if (i == kLoads - 1 && kLastWaves * 64 < S::kThreadCount && wave >= kLastWaves) continue;
-      const auto* src = (const __attribute__((address_space(1))) uint32_t*)from[i];
       auto* dst = (__attribute__((address_space(3))) uint32_t*)(lds + buf * kUnits + i * S::kThreadCount + wave * 64);
-      __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
-      from[i] += S::BK;
+      const bool tokens = (i + 1) * S::kThreadCount <= kUnitsA || (i * S::kThreadCount < kUnitsA && i * S::kThreadCount + wave * 64 < kUnitsA);
+      constexpr int kPart = S::BM * S::kRow;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(tokens ? a[PARTS == 1 ? 0 : min(i * S::kThreadCount / kPart, PARTS - 1)] : w, dst, 16, from[i], at, 0, 0);
     }
+    at += S::BK * 2;
   }
   // Until at most `stages` stages of this wave's are outstanding.
   template <int stages>
   __device__ __forceinline__ void wait() const {
-    if (kLastWaves * 64 == S::kThreadCount || wave < kLastWaves) wait_outstanding<stages * kLoads>();
-    else wait_outstanding<stages * (kLoads - 1)>();
+    if (kLastWaves * 64 == S::kThreadCount || wave < kLastWaves) wait_known<stages * kLoads>();
+    else wait_known<stages * (kLoads - 1)>();
   }
   __device__ __forceinline__ void fragments(int buf, int q, int wm, int wn, Frag<u16> (&fa)[PARTS][S::kTm], Frag<u16> (&fw)[S::kTn]) const {
     const Lds *la = lds + buf * kUnits, *lw = la + kRowsA * S::kRow;
@@ -579,18 +639,20 @@ struct Stages {
 template <class S, int PARTS>
 __device__ __forceinline__ void multiply(const Frag<u16> (&fa)[PARTS][S::kTm], const Frag<u16> (&fw)[S::kTn], f32x4 (&acc)[S::kTn][S::kTm]) {
 #pragma unroll
-  for (int i = 0; i < S::kTm; ++i)
+  for (int i = 0; i < S::kTm; ++i) {
+    if constexpr (PARTS == 1) {
 #pragma unroll
-    for (int j = 0; j < S::kTn; ++j) {
-      if constexpr (PARTS == 1) {
-        acc[j][i] = mma(fw[j], fa[0][i], acc[j][i]);
-      } else {      // 32 columns by themselves, small parts first, then one rounded addition
-        f32x4 t = {};
+      for (int j = 0; j < S::kTn; ++j) acc[j][i] = mma(fw[j], fa[0][i], acc[j][i]);
+    } else {      // 32 columns by themselves, small parts first, then one rounded addition
+      f32x4 t[S::kTn] = {};
 #pragma unroll
-        for (int part = PARTS - 1; part >= 0; --part) t = mma(fw[j], fa[part][i], t);
-        acc[j][i] += t;
-      }
+      for (int part = PARTS - 1; part >= 0; --part)
+#pragma unroll
+        for (int j = 0; j < S::kTn; ++j) t[j] = mma(fw[j], fa[part][i], t[j]);
+#pragma unroll
+      for (int j = 0; j < S::kTn; ++j) acc[j][i] += t[j];
     }
+  }
 }
 
 // An infinite value on the bf16 side makes products with those parts of a finite value that are zero undefined, where the product with the whole
@@ -613,16 +675,25 @@ __device__ __forceinline__ void resolve_undefined(const Place& p, f32x4 (&acc)[S
     }
 }
 
-// out[m][n] = sum_k a[m][k] w[n][k], bf16 x bf16 or the tokens' side in three parts, K a multiple of BK.  The weights are the matrix instruction's first operand,
+template <class S>
+__device__ __forceinline__ void resolve_undefined(const GemmArgs& g, const Place& p, int wm, int wn, f32x4 (&acc)[S::kTn][S::kTm]) {
+  const int lane = threadIdx.x & 63;
+  const u16 *a = static_cast<const u16*>(g.a) + p.group * g.a_step + (lane >> 4) * 8, *w = static_cast<const u16*>(g.w) + p.group * g.w_step + (lane >> 4) * 8;
+  resolve_undefined<S>(
+      p, acc, [&](int i, int k) { return load_frag(a + static_cast<size_t>(min(p.m0 + wm * S::WM + i * 16 + (lane & 15), g.M - 1)) * g.lda + k); },
+      [&](int j, int k) { return load_frag(w + static_cast<size_t>(min(p.n0 + wn * S::WN + j * 16 + (lane & 15), p.N - 1)) * g.ldw + k); });
+}
+
+// out[m][n] = sum_k a[m][k] w[n][k], bf16 x bf16, K a multiple of BK.  The weights are the matrix instruction's first operand,
 // so a lane ends up with four consecutive outputs of one token.  Two to eight waves; several workgroups share a CU where LDS has room.
-template <class T, class S, int PARTS = 1>
-__global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g) {
-  constexpr int kAhead = S::kStages - 1, kStageUnits = S::kStages * Stages<S, PARTS>::kUnits, kLds = kStageUnits > S::kLds ? kStageUnits : S::kLds;
-  __shared__ __align__(16) v4u lds[kLds + 1];
+template <class T, class S>
+__global__ __launch_bounds__(S::kThreadCount, S::kThreadCount == 512 ? 4 : 1) void gemm_direct(const GemmArgs g) {
+  constexpr int kAhead = S::kStages - 1;
+  __shared__ __align__(16) v4u lds[S::kLds + 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % S::kWavesM, wn = wave / S::kWavesM;
   const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
-  Stages<S, PARTS> stages(g, p, lds, wave);
+  Stages<S> stages(g, p, lds, wave);
   f32x4 acc[S::kTn][S::kTm] = {};
 #pragma unroll
   for (int s = 0; s < kAhead; ++s)
@@ -638,19 +709,88 @@ __global__ __launch_bounds__(S::kThreadCount) void gemm_direct(const GemmArgs g)
     if (s + kAhead < p.steps) stages.issue(buf == 0 ? S::kStages - 1 : buf - 1);
 #pragma unroll
     for (int kk = 0; kk < S::kSteps; ++kk) {
-      Frag<u16> fa[PARTS][S::kTm], fw[S::kTn];
+      Frag<u16> fa[1][S::kTm], fw[S::kTn];
       stages.fragments(buf, kk * 4 + (lane >> 4), wm, wn, fa, fw);
-      multiply<S, PARTS>(fa, fw, acc);
+      multiply<S, 1>(fa, fw, acc);
     }
     buf = buf + 1 == S::kStages ? 0 : buf + 1;
   }
-  if constexpr (PARTS > 1) {
-    const u16 *a = static_cast<const u16*>(g.a) + p.group * g.a_step + (lane >> 4) * 8, *w = static_cast<const u16*>(g.w) + p.group * g.w_step + (lane >> 4) * 8;
-    resolve_undefined<S>(
-        p, acc, [&](int i, int k) { return load_frag(a + static_cast<size_t>(min(p.m0 + wm * S::WM + i * 16 + (lane & 15), g.M - 1)) * g.lda + k); },
-        [&](int j, int k) { return load_frag(w + static_cast<size_t>(min(p.n0 + wn * S::WN + j * 16 + (lane & 15), p.N - 1)) * g.ldw + k); });
+  finish_tile<T, S, S::kLds, 2>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+}
+
+// Scheduling of a block of matrix instructions: one LDS read ahead of each of the first, the requests for a stage among the rest.
+template <int PRODUCTS, int READS, int REQUESTS>
+__device__ __forceinline__ void interleave() {
+#pragma unroll
+  for (int i = 0; i < READS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    if (i < PRODUCTS) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
   }
-  finish_tile<T, S, kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+  constexpr int kEach = REQUESTS > 0 && PRODUCTS - READS >= 2 * REQUESTS ? 2 : 1;
+#pragma unroll
+  for (int i = 0; i < REQUESTS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+    if (READS + i * kEach < PRODUCTS) __builtin_amdgcn_sched_group_barrier(0x008, kEach, 0);
+  }
+}
+
+// The same as gemm_direct for larger tiles of bf16, one workgroup a CU or two.  What bounds them is LDS: a tile's rows are read by every wave that shares them,
+// 128 bytes a cycle, so waves take 64 x 64 where they can, and no wave may wait for its reads.  32 columns are multiplied while the fragments of the next 32 are
+// read into a second set of registers; one barrier a stage lies ahead of the first reads of the next one, where everybody has read the last of this one: its
+// buffer is filled again at once, kStages stages ahead.  (Launch bounds of eight waves also for four: with more registers to give away this compiler keeps
+// accumulators in the other half of the file and moves them at every step.)
+template <class T, class S, int PARTS = 1>
+__global__ __launch_bounds__(512, 2) void gemm_pipe(const GemmArgs g) {
+  static_assert(S::kSteps == 2 && S::kStages >= 2, "two matrix steps a stage");
+  constexpr int kDeep = S::kStages, kProducts = PARTS * S::kTm * S::kTn, kReads = PARTS * S::kTm + S::kTn, kRequests = Stages<S, PARTS>::kLoads;
+  constexpr int kStageUnits = kDeep * Stages<S, PARTS>::kUnits, kLds = kStageUnits > S::kLds ? kStageUnits : S::kLds;
+  __shared__ __align__(16) v4u lds[kLds + 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
+  const Place p = place_of<S>(g);
+  if (p.n0 >= p.N) return;
+  Stages<S, PARTS> stages(g, p, lds, wave);
+  auto barrier = [] {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4 acc[S::kTn][S::kTm] = {};
+  struct Fragments {
+    Frag<u16> a[PARTS][S::kTm], w[S::kTn];
+  } f[2];
+#pragma unroll
+  for (int s = 0; s < kDeep; ++s)
+    if (s < p.steps) stages.issue(s);
+  if (kDeep <= p.steps) stages.template wait<kDeep - 1>();
+  else wait_known<0>();
+  barrier();
+  stages.fragments(0, lane >> 4, wm, wn, f[0].a, f[0].w);
+  int buf = 0;
+  auto step = [&](auto more) {
+    constexpr bool MORE = decltype(more)::value;
+    wait_known<63>();      // (the first fragments)
+    __builtin_amdgcn_sched_barrier(0);
+    stages.fragments(buf, 4 + (lane >> 4), wm, wn, f[1].a, f[1].w);
+    multiply<S, PARTS>(f[0].a, f[0].w, acc);
+    if constexpr (MORE) interleave<kProducts, kReads, 0>();
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (MORE) stages.template wait<kDeep - 2>();
+    else wait_known<0>();
+    barrier();
+    const int next = buf + 1 == S::kStages ? 0 : buf + 1;
+    stages.fragments(next, lane >> 4, wm, wn, f[0].a, f[0].w);      // (behind the last stage: of a buffer that is there, for nobody)
+    if constexpr (MORE) stages.issue(buf);
+    multiply<S, PARTS>(f[1].a, f[1].w, acc);
+    if constexpr (MORE) interleave<kProducts, kReads, kRequests>();
+    __builtin_amdgcn_sched_barrier(0);
+    buf = next;
+  };
+  int s = 0;
+  for (; s + kDeep < p.steps; ++s) step(std::true_type{});
+  for (; s < p.steps; ++s) step(std::false_type{});
+  if constexpr (PARTS > 1) resolve_undefined<S>(g, p, wm, wn, acc);
+  finish_tile<T, S, kLds, 4>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
 
 // The same with eight waves, one workgroup a CU.  Two waves share a SIMD's matrix unit, and the halves of the workgroup take
@@ -881,26 +1021,28 @@ __global__ __launch_bounds__(kPfThreads) void gemm_short(const GemmArgs g) {
 
 // ---- which tiles ----
 // Few tokens: weight rows of a workgroup, deep steps, since a step's barrier and reads are most of its time (us, M x N x K, 64 x 16 in steps of 64 columns, of
-// 128, 32 x 16 in steps of 256: 43 x 2048 x 2048 with the residual's streams 12.2, 10.1, 9.5; 43 x 2048 x 6144 with them 26.4, 19.9, 17.3).
+// 128, 32 x 16 in steps of 256: 43 x 2048 x 2048 with the residual's streams 12.2, 10.1, 9.5; 43 x 2048 x 6144 with them 26.4, 19.9, 17.3; the last one now 7.9 and 14.9).
 using Few32 = Tile<32, 16, 256, 16, 16, 2, 4>;
 using Few64 = Tile<64, 16, 128, 16, 16, 4, 3>;
 using Tiles32 = Tile<64, 32, 64, 32, 16, 4, 4>;
-using Tiles64 = Tile<64, 64, 64, 32, 32, 4, 4>;
 using Wide64 = Tile<128, 64, 64, 32, 32, 8, 3>;
-// The tokens' side in three parts: it is what fills LDS, so few tokens a tile (us, 32 x 128 and 64 x 64 and 64 x 128 and 128 x 128: 200 x 2048 x 6144
-// 32, 35, 54, 169; 200 x 12288 x 2048 52, 58, 52, 63; 2048 x 2048 x 8192 260, 420, 291, 280).
-using TilesParts = Tile<32, 128, 64, 16, 64, 4, 2>;
-// Two matrix steps a turn where a wave's part is small: a turn's reads and products then outlast its barriers (us, M x N x K: 1531 x 2048 x 8192 with the residual's
-// streams Turns96 90, Wide64 120; 2048 x 2048 x 6144 Turns128 60, Wide64 75, 128 x 128 in steps of 32 columns 78).
+// Below with gemm_pipe (us, M x N x K, before -> with it: 512 x 2048 x 2048 Tiles64 14.5 -> 11.8; 2048 x 2048 x 2048 and x 8192 Turns128, halves of the workgroup in turns, 28.5
+// and 88 -> 22.6 and 73, on four waves of 64 x 64 26 and 76; 1536 x 4096 x 8192 Tall192 119 -> 95, 2048 x 4096 x 8192 Tall256 139 -> 122).
+using Tiles64 = Tile<64, 64, 64, 32, 32, 4, 4>;
 using Turns96 = Tile<96, 128, 64, 48, 32, 8, 4>;
 using Turns128 = Tile<128, 128, 64, 32, 64, 8, 4>;
-// Three stages where four do not fit (two workgroups of 128 x 128 on four waves a CU, which these replace: 4096 x 2048 x 8192 with the streams 188, Tall256 173; 3000 x
-// 2048 x 8192 with them 162, Tall192 133; 1900 x 8256 x 2048 76, Wide256 72).
-using Tall192 = Tile<192, 128, 64, 96, 32, 8, 3>;
+// Three stages where four do not fit.
+using Tall192 = Tile<192, 128, 64, 48, 64, 8, 3>;
 using Tall256 = Tile<256, 128, 64, 64, 64, 8, 3>;
 using Wide256 = Tile<128, 256, 64, 64, 64, 8, 3>;
+// With gemm_turns: accumulators leave no registers for a second set of fragments of 64 columns, and with steps of 32 the turns are as fast (2048 x 16384 x 2048 141, gemm_pipe 143).
 using Turns192 = Tile<192, 256, 32, 96, 64, 8, 4>;
 using Turns256 = Tile<256, 256, 32, 128, 64, 8, 4>;
+// The tokens' side in three parts, with gemm_pipe: it is what fills LDS (us, 32 x 128 in two stages without a second set of fragments -> the kind that is taken: 200 x
+// 2048 x 6144 with the streams 43 -> 34, 200 x 12288 x 2048 65 -> 40, 200 x 5696 x 2048 33 -> 26, 20 x 12288 x 2048 21 -> 16).
+using Parts32 = Tile<32, 128, 64, 16, 64, 4, 3>;
+using Parts64 = Tile<64, 128, 64, 32, 64, 4, 3>;
+using PartsWide = Tile<64, 192, 64, 32, 96, 4, 3>;
 
 }  // namespace hybrid
 }  // namespace qmk

@@ -76,15 +76,41 @@ inline RegisterTiles choose_register_tiles(int M, int N, int K, int groups, bool
   return c;
 }
 
-// Products whose tokens' side is in parts, cut along K until every CU has a workgroup (us, in 1, 2, 4, 8: 200 x 2048 x 6144 75, 44, 32, 42;
-// 200 x 5696 x 2048, 315 tiles 31, 39, 42; 20 x 12288 x 2048 24, 19, 18, 25).
-constexpr int kPartTileTokens = 32, kPartTileRows = 128;
-inline int choose_part_splits(int M, int N, int K, int groups) {
-  const long long tiles = static_cast<long long>((M + kPartTileTokens - 1) / kPartTileTokens) * ((N + kPartTileRows - 1) / kPartTileRows) * groups;
-  int splits = 1;
-  while (splits < 8 && tiles * splits < 256 && K / splits >= 512) splits *= 2;
-  return splits;
+// Products whose tokens' side is in three parts: the kind of tile and the number of parts along K, priced like the bf16 ones, an epilogue of the usual mixture
+// within `fixed`, and what a cut costs.  What decides is how full the chip is: a workgroup has it 256 at a time, and larger tiles read LDS less often
+// for a product.  us by (tokens x rows, cuts), x 12288 x 2048, 20 tokens: (32 x 128, 2) 15.8, (32 x 128, 4) 21.5, (64 x 128, 2) 19.8; 100: (64 x 128, 1) 27.2, (32 x 128, 1) 37,
+// (64 x 192, 1) 34; 200: (64 x 192, 1) 39.6, (64 x 128, 1) 53, (32 x 128, 1) 54; 200 x 2048 x 6144 with the streams: (32 x 128, 2) 34, (64 x 128, 4) 37, (64 x 192, 4) 48; 200 x
+// 2048 x 2048: (32 x 128, 2) 19.2, (32 x 128, 4) 28, (64 x 128, 4) 25; 20 x 2048 x 2048: (32 x 128, 4) 13.1, (32 x 128, 8) 13.3, (64 x 128, 4) 17.2.
+struct PartCost {
+  int bm, bn;
+  double step, fixed;
+};
+constexpr int kPartKinds = 3;
+constexpr PartCost kPartCosts[kPartKinds] = {{32, 128, 15.5, 3.0}, {64, 128, 20.5, 9.0}, {64, 192, 29.0, 13.0}};      // Parts32, Parts64, PartsWide
+struct PartTiles {
+  int kind = 0, splits = 1;
+};
+inline PartTiles choose_part_tiles(int M, int N, int K, int groups) {
+  PartTiles best;
+  double least = 0.;
+  const auto tiles_of = [&](int bm, int bn) { return static_cast<long long>((M + bm - 1) / bm) * ((N + bn - 1) / bn) * groups; };
+  for (int kind = 0; kind < kPartKinds; ++kind) {
+    const PartCost& t = kPartCosts[kind];
+    const long long tiles = tiles_of(t.bm, t.bn);
+    for (int splits = 1; splits <= 8; splits *= 2) {
+      // a ticket a tile, room for all parts, columns for every part
+      if (splits > 1 && (tiles_of(32, 128) > kMaxTickets || tiles * splits * t.bm * t.bn / 4 > kPartialUnits || tiles_of(32, 128) * splits * 32 * 128 / 4 > kPartialUnits || K / splits < 256)) break;
+      const double cut = splits == 1 ? 0. : splits == 2 ? 3.5 : splits == 4 ? 6. : 8.;
+      const double us = static_cast<double>((tiles * splits + 255) / 256) * (t.step * K / splits / 2048. + t.fixed) + cut;
+      if ((kind == 0 && splits == 1) || us < least) {
+        least = us;
+        best = PartTiles{kind, splits};
+      }
+    }
+  }
+  return best;
 }
+inline int choose_part_splits(int M, int N, int K, int groups) { return choose_part_tiles(M, N, K, groups).splits; }
 
 }  // namespace hybrid
 }  // namespace qmk
