@@ -495,7 +495,7 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
         case 6: pipe(Tall256{}); break;
         case 7: turns(Turns192{}); break;
         case 8: turns(Turns256{}); break;
-        case 9: direct(Tiles32{}); break;
+        case 9: pipe(Tiles32{}); break;
         case 10: direct(Few64{}); break;
         default: direct(Few32{}); break;
       }

@@ -464,7 +464,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
   if constexpr (S::kSplits && sizeof(T) == 4)
     if (g.splits > 1 && !sum_parts<S::kTn * kTm, S::kThreadCount>(g, tile, part, sums, reinterpret_cast<int*>(lds + LDS))) return;
   f32x4 *all = reinterpret_cast<f32x4*>(lds), *out = all + wave * kPassM * kQuads;
-  auto place = [](int r, int quad) { return r * kQuads + (quad ^ (r & (kQuads - 1) & 15)); };
+  auto place = [](int r, int quad) { return r * kQuads + (quad ^ (r & ((kQuads & -kQuads) - 1) & 15)); };      // (within a power of two that divides a row)
   const int column = n0 + wn * S::WN;
 #pragma unroll
   for (int pass = 0; pass < S::kPasses; ++pass) {
@@ -741,7 +741,7 @@ __device__ __forceinline__ void interleave() {
 // accumulators in the other half of the file and moves them at every step.)
 template <class T, class S, int PARTS = 1>
 __global__ __launch_bounds__(512, 2) void gemm_pipe(const GemmArgs g) {
-  static_assert(S::kSteps == 2 && S::kStages >= 2, "two matrix steps a stage");
+  static_assert(S::kSteps % 2 == 0 && S::kStages >= 2, "pairs of matrix steps a stage");
   constexpr int kDeep = S::kStages, kProducts = PARTS * S::kTm * S::kTn, kReads = PARTS * S::kTm + S::kTn, kRequests = Stages<S, PARTS>::kLoads;
   constexpr int kStageUnits = kDeep * Stages<S, PARTS>::kUnits, kLds = kStageUnits > S::kLds ? kStageUnits : S::kLds;
   __shared__ __align__(16) v4u lds[kLds + 1];
@@ -771,10 +771,18 @@ __global__ __launch_bounds__(512, 2) void gemm_pipe(const GemmArgs g) {
     constexpr bool MORE = decltype(more)::value;
     wait_known<63>();      // (the first fragments)
     __builtin_amdgcn_sched_barrier(0);
-    stages.fragments(buf, 4 + (lane >> 4), wm, wn, f[1].a, f[1].w);
-    multiply<S, PARTS>(f[0].a, f[0].w, acc);
-    if constexpr (MORE) interleave<kProducts, kReads, 0>();
-    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk + 1 < S::kSteps; ++kk) {
+      Fragments &now = f[kk & 1], &next = f[(kk + 1) & 1];
+      if (kk > 0) {
+        wait_known<63>();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      stages.fragments(buf, (kk + 1) * 4 + (lane >> 4), wm, wn, next.a, next.w);
+      multiply<S, PARTS>(now.a, now.w, acc);
+      if constexpr (MORE) interleave<kProducts, kReads, 0>();
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if constexpr (MORE) stages.template wait<kDeep - 2>();
     else wait_known<0>();
     barrier();
@@ -1024,10 +1032,10 @@ __global__ __launch_bounds__(kPfThreads) void gemm_short(const GemmArgs g) {
 // 128, 32 x 16 in steps of 256: 43 x 2048 x 2048 with the residual's streams 12.2, 10.1, 9.5; 43 x 2048 x 6144 with them 26.4, 19.9, 17.3; the last one now 7.9 and 14.9).
 using Few32 = Tile<32, 16, 256, 16, 16, 2, 4>;
 using Few64 = Tile<64, 16, 128, 16, 16, 4, 3>;
-using Tiles32 = Tile<64, 32, 64, 32, 16, 4, 4>;
 using Wide64 = Tile<128, 64, 64, 32, 32, 8, 3>;
-// Below with gemm_pipe (us, M x N x K, before -> with it: 512 x 2048 x 2048 Tiles64 14.5 -> 11.8; 2048 x 2048 x 2048 and x 8192 Turns128, halves of the workgroup in turns, 28.5
+// Below with gemm_pipe (us, M x N x K, before -> with it: 512 x 2048 x 2048 Tiles64 14.5 -> 11.8; 43 x 5696 x 2048 Tiles32 10.7 -> 9.0; 2048 x 2048 x 2048 and x 8192 Turns128, halves of the workgroup in turns, 28.5
 // and 88 -> 22.6 and 73, on four waves of 64 x 64 26 and 76; 1536 x 4096 x 8192 Tall192 119 -> 95, 2048 x 4096 x 8192 Tall256 139 -> 122).
+using Tiles32 = Tile<64, 32, 64, 32, 16, 4, 6>;
 using Tiles64 = Tile<64, 64, 64, 32, 32, 4, 4>;
 using Turns96 = Tile<96, 128, 64, 48, 32, 8, 4>;
 using Turns128 = Tile<128, 128, 64, 32, 64, 8, 4>;

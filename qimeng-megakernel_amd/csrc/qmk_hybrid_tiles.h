@@ -16,33 +16,31 @@ constexpr int kPartialUnits = 256 * 128 * 128 / 4;     // quads its parts leave:
 // in the attention and eight waves in the scan 43 tokens of the 2b shape took 2.72 ms instead of 2.98, 2 x 2048 of the looped 1b shape 14.4 instead of 15.1.)
 
 // The tiles of a bf16 product.  It takes as many rounds as its tiles fill the chip, `slots` at a time, each about `step` us for 2048 columns and `fixed` us
-// besides, `streams` us more where the epilogue moves the residual's streams, and `overlapped` us once.  Fitted to measurements of every kind at 20 to
-// 4096 tokens and 12 of the N x K of the four shapes (weights from memory): the kind that comes out cheapest takes 0.4 % longer than the fastest one
-// on the average up to 1024 tokens, 0.4 % up to 2048 and 0.5 % beyond, at most 9 %.  Tiles32 ends at 128 tokens: beyond, its price is off by up to 30 %
-// for many rows of weights (192 x 8256 x 2048 24.0, Tiles64 18.3), at what it would save for few (300 x 2048 x 2048 with the streams 17.9, Tiles64 21.7).
-// us, M x N x K, the kinds around the line: 43 x 2048 x 2048 with the streams Few32 9.3, Few64 10.0, Tiles32 14.1; 128 x 5696 x 2048 Tiles32 12.3, Tiles64 13.2; 1024 x 2048 x
-// 6144 with the streams Wide64 58, Tiles64 65, Turns96 70; 1531 x 2048 x 8192 with them Turns96 90, Turns128 104, Wide64 120; 2048 x 2048 x 8192 with them Turns128 104, Wide64
-// 120, Tall192 126; 3000 x 2048 x 8192 Tall192 103, Tall256 118, Turns96 137; 4096 x 2048 x 8192 Tall256 123, Turns192 154, with them 173, 216; 2048 x 12288 x 2048 Tall256 107,
-// Turns256 122; 2048 x 16384 x 2048 Turns256 129, Tall256 141, Turns192 160; 520 x 12288 x 2048 Wide256 36, Turns128 46, Wide64 49.  Memory is not priced: it bounds
-// all kinds alike where there are many rows for few tokens (1 x 128256 x 2048 Tiles32 95, Tiles64 99, Wide64 108).
+// besides, `streams` us more where the epilogue moves the residual's streams, and `overlapped` us once.  Fitted to measurements of every kind at 4 to 4096 tokens and
+// nine of the N x K of the four shapes (weights from memory), so that the kind that comes out cheapest is close to the fastest one, which is more than that
+// its price is its time: it takes 0.8 % longer than the fastest one on the average, at most 12 %.  Tiles32 ends at 128 tokens, where its price begins to be off.
+// us, M x N x K, the kinds around the line: 43 x 2048 x 2048 with the streams Few32 7.9, Few64 9.1, Tiles32 10.7; 43 x 5696 x 2048 Tiles32 9.0, Few64 10.7, Tiles64 11.2; 43 x 12288 x
+// 2048 Tiles64 14.4, Tiles32 16.2; 1024 x 2048 x 6144 with the streams Wide64 58, Tiles64 60, Turns96 67; 520 x 12288 x 2048 Wide256 35, Turns128 41; 1531 x 2048 x 8192 with them
+// Turns96 80, Turns128 85; 2048 x 2048 x 8192 Turns128 73, Tall192 84, Wide64 94; 1531 x 16384 x 2048 Tall256 104, Wide256 108; 2048 x 16384 x 2048 Turns256 144, Wide256 147.
+// Memory is not priced: it bounds all kinds alike where there are many rows for few tokens.
 struct TileCost {
   int most_tokens, bm, bn, bk, slots;
   double step, fixed, overlapped, streams;
 };
 constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 12;
 constexpr TileCost kTileCosts[kTileKinds] = {
-    {kAnyTokens, 64, 64, 64, 256, 7.9, 0.0, 3.5, 7.0},         // Tiles64
+    {kAnyTokens, 64, 64, 64, 256, 5.5, 1.0, 4.4, 6.9},         // Tiles64
     {kAnyTokens, 128, 256, 64, 256, 23.4, 9.9, 0.0, 44.0},     // Wide256
-    {kAnyTokens, 128, 64, 64, 256, 11.7, 0.9, 1.4, 8.4},       // Wide64
-    {kAnyTokens, 96, 128, 64, 256, 14.3, 5.2, 1.9, 22.0},      // Turns96
+    {kAnyTokens, 128, 64, 64, 256, 12.3, 4.4, 0.7, 3.8},       // Wide64
+    {kAnyTokens, 96, 128, 64, 256, 12.2, 2.0, 4.6, 23.1},      // Turns96
     {kAnyTokens, 128, 128, 64, 256, 16.3, 6.4, 1.0, 22.4},     // Turns128
     {kAnyTokens, 192, 128, 64, 256, 20.6, 8.4, 0.3, 32.0},     // Tall192
     {kAnyTokens, 256, 128, 64, 256, 23.6, 7.2, 1.5, 41.2},     // Tall256
     {kAnyTokens, 192, 256, 32, 256, 32.3, 14.7, 0.0, 53.5},    // Turns192
     {kAnyTokens, 256, 256, 32, 256, 39.7, 16.8, 0.0, 64.4},    // Turns256
-    {128, 64, 32, 64, 512, 7.1, 1.5, 2.8, 3.6},                // Tiles32
-    {256, 64, 16, 128, 512, 5.8, 2.3, 0.9, 2.2},               // Few64
-    {64, 32, 16, 256, 256, 4.1, 1.4, 1.6, 2.2},                // Few32
+    {128, 64, 32, 64, 256, 5.3, 1.2, 2.1, 2.7},                // Tiles32
+    {256, 64, 16, 128, 256, 3.7, 0.0, 3.2, 1.6},               // Few64
+    {64, 32, 16, 256, 256, 3.1, 0.0, 3.3, 1.8},                // Few32
 };
 inline int choose_tiles(int M, int N, int K, int groups, bool streams) {
   int best = 0;
