@@ -339,26 +339,33 @@ __global__ __launch_bounds__(kPfThreads) void keep_inputs(const float* x, QmkHyb
 // waves' sums through LDS, T (v - X), the state's update.  So in fp32 eight waves hold the tiles of a gated linear attention's heads of more than
 // 64 channels (bf16 portions keep one order, four waves, qmk_hybrid_tiles.h); and what only the output needs is off the chain: G q S is taken while the sums are on their way, and a chunk's outputs
 // are added up and stored behind the next chunk's barrier.
+// A wave's instructions are on that chain too, one wave a SIMD: chunks are read and written by buffer accesses (places of 32 bits that stay, bases that move on by
+// one scalar addition, tokens behind the last one read as zero and not written).  Without the delta rule launch bounds of eight waves, also for four, keep accumulators where
+// vector instructions reach them; with it a chunk has too many registers for that.  us, 2048 tokens, addresses of 64 bits worked out for every access -> now: 16 heads of
+// 128 | 128 of the delta rule 134 -> 120, 8 of 128 | 256 of gated linear attention 92 -> 70.  Lines of chunks further ahead asked for into L2: 141 and 88.
 template <int TILES, int WAVES, bool DELTA>
-__global__ __launch_bounds__(WAVES * 64) void chunk_scan(const ChunkArgs g) {
-  // Chunks in flight: what the registers hold (gated linear attention, 8 heads of 256 | 256, 4000 tokens in fp32, us a portion of one layer: eight waves with
-  // 4 ahead, 44 of them spilled, 603, with 3 597, with 2 628, four waves with 2 623).
-  constexpr int kAhead = TILES * WAVES == 16 && WAVES == 8 ? 3 : TILES <= 2 ? 4 : 2;
+__global__ __launch_bounds__(DELTA ? WAVES * 64 : 512, DELTA ? 1 : 2) void chunk_scan(const ChunkArgs g) {
+  // Chunks in flight: what the registers hold (us, the two shapes above, with 2, 3 and 4 ahead: 131, 120, 123; 87, 70 and, 12 registers of them spilled, 68; 8 heads of 256 | 256 in
+  // fp32, 4000 tokens, a portion of one layer with eight waves: 2 628, 3 597, 4 603).
+  constexpr int kAhead = TILES == 1 ? 4 : TILES == 2 ? 3 : 2;
   __shared__ f32x4 px[2][WAVES][64], po[2][WAVES][64];
   const QmkHybridLayer& l = g.layer;
   const int dim = l.head_dim, n = l.v_dim, head = blockIdx.x, v0 = blockIdx.y * 16;
   constexpr int tiles = TILES * WAVES;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, quad = lane >> 4;
   const int tile0 = wave * TILES, mine = min(max(dim / 16 - tile0, 0), TILES);
-  const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens;
-  const size_t step = static_cast<size_t>(l.heads) * chunk_floats(dim);
-  const float* rec = g.chunks + static_cast<size_t>(head) * chunk_floats(dim);
+  const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens, out_ld = l.heads * n;
   float* state = l.state + (static_cast<size_t>(g.slot) * l.heads + head) * dim * n + v0 + col;
-  // Values: one base per chunk for the whole wave, four fixed offsets per lane, cut off at the portion's last token.
-  const float* values = g.values + g.value_at + head * n + v0;
-  uint32_t value_at[4];
+  auto buffer = [](const float* base, int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000); };
+  // Bytes from a chunk's first value (output) to behind its last one, of rows of `ld`.
+  auto extent = [&](int chunk, int ld) { return ((min(g.M - chunk * kChunkTokens, kChunkTokens) - 1) * ld + 16) * 4; };
+  uint32_t value_at[4], out_at[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) value_at[i] = (quad * 4 + i) * g.value_ld + col;
+  for (int i = 0; i < 4; ++i) {
+    value_at[i] = ((quad * 4 + i) * g.value_ld + col) * 4;
+    out_at[i] = ((quad * 4 + i) * out_ld + col) * 4;
+  }
+  const uint32_t fragment_at = tile0 * 1024 + lane * 16, decay_at = tile0 * 64 + quad * 16, shared_at = lane * 16;
   f32x4 s[TILES];
 #pragma unroll
   for (int j = 0; j < TILES; ++j)
@@ -368,40 +375,45 @@ __global__ __launch_bounds__(WAVES * 64) void chunk_scan(const ChunkArgs g) {
   struct Fragments {
     f32x4 q[TILES], k[TILES], d[TILES], g[TILES], b, t, v;
   };
-  auto fetch = [&](Fragments& f, int chunk) {
-    chunk = min(chunk, chunks - 1);
-    const float* r = rec + chunk * step;
+  // Chunks are fetched in their order; behind the last one it is the last one again.
+  const size_t rec_step = static_cast<size_t>(l.heads) * chunk_floats(dim), value_step = static_cast<size_t>(kChunkTokens) * g.value_ld;
+  const float *rec = g.chunks + static_cast<size_t>(head) * chunk_floats(dim), *values = g.values + g.value_at + head * n + v0;
+  int fetched = 0;
+  auto fetch = [&](Fragments& f) {
+    const auto r = buffer(rec, chunk_floats(tiles * 16) * 4), v = buffer(values, extent(fetched, g.value_ld));
+    auto read = [&](uint32_t at, int first) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, first * 4, 0)); };
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
-      const int at = (tile0 + j) * 256 + lane * 4;
-      if constexpr (DELTA) f.k[j] = read4(r + tiles * 256 + at);
-      f.q[j] = read4(r + at);
-      f.d[j] = read4(r + tiles * 512 + at);
-      f.g[j] = read4(r + tiles * 768 + (tile0 + j) * 16 + quad * 4);
+      if constexpr (DELTA) f.k[j] = read(fragment_at + j * 1024, tiles * 256);
+      f.q[j] = read(fragment_at + j * 1024, 0);
+      f.d[j] = read(fragment_at + j * 1024, tiles * 512);
+      f.g[j] = read(decay_at + j * 64, tiles * 768);
     }
-    f.b = read4(r + tiles * 784 + lane * 4);
-    if constexpr (DELTA) f.t = read4(r + tiles * 784 + 256 + lane * 4);
-    const float* v = values + static_cast<size_t>(chunk) * kChunkTokens * g.value_ld;
-    const uint32_t most = min(g.M - 1 - chunk * kChunkTokens, kChunkTokens - 1) * g.value_ld + col;
+    f.b = read(shared_at, tiles * 784);
+    if constexpr (DELTA) f.t = read(shared_at, tiles * 784 + 256);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) f.v[i] = v[min(value_at[i], most)];
+    for (int i = 0; i < 4; ++i) f.v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(v, value_at[i], 0, 0));
+    const bool more = fetched + 1 < chunks;
+    rec += more ? rec_step : 0;
+    values += more ? value_step : 0;
+    fetched += more;
   };
   auto product = [](f32x4 a, f32x4 b, f32x4 c) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
     return c;
   };
+  // Ahead of a branch's end: this compiler has left out the wait between a product and the move of its result where paths meet.
+  auto settle = [](f32x4& v) { asm volatile("s_nop 15" : "+v"(v)); };
   f32x4 inner = {};       // B u of the last chunk whose outputs are this wave's
   auto outputs = [&](int chunk) {
     if (chunk < 0 || wave != (chunk & (WAVES - 1))) return;
     f32x4 o = inner;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) o += po[chunk & 1][w][lane];
+    const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, extent(chunk, out_ld));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = chunk * kChunkTokens + quad * 4 + i;
-      if (m < g.M) g.out[static_cast<size_t>(m) * l.heads * n + head * n + v0 + col] = o[i];
-    }
+    for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[i]), to, out_at[i], 0, 0);
   };
   auto advance = [&](const Fragments& f, int chunk) {
     const int buf = chunk & 1;
@@ -425,22 +437,29 @@ __global__ __launch_bounds__(WAVES * 64) void chunk_scan(const ChunkArgs g) {
 #pragma unroll
     for (int j = 0; j < TILES; ++j) s[j] = product(f.d[j], u, s[j] * f.g[j]);
     outputs(chunk - 1);
-    if (wave == (chunk & (WAVES - 1))) inner = product(f.b, u, f32x4{0.f, 0.f, 0.f, 0.f});
+    if (wave == (chunk & (WAVES - 1))) {
+      inner = product(f.b, u, f32x4{0.f, 0.f, 0.f, 0.f});
+      settle(inner);
+    }
   };
   Fragments f[kAhead];
 #pragma unroll
-  for (int a = 0; a < kAhead; ++a) fetch(f[a], a);
+  for (int a = 0; a < kAhead; ++a) fetch(f[a]);
   int chunk = 0;
   for (; chunk + kAhead <= chunks; chunk += kAhead) {
 #pragma unroll
     for (int a = 0; a < kAhead; ++a) {
       advance(f[a], chunk + a);
-      fetch(f[a], chunk + a + kAhead);
+      fetch(f[a]);
     }
   }
 #pragma unroll
   for (int a = 0; a < kAhead - 1; ++a)
-    if (chunk + a < chunks) advance(f[a], chunk + a);
+    if (chunk + a < chunks) {
+      advance(f[a], chunk + a);
+#pragma unroll
+      for (int j = 0; j < TILES; ++j) settle(s[j]);
+    }
   __syncthreads();
   outputs(chunks - 1);
 #pragma unroll
