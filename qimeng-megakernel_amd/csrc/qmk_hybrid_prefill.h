@@ -343,6 +343,8 @@ __global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const T*
 // The wkv recurrence: one head and eight value columns a workgroup; sixteen lanes share a column, KPL neighbouring key
 // rows each, in registers.  TB tokens at a time: the next block's r, k, w, v are in flight while this one runs, a block's
 // outputs leave together.  Places behind the last token or key row hold r = k = 0, w = 1, which changes nothing.
+// What bounds it is a wave's chain of tokens, one wave on half of the SIMDs: heads of up to 64 read four tokens ahead out of LDS (1531 tokens, 32 heads of 64, us, read
+// where they are used -> so: 141 -> 122; larger heads have no registers for it).
 constexpr int kWkvColumns = 8, kWkvThreads = 16 * kWkvColumns;
 template <int KPL, int TB>
 __global__ __launch_bounds__(kWkvThreads) void wkv_scan(const float* r, const float* k, const float* v, const float* w, QmkHybridLayer l, int slot, int M, float* out) {
@@ -385,6 +387,10 @@ __global__ __launch_bounds__(kWkvThreads) void wkv_scan(const float* r, const fl
     }
     if (tid < kValueQuads) *reinterpret_cast<f32x4*>(&sv[buf][tid / (kWkvColumns / 4)][tid % (kWkvColumns / 4) * 4]) = fv;
   };
+  struct Four {      // tokens, as a lane takes them
+    f32x4 r[4][KPL / 4], k[4][KPL / 4], w[4][KPL / 4];
+    float v[4];
+  };
   fetch(0);
   stash(0);
   __syncthreads();
@@ -393,23 +399,28 @@ __global__ __launch_bounds__(kWkvThreads) void wkv_scan(const float* r, const fl
     if (base + TB < M) fetch(base + TB);
     // Four tokens at a time: their sums over the sixteen lanes are taken together (two steps that halve the values while
     // they pair lanes, then plain sums), and lane p of sixteen ends up with token p % 4.
-    for (int t0 = 0; t0 < TB; t0 += 4) {
+    auto read = [&](Four& f, int t0) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f.v[q] = sv[buf][t0 + q][e];
+#pragma unroll
+        for (int i = 0; i < KPL / 4; ++i) {
+          f.r[q][i] = *reinterpret_cast<const f32x4*>(&sr[buf][t0 + q][part * KPL + i * 4]);
+          f.k[q][i] = *reinterpret_cast<const f32x4*>(&sk[buf][t0 + q][part * KPL + i * 4]);
+          f.w[q][i] = *reinterpret_cast<const f32x4*>(&sw[buf][t0 + q][part * KPL + i * 4]);
+        }
+      }
+    };
+    auto walk = [&](const Four& f, int t0) {
       float o[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int t = t0 + q;
-        const float vt = sv[buf][t][e];
         o[q] = 0.f;
 #pragma unroll
-        for (int i = 0; i < KPL; i += 4) {
-          const f32x4 r4 = *reinterpret_cast<const f32x4*>(&sr[buf][t][part * KPL + i]), k4 = *reinterpret_cast<const f32x4*>(&sk[buf][t][part * KPL + i]),
-                      w4 = *reinterpret_cast<const f32x4*>(&sw[buf][t][part * KPL + i]);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float kv = k4[j] * vt;
-            o[q] = fmaf(r4[j], fmaf(u[i + j], kv, s[i + j]), o[q]);
-            s[i + j] = fmaf(w4[j], s[i + j], kv);
-          }
+        for (int i = 0; i < KPL; ++i) {
+          const float kv = f.k[q][i / 4][i % 4] * f.v[q];
+          o[q] = fmaf(f.r[q][i / 4][i % 4], fmaf(u[i], kv, s[i]), o[q]);
+          s[i] = fmaf(f.w[q][i / 4][i % 4], s[i], kv);
         }
       }
       const bool b0 = part & 1, b1 = part & 2;
@@ -419,6 +430,25 @@ __global__ __launch_bounds__(kWkvThreads) void wkv_scan(const float* r, const fl
       sum += dpp_f32<0x124>(0.f, sum);        // row_ror:4
       sum += dpp_f32<0x128>(0.f, sum);        // row_ror:8
       if (part < 4) so[buf][t0 + part][e] = sum;
+    };
+    if constexpr (KPL == 4) {
+      Four f[2];
+      read(f[0], 0);
+#pragma unroll
+      for (int t0 = 0; t0 < TB; t0 += 8) {
+        read(f[1], t0 + 4);
+        __builtin_amdgcn_sched_barrier(0);
+        walk(f[0], t0);
+        if (t0 + 8 < TB) read(f[0], t0 + 8);
+        __builtin_amdgcn_sched_barrier(0);
+        walk(f[1], t0 + 4);
+      }
+    } else {
+      for (int t0 = 0; t0 < TB; t0 += 4) {
+        Four f;
+        read(f, t0);
+        walk(f, t0);
+      }
     }
     if (base + TB < M) stash(buf ^ 1);
     __syncthreads();
