@@ -403,7 +403,9 @@ __global__ __launch_bounds__(DELTA ? WAVES * 64 : 512, DELTA ? 1 : 2) void chunk
     for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
     return c;
   };
-  // Ahead of a branch's end: this compiler has left out the wait between a product and the move of its result where paths meet.
+  // Ahead of a branch's end: this compiler (clang 22 of ROCm 7.2.0) has left out the wait between a product and the move of its result where paths meet; without
+  // this <1, 4> moves one two instructions behind its product.  The rule, for any kernel: an accumulator that lives across the end of a branch with a product in it is
+  // settled there if its built code has such a move (tests/test_matrix_waits.py walks every path of every kernel for it); none but these two places has.
   auto settle = [](f32x4& v) { asm volatile("s_nop 15" : "+v"(v)); };
   f32x4 inner = {};       // B u of the last chunk whose outputs are this wave's
   auto outputs = [&](int chunk) {
