@@ -27,7 +27,7 @@ __device__ __forceinline__ float max_of_quarters(float v) {
 // Windowed causal attention over expanded keys: 64 queries of one head a workgroup (16 a wave), KEYS keys a stage, QT 32-column steps of a query,
 // at most VT 16-row tiles of a value.  Scores are computed transposed (keys x queries), so a lane holds eight weights of ONE query in exactly the shape
 // the value product's second operand wants.  A query takes its keys 32 at a time in their order, as bf16 portions have to (qmk_hybrid_tiles.h);
-// parts of a stage that no query of a wave sees are left out, which changes nothing.
+// 32 keys that no query of a wave sees are left out, which changes nothing but that a value among them that is not finite stays out of the sums (0 x inf).
 //
 // What bounds it is the chain of 32 keys in a wave (fragments, scores, maximum over the lanes, weights, values; about 700 instructions' time), with two waves a
 // SIMD at 2048 queries of 16 heads.  So both halves of 64 keys take their scores together, all fragments are asked for at once (asked for
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(con
       }
 #pragma unroll
     for (int sub = 0; sub < kSubs; ++sub, base += 32) {
-      if (MASKED && base >= hi) break;
+      if (MASKED && (base >= hi || base > last_pos || first_pos - (base + 31) >= window)) continue;      // 32 keys that no query of this wave sees
       float w[8], best = top, step_sum = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) w[j] = d[sub][j >> 2][j & 3] * scale;

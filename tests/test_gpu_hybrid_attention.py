@@ -59,3 +59,22 @@ def test_attention_at_the_edges_of_its_tiles(name, past, n):
     d = d - d.mean(-1, keepdim=True)
     err = float((d.pow(2).mean(-1).sqrt() / want.pow(2).mean().sqrt()).max())
     assert err < (8e-2 if shape.plain else 4e-2), f"{err:.3g}"
+
+
+@pytest.mark.parametrize("name", sorted(n for n, shape in SHAPES.items() if not shape.plain))
+@pytest.mark.parametrize("at", [3, 40, 100])
+def test_an_undefined_value_stays_out_of_what_no_query_of_a_wave_sees(name, at):
+    """Sixteen queries take 32 keys together, with weights of zero where one does not see a key; keys that none of the sixteen sees do not enter at all."""
+    shape, w, tokens, _ = model(name)
+    n, window, undefined = 200, shape.entries[0].shape.window, shape.vocab - 1
+    tokens = tokens[:n].clamp(max=undefined - 1).index_fill(0, torch.tensor([at]), undefined)
+    w = {**w, "embed": w["embed"].index_fill(0, torch.tensor([undefined], device=DEVICE), float("nan"))}
+    g = build_globals(shape, weights.pack(shape, w, DEVICE), dtype=torch.bfloat16, max_positions=n, portion_rows=n)
+    got = decode_hybrid.run_tokens(g, mk_kernel.get_mk(), RequestTable(g).open(0), tokens, range(n))
+    defined, block = torch.isfinite(got).all(-1).tolist(), at & ~31
+    for i in range(n):
+        wave = i & ~15
+        if block > wave + 15 or wave - (block + 31) >= window:      # none of its sixteen queries sees any of the 32 keys
+            assert defined[i], i
+        if 0 <= i - at < window:
+            assert not defined[i], i
