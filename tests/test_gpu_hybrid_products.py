@@ -31,11 +31,14 @@ SHAPES = {
     "plain": synthetic.looped_shape("pgp", width=2048, vocab=336, ff={"p": 4040, "g": 2856}, loop=(1, 2, 2), heads=4, kv_heads=2, delta_heads=4, delta_kv_heads=2,
                                     delta_rank=144, gate_rank=72, gla_heads=11, gla_rank=80),
 }
+#: rows so long that few of them are cut in four along K, with tiles of 64 tokens of either width (fp32: its tokens' side in parts)
+LONG = synthetic.hybrid_shape("a", width=2048, vocab=336, streams=2, ff={"a": 8192}, heads=2, dim=128, rot_dim=64, v_dim=128, rank=128, window=512)
+LONG_LENGTHS = (200, 260)
 
 
 @functools.lru_cache(maxsize=None)
 def expected(name):
-    shape = SHAPES[name]
+    shape = {**SHAPES, "long": LONG}[name]
     w = synthetic.random_hybrid_weights(shape, 3, DEVICE)
     tokens = torch.randint(0, shape.vocab, (MOST,), generator=torch.Generator().manual_seed(5))
     with torch.device(DEVICE):
@@ -47,7 +50,15 @@ def expected(name):
 @pytest.mark.parametrize("n", LENGTHS)
 @pytest.mark.parametrize("name", sorted(SHAPES))
 def test_products_at_the_edges_of_tiles(name, n, dtype):
-    shape = SHAPES[name]
+    check(name, SHAPES[name], n, dtype)
+
+
+@pytest.mark.parametrize("n", LONG_LENGTHS)
+def test_long_rows_cut_in_four(n):
+    check("long", LONG, n, torch.float32)
+
+
+def check(name, shape, n, dtype):
     w, tokens, want = expected(name)
     g = build_globals(shape, weights.pack(shape, w, DEVICE), dtype=dtype, max_positions=MOST, portion_rows=MOST)
     got = decode_hybrid.run_tokens(g, mk_kernel.get_mk(), RequestTable(g).open(0), tokens[:n], range(n)).double()

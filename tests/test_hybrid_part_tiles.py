@@ -1,12 +1,13 @@
 """The rule that chooses tiles and cuts for products whose tokens' side is in three parts (csrc/qmk_hybrid_tiles.h, compiled for the host): the GPU tests of the products
-reach every kind, cut and not, and a cut has room for its tickets and sums at any size."""
+reach every kind with every cut that a shape of the registry takes it with, and a cut has room for its tickets and sums at any size."""
 import random
 import subprocess
 
 import pytest
 
 from conftest import ROOT
-from test_gpu_hybrid_products import LENGTHS, SHAPES
+from qimeng_megakernel_amd import registry
+from test_gpu_hybrid_products import LENGTHS, LONG, LONG_LENGTHS, SHAPES
 from test_hybrid_tiles import products
 
 DRIVER = """
@@ -36,10 +37,17 @@ def choose(tmp_path_factory):
     return run
 
 
-def test_the_gpu_tests_reach_every_kind(choose):
-    sizes = {(M, N, K, groups) for shape in SHAPES.values() for n in LENGTHS for M, N, K, groups, _, may in products(shape, n) if may and K > 64 and K % 64 == 0}
-    found = {(kind, splits > 1) for kind, splits, *_ in choose(sorted(sizes))}
-    assert {kind for kind, _ in found} == {0, 1, 2} and {(0, True), (1, True)} <= found
+def pairs(choose, portions):
+    """{(kind, cuts)} of the products of (shape, tokens) whose tokens' side is in parts."""
+    sizes = {(M, N, K, groups) for shape, n in portions for M, N, K, groups, _, may in products(shape, n) if may and K > 64 and K % 64 == 0}
+    return {(kind, cuts) for kind, cuts, *_ in choose(sorted(sizes))}
+
+
+def test_the_gpu_tests_reach_every_kind_and_cut(choose):
+    tested = pairs(choose, [(shape, n) for shape in SHAPES.values() for n in LENGTHS] + [(LONG, n) for n in LONG_LENGTHS])
+    shapes = [registry.shape_of(name) for name, (family, *_) in registry.MODELS.items() if family is registry.HYBRID]
+    used = pairs(choose, [(shape, n) for shape in shapes for n in (*range(2, 700), *range(700, 4097, 31))])
+    assert len(shapes) >= 4 and used == {(0, 1), (0, 2), (0, 4), (0, 8), (1, 1), (1, 2), (1, 4), (2, 1), (2, 2), (2, 4)} and used <= tested
 
 
 def test_what_is_cut_has_room(choose):
