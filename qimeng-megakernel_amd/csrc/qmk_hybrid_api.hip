@@ -504,9 +504,10 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   }
   if constexpr (sizeof(TA) == 4 && sizeof(TW) == 2) {
     if (g.a_part != 0) {
-      g.splits = choose_part_splits(g.M, n, g.K, g.groups);
+      const PartTiles tiles = choose_part_tiles(g.M, n, g.K, g.groups);
+      g.splits = tiles.splits;
       auto parts = [&](auto s) { using S = decltype(s); launch(gemm_pipe<T, S, 3>, S::BM, S::BN, S::kThreadCount); };
-      switch (choose_part_tiles(g.M, n, g.K, g.groups).kind) {
+      switch (tiles.kind) {
         case 0: parts(Parts32{}); break;
         case 1: parts(Parts64{}); break;
         default: parts(PartsWide{}); break;

@@ -91,13 +91,12 @@ struct PartTiles {
 inline PartTiles choose_part_tiles(int M, int N, int K, int groups) {
   PartTiles best;
   double least = 0.;
-  const auto tiles_of = [&](int bm, int bn) { return static_cast<long long>((M + bm - 1) / bm) * ((N + bn - 1) / bn) * groups; };
   for (int kind = 0; kind < kPartKinds; ++kind) {
     const PartCost& t = kPartCosts[kind];
-    const long long tiles = tiles_of(t.bm, t.bn);
+    const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * groups;
     for (int splits = 1; splits <= 8; splits *= 2) {
       // a ticket a tile, room for all parts, columns for every part
-      if (splits > 1 && (tiles_of(32, 128) > kMaxTickets || tiles * splits * t.bm * t.bn / 4 > kPartialUnits || tiles_of(32, 128) * splits * 32 * 128 / 4 > kPartialUnits || K / splits < 256)) break;
+      if (splits > 1 && (tiles > kMaxTickets || tiles * splits * t.bm * t.bn / 4 > kPartialUnits || K / splits < 256)) break;
       const double cut = splits == 1 ? 0. : splits == 2 ? 3.5 : splits == 4 ? 6. : 8.;
       const double us = static_cast<double>((tiles * splits + 255) / 256) * (t.step * K / splits / 2048. + t.fixed) + cut;
       if ((kind == 0 && splits == 1) || us < least) {
@@ -108,7 +107,6 @@ inline PartTiles choose_part_tiles(int M, int N, int K, int groups) {
   }
   return best;
 }
-inline int choose_part_splits(int M, int N, int K, int groups) { return choose_part_tiles(M, N, K, groups).splits; }
 
 }  // namespace hybrid
 }  // namespace qmk

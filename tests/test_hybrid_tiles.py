@@ -18,7 +18,7 @@ int main() {
   while (scanf("%d %d %d %d %d %d", &M, &N, &K, &groups, &streams, &cut) == 6) {
     const RegisterTiles r = choose_register_tiles(M, N, K, groups, cut);
     const int kind = K % 64 ? -1 : choose_tiles(M, N, K, groups, streams);
-    printf("%d %d %d %d %d %d %d\\n", kind, kind < 0 ? 1 : kTileCosts[kind].bm, kind < 0 ? 1 : kTileCosts[kind].bn, kind < 0 ? 1 : kTileCosts[kind].bk, choose_part_splits(M, N, K, groups),
+    printf("%d %d %d %d %d %d %d\\n", kind, kind < 0 ? 1 : kTileCosts[kind].bm, kind < 0 ? 1 : kTileCosts[kind].bn, kind < 0 ? 1 : kTileCosts[kind].bk, choose_part_tiles(M, N, K, groups).splits,
            r.large, r.splits);
   }
 }
