@@ -552,10 +552,10 @@ void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* 
     auto launch = [&](auto kernel, int groups) {
       hipLaunchKernelGGL(kernel, dim3(runs, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
     };
-    if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<T, 4, 4, 2>, 2);
-    else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<T, 4, 8, 2>, 2);
-    else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<T, 6, 8, 2>, 2);
-    else launch(window_attention<T, 8, 16, 1>, 1);
+    if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<4, 4, 2>, 2);
+    else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<4, 8, 2>, 2);
+    else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<6, 8, 2>, 2);
+    else launch(window_attention<8, 16, 1>, 1);
   }
 }
 

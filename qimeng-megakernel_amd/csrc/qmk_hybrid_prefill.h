@@ -170,17 +170,15 @@ __global__ __launch_bounds__(kPfThreads) void latent_rows(const float* raw, QmkH
 }
 
 // The same as attention_rows for fp32 portions, values in the order of their keys, 32 keys a step through registers.
-// GROUPS = 2: two groups of four waves take the 32-key steps in
-// turn, for the same queries, and meet at the end: a step is a chain (keys into LDS, scores, maximum over the lanes, weights, values), and a CU
-// that holds one or two workgroups of four waves mostly waits for it (us, one group -> two: 200 queries of 16 heads of 192 | 128 34 -> 29).
-template <class T, int QT, int VT, int GROUPS>   // most 32-column steps of a query, most 16-row tiles of a value
-__global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const T* q, Keys<T> keys, const T* rows, const T* v_t, const T* gate, QmkHybridLayer l,
-                                                               int first, int position, int M, int keys_cap, Operand<T> out) {
-  constexpr int kKeys = 32;
-  constexpr int kPadK = 16 / sizeof(T), kPadV = 16 / sizeof(T);
+// GROUPS = 2: two groups of four waves take the 32-key steps in turn, for the same queries, and meet at the end: a step is a chain (keys into LDS, scores, maximum
+// over the lanes, weights, values), and a CU that holds one or two workgroups of four waves mostly waits for it (us, one group -> two: 200 queries of 16 heads of 192 | 128 34 -> 29).
+template <int QT, int VT, int GROUPS>   // most 32-column steps of a query, most 16-row tiles of a value
+__global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const float* q, Keys<float> keys, const float* rows, const float* v_t, const float* gate, QmkHybridLayer l,
+                                                               int first, int position, int M, int keys_cap, Operand<float> out) {
+  constexpr int kKeys = 32, kU = 4;      // keys a step; a unit of 16 bytes, which also sets rows apart
   struct Step {
-    T k[kKeys][QT * 32 + kPadK];
-    T v[VT * 16][kKeys + kPadV];
+    float k[kKeys][QT * 32 + kU];
+    float v[VT * 16][kKeys + kU];
   };
   __shared__ __align__(16) Step stage[GROUPS];
   const int tid = threadIdx.x % kPfThreads, lane = tid & 63, wave = tid >> 6, g = lane >> 4, col = lane & 15;
@@ -193,7 +191,7 @@ __global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const T*
   const int head = blockIdx.y, kv = head / keys.heads_per, q0 = (mirrored ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * 64;
   const int dq = l.q_stride, steps = dq / 32, vt = l.v_dim / 16, width = l.rank + l.rot_dim;
   const int m = q0 + wave * 16 + col, pos = position + m;
-  Frag<T> fq[QT];
+  Frag<float> fq[QT];
 #pragma unroll
   for (int s = 0; s < QT; ++s)
     if (s < steps) fq[s] = load_frag(q + static_cast<size_t>(min(m, M - 1)) * l.heads * dq + head * dq + s * 32 + g * 8);
@@ -202,13 +200,12 @@ __global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const T*
   const float scale = l.scale * kLog2e;
   const int lo = max(first, position + q0 + 1 - l.window);      // the first key any of the 64 queries sees
   const int hi = min(position + q0 + 64, position + M);          // behind the last one
-  constexpr int kU = 16 / sizeof(T);
   // Staging: each thread has fixed places in a tile of keys and of transposed values; the next tile is in flight while
   // this one is used.
   constexpr int kKLoads = kKeys * QT * 32 / kU / kPfThreads, kVLoads = VT * 16 * kKeys / kU / kPfThreads;
   static_assert(kKLoads * kPfThreads * kU == kKeys * QT * 32 && kVLoads * kPfThreads * kU == VT * 16 * kKeys, "every thread stages the same number of units");
   const int begin = first + ((lo - first) & ~(kKeys - 1)), base0 = begin + part * kKeys;
-  const T* k_at[kKLoads];
+  const float* k_at[kKLoads];
   int k_step[kKLoads];
   v4u rk[kKLoads], rv[kVLoads];
 #pragma unroll
@@ -238,10 +235,10 @@ __global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const T*
       rv[i] = v4u{0u, 0u, 0u, 0u};
       if (r < l.v_dim && base + c < hi) rv[i] = *reinterpret_cast<const v4u*>(v_t + static_cast<size_t>(kv * l.v_dim + r) * keys_cap + base - first + c);
       if (base + c + kU > hi) {   // keys behind the last one: whatever the buffer holds there must not enter a sum
-        T* e = reinterpret_cast<T*>(&rv[i]);
+        float* e = reinterpret_cast<float*>(&rv[i]);
 #pragma unroll
         for (int j = 0; j < kU; ++j)
-          if (base + c + j >= hi) e[j] = from_f32<T>(0.f);
+          if (base + c + j >= hi) e[j] = 0.f;
       }
     }
   };
@@ -286,20 +283,20 @@ __global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const T*
       const float ref = best == -INFINITY ? 0.f : best;      // no key of this query yet
       const float shrink = exp2_fast(top - ref);
       float step_sum = 0.f;
-      Frag<T> fp;
+      Frag<float> fp;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         w[j] = exp2_fast(w[j] - ref);
         step_sum += w[j];
-        fp.set(j, from_f32<T>(w[j]));
+        fp.set(j, w[j]);
       }
       sum = sum * shrink + step_sum;
       top = best;
 #pragma unroll
       for (int t = 0; t < VT; ++t)
         if (t < vt) {
-          Frag<T> fv;
-          const T* r = &sv[t * 16 + col][0];
+          Frag<float> fv;
+          const float* r = &sv[t * 16 + col][0];
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             fv.set(j, r[g * 4 + j]);
