@@ -1,6 +1,8 @@
 // Which tiles a product of the hybrid route's prefill takes: rules of the host, over sizes alone.
 #pragma once
 
+#include <algorithm>
+
 namespace qmk {
 namespace hybrid {
 
@@ -15,32 +17,35 @@ constexpr int kPartialUnits = 256 * 128 * 128 / 4;     // quads its parts leave:
 // 0.053, and in one cache a value that differs by twice its root mean square.  The median is 0.008 to 0.024 at every length.  (With cuts along K, two groups
 // in the attention and eight waves in the scan 43 tokens of the 2b shape took 2.72 ms instead of 2.98, 2 x 2048 of the looped 1b shape 14.4 instead of 15.1.)
 
-// The tiles of a bf16 product.  It takes as many rounds as its tiles fill the chip, `slots` at a time, each about `step` us for 2048 columns and `fixed` us
-// besides, `streams` us more where the epilogue moves the residual's streams, and `overlapped` us once.  Fitted to measurements of every kind at 4 to 4096 tokens and
-// nine of the N x K of the four shapes (weights from memory), so that the kind that comes out cheapest is close to the fastest one, which is more than that
-// its price is its time: it takes 0.8 % longer than the fastest one on the average, at most 12 %.  Tiles32 ends at 128 tokens, where its price begins to be off.
-// us, M x N x K, the kinds around the line: 43 x 2048 x 2048 with the streams Few32 7.9, Few64 9.1, Tiles32 10.7; 43 x 5696 x 2048 Tiles32 9.0, Few64 10.7, Tiles64 11.2; 43 x 12288 x
-// 2048 Tiles64 14.4, Tiles32 16.2; 1024 x 2048 x 6144 with the streams Wide64 58, Tiles64 60, Turns96 67; 520 x 12288 x 2048 Wide256 35, Turns128 41; 1531 x 2048 x 8192 with them
-// Turns96 80, Turns128 85; 2048 x 2048 x 8192 Turns128 73, Tall192 84, Wide64 94; 1531 x 16384 x 2048 Tall256 104, Wide256 108; 2048 x 16384 x 2048 Turns256 144, Wide256 147.
+// The tiles of a bf16 product.  It takes as many rounds as its tiles fill the chip, 256 at a time, each about `step` us for 2048 columns and `fixed` us besides, `streams` us
+// more where the epilogue moves the residual's streams, and `overlapped` us once.  Where two workgroups share a CU (`a_cu`) a round that is not full takes its part of one.
+// Fitted to every kind's launches in whole portions of 1 to 4096 tokens of the four shapes (90 lengths, 2011 products; weights and streams from memory), each portion with all its
+// products on one kind, so that the kind that comes out cheapest is close to the fastest one, which is more than that its price is its time: it takes 0.8 % longer than the fastest
+// one on the average, at most 24 % (with prices fitted to single launches 2.1 and 48 %; of lengths that a first fit had not seen 0.7, and 2.0).  Whole portions, those prices / these: 0.99 (200 tokens of
+// the looped shapes) to 1.04 (1750 and 2048 of the others), 1.008 on the average of 43 lengths.  Tiles32 ends at 128 tokens, where its price begins to be off.
+// us, M x N x K, the kinds around the line: 43 x 2048 x 6144 with the streams Few32 15.0, Few64 20.9; 43 x 5696 x 2048 Tiles32 10.6, Few64 11.8, Tiles64 13.5; 43 x 12288 x 2048 Tiles64 15.2,
+// Tiles32 16.7; 520 x 2048 x 6144 with them Tiles64 41.9, Wide64 47.0; 1024 x 2048 x 6144 with them Wide64 54.6, Turns96 56.5, Tiles64 64.8; 520 x 12288 x 2048 Wide256 31.8, Turns128 36.2;
+// 1531 x 2048 x 2048 with them Turns96 33.6, Turns128 36.8, Wide64 42.6; 2048 x 2048 x 2048 with them Turns128 42.8, Tall192 49.1, Wide64 53.2; 1531 x 2048 x 8192 with them Turns96 72.6,
+// Turns128 84.6; 3000 x 2048 x 8192 Tall192 97.8, Tall256 111.5; 1531 x 16384 x 2048 Tall256 94.9, Wide256 100.1; 2048 x 16384 x 2048 Turns256 123.2, Tall256 125.4.
 // Memory is not priced: it bounds all kinds alike where there are many rows for few tokens.
 struct TileCost {
-  int most_tokens, bm, bn, bk, slots;
+  int most_tokens, bm, bn, bk, a_cu;
   double step, fixed, overlapped, streams;
 };
 constexpr int kAnyTokens = 0x7fffffff, kTileKinds = 12;
 constexpr TileCost kTileCosts[kTileKinds] = {
-    {kAnyTokens, 64, 64, 64, 256, 5.5, 1.0, 4.4, 6.9},         // Tiles64
-    {kAnyTokens, 128, 256, 64, 256, 23.4, 9.9, 0.0, 44.0},     // Wide256
-    {kAnyTokens, 128, 64, 64, 256, 12.3, 4.4, 0.7, 3.8},       // Wide64
-    {kAnyTokens, 96, 128, 64, 256, 12.2, 2.0, 4.6, 23.1},      // Turns96
-    {kAnyTokens, 128, 128, 64, 256, 16.3, 6.4, 1.0, 22.4},     // Turns128
-    {kAnyTokens, 192, 128, 64, 256, 20.6, 8.4, 0.3, 32.0},     // Tall192
-    {kAnyTokens, 256, 128, 64, 256, 23.6, 7.2, 1.5, 41.2},     // Tall256
-    {kAnyTokens, 192, 256, 32, 256, 32.3, 14.7, 0.0, 53.5},    // Turns192
-    {kAnyTokens, 256, 256, 32, 256, 39.7, 16.8, 0.0, 64.4},    // Turns256
-    {128, 64, 32, 64, 256, 5.3, 1.2, 2.1, 2.7},                // Tiles32
-    {256, 64, 16, 128, 256, 3.7, 0.0, 3.2, 1.6},               // Few64
-    {64, 32, 16, 256, 256, 3.1, 0.0, 3.3, 1.8},                // Few32
+    {kAnyTokens, 64, 64, 64, 2, 6.7, 2.0, 3.0, 17.2},          // Tiles64
+    {kAnyTokens, 128, 256, 64, 1, 21.3, 14.3, 0.0, 42.9},      // Wide256
+    {kAnyTokens, 128, 64, 64, 2, 12.4, 1.8, 4.7, 10.0},        // Wide64
+    {kAnyTokens, 96, 128, 64, 1, 12.7, 6.8, 0.0, 9.5},         // Turns96
+    {kAnyTokens, 128, 128, 64, 1, 13.1, 7.8, 1.6, 13.8},       // Turns128
+    {kAnyTokens, 192, 128, 64, 1, 17.3, 9.9, 0.8, 20.2},       // Tall192
+    {kAnyTokens, 256, 128, 64, 1, 20.4, 11.4, 1.8, 26.7},      // Tall256
+    {kAnyTokens, 192, 256, 32, 1, 38.7, 12.0, 3.5, 57.7},      // Turns192
+    {kAnyTokens, 256, 256, 32, 1, 44.5, 16.0, 0.7, 70.4},      // Turns256
+    {128, 64, 32, 64, 2, 4.5, 4.5, 0.5, 2.3},                  // Tiles32
+    {256, 64, 16, 128, 2, 4.9, 0.8, 2.6, 2.1},                 // Few64
+    {64, 32, 16, 256, 1, 3.2, 2.2, 1.6, 1.4},                  // Few32
 };
 inline int choose_tiles(int M, int N, int K, int groups, bool streams) {
   int best = 0;
@@ -49,7 +54,8 @@ inline int choose_tiles(int M, int N, int K, int groups, bool streams) {
     const TileCost& t = kTileCosts[kind];
     if (M > t.most_tokens || K % t.bk != 0) continue;
     const long long tiles = static_cast<long long>((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * groups;
-    const double us = static_cast<double>((tiles + t.slots - 1) / t.slots) * (t.step * K / 2048. + t.fixed + (streams ? t.streams : 0.)) + t.overlapped;
+    const double rounds = t.a_cu > 1 ? std::max(1., tiles / 256.) : static_cast<double>((tiles + 255) / 256);
+    const double us = rounds * (t.step * K / 2048. + t.fixed + (streams ? t.streams : 0.)) + t.overlapped;
     if (kind == 0 || us < least) {
       least = us;
       best = kind;

@@ -102,23 +102,38 @@ def test_rules_hold_for_any_size(choose):
         assert not large or small_cuts == 1
 
 
-#: us by kind where kinds are far apart or an epilogue decides between them (weights from memory, one MI355X)
+#: us by kind of (tokens, rows of weights, columns, whether the epilogue moves the residual's streams): a launch in a whole portion of a shape that has the product, all of
+#: whose products take the kind (so weights and streams come from memory); mean over its launches on one MI355X, the three fastest kinds
 MEASURED = [
-    ((1531, 2048, 2048, 1), {"Wide64": 38.0, "Turns96": 41.9, "Turns128": 49.9}),
-    ((1531, 2048, 8192, 1), {"Turns96": 89.6, "Turns128": 103.6, "Wide64": 119.8}),
-    ((3000, 2048, 2048, 1), {"Tall192": 68.9, "Turns96": 77.4, "Wide64": 79.3}),
-    ((3000, 2048, 8192, 0), {"Tall192": 102.8, "Tall256": 118.3, "Turns96": 137.2}),
-    ((4096, 2048, 8192, 0), {"Tall256": 123.4, "Turns192": 154.3, "Turns128": 166.5}),
-    ((4096, 2048, 8192, 1), {"Tall256": 173.4, "Turns128": 213.8, "Turns192": 216.4}),
-    ((4096, 16384, 2048, 0), {"Turns256": 262.5, "Tall256": 285.1, "Turns192": 303.7}),
-    ((2048, 2048, 8192, 1), {"Turns128": 103.7, "Wide64": 120.1, "Tall192": 126.2}),
-    ((2048, 12288, 2048, 0), {"Tall256": 107.0, "Turns256": 121.7}),
-    ((520, 12288, 2048, 0), {"Wide256": 35.5, "Turns128": 46.0, "Wide64": 49.0}),
-    ((1024, 2048, 6144, 1), {"Wide64": 57.9, "Tiles64": 64.5, "Turns96": 70.1}),
-    ((43, 2048, 6144, 1), {"Few32": 17.3, "Few64": 19.9, "Tiles32": 27.2}),
+    ((43, 2048, 6144, 1), {"Few32": 15.0, "Few64": 20.9, "Tiles32": 22.8}),
+    ((43, 2048, 2048, 1), {"Few32": 8.7, "Few64": 10.4, "Tiles32": 12.8}),
+    ((43, 5696, 2048, 0), {"Tiles32": 10.6, "Few64": 11.8, "Tiles64": 13.5}),
+    ((43, 12288, 2048, 0), {"Tiles64": 15.2, "Tiles32": 16.7, "Wide64": 18.4}),
+    ((128, 2048, 8192, 1), {"Few64": 26.9, "Tiles32": 30.7, "Tiles64": 41.5}),
+    ((200, 2048, 6144, 1), {"Few64": 28.2, "Tiles64": 32.1, "Wide64": 46.7}),
+    ((260, 6144, 2048, 0), {"Tiles64": 19.9, "Turns128": 22.1, "Turns96": 24.2}),
+    ((400, 5696, 2048, 0), {"Turns128": 20.4, "Turns96": 20.8, "Wide64": 25.5}),
+    ((520, 2048, 6144, 1), {"Tiles64": 41.9, "Wide64": 47.0, "Turns128": 52.4}),
+    ((520, 12288, 2048, 0), {"Wide256": 31.8, "Turns128": 36.2, "Wide64": 44.2}),
+    ((1024, 2048, 6144, 1), {"Wide64": 54.6, "Turns96": 56.5, "Tiles64": 64.8}),
+    ((1531, 2048, 2048, 1), {"Turns96": 33.6, "Turns128": 36.8, "Wide64": 42.6}),
+    ((1531, 2048, 8192, 1), {"Turns96": 72.6, "Turns128": 84.6, "Tall192": 100.7}),
+    ((1531, 16384, 2048, 0), {"Tall256": 94.9, "Wide256": 100.1, "Turns192": 101.6}),
+    ((1531, 5696, 2048, 0), {"Tall192": 56.4, "Turns192": 56.5, "Tall256": 58.5}),
+    ((2048, 2048, 2048, 1), {"Turns128": 42.8, "Tall192": 49.1, "Turns96": 52.4}),
+    ((2048, 2048, 2048, 0), {"Turns128": 25.3, "Tall192": 28.0, "Wide64": 32.3}),
+    ((2048, 2048, 8192, 1), {"Turns128": 93.6, "Tall192": 103.5, "Tall256": 121.5}),
+    ((2048, 12288, 2048, 0), {"Tall256": 94.5, "Wide256": 99.8, "Turns256": 117.7}),
+    ((2048, 16384, 2048, 0), {"Turns256": 123.2, "Tall256": 125.4, "Wide256": 134.2}),
+    ((3000, 2048, 2048, 1), {"Tall192": 61.4, "Tall256": 67.3, "Turns96": 67.8}),
+    ((3000, 2048, 8192, 0), {"Tall192": 97.8, "Tall256": 111.5, "Wide256": 115.4}),
+    ((4096, 2048, 8192, 0), {"Wide256": 131.6, "Tall256": 132.1, "Turns192": 161.0}),
+    ((4096, 2048, 8192, 1), {"Wide256": 166.2, "Tall256": 172.4, "Turns128": 207.1}),
+    ((4096, 16384, 2048, 0), {"Turns256": 248.9, "Tall256": 253.5, "Wide256": 273.3}),
 ]
 
 
-def test_choices_where_kinds_are_far_apart(choose):
+def test_choices_where_kinds_were_measured(choose):
     got = choose([(M, N, K, 1, streams, 0) for (M, N, K, streams), _ in MEASURED])
-    assert [KINDS[kind] for kind, *_ in got] == [min(us, key=us.get) for _, us in MEASURED]
+    slower = {size: us.get(KINDS[kind], float("inf")) / min(us.values()) for (size, us), (kind, *_) in zip(MEASURED, got)}
+    assert max(slower.values()) < 1.04, slower
