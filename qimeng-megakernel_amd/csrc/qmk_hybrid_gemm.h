@@ -1038,6 +1038,7 @@ __global__ __launch_bounds__(kPfThreads) void gemm_short(const GemmArgs g) {
 }
 
 // ---- which tiles ----
+// (Figures here are of single launches one after another, weights from memory; inside a portion they differ by up to a fifth, qmk_hybrid_tiles.h.)
 // Few tokens: weight rows of a workgroup, deep steps, since a step's barrier and reads are most of its time (us, M x N x K, 64 x 16 in steps of 64 columns, of
 // 128, 32 x 16 in steps of 256: 43 x 2048 x 2048 with the residual's streams 12.2, 10.1, 9.5; 43 x 2048 x 6144 with them 26.4, 19.9, 17.3; the last one now 7.9 and 14.9).
 using Few32 = Tile<32, 16, 256, 16, 16, 2, 4>;

@@ -82,7 +82,7 @@ inline RegisterTiles choose_register_tiles(int M, int N, int K, int groups, bool
 
 // Products whose tokens' side is in three parts: the kind of tile and the number of parts along K, priced like the bf16 ones, an epilogue of the usual mixture
 // within `fixed`, and what a cut costs.  What decides is how full the chip is: a workgroup has it 256 at a time, and larger tiles read LDS less often
-// for a product.  us by (tokens x rows, cuts), x 12288 x 2048, 20 tokens: (32 x 128, 2) 15.8, (32 x 128, 4) 21.5, (64 x 128, 2) 19.8; 100: (64 x 128, 1) 27.2, (32 x 128, 1) 37,
+// for a product.  us by (tokens x rows, cuts), single launches, x 12288 x 2048, 20 tokens: (32 x 128, 2) 15.8, (32 x 128, 4) 21.5, (64 x 128, 2) 19.8; 100: (64 x 128, 1) 27.2, (32 x 128, 1) 37,
 // (64 x 192, 1) 34; 200: (64 x 192, 1) 39.6, (64 x 128, 1) 53, (32 x 128, 1) 54; 200 x 2048 x 6144 with the streams: (32 x 128, 2) 34, (64 x 128, 4) 37, (64 x 192, 4) 48; 200 x
 // 2048 x 2048: (32 x 128, 2) 19.2, (32 x 128, 4) 28, (64 x 128, 4) 25; 20 x 2048 x 2048: (32 x 128, 4) 13.1, (32 x 128, 8) 13.3, (64 x 128, 4) 17.2.
 struct PartCost {
