@@ -38,6 +38,9 @@ __global__ __launch_bounds__(kThreads, 1) void decode_megakernel_hybrid(const De
   if (threadIdx.x == 0) {
     s.best_val = -INFINITY;
     s.best_idx = 0x7fffffff;
+    s.ctl[0] = 1;
+    s.ctl[2] = 0;
+    s.ctl[3] = OP_NOOP;
   }
   const int num_insts = p_loop.num_insts;
   const int32_t* queue = p_loop.instructions + static_cast<size_t>(blockIdx.x) * num_insts * kInstWords;
@@ -45,25 +48,27 @@ __global__ __launch_bounds__(kThreads, 1) void decode_megakernel_hybrid(const De
   // The words of instruction i + 2 are asked for while instruction i runs.
   int32_t word = (threadIdx.x < kInstWords && num_insts > 0) ? queue[threadIdx.x] : 0;
   int32_t word1 = (threadIdx.x < kInstWords && num_insts > 1) ? queue[kInstWords + threadIdx.x] : 0;
+  if (threadIdx.x < kInstWords) s.inst[0][threadIdx.x] = word;
+  __syncthreads();
+  if (uniform(threadIdx.x) < kWaveSize) plan_of<PLAIN>(p_loop, s, 0);
   for (int i = 0; i < num_insts && ok; ++i) {
     if (threadIdx.x < kInstWords) {
-      s.inst[threadIdx.x] = word;
-      if (threadIdx.x == 1) s.next_layer = word1;
-      word = word1;
+      s.inst[(i + 1) & 1][threadIdx.x] = word1;
       word1 = (i + 2 < num_insts) ? queue[(i + 2) * kInstWords + threadIdx.x] : 0;
     }
     __syncthreads();
     const DecodeParams& p = params_of_this_instruction();
-    auto operand = [&](int w) { return __builtin_amdgcn_readfirstlane(s.inst[w]); };
-    const int next_layer = __builtin_amdgcn_readfirstlane(s.next_layer);
-    const Op o{next_layer >= 0 && next_layer < p.num_layers ? next_layer : 0, i, operand(0), operand(1), operand(2), operand(3), operand(4), operand(5), operand(6), operand(7), operand(8)};
+    auto operand = [&](int w) { return static_cast<int>(uniform(s.inst[i & 1][w])); };
+    const Op o{i, operand(0), operand(1), operand(2), operand(3), operand(4), operand(5), operand(6), operand(7), operand(8)};
     unsigned long long t_start = 0;
     if (p.timeline != nullptr && threadIdx.x == 0) t_start = s.t_wait = wall_clock64();
     if (o.opcode != OP_NOOP && (o.layer < 0 || o.layer >= p.num_layers || o.wait_stage >= 4 * p.groups || o.arrive_stage >= 4 * p.groups)) {
       ok = bad_operand(p, o, o.layer);
     } else {
       switch (o.opcode) {
-        case OP_NOOP: break;
+        case OP_NOOP:
+          if constexpr (!PLAIN) plan_next<PLAIN>(p, s, o);
+          break;
         case OP_IN_PROJECT:
         case OP_LRU_STEP:
         case OP_LATENT_ABSORB:
@@ -86,6 +91,7 @@ __global__ __launch_bounds__(kThreads, 1) void decode_megakernel_hybrid(const De
           break;
       }
     }
+    if constexpr (PLAIN) plan_next<PLAIN>(p, s, o);
     if (p.timeline != nullptr && threadIdx.x == 0) {
       uint64_t* rec = p.timeline + (static_cast<size_t>(blockIdx.x) * p.num_insts + i) * 8;
       rec[0] = t_start;
@@ -95,12 +101,12 @@ __global__ __launch_bounds__(kThreads, 1) void decode_megakernel_hybrid(const De
       for (int k = 0; k < 4; ++k) rec[4 + k] = s.stamps[k];
     }
     __syncthreads();
+    if (threadIdx.x == 0 && o.opcode != OP_NOOP) s.ctl[3] = o.opcode;      // (read behind the next instruction's barriers)
   }
-  if (!ok) return;
   const DecodeParams& p = params_of_this_instruction();
 
-  // Retire: the last workgroup to arrive owns the counters alone, clears them and picks the token among the
-  // workgroups' candidates (largest logit, smallest row among equals).
+  // Retire, also behind an error: the last workgroup to arrive owns the counters and units alone, clears them (its and the others' shares have been, behind
+  // the last norm's input) and picks the token among the workgroups' candidates (largest logit, smallest row among equals).
   const bool sampling = p.token_out != nullptr;
   if (sampling && threadIdx.x == 0) {
     const uint32_t bits = __float_as_uint(s.best_val);
@@ -111,10 +117,17 @@ __global__ __launch_bounds__(kThreads, 1) void decode_megakernel_hybrid(const De
   release_stores();
   __syncthreads();
   int32_t* done = counter_ptr(counters_of(p), 0, kStageGroupRows - 1, kStageGroupSlots - 1);
-  if (threadIdx.x == 0)
-    s.ctl[1] = __hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == static_cast<int>(gridDim.x) - 1;
+  if (threadIdx.x == 0) {      // upper half: workgroups that have cleared nothing
+    const int mine = s.ctl[2] ? 1 : 0x10001, all = __hip_atomic_fetch_add(done, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine;
+    s.ctl[1] = (all & 0xffff) == static_cast<int>(gridDim.x);
+    s.ctl[2] = all >> 16 == 0;
+  }
   __syncthreads();
   if (!s.ctl[1]) return;
+  const int copy = PLAIN ? layer_of(p, p.num_layers - 1).x_from : -1;
+  if (!s.ctl[2]) clear_units(p.units, p.all_units, threadIdx.x, kThreads);
+  else if (copy >= 0) clear_units(copy_of(p, copy), (2 + QMK_HYBRID_MAX_BRANCHES) * p.width, threadIdx.x, kThreads);
+  else clear_units(p.units + p.early_units, p.all_units - p.early_units, threadIdx.x, kThreads);
   const int total = p.groups * kStageGroupRows * kStageGroupSlots;
   for (int i = threadIdx.x; i < total; i += kThreads) __hip_atomic_store(p.barriers + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (!sampling || threadIdx.x >= kWaveSize) return;
@@ -285,8 +298,9 @@ struct Carver {
 };
 
 struct DecodeBuffers {
-  uint64_t* candidates;
-  float *u, *x, *out, *proj, *mix, *absorbed, *part, *ml;
+  uint64_t *candidates, *units, *proj, *mix, *absorbed, *u, *sums;
+  float *x, *part, *ml;
+  int early_units, all_units;
 };
 size_t decode_buffers(const QmkHybridArgs* a, void* base, DecodeBuffers* b) {
   size_t proj = 0, mix = 0, absorbed = 0, part = 0, ml = 0;
@@ -309,12 +323,16 @@ size_t decode_buffers(const QmkHybridArgs* a, void* base, DecodeBuffers* b) {
   }
   Carver c{static_cast<char*>(base)};
   b->candidates = c.take<uint64_t>(kMaxQueues);
-  b->u = c.take<float>(a->width);
-  b->x = c.take<float>(static_cast<size_t>(a->streams > 0 ? a->streams : 2) * a->width);
-  b->out = c.take<float>(a->streams > 0 ? 0 : static_cast<size_t>(QMK_HYBRID_MAX_BRANCHES + 1) * a->width);
-  b->proj = c.take<float>(proj);
-  b->mix = c.take<float>(mix);
-  b->absorbed = c.take<float>(absorbed);
+  const size_t units = c.used;
+  b->proj = c.take<uint64_t>(proj);
+  b->mix = c.take<uint64_t>(mix);
+  b->absorbed = c.take<uint64_t>(absorbed);
+  b->early_units = static_cast<int>((c.used - units) / sizeof(uint64_t));
+  b->u = c.take<uint64_t>(a->streams > 0 ? a->width : 0);
+  b->sums = c.take<uint64_t>(a->streams > 0 ? 0 : static_cast<size_t>(2 * (2 + QMK_HYBRID_MAX_BRANCHES)) * a->width);
+  b->all_units = static_cast<int>((c.used - units) / sizeof(uint64_t));
+  b->units = b->proj;
+  b->x = c.take<float>(static_cast<size_t>(a->streams) * a->width);
   b->part = c.take<float>(part);
   b->ml = c.take<float>(ml);
   return c.used;
@@ -822,7 +840,7 @@ extern "C" int qmk_hybrid_decode_step(const QmkHybridArgs* a) {
   DecodeParams p{};
   p.instructions = a->instructions; p.layers = a->layers_device; p.barriers = a->barriers; p.status = dev->status; p.timeline = a->timeline;
   p.candidates = b.candidates; p.embed = a->embed; p.head = a->head; p.final_norm = a->final_norm; p.token_in = a->token_in; p.token_out = a->token_out;
-  p.logits = a->logits; p.u = b.u; p.x = b.x; p.out = b.out; p.proj = b.proj; p.mix = b.mix; p.absorbed = b.absorbed; p.part = b.part; p.ml = b.ml;
+  p.logits = a->logits; p.units = b.units; p.early_units = b.early_units; p.all_units = b.all_units; p.u = b.u; p.x = b.x; p.sums = b.sums; p.proj = b.proj; p.mix = b.mix; p.absorbed = b.absorbed; p.part = b.part; p.ml = b.ml;
   p.num_insts = a->num_insts; p.num_layers = a->num_layers; p.groups = a->barrier_groups; p.width = a->width; p.width_true = a->width_true;
   p.streams = a->streams; p.vocab = a->vocab; p.vocab_rows = a->vocab_rows; p.slot = a->slot; p.position = a->position; p.flip = a->flip;
   p.max_splits = a->max_splits; p.eps = a->eps; p.logit_scale = a->logit_scale; p.logit_softcap = a->logit_softcap; p.spin_limit = a->spin_limit != 0 ? a->spin_limit : kDefaultSpinLimit;

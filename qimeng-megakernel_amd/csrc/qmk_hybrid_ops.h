@@ -1,14 +1,19 @@
 // Decode ops of the hybrid route: one workgroup executes one instruction of the tensor built by
 // decode_schedule_hybrid/instructions/scheduler.py.
 //
-// A step is a chain of stages; an instruction waits until every instruction of the stage before its own has arrived
-// (all-to-all edges on the per-XCD counters of qmk_device.h), so a buffer written in one stage may be overwritten two
-// stages later.  Activations between stages are fp32 and travel with device-coherent loads and stores; weights are
-// streamed once, bf16, and multiplied in fp32.  On a plain residual no stage adds to it: the instructions that read it next
+// A step is a chain of stages; an instruction waits for the units of the stages before that it reads, and only an attention's
+// parts are counted in (the per-XCD counters of qmk_device.h).  Activations between stages are fp32 and travel as tagged units
+// with device-coherent loads and stores; weights are streamed once, bf16, and multiplied in fp32.  On a plain residual no stage adds to it: the instructions that read it next
 // add what the layer run before has left (each for itself, one of them keeps the sum), so a norm over a branch's whole
 // output costs no stage of its own.  What does not depend on this step's earlier stages is asked for before an
 // instruction waits: its first weight rows, norm weights, recurrent states, old cache rows, the streams it will update.
+//
+// What bounds a step beside its bytes is the way from a stage's last store to the next one's first products, 3 to 4 us on the average of lusupel-1b's 89 stages:
+// the store's way, a look's way, the norm, rows behind the look.  Work that an instruction does ahead of its first look counts in full for the workgroup that
+// the others wait for, so its addresses are worked out while the instruction before waits (plan_of).
 #pragma once
+
+#include <type_traits>
 
 #include "qmk_device.h"
 #include "qmk_hybrid.h"
@@ -20,8 +25,8 @@ enum : int {
   OP_NOOP = 0,
   OP_IN_PROJECT = 1,      // norm1 + the mixer's input projections, with what can be done per output behind them
   OP_LRU_STEP = 2,        // gates of one block + the recurrence of its channels
-  OP_LATENT_ABSORB = 3,   // W_uk^T q per head; its leading instruction appends the cache row
-  OP_ATTEND = 4,          // one part of the visible keys for 16 heads
+  OP_LATENT_ABSORB = 3,   // W_uk^T q per head
+  OP_ATTEND = 4,          // one part of the visible keys for 16 heads; the one that holds the step's position appends the cache row
   OP_LATENT_VALUE = 5,    // merge of the parts, W_uv, output gate
   OP_WKV_STEP = 6,        // decay, recurrence, per-head norm and gate of one head
   OP_OUT_PROJECT = 7,     // output (sub 0) or down (sub 1) projection + all streams of the residual
@@ -48,7 +53,10 @@ constexpr int kStateBatch = 8;                // ... taken together, without bra
 constexpr int kStateVector = kMaxHeadDim + kStateBatch * kThreads / 16;   // places of q, k and the decays in LDS, zeros behind head_dim
 constexpr int kMaxParts = 64;
 constexpr int kDepth = 8;                     // weight rows a wave keeps in flight and reduces together
-constexpr int kAhead = 2;                     // quads of a vector a thread holds in registers (4096 elements a workgroup)
+// ... of which so many are asked for ahead of the wait, the others when the vector has come: looks and stores of a hand-over stand behind the requests for rows
+// in the memory system's queues (us a step with 2, 4, 6 and 8 ahead: lusupel-1b 760, 749, 761, 767; givopel-1b with 4, 6 and 8 580, 601, 612).
+constexpr int kRowsFirst = 4;
+constexpr int kFewTaps = 4;                   // taps of a convolution whose inputs and weights a thread holds
 constexpr int kStageGroupRows = 54;           // the counter layout of one group of four stages (qmk_device.h)
 constexpr int kStageGroupSlots = 48;
 
@@ -65,12 +73,14 @@ struct DecodeParams {
   const int64_t* token_in;
   int64_t* token_out;
   float* logits;
-  float* u;          // [D] input of the next sublayer before its norm
-  float* x;          // [streams][D], plain: [2][D]
-  float* out;        // plain: [branches, feed-forward][D] what a layer run adds to x
-  float* proj;       // outputs of OP_IN_PROJECT
-  float* mix;        // what the output / down projection reads
-  float* absorbed;   // [heads][rank]
+  // units (below), but for the streams
+  uint64_t* u;          // [D] input of the next sublayer before its norm
+  uint64_t* sums;       // plain: [2][1 + branches + 1][D] a copy of the residual and what the run that has left it adds: branches, feed-forward
+  uint64_t* proj;       // outputs of OP_IN_PROJECT
+  uint64_t* mix;        // what the output / down projection reads
+  uint64_t* absorbed;   // [heads][rank], in bf16 mode pairs of rounded values
+  uint64_t* units;      // all of them
+  float* x;             // [streams][D], each element's owner alone
   float* part;       // [parts][heads16][rank] unnormalised sums
   float* ml;         // [parts][heads16][2] maximum (log2) and sum
   int32_t num_insts;
@@ -80,9 +90,30 @@ struct DecodeParams {
   int32_t vocab, vocab_rows;
   int32_t slot, position, flip;
   int32_t max_splits;
+  int32_t early_units, all_units;      // those that nobody reads any more when the last norm's input has come stand first
   float eps, logit_scale, logit_softcap;
   uint32_t spin_limit;
 };
+
+// What the first requests of an instruction that streams rows need, worked out while the instruction before it ends: its rows, the vector that they are
+// multiplied with; plain: what makes the residual (x, two branches).
+struct Plan {
+  const u16* w;
+  int rows, columns;           // rows 0: an operand is out of range
+  const uint64_t* from;
+  int length;
+  uint32_t tag;
+  const uint64_t* sum[3];
+  uint32_t sum_tag[3];
+};
+
+// Values that are the same in all lanes, in scalar registers.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(v)); }
+template <class P>
+__device__ __forceinline__ P* uniform(P* v) {
+  const uint64_t bits = reinterpret_cast<uint64_t>(v);
+  return reinterpret_cast<P*>(static_cast<uint64_t>(uniform(static_cast<uint32_t>(bits >> 32))) << 32 | uniform(static_cast<uint32_t>(bits)));
+}
 
 struct Smem {
   union {
@@ -94,9 +125,9 @@ struct Smem {
   };
   float aux[3072];
   float scratch[3 * kWaves];
-  int32_t inst[kInstWords];
-  int32_t next_layer;
-  int32_t ctl[4];          // [0] wait result, [1] last to retire
+  int32_t inst[2][kInstWords];      // of even and of odd index: this instruction and the one behind it
+  Plan plan[2];                     // of an instruction of even and of odd index
+  int32_t ctl[4];          // [0] no wait has failed, [1] last to retire, [2] this workgroup has cleared its share of the units
   uint64_t t_wait;
   uint64_t stamps[4];      // timeline only: requests made, vector in LDS, rows multiplied, results stored
   float best_val;
@@ -110,7 +141,6 @@ using ConstFloat = const __attribute__((address_space(4))) float;
 __device__ __forceinline__ LayerRef& layer_of(const DecodeParams& p, int layer) { return ((LayerRef*)p.layers)[layer]; }
 
 struct Op {                // decoded instruction
-  int next_layer;          // the instruction behind it: its layer's table entry is fetched during the wait
   int index, opcode, layer, sub, start, count, wait_stage, wait_count, arrive_stage, extra;
 };
 
@@ -135,31 +165,100 @@ __device__ __forceinline__ void stamp(const DecodeParams& p, Smem& s, int which)
   if (p.timeline != nullptr && threadIdx.x == 0) s.stamps[which] = wall_clock64();
 }
 
+// ---- hand-over ----
+// What a workgroup leaves for others of the same launch is 8-byte units {value, tag}, each stored at once: a reader looks at the units it needs until all carry
+// the tag of their entry and half of it, so nobody waits for stores to be acknowledged, counts arrivals or fetches behind a count.  Tags grow along the
+// model: a unit's next writer depends on all of its readers through the data (an output row needs every product before it), but for rows of padding,
+// whose readers may find the next one there already.  What is read is cleared before the launch ends (OP_LM_HEAD, retirement), failed launches included:
+// nothing is kept, and a tag is a pattern (a float of 2.3e18) that nothing else that may use the buffer leaves there.  Only the parts of an attention,
+// up to 64 KB for each reader, stay on counters: their readers would look at them all through the attention.
+// us a step, counters and leaders on every stage -> so: lusupel-1b, 1000 positions 804 -> 745, givopel-1b, 600 positions 605 -> 580.
+constexpr uint32_t kTagBase = 0x5e000000u, kTags = 1u << 20;
+__device__ __forceinline__ uint32_t tag_of(int entry, int half) { return kTagBase + 2 * static_cast<uint32_t>(entry) + half; }
+__device__ __forceinline__ bool has_come(uint64_t unit, uint32_t tag) { return static_cast<uint32_t>(unit >> 32) - tag < kTags; }
+__device__ __forceinline__ void put_bits(uint64_t* at, uint32_t bits, uint32_t tag) {
+  __hip_atomic_store(at, static_cast<uint64_t>(tag) << 32 | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void put_unit(uint64_t* at, float v, uint32_t tag) { put_bits(at, __float_as_uint(v), tag); }
+__device__ __forceinline__ float value_of(uint64_t unit) { return __uint_as_float(static_cast<uint32_t>(unit)); }
+
+__device__ __forceinline__ void wait_failed(const DecodeParams& p, Smem& s, const Op& o) {
+  if (static_cast<int>(threadIdx.x) == __builtin_amdgcn_readfirstlane(threadIdx.x)) {
+    s.ctl[0] = 0;
+    report_error(counters_of(p), QMK_DEV_WAIT_TIMEOUT, o.index, o.opcode, o.wait_stage);
+  }
+}
+
+// Behind a failed wait of this workgroup the others end early.
+__device__ __forceinline__ bool out_of_looks(const DecodeParams& p, Smem& s, const Op& o, uint32_t looks) {
+  if (looks > p.spin_limit) {
+    wait_failed(p, s, o);
+    return true;
+  }
+  return (looks & 63) == 0 && *const_cast<volatile int32_t*>(s.ctl) == 0;
+}
+
+// Units first, first + step, .. of v[0 .. end): `ask` makes the first look, `wait` the others.  A wait that runs out of looks leaves what is there, and
+// ctl[0] = 0 behind the next barrier.
+template <int N>
+struct Units {
+  uint64_t r[N];
+  __device__ __forceinline__ void ask(const uint64_t* v, int first, int step, int end) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) r[j] = ld_shared64(v + min(first + j * step, end - 1));
+  }
+  __device__ __forceinline__ void wait(const DecodeParams& p, Smem& s, const Op& o, const uint64_t* v, int first, int step, int end, uint32_t tag) {
+    uint32_t looks = 0;
+    while (true) {
+      bool all = true;
+#pragma unroll
+      for (int j = 0; j < N; ++j) all = all && has_come(r[j], tag);
+      if (__all(all)) return;
+      if (out_of_looks(p, s, o, ++looks)) return;
+      ask(v, first, step, end);
+    }
+  }
+  __device__ __forceinline__ float operator[](int j) const { return value_of(r[j]); }
+};
+// The same of units at places of their own.
+template <int N>
+struct Gather {
+  const uint64_t* at[N];
+  uint64_t r[N];
+  __device__ __forceinline__ void ask() {
+#pragma unroll
+    for (int j = 0; j < N; ++j) r[j] = ld_shared64(at[j]);
+  }
+  __device__ __forceinline__ void wait(const DecodeParams& p, Smem& s, const Op& o, uint32_t tag) {
+    uint32_t looks = 0;
+    while (true) {
+      bool all = true;
+#pragma unroll
+      for (int j = 0; j < N; ++j) all = all && has_come(r[j], tag);
+      if (__all(all)) return;
+      if (out_of_looks(p, s, o, ++looks)) return;
+      ask();
+    }
+  }
+  __device__ __forceinline__ float operator[](int j) const { return value_of(r[j]); }
+};
+// One unit of every active lane.
+__device__ __forceinline__ float unit_of(const DecodeParams& p, Smem& s, const Op& o, const uint64_t* at, uint32_t tag) {
+  Units<1> u;
+  u.ask(at, 0, 0, 1);
+  u.wait(p, s, o, at, 0, 0, 1, tag);
+  return u[0];
+}
+
+// The attention's parts: counted arrivals of a whole stage.
 __device__ __forceinline__ bool wait_stage(const DecodeParams& p, Smem& s, const Op& o) {
   if (o.wait_stage < 0) return true;
   const Params c = counters_of(p);
-  if (threadIdx.x < kWaveSize) {
-    const bool ok = wait_edge_xcd(c, o.wait_stage >> 2, 2 + (o.wait_stage & 3), o.wait_count, p.spin_limit);
-    if (threadIdx.x == 0) {
-      s.ctl[0] = ok;
-      if (!ok) report_error(c, QMK_DEV_WAIT_TIMEOUT, o.index, o.opcode, o.wait_stage);
-      if (p.timeline != nullptr) s.t_wait = wall_clock64();
-    }
-  } else if (threadIdx.x < 2 * kWaveSize) {
-    const auto* line = (const __attribute__((address_space(4))) int32_t*)(p.layers + o.next_layer);
-#pragma unroll
-    for (int i = 0; i < static_cast<int>(sizeof(QmkHybridLayer) / 64); ++i) {
-      const int32_t v = line[i * 16];
-      asm volatile("" ::"s"(v));
-    }
-  }
+  if (threadIdx.x < kWaveSize && !wait_edge_xcd(c, o.wait_stage >> 2, 2 + (o.wait_stage & 3), o.wait_count, p.spin_limit)) wait_failed(p, s, o);
   __syncthreads();
   return s.ctl[0] != 0;
 }
-
 __device__ __forceinline__ void arrive_stage(const DecodeParams& p, const Op& o) {
-  release_stores();
-  __syncthreads();
   if (threadIdx.x == 0 && o.arrive_stage >= 0) arrive_all(counters_of(p), o.arrive_stage >> 2, 2 + (o.arrive_stage & 3), 1);
 }
 
@@ -223,7 +322,14 @@ struct RowStream {
     at = w + first * pitch;
     const u16* top = at + column(chunk);
 #pragma unroll
-    for (int j = 0; j < kDepth; ++j)
+    for (int j = 0; j < kRowsFirst; ++j)
+      if (j < n) r[j] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(top + j * pitch));
+  }
+  // Behind the wait.
+  __device__ __forceinline__ void rest() {
+    const u16* top = at + column(chunk);
+#pragma unroll
+    for (int j = kRowsFirst; j < kDepth; ++j)
       if (j < n) r[j] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(top + j * pitch));
   }
   // part[wave][row] += sums; part must be zero, one barrier behind it.
@@ -330,25 +436,30 @@ __device__ __forceinline__ float row_total(const Smem& s, int row) {
   return t;
 }
 
-__device__ __forceinline__ float4 ld_shared_quad(const float* v) {
-  const uint64_t a = ld_shared64(v), b = ld_shared64(v + 2);
-  return make_float4(__uint_as_float(static_cast<uint32_t>(a)), __uint_as_float(static_cast<uint32_t>(a >> 32)),
-                     __uint_as_float(static_cast<uint32_t>(b)), __uint_as_float(static_cast<uint32_t>(b >> 32)));
-}
-__device__ __forceinline__ float4& xs_quad(Smem& s, int i) { return *reinterpret_cast<float4*>(s.xs + xs_at(i)); }   // i % 4 == 0
+__device__ __forceinline__ float& xs_value(Smem& s, int i) { return s.xs[xs_at(i)]; }
 
-// fp32 vector that other workgroups wrote in this launch -> xs (n a multiple of 4), four requests of a thread at a time
-__device__ __forceinline__ void load_vector(Smem& s, const float* v, int n) {
-  constexpr int kStep = kThreads * 4, kBatch = 4;
+// A thread's elements of a vector: tid, tid + 512, .., the first kHeld of them in registers.
+constexpr int kHeld = 4, kHeldSpan = kHeld * kThreads;
+using Look = Units<kHeld>;
+
+// Behind a first look at the first kHeldSpan of them: units v[0 .. n) -> xs.
+template <class F>
+__device__ __forceinline__ void load_vector(const DecodeParams& p, Smem& s, const Op& o, Look& look, const uint64_t* v, int n, uint32_t tag, F&& seen) {
+  const int tid = threadIdx.x;
+  look.wait(p, s, o, v, tid, kThreads, n, tag);
+  seen();
+#pragma unroll
+  for (int j = 0; j < kHeld; ++j)
+    if (tid + j * kThreads < n) xs_value(s, tid + j * kThreads) = look[j];
+  constexpr int kBatch = 12;
 #pragma unroll 1
-  for (int base = threadIdx.x * 4; base < n; base += kBatch * kStep) {
-    float4 t[kBatch];
+  for (int base = kHeldSpan; base < n; base += kBatch * kThreads) {
+    Units<kBatch> more;
+    more.ask(v, base + tid, kThreads, n);
+    more.wait(p, s, o, v, base + tid, kThreads, n, tag);
 #pragma unroll
     for (int j = 0; j < kBatch; ++j)
-      if (base + j * kStep < n) t[j] = ld_shared_quad(v + base + j * kStep);
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j)
-      if (base + j * kStep < n) xs_quad(s, base + j * kStep) = t[j];
+      if (base + tid + j * kThreads < n) xs_value(s, base + tid + j * kThreads) = more[j];
   }
 }
 
@@ -363,207 +474,250 @@ __device__ __forceinline__ float weight_sum(const float* w, int n) {
   return t;
 }
 
-// A thread's quads i = 4 tid + 2048 j of a [n] vector, j < kAhead
-__device__ __forceinline__ void load_ahead(float4 (&v)[kAhead], const float* from, int n) {
+// A thread's first elements of a [n] vector that no one writes.
+__device__ __forceinline__ void load_ahead(float (&v)[kHeld], const float* from, int n) {
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    const int i = (j * kThreads + static_cast<int>(threadIdx.x)) * 4;
-    if (i < n) v[j] = *reinterpret_cast<const float4*>(from + i);
-  }
-}
-__device__ __forceinline__ float4 times(float4 a, float4 b, float c) { return make_float4(a.x * b.x * c, a.y * b.y * c, a.z * b.z * c, a.w * b.w * c); }
-__device__ __forceinline__ float square(float4 a, float t) { return fmaf(a.w, a.w, fmaf(a.z, a.z, fmaf(a.y, a.y, fmaf(a.x, a.x, t)))); }
-
-// A quad of the sublayer input.  `first`: the embedding seen through the first layer's weights (their sum `g`).
-__device__ __forceinline__ float4 input_quad(const DecodeParams& p, bool first, const u16* e, float g, int i) {
-  if (!first) return ld_shared_quad(p.u + i);
-  const uint2 t = *reinterpret_cast<const uint2*>(e + i);
-  return make_float4(bf_lo(t.x) * g, bf_hi(t.x) * g, bf_lo(t.y) * g, bf_hi(t.y) * g);
+  for (int j = 0; j < kHeld; ++j) v[j] = from[min(static_cast<int>(threadIdx.x) + j * kThreads, n - 1)];
 }
 
-// RMS norm of the sublayer input -> xs; `ahead`: the thread's first norm weights.
-__device__ __forceinline__ void norm_to_xs(const DecodeParams& p, Smem& s, const float* weight, const float4 (&ahead)[kAhead], bool first, const float* hc_in) {
+// RMS norm of the sublayer input -> xs; `ahead`: the thread's first norm weights.  `first`: the input is the embedding seen through the first layer's
+// weights (their sum).
+template <class F>
+__device__ __forceinline__ void norm_to_xs(const DecodeParams& p, Smem& s, const Op& o, Look& look, uint32_t tag, const float* weight, const float (&ahead)[kHeld], bool first,
+                                           const float* hc_in, F&& seen) {
   const int D = p.width, tid = threadIdx.x;
   const u16* e = p.embed;
   float g = 0.f;
   if (first) {
     e += static_cast<size_t>(token_of(p)) * D;
     g = weight_sum(hc_in, p.streams);
+  } else {
+    look.wait(p, s, o, p.u, tid, kThreads, D, tag);
   }
-  float4 v[kAhead];
-  float sq = 0.f;
+  seen();
+  float v[kHeld], sq = 0.f;
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    const int i = (j * kThreads + tid) * 4;
-    v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i < D) v[j] = input_quad(p, first, e, g, i);
+  for (int j = 0; j < kHeld; ++j) {
+    const int i = tid + j * kThreads;
+    v[j] = i < D ? first ? bf2f(e[i]) * g : look[j] : 0.f;
+    sq = fmaf(v[j], v[j], sq);
   }
-#pragma unroll
-  for (int j = 0; j < kAhead; ++j) sq = square(v[j], sq);
 #pragma unroll 1
-  for (int i = (kAhead * kThreads + tid) * 4; i < D; i += kThreads * 4) {
-    const float4 t = input_quad(p, first, e, g, i);
-    sq = square(t, sq);
-    xs_quad(s, i) = t;
+  for (int base = kHeldSpan; base < D; base += kHeldSpan) {
+    Look more;
+    if (!first) {
+      more.ask(p.u, base + tid, kThreads, D);
+      more.wait(p, s, o, p.u, base + tid, kThreads, D, tag);
+    }
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) {
+      const int i = base + tid + j * kThreads;
+      if (i < D) {
+        const float t = first ? bf2f(e[i]) * g : more[j];
+        sq = fmaf(t, t, sq);
+        xs_value(s, i) = t;
+      }
+    }
   }
   const float inv = 1.f / sqrtf(block_sum(sq, s.scratch) / p.width_true + p.eps);
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    const int i = (j * kThreads + tid) * 4;
-    if (i < D) xs_quad(s, i) = times(v[j], ahead[j], inv);
-  }
+  for (int j = 0; j < kHeld; ++j)
+    if (tid + j * kThreads < D) xs_value(s, tid + j * kThreads) = v[j] * ahead[j] * inv;
 #pragma unroll 1
-  for (int i = (kAhead * kThreads + tid) * 4; i < D; i += kThreads * 4)
-    xs_quad(s, i) = times(xs_quad(s, i), *reinterpret_cast<const float4*>(weight + i), inv);
+  for (int i = kHeldSpan + tid; i < D; i += kThreads) xs_value(s, i) = xs_value(s, i) * weight[i] * inv;
 }
 
-__device__ __forceinline__ void st_shared_quad(float* to, float4 v) {
-  auto pair = [](float lo, float hi) { return (static_cast<uint64_t>(__float_as_uint(hi)) << 32) | __float_as_uint(lo); };
-  __hip_atomic_store(reinterpret_cast<uint64_t*>(to), pair(v.x, v.y), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(reinterpret_cast<uint64_t*>(to) + 1, pair(v.z, v.w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float4 embed_quad(const u16* e, int i) {
-  const uint2 t = *reinterpret_cast<const uint2*>(e + i);
-  return make_float4(bf_lo(t.x), bf_hi(t.x), bf_lo(t.y), bf_hi(t.y));
-}
-__device__ __forceinline__ float4 plus(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-__device__ __forceinline__ float4 multiply_add(float4 a, float4 b, float c, float4 t) {   // a b c + t
-  return make_float4(fmaf(a.x * b.x, c, t.x), fmaf(a.y * b.y, c, t.y), fmaf(a.z * b.z, c, t.z), fmaf(a.w * b.w, c, t.w));
-}
+// A copy of the plain residual and, behind it, what the run that leaves it adds.  (Two of both: a run's first outputs may be ready before the last of the
+// workgroups that read the run before has read it.)
+__device__ __forceinline__ uint64_t* copy_of(const DecodeParams& p, int copy) { return p.sums + static_cast<size_t>(copy) * (2 + QMK_HYBRID_MAX_BRANCHES) * p.width; }
+
+// First looks at what makes the plain residual.
+struct ResidualLook {
+  Look x, a, b;
+  const uint64_t *x_at, *a_at, *b_at;
+  uint32_t x_tag, a_tag, b_tag;
+  __device__ __forceinline__ void ask(const DecodeParams& p, const Plan& plan) {
+    const int D = p.width, tid = threadIdx.x;
+    x_at = uniform(plan.sum[0]);
+    a_at = uniform(plan.sum[1]);
+    b_at = uniform(plan.sum[2]);
+    x_tag = uniform(plan.sum_tag[0]);
+    a_tag = uniform(plan.sum_tag[1]);
+    b_tag = uniform(plan.sum_tag[2]);
+    x.ask(x_at, tid, kThreads, D);
+    a.ask(a_at, tid, kThreads, D);
+    b.ask(b_at, tid, kThreads, D);
+  }
+};
 
 // The plain residual as a run (or the model's norm, or a loop's pass) reads it: the copy `x_from` plus what the run `prev`
 // left.  normed: its norm under `weight` -> xs (`ahead`: the thread's first weights); otherwise [x; embedding] -> xs.
 // keep: also leaves the sum in copy `x_to`.
-__device__ __forceinline__ void residual_to_xs(const DecodeParams& p, Smem& s, LayerRef& l, bool normed, bool keep, const float* weight, const float4 (&ahead)[kAhead]) {
+template <class F>
+__device__ __forceinline__ void residual_to_xs(const DecodeParams& p, Smem& s, const Op& o, LayerRef& l, int lead, ResidualLook& look, bool normed, bool keep, const float* weight,
+                                               const float (&ahead)[kHeld], F&& seen) {
   const int D = p.width, tid = threadIdx.x;
   const u16* e = p.embed;
-  if (l.x_from < 0 || !normed) e += static_cast<size_t>(token_of(p)) * D;
-  const float* x = l.x_from < 0 ? nullptr : p.x + static_cast<size_t>(l.x_from) * D;
-  const bool added = l.prev >= 0;
-  LayerRef& before = layer_of(p, added ? l.prev : 0);
-  const bool two = added && before.branches == 2, ff = added && before.has_mlp;
+  const bool embed = l.x_from < 0, added = l.prev >= 0;
+  if (embed || !normed) e += static_cast<size_t>(token_of(p)) * D;
+  LayerRef& run = layer_of(p, added ? l.prev : 0);
+  const bool two = added && run.branches == 2;
   const float *wa = nullptr, *wb = nullptr;
   if (two) {
-    wa = before.out_norm;
+    wa = run.out_norm;
     wb = layer_of(p, l.prev + 1).out_norm;
   }
-  // x, feed-forward and a lone branch in `v`; two branches in `a` and `b`, their norm weights in `na` and `nb`
-  auto fetch = [&](int i, float4& v, float4& a, float4& b, float4& na, float4& nb) {
-    v = x == nullptr ? embed_quad(e, i) : ld_shared_quad(x + i);
-    if (!added) return;
-    a = ld_shared_quad(p.out + i);
-    if (two) {
-      b = ld_shared_quad(p.out + D + i);
-      na = *reinterpret_cast<const float4*>(wa + i);
-      nb = *reinterpret_cast<const float4*>(wb + i);
-    }
-    if (ff) v = plus(v, ld_shared_quad(p.out + static_cast<size_t>(QMK_HYBRID_MAX_BRANCHES) * D + i));
-    if (!two) v = plus(v, a);
-  };
-  float4 v[kAhead], a[kAhead], b[kAhead], na[kAhead], nb[kAhead];
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  float sum[3] = {0.f, 0.f, 0.f};
+  // x and a lone branch in `v`; two branches in `a` and `b`, their norm weights in `na` and `nb`
+  auto fetch = [&](ResidualLook& k, int first, float (&v)[kHeld], float (&a)[kHeld], float (&b)[kHeld], float (&na)[kHeld], float (&nb)[kHeld]) {
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    const int i = (j * kThreads + tid) * 4;
-    v[j] = a[j] = b[j] = na[j] = nb[j] = zero;
-    if (i < D) fetch(i, v[j], a[j], b[j], na[j], nb[j]);
-  }
+    for (int j = 0; j < kHeld; ++j) {
+      const int i = min(first + j * kThreads, D - 1);
+      v[j] = a[j] = b[j] = na[j] = nb[j] = 0.f;
+      if (two) {
+        na[j] = wa[i];
+        nb[j] = wb[i];
+      }
+      if (embed) v[j] = bf2f(e[i]);
+    }
+    if (!embed) k.x.wait(p, s, o, look.x_at, first, kThreads, D, look.x_tag);
+    if (added) k.a.wait(p, s, o, look.a_at, first, kThreads, D, look.a_tag);
+    if (two) k.b.wait(p, s, o, look.b_at, first, kThreads, D, look.b_tag);
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) {
+      const bool in = first + j * kThreads < D;
+      if (!embed) v[j] = k.x[j];
+      if (two) {
+        a[j] = in ? k.a[j] : 0.f;
+        b[j] = in ? k.b[j] : 0.f;
+      } else if (added) {
+        v[j] += k.a[j];
+      }
+      if (!in) v[j] = 0.f;
+    }
+  };
+  auto again = [&](ResidualLook& k, int first) {
+    k.x.ask(look.x_at, first, kThreads, D);
+    k.a.ask(look.a_at, first, kThreads, D);
+    k.b.ask(look.b_at, first, kThreads, D);
+  };
+  float v[kHeld], a[kHeld], b[kHeld], na[kHeld], nb[kHeld];
+  float sum[3] = {0.f, 0.f, 0.f};
+  fetch(look, tid, v, a, b, na, nb);
+  seen();
   float sa = 0.f, sb = 0.f;
   if (two) {
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      sum[0] = square(a[j], sum[0]);
-      sum[1] = square(b[j], sum[1]);
+    for (int j = 0; j < kHeld; ++j) {
+      sum[0] = fmaf(a[j], a[j], sum[0]);
+      sum[1] = fmaf(b[j], b[j], sum[1]);
     }
 #pragma unroll 1
-    for (int i = (kAhead * kThreads + tid) * 4; i < D; i += kThreads * 4) {
-      sum[0] = square(ld_shared_quad(p.out + i), sum[0]);
-      sum[1] = square(ld_shared_quad(p.out + D + i), sum[1]);
+    for (int base = kHeldSpan; base < D; base += kHeldSpan) {
+      Look ma, mb;
+      ma.ask(look.a_at, base + tid, kThreads, D);
+      mb.ask(look.b_at, base + tid, kThreads, D);
+      ma.wait(p, s, o, look.a_at, base + tid, kThreads, D, look.a_tag);
+      mb.wait(p, s, o, look.b_at, base + tid, kThreads, D, look.b_tag);
+#pragma unroll
+      for (int j = 0; j < kHeld; ++j) {
+        const bool in = base + tid + j * kThreads < D;
+        const float ta = in ? ma[j] : 0.f, tb = in ? mb[j] : 0.f;
+        sum[0] = fmaf(ta, ta, sum[0]);
+        sum[1] = fmaf(tb, tb, sum[1]);
+      }
     }
     block_sum3(sum, s.scratch);
-    sa = before.out_scale / sqrtf(sum[0] / p.width_true + p.eps);
-    sb = before.out_scale / sqrtf(sum[1] / p.width_true + p.eps);
+    const float scale = run.out_scale;
+    sa = scale / sqrtf(sum[0] / p.width_true + p.eps);
+    sb = scale / sqrtf(sum[1] / p.width_true + p.eps);
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) v[j] = multiply_add(b[j], nb[j], sb, multiply_add(a[j], na[j], sa, v[j]));
+    for (int j = 0; j < kHeld; ++j) v[j] = fmaf(b[j] * nb[j], sb, fmaf(a[j] * na[j], sa, v[j]));
   }
-  float* x_to = p.x + static_cast<size_t>(l.x_to) * D;
+  uint64_t* x_to = copy_of(p, l.x_to);
+  const uint32_t kept = tag_of(lead, 0);
   float total = 0.f;
-  auto take = [&](int i, float4 t) {
-    total += t.x + t.y + t.z + t.w;
-    if (keep) st_shared_quad(x_to + i, t);
+  auto take = [&](int i, float t) {
+    total += t;
+    if (keep) put_unit(x_to + i, t, kept);
     if (!normed) {
-      xs_quad(s, i) = t;
-      xs_quad(s, D + i) = embed_quad(e, i);
+      xs_value(s, i) = t;
+      xs_value(s, D + i) = bf2f(e[i]);
     }
   };
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    const int i = (j * kThreads + tid) * 4;
-    if (i < D) take(i, v[j]);
-  }
+  for (int j = 0; j < kHeld; ++j)
+    if (tid + j * kThreads < D) take(tid + j * kThreads, v[j]);
 #pragma unroll 1
-  for (int i = (kAhead * kThreads + tid) * 4; i < D; i += kThreads * 4) {
-    float4 t = zero, ta = zero, tb = zero, ua = zero, ub = zero;
-    fetch(i, t, ta, tb, ua, ub);
-    if (two) t = multiply_add(tb, ub, sb, multiply_add(ta, ua, sa, t));
-    take(i, t);
-    if (normed) xs_quad(s, i) = t;
+  for (int base = kHeldSpan; base < D; base += kHeldSpan) {
+    ResidualLook more;
+    float t[kHeld], ta[kHeld], tb[kHeld], ua[kHeld], ub[kHeld];
+    again(more, base + tid);
+    fetch(more, base + tid, t, ta, tb, ua, ub);
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) {
+      const int i = base + tid + j * kThreads;
+      if (i >= D) continue;
+      if (two) t[j] = fmaf(tb[j] * ub[j], sb, fmaf(ta[j] * ua[j], sa, t[j]));
+      take(i, t[j]);
+      if (normed) xs_value(s, i) = t[j];
+    }
   }
   if (!normed) return;
   const float mean = l.norm == QMK_NORM_LAYER ? block_sum(total, s.scratch) / p.width_true : 0.f;
-  auto centred = [&](int i, float4 t) {   // storage columns behind the true width stay zero
-    return make_float4(i < p.width_true ? t.x - mean : 0.f, i + 1 < p.width_true ? t.y - mean : 0.f, i + 2 < p.width_true ? t.z - mean : 0.f,
-                       i + 3 < p.width_true ? t.w - mean : 0.f);
-  };
+  auto centred = [&](int i, float t) { return i < p.width_true ? t - mean : 0.f; };   // storage columns behind the true width stay zero
   float sq = 0.f;
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    v[j] = centred((j * kThreads + tid) * 4, v[j]);
-    sq = square(v[j], sq);
+  for (int j = 0; j < kHeld; ++j) {
+    v[j] = centred(tid + j * kThreads, v[j]);
+    sq = fmaf(v[j], v[j], sq);
   }
 #pragma unroll 1
-  for (int i = (kAhead * kThreads + tid) * 4; i < D; i += kThreads * 4) {
-    const float4 t = centred(i, xs_quad(s, i));
-    sq = square(t, sq);
-    xs_quad(s, i) = t;
+  for (int i = kHeldSpan + tid; i < D; i += kThreads) {
+    const float t = centred(i, xs_value(s, i));
+    sq = fmaf(t, t, sq);
+    xs_value(s, i) = t;
   }
   const float inv = 1.f / sqrtf(block_sum(sq, s.scratch) / p.width_true + p.eps);
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j) {
-    const int i = (j * kThreads + tid) * 4;
-    if (i < D) xs_quad(s, i) = times(v[j], ahead[j], inv);
-  }
+  for (int j = 0; j < kHeld; ++j)
+    if (tid + j * kThreads < D) xs_value(s, tid + j * kThreads) = v[j] * ahead[j] * inv;
 #pragma unroll 1
-  for (int i = (kAhead * kThreads + tid) * 4; i < D; i += kThreads * 4)
-    xs_quad(s, i) = times(xs_quad(s, i), *reinterpret_cast<const float4*>(weight + i), inv);
+  for (int i = kHeldSpan + tid; i < D; i += kThreads) xs_value(s, i) = xs_value(s, i) * weight[i] * inv;
 }
 
-// What a gla or delta entry left in xs, head by head: RMS norm over the head's values, weight, output gate.
-__device__ __forceinline__ void norm_heads(const DecodeParams& p, Smem& s, LayerRef& l) {
-  const int lane = threadIdx.x & (kWaveSize - 1), wave = threadIdx.x / kWaveSize, n = l.v_dim;
-  const float* gate = p.proj + l.proj_at + (l.type == QMK_MIXER_DELTA ? l.in_rows : 2 * l.heads * l.head_dim + l.mix_width);
+// What a gla or delta entry left in xs, head by head, a wave each: RMS norm over the head's values, weight, output gate.  The first head's gates are asked for ahead
+// of the wait, the others' while the head before is normed.
+struct HeadGates {
+  static constexpr int kPer = kMaxHeadDim / kWaveSize;
+  Units<kPer> g;
+  __device__ __forceinline__ static const uint64_t* of(const DecodeParams& p, LayerRef& l, int head) {
+    return p.proj + l.proj_at + (l.type == QMK_MIXER_DELTA ? l.in_rows : 2 * l.heads * l.head_dim + l.mix_width) + min(head, l.heads - 1) * l.v_dim;
+  }
+  __device__ __forceinline__ void ask(const DecodeParams& p, LayerRef& l, int head) { g.ask(of(p, l, head), threadIdx.x & (kWaveSize - 1), kWaveSize, l.v_dim); }
+};
+__device__ __forceinline__ void norm_heads(const DecodeParams& p, Smem& s, const Op& o, LayerRef& l, HeadGates& gates) {
+  constexpr int kPer = HeadGates::kPer;
+  const int lane = threadIdx.x & (kWaveSize - 1), wave = uniform(threadIdx.x / kWaveSize), n = l.v_dim;
   __syncthreads();
-  constexpr int kPer = kMaxHeadDim / kWaveSize;
 #pragma unroll 1
   for (int head = wave; head < l.heads; head += kWaves) {
-    float v[kPer], g[kPer], sq = 0.f;
+    HeadGates next;
+    next.ask(p, l, head + kWaves);
+    gates.g.wait(p, s, o, HeadGates::of(p, l, head), lane, kWaveSize, n, tag_of(o.layer, 0));
+    float v[kPer], sq = 0.f;
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
       const int i = j * kWaveSize + lane;
-      v[j] = g[j] = 0.f;
-      if (i < n) {
-        v[j] = s.xs[xs_at(head * n + i)];
-        g[j] = ld_shared_f32(gate + head * n + i) * l.vec0[i];
-      }
+      v[j] = i < n ? s.xs[xs_at(head * n + i)] : 0.f;
       sq = fmaf(v[j], v[j], sq);
     }
     const float inv = 1.f / sqrtf(wave_sum(sq) / l.v_true + p.eps);
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
       const int i = j * kWaveSize + lane;
-      if (i < n) s.xs[xs_at(head * n + i)] = v[j] * inv * g[j];
+      if (i < n) s.xs[xs_at(head * n + i)] = v[j] * inv * (gates.g[j] * l.vec0[i]);
     }
+    gates = next;
   }
 }
 
@@ -585,11 +739,6 @@ __device__ __forceinline__ void rotate(const Layer& l, int position, int d, floa
   const float x = a * c - b * sn;
   b = b * c + a * sn;
   a = x;
-}
-
-template <class T>
-__device__ __forceinline__ T* cache_row(const DecodeParams& p, LayerRef& l, int position) {
-  return static_cast<T*>(l.cache) + (static_cast<size_t>(p.slot) * l.ring + position % l.ring) * (l.rank + l.rot_dim);
 }
 
 // ---- the ops that stream weight rows: one body, so that the streaming code exists once ----
@@ -637,86 +786,186 @@ __device__ __forceinline__ bool rows_of(const DecodeParams& p, LayerRef& l, cons
   }
 }
 
+// The plan of an instruction, by one wave.
+template <bool PLAIN>
+__device__ __forceinline__ void plan_of(const DecodeParams& p, Smem& s, int index) {
+  const int32_t* words = s.inst[index & 1];
+  auto operand = [&](int w) { return static_cast<int>(uniform(words[w])); };
+  const Op o{index, operand(0), operand(1), operand(2), operand(3), operand(4), operand(5), operand(6), operand(7), operand(8)};
+  Plan t{};
+  if (o.opcode != OP_NOOP && o.layer >= 0 && o.layer < p.num_layers) {
+    LayerRef& l = layer_of(p, o.layer);
+    Rows m{};
+    if (rows_of(p, l, o, m)) {
+      const int op = o.opcode, D = p.width;
+      const bool delta = l.type == QMK_MIXER_DELTA;
+      t.w = m.w;
+      t.rows = m.rows;
+      t.columns = m.columns;
+      t.from = p.proj;
+      t.length = m.columns;
+      t.tag = tag_of(o.layer, 0);
+      if (op == OP_OUT_PROJECT) {
+        t.from = p.mix + (o.sub == 1 ? l.ff_at : l.mix_at);
+        t.tag = tag_of(o.layer, o.sub);
+      } else if constexpr (!PLAIN) {
+        if (op == OP_IN_PROJECT || op == OP_UP_GATE || op == OP_LM_HEAD) {
+          const int before = op == OP_IN_PROJECT ? max(o.layer - 1, 0) : o.layer;
+          t.from = p.u;
+          t.tag = tag_of(before, op == OP_UP_GATE ? 0 : layer_of(p, before).has_mlp != 0);
+        } else if (op == OP_LRU_STEP) {
+          t.from = p.proj + l.mix_width + o.sub * l.block_dim;
+        } else if (op == OP_LATENT_ABSORB) {
+          t.from = p.proj + o.sub * l.q_stride;
+          t.length = l.q_stride;      // (with what lies behind the head's query: whoever makes it is waited for too)
+        } else if (op == OP_WKV_STEP) {
+          t.from = p.proj + 4 * l.heads * l.head_dim;
+        } else {      // OP_LATENT_VALUE: merged of parts
+          t.length = 1;
+        }
+      } else if (op == OP_STATE_STEP) {
+        t.from = p.proj + l.proj_at + 2 * l.kv_heads * l.head_dim + l.heads * l.v_dim * (delta ? 1 : 2);
+      } else if (op == OP_GATE) {
+        t.from = p.proj + l.proj_at + conv_channels(l) + l.rank;
+      } else {
+        const int first = o.layer - l.branch;
+        LayerRef& lead = layer_of(p, first);
+        const int prev = lead.prev, copy = lead.x_from;
+        int writer = first - 1;      // whose lead has left copy x_from: the last one ahead that leaves that copy
+        if (copy >= 0) {
+#pragma unroll 1
+          while (writer > 0 && (layer_of(p, writer).branch != 0 || layer_of(p, writer).x_to != copy)) --writer;
+        }
+        LayerRef& run = layer_of(p, max(prev, 0));
+        uint64_t* out = copy_of(p, prev >= 0 ? run.x_to : 0) + D;
+        const bool ff = prev >= 0 && run.has_mlp;      // (the down projection has added x to its rows)
+        t.sum[0] = ff ? out + static_cast<size_t>(QMK_HYBRID_MAX_BRANCHES) * D : copy_of(p, max(copy, 0));
+        t.sum[1] = out;
+        t.sum[2] = out + (prev >= 0 && run.branches == 2 ? D : 0);
+        t.sum_tag[0] = ff ? tag_of(prev, 1) : tag_of(writer, 0);
+        t.sum_tag[1] = tag_of(prev, 0);
+        t.sum_tag[2] = tag_of(prev + 1, 0);
+      }
+    }
+  }
+  if ((threadIdx.x & (kWaveSize - 1)) == 0) s.plan[index & 1] = t;
+}
+// The last wave plans the instruction behind this one while its first requests are on their way.
+template <bool PLAIN>
+__device__ __forceinline__ void plan_next(const DecodeParams& p, Smem& s, const Op& o) {
+  if (uniform(threadIdx.x) >= kThreads - kWaveSize) plan_of<PLAIN>(p, s, o.index + 1);
+}
+// The last norm's input has come, so everything before it has been read: every workgroup clears its share of those units, once.
+__device__ __forceinline__ void clear_units(uint64_t* at, int count, int first, int step) {
+#pragma unroll 1
+  for (int i = first; i < count; i += step) __hip_atomic_store(at + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void clear_share(const DecodeParams& p, Smem& s, int copy) {      // copy: of the plain residual, that the last norm has read
+  const int first = blockIdx.x * kThreads + threadIdx.x, step = gridDim.x * kThreads;
+  clear_units(p.units, p.early_units, first, step);
+  if (copy >= 0) clear_units(copy_of(p, 1 - copy), (2 + QMK_HYBRID_MAX_BRANCHES) * p.width, first, step);
+  if (threadIdx.x == 0) s.ctl[2] = 1;
+}
+
 // PLAIN: the kernel of a plain residual (its entries, its ops), which holds none of the other kernel's code, nor that of its.
 template <class T, bool PLAIN>
 __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op& o) {
-  LayerRef& l = layer_of(p, o.layer);
   constexpr bool plain = PLAIN;
   constexpr unsigned kOps = 1u << OP_IN_PROJECT | 1u << OP_OUT_PROJECT | 1u << OP_UP_GATE | 1u << OP_LM_HEAD |
                             (plain ? 1u << OP_STATE_STEP | 1u << OP_JOIN | 1u << OP_GATE : 1u << OP_LRU_STEP | 1u << OP_LATENT_ABSORB | 1u << OP_LATENT_VALUE | 1u << OP_WKV_STEP);
-  const int op = o.opcode, type = l.type;
+  const int op = o.opcode;
   if (!(kOps >> op & 1)) return bad_operand(p, o, o.opcode);
   __builtin_assume(kOps >> op & 1);
-  __builtin_assume(plain ? type >= QMK_MIXER_GLA : type <= QMK_MIXER_WKV);
-  Rows m;
-  if (!rows_of(p, l, o, m)) return bad_operand(p, o, o.start);
+  const Plan& plan = s.plan[o.index & 1];
+  struct {
+    const u16* w;
+    int rows, columns;
+  } const m{uniform(plan.w), static_cast<int>(uniform(plan.rows)), static_cast<int>(uniform(plan.columns))};
+  if (m.rows == 0) return bad_operand(p, o, o.start);
   const int tid = threadIdx.x, D = p.width, S = p.streams;
-  LayerRef& lead = layer_of(p, o.layer - l.branch);      // the run's first entry
+  const uint32_t tag = tag_of(o.layer, 0);     // of this entry's projections and what its mixer leaves
+  const bool normed = op == OP_IN_PROJECT || op == OP_UP_GATE || op == OP_LM_HEAD;
+  const bool reads_x = plain && (normed || op == OP_JOIN);
+  const bool down = op == OP_OUT_PROJECT && o.sub == 1;
+  const bool first = !plain && o.layer == 0 && (op == OP_IN_PROJECT || (op == OP_OUT_PROJECT && o.sub == 0));
+
+  // The first look at the vector, ahead of everything: the last workgroup of a stage finds it there, and has it normed while its rows are on their way.  (A look
+  // behind the rows' requests returns behind the rows.)
+  const uint64_t* from = uniform(plan.from);
+  const int length = uniform(plan.length);
+  const uint32_t from_tag = uniform(plan.tag);
+  Look look;
+  ResidualLook residual;
+  if (reads_x) residual.ask(p, plan);
+  else look.ask(from, tid, kThreads, length);
+  __builtin_amdgcn_sched_barrier(0);
   RowStream g;
   g.start(m.w, m.rows, m.columns);
   clear_part(s, m.rows);
+  LayerRef& l = layer_of(p, o.layer);
+  const int type = l.type;
+  __builtin_assume(plain ? type >= QMK_MIXER_GLA : type <= QMK_MIXER_WKV);
+  const int lead_at = o.layer - l.branch;      // the run's first entry
+  LayerRef& lead = layer_of(p, lead_at);
+  const bool wkv_in = !plain && op == OP_IN_PROJECT && type == QMK_MIXER_WKV;
 
-  // Asked for ahead of the wait; what the arrays hold depends on the op.  Thread r of the workgroup owns row r.
+  // Asked for ahead of the wait: what no one writes in this launch, or this workgroup alone.  Thread r of the workgroup owns row r.  (A variable of its own for
+  // everything: where values of several branches meet in one register, this compiler waits for them, and so for all rows ahead of them.)
   const int row = o.start + tid;
   const bool mine = tid < m.rows;
-  const bool normed = op == OP_IN_PROJECT || op == OP_UP_GATE || op == OP_LM_HEAD;
-  const bool wkv_in = !plain && op == OP_IN_PROJECT && type == QMK_MIXER_WKV;
-  const bool reads_x = plain && (normed || op == OP_JOIN);
-  const bool first = !plain && o.layer == 0 && (op == OP_IN_PROJECT || (op == OP_OUT_PROJECT && o.sub == 0));
   const float* norm = plain ? lead.norm1 : op == OP_IN_PROJECT ? l.norm1 : op == OP_UP_GATE ? l.norm2 : p.final_norm;
   const int channels = type == QMK_MIXER_DELTA ? conv_channels(l) : l.mix_width;
   const size_t shift_copy = type == QMK_MIXER_WKV ? static_cast<size_t>(D) : static_cast<size_t>(l.taps - 1) * channels;
   const float* shift_old = l.shift + (static_cast<size_t>(p.slot) * 2 + p.flip) * shift_copy;
   float* shift_new = l.shift + (static_cast<size_t>(p.slot) * 2 + 1 - p.flip) * shift_copy;
   const float* mu = l.vec2 + static_cast<size_t>(o.sub) * D;
-  float4 w0[kAhead], w1[kAhead], w2[kAhead];
-  float a[kMaxStreams] = {}, b[kMaxStreams] = {};
-  float out_weight = 0.f, next_weight = 0.f;
+  float norm_weight[kHeld], before[kHeld], mix_weight[kHeld];
+  // OP_IN_PROJECT: a convolution's inputs and weights, the present one's last
+  const bool convolves = op == OP_IN_PROJECT && type == (plain ? QMK_MIXER_DELTA : QMK_MIXER_RGLRU);
+  const int channel = plain ? row : row - l.mix_width;
+  const bool conv_row = convolves && mine && channel >= 0 && channel < channels;
+  float in_bias = 0.f, conv_bias = 0.f, conv_in[kFewTaps - 1], conv_weight[kFewTaps - 1], conv_now = 0.f;
+  float lru_bias, lru_rate, lru_state;
+  float wkv_state[kMaxStreams], wkv_decay, wkv_bonus, wkv_norm;
+  float step_bias;
+  float mixes[kMaxStreams], streams[kMaxStreams], out_weight, next_weight;
   float held[kStateRows];      // OP_STATE_STEP: this thread's rows of the state
   float* state = nullptr;
-  if (normed) {
-    load_ahead(w0, norm, D);
-    if (wkv_in) {
-      load_ahead(w1, shift_old, D);
-      load_ahead(w2, mu, D);
-    } else if (op == OP_IN_PROJECT && type == (plain ? QMK_MIXER_DELTA : QMK_MIXER_RGLRU) && mine) {
-      // Everything of the convolution but the current input; the kept inputs move up by one.
-      constexpr bool lru = !plain;
-      const int W = channels, c = lru ? row - W : row;
-      if (lru) a[0] = l.in_b[row];
-      if (c >= 0 && c < W) {
-        float acc = lru ? l.vec1[c] : 0.f;
-#pragma unroll 1
-        for (int j = 0; j < l.taps - 1; ++j) {
-          const float x = shift_old[static_cast<size_t>(j) * W + c];
-          acc = fmaf(l.vec2[static_cast<size_t>(j) * W + c], x, acc);
-          if (j > 0) shift_new[static_cast<size_t>(j - 1) * W + c] = x;
-        }
-        a[1] = acc;
-        a[2] = l.vec2[static_cast<size_t>(l.taps - 1) * W + c];
+  if (normed) load_ahead(norm_weight, norm, D);
+  if (wkv_in) {
+    load_ahead(before, shift_old, D);
+    load_ahead(mix_weight, mu, D);
+  }
+  if (conv_row) {
+    if constexpr (!plain) conv_bias = l.vec1[channel];
+#pragma unroll
+    for (int j = 0; j < kFewTaps - 1; ++j) {
+      if (j < l.taps - 1 && l.taps <= kFewTaps) {
+        conv_in[j] = shift_old[static_cast<size_t>(j) * channels + channel];
+        conv_weight[j] = l.vec2[static_cast<size_t>(j) * channels + channel];
       }
     }
-  } else if (!plain && op == OP_LRU_STEP) {
-    if (mine) {   // rows (r, i) of a channel: neighbouring threads
-      const int c = o.sub * l.block_dim + o.start + (tid >> 1);
-      state = l.state + static_cast<size_t>(p.slot) * l.mix_width + c;
-      a[0] = l.mid_b[2 * c + (tid & 1)];
-      a[1] = l.vec0[c];
-      a[2] = *state;
-    }
-  } else if (!plain && op == OP_WKV_STEP) {
+    conv_now = l.vec2[static_cast<size_t>(l.taps - 1) * channels + channel];
+  }
+  if (!plain && convolves && mine) in_bias = l.in_b[row];
+  if (!plain && op == OP_LRU_STEP && mine) {   // rows (r, i) of a channel: neighbouring threads
+    const int c = o.sub * l.block_dim + o.start + (tid >> 1);
+    state = l.state + static_cast<size_t>(p.slot) * l.mix_width + c;
+    lru_bias = l.mid_b[2 * c + (tid & 1)];
+    lru_rate = l.vec0[c];
+    lru_state = *state;
+  }
+  if (!plain && op == OP_WKV_STEP) {
     const int n = l.head_dim, groups = kThreads / n, e = tid % n, group = tid / n;
     state = l.state + (static_cast<size_t>(p.slot) * l.heads + o.sub) * n * n + e;
 #pragma unroll
-    for (int j = 0; j < kMaxStreams; ++j) {
-      const int i = group + j * groups;
-      if (group < groups && i < n) a[j] = state[i * n];
-    }
-    if (mine) {
-      const int at = o.sub * n + tid;
-      w0[0] = make_float4(l.mid_b[at], l.vec1[at], l.vec0[at], 0.f);
-    }
-  } else if (plain && op == OP_STATE_STEP) {
+    for (int j = 0; j < kMaxStreams; ++j) wkv_state[j] = state[min(group + j * groups, n - 1) * n];      // (rows behind the last one are not used)
+    const int at = o.sub * n + min(tid, n - 1);
+    wkv_decay = l.mid_b[at];
+    wkv_bonus = l.vec1[at];
+    wkv_norm = l.vec0[at];
+  }
+  if (plain && op == OP_STATE_STEP) {
     const int n = o.count, groups = kThreads / n, e = tid % n, group = tid / n;
     state = l.state + (static_cast<size_t>(p.slot) * l.heads + o.sub) * l.head_dim * l.v_dim + o.start + e;
 #pragma unroll
@@ -730,71 +979,74 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
 #pragma unroll
     for (int i = 0; i < 3; ++i)
       for (int at = l.head_dim + tid; at < kStateVector; at += kThreads) s.aux[i * kStateVector + at] = 0.f;
-    if (mine) a[0] = l.mid_b[o.sub * l.head_dim + tid];
-  } else if (op == OP_OUT_PROJECT && !plain) {
-    // Eight lanes per row, one per stream: all streams of the row, the stream's column of the mix, its output weight and
-    // its weight in the next sublayer's input.  The streams may be read before the wait: every output projection of a
-    // schedule deals the rows to the queues alike, so their last writer is this workgroup, and it has seen its stores
-    // acknowledged.
-    const int r = o.start + (tid >> 3), q = tid & 7;
-    if ((tid >> 3) < m.rows && q < S) {
-      const bool down = o.sub == 1;
-      const float* hc = l.hc + (down ? S * (S + 2) : 0) + S;
-      const float e = first ? bf2f(p.embed[static_cast<size_t>(token_of(p)) * D + r]) : 0.f;
+    if (mine) step_bias = l.mid_b[o.sub * l.head_dim + tid];
+  }
+  if (!plain && op == OP_OUT_PROJECT) {
+    // Eight lanes per row, one per stream: the stream's column of the mix, its output weight and its weight in the next sublayer's input.
+    const int q = min(tid & 7, S - 1);
+    const float* hc = l.hc + (down ? S * (S + 2) : 0) + S;
 #pragma unroll
-      for (int f = 0; f < kMaxStreams; ++f) {
-        if (f < S) {
-          a[f] = first ? e : ld_shared_f32(p.x + static_cast<size_t>(f) * D + r);
-          b[f] = hc[S + f * S + q];
-        }
-      }
-      out_weight = hc[q];
-      next_weight = (down ? l.next2 : l.next1)[q];
+    for (int f = 0; f < kMaxStreams; ++f) mixes[f] = hc[S + min(f, S - 1) * S + q];
+    out_weight = hc[q];
+    next_weight = (down ? l.next2 : l.next1)[q];
+    // All streams of the rows this workgroup owns: every output projection of a schedule deals the rows to the queues alike.  Their last writer is this thread's
+    // wave, which has waited for its own later requests since, or does here.
+    const int r = o.start + min(tid >> 3, m.rows - 1);
+    if (s.ctl[3] == OP_OUT_PROJECT) release_stores();
+    if (first) {
+      const float e = bf2f(p.embed[static_cast<size_t>(token_of(p)) * D + r]);
+#pragma unroll
+      for (int f = 0; f < kMaxStreams; ++f) streams[f] = e;
+    } else {
+#pragma unroll
+      for (int f = 0; f < kMaxStreams; ++f) streams[f] = ld_shared_f32(p.x + static_cast<size_t>(min(f, S - 1)) * D + r);
     }
   }
+  HeadGates gates;
+  const bool norms_heads = plain && op == OP_OUT_PROJECT && !down && type != QMK_MIXER_ATTENTION;
+  if (norms_heads) gates.ask(p, l, uniform(tid / kWaveSize));
   stamp(p, s, 0);
-  if (!wait_stage(p, s, o)) return false;
+  if constexpr (!plain) plan_next<PLAIN>(p, s, o);
+  if (!plain && op == OP_LATENT_VALUE && !wait_stage(p, s, o)) return false;
 
   // The activation vector.
-  if (plain && reads_x) {
-    residual_to_xs(p, s, lead, normed, op == OP_IN_PROJECT && o.extra, norm, w0);
+  float lru_gate, value_gate, wkv_gate, beta, unit_dot;
+  if (reads_x) {
+    residual_to_xs(p, s, o, lead, lead_at, residual, normed, op == OP_IN_PROJECT && o.extra, norm, norm_weight, [&] { g.rest(); });
   } else if (normed) {
-    norm_to_xs(p, s, norm, w0, first, l.hc);
+    norm_to_xs(p, s, o, look, from_tag, norm, norm_weight, first, l.hc, [&] { g.rest(); });
     if (wkv_in) {
-      auto mix = [&](int i, float4 before, float4 m4) {
-        const float4 h = xs_quad(s, i);
-        if (o.extra) *reinterpret_cast<float4*>(shift_new + i) = h;
-        xs_quad(s, i) = make_float4(h.x + (before.x - h.x) * m4.x, h.y + (before.y - h.y) * m4.y, h.z + (before.z - h.z) * m4.z, h.w + (before.w - h.w) * m4.w);
+      auto mix = [&](int i, float was, float weight) {
+        const float h = xs_value(s, i);
+        if (o.extra) shift_new[i] = h;
+        xs_value(s, i) = h + (was - h) * weight;
       };
 #pragma unroll
-      for (int j = 0; j < kAhead; ++j) {
-        const int i = (j * kThreads + tid) * 4;
-        if (i < D) mix(i, w1[j], w2[j]);
-      }
+      for (int j = 0; j < kHeld; ++j)
+        if (tid + j * kThreads < D) mix(tid + j * kThreads, before[j], mix_weight[j]);
 #pragma unroll 1
-      for (int i = (kAhead * kThreads + tid) * 4; i < D; i += kThreads * 4)
-        mix(i, *reinterpret_cast<const float4*>(shift_old + i), *reinterpret_cast<const float4*>(mu + i));
+      for (int i = kHeldSpan + tid; i < D; i += kThreads) mix(i, shift_old[i], mu[i]);
     }
   } else if (!plain && op == OP_LATENT_VALUE) {   // merge the parts of this head
     const int heads16 = (l.heads + 15) & ~15, parts = o.extra;
-    const float* from = p.part + static_cast<size_t>(o.sub) * l.rank;
+    const float* sums = p.part + static_cast<size_t>(o.sub) * l.rank;
     const int pitch = heads16 * l.rank;
     if (tid < parts) {
       const uint64_t ml = ld_shared64(p.ml + (static_cast<size_t>(tid) * heads16 + o.sub) * 2);
       s.aux[tid] = __uint_as_float(static_cast<uint32_t>(ml));
       s.aux[kMaxParts + tid] = __uint_as_float(static_cast<uint32_t>(ml >> 32));
     }
-    if (mine) a[0] = ld_shared_f32(p.proj + l.heads * l.q_stride + o.sub * l.v_dim + row);
     constexpr int kBatch = 16;
     static_assert(kMaxRank <= kThreads && kMaxParts <= kWaveSize, "one thread per latent element, one lane per part");
     const bool in = tid < l.rank;
     float v[kBatch];
-    const float* column = from + min(tid, l.rank - 1);
+    const float* column = sums + min(tid, l.rank - 1);
     auto request = [&](int base) {   // no branches: sixteen requests leave back to back
 #pragma unroll
       for (int j = 0; j < kBatch; ++j) v[j] = ld_shared_f32(column + min(base + j, parts - 1) * pitch);
     };
     request(0);
+    value_gate = unit_of(p, s, o, p.proj + l.heads * l.q_stride + o.sub * l.v_dim + o.start + min(tid, m.rows - 1), tag);
     __syncthreads();
     if (tid < kWaveSize) {   // weights of the parts
       const float mx = tid < parts ? s.aux[tid] : -INFINITY, top = wave_max(mx);
@@ -810,21 +1062,23 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
       for (int j = 0; j < kBatch; ++j) acc = fmaf(s.aux[base + j], v[j], acc);
     }
     if (in) s.xs[xs_at(tid)] = acc;
+    g.rest();
   } else {
-    const float* from = p.mix + (op == OP_OUT_PROJECT && o.sub == 1 ? l.ff_at : l.mix_at);
+    load_vector(p, s, o, look, from, length, from_tag, [&] { g.rest(); });
     if (plain && op == OP_STATE_STEP) {
       // query, key (unit vectors for the delta rule) and values of the head
       const bool delta = type == QMK_MIXER_DELTA;
-      const int n = l.v_dim, dim = l.head_dim, keys = l.kv_heads * dim, kv = o.sub / (l.heads / l.kv_heads);
-      const float* proj = p.proj + l.proj_at;
-      float q = 0.f, k = 0.f;
-      if (tid < dim) {
-        q = ld_shared_f32(proj + kv * dim + tid);
-        k = ld_shared_f32(proj + keys + kv * dim + tid);
-      }
-      if (tid < o.count) s.aux[3 * kStateVector + tid] = ld_shared_f32(proj + 2 * keys + o.sub * n + o.start + tid);
-      from = proj + 2 * keys + l.heads * n * (delta ? 1 : 2);
-      if (delta) a[3] = ld_shared_f32(from + l.rank + l.gate_rank + o.sub);      // beta
+      const int dim = l.head_dim, keys = l.kv_heads * dim, kv = o.sub / (l.heads / l.kv_heads), c = min(tid, dim - 1);
+      const uint64_t *proj = p.proj + l.proj_at, *steps = delta ? from + l.rank + l.gate_rank : proj;      // (all step sizes: whoever makes those of padding is waited for too)
+      Gather<5> more{{proj + kv * dim + c, proj + keys + kv * dim + c, proj + 2 * keys + o.sub * l.v_dim + o.start + min(tid, o.count - 1), steps + (delta ? o.sub : 0),
+                      steps + (delta ? min(tid, (l.heads + 15) / 16 * 16 - 1) : 0)}};
+      more.ask();
+      more.wait(p, s, o, tag);
+      float q = more[0], k = more[1];
+      const float v = more[2];
+      beta = more[3];
+      if (tid >= dim) q = k = 0.f;
+      if (tid < o.count) s.aux[3 * kStateVector + tid] = v;
       if (!delta) q *= l.q_scale;                       // (the projection is left unscaled)
       float dots[3] = {q * q, k * k, q * k};
       block_sum3(dots, s.scratch);
@@ -834,34 +1088,32 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
         k *= ik;
         dots[2] *= iq * ik;
       }
-      a[4] = dots[2];
+      unit_dot = dots[2];
       if (tid < dim) {
         s.aux[tid] = q;
         s.aux[kStateVector + tid] = k;
       }
-    } else if (plain && op == OP_GATE) {
-      from = p.proj + l.proj_at + conv_channels(l) + l.rank;
     } else if (!plain && op == OP_LRU_STEP) {
-      if (mine && !(tid & 1)) a[3] = ld_shared_f32(p.proj + o.sub * l.block_dim + o.start + (tid >> 1));
-      from = p.proj + l.mix_width + o.sub * l.block_dim;
-    } else if (!plain && op == OP_LATENT_ABSORB) {
-      from = p.proj + o.sub * l.q_stride;
+      lru_gate = unit_of(p, s, o, p.proj + o.sub * l.block_dim + o.start + (min(tid, m.rows - 1) >> 1), tag);
     } else if (!plain && op == OP_WKV_STEP) {
-      const int n = l.head_dim, N = l.heads * n, at = o.sub * n + tid;
+      const int n = l.head_dim, N = l.heads * n;
+      const uint64_t* at = p.proj + o.sub * n + min(tid, n - 1);
+      Gather<4> more{{at, at + N, at + 2 * N, at + 3 * N}};
+      more.ask();
+      more.wait(p, s, o, tag);
+      wkv_gate = more[3];
       if (mine) {
-        const float r = ld_shared_f32(p.proj + at), k = ld_shared_f32(p.proj + N + at), v = ld_shared_f32(p.proj + 2 * N + at);
-        w0[0].w = ld_shared_f32(p.proj + 3 * N + at);
-        s.aux[tid] = r;
-        s.aux[kMaxHeadDim + tid] = k;
-        s.aux[2 * kMaxHeadDim + tid] = v;
-        s.aux[4 * kMaxHeadDim + tid] = w0[0].y;
+        s.aux[tid] = more[0];
+        s.aux[kMaxHeadDim + tid] = more[1];
+        s.aux[2 * kMaxHeadDim + tid] = more[2];
+        s.aux[4 * kMaxHeadDim + tid] = wkv_bonus;
       }
-      from = p.proj + 4 * N;
     }
-    load_vector(s, from, m.columns);
-    if (plain && op == OP_OUT_PROJECT && o.sub == 0 && l.type != QMK_MIXER_ATTENTION) norm_heads(p, s, l);
+    if (norms_heads) norm_heads(p, s, o, l, gates);
   }
+  if (p.timeline != nullptr && tid == 0) s.t_wait = wall_clock64();
   __syncthreads();
+  if (s.ctl[0] == 0) return false;
   stamp(p, s, 1);
   g.run(s);
   __syncthreads();
@@ -871,35 +1123,56 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
   float t = mine && (plain || op != OP_OUT_PROJECT) ? row_total(s, tid) : 0.f;
   static_assert(kMaxRows <= kThreads && kMaxStreams == 8, "one row per thread, eight values ahead");
   if (plain && op == OP_JOIN) {
-    if (mine) st_shared_f32(p.x + static_cast<size_t>(l.x_to) * D + row, t);
+    if (mine) put_unit(copy_of(p, l.x_to) + row, t, tag);
   } else if (op == OP_OUT_PROJECT && plain) {
-    if (mine) st_shared_f32(p.out + static_cast<size_t>(o.sub == 1 ? QMK_HYBRID_MAX_BRANCHES : l.branch) * D + row, t);
+    // (The feed-forward's rows with the residual that the run has read: its next reader looks at one vector less.)
+    if (down) t += unit_of(p, s, o, copy_of(p, lead.x_to) + o.start + min(tid, m.rows - 1), tag_of(lead_at, 0));
+    if (mine) put_unit(copy_of(p, lead.x_to) + static_cast<size_t>(1 + (down ? QMK_HYBRID_MAX_BRANCHES : l.branch)) * D + row, t, from_tag);
   } else if (op == OP_OUT_PROJECT) {
     const int r = tid >> 3, q = tid & 7;
     if (r < m.rows) {      // whole groups of eight lanes
       float now = out_weight * row_total(s, r);
 #pragma unroll
-      for (int f = 0; f < kMaxStreams; ++f) now = fmaf(b[f], a[f], now);
-      const float u = group8_sum(next_weight * now);
-      if (q == 0) st_shared_f32(p.u + o.start + r, u);
+      for (int f = 0; f < kMaxStreams; ++f)
+        if (f < S) now = fmaf(mixes[f], streams[f], now);
+      const float u = group8_sum(q < S ? next_weight * now : 0.f);
+      if (q == 0) put_unit(p.u + o.start + r, u, from_tag);
       if (q < S) st_shared_f32(p.x + static_cast<size_t>(q) * D + o.start + r, now);
     }
   } else if (op == OP_UP_GATE) {
     const float up = dpp_f32<kDppQuadXor1>(0.f, t);
-    if (mine && !(tid & 1)) st_shared_f32(p.mix + l.ff_at + o.start + (tid >> 1), (l.act == QMK_ACT_SILU ? t * sigmoid(t) : gelu_tanh(t)) * up);
+    if (mine && !(tid & 1)) put_unit(p.mix + l.ff_at + o.start + (tid >> 1), (l.act == QMK_ACT_SILU ? t * sigmoid(t) : gelu_tanh(t)) * up, tag_of(o.layer, 1));
   } else if (op == OP_IN_PROJECT) {
     const float pair = dpp_f32<kDppQuadXor1>(0.f, t);
     if (mine) {
       const int W = l.mix_width;
       int gate = 0;          // 1: sigmoid, 2: times sigmoid (silu), 3: gelu
-      if (!plain && type == QMK_MIXER_RGLRU) {
-        t += a[0];
-        if (row < W) {
-          gate = 3;
+      // Everything of the convolution but the current input; the kept inputs move up by one.
+      auto convolved = [&](float bias) {
+        float acc = bias;
+        if (l.taps <= kFewTaps) {
+#pragma unroll
+          for (int j = 0; j < kFewTaps - 1; ++j) {
+            if (j < l.taps - 1) {
+              acc = fmaf(conv_weight[j], conv_in[j], acc);
+              if (j > 0) shift_new[static_cast<size_t>(j - 1) * channels + channel] = conv_in[j];
+            }
+          }
         } else {
-          if (l.taps > 1) shift_new[static_cast<size_t>(l.taps - 2) * W + row - W] = t;
-          t = fmaf(a[2], t, a[1]);
+#pragma unroll 1
+          for (int j = 0; j < l.taps - 1; ++j) {
+            const float x = shift_old[static_cast<size_t>(j) * channels + channel];
+            acc = fmaf(l.vec2[static_cast<size_t>(j) * channels + channel], x, acc);
+            if (j > 0) shift_new[static_cast<size_t>(j - 1) * channels + channel] = x;
+          }
         }
+        if (l.taps > 1) shift_new[static_cast<size_t>(l.taps - 2) * channels + channel] = t;
+        return fmaf(conv_now, t, acc);
+      };
+      if (!plain && type == QMK_MIXER_RGLRU) {
+        t += in_bias;
+        if (row < W) gate = 3;
+        else t = convolved(conv_bias);
       } else if (!plain && type == QMK_MIXER_LATENT) {
         const int q_rows = l.heads * l.q_stride, g_rows = l.heads * l.v_dim;
         int d = -1;
@@ -922,8 +1195,7 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
         if (row >= q_rows + k_rows + v_rows) gate = 1;
       } else if (plain && type == QMK_MIXER_DELTA) {
         if (row < channels) {
-          if (l.taps > 1) shift_new[static_cast<size_t>(l.taps - 2) * channels + row] = t;
-          t = fmaf(a[2], t, a[1]);
+          t = convolved(0.f);
           gate = 2;
         } else if (row >= channels + l.rank + l.gate_rank) {
           gate = 1;
@@ -941,48 +1213,32 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
         const float sg = sigmoid(z);
         t = gate == 1 ? sg : t * sg;
       }
-      st_shared_f32(p.proj + l.proj_at + row, t);
+      put_unit(p.proj + l.proj_at + row, t, tag);
     }
   } else if (!plain && op == OP_LRU_STEP) {
-    const float gate = sigmoid(t + a[0]), in_gate = dpp_f32<kDppQuadXor1>(0.f, gate);
+    const float gate = sigmoid(t + lru_bias), in_gate = dpp_f32<kDppQuadXor1>(0.f, gate);
     if (mine && !(tid & 1)) {
       const int c = o.start + (tid >> 1);
-      const float log_a = gate * a[1];
+      const float log_a = gate * lru_rate;
       const float b = sqrtf(-expm1f(2.f * log_a)) * in_gate * s.xs[xs_at(c)];
-      const float now = fmaf(expf(log_a), a[2], b);
+      const float now = fmaf(expf(log_a), lru_state, b);
       *state = now;
-      st_shared_f32(p.mix + o.sub * l.block_dim + c, now * a[3]);
+      put_unit(p.mix + o.sub * l.block_dim + c, now * lru_gate, tag);
     }
   } else if (!plain && op == OP_LATENT_VALUE) {
-    if (mine) st_shared_f32(p.mix + o.sub * l.v_dim + row, t * a[0]);
+    if (mine) put_unit(p.mix + o.sub * l.v_dim + row, t * value_gate, tag);
   } else if (!plain && op == OP_LATENT_ABSORB) {
-    if (mine) st_shared_f32(p.absorbed + o.sub * l.rank + row, t);
-    if (o.extra) {   // the step's cache row: normed latent, rotated key part
-      const float* c = p.proj + l.heads * (l.q_stride + l.v_dim);
-      const int width = l.rank + l.rot_dim;
-      static_assert(kMaxRank <= kThreads, "one latent element per thread");
-      const float v = tid < l.rank ? ld_shared_f32(c + tid) : 0.f;
-      const float inv = 1.f / sqrtf(block_sum(v * v, s.scratch) / l.rank_true + p.eps);
-      T* to = cache_row<T>(p, l, p.position);
-      auto put = [&](int i, float e) {   // a pair of elements is a pair of lanes
-        const float odd = dpp_f32<kDppQuadXor1>(0.f, e);
-        if constexpr (sizeof(T) == 2) {
-          if (i < width && !(i & 1)) st_shared32(to + i, f2bf2(e, odd));
-        } else {
-          if (i < width) st_shared_f32(to + i, e);
-        }
-      };
-      put(tid < l.rank ? tid : width, tid < l.rank ? v * inv * l.vec0[tid] : 0.f);
-#pragma unroll 1
-      for (int base = 0; base < l.rot_dim; base += kThreads) {
-        const int i = base + tid;
-        put(i < l.rot_dim ? l.rank + i : width, i < l.rot_dim ? ld_shared_f32(c + l.rank + i) : 0.f);
-      }
+    // What the attention's matrix tiles hold of it: in bf16 mode two rounded values a unit.
+    if constexpr (sizeof(T) == 2) {
+      const float odd = dpp_f32<kDppQuadXor1>(0.f, t);
+      if (mine && !(tid & 1)) put_bits(p.absorbed + (o.sub * l.rank + row) / 2, f2bf2(t, odd), tag);
+    } else {
+      if (mine) put_unit(p.absorbed + o.sub * l.rank + row, t, tag);
     }
   } else if (!plain && op == OP_WKV_STEP) {
     const int n = l.head_dim, groups = kThreads / n, e = tid % n, group = tid / n;
     const float *r = s.aux, *k = r + kMaxHeadDim, *v = k + kMaxHeadDim, *w = v + kMaxHeadDim, *u = w + kMaxHeadDim;
-    if (mine) s.aux[3 * kMaxHeadDim + tid] = expf(-expf(t + w0[0].x));
+    if (mine) s.aux[3 * kMaxHeadDim + tid] = expf(-expf(t + wkv_decay));
     __syncthreads();
     if (group < groups) {
       float acc = 0.f;
@@ -993,7 +1249,7 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
       };
 #pragma unroll
       for (int j = 0; j < kMaxStreams; ++j)
-        if (group + j * groups < n) key_row(group + j * groups, a[j]);
+        if (group + j * groups < n) key_row(group + j * groups, wkv_state[j]);
 #pragma unroll 1
       for (int i = group + kMaxStreams * groups; i < n; i += groups) key_row(i, state[i * n]);
       s.xs[group * n + e] = acc;
@@ -1006,14 +1262,14 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
     }
     const float sq = block_sum(val * val, s.scratch);   // storage columns behind the true head size hold zeros
     const float inv = 1.f / sqrtf(sq / l.head_dim_true + p.eps);
-    if (mine) st_shared_f32(p.mix + o.sub * n + tid, val * inv * w0[0].z * w0[0].w);
+    if (mine) put_unit(p.mix + o.sub * n + tid, val * inv * wkv_norm * wkv_gate, tag);
   } else if (plain && op == OP_STATE_STEP) {
     // S <- decay S, u = beta (v - S^T k), S <- S + k u^T, o = S^T q, with S^T k and S^T q taken together:
     // o = (decay S)^T q + (q . k) u.  Without the delta rule u = v.
     const bool delta = type == QMK_MIXER_DELTA;
     const int n = o.count, dim = l.head_dim, groups = kThreads / n, e = tid % n, group = tid / n;
     float *q = s.aux, *k = q + kStateVector, *w = k + kStateVector, *v = w + kStateVector;
-    if (mine) w[tid] = delta ? delta_decay(l, o.sub, t + a[0]) : gla_decay(l, t + a[0]);
+    if (mine) w[tid] = delta ? delta_decay(l, o.sub, t + step_bias) : gla_decay(l, t + step_bias);
     __syncthreads();
     float ak = 0.f, aq = 0.f;
 #pragma unroll
@@ -1039,10 +1295,10 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
       ak += s.xs[i * n + e];
       aq += s.xs[(groups + i) * n + e];
     }
-    const float u = delta ? a[3] * (v[e] - ak) : v[e];
-    if (tid < n) st_shared_f32(p.mix + l.mix_at + o.sub * l.v_dim + o.start + tid, fmaf(a[4], u, aq));
+    const float u = delta ? beta * (v[e] - ak) : v[e];
+    if (tid < n) put_unit(p.mix + l.mix_at + o.sub * l.v_dim + o.start + tid, fmaf(unit_dot, u, aq), tag);
     stamp(p, s, 3);
-    arrive_stage(p, o);      // nobody else reads the state in this launch: its stores need no acknowledgement before the arrival
+    arrive_stage(p, o);      // (counted with the attention's parts of its stage, whose readers read nothing of it)
     if (group < groups) {
 #pragma unroll
       for (int j0 = 0; j0 < kStateRows; j0 += kStateBatch) {
@@ -1058,10 +1314,12 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
     }
     return true;
   } else if (plain && op == OP_GATE) {
-    if (mine) st_shared_f32(p.proj + l.proj_at + l.in_rows + row, sigmoid(t));
+    if (mine) put_unit(p.proj + l.proj_at + l.in_rows + row, sigmoid(t), tag);
+    arrive_stage(p, o);
   } else {   // OP_LM_HEAD
     if (plain) t = soft_cap(t * p.logit_scale, p.logit_softcap);
     if (mine) p.logits[row] = t;
+    clear_share(p, s, plain ? l.x_from : -1);
     const bool real = mine && row < p.vocab;
     const float top = block_max(real ? t : -INFINITY, s.scratch);
     int where = wave_min_i32(real && t == top ? row : 0x7fffffff);   // smallest row among equals
@@ -1078,7 +1336,6 @@ __device__ __forceinline__ bool op_rows(const DecodeParams& p, Smem& s, const Op
     }
   }
   stamp(p, s, 3);
-  arrive_stage(p, o);
   return true;
 }
 
@@ -1144,6 +1401,7 @@ __device__ __forceinline__ bool op_attend(const DecodeParams& p, Smem& s, const 
   constexpr int kUnit = 16 / sizeof(T);
   LayerRef& l = layer_of(p, o.layer);
   const int heads16 = (l.heads + 15) & ~15;
+  const uint32_t tag = tag_of(o.layer, 0);
   constexpr bool latent = !PLAIN;
   if (l.type != (latent ? QMK_MIXER_LATENT : QMK_MIXER_ATTENTION) || o.sub < 0 || o.start < 0 || o.count <= 0 || o.count > p.max_splits || o.start >= o.count || o.extra < 0)
     return bad_operand(p, o, o.start);
@@ -1169,39 +1427,43 @@ __device__ __forceinline__ bool op_attend(const DecodeParams& p, Smem& s, const 
   T* cache = static_cast<T*>(l.cache) + kv * width;
   // Rows base .. base + kKeys - 1 -> sc, but for the row another workgroup of this launch appends.  (A part is never
   // longer than the ring, so a position wraps at most once.)
+  const uint32_t per_unit = 0xffffffffu / units + 1u;      // exact: units of a tile times units of a row stay far below 2^32
   auto load_tile = [&](int base) {
-    constexpr int kBatch = 4;
-    const int at0 = base % rows;
+    constexpr int kBatch = 9;      // 64 rows of 576 bf16: all requests at once
+    const int at0 = base % rows, count = kKeys * units;
 #pragma unroll 1
-    for (int r0 = wave; r0 < kKeys; r0 += kBatch * kWaves) {
-#pragma unroll 1
-      for (int c = lane; c < units; c += kWaveSize) {
-        v4u v[kBatch];
+    for (int first = tid; first < count; first += kBatch * kThreads) {
+      v4u v[kBatch];
 #pragma unroll
-        for (int j = 0; j < kBatch; ++j) {
-          const int r = r0 + j * kWaves, at = at0 + r >= rows ? at0 + r - rows : at0 + r;
-          v[j] = v4u{0u, 0u, 0u, 0u};
-          if (base + r < hi && base + r != p.position && c * kUnit < width)
-            v[j] = *reinterpret_cast<const v4u*>(cache + static_cast<size_t>(offset + at) * pitch + c * kUnit);
-        }
+      for (int j = 0; j < kBatch; ++j) {
+        const int id = first + j * kThreads, r = __umulhi(id, per_unit), c = id - r * units, at = at0 + r >= rows ? at0 + r - rows : at0 + r;
+        v[j] = v4u{0u, 0u, 0u, 0u};
+        if (id < count && base + r < hi && base + r != p.position && c * kUnit < width)
+          v[j] = *reinterpret_cast<const v4u*>(cache + static_cast<size_t>(offset + at) * pitch + c * kUnit);
+      }
 #pragma unroll
-        for (int j = 0; j < kBatch; ++j) *reinterpret_cast<v4u*>(sc + (r0 + j * kWaves) * stride + c * kUnit) = v[j];
+      for (int j = 0; j < kBatch; ++j) {
+        const int id = first + j * kThreads, r = __umulhi(id, per_unit), c = id - r * units;
+        if (id < count) *reinterpret_cast<v4u*>(sc + r * stride + c * kUnit) = v[j];
       }
     }
   };
   // The appended row, where this part holds it (it is then the part's last).
   auto load_appended = [&](int base) {
     if (p.position >= hi || p.position < base || p.position >= base + kKeys) return;
-    T* row = cache + static_cast<size_t>(offset + p.position % rows) * pitch;
     if (!latent) {   // neighbouring elements, both of the key or both of the value
-      const float* from = p.proj + l.proj_at + l.heads * l.q_stride;
+      const uint64_t* from = p.proj + l.proj_at + l.heads * l.q_stride;
       const bool put = block == 0 && o.extra == 0;
+      T* row = cache + static_cast<size_t>(offset + p.position % rows) * pitch;
 #pragma unroll 1
       for (int c = tid * 2; c < width; c += kThreads * 2) {
-        const uint64_t v = ld_shared64(from + (c < l.head_dim ? kv * l.head_dim + c : l.kv_heads * l.head_dim + kv * l.v_dim + c - l.head_dim));
+        const uint64_t* pair = from + (c < l.head_dim ? kv * l.head_dim + c : l.kv_heads * l.head_dim + kv * l.v_dim + c - l.head_dim);
+        Units<2> v;
+        v.ask(pair, 0, 1, 2);
+        v.wait(p, s, o, pair, 0, 1, 2, tag);
         T* at = sc + (p.position - base) * stride + c;
-        at[0] = from_f32<T>(__uint_as_float(static_cast<uint32_t>(v)));
-        at[1] = from_f32<T>(__uint_as_float(static_cast<uint32_t>(v >> 32)));
+        at[0] = from_f32<T>(v[0]);
+        at[1] = from_f32<T>(v[1]);
         if (put) {
           row[c] = at[0];
           row[c + 1] = at[1];
@@ -1209,30 +1471,83 @@ __device__ __forceinline__ bool op_attend(const DecodeParams& p, Smem& s, const 
       }
       return;
     }
+    // Normed latent, rotated key part: every workgroup that needs the row makes it, which takes no longer than to fetch it.
+    const uint64_t* from = p.proj + l.heads * (l.q_stride + l.v_dim);
+    T *to = sc + (p.position - base) * stride, *row = cache + static_cast<size_t>(offset + p.position % rows) * pitch;
+    const bool put = o.sub == 0 && o.extra == 0;
+    static_assert(kMaxRank <= kThreads, "one latent element per thread");
+    const float v = unit_of(p, s, o, from + min(tid, l.rank - 1), tag);
+    const float inv = 1.f / sqrtf(block_sum(tid < l.rank ? v * v : 0.f, s.scratch) / l.rank_true + p.eps);
+    auto leave = [&](int i, float e) {
+      to[i] = from_f32<T>(e);
+      if (put) row[i] = to[i];
+    };
+    if (tid < l.rank) leave(tid, v * inv * l.vec0[tid]);
 #pragma unroll 1
-    for (int c = tid; c * kUnit < width; c += kThreads) *reinterpret_cast<v4u*>(sc + (p.position - base) * stride + c * kUnit) = ld_shared128(row + c * kUnit);
+    for (int i = tid; i < l.rot_dim; i += kThreads) leave(l.rank + i, unit_of(p, s, o, from + l.rank + i, tag));
   };
-  if (lo < hi) load_tile(lo);
-  stamp(p, s, 0);
-  if (!wait_stage(p, s, o)) return false;
-  if (lo < hi) {
-#pragma unroll 1
-    for (int k = tid * 2; k < width32; k += kThreads * 2) {
-      uint64_t v[16];
-      const float* from = !latent ? p.proj + l.proj_at + head0 * l.q_stride + k
-                          : k < l.rank ? p.absorbed + head0 * l.rank + k : p.proj + head0 * l.q_stride + l.head_dim + k - l.rank;
-      const int step = latent && k < l.rank ? l.rank : l.q_stride, end = latent ? width : l.q_stride;
+  // Queries of the sixteen heads: units of the absorbed ones (in bf16 mode pairs) and of the projections, as they lie side by side, dealt to the threads; the first
+  // look ahead of the keys.
+  constexpr int kPair = latent && sizeof(T) == 2 ? 2 : 1, kQueries = 8;
+  const int per_a = latent ? l.rank / kPair : 0, per_b = latent ? l.rot_dim : l.q_stride, count_a = heads * per_a, count_b = heads * per_b;
+  const uint32_t inverse_a = 0xffffffffu / max(per_a, 1) + 1u, inverse_b = 0xffffffffu / per_b + 1u;
+  Gather<latent ? kQueries : 1> queries;
+  Gather<latent ? 2 : kQueries> rest;
+  int asked = 0;
+  auto ask_queries = [&](int base) {
+    asked = base;
 #pragma unroll
-      for (int h = 0; h < 16; ++h) v[h] = h < heads && k < end ? ld_shared64(from + h * step) : 0;
+    for (int j = 0; j < (latent ? kQueries : 1); ++j) queries.at[j] = latent ? p.absorbed + head0 * per_a + min(base + tid + j * kThreads, count_a - 1) : p.proj + l.proj_at + head0 * per_b;
 #pragma unroll
-      for (int h = 0; h < 16; ++h) {
-        sq[h * stride + k] = from_f32<T>(__uint_as_float(static_cast<uint32_t>(v[h])));
-        sq[h * stride + k + 1] = from_f32<T>(__uint_as_float(static_cast<uint32_t>(v[h] >> 32)));
+    for (int j = 0; j < (latent ? 2 : kQueries); ++j) {
+      const int id = min((latent ? base / (kQueries / 2) : base) + tid + j * kThreads, count_b - 1), h = __umulhi(id, inverse_b), c = id - h * per_b;
+      rest.at[j] = latent ? p.proj + (head0 + h) * l.q_stride + l.head_dim + c : p.proj + l.proj_at + head0 * l.q_stride + id;
+    }
+    queries.ask();
+    rest.ask();
+  };
+  auto put_queries = [&] {
+    if constexpr (latent) {
+#pragma unroll
+      for (int j = 0; j < kQueries; ++j) {
+        const int id = asked + tid + j * kThreads, h = __umulhi(id, inverse_a), c = id - h * per_a;
+        if (id >= count_a) continue;
+        if constexpr (kPair == 2) reinterpret_cast<uint32_t*>(sq + h * stride)[c] = static_cast<uint32_t>(queries.r[j]);
+        else sq[h * stride + c] = from_f32<T>(queries[j]);
       }
     }
+#pragma unroll
+    for (int j = 0; j < (latent ? 2 : kQueries); ++j) {
+      const int id = (latent ? asked / (kQueries / 2) : asked) + tid + j * kThreads, h = __umulhi(id, inverse_b), c = id - h * per_b;
+      if (id < count_b) sq[h * stride + (latent ? l.rank : 0) + c] = from_f32<T>(rest[j]);
+    }
+  };
+  if (lo < hi) {
+    ask_queries(0);
+    // Heads and columns that are not there.
+    const int end = latent ? width : l.q_stride;
+#pragma unroll 1
+    for (int h = wave; h < 16; h += kWaves)
+      for (int c = (h < heads ? end : 0) + lane; c < (latent ? width32 : end); c += kWaveSize) sq[h * stride + c] = from_f32<T>(0.f);
+    load_tile(lo);
     __syncthreads();     // the tile's row that load_appended fills has been zeroed
     load_appended(lo);
   }
+  stamp(p, s, 0);
+  if constexpr (latent) plan_next<PLAIN>(p, s, o);
+  if (lo < hi) {
+    queries.wait(p, s, o, tag);
+    rest.wait(p, s, o, tag);
+    put_queries();
+#pragma unroll 1
+    for (int base = kQueries * kThreads; base < max(count_a, count_b * (latent ? kQueries / 2 : 1)); base += kQueries * kThreads) {
+      ask_queries(base);
+      queries.wait(p, s, o, tag);
+      rest.wait(p, s, o, tag);
+      put_queries();
+    }
+  }
+  if (p.timeline != nullptr && tid == 0) s.t_wait = wall_clock64();
 
   stamp(p, s, 1);
   const int head = tid & 15, key0 = tid >> 4;      // this thread's scores: keys key0, key0 + 32, ...
@@ -1325,6 +1640,9 @@ __device__ __forceinline__ bool op_attend(const DecodeParams& p, Smem& s, const 
                          __HIP_MEMORY_SCOPE_AGENT);
   }
   stamp(p, s, 3);
+  release_stores();
+  __syncthreads();
+  if (s.ctl[0] == 0) return false;
   arrive_stage(p, o);
   return true;
 }
@@ -1341,7 +1659,6 @@ __device__ __forceinline__ bool op_attend_merge(const DecodeParams& p, Smem& s, 
     s.aux[tid] = __uint_as_float(static_cast<uint32_t>(ml));
     s.aux[kMaxParts + tid] = __uint_as_float(static_cast<uint32_t>(ml >> 32));
   }
-  const float gate = tid < n ? ld_shared_f32(p.proj + l.proj_at + l.heads * l.q_stride + l.kv_heads * (l.head_dim + n) + o.sub * n + tid) : 0.f;
   constexpr int kBatch = 8;
   float v[kBatch];
   const float* column = p.part + static_cast<size_t>(o.sub) * n + e;
@@ -1350,6 +1667,7 @@ __device__ __forceinline__ bool op_attend_merge(const DecodeParams& p, Smem& s, 
     for (int j = 0; j < kBatch; ++j) v[j] = ld_shared_f32(column + static_cast<size_t>(min(base + j * groups, parts - 1)) * heads16 * n);
   };
   request(group);
+  const float gate = unit_of(p, s, o, p.proj + l.proj_at + l.heads * l.q_stride + l.kv_heads * (l.head_dim + n) + o.sub * n + min(tid, n - 1), tag_of(o.layer, 0));
   __syncthreads();
   if (tid < kWaveSize) {   // weights of the parts
     const float mx = tid < parts ? s.aux[tid] : -INFINITY, top = wave_max(mx);
@@ -1373,10 +1691,9 @@ __device__ __forceinline__ bool op_attend_merge(const DecodeParams& p, Smem& s, 
     acc = 0.f;
 #pragma unroll 4
     for (int i = 0; i < groups; ++i) acc += s.xs[i * n + tid];
-    st_shared_f32(p.mix + l.mix_at + o.sub * n + tid, acc * gate);
+    put_unit(p.mix + l.mix_at + o.sub * n + tid, acc * gate, tag_of(o.layer, 0));
   }
-  arrive_stage(p, o);
-  return true;
+  return s.ctl[0] != 0;
 }
 
 }  // namespace hybrid

@@ -5,9 +5,10 @@ g, decay), the gate block, the head, the group of at most sixteen heads (of one 
 0 / 1 for the output / down projection; ``start`` and ``count`` are output rows (pairs of rows for opcodes 2 and 8, part
 number and number of parts for opcode 4).
 
-A step is a chain of stages.  An instruction waits until ``wait_count`` arrivals are counted on ``wait_stage`` (-1: none)
-and counts one arrival on ``arrive_stage``; the schedule's stages are all-to-all, so ``wait_count`` is the number of
-instructions of the stage before.  Stage s is counted in group ``s // 4`` of ``barriers`` on counter row ``2 + s % 4`` of
+A step is a chain of stages; ``wait_stage`` (-1: none) is the one an instruction depends on, ``wait_count`` the number of its
+instructions, ``arrive_stage`` its own.  The kernel hands values over as tagged units, which carry the order themselves; only
+the parts of an attention, and what shares their stage, count an arrival each, for which the opcodes that merge them wait.
+Stage s is counted in group ``s // 4`` of ``barriers`` on counter row ``2 + s % 4`` of
 the dense route's layout, one line per XCD.
 """
 from __future__ import annotations
@@ -49,13 +50,15 @@ class GatedRecurrence(StageInstruction):
 
 @dataclass
 class LatentAbsorb(StageInstruction):
-    """``extra`` = 1: also norms the latent and appends the cache row."""
+    """``extra`` = 1: the stage's leading instruction (which no longer does more than the others: the attention's parts that
+    hold the step's position make and append the cache row)."""
     OPCODE: ClassVar[int] = 3
 
 
 @dataclass
 class AttendSplitKV(StageInstruction):
-    """Over latents or over keys and values.  ``extra``: which 128 columns of the latent or value."""
+    """Over latents or over keys and values.  ``extra``: which 128 columns of the latent or value.  The parts that hold the
+    step's position work its cache row out of the projections, and one of them appends it."""
     OPCODE: ClassVar[int] = 4
 
 
