@@ -55,8 +55,8 @@ def run_tokens(globs: Globals, mk: Any, request: Request, tokens: Sequence[int] 
         if n == 1:
             globs.token.copy_(part)
             _mk_kernel.call_mk(globs, mk)
-            if rows:
-                out[rows] = globs.logits[:vocab]
+            for k in rows:
+                out[k] = globs.logits[:vocab]
         else:
             places = sorted({want[k] - start for k in rows})
             logits = mk.prefill(globs, part.contiguous(), torch.tensor(places, dtype=torch.int32, device=globs.device) if places else None)
