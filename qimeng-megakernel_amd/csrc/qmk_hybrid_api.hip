@@ -12,6 +12,7 @@
 #include "qmk_hybrid_ops.h"
 #include "qmk_hybrid_prefill.h"
 #include "qmk_hybrid_plain.h"
+#include "qmk_hybrid_chunks.h"
 
 namespace qmk {
 namespace hybrid {
@@ -366,17 +367,37 @@ struct OperandRows {
   Operand<T> of(int columns) const { return Operand<T>{at, sizeof(T) == 4 && columns > 64 && columns % 64 == 0 ? count : 0}; }
 };
 
+// What the recurrences of portions keep between their launches: as large as the largest of its layers needs.
+struct ChunkBuffers {
+  float *chunks = nullptr, *starts = nullptr, *fades = nullptr;
+  size_t chunk_count = 0, start_count = 0, fade_count = 0;
+  void fit(size_t tokens, size_t heads, size_t dim, size_t n, bool segments) {
+    chunk_count = std::max(chunk_count, chunks_of(static_cast<int>(tokens)) * heads * chunk_floats(static_cast<int>(dim)));
+    if (!segments) return;
+    const size_t most = segments_of(static_cast<int>(tokens), kSegmentChunks);
+    start_count = std::max(start_count, most * heads * dim * n);
+    fade_count = std::max(fade_count, most * heads * dim);
+  }
+  void take(Carver& c) {
+    chunks = c.take<float>(chunk_count);
+    starts = c.take<float>(start_count);
+    fades = c.take<float>(fade_count);
+  }
+};
+
 template <class T>
 struct PlainBuffers {
   SplitBuffers split;
-  float *x, *branch, *qkv, *values, *decay, *beta, *o, *chunks;
+  float *x, *branch, *qkv, *values, *decay, *beta, *o;
+  ChunkBuffers state;
   T *q, *low, *gate, *vt;
   OperandRows<T> h, mix;
 };
 template <class T>
 size_t plain_buffers(const QmkHybridArgs* a, void* base, PlainBuffers<T>* b) {
-  const size_t P = a->portion_rows, D = a->width, chunks_of = (P + kChunkTokens - 1) / kChunkTokens;
-  size_t h = P * D, branch = 0, qkv = 0, values = 0, decay = 0, beta = 0, o = 0, chunks = 0, q = 0, low = 0, gate = 0, mix = 0, vt = 0;
+  const size_t P = a->portion_rows, D = a->width;
+  ChunkBuffers state;
+  size_t h = P * D, branch = 0, qkv = 0, values = 0, decay = 0, beta = 0, o = 0, q = 0, low = 0, gate = 0, mix = 0, vt = 0;
   for (int i = 0; i < a->num_layers; ++i) {
     const QmkHybridLayer& l = a->layers[i];
     if (l.type == QMK_ENTRY_JOIN) h = std::max(h, 2 * P * D);
@@ -392,7 +413,7 @@ size_t plain_buffers(const QmkHybridArgs* a, void* base, PlainBuffers<T>* b) {
     decay = std::max(decay, P * l.heads * l.head_dim);
     o = std::max(o, P * l.mix_width);
     low = std::max(low, P * (l.rank + l.gate_rank));
-    chunks = std::max(chunks, chunks_of * l.heads * chunk_floats(l.head_dim));
+    state.fit(P, l.heads, l.head_dim, l.v_dim, l.type == QMK_MIXER_GLA);
     if (l.type == QMK_MIXER_DELTA) {
       qkv = std::max(qkv, P * conv_channels(l));
       values = std::max(values, P * l.mix_width);
@@ -412,7 +433,8 @@ size_t plain_buffers(const QmkHybridArgs* a, void* base, PlainBuffers<T>* b) {
   b->decay = c.take<float>(decay);
   b->beta = c.take<float>(beta);
   b->o = c.take<float>(o);
-  b->chunks = c.take<float>(chunks);
+  state.take(c);
+  b->state = state;
   b->h = OperandRows<T>(c, h);
   b->q = c.take<T>(q);
   b->low = c.take<T>(low);
@@ -428,6 +450,7 @@ template <class T>
 struct PrefillBuffers {
   SplitBuffers split;
   float *x, *u, *fa, *fb, *raw;
+  ChunkBuffers state;
   T *p0, *p1, *p2, *rows, *kn, *vt;
   OperandRows<T> h, mix;
 };
@@ -435,6 +458,7 @@ template <class T>
 size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b) {
   if (a->streams == 0) return plain_buffers<T>(a, base, nullptr);
   const size_t P = a->portion_rows, D = a->width;
+  ChunkBuffers state;
   size_t h = P * D, fa = 0, fb = 0, raw = 0, p0 = 0, p1 = 0, p2 = 0, mix = 0, rows = 0, kn = 0, vt = 0;
   for (int i = 0; i < a->num_layers; ++i) {
     const QmkHybridLayer& l = a->layers[i];
@@ -461,6 +485,7 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
       fa = std::max(fa, 3 * P * W);
       fb = std::max(fb, P * W);
       raw = std::max(raw, P * W);
+      state.fit(P, l.heads, l.head_dim, l.head_dim, true);
     }
   }
   Carver c{static_cast<char*>(base)};
@@ -470,6 +495,8 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
   b->fa = c.take<float>(fa);
   b->fb = c.take<float>(fb);
   b->raw = c.take<float>(raw);
+  state.take(c);
+  b->state = state;
   b->h = OperandRows<T>(c, h);
   b->p0 = c.take<T>(p0);
   b->p1 = c.take<T>(p1);
@@ -577,6 +604,33 @@ void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* 
   }
 }
 
+// A recurrence over the portion, from its projections to what its norm reads.
+template <class T, int KIND>
+void run_chunks(ChunkArgs g, hipStream_t st) {
+  g.segment = segment_chunks<T>(g.M);
+  const int chunks = chunks_of(g.M), segments = segments_of(g.M, g.segment);
+  auto run = [&](auto wave_tiles) {
+    constexpr int kTiles = decltype(wave_tiles)::value;
+    const dim3 block(kPfThreads);
+    hipLaunchKernelGGL((chunk_prepare<KIND, kTiles>), dim3(chunks, g.heads), block, 0, st, g);
+    if constexpr (KIND == CHUNK_DELTA) {
+      hipLaunchKernelGGL((chunk_scan<kTiles, 4>), dim3(g.heads, g.n / 16), block, 0, st, g);
+    } else {
+      const unsigned groups = g.heads * ((g.n + 63) / 64);
+      if (segments > 1) {
+        hipLaunchKernelGGL((segment_scan<kTiles * 4, false>), dim3(groups * (segments - 1)), block, 0, st, g);
+        if (segments > kOwnStarts) hipLaunchKernelGGL(segment_starts, dim3((g.heads * g.dim * (g.n / 4) + kPfThreads - 1) / kPfThreads), block, 0, st, g);
+      }
+      hipLaunchKernelGGL((segment_scan<kTiles * 4, true>), dim3(groups * segments), block, 0, st, g);
+    }
+  };
+  switch (chunk_tiles(g.dim)) {
+    case 4: return run(std::integral_constant<int, 1>{});
+    case 8: return run(std::integral_constant<int, 2>{});
+    default: return run(std::integral_constant<int, 4>{});
+  }
+}
+
 template <class T>
 int prefill_plain(const QmkHybridArgs* a);
 
@@ -633,7 +687,7 @@ int prefill(const QmkHybridArgs* a) {
       const Keys<T> expanded{b.kn, l.heads * l.head_dim, l.head_dim, 1};
       launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), st);
     } else {
-      const int N = W, n = l.head_dim;
+      const int N = W;
       hipLaunchKernelGGL(shift_mix<T>, dim3(M), block, 0, st, b.u, l, a->slot, a->flip, M, P, D, a->width_true, a->eps, b.h.of(D));
       GemmArgs g = gemm_args(b.h.of(D), D, l.in_w, N, D, l, EPI_WKV_IN);
       g.groups = 5; g.last_n = l.rank; g.a_step = static_cast<long long>(P) * D; g.w_step = static_cast<long long>(N) * D;
@@ -643,11 +697,11 @@ int prefill(const QmkHybridArgs* a) {
       d.f0 = b.fb; d.ldo = N;
       launch_gemm<T, u16, T>(d, b.split, st);
       const size_t step = static_cast<size_t>(P) * N;
-      const dim3 grid(n / kWkvColumns, l.heads), lanes(kWkvThreads);
-      const float *r = b.fa, *k = b.fa + step, *v = b.fa + 2 * step;
-      if (n <= 64) hipLaunchKernelGGL((wkv_scan<4, 32>), grid, lanes, 0, st, r, k, v, b.fb, l, a->slot, M, b.raw);
-      else if (n <= 128) hipLaunchKernelGGL((wkv_scan<8, 16>), grid, lanes, 0, st, r, k, v, b.fb, l, a->slot, M, b.raw);
-      else hipLaunchKernelGGL((wkv_scan<16, 8>), grid, lanes, 0, st, r, k, v, b.fb, l, a->slot, M, b.raw);
+      ChunkArgs c{};
+      c.layer = l; c.q = b.fa; c.k = b.fa + step; c.values = b.fa + 2 * step; c.decay = b.fb; c.out = b.raw;
+      c.chunks = b.state.chunks; c.starts = b.state.starts; c.fades = b.state.fades;
+      c.M = M; c.heads = l.heads; c.dim = c.n = l.head_dim; c.ld = c.value_ld = N; c.slot = a->slot; c.flip = a->flip;
+      run_chunks<T, CHUNK_WKV>(c, st);
       hipLaunchKernelGGL(wkv_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.raw, b.p0, l, M, a->eps, b.mix.of(W));
     }
     residual(l.o_w, W, l, false);
@@ -668,21 +722,6 @@ int prefill(const QmkHybridArgs* a) {
     launch_gemm<T, u16, T>(g, b.split, st);
   }
   return hipGetLastError() == hipSuccess ? QMK_OK : QMK_ERR_LAUNCH;
-}
-
-// The recurrence of a gla or delta entry over the portion, from its projections to what its output projection reads.
-template <class T, bool DELTA>
-void run_chunks(const ChunkArgs& g, hipStream_t st) {
-  constexpr bool kEight = sizeof(T) == 4 && !DELTA;
-  const QmkHybridLayer& l = g.layer;
-  const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens;
-  hipLaunchKernelGGL(chunk_prepare<DELTA>, dim3(chunks, l.heads), dim3(kPfThreads), 0, st, g);
-  auto launch = [&](auto kernel, int waves) { hipLaunchKernelGGL(kernel, dim3(l.heads, l.v_dim / 16), dim3(waves * 64), 0, st, g); };
-  switch (chunk_tiles(l.head_dim)) {
-    case 4: return launch(chunk_scan<1, 4, DELTA>, 4);
-    case 8: return launch(chunk_scan<kEight ? 1 : 2, kEight ? 8 : 4, DELTA>, kEight ? 8 : 4);
-    default: return launch(chunk_scan<kEight ? 2 : 4, kEight ? 8 : 4, DELTA>, kEight ? 8 : 4);
-  }
 }
 
 template <class T>
@@ -749,7 +788,8 @@ int prefill_plain(const QmkHybridArgs* a) {
       launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix.of(W), st);
     } else {
       ChunkArgs c{};
-      c.layer = l; c.decay = b.decay; c.chunks = b.chunks; c.out = b.o; c.M = M; c.slot = a->slot; c.flip = a->flip;
+      c.layer = l; c.decay = b.decay; c.chunks = b.state.chunks; c.starts = b.state.starts; c.fades = b.state.fades; c.out = b.o;
+      c.M = M; c.heads = l.heads; c.dim = l.head_dim; c.n = l.v_dim; c.slot = a->slot; c.flip = a->flip;
       if (l.type == QMK_MIXER_DELTA) {
         const int channels = conv_channels(l), ranks = l.rank + l.gate_rank, beta_ld = (l.heads + 15) / 16 * 16;
         GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_DELTA_IN);
@@ -762,8 +802,8 @@ int prefill_plain(const QmkHybridArgs* a) {
         GemmArgs f = gemm_args(whole(b.low + l.rank), l.gate_w, W, l.gate_rank, l, EPI_SIGMOID);
         f.lda = ranks; f.out = b.gate; f.ldo = W;
         launch_gemm<T, u16, T>(f, b.split, st);
-        c.qkv = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = W;
-        run_chunks<T, true>(c, st);
+        c.q = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = W;
+        run_chunks<T, CHUNK_DELTA>(c, st);
         if (l.taps > 1)
           hipLaunchKernelGGL(keep_inputs, dim3((channels + kPfThreads - 1) / kPfThreads), block, 0, st, b.qkv, l, channels, a->slot, a->flip, M);
       } else {
@@ -774,8 +814,8 @@ int prefill_plain(const QmkHybridArgs* a) {
         GemmArgs e = gemm_args(whole(b.low), l.mid_w, keys, l.rank, l, EPI_GLA_DECAY);
         e.f0 = b.decay; e.ldo = keys;
         launch_gemm<T, u16, T>(e, b.split, st);
-        c.qkv = b.qkv; c.values = b.qkv; c.value_ld = 2 * keys + W; c.value_at = 2 * keys;
-        run_chunks<T, false>(c, st);
+        c.q = b.qkv; c.k = b.qkv + keys; c.values = b.qkv; c.ld = c.value_ld = 2 * keys + W; c.value_at = 2 * keys;
+        run_chunks<T, CHUNK_GLA>(c, st);
       }
       hipLaunchKernelGGL(state_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.o, b.gate, l, M, a->eps, b.mix.of(W));
     }

@@ -1,0 +1,577 @@
+// Recurrences of prefill that keep a state [keys][values] a head: wkv, gated linear attention, gated delta rule, in chunks of sixteen tokens on the matrix cores.
+//
+// Recurrence of one head, state S, decay g_t per key channel:
+//   S <- g_t S,  u_t = beta_t (v_t - S^T k_t),  S <- S + k_t u_t^T,  o_t = S^T q_t        (gla: u_t = v_t)
+//   wkv: o_t = (S + diag(bonus) k_t v_t^T)^T r_t ahead of S <- g_t S + k_t v_t^T
+// Over a chunk that starts from S, with G_t = g_1 .. g_t and D_ts = g_{s+1} .. g_t (products, never quotients: a decay may
+// be small enough for its inverse to overflow):
+//   X_t = (G_t k_t)^T S           u = T (v - X),  T = (I + diag(beta) A)^-1 diag(beta),  A_ts = sum_i k_t D_ts k_s  (s < t)
+//   o_t = (G_t q_t)^T S + sum_{s <= t} B_ts u_s,  B_ts = sum_i q_t D_ts k_s               (wkv: G_{t-1}, D_{t-1,s}, B_tt = sum_i r_t bonus k_t)
+//   S  <- G_16 S + sum_s (D_16,s k_s) u_s^T
+// chunk_prepare works out everything that no state enters, for all chunks at once.  Where u is v a chunk's state is a sum that may be cut anywhere: segments of
+// eight chunks are walked side by side, once from nothing for what they leave (segment_scan<.., false>), then, from the states that segment_starts puts
+// together, for the outputs.  Segments lie where they do from the portion's start on whatever its length, so a token's bits do not depend on it.  The delta rule's
+// chunks are walked one after the other (chunk_scan).
+#pragma once
+
+#include "qmk_hybrid_prefill.h"
+
+namespace qmk {
+namespace hybrid {
+
+constexpr int kChunkTokens = 16;
+constexpr int kChunkWaves = 4;
+constexpr int kSegmentChunks = 8, kShortChunks = 16;
+// Chunks of a segment.  In fp32, where orders may depend on the length, up to kShortChunks are one segment: walking them twice in halves takes longer (us, 200 tokens
+// of 32 heads of 64: prepared and walked once 21.0, in halves 23.5).
+template <class T>
+__host__ __device__ constexpr int segment_chunks(int tokens) { return sizeof(T) == 4 && tokens <= kShortChunks * kChunkTokens ? kShortChunks : kSegmentChunks; }
+// Up to so many segments put their own starts together (the same sums in the same order; a launch less, but every segment reads all before it).
+constexpr int kOwnStarts = 4;
+
+// Tiles of sixteen key channels of a head, the last ones zeros.
+__host__ __device__ constexpr int chunk_tiles(int head_dim) { return head_dim <= 64 ? 4 : head_dim <= 128 ? 8 : 16; }
+// Floats of one (chunk, head): per tile the fragments of G q, G k and D k and the decays G over the whole chunk, then B and
+// T.  A fragment is in the order the matrix instruction takes it: [lane][4].
+__host__ __device__ constexpr int chunk_floats(int head_dim) { return chunk_tiles(head_dim) * (3 * 256 + 16) + 2 * 256; }
+__host__ __device__ constexpr int chunks_of(int tokens) { return (tokens + kChunkTokens - 1) / kChunkTokens; }
+__host__ __device__ constexpr int segments_of(int tokens, int chunks) { return (chunks_of(tokens) + chunks - 1) / chunks; }
+
+enum : int { CHUNK_GLA, CHUNK_DELTA, CHUNK_WKV };
+struct ChunkArgs {
+  QmkHybridLayer layer;
+  const float *q, *k;    // [M][ld]; delta: q alone, q, k, v ahead of the convolution
+  const float* decay;    // [M][heads * dim]
+  const float* beta;     // delta: [M][beta_ld]
+  float* chunks;         // [chunk][head][chunk_floats]
+  float* values;         // [M][value_ld] at value_at; delta: written here
+  float* out;            // [M][heads * n]
+  float* starts;         // [segment][head][dim][n]: what the segment before leaves, then the state the segment starts from
+  float* fades;          // [segment][head][dim]: decays over the segment before
+  int M, heads, dim, n, ld, beta_ld, value_ld, value_at, slot, flip, segment;      // segment: chunks of one
+};
+
+// One workgroup per (chunk, head).  delta: convolution, silu and unit norm of the head's q and k, convolution and silu of its v.
+// A lane holds one token's four channels of every tile of its wave.  Pairs s < t differ first in some bit h of their numbers: with the decays of t from the last
+// multiple of h on and those behind s up to it, each of them at most one, all pairs of that bit are one matrix product over the channels; the products of decays
+// over blocks of h tokens become those of 2h by one exchange between lanes of a row.  So four levels of products replace sixteen running keys a pair of threads
+// (us, 2048 tokens: 8 heads of 128 of gated linear attention 29 -> 13, 16 of 128 | 128 of the delta rule 71 -> 54).  What is left is memory: it writes 27 KB a chunk and head of 128 channels.
+template <int KIND, int TILES>      // of a wave
+__global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
+  constexpr int C = kChunkTokens, kSums = KIND == CHUNK_DELTA ? 2 : 1;
+  __shared__ f32x4 sums[kSums][kChunkWaves][64];
+  __shared__ float diagonal[kChunkWaves][C], norms[2][kChunkWaves][C], step[C];
+  __shared__ __align__(16) float turned[kChunkWaves][C][C + 4];
+  __shared__ __align__(16) float sa[C][C];
+  const QmkHybridLayer& l = g.layer;
+  const int head = blockIdx.y, chunk = blockIdx.x, m0 = chunk * C, count = min(C, g.M - m0);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, quad = lane >> 4;
+  const size_t row = min(m0 + t, g.M - 1);
+  const bool real = t < count;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
+
+  f32x4 q[TILES], k[TILES], w[TILES];
+  float dot = 0.f;      // of this token's q and k: where decays are strong it may be all of an output, whose norm leaves its sign, so it is taken of whole values
+  if constexpr (KIND == CHUNK_DELTA) {
+    const int kv = head / (l.heads / l.kv_heads), keys = l.kv_heads * g.dim, W = conv_channels(l), taps = l.taps;
+    const float* old = l.shift + (static_cast<size_t>(g.slot) * 2 + g.flip) * (taps - 1) * W;
+    // Four channels from `ch` on at this lane's token, behind silu.
+    auto convolved = [&](int ch) {
+      constexpr int kFew = 4;
+      auto input = [&](int back) {      // tokens behind the portion are not used
+        const int at = min(m0 + t - back, g.M - 1);
+        return read4((at >= 0 ? g.q + static_cast<size_t>(at) * W : old + static_cast<size_t>(at + taps - 1) * W) + ch);
+      };
+      f32x4 v = zero;
+      if (taps <= kFew) {
+        f32x4 in[kFew], weight[kFew];
+#pragma unroll
+        for (int j = 0; j < kFew; ++j) {
+          const bool there = j >= kFew - taps;
+          in[j] = input(there ? kFew - 1 - j : 0);
+          weight[j] = there ? read4(l.vec2 + static_cast<size_t>(j - kFew + taps) * W + ch) : zero;
+        }
+#pragma unroll
+        for (int j = 0; j < kFew; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = j >= kFew - taps ? fmaf(weight[j][i], in[j][i], v[i]) : v[i];
+      } else {
+        for (int j = 0; j < taps; ++j) {
+          const f32x4 in = input(taps - 1 - j), weight = read4(l.vec2 + static_cast<size_t>(j) * W + ch);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = fmaf(weight[i], in[i], v[i]);
+        }
+      }
+      return each(v, [](float x) { return x * sigmoid(x); });
+    };
+    float nq = 0.f, nk = 0.f;
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      const int c = (wave * TILES + j) * 16 + quad * 4;
+      q[j] = k[j] = zero;
+      if ((wave * TILES + j) * 16 < g.dim) {
+        q[j] = convolved(kv * g.dim + c);
+        k[j] = convolved(keys + kv * g.dim + c);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        nq = fmaf(q[j][i], q[j][i], nq);
+        nk = fmaf(k[j][i], k[j][i], nk);
+        dot = fmaf(q[j][i], k[j][i], dot);
+      }
+    }
+    for (int tile = wave; tile * 16 < g.n; tile += kChunkWaves) {
+      const int c = head * g.n + tile * 16 + quad * 4;
+      const f32x4 v = convolved(2 * keys + c);
+      if (real) store4(g.values + row * g.value_ld + g.value_at + c, v);
+    }
+    if (tid < count) step[tid] = g.beta[static_cast<size_t>(m0 + tid) * g.beta_ld + head];
+    nq += __shfl_xor(nq, 16);
+    nk += __shfl_xor(nk, 16);
+    nq += __shfl_xor(nq, 32);
+    nk += __shfl_xor(nk, 32);
+    if (quad == 0) {
+      norms[0][wave][t] = nq;
+      norms[1][wave][t] = nk;
+    }
+    __syncthreads();
+    nq = nk = 0.f;
+#pragma unroll
+    for (int i = 0; i < kChunkWaves; ++i) {
+      nq += norms[0][i][t];
+      nk += norms[1][i][t];
+    }
+    const float iq = l.q_scale / sqrtf(nq + 1e-6f), ik = 1.f / sqrtf(nk + 1e-6f);      // unit vectors
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      q[j] *= iq;
+      k[j] *= ik;
+    }
+    dot = real ? dot * iq * ik : 0.f;
+  } else {
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      const int c = head * g.dim + min((wave * TILES + j) * 16, g.dim - 16) + quad * 4;
+      q[j] = read4(g.q + row * g.ld + c);
+      k[j] = read4(g.k + row * g.ld + c);
+      if constexpr (KIND == CHUNK_GLA) q[j] *= l.q_scale;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) {
+    const bool there = (wave * TILES + j) * 16 < g.dim;
+    const int c = head * g.dim + min((wave * TILES + j) * 16, g.dim - 16) + quad * 4;
+    w[j] = read4(g.decay + row * g.heads * g.dim + c);
+    q[j] = there && real ? q[j] : zero;
+    k[j] = there && real ? k[j] : zero;
+    w[j] = there && real ? w[j] : one;
+    const f32x4 bonus = KIND == CHUNK_WKV ? read4(l.vec1 + c) : one;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if constexpr (KIND != CHUNK_DELTA) dot = fmaf(q[j][i] * bonus[i], k[j][i], dot);
+  }
+  dot += __shfl_xor(dot, 16);
+  dot += __shfl_xor(dot, 32);
+  if (quad == 0) diagonal[wave][t] = dot;
+
+  // Products of decays within this token's block of h: ahead of it, behind it, all; from now on q (delta: and k') with its own decay but for wkv.
+  f32x4 ahead[TILES], behind[TILES], all[TILES], key[KIND == CHUNK_DELTA ? TILES : 1];
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) {
+    ahead[j] = behind[j] = one;
+    all[j] = w[j];
+    if constexpr (KIND != CHUNK_WKV) q[j] *= w[j];
+    if constexpr (KIND == CHUNK_DELTA) key[j] = k[j] * w[j];
+  }
+  f32x4 pairs[kSums] = {};
+  auto level = [&](auto size, auto exchange) {
+    constexpr int h = decltype(size)::value;
+    const bool later = (t & h) != 0;
+    f32x4 p[kSums] = {};
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      const f32x4 to = later ? q[j] * ahead[j] : zero, from = later ? zero : k[j] * behind[j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(to[i], from[i], p[0], 0, 0, 0);
+      if constexpr (KIND == CHUNK_DELTA) {
+        const f32x4 also = later ? key[j] * ahead[j] : zero;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(also[i], from[i], p[1], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float other = dpp_f32<decltype(exchange)::value>(1.f, all[j][i]);
+        ahead[j][i] *= later ? other : 1.f;
+        behind[j][i] *= later ? 1.f : other;
+        all[j][i] *= other;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)      // row (later token) quad 4 + i, column (earlier one) t: of one block of 2h
+#pragma unroll
+      for (int e = 0; e < kSums; ++e) pairs[e][i] += ((quad * 4 + i) ^ t) < 2 * h ? p[e][i] : 0.f;
+  };
+  level(std::integral_constant<int, 1>{}, std::integral_constant<int, kDppQuadXor1>{});
+  level(std::integral_constant<int, 2>{}, std::integral_constant<int, kDppQuadXor2>{});
+  level(std::integral_constant<int, 4>{}, std::integral_constant<int, kDppHalfMirror>{});
+  level(std::integral_constant<int, 8>{}, std::integral_constant<int, 0x140>{});      // row_mirror
+#pragma unroll
+  for (int e = 0; e < kSums; ++e) sums[e][wave][lane] = pairs[e];
+
+  float* rec = g.chunks + (static_cast<size_t>(chunk) * g.heads + head) * chunk_floats(g.dim);
+  constexpr int stored = TILES * kChunkWaves;
+  float *rq = rec, *rk = rq + stored * 256, *rd = rk + stored * 256, *rg = rd + stored * 256, *rb = rg + stored * 16, *rt = rb + 256;
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) {
+    const int tile = wave * TILES + j;
+    store4(rq + tile * 256 + lane * 4, q[j] * ahead[j]);
+    if constexpr (KIND == CHUNK_DELTA) store4(rk + tile * 256 + lane * 4, key[j] * ahead[j]);
+    if (t == 0) store4(rg + tile * 16 + quad * 4, all[j]);
+    store4(&turned[wave][t][quad * 4], k[j] * behind[j]);
+    __builtin_amdgcn_wave_barrier();
+    store4(rd + tile * 256 + lane * 4, f32x4{turned[wave][quad * 4][t], turned[wave][quad * 4 + 1][t], turned[wave][quad * 4 + 2][t], turned[wave][quad * 4 + 3][t]});
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  {
+    const int to = (tid >> 2) & 15, from = (tid >> 6) * 4 + (tid & 3), at = (to >> 2) * 16 + from;
+    float b = 0.f, a = 0.f;
+#pragma unroll
+    for (int i = 0; i < kChunkWaves; ++i) {
+      b += sums[0][i][at][to & 3] + (to == from ? diagonal[i][to] : 0.f);
+      if constexpr (KIND == CHUNK_DELTA) a += sums[1][i][at][to & 3];
+    }
+    rb[tid] = b;
+    if constexpr (KIND == CHUNK_DELTA) sa[to][from] = a;
+  }
+  if constexpr (KIND == CHUNK_DELTA) {
+    __syncthreads();
+    if (tid < C) {     // column tid of T
+      float col[C];
+#pragma unroll
+      for (int r = 0; r < C; ++r) {
+        float acc = r == tid ? 1.f : 0.f;
+#pragma unroll
+        for (int j = 0; j < r; ++j) acc = fmaf(-sa[r][j], col[j], acc);
+        col[r] = r < count ? acc * step[r] : 0.f;
+        rt[((tid >> 2) * 16 + r) * 4 + (tid & 3)] = col[r];
+      }
+    }
+  }
+}
+
+// Sixteen value columns a wave, all key channels; one segment and head a workgroup.  A chunk's record goes from memory to LDS by itself while the one before is
+// multiplied: the state's tiles are the matrix instruction's accumulators and at the same time the second operand of the products that read them, and nothing is
+// exchanged between waves.  OUT: from the segment's start, with outputs, and the last segment leaves the portion's state; otherwise from nothing, for what it
+// leaves.  What bounds it is the fp32 matrix instruction (68 of 43 cycles a chunk and wave, 36 without outputs) and, where a launch begins, all its workgroups' first loads (12 us of
+// 29).  us in whole portions, chunks one after the other with keys split over waves -> three launches side by side: 2048 tokens of 8 heads of 128 | 256 68 -> 29 + 17 + 8, 1531 of 32
+// heads of 64 (wkv, before: token by token, with chunk_prepare's 16) 117 -> 17 + 10 + 5 + 16.  Segments of 16 chunks: 33 + 19 + 6 and 20 + 12 + 5.
+template <int TILES, bool OUT>
+__global__ __launch_bounds__(kPfThreads, TILES == 16 ? 1 : 2) void segment_scan(const ChunkArgs g) {
+  constexpr int kFirst = OUT ? TILES : 0, kRest = (TILES * 256 + TILES * 16 + (OUT ? 256 : 0) + 255) / 256;      // loads of 1 KB of a record: G q; D k, G and B
+  constexpr int kRecord = (kFirst + kRest + 3) / 4, kEach = kRecord + 1;      // loads of a wave: of the record (the last ones twice), its part of the values
+  constexpr int kStage = kEach * 4 * 64, kValues = kRecord * 4 * 64, kStages = TILES == 16 ? 2 : 3;
+  __shared__ __align__(16) v4u lds[kStages * kStage];
+  using Lds = __attribute__((address_space(3))) v4u;
+  Lds* const stages = (Lds*)lds;
+  const QmkHybridLayer& l = g.layer;
+  // (Workgroups of one segment and head, which read the same records, on one XCD.)
+  const int dim = g.dim, n = g.n, groups = (n + 63) / 64, id = xcd_order(blockIdx.x, gridDim.x), group = id % groups, head = id / groups % g.heads, segment = id / groups / g.heads;
+  const int out_ld = g.heads * n;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, quad = lane >> 4;
+  const int column = group * 64, v0 = column + wave * 16, tiles = dim / 16;
+  const bool mine = v0 < n;
+  const int first = segment * g.segment, chunks = min(chunks_of(g.M) - first, g.segment), segments = segments_of(g.M, g.segment);
+  const size_t size = static_cast<size_t>(dim) * n, place = v0 + col;
+  float* state = l.state + (static_cast<size_t>(g.slot) * g.heads + head) * size + place;
+  f32x4 s[TILES], fade[OUT ? 1 : TILES];
+#pragma unroll
+  for (int j = 0; j < TILES; ++j) {
+    s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (!OUT) fade[j] = f32x4{1.f, 1.f, 1.f, 1.f};
+  }
+  if constexpr (OUT) {
+    const bool own = segments <= kOwnStarts;
+    const int from = own ? 0 : segment;
+    const float* start = segments == 1 ? state : g.starts + (static_cast<size_t>(from) * g.heads + head) * size + place;
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < TILES; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (j < tiles) s[j][i] = start[static_cast<size_t>(j * 16 + quad * 4 + i) * n];
+#pragma unroll 1
+      for (int before = from; before < segment; ++before) {
+        start += g.heads * size;
+        const float* fades = g.fades + (static_cast<size_t>(before + 1) * g.heads + head) * dim + quad * 4;
+        f32x4 left[TILES];
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (j < tiles) left[j][i] = start[static_cast<size_t>(j * 16 + quad * 4 + i) * n];
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+          if (j < tiles) s[j] = s[j] * read4(fades + j * 16) + left[j];
+      }
+    }
+  }
+  // Tokens and columns behind the last ones are that one and the head's last four again: they meet zeros of the record, or nobody reads them.
+  auto issue = [&](int c) {
+    const int chunk = first + c;
+    Lds* to = stages + c % kStages * kStage;
+    auto load = [&](const float* from, int place) {
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint32_t*)from, (__attribute__((address_space(3))) uint32_t*)(to + place * 64), 16, 0, 0);
+    };
+    const float* rec = g.chunks + (static_cast<size_t>(chunk) * g.heads + head) * chunk_floats(dim) + lane * 4;
+#pragma unroll
+    for (int i = 0; i < kRecord; ++i) {
+      const int part = min(i * 4 + wave, kFirst + kRest - 1);
+      load(rec + (part < kFirst ? part * 256 : TILES * 512 + (part - kFirst) * 256), part);
+    }
+    const int token = min(chunk * kChunkTokens + wave * 4 + quad, g.M - 1), at = min(column + col * 4, n - 4);
+    load(g.values + static_cast<size_t>(token) * g.value_ld + g.value_at + head * n + at, kRecord * 4 + wave);
+  };
+  auto buffer = [](const float* base, int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000); };
+  // Bytes from a chunk's first value (output) to behind its last one, of rows of `ld`: tokens behind the last one are read as zero and not written.
+  auto extent = [&](int chunk, int ld) { return ((min(g.M - chunk * kChunkTokens, kChunkTokens) - 1) * ld + 16) * 4; };
+  // Until all but the last `later` of this wave's requests are done, and everybody's.
+  auto landed = [&](auto later) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(later)::value) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto product = [](f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+    return c;
+  };
+  constexpr int kAhead = kStages - 1;
+#pragma unroll
+  for (int c = 0; c < kAhead; ++c)
+    if (c < chunks) issue(c);
+#pragma unroll 1
+  for (int c = 0; c < chunks; ++c) {
+    // This chunk's stage has landed, and everybody has read the one that is filled next.  Behind its requests come those of the stages since and, from the second
+    // chunk on, at least one chunk's four stores of outputs, which count like loads.
+    constexpr int kLater = (kAhead - 1) * kEach;
+    if (kLater == 0 || c + kAhead > chunks) landed(std::integral_constant<int, 0>{});
+    else if (OUT && mine && c > 0) landed(std::integral_constant<int, kLater + 4>{});
+    else landed(std::integral_constant<int, kLater>{});
+    if (c + kAhead < chunks) issue(c + kAhead);
+    const int chunk = first + c;
+    const Lds *q = stages + c % kStages * kStage, *d = q + kFirst * 64, *decay = d + TILES * 64, *b = decay + TILES * 4;
+    const auto* value = (const __attribute__((address_space(3))) float*)(stages + c % kStages * kStage + kValues) + wave * 16 + col;
+    const f32x4 u = {value[quad * 256], value[quad * 256 + 64], value[quad * 256 + 128], value[quad * 256 + 192]};
+    auto fragment = [&](const Lds* at) { return __builtin_bit_cast(f32x4, at[lane]); };
+    if constexpr (OUT) {
+      f32x4 o[2] = {};
+#pragma unroll
+      for (int j = 0; j < TILES; ++j) o[j & 1] = product(fragment(q + j * 64), s[j], o[j & 1]);
+      o[1] = product(fragment(b), u, o[1]);
+      o[0] += o[1];
+      if (mine) {
+        const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, extent(chunk, out_ld));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[0][i]), to, ((quad * 4 + i) * out_ld + col) * 4, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      const f32x4 g4 = __builtin_bit_cast(f32x4, decay[j * 4 + quad]);
+      if constexpr (!OUT) fade[j] *= g4;
+      s[j] = product(fragment(d + j * 64), u, s[j] * g4);
+    }
+  }
+  if (!mine) return;
+  if (!OUT && segment == 0 && segments <= kOwnStarts) {      // a copy of the portion's state, which the last segment overwrites, for the others to start from
+    f32x4 held[TILES];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (j < tiles) held[j][i] = state[static_cast<size_t>(j * 16 + quad * 4 + i) * n];
+    float* copy = g.starts + head * size + place;
+#pragma unroll
+    for (int j = 0; j < TILES; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (j < tiles) copy[static_cast<size_t>(j * 16 + quad * 4 + i) * n] = held[j][i];
+  }
+  float* to = OUT ? state : g.starts + (static_cast<size_t>(segment + 1) * g.heads + head) * size + place;
+  if (OUT && segment + 1 < segments) return;
+#pragma unroll
+  for (int j = 0; j < TILES; ++j)
+    if (j < tiles) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) to[static_cast<size_t>(j * 16 + quad * 4 + i) * n] = s[j][i];
+      if constexpr (!OUT)
+        if (v0 == 0 && col == 0) store4(g.fades + (static_cast<size_t>(segment + 1) * g.heads + head) * dim + j * 16 + quad * 4, fade[j]);
+    }
+}
+
+// The state every segment starts from, out of the portion's and what the segments leave: four columns of a key row a thread.
+__global__ __launch_bounds__(kPfThreads) void segment_starts(const ChunkArgs g) {
+  const int rows = g.heads * g.dim, quads = g.n / 4, id = blockIdx.x * kPfThreads + threadIdx.x, segments = segments_of(g.M, g.segment);
+  if (id >= rows * quads) return;
+  const int row = id / quads;
+  const size_t at = static_cast<size_t>(row) * g.n + id % quads * 4, step = static_cast<size_t>(rows) * g.n;
+  f32x4 s = read4(g.layer.state + static_cast<size_t>(g.slot) * step + at);
+  store4(g.starts + at, s);      // (the last segment overwrites it where it was)
+  constexpr int kBatch = 8;      // segments asked for together: each is read and written in one place
+#pragma unroll 1
+  for (int first = 1; first < segments; first += kBatch) {
+    f32x4 left[kBatch];
+    float fade[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int segment = min(first + i, segments - 1);
+      left[i] = read4(g.starts + segment * step + at);
+      fade[i] = g.fades[static_cast<size_t>(segment) * rows + row];
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      if (first + i >= segments) break;
+      s = s * fade[i] + left[i];
+      store4(g.starts + (first + i) * step + at, s);
+    }
+  }
+}
+
+// One head and sixteen value columns a workgroup; a wave holds TILES tiles of sixteen key channels of the state as the
+// accumulators of the matrix instruction, which are also the second operand of the products that read it.  Tiles behind the
+// last one are zeros and take part: with a branch around each tile's products this compiler has left out the wait between a
+// tile's last product and the first use of its result on the path that skips the next tile.  Loads have no branches either,
+// so that kAhead chunks are in flight: a chunk, or token, behind the last one is the last one again, and its value is either
+// not used or multiplied by zero.
+// What bounds it is the chain of a chunk: products of the state with the keys (four dependent instructions of 32 cycles a tile), the
+// waves' sums through LDS, T (v - X), the state's update.  So what only the output needs is off the chain: G q S is taken while the sums are on their way, and a
+// chunk's outputs are added up and stored behind the next chunk's barrier.
+// A wave's instructions are on that chain too, one wave a SIMD: chunks are read and written by buffer accesses (places of 32 bits that stay, bases that move on by
+// one scalar addition, tokens behind the last one read as zero and not written).  us, 2048 tokens of 16 heads of 128 | 128, addresses of 64 bits worked out for every
+// access -> now 134 -> 120; lines of chunks further ahead asked for into L2: 141.
+template <int TILES, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 1) void chunk_scan(const ChunkArgs g) {
+  // Chunks in flight: what the registers hold (us, the shape above, with 2, 3 and 4 ahead: 131, 120, 123).
+  constexpr int kAhead = TILES == 1 ? 4 : TILES == 2 ? 3 : 2;
+  __shared__ f32x4 px[2][WAVES][64], po[2][WAVES][64];
+  const QmkHybridLayer& l = g.layer;
+  const int dim = g.dim, n = g.n, head = blockIdx.x, v0 = blockIdx.y * 16;
+  constexpr int tiles = TILES * WAVES;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, quad = lane >> 4;
+  const int tile0 = wave * TILES, mine = min(max(dim / 16 - tile0, 0), TILES);
+  const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens, out_ld = l.heads * n;
+  float* state = l.state + (static_cast<size_t>(g.slot) * l.heads + head) * dim * n + v0 + col;
+  auto buffer = [](const float* base, int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000); };
+  // Bytes from a chunk's first value (output) to behind its last one, of rows of `ld`.
+  auto extent = [&](int chunk, int ld) { return ((min(g.M - chunk * kChunkTokens, kChunkTokens) - 1) * ld + 16) * 4; };
+  uint32_t value_at[4], out_at[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    value_at[i] = ((quad * 4 + i) * g.value_ld + col) * 4;
+    out_at[i] = ((quad * 4 + i) * out_ld + col) * 4;
+  }
+  const uint32_t fragment_at = tile0 * 1024 + lane * 16, decay_at = tile0 * 64 + quad * 16, shared_at = lane * 16;
+  f32x4 s[TILES];
+#pragma unroll
+  for (int j = 0; j < TILES; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[j][i] = j < mine ? state[static_cast<size_t>((tile0 + j) * 16 + quad * 4 + i) * n] : 0.f;
+
+  struct Fragments {
+    f32x4 q[TILES], k[TILES], d[TILES], g[TILES], b, t, v;
+  };
+  // Chunks are fetched in their order; behind the last one it is the last one again.
+  const size_t rec_step = static_cast<size_t>(l.heads) * chunk_floats(dim), value_step = static_cast<size_t>(kChunkTokens) * g.value_ld;
+  const float *rec = g.chunks + static_cast<size_t>(head) * chunk_floats(dim), *values = g.values + g.value_at + head * n + v0;
+  int fetched = 0;
+  auto fetch = [&](Fragments& f) {
+    const auto r = buffer(rec, chunk_floats(tiles * 16) * 4), v = buffer(values, extent(fetched, g.value_ld));
+    auto read = [&](uint32_t at, int first) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, first * 4, 0)); };
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      f.k[j] = read(fragment_at + j * 1024, tiles * 256);
+      f.q[j] = read(fragment_at + j * 1024, 0);
+      f.d[j] = read(fragment_at + j * 1024, tiles * 512);
+      f.g[j] = read(decay_at + j * 64, tiles * 768);
+    }
+    f.b = read(shared_at, tiles * 784);
+    f.t = read(shared_at, tiles * 784 + 256);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f.v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(v, value_at[i], 0, 0));
+    const bool more = fetched + 1 < chunks;
+    rec += more ? rec_step : 0;
+    values += more ? value_step : 0;
+    fetched += more;
+  };
+  auto product = [](f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+    return c;
+  };
+  // Ahead of a branch's end: this compiler (clang 22 of ROCm 7.2.0) has left out the wait between a product and the move of its result where paths meet; without
+  // this <1, 4> moves one two instructions behind its product.  The rule, for any kernel: an accumulator that lives across the end of a branch with a product in it is
+  // settled there if its built code has such a move (tests/test_matrix_waits.py walks every path of every kernel for it); none but these two places has.
+  auto settle = [](f32x4& v) { asm volatile("s_nop 15" : "+v"(v)); };
+  f32x4 inner = {};       // B u of the last chunk whose outputs are this wave's
+  auto outputs = [&](int chunk) {
+    if (chunk < 0 || wave != (chunk & (WAVES - 1))) return;
+    f32x4 o = inner;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) o += po[chunk & 1][w][lane];
+    const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, extent(chunk, out_ld));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[i]), to, out_at[i], 0, 0);
+  };
+  auto advance = [&](const Fragments& f, int chunk) {
+    const int buf = chunk & 1;
+    f32x4 x = {};
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) x = product(f.k[j], s[j], x);
+    px[buf][wave][lane] = x;
+    __syncthreads();      // everybody's X; the chunk before's G q S
+    f32x4 u = f.v;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) u -= px[buf][w][lane];
+    f32x4 o = {};
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) o = product(f.q[j], s[j], o);
+    po[buf][wave][lane] = o;
+    u = product(f.t, u, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) s[j] = product(f.d[j], u, s[j] * f.g[j]);
+    outputs(chunk - 1);
+    if (wave == (chunk & (WAVES - 1))) {
+      inner = product(f.b, u, f32x4{0.f, 0.f, 0.f, 0.f});
+      settle(inner);
+    }
+  };
+  Fragments f[kAhead];
+#pragma unroll
+  for (int a = 0; a < kAhead; ++a) fetch(f[a]);
+  int chunk = 0;
+  for (; chunk + kAhead <= chunks; chunk += kAhead) {
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) {
+      advance(f[a], chunk + a);
+      fetch(f[a]);
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < kAhead - 1; ++a)
+    if (chunk + a < chunks) {
+      advance(f[a], chunk + a);
+#pragma unroll
+      for (int j = 0; j < TILES; ++j) settle(s[j]);
+    }
+  __syncthreads();
+  outputs(chunks - 1);
+#pragma unroll
+  for (int j = 0; j < TILES; ++j)
+    if (j < mine)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) state[static_cast<size_t>((tile0 + j) * 16 + quad * 4 + i) * n] = s[j][i];
+}
+
+}  // namespace hybrid
+}  // namespace qmk

@@ -337,130 +337,6 @@ __global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const fl
     if (t < vt) put4(out, at + t * 16 + g * 4, acc[t] * inv * read4(gate + at + t * 16 + g * 4));
 }
 
-// The wkv recurrence: one head and eight value columns a workgroup; sixteen lanes share a column, KPL neighbouring key
-// rows each, in registers.  TB tokens at a time: the next block's r, k, w, v are in flight while this one runs, a block's
-// outputs leave together.  Places behind the last token or key row hold r = k = 0, w = 1, which changes nothing.
-// What bounds it is a wave's chain of tokens, one wave on half of the SIMDs: heads of up to 64 read four tokens ahead out of LDS (1531 tokens, 32 heads of 64, us, read
-// where they are used -> so: 141 -> 122; larger heads have no registers for it).
-constexpr int kWkvColumns = 8, kWkvThreads = 16 * kWkvColumns;
-template <int KPL, int TB>
-__global__ __launch_bounds__(kWkvThreads) void wkv_scan(const float* r, const float* k, const float* v, const float* w, QmkHybridLayer l, int slot, int M, float* out) {
-  constexpr int kKeys = 16 * KPL, kQuads = TB * kKeys / 4 / kWkvThreads, kValueQuads = TB * kWkvColumns / 4;
-  static_assert(kQuads * kWkvThreads * 4 == TB * kKeys && kValueQuads <= kWkvThreads, "every thread stages the same number of quads");
-  __shared__ __align__(16) float sr[2][TB][kKeys], sk[2][TB][kKeys], sw[2][TB][kKeys], sv[2][TB][kWkvColumns], so[2][TB][kWkvColumns];
-  const int n = l.head_dim, N = l.heads * n, head = blockIdx.y, v0 = blockIdx.x * kWkvColumns;
-  const int tid = threadIdx.x, part = tid & 15, e = tid >> 4;
-  float* st = l.state + (static_cast<size_t>(slot) * l.heads + head) * n * n + v0 + e;
-  float s[KPL], u[KPL];
-#pragma unroll
-  for (int i = 0; i < KPL; ++i) {
-    const int row = part * KPL + i;
-    s[i] = row < n ? st[row * n] : 0.f;
-    u[i] = row < n ? l.vec1[head * n + row] : 0.f;
-  }
-  f32x4 fr[kQuads], fk[kQuads], fw[kQuads], fv = {};
-  auto fetch = [&](int base) {
-#pragma unroll
-    for (int q = 0; q < kQuads; ++q) {
-      const int id = tid + q * kWkvThreads, t = base + id / (kKeys / 4), c = id % (kKeys / 4) * 4;
-      const size_t at = static_cast<size_t>(t) * N + head * n + c;
-      const bool real = t < M && c < n;
-      fr[q] = real ? *reinterpret_cast<const f32x4*>(r + at) : f32x4{0.f, 0.f, 0.f, 0.f};
-      fk[q] = real ? *reinterpret_cast<const f32x4*>(k + at) : f32x4{0.f, 0.f, 0.f, 0.f};
-      fw[q] = real ? *reinterpret_cast<const f32x4*>(w + at) : f32x4{1.f, 1.f, 1.f, 1.f};
-    }
-    if (tid < kValueQuads) {
-      const int t = base + tid / (kWkvColumns / 4);
-      fv = t < M ? *reinterpret_cast<const f32x4*>(v + static_cast<size_t>(t) * N + head * n + v0 + tid % (kWkvColumns / 4) * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-  };
-  auto stash = [&](int buf) {
-#pragma unroll
-    for (int q = 0; q < kQuads; ++q) {
-      const int id = tid + q * kWkvThreads, t = id / (kKeys / 4), c = id % (kKeys / 4) * 4;
-      *reinterpret_cast<f32x4*>(&sr[buf][t][c]) = fr[q];
-      *reinterpret_cast<f32x4*>(&sk[buf][t][c]) = fk[q];
-      *reinterpret_cast<f32x4*>(&sw[buf][t][c]) = fw[q];
-    }
-    if (tid < kValueQuads) *reinterpret_cast<f32x4*>(&sv[buf][tid / (kWkvColumns / 4)][tid % (kWkvColumns / 4) * 4]) = fv;
-  };
-  struct Four {      // tokens, as a lane takes them
-    f32x4 r[4][KPL / 4], k[4][KPL / 4], w[4][KPL / 4];
-    float v[4];
-  };
-  fetch(0);
-  stash(0);
-  __syncthreads();
-  int buf = 0;
-  for (int base = 0; base < M; base += TB, buf ^= 1) {
-    if (base + TB < M) fetch(base + TB);
-    // Four tokens at a time: their sums over the sixteen lanes are taken together (two steps that halve the values while
-    // they pair lanes, then plain sums), and lane p of sixteen ends up with token p % 4.
-    auto read = [&](Four& f, int t0) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        f.v[q] = sv[buf][t0 + q][e];
-#pragma unroll
-        for (int i = 0; i < KPL / 4; ++i) {
-          f.r[q][i] = *reinterpret_cast<const f32x4*>(&sr[buf][t0 + q][part * KPL + i * 4]);
-          f.k[q][i] = *reinterpret_cast<const f32x4*>(&sk[buf][t0 + q][part * KPL + i * 4]);
-          f.w[q][i] = *reinterpret_cast<const f32x4*>(&sw[buf][t0 + q][part * KPL + i * 4]);
-        }
-      }
-    };
-    auto walk = [&](const Four& f, int t0) {
-      float o[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        o[q] = 0.f;
-#pragma unroll
-        for (int i = 0; i < KPL; ++i) {
-          const float kv = f.k[q][i / 4][i % 4] * f.v[q];
-          o[q] = fmaf(f.r[q][i / 4][i % 4], fmaf(u[i], kv, s[i]), o[q]);
-          s[i] = fmaf(f.w[q][i / 4][i % 4], s[i], kv);
-        }
-      }
-      const bool b0 = part & 1, b1 = part & 2;
-      const float lo = (b0 ? o[1] : o[0]) + dpp_f32<kDppQuadXor1>(0.f, b0 ? o[0] : o[1]);
-      const float hi = (b0 ? o[3] : o[2]) + dpp_f32<kDppQuadXor1>(0.f, b0 ? o[2] : o[3]);
-      float sum = (b1 ? hi : lo) + dpp_f32<kDppQuadXor2>(0.f, b1 ? lo : hi);
-      sum += dpp_f32<0x124>(0.f, sum);        // row_ror:4
-      sum += dpp_f32<0x128>(0.f, sum);        // row_ror:8
-      if (part < 4) so[buf][t0 + part][e] = sum;
-    };
-    if constexpr (KPL == 4) {
-      Four f[2];
-      read(f[0], 0);
-#pragma unroll
-      for (int t0 = 0; t0 < TB; t0 += 8) {
-        read(f[1], t0 + 4);
-        __builtin_amdgcn_sched_barrier(0);
-        walk(f[0], t0);
-        if (t0 + 8 < TB) read(f[0], t0 + 8);
-        __builtin_amdgcn_sched_barrier(0);
-        walk(f[1], t0 + 4);
-      }
-    } else {
-      for (int t0 = 0; t0 < TB; t0 += 4) {
-        Four f;
-        read(f, t0);
-        walk(f, t0);
-      }
-    }
-    if (base + TB < M) stash(buf ^ 1);
-    __syncthreads();
-    for (int id = tid; id < TB * kWkvColumns; id += kWkvThreads) {
-      const int t = id / kWkvColumns, c = id % kWkvColumns;
-      if (base + t < M) out[static_cast<size_t>(base + t) * N + head * n + v0 + c] = so[buf][t][c];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < KPL; ++i) {
-    const int row = part * KPL + i;
-    if (row < n) st[row * n] = s[i];
-  }
-}
-
 // Per-head norm, weight and gate behind the recurrence: one wave per (token, head).
 template <class T>
 __global__ __launch_bounds__(kPfThreads) void wkv_out(const float* o, const T* gate, QmkHybridLayer l, int M, float eps, Operand<T> out) {
