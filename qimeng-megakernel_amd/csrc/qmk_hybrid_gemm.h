@@ -175,12 +175,18 @@ template <class F>
 __device__ __forceinline__ f32x4 each(f32x4 v, F&& f) { return f32x4{f(v[0]), f(v[1]), f(v[2]), f(v[3])}; }
 
 // Eight consecutive outputs n .. n+7 of a token (sizes of storage are multiples of sixteen, so they are of one kind).  What depends on the columns alone
-// is read once, ahead of the tokens.
+// is worked out once, ahead of the tokens; four pairs' angles of a rotation are read together (us, 2048 x 6144 x 2048 into an attention, inside a portion, pair by pair with
+// places worked out for every token -> so: 79 -> 70; 1531 x 5696 x 2048 into a latent one 58 -> 56).
+struct Angles {
+  f32x4 cos, sin;
+};
 template <class T, int EPI>
 struct Epilogue {
   const GemmArgs& g;
   const int group, n;
   f32x4 b[2] = {};       // constants of the eight outputs
+  int dim = -1;          // rotated dimensions: the first of the eight (-1: none is)
+  int place = 0;         // keys and values of an attention: where they lie in a cache row
 
   __device__ __forceinline__ Epilogue(const GemmArgs& args, int group_, int n_) : g(args), group(group_), n(n_) {
     const QmkHybridLayer& l = g.layer;
@@ -191,13 +197,51 @@ struct Epilogue {
       b[0] = read4(from);
       b[1] = read4(from + 4);
     }
+    if constexpr (EPI == EPI_LATENT_IN) {
+      if (n < l.heads * l.q_stride) dim = max(n % l.q_stride - l.head_dim, -1);
+    } else if constexpr (EPI == EPI_ATTENTION_IN) {
+      const int c = n - l.heads * l.q_stride, width = l.head_dim + l.v_dim, k_rows = l.kv_heads * l.head_dim;
+      if (c < 0) {
+        dim = n % l.q_stride;
+      } else if (c < k_rows) {
+        dim = c % l.head_dim;
+        place = c / l.head_dim * width + dim;
+      } else {
+        place = (c - k_rows) / l.v_dim * width + l.head_dim + (c - k_rows) % l.v_dim;
+      }
+    }
+    if (dim >= l.rot_true) dim = -1;
   }
 
-  // Pairs (d, d+1) .. (d+6, d+7) of a head turned to their position.
-  __device__ __forceinline__ void turn(int position, int d, f32x4& lo, f32x4& hi) const {
+  __device__ __forceinline__ Angles angles(int m) const {
+    const QmkHybridLayer& l = g.layer;
+    Angles t{};
+    if (dim < 0) return t;
+    const size_t at = static_cast<size_t>(g.position + m) * (l.rot_true / 2) + (dim >> 1);
+    if (l.rot_true % 8 == 0) {
+      t.cos = read4(l.rope_cos + at);
+      t.sin = read4(l.rope_sin + at);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const size_t pair = at + min(i, (l.rot_true - dim) / 2 - 1);
+        t.cos[i] = l.rope_cos[pair];
+        t.sin[i] = l.rope_sin[pair];
+      }
+    }
+    return t;
+  }
+
+  // Pairs (dim, dim + 1) .. (dim + 6, dim + 7) of a head turned to their position.
+  __device__ __forceinline__ void turn(const Angles& t, f32x4& lo, f32x4& hi) const {
     float e[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 #pragma unroll
-    for (int i = 0; i < 8; i += 2) rotate(g.layer, position, d + i, e[i], e[i + 1]);
+    for (int i = 0; i < 4; ++i) {
+      if (dim + 2 * i >= g.layer.rot_true) continue;
+      const float x = e[2 * i] * t.cos[i] - e[2 * i + 1] * t.sin[i];
+      e[2 * i + 1] = e[2 * i + 1] * t.cos[i] + e[2 * i] * t.sin[i];
+      e[2 * i] = x;
+    }
     lo = f32x4{e[0], e[1], e[2], e[3]};
     hi = f32x4{e[4], e[5], e[6], e[7]};
   }
@@ -235,8 +279,7 @@ struct Epilogue {
     } else if constexpr (EPI == EPI_LATENT_IN) {
       const int q_rows = l.heads * l.q_stride, g_rows = l.heads * l.v_dim;
       if (n < q_rows) {
-        const int d = n % l.q_stride - l.head_dim;
-        if (d >= 0) turn(g.position + m, d, lo, hi);
+        if (dim >= 0) turn(angles(m), lo, hi);
         store8(out + row * q_rows + n, lo, hi);
       } else if (n < q_rows + g_rows) {
         store8(out2 + row * g_rows + n - q_rows, each(lo, gate), each(hi, gate));
@@ -266,17 +309,15 @@ struct Epilogue {
       float* x = g.f0 + row * g.ldo + n;
       store8(x, read4(x) + lo, read4(x + 4) + hi);
     } else if constexpr (EPI == EPI_ATTENTION_IN) {
-      const int q_rows = l.heads * l.q_stride, k_rows = l.kv_heads * l.head_dim, v_rows = l.kv_heads * l.v_dim, width = l.head_dim + l.v_dim, pos = g.position + m;
-      T* cache = static_cast<T*>(l.cache) + (static_cast<size_t>(g.slot) * l.ring + pos % l.ring) * l.kv_heads * width;
-      if (n < q_rows + k_rows) {
-        const int d = n < q_rows ? n % l.q_stride : (n - q_rows) % l.head_dim;
-        turn(pos, d, lo, hi);
-        store8(n < q_rows ? out + row * q_rows + n : cache + (n - q_rows) / l.head_dim * width + d, lo, hi);
-      } else if (n < q_rows + k_rows + v_rows) {
-        const int c = n - q_rows - k_rows;
-        store8(cache + c / l.v_dim * width + l.head_dim + c % l.v_dim, lo, hi);
+      const int q_rows = l.heads * l.q_stride, kv_rows = l.kv_heads * (l.head_dim + l.v_dim), pos = g.position + m;
+      if (dim >= 0) turn(angles(m), lo, hi);
+      if (n < q_rows) {
+        store8(out + row * q_rows + n, lo, hi);
+      } else if (n < q_rows + kv_rows) {
+        const int ring = pos < l.ring ? pos : pos % l.ring;
+        store8(static_cast<T*>(l.cache) + (static_cast<size_t>(g.slot) * l.ring + ring) * kv_rows + place, lo, hi);
       } else {
-        store8(out2 + row * l.mix_width + n - q_rows - k_rows - v_rows, each(lo, gate), each(hi, gate));
+        store8(out2 + row * l.mix_width + n - q_rows - kv_rows, each(lo, gate), each(hi, gate));
       }
     } else if constexpr (EPI == EPI_DELTA_IN) {
       const int channels = conv_channels(l), ranks = l.rank + l.gate_rank;
@@ -466,6 +507,8 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
   f32x4 *all = reinterpret_cast<f32x4*>(lds), *out = all + wave * kPassM * kQuads;
   auto place = [](int r, int quad) { return r * kQuads + (quad ^ (r & ((kQuads & -kQuads) - 1) & 15)); };      // (within a power of two that divides a row)
   const int column = n0 + wn * S::WN;
+  // (Epilogues that together grow much longer keep this compiler from unrolling the passes, which costs a third of a product's rate; passes that share their
+  // code cost 2 to 6 %.)
 #pragma unroll
   for (int pass = 0; pass < S::kPasses; ++pass) {
     const int first = m0 + wm * S::WM + pass * kPassM;
