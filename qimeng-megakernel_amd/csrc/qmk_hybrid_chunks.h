@@ -60,7 +60,8 @@ template <int KIND, int TILES>      // of a wave
 __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
   constexpr int C = kChunkTokens, kSums = KIND == CHUNK_DELTA ? 2 : 1;
   __shared__ f32x4 sums[kSums][kChunkWaves][64];
-  __shared__ float diagonal[kChunkWaves][C], norms[2][kChunkWaves][C], step[C];
+  __shared__ double diagonal[kChunkWaves][C];
+  __shared__ float norms[2][kChunkWaves][C], step[C];
   __shared__ __align__(16) float turned[kChunkWaves][C][C + 4];
   __shared__ __align__(16) float sa[C][C];
   const QmkHybridLayer& l = g.layer;
@@ -71,7 +72,7 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
 
   f32x4 q[TILES], k[TILES], w[TILES];
-  float dot = 0.f;      // of this token's q and k: where decays are strong it may be all of an output, whose norm leaves its sign, so it is taken of whole values
+  double dot = 0.;      // of this token's q and k: at a first token, or behind strong decays, it is all of an output, whose norm may leave little but its sign
   if constexpr (KIND == CHUNK_DELTA) {
     const int kv = head / (l.heads / l.kv_heads), keys = l.kv_heads * g.dim, W = conv_channels(l), taps = l.taps;
     const float* old = l.shift + (static_cast<size_t>(g.slot) * 2 + g.flip) * (taps - 1) * W;
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
       for (int i = 0; i < 4; ++i) {
         nq = fmaf(q[j][i], q[j][i], nq);
         nk = fmaf(k[j][i], k[j][i], nk);
-        dot = fmaf(q[j][i], k[j][i], dot);
+        dot = fma(static_cast<double>(q[j][i]), static_cast<double>(k[j][i]), dot);
       }
     }
     for (int tile = wave; tile * 16 < g.n; tile += kChunkWaves) {
@@ -147,7 +148,7 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
       q[j] *= iq;
       k[j] *= ik;
     }
-    dot = real ? dot * iq * ik : 0.f;
+    dot = real ? dot * iq * ik : 0.;
   } else {
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
@@ -168,7 +169,7 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
     const f32x4 bonus = KIND == CHUNK_WKV ? read4(l.vec1 + c) : one;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if constexpr (KIND != CHUNK_DELTA) dot = fmaf(q[j][i] * bonus[i], k[j][i], dot);
+      if constexpr (KIND != CHUNK_DELTA) dot = fma(static_cast<double>(q[j][i]) * bonus[i], static_cast<double>(k[j][i]), dot);
   }
   dot += __shfl_xor(dot, 16);
   dot += __shfl_xor(dot, 32);
@@ -236,12 +237,14 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
   {
     const int to = (tid >> 2) & 15, from = (tid >> 6) * 4 + (tid & 3), at = (to >> 2) * 16 + from;
     float b = 0.f, a = 0.f;
+    double d = 0.;
 #pragma unroll
     for (int i = 0; i < kChunkWaves; ++i) {
-      b += sums[0][i][at][to & 3] + (to == from ? diagonal[i][to] : 0.f);
+      b += sums[0][i][at][to & 3];
+      d += diagonal[i][to];
       if constexpr (KIND == CHUNK_DELTA) a += sums[1][i][at][to & 3];
     }
-    rb[tid] = b;
+    rb[tid] = to == from ? static_cast<float>(d) : b;      // (no pair is on the diagonal)
     if constexpr (KIND == CHUNK_DELTA) sa[to][from] = a;
   }
   if constexpr (KIND == CHUNK_DELTA) {
