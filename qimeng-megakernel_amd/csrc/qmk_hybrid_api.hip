@@ -529,6 +529,7 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
     if (g.K % 64 == 0) {
       auto direct = [&](auto s) { using S = decltype(s); launch(gemm_direct<T, S>, S::BM, S::BN, S::kThreadCount); };
       auto pipe = [&](auto s) { using S = decltype(s); launch(gemm_pipe<T, S>, S::BM, S::BN, S::kThreadCount); };
+      auto few = [&](auto s) { using S = decltype(s); launch(gemm_few<T, S>, S::BM, S::BN, S::kThreadCount); };
       auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S>, S::BM, S::BN, S::kThreadCount); };
       switch (choose_tiles(g.M, n, g.K, g.groups, g.epi == EPI_RESIDUAL)) {
         case 0: pipe(Tiles64{}); break;
@@ -542,7 +543,7 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
         case 8: turns(Turns256{}); break;
         case 9: pipe(Tiles32{}); break;
         case 10: direct(Few64{}); break;
-        default: direct(Few32{}); break;
+        default: few(Few32{}); break;
       }
       return;
     }
@@ -570,6 +571,24 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   g.splits = c.splits;
   if (c.large) launch(gemm<TA, TW, T, 128, 128, 2>, 128, 128, kPfThreads);
   else launch(gemm<TA, TW, T, 64, 64, 1>, 64, 64, kPfThreads);
+}
+
+// Two bf16 products that need nothing of each other: in one launch where both are of small tiles, whose time is mostly a launch's beginning and end (us, 443 x 2048 x 512 and
+// 2048 x 443 x 512, two launches -> one: 12.0 -> 8.4; larger tiles fill the chip by themselves).
+template <class T>
+void launch_gemm_pair(GemmPair pair, const SplitBuffers& split, hipStream_t st) {
+  auto small = [](const GemmArgs& g) { return g.groups == 1 && g.K % 64 == 0 && choose_tiles(g.M, g.N, g.K, 1, g.epi == EPI_RESIDUAL) == 0; };
+  if (!small(pair.g[0]) || !small(pair.g[1])) {
+    for (const GemmArgs& g : pair.g) launch_gemm<u16, u16, T>(g, split, st);
+    return;
+  }
+  using S = Tiles64;
+  unsigned tiles = 0;
+  for (GemmArgs& g : pair.g) {
+    g.splits = 1;
+    tiles = std::max(tiles, static_cast<unsigned>((g.N + S::BN - 1) / S::BN * ((g.M + S::BM - 1) / S::BM)));
+  }
+  hipLaunchKernelGGL((gemm_pipe_pair<T, S>), dim3(tiles, 2), dim3(S::kThreadCount), 0, st, pair);
 }
 
 // Ahead of a portion's other launches.
@@ -680,10 +699,14 @@ int prefill(const QmkHybridArgs* a) {
       hipLaunchKernelGGL(latent_rows<T>, dim3(keys), block, 0, st, b.raw, l, a->slot, first, a->position, a->eps, b.rows);
       GemmArgs k = gemm_args(whole(b.rows), width, l.uk_w, l.heads * l.head_dim, l.rank, l, EPI_STORE);
       k.M = keys; k.out = b.kn; k.ldo = l.heads * l.head_dim;
-      launch_gemm<T, u16, T>(k, b.split, st);
       GemmArgs v = gemm_args(whole(nullptr), l.rank, nullptr, keys, l.rank, l, sizeof(T) == 2 ? EPI_STORE_VALUES : EPI_STORE);   // transposed: W_uv rows x keys
       v.a = l.uv_w; v.w = b.rows; v.ldw = width; v.M = l.heads * l.v_dim; v.out = b.vt; v.ldo = cap;
-      launch_gemm<u16, T, T>(v, b.split, st);
+      if constexpr (sizeof(T) == 2) {
+        launch_gemm_pair<T>({{k, v}}, b.split, st);
+      } else {
+        launch_gemm<T, u16, T>(k, b.split, st);
+        launch_gemm<u16, T, T>(v, b.split, st);
+      }
       const Keys<T> expanded{b.kn, l.heads * l.head_dim, l.head_dim, 1};
       launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), st);
     } else {

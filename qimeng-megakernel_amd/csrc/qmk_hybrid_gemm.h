@@ -347,9 +347,10 @@ struct Epilogue {
 
 // ---- tiles ----
 // A tile is BM tokens x BN weight rows, BK columns a step; a wave owns WM x WN of it and takes all columns, one after the other.
-template <int BM_, int BN_, int BK_, int WM_, int WN_, int WAVES_, int STAGES_>
+// LOADERS: waves besides that request stages and multiply nothing.
+template <int BM_, int BN_, int BK_, int WM_, int WN_, int WAVES_, int STAGES_, int LOADERS_ = 0>
 struct Tile {
-  static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, kStages = STAGES_, kThreadCount = WAVES_ * 64;
+  static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_, kStages = STAGES_, kLoaders = LOADERS_, kThreadCount = (WAVES_ + LOADERS_) * 64;
   static constexpr int kWavesM = BM / WM, kWavesN = BN / WN;
   static constexpr int kTm = WM / 16, kTn = WN / 16;     // a wave's fragments
   static constexpr int kRow = BK / 8;                                           // a row of a step: units of 16 bytes
@@ -499,6 +500,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
   ResidualQuads<BATCH, kFewStreams> early{g};
   const bool few_streams = g.epi == EPI_RESIDUAL && g.streams <= kFewStreams;
   if (kEarly && few_streams) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(0));
+  const bool multiplies = S::kLoaders == 0 || wave < S::kWavesM * S::kWavesN;
   __syncthreads();
 #pragma unroll
   for (int c = 0; c < S::kTn * kTm; ++c) sums[c] = acc[c / kTm][c % kTm];
@@ -517,13 +519,13 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
 #pragma unroll
       for (int j = 0; j < S::kTn; ++j) {
         const int r = i * 16 + (lane & 15), quad = j * 4 + (lane >> 4);
-        out[place(r, quad)] = sums[j * kTm + pass * (kTm / S::kPasses) + i];
+        if (multiplies) out[place(r, quad)] = sums[j * kTm + pass * (kTm / S::kPasses) + i];
       }
     __builtin_amdgcn_wave_barrier();
     auto rows = [&](auto epi) {
       constexpr int kEachTime = 64 / kGroups;      // tokens (of 96 columns five, by 60 lanes)
       const int n = column + lane % kGroups * 8;
-      if (n >= N || lane >= kEachTime * kGroups) return;
+      if (n >= N || lane >= kEachTime * kGroups || !multiplies) return;
       const Epilogue<T, decltype(epi)::value> put(g, group, n);
       const int end = min(kPassM, g.M - first);
 #pragma unroll 2
@@ -615,12 +617,12 @@ __device__ __forceinline__ void wait_known() {
 // by its number on the memory side (the LDS side of such a load is one run of 64 units per wave), so that fragment reads do
 // not conflict.  A lane's places are offsets of 32 bits that stay, and one scalar moves on, so that a request is one instruction (with pointers that move on
 // it is two more).
-template <class S, int PARTS = 1>      // of the tokens' side
+template <class S, int PARTS = 1, int ISSUERS = S::kThreadCount>      // PARTS: of the tokens' side; ISSUERS: threads that request
 struct Stages {
-  static constexpr int kRowsA = S::BM * PARTS, kUnitsA = kRowsA * S::kRow, kUnits = (kRowsA + S::BN) * S::kRow, kLoads = (kUnits + S::kThreadCount - 1) / S::kThreadCount;
-  static constexpr int kLastWaves = (kUnits - (kLoads - 1) * S::kThreadCount) / 64;      // waves that take part in a stage's last load
+  static constexpr int kRowsA = S::BM * PARTS, kUnitsA = kRowsA * S::kRow, kUnits = (kRowsA + S::BN) * S::kRow, kLoads = (kUnits + ISSUERS - 1) / ISSUERS;
+  static constexpr int kLastWaves = (kUnits - (kLoads - 1) * ISSUERS) / 64;      // waves that take part in a stage's last load
   static_assert(kUnits % 64 == 0 && kUnitsA % 64 == 0, "a wave's loads are whole, and of one side");
-  static_assert(PARTS == 1 || S::BM * S::kRow % S::kThreadCount == 0, "a load is of one part");
+  static_assert(PARTS == 1 || S::BM * S::kRow % ISSUERS == 0, "a load is of one part");
   using Lds = __attribute__((address_space(3))) v4u;      // said outright: a pointer kept in a struct may become a generic one
   __amdgpu_buffer_rsrc_t a[PARTS], w;      // from the tile's first rows on: they are far less than 4 GB
   uint32_t from[kLoads], at = 0;           // this thread's places in a stage: unit i * threads + tid, tokens first; columns of the stage
@@ -638,25 +640,25 @@ struct Stages {
     w = rows(g.w, p.group * g.w_step, p.n0, g.ldw);
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
-      const int u = i * S::kThreadCount + threadIdx.x, r = u / S::kRow, c = ((u % S::kRow) ^ exchange(r)) * 8;
+      const int u = i * ISSUERS + (ISSUERS == S::kThreadCount ? static_cast<int>(threadIdx.x) : wave * 64 + static_cast<int>(threadIdx.x & 63)), r = u / S::kRow, c = ((u % S::kRow) ^ exchange(r)) * 8;
       from[i] = (r < kRowsA ? min(PARTS == 1 ? r : r % S::BM, g.M - 1 - p.m0) * g.lda + c : min(r - kRowsA, p.N - 1 - p.n0) * g.ldw + c) * 2;
     }
   }
   __device__ __forceinline__ void issue(int buf) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
-      if (i == kLoads - 1 && kLastWaves * 64 < S::kThreadCount && wave >= kLastWaves) continue;
-      auto* dst = (__attribute__((address_space(3))) uint32_t*)(lds + buf * kUnits + i * S::kThreadCount + wave * 64);
-      const bool tokens = (i + 1) * S::kThreadCount <= kUnitsA || (i * S::kThreadCount < kUnitsA && i * S::kThreadCount + wave * 64 < kUnitsA);
+      if (i == kLoads - 1 && kLastWaves * 64 < ISSUERS && wave >= kLastWaves) continue;
+      auto* dst = (__attribute__((address_space(3))) uint32_t*)(lds + buf * kUnits + i * ISSUERS + wave * 64);
+      const bool tokens = (i + 1) * ISSUERS <= kUnitsA || (i * ISSUERS < kUnitsA && i * ISSUERS + wave * 64 < kUnitsA);
       constexpr int kPart = S::BM * S::kRow;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(tokens ? a[PARTS == 1 ? 0 : min(i * S::kThreadCount / kPart, PARTS - 1)] : w, dst, 16, from[i], at, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(tokens ? a[PARTS == 1 ? 0 : min(i * ISSUERS / kPart, PARTS - 1)] : w, dst, 16, from[i], at, 0, 0);
     }
     at += S::BK * 2;
   }
   // Until at most `stages` stages of this wave's are outstanding.
   template <int stages>
   __device__ __forceinline__ void wait() const {
-    if (kLastWaves * 64 == S::kThreadCount || wave < kLastWaves) wait_known<stages * kLoads>();
+    if (kLastWaves * 64 == ISSUERS || wave < kLastWaves) wait_known<stages * kLoads>();
     else wait_known<stages * (kLoads - 1)>();
   }
   __device__ __forceinline__ void fragments(int buf, int q, int wm, int wn, Frag<u16> (&fa)[PARTS][S::kTm], Frag<u16> (&fw)[S::kTn]) const {
@@ -761,6 +763,56 @@ __global__ __launch_bounds__(S::kThreadCount, S::kThreadCount == 512 ? 4 : 1) vo
   finish_tile<T, S, S::kLds, 2>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
 
+// The same for the fewest tokens, whose workgroups have few waves that multiply: on their chain of products, fragments and barriers requests for stages take as long
+// as the products, so other waves make them.  A stage has landed for everybody behind the barrier that its loaders reach when it has landed for them; fragments of 32
+// columns are read while the 32 before are multiplied (us, the mean of 43 x 2048 x 2048 and x 6144 with the residual's streams, inside a portion: 12.0 with two waves that do both -> 10.8; four
+// loaders 10.9, three or six stages 11.5 and 11.1; the same with all weights in the last cache, so what is left is not memory's rate).
+template <class T, class S>
+__global__ __launch_bounds__(S::kThreadCount, 1) void gemm_few(const GemmArgs g) {
+  constexpr int kAhead = S::kStages - 1, kMultipliers = S::kWavesM * S::kWavesN;
+  __shared__ __align__(16) v4u lds[S::kLds + 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % S::kWavesM, wn = wave / S::kWavesM % S::kWavesN;
+  const Place p = place_of<S>(g);
+  if (p.n0 >= p.N) return;
+  Stages<S, 1, S::kLoaders * 64> stages(g, p, lds, wave - kMultipliers);
+  f32x4 acc[S::kTn][S::kTm] = {};
+  auto barrier = [] {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (wave >= kMultipliers) {
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s)
+      if (s < p.steps) stages.issue(s);
+    int buf = S::kStages - 1;
+    for (int s = 0; s < p.steps; ++s) {
+      if (s + kAhead - 1 < p.steps) stages.template wait<kAhead - 1>();
+      else wait_outstanding<0>();
+      barrier();      // stage s has landed, and stage s - 1 is no longer read
+      if (s + kAhead < p.steps) stages.issue(buf);
+      buf = buf + 1 == S::kStages ? 0 : buf + 1;
+    }
+  } else {
+    struct Fragments {
+      Frag<u16> a[1][S::kTm], w[S::kTn];
+    } f[2];
+    int buf = 0;
+    for (int s = 0; s < p.steps; ++s) {
+      wait_known<63>();      // (the last fragments of the step before)
+      barrier();
+      stages.fragments(buf, lane >> 4, wm, wn, f[0].a, f[0].w);
+#pragma unroll
+      for (int kk = 0; kk < S::kSteps; ++kk) {
+        if (kk + 1 < S::kSteps) stages.fragments(buf, (kk + 1) * 4 + (lane >> 4), wm, wn, f[(kk + 1) & 1].a, f[(kk + 1) & 1].w);
+        multiply<S, 1>(f[kk & 1].a, f[kk & 1].w, acc);
+      }
+      buf = buf + 1 == S::kStages ? 0 : buf + 1;
+    }
+  }
+  finish_tile<T, S, S::kLds, 2>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+}
+
 // Scheduling of a block of matrix instructions: one LDS read ahead of each of the first, the requests for a stage among the rest.
 template <int PRODUCTS, int READS, int REQUESTS>
 __device__ __forceinline__ void interleave() {
@@ -782,12 +834,12 @@ __device__ __forceinline__ void interleave() {
 // read into a second set of registers; one barrier a stage lies ahead of the first reads of the next one, where everybody has read the last of this one: its
 // buffer is filled again at once, kStages stages ahead.  (Launch bounds of eight waves also for four: with more registers to give away this compiler keeps
 // accumulators in the other half of the file and moves them at every step.)
-template <class T, class S, int PARTS = 1>
-__global__ __launch_bounds__(512, 2) void gemm_pipe(const GemmArgs g) {
+template <class S, int PARTS>
+constexpr int kPipeLds = S::kStages * Stages<S, PARTS>::kUnits > S::kLds ? S::kStages * Stages<S, PARTS>::kUnits : S::kLds;
+template <class T, class S, int PARTS>
+__device__ __forceinline__ void pipe_tile(const GemmArgs& g, v4u* lds) {
   static_assert(S::kSteps % 2 == 0 && S::kStages >= 2, "pairs of matrix steps a stage");
-  constexpr int kDeep = S::kStages, kProducts = PARTS * S::kTm * S::kTn, kReads = PARTS * S::kTm + S::kTn, kRequests = Stages<S, PARTS>::kLoads;
-  constexpr int kStageUnits = kDeep * Stages<S, PARTS>::kUnits, kLds = kStageUnits > S::kLds ? kStageUnits : S::kLds;
-  __shared__ __align__(16) v4u lds[kLds + 1];
+  constexpr int kDeep = S::kStages, kProducts = PARTS * S::kTm * S::kTn, kReads = PARTS * S::kTm + S::kTn, kRequests = Stages<S, PARTS>::kLoads, kLds = kPipeLds<S, PARTS>;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
   const Place p = place_of<S>(g);
@@ -852,6 +904,20 @@ __global__ __launch_bounds__(512, 2) void gemm_pipe(const GemmArgs g) {
     resolve_undefined<S>(g, p, wm, wn, acc);
   }
   finish_tile<T, S, kLds, 4>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+}
+template <class T, class S, int PARTS = 1>
+__global__ __launch_bounds__(512, 2) void gemm_pipe(const GemmArgs g) {
+  __shared__ __align__(16) v4u lds[kPipeLds<S, PARTS> + 1];
+  pipe_tile<T, S, PARTS>(g, lds);
+}
+// Two products that need nothing of each other.
+struct GemmPair {
+  GemmArgs g[2];
+};
+template <class T, class S>
+__global__ __launch_bounds__(512, 2) void gemm_pipe_pair(const GemmPair pair) {
+  __shared__ __align__(16) v4u lds[kPipeLds<S, 1> + 1];
+  pipe_tile<T, S, 1>(pair.g[blockIdx.y], lds);
 }
 
 // The same with eight waves, one workgroup a CU.  Two waves share a SIMD's matrix unit, and the halves of the workgroup take
@@ -1083,8 +1149,8 @@ __global__ __launch_bounds__(kPfThreads) void gemm_short(const GemmArgs g) {
 // ---- which tiles ----
 // (Figures here are of single launches one after another, weights from memory; inside a portion they differ by up to a fifth, qmk_hybrid_tiles.h.)
 // Few tokens: weight rows of a workgroup, deep steps, since a step's barrier and reads are most of its time (us, M x N x K, 64 x 16 in steps of 64 columns, of
-// 128, 32 x 16 in steps of 256: 43 x 2048 x 2048 with the residual's streams 12.2, 10.1, 9.5; 43 x 2048 x 6144 with them 26.4, 19.9, 17.3; the last one now 7.9 and 14.9).
-using Few32 = Tile<32, 16, 256, 16, 16, 2, 4>;
+// 128, 32 x 16 in steps of 256: 43 x 2048 x 2048 with the residual's streams 12.2, 10.1, 9.5; 43 x 2048 x 6144 with them 26.4, 19.9, 17.3; the last one now 7.9 and 14.9, and with waves that only load a tenth less).
+using Few32 = Tile<32, 16, 256, 16, 16, 2, 4, 2>;
 using Few64 = Tile<64, 16, 128, 16, 16, 4, 3>;
 using Wide64 = Tile<128, 64, 64, 32, 32, 8, 3>;
 // Below with gemm_pipe (us, M x N x K, before -> with it: 512 x 2048 x 2048 Tiles64 14.5 -> 11.8; 43 x 5696 x 2048 Tiles32 10.7 -> 9.0; 2048 x 2048 x 2048 and x 8192 Turns128, halves of the workgroup in turns, 28.5
