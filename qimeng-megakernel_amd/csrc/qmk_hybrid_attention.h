@@ -35,23 +35,29 @@ __device__ __forceinline__ float max_of_quarters(float v) {
 // are scaled down only where a maximum has moved.  us, through registers with 32 keys a step -> now: 2048 queries behind 2048 keys, 16 heads
 // of 128 | 128 212 -> 90; 1531 queries of 192 | 128, window 1024, 72 -> 33; 43 behind 400 27.7 -> 15.  Stages of 32 keys 124, 42, 16.6; of 128, 179 (one workgroup a CU);
 // 128 queries a workgroup, 32 a wave: 160, 60, 25; on eight waves 119, 42, 17.5.
-template <int QT, int VT, int KEYS, int STAGES, int WAVES_PER_SIMD>
+//
+// SHARED, for few workgroups: 16 queries a workgroup, its waves share a stage's work.  Each takes the scores of 16 of 64 keys, everybody the weights of all of them, and each
+// a quarter of a value's tiles: the same sums in the same order, a third of the fragments to read (us, 43 queries of 192 | 128 behind 400, 16 heads: 16.2 -> 13.4; with three stages
+// 13.9, so it is not the loads; three stages for 64 queries 18.7).
+template <int QT, int VT, int KEYS, int STAGES, int WAVES_PER_SIMD, bool SHARED = false>
 __global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(const u16* q, Keys<u16> keys, const u16* rows, const u16* v_t, const u16* gate, QmkHybridLayer l, int first,
                                                                              int position, int M, int keys_cap, u16* out) {
   constexpr int kRowK = QT * 4, kRowV = KEYS / 8;      // units of 16 bytes
   constexpr int kUnitsK = KEYS * kRowK, kUnits = kUnitsK + VT * 16 * kRowV;
   constexpr int kLoadsK = kUnitsK / kPfThreads, kLoads = kUnits / kPfThreads, kAhead = STAGES - 1, kSubs = KEYS / 32;
+  constexpr int kWaves = kPfThreads / 64, kQueries = SHARED ? 16 : 64, kTiles = SHARED ? VT / kWaves : VT;      // tiles of a value: of this wave
   static_assert(kLoadsK * kPfThreads == kUnitsK && kLoads * kPfThreads == kUnits, "every thread stages the same number of units");
-  __shared__ __align__(16) v4u lds[STAGES * kUnits];
+  static_assert(!SHARED || (KEYS == kWaves * 16 && VT % kWaves == 0), "a wave has 16 keys and whole tiles");
+  __shared__ __align__(16) v4u lds[STAGES * kUnits + (SHARED ? KEYS * 16 / 4 : 0)];
   using Lds = __attribute__((address_space(3))) v4u;
   Lds* const buffers = (Lds*)lds;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, col = lane & 15;
   // The longest rows of keys first, and the workgroups of one key head on one XCD where there are eight of them, so that they share its keys.
   const int kv_heads = l.heads / keys.heads_per, order = blockIdx.x % l.heads, kv = order % kv_heads, head = kv * keys.heads_per + order / kv_heads;
-  const int q0 = (gridDim.x / l.heads - 1 - blockIdx.x / l.heads) * 64;
+  const int q0 = (gridDim.x / l.heads - 1 - blockIdx.x / l.heads) * kQueries;
   const int dq = l.q_stride, width = l.rank + l.rot_dim;
-  const int lo = max(first, position + q0 + 1 - l.window);      // the first key any of the 64 queries sees
-  const int hi = min(position + q0 + 64, position + M);          // behind the last one
+  const int lo = max(first, position + q0 + 1 - l.window);      // the first key any of these queries sees
+  const int hi = min(position + q0 + kQueries, position + M);          // behind the last one
   const int begin = first + ((lo - first) & ~31), count = (hi - begin + KEYS - 1) / KEYS;
 
   // Staging: a thread has fixed places in a stage, keys first; a row's units are exchanged by its number.
@@ -100,7 +106,7 @@ __global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(con
       }
     }
   };
-  const int m = q0 + wave * 16 + col;
+  const int own_q = SHARED ? 0 : wave * 16, own_tile = SHARED ? wave * kTiles : 0, m = q0 + own_q + col;
   Frag<u16> fq[QT];
 #pragma unroll
   for (int s = 0; s < QT; ++s) {
@@ -110,38 +116,59 @@ __global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(con
 #pragma unroll
   for (int s = 0; s < kAhead; ++s)
     if (s < count) issue(s, s);
-  f32x4 acc[VT] = {};
+  f32x4 acc[kTiles] = {};
   float top = -INFINITY, sum = 0.f;
   const float scale = l.scale * kLog2e;
-  const int first_pos = position + q0 + wave * 16, last_pos = first_pos + 15, window = l.window;      // this wave's queries
+  const int first_pos = position + q0 + own_q, last_pos = first_pos + 15, window = l.window;      // this wave's queries
   // A stage of keys base .. base + KEYS - 1.  MASKED: some query does not see some of them.
   auto take = [&](auto masked, int base, const Lds* sk, const Lds* sv) {
     constexpr bool MASKED = decltype(masked)::value;
-    Frag<u16> fk[kSubs][2][QT], fv[kSubs][VT];
-#pragma unroll
-    for (int s = 0; s < QT; ++s)
+    Frag<u16> fv[kSubs][kTiles];
+    f32x4 d[kSubs][2] = {};
+    auto values = [&] {
 #pragma unroll
       for (int sub = 0; sub < kSubs; ++sub)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int r = sub * 32 + t * 16 + col;
-          fk[sub][t][s] = Frag<u16>{__builtin_bit_cast(bf16x8_t, sk[r * kRowK + ((s * 4 + g) ^ (r & 7))])};
+        for (int t = 0; t < kTiles; ++t) {
+          const int r = (own_tile + t) * 16 + col;
+          fv[sub][t] = Frag<u16>{__builtin_bit_cast(bf16x8_t, sv[r * kRowV + ((sub * 4 + g) ^ exchange_v(r))])};
         }
-    __builtin_amdgcn_sched_barrier(0);
-    f32x4 d[kSubs][2] = {};
+    };
+    auto key = [&](int r, int s) { return Frag<u16>{__builtin_bit_cast(bf16x8_t, sk[r * kRowK + ((s * 4 + g) ^ (r & 7))])}; };
+    if constexpr (SHARED) {
+      Lds* const scores = buffers + STAGES * kUnits;
+      Frag<u16> fk[QT];
 #pragma unroll
-    for (int sub = 0; sub < kSubs; ++sub)
+      for (int s = 0; s < QT; ++s) fk[s] = key(wave * 16 + col, s);
+      values();
+      f32x4 own = {};
+#pragma unroll
+      for (int s = 0; s < QT; ++s) own = mma(fk[s], fq[s], own);
+      scores[wave * 64 + lane] = __builtin_bit_cast(v4u, own);
+      wait_known<63>();      // (not for the next stage, as __syncthreads would; the scores are read before its barrier)
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int sub = 0; sub < kSubs; ++sub)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) d[sub][t] = __builtin_bit_cast(f32x4, scores[(sub * 2 + t) * 64 + lane]);
+    } else {
+      Frag<u16> fk[kSubs][2][QT];
 #pragma unroll
       for (int s = 0; s < QT; ++s)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) d[sub][t] = mma(fk[sub][t][s], fq[s], d[sub][t]);
+        for (int sub = 0; sub < kSubs; ++sub)
 #pragma unroll
-    for (int sub = 0; sub < kSubs; ++sub)
+          for (int t = 0; t < 2; ++t) fk[sub][t][s] = key(sub * 32 + t * 16 + col, s);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int t = 0; t < VT; ++t) {
-        const int r = t * 16 + col;
-        fv[sub][t] = Frag<u16>{__builtin_bit_cast(bf16x8_t, sv[r * kRowV + ((sub * 4 + g) ^ exchange_v(r))])};
-      }
+      for (int sub = 0; sub < kSubs; ++sub)
+#pragma unroll
+        for (int s = 0; s < QT; ++s)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) d[sub][t] = mma(fk[sub][t][s], fq[s], d[sub][t]);
+      values();
+    }
 #pragma unroll
     for (int sub = 0; sub < kSubs; ++sub, base += 32) {
       if (MASKED && (base >= hi || base > last_pos || first_pos - (base + 31) >= window)) continue;      // 32 keys that no query of this wave sees
@@ -173,10 +200,10 @@ __global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(con
       top = best;
       if (!__all(shrink == 1.f)) {
 #pragma unroll
-        for (int t = 0; t < VT; ++t) acc[t] = acc[t] * shrink;
+        for (int t = 0; t < kTiles; ++t) acc[t] = acc[t] * shrink;
       }
 #pragma unroll
-      for (int t = 0; t < VT; ++t) {
+      for (int t = 0; t < kTiles; ++t) {
         Frag<u16> f = fv[sub][t];
         if (MASKED && base + 32 > hi) {      // whatever the buffer holds behind the last key must not enter a sum
           v4u bits = __builtin_bit_cast(v4u, f.v);
@@ -211,8 +238,10 @@ __global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(con
   const float inv = 1.f / sum;
   const size_t o = static_cast<size_t>(m) * l.heads * l.v_dim + head * l.v_dim;
 #pragma unroll
-  for (int t = 0; t < VT; ++t)
-    if (t * 16 < l.v_dim) store4(out + o + t * 16 + g * 4, acc[t] * inv * read4(gate + o + t * 16 + g * 4));
+  for (int t = 0; t < kTiles; ++t) {
+    const int at = (own_tile + t) * 16 + g * 4;
+    if (at < l.v_dim) store4(out + o + at, acc[t] * inv * read4(gate + o + at));
+  }
 }
 
 }  // namespace hybrid
