@@ -603,6 +603,8 @@ void begin_portion(const SplitBuffers& split, hipStream_t st) {
 // In bf16 heads of 128 and of 192 share a stage's work among the waves of 16 queries while such workgroups do not outnumber the CUs (us, 16 heads behind 400 keys, a wave's queries by
 // themselves -> shared: 192 | 128, 43 tokens 16.2 -> 13.4, 200 tokens 19.3 -> 16.3, 500 tokens 25.6 -> 32.4, 1000 tokens 36.1 -> 79.6; 128 | 128, 20 tokens 16.6 -> 11.8,
 // 200 tokens 19.0 -> 14.8, 500 tokens 25.4 -> 21.2, 1000 tokens 35.1 -> 46.9).
+// In fp32 the same heads take few_attention up to there (us, 16 heads, window_attention -> few_attention: 192 | 128, 43 tokens 16.1 -> 12.2, 200 tokens 30.0 -> 20.7, 400 tokens 50.2 -> 55.8;
+// 128 | 128 behind 200 keys, 43 tokens 29.2 -> 19.0, 400 tokens 58.6 -> 63.2).
 template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
                       hipStream_t st) {
@@ -617,12 +619,17 @@ void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* 
     else if (l.q_stride <= 192 && l.v_dim <= 128) rows_of(attention_rows<6, 8, 64, 2, 1, true>, attention_rows<6, 8, 64, 2, 2>);
     else launch(attention_rows<8, 16, 32, 3, 1>, 64);
   } else {
+    const int few_runs = (a->tokens + 15) / 16;
+    auto launch_few = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(few_runs, l.heads), dim3(kPfThreads), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
+    };
     auto launch = [&](auto kernel, int groups) {
       hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
     };
+    const bool few = few_runs * l.heads <= 256;
     if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<4, 4, 2>, 2);
-    else if (l.q_stride <= 128 && l.v_dim <= 128) launch(window_attention<4, 8, 2>, 2);
-    else if (l.q_stride <= 192 && l.v_dim <= 128) launch(window_attention<6, 8, 2>, 2);
+    else if (l.q_stride <= 128 && l.v_dim <= 128) few ? launch_few(few_attention<4, 8>) : launch(window_attention<4, 8, 2>, 2);
+    else if (l.q_stride <= 192 && l.v_dim <= 128) few ? launch_few(few_attention<6, 8>) : launch(window_attention<6, 8, 2>, 2);
     else launch(window_attention<8, 16, 1>, 1);
   }
 }

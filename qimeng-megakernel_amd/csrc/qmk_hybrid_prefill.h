@@ -361,6 +361,149 @@ __global__ __launch_bounds__(kPfThreads * GROUPS) void window_attention(const fl
     if (t < vt) put4(out, at + t * 16 + g * 4, acc[t] * inv * read4(gate + at + t * 16 + g * 4));
 }
 
+// The same for few workgroups: 16 queries of a head, whose four waves take the 32-key steps in turn and meet at the end.  A step's keys and values have one reader, so they go from
+// memory to its registers, the next step's keys behind the scores and its values behind the sums; what bounds it is the fp32 matrix instruction, 160 a step of 192 | 128 (us,
+// 16 heads, 64 queries a workgroup -> now: 200 of 192 | 128 30.0 -> 20.7, behind 400 keys 69.5 -> 45.6).
+template <int QT, int VT>
+__global__ __launch_bounds__(kPfThreads, 1) void few_attention(const float* q, Keys<float> keys, const float* rows, const float* v_t, const float* gate, QmkHybridLayer l, int first,
+                                                               int position, int M, int keys_cap, Operand<float> out) {
+  constexpr int kKeys = 32, kWaves = kPfThreads / 64, kTiles = VT / kWaves;      // tiles of a value a wave finishes
+  static_assert(VT % kWaves == 0, "whole tiles");
+  __shared__ f32x4 box[kWaves][VT][64];
+  __shared__ float tops[kWaves][64], sums[kWaves][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, col = lane & 15;
+  const int head = blockIdx.y, kv = head / keys.heads_per, q0 = blockIdx.x * 16, m = q0 + col, pos = position + m;
+  const int dq = l.q_stride, steps = dq / 32, vt = l.v_dim / 16, width = l.rank + l.rot_dim;
+  const int lo = max(first, position + q0 + 1 - l.window), hi = min(position + q0 + 16, position + M);      // keys that any of these queries sees
+  const int begin = first + ((lo - first) & ~(kKeys - 1));
+  const float* zeros = reinterpret_cast<const float*>(kZeroUnit);
+  f32x4 k[2][QT][2], v[VT][2];
+  auto load_keys = [&](int base) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int row = min(base + t * 16 + col, hi - 1) - first;      // (keys behind the last one are that one again, and masked)
+      const float* at = keys.at + static_cast<size_t>(row) * keys.pitch + kv * keys.head;
+      const float* turned = rows + static_cast<size_t>(row) * width + l.rank - l.head_dim;
+#pragma unroll
+      for (int s = 0; s < QT; ++s)
+        if (s < steps) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int c = s * 32 + g * 8 + u * 4;
+            k[t][s][u] = read4(c < l.head_dim ? at + c : rows != nullptr && c < l.head_dim + l.rot_dim ? turned + c : zeros);
+          }
+        }
+    }
+  };
+  auto load_values = [&](int base) {
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+      if (t < vt) {
+        const float* at = v_t + static_cast<size_t>(kv * l.v_dim + t * 16 + col) * keys_cap - first;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int key = base + u * 16 + g * 4;
+          v[t][u] = read4(key < hi ? at + key : zeros);
+        }
+      }
+  };
+  Frag<float> fq[QT];
+#pragma unroll
+  for (int s = 0; s < QT; ++s)
+    if (s < steps) fq[s] = load_frag(q + static_cast<size_t>(min(m, M - 1)) * l.heads * dq + head * dq + s * 32 + g * 8);
+  f32x4 acc[VT] = {};
+  float top = -INFINITY, sum = 0.f;
+  const float scale = l.scale * kLog2e;
+  const int own = begin + wave * kKeys;
+  if (own < hi) {
+    load_keys(own);
+    load_values(own);
+  }
+  for (int base = own; base < hi; base += kWaves * kKeys) {
+    f32x4 d[2] = {};
+#pragma unroll
+    for (int s = 0; s < QT; ++s)
+      if (s < steps) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          Frag<float> f;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) f.set(j, k[t][s][j >> 2][j & 3]);
+          d[t] = mma(f, fq[s], d[t]);
+        }
+      }
+    const int next = base + kWaves * kKeys;
+    if (next < hi) load_keys(next);
+    float w[8], best = top;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = d[j >> 2][j & 3] * scale;
+    if (base + kKeys - 1 > position + q0 || position + q0 + 15 - base >= l.window) {   // some query does not see some key
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int dist = pos - (base + (j >> 2) * 16 + g * 4 + (j & 3));
+        if (dist < 0 || dist >= l.window) w[j] = -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) best = fmaxf(best, w[j]);
+    best = fmaxf(best, __shfl_xor(best, 16));
+    best = fmaxf(best, __shfl_xor(best, 32));
+    const float ref = best == -INFINITY ? 0.f : best;      // no key of this query yet
+    const float shrink = exp2_fast(top - ref);
+    float step_sum = 0.f;
+    Frag<float> fp;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      w[j] = exp2_fast(w[j] - ref);
+      step_sum += w[j];
+      fp.set(j, w[j]);
+    }
+    sum = sum * shrink + step_sum;
+    top = best;
+    const bool last = base + kKeys > hi;
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+      if (t < vt) {
+        Frag<float> f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {      // keys behind the last one: whatever the buffer holds there must not enter a sum
+          const float x = v[t][j >> 2][j & 3];
+          f.set(j, last && base + (j >> 2) * 16 + g * 4 + (j & 3) >= hi ? 0.f : x);
+        }
+        acc[t] = mma(f, fp, acc[t] * shrink);
+      }
+    if (next < hi) load_values(next);
+  }
+  sum += __shfl_xor(sum, 16);
+  sum += __shfl_xor(sum, 32);
+  tops[wave][lane] = top;
+  sums[wave][lane] = sum;
+#pragma unroll
+  for (int t = 0; t < VT; ++t) box[wave][t][lane] = acc[t];
+  __syncthreads();
+  if (m >= M) return;
+  float most = -INFINITY, part[kWaves], total = 0.f;
+#pragma unroll
+  for (int p = 0; p < kWaves; ++p) most = fmaxf(most, tops[p][lane]);
+  const float ref = most == -INFINITY ? 0.f : most;
+#pragma unroll
+  for (int p = 0; p < kWaves; ++p) {
+    part[p] = exp2_fast(tops[p][lane] - ref);
+    total += sums[p][lane] * part[p];
+  }
+  const float inv = 1.f / total;
+  const size_t at = static_cast<size_t>(m) * l.heads * l.v_dim + head * l.v_dim;
+#pragma unroll
+  for (int i = 0; i < kTiles; ++i) {
+    const int t = wave * kTiles + i;
+    if (t >= vt) continue;
+    f32x4 o = {};
+#pragma unroll
+    for (int p = 0; p < kWaves; ++p) o += box[p][t][lane] * part[p];
+    put4(out, at + t * 16 + g * 4, o * inv * read4(gate + at + t * 16 + g * 4));
+  }
+}
+
 // Per-head norm, weight and gate behind the recurrence: one wave per (token, head).
 template <class T>
 __global__ __launch_bounds__(kPfThreads) void wkv_out(const float* o, const T* gate, QmkHybridLayer l, int M, float eps, Operand<T> out) {
