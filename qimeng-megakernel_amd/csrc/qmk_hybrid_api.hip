@@ -1,8 +1,8 @@
 // The hybrid route's kernels for gfx950 and their C ABI (include/qmk_hybrid.h).
 //
-// Decode: the persistent interpreter of the other routes (one workgroup per instruction queue, monotone counters with
+// Decode: the persistent interpreter of the other routes (one workgroup per instruction queue, tagged units and, for attention parts, counters with
 // bounded waits, the last workgroup to retire clears them) over the ops of qmk_hybrid_ops.h.  Prefill: the launches of
-// qmk_hybrid_prefill.h, layer by layer, on the caller's stream.
+// qmk_hybrid_prefill.h, qmk_hybrid_plain.h and qmk_hybrid_chunks.h, layer by layer, on the caller's stream.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
