@@ -600,11 +600,12 @@ void begin_portion(const SplitBuffers& split, hipStream_t st) {
 // rows: where the rotated part of a latent attention's keys is, behind the latent.  In fp32 two groups of waves share a workgroup's queries, except for
 // the largest heads, where they take 140 KB of LDS and more registers than there are (us a portion of one layer, 16 heads of 256 | 256, one group -> two:
 // 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508).  In bf16 the largest heads leave no registers for a second wave a SIMD, and take stages of 32 keys.
-// In bf16 heads of 128 and of 192 share a stage's work among the waves of 16 queries while such workgroups do not outnumber the CUs (us, 16 heads behind 400 keys, a wave's queries by
-// themselves -> shared: 192 | 128, 43 tokens 16.2 -> 13.4, 200 tokens 19.3 -> 16.3, 500 tokens 25.6 -> 32.4, 1000 tokens 36.1 -> 79.6; 128 | 128, 20 tokens 16.6 -> 11.8,
-// 200 tokens 19.0 -> 14.8, 500 tokens 25.4 -> 21.2, 1000 tokens 35.1 -> 46.9).
-// In fp32 the same heads take few_attention up to there (us, 16 heads, window_attention -> few_attention: 192 | 128, 43 tokens 16.1 -> 12.2, 200 tokens 30.0 -> 20.7, 400 tokens 50.2 -> 55.8;
-// 128 | 128 behind 200 keys, 43 tokens 29.2 -> 19.0, 400 tokens 58.6 -> 63.2).
+// In bf16 heads of 128 and of 192 share a stage's work among the waves of 16 queries while such workgroups are all on the chip at once, two a CU of 128 and one of 192 (us, 16 heads behind
+// 400 keys, a wave's queries by themselves -> shared: 192 | 128, 43 tokens 16.2 -> 13.4, 200 tokens 19.3 -> 16.3, 500 tokens 25.6 -> 32.4; 128 | 128, 20 tokens 16.6 -> 11.8,
+// 200 tokens 19.0 -> 14.8, 500 tokens 25.4 -> 21.2, 1000 tokens 35.1 -> 46.9; behind 1000 keys 192 | 128, 43 tokens 28.2 -> 24.3, 250 tokens 32.0 -> 27.9; 128 | 128, 43 tokens 27.6 -> 22.2,
+// 250 tokens 31.2 -> 26.0, 500 tokens 35.9 -> 33.3).
+// In fp32 the same heads take few_attention with one a CU (us, 16 heads, window_attention -> few_attention: 192 | 128, 43 tokens 16.1 -> 12.2, 200 tokens 30.0 -> 20.7, 400 tokens 50.2 -> 55.8;
+// behind 1000 keys 250 tokens 133 -> 83; 128 | 128 behind 200 keys, 43 tokens 29.2 -> 19.0, 400 tokens 58.6 -> 63.2, behind 1000 keys 250 tokens 113 -> 72).
 template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
                       hipStream_t st) {
@@ -612,11 +613,10 @@ void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* 
     auto launch = [&](auto kernel, int queries) {
       hipLaunchKernelGGL(kernel, dim3((a->tokens + queries - 1) / queries * l.heads), dim3(kPfThreads), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out.at);
     };
-    const bool few = (a->tokens + 15) / 16 * l.heads <= 256;
-    auto rows_of = [&](auto shared, auto all) { few ? launch(shared, 16) : launch(all, 64); };
+    auto rows_of = [&](auto shared, auto all, int a_cu) { (a->tokens + 15) / 16 * l.heads <= 256 * a_cu ? launch(shared, 16) : launch(all, 64); };
     if (l.q_stride <= 128 && l.v_dim <= 64) launch(attention_rows<4, 4, 64, 2, 2>, 64);
-    else if (l.q_stride <= 128 && l.v_dim <= 128) rows_of(attention_rows<4, 8, 64, 2, 2, true>, attention_rows<4, 8, 64, 2, 2>);
-    else if (l.q_stride <= 192 && l.v_dim <= 128) rows_of(attention_rows<6, 8, 64, 2, 1, true>, attention_rows<6, 8, 64, 2, 2>);
+    else if (l.q_stride <= 128 && l.v_dim <= 128) rows_of(attention_rows<4, 8, 64, 2, 2, true>, attention_rows<4, 8, 64, 2, 2>, 2);
+    else if (l.q_stride <= 192 && l.v_dim <= 128) rows_of(attention_rows<6, 8, 64, 2, 1, true>, attention_rows<6, 8, 64, 2, 2>, 1);
     else launch(attention_rows<8, 16, 32, 3, 1>, 64);
   } else {
     const int few_runs = (a->tokens + 15) / 16;
