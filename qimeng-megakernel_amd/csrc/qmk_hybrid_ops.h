@@ -1546,6 +1546,8 @@ __device__ __forceinline__ bool op_attend(const DecodeParams& p, Smem& s, const 
       rest.wait(p, s, o, tag);
       put_queries();
     }
+  } else {      // No keys.  What it leaves all the same takes the place of parts that the attention before may still be merging: every query comes behind that.
+    unit_of(p, s, o, latent ? p.absorbed + head0 * per_a : p.proj + l.proj_at + head0 * per_b, tag);
   }
   if (p.timeline != nullptr && tid == 0) s.t_wait = wall_clock64();
 
