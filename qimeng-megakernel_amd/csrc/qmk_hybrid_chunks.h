@@ -208,9 +208,12 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
       }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)      // row (later token) quad 4 + i, column (earlier one) t: of one block of 2h
+    for (int i = 0; i < 4; ++i) {      // row (later token) r, column (earlier one) t: of one block of 2h.  All others are zeros, also where an operand is not finite
+      const int r = quad * 4 + i;
+      const bool pair = (r ^ t) < 2 * h && (r & ~t & h) != 0;
 #pragma unroll
-      for (int e = 0; e < kSums; ++e) pairs[e][i] += ((quad * 4 + i) ^ t) < 2 * h ? p[e][i] : 0.f;
+      for (int e = 0; e < kSums; ++e) pairs[e][i] += pair ? p[e][i] : 0.f;
+    }
   };
   level(std::integral_constant<int, 1>{}, std::integral_constant<int, kDppQuadXor1>{});
   level(std::integral_constant<int, 2>{}, std::integral_constant<int, kDppQuadXor2>{});
@@ -368,10 +371,28 @@ __global__ __launch_bounds__(kPfThreads, TILES == 16 ? 1 : 2) void segment_scan(
     const f32x4 u = {value[quad * 256], value[quad * 256 + 64], value[quad * 256 + 128], value[quad * 256 + 192]};
     auto fragment = [&](const Lds* at) { return __builtin_bit_cast(f32x4, at[lane]); };
     if constexpr (OUT) {
-      f32x4 o[2] = {};
+      // A value that is not finite reaches its own token and later ones alone: above B's diagonal it would meet zeros.
+      f32x4 o[2] = {}, finite = u;
+      bool whole = true;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) whole = whole && __builtin_isfinite(u[i]);
+      if (!__all(whole)) {
+        const auto* pair = (const __attribute__((address_space(3))) float*)b;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) finite[i] = __builtin_isfinite(u[i]) ? u[i] : 0.f;
+#pragma unroll 1
+        for (int from = 0; from < kChunkTokens; ++from) {
+          const float v = value[from * 64];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int t = quad * 4 + i;
+            if (from <= t && !__builtin_isfinite(v)) o[1][i] += pair[((from >> 2) * 16 + t) * 4 + (from & 3)] * v;
+          }
+        }
+      }
 #pragma unroll
       for (int j = 0; j < TILES; ++j) o[j & 1] = product(fragment(q + j * 64), s[j], o[j & 1]);
-      o[1] = product(fragment(b), u, o[1]);
+      o[1] = product(fragment(b), finite, o[1]);
       o[0] += o[1];
       if (mine) {
         const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, extent(chunk, out_ld));

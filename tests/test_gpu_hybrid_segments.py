@@ -55,3 +55,29 @@ def test_portions(name, dtype):
         d = d - d.mean(-1, keepdim=True)
         err = float((d.pow(2).mean(-1).sqrt() / want.pow(2).mean().sqrt()).max())
         assert err < TOLERANCE[oracle, dtype], f"{n} tokens: {err:.3g}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("n, at", [(40, 20), (40, 39), (330, 261)], ids=["inside a chunk", "the last token", "a later segment"])
+@pytest.mark.parametrize("what", ["gla, undefined embedding", "wkv, undefined embedding", "wkv, infinite embedding", "wkv, infinite keys", "wkv, infinite values"])
+def test_a_token_that_is_not_finite_reaches_none_before_it(what, n, at, dtype):
+    kind, what = what.split(", ")
+    shape = SHAPES["wkv 80" if kind == "wkv" else "gla 64 | 80"]
+    w = synthetic.random_hybrid_weights(shape, 5)
+    if what.endswith("embedding"):
+        w["embed"][7, 3] = float("nan" if what.startswith("undefined") else "inf")
+    else:       # a column of the weights that this token alone meets
+        w["embed"][:, 3] = 0
+        w["embed"][7] = 0
+        w["embed"][7, 3] = 1
+        w["l0.mix." + what.split()[1][0]][:, 3] = 3e38
+    g = build_globals(shape, weights.pack(shape, w, DEVICE), dtype=dtype, max_positions=MOST, portion_rows=640)
+    mk, ids, got = mk_kernel.get_mk(), torch.arange(n) % 6, []
+    for token in (5, 7):
+        ids[at] = token
+        table = RequestTable(g)
+        got.append(decode_hybrid.run_tokens(g, mk, table.open(0), ids, range(n)))
+        table.close(0)
+    mk.check()
+    assert torch.isfinite(got[0]).all() and torch.equal(got[0][:at], got[1][:at])
+    assert not torch.isfinite(got[1][at:]).any(dim=-1).any()
