@@ -269,7 +269,9 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
 // Sixteen value columns a wave, all key channels; one segment and head a workgroup.  A chunk's record goes from memory to LDS by itself while the one before is
 // multiplied: the state's tiles are the matrix instruction's accumulators and at the same time the second operand of the products that read them, and nothing is
 // exchanged between waves.  OUT: from the segment's start, with outputs, and the last segment leaves the portion's state; otherwise from nothing, for what it
-// leaves.  What bounds it is the fp32 matrix instruction (68 of 43 cycles a chunk and wave, 36 without outputs) and, where a launch begins, all its workgroups' first loads (12 us of
+// leaves.  What a chunk adds to a state is summed by itself, so that the state is rounded once a chunk and not with every product (error against 64 bits, the state
+// as the products' own accumulator -> so: 640 tokens without decay 2.9e-7 -> 1.1e-7; a first wkv state of the 2b shape behind 200 tokens in fp32, beside token after token, x 1.012 -> x 0.991).
+// What bounds it is the fp32 matrix instruction (of eight tiles 68 of 32 cycles a chunk and wave, 32 without outputs) and, where a launch begins, all its workgroups' first loads (12 us of
 // 29).  us in whole portions, chunks one after the other with keys split over waves -> three launches side by side: 2048 tokens of 8 heads of 128 | 256 68 -> 29 + 17 + 8, 1531 of 32
 // heads of 64 (wkv, before: token by token, with chunk_prepare's 16) 117 -> 17 + 10 + 5 + 16.  Segments of 16 chunks: 33 + 19 + 6 and 20 + 12 + 5.
 template <int TILES, bool OUT>
@@ -372,7 +374,7 @@ __global__ __launch_bounds__(kPfThreads, TILES == 16 ? 1 : 2) void segment_scan(
     auto fragment = [&](const Lds* at) { return __builtin_bit_cast(f32x4, at[lane]); };
     if constexpr (OUT) {
       // A value that is not finite reaches its own token and later ones alone: above B's diagonal it would meet zeros.
-      f32x4 o[2] = {}, finite = u;
+      f32x4 o[4] = {}, own = {}, finite = u;
       bool whole = true;
 #pragma unroll
       for (int i = 0; i < 4; ++i) whole = whole && __builtin_isfinite(u[i]);
@@ -386,14 +388,14 @@ __global__ __launch_bounds__(kPfThreads, TILES == 16 ? 1 : 2) void segment_scan(
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int t = quad * 4 + i;
-            if (from <= t && !__builtin_isfinite(v)) o[1][i] += pair[((from >> 2) * 16 + t) * 4 + (from & 3)] * v;
+            if (from <= t && !__builtin_isfinite(v)) own[i] += pair[((from >> 2) * 16 + t) * 4 + (from & 3)] * v;
           }
         }
       }
 #pragma unroll
-      for (int j = 0; j < TILES; ++j) o[j & 1] = product(fragment(q + j * 64), s[j], o[j & 1]);
-      o[1] = product(fragment(b), finite, o[1]);
-      o[0] += o[1];
+      for (int j = 0; j < TILES; ++j) o[j & 3] = product(fragment(q + j * 64), s[j], o[j & 3]);
+      own = product(fragment(b), finite, own);
+      o[0] = ((o[0] + o[1]) + (o[2] + o[3])) + own;
       if (mine) {
         const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, extent(chunk, out_ld));
 #pragma unroll
@@ -404,7 +406,9 @@ __global__ __launch_bounds__(kPfThreads, TILES == 16 ? 1 : 2) void segment_scan(
     for (int j = 0; j < TILES; ++j) {
       const f32x4 g4 = __builtin_bit_cast(f32x4, decay[j * 4 + quad]);
       if constexpr (!OUT) fade[j] *= g4;
-      s[j] = product(fragment(d + j * 64), u, s[j] * g4);
+      const f32x4 added = product(fragment(d + j * 64), u, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[j][i] = fmaf(s[j][i], g4[i], added[i]);
     }
   }
   if (!mine) return;

@@ -81,3 +81,27 @@ def test_a_token_that_is_not_finite_reaches_none_before_it(what, n, at, dtype):
     mk.check()
     assert torch.isfinite(got[0]).all() and torch.equal(got[0][:at], got[1][:at])
     assert not torch.isfinite(got[1][at:]).any(dim=-1).any()
+
+
+@pytest.mark.parametrize("n", [250, 640])
+def test_states_that_do_not_fade_are_summed_by_chunks(n):
+    """A state of n tokens without decay.  A sum by tokens is rounded n times, each time by up to half a last place (2^-24 / sqrt 3 evenly spread, three quarters of it on the average
+    place between two powers of two: 2.6e-8) of the sum so far: sqrt(n / 2) x 2.6e-8 of the last one.  A sum by chunks of sixteen tokens is rounded a sixteenth as often, so a quarter as
+    far; keys and values bring up to 1e-7."""
+    shape = synthetic.hybrid_shape("w", width=128, vocab=96, streams=1, wkv_heads=2, wkv_dim=64, wkv_rank=16)
+    w, ids = synthetic.random_hybrid_weights(shape, 2), torch.randint(0, 96, (n,), generator=torch.Generator().manual_seed(8))
+    w["l0.mix.w2"].zero_()
+    w["l0.mix.w0"].fill_(-30)      # decays of one, to 1e-13
+    g = build_globals(shape, weights.pack(shape, w, DEVICE), dtype=torch.float32, max_positions=MOST, portion_rows=640)
+    mk, request = mk_kernel.get_mk(), RequestTable(g).open(0)
+    decode_hybrid.run_tokens(g, mk, request, ids)
+    mk.check()
+    d = {name: t.double() for name, t in w.items()}
+    x = d["embed"][ids] * d["l0.hc1.in"]
+    h = x / torch.sqrt((x * x).mean(-1, keepdim=True) + shape.eps) * d["l0.norm1"]
+    before = torch.cat((torch.zeros_like(h[:1]), h[:-1]))
+    k, v = (((h + (before - h) * d["l0.mix.mu." + c]) @ d["l0.mix." + c].T).view(n, 2, 64) for c in "kv")
+    want = torch.stack([k[:, head].T @ v[:, head] for head in range(2)])
+    got = g.layer_state[0]["state"][0].double().cpu().view_as(want)
+    err = float((got - want).norm() / want.norm())
+    assert err < 1e-7 + 0.25 * (n / 2) ** 0.5 * 2.6e-8, f"{err:.3g}"
