@@ -372,43 +372,57 @@ __global__ __launch_bounds__(kPfThreads, TILES == 16 ? 1 : 2) void segment_scan(
     const auto* value = (const __attribute__((address_space(3))) float*)(stages + c % kStages * kStage + kValues) + wave * 16 + col;
     const f32x4 u = {value[quad * 256], value[quad * 256 + 64], value[quad * 256 + 128], value[quad * 256 + 192]};
     auto fragment = [&](const Lds* at) { return __builtin_bit_cast(f32x4, at[lane]); };
+    f32x4 fq[OUT ? TILES : 1], fd[TILES], faded[TILES], fb, o[4] = {}, finite = u;
+    bool whole = true;
     if constexpr (OUT) {
-      // A value that is not finite reaches its own token and later ones alone: above B's diagonal it would meet zeros.
-      f32x4 o[4] = {}, own = {}, finite = u;
-      bool whole = true;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) whole = whole && __builtin_isfinite(u[i]);
-      if (!__all(whole)) {
+      for (int j = 0; j < TILES; ++j) fq[j] = fragment(q + j * 64);
+      fb = fragment(b);
+    }
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      fd[j] = fragment(d + j * 64);
+      faded[j] = __builtin_bit_cast(f32x4, decay[j * 4 + quad]);
+    }
+    __builtin_amdgcn_sched_barrier(0);      // (all fragments are asked for ahead of the products: read between them, they wait for registers)
+    if constexpr (OUT) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        whole = whole && __builtin_isfinite(u[i]);
+        finite[i] = __builtin_isfinite(u[i]) ? u[i] : 0.f;
+      }
+#pragma unroll
+      for (int j = 0; j < TILES; ++j) o[j & 3] = product(fq[j], s[j], o[j & 3]);
+      o[0] = ((o[0] + o[1]) + (o[2] + o[3])) + product(fb, finite, f32x4{0.f, 0.f, 0.f, 0.f});
+    }
+    f32x4 added[TILES];
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) added[j] = product(fd[j], u, f32x4{0.f, 0.f, 0.f, 0.f});
+    if constexpr (!OUT) __builtin_amdgcn_sched_barrier(0);      // (nothing else is left to do while a product is waited for)
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      if constexpr (!OUT) fade[j] *= faded[j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[j][i] = fmaf(s[j][i], faded[j][i], added[j][i]);
+    }
+    if constexpr (OUT) {      // (branches behind all products, which are scheduled together)
+      if (!__all(whole)) {      // A value that is not finite reaches its own token and later ones alone: above B's diagonal it would meet zeros.
         const auto* pair = (const __attribute__((address_space(3))) float*)b;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) finite[i] = __builtin_isfinite(u[i]) ? u[i] : 0.f;
 #pragma unroll 1
         for (int from = 0; from < kChunkTokens; ++from) {
           const float v = value[from * 64];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int t = quad * 4 + i;
-            if (from <= t && !__builtin_isfinite(v)) own[i] += pair[((from >> 2) * 16 + t) * 4 + (from & 3)] * v;
+            if (from <= t && !__builtin_isfinite(v)) o[0][i] += pair[((from >> 2) * 16 + t) * 4 + (from & 3)] * v;
           }
         }
       }
-#pragma unroll
-      for (int j = 0; j < TILES; ++j) o[j & 3] = product(fragment(q + j * 64), s[j], o[j & 3]);
-      own = product(fragment(b), finite, own);
-      o[0] = ((o[0] + o[1]) + (o[2] + o[3])) + own;
       if (mine) {
         const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, extent(chunk, out_ld));
 #pragma unroll
         for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[0][i]), to, ((quad * 4 + i) * out_ld + col) * 4, 0, 0);
       }
-    }
-#pragma unroll
-    for (int j = 0; j < TILES; ++j) {
-      const f32x4 g4 = __builtin_bit_cast(f32x4, decay[j * 4 + quad]);
-      if constexpr (!OUT) fade[j] *= g4;
-      const f32x4 added = product(fragment(d + j * 64), u, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-      for (int i = 0; i < 4; ++i) s[j][i] = fmaf(s[j][i], g4[i], added[i]);
     }
   }
   if (!mine) return;
