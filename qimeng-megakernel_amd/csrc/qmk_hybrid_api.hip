@@ -573,8 +573,9 @@ void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   else launch(gemm<TA, TW, T, 64, 64, 1>, 64, 64, kPfThreads);
 }
 
-// Two bf16 products that need nothing of each other: in one launch where both are of small tiles, whose time is mostly a launch's beginning and end (us, 443 x 2048 x 512 and
-// 2048 x 443 x 512, two launches -> one: 12.0 -> 8.4; larger tiles fill the chip by themselves).
+// Two bf16 products that need nothing of each other: in one launch where both take tiles of 64 x 64, whose time is mostly a launch's beginning and end (us, 443 x 2048 x 512 and
+// 2048 x 443 x 512, two launches -> one: 12.0 -> 8.4; larger tiles fill the chip by themselves; the kinds for fewer tokens, as of a short portion with nothing before it, stay two launches:
+// not tried).
 template <class T>
 void launch_gemm_pair(GemmPair pair, const SplitBuffers& split, hipStream_t st) {
   auto small = [](const GemmArgs& g) { return g.groups == 1 && g.K % 64 == 0 && choose_tiles(g.M, g.N, g.K, 1, g.epi == EPI_RESIDUAL) == 0; };
@@ -603,9 +604,11 @@ void begin_portion(const SplitBuffers& split, hipStream_t st) {
 // In bf16 heads of 128 and of 192 share a stage's work among the waves of 16 queries while such workgroups are all on the chip at once, two a CU of 128 and one of 192 (us, 16 heads behind
 // 400 keys, a wave's queries by themselves -> shared: 192 | 128, 43 tokens 16.2 -> 13.4, 200 tokens 19.3 -> 16.3, 500 tokens 25.6 -> 32.4; 128 | 128, 20 tokens 16.6 -> 11.8,
 // 200 tokens 19.0 -> 14.8, 500 tokens 25.4 -> 21.2, 1000 tokens 35.1 -> 46.9; behind 1000 keys 192 | 128, 43 tokens 28.2 -> 24.3, 250 tokens 32.0 -> 27.9; 128 | 128, 43 tokens 27.6 -> 22.2,
-// 250 tokens 31.2 -> 26.0, 500 tokens 35.9 -> 33.3).
+// 250 tokens 31.2 -> 26.0, 500 tokens 35.9 -> 33.3; behind 4000 and 16000 keys 128 | 128, 260 tokens 81 -> 74 and 284 -> 262, 500 tokens 88 -> 84 and 291 -> 287; 192 | 128, 250 tokens 86 -> 80 and
+// 297 -> 281: keys are read four times as often, but out of the caches).
 // In fp32 the same heads take few_attention with one a CU (us, 16 heads, window_attention -> few_attention: 192 | 128, 43 tokens 16.1 -> 12.2, 200 tokens 30.0 -> 20.7, 400 tokens 50.2 -> 55.8;
-// behind 1000 keys 250 tokens 133 -> 83; 128 | 128 behind 200 keys, 43 tokens 29.2 -> 19.0, 400 tokens 58.6 -> 63.2, behind 1000 keys 250 tokens 113 -> 72).
+// behind 1000 keys 250 tokens 133 -> 83, behind 16000 1641 -> 1027; 128 | 128 behind 200 keys, 43 tokens 29.2 -> 19.0, 400 tokens 58.6 -> 63.2, behind 1000 keys 250 tokens 113 -> 72, behind
+// 16000 1294 -> 796).
 template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
                       hipStream_t st) {

@@ -27,7 +27,8 @@ constexpr int kPartialUnits = 256 * 128 * 128 / 4;     // quads its parts leave:
 // Tiles32 16.7; 520 x 2048 x 6144 with them Tiles64 41.9, Wide64 47.0; 1024 x 2048 x 6144 with them Wide64 54.6, Turns96 56.5, Tiles64 64.8; 520 x 12288 x 2048 Wide256 31.8, Turns128 36.2;
 // 1531 x 2048 x 2048 with them Turns96 33.6, Turns128 36.8, Wide64 42.6; 2048 x 2048 x 2048 with them Turns128 42.8, Tall192 49.1, Wide64 53.2; 1531 x 2048 x 8192 with them Turns96 72.6,
 // Turns128 84.6; 3000 x 2048 x 8192 Tall192 97.8, Tall256 111.5; 1531 x 16384 x 2048 Tall256 94.9, Wide256 100.1; 2048 x 16384 x 2048 Turns256 123.2, Tall256 125.4.
-// Memory is not priced: it bounds all kinds alike where there are many rows for few tokens.
+// Memory is not priced: it bounds all kinds alike where there are many rows for few tokens.  Two kinds of launches have become a tenth faster since the fit and were not fitted again: Few32 (with waves that
+// only load) is priced too dear, products into an attention in all kinds.
 struct TileCost {
   int most_tokens, bm, bn, bk, a_cu;
   double step, fixed, overlapped, streams;

@@ -7,7 +7,9 @@ number and number of parts for opcode 4).
 
 A step is a chain of stages; ``wait_stage`` (-1: none) is the one an instruction depends on, ``wait_count`` the number of its
 instructions, ``arrive_stage`` its own.  The kernel hands values over as tagged units, which carry the order themselves; only
-the parts of an attention, and what shares their stage, count an arrival each, for which the opcodes that merge them wait.
+the parts of an attention, and the state steps and output gates that may share their stage, count an arrival each, for which the
+opcodes that merge the parts wait (where a stage has no part nobody waits; ``wait_stage`` of the other opcodes is what an error names).  So whoever writes a buffer must come behind all that
+reads what was there through the units that it has waited for itself, parts without keys included.
 Stage s is counted in group ``s // 4`` of ``barriers`` on counter row ``2 + s % 4`` of
 the dense route's layout, one line per XCD.
 """
@@ -50,8 +52,7 @@ class GatedRecurrence(StageInstruction):
 
 @dataclass
 class LatentAbsorb(StageInstruction):
-    """``extra`` = 1: the stage's leading instruction (which no longer does more than the others: the attention's parts that
-    hold the step's position make and append the cache row)."""
+    """Rows of W_uk^T q of one head.  ``extra`` = 1 marks the stage's first one; the kernel does not read it."""
     OPCODE: ClassVar[int] = 3
 
 
