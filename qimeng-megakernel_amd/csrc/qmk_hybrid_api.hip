@@ -598,46 +598,7 @@ void begin_portion(const SplitBuffers& split, hipStream_t st) {
   if constexpr (sizeof(T) == 4) hipLaunchKernelGGL(clear_tickets, dim3(1), dim3(kPfThreads), 0, st, split.tickets, kMaxTickets);
 }
 
-// rows: where the rotated part of a latent attention's keys is, behind the latent.  In fp32 two groups of waves share a workgroup's queries, except for
-// the largest heads, where they take 140 KB of LDS and more registers than there are (us a portion of one layer, 16 heads of 256 | 256, one group -> two:
-// 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508).  In bf16 the largest heads leave no registers for a second wave a SIMD, and take stages of 32 keys.
-// In bf16 heads of 128 and of 192 share a stage's work among the waves of 16 queries while such workgroups are all on the chip at once, two a CU of 128 and one of 192 (us, 16 heads behind
-// 400 keys, a wave's queries by themselves -> shared: 192 | 128, 43 tokens 16.2 -> 13.4, 200 tokens 19.3 -> 16.3, 500 tokens 25.6 -> 32.4; 128 | 128, 20 tokens 16.6 -> 11.8,
-// 200 tokens 19.0 -> 14.8, 500 tokens 25.4 -> 21.2, 1000 tokens 35.1 -> 46.9; behind 1000 keys 192 | 128, 43 tokens 28.2 -> 24.3, 250 tokens 32.0 -> 27.9; 128 | 128, 43 tokens 27.6 -> 22.2,
-// 250 tokens 31.2 -> 26.0, 500 tokens 35.9 -> 33.3; behind 4000 and 16000 keys 128 | 128, 260 tokens 81 -> 74 and 284 -> 262, 500 tokens 88 -> 84 and 291 -> 287; 192 | 128, 250 tokens 86 -> 80 and
-// 297 -> 281: keys are read four times as often, but out of the caches).
-// In fp32 the same heads take few_attention with one a CU (us, 16 heads, window_attention -> few_attention: 192 | 128, 43 tokens 16.1 -> 12.2, 200 tokens 30.0 -> 20.7, 400 tokens 50.2 -> 55.8;
-// behind 1000 keys 250 tokens 133 -> 83, behind 16000 1641 -> 1027; 128 | 128 behind 200 keys, 43 tokens 29.2 -> 19.0, 400 tokens 58.6 -> 63.2, behind 1000 keys 250 tokens 113 -> 72, behind
-// 16000 1294 -> 796).
-template <class T>
-void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
-                      hipStream_t st) {
-  if constexpr (sizeof(T) == 2) {
-    auto launch = [&](auto kernel, int queries) {
-      hipLaunchKernelGGL(kernel, dim3((a->tokens + queries - 1) / queries * l.heads), dim3(kPfThreads), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out.at);
-    };
-    auto rows_of = [&](auto shared, auto all, int a_cu) { (a->tokens + 15) / 16 * l.heads <= 256 * a_cu ? launch(shared, 16) : launch(all, 64); };
-    if (l.q_stride <= 128 && l.v_dim <= 64) launch(attention_rows<4, 4, 64, 2, 2>, 64);
-    else if (l.q_stride <= 128 && l.v_dim <= 128) rows_of(attention_rows<4, 8, 64, 2, 2, true>, attention_rows<4, 8, 64, 2, 2>, 2);
-    else if (l.q_stride <= 192 && l.v_dim <= 128) rows_of(attention_rows<6, 8, 64, 2, 1, true>, attention_rows<6, 8, 64, 2, 2>, 1);
-    else launch(attention_rows<8, 16, 32, 3, 1>, 64);
-  } else {
-    const int few_runs = (a->tokens + 15) / 16;
-    auto launch_few = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(few_runs, l.heads), dim3(kPfThreads), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
-    };
-    auto launch = [&](auto kernel, int groups) {
-      hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
-    };
-    const bool few = few_runs * l.heads <= 256;
-    if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<4, 4, 2>, 2);
-    else if (l.q_stride <= 128 && l.v_dim <= 128) few ? launch_few(few_attention<4, 8>) : launch(window_attention<4, 8, 2>, 2);
-    else if (l.q_stride <= 192 && l.v_dim <= 128) few ? launch_few(few_attention<6, 8>) : launch(window_attention<6, 8, 2>, 2);
-    else launch(window_attention<8, 16, 1>, 1);
-  }
-}
-
-// A recurrence over the portion, from its projections to what its norm reads.
+// A recurrence over the portion, from its projections to what its norm reads; of the delta rule all but its scan.
 template <class T, int KIND>
 void run_chunks(ChunkArgs g, hipStream_t st) {
   g.segment = segment_chunks<T>(g.M);
@@ -646,9 +607,7 @@ void run_chunks(ChunkArgs g, hipStream_t st) {
     constexpr int kTiles = decltype(wave_tiles)::value;
     const dim3 block(kPfThreads);
     hipLaunchKernelGGL((chunk_prepare<KIND, kTiles>), dim3(chunks, g.heads), block, 0, st, g);
-    if constexpr (KIND == CHUNK_DELTA) {
-      hipLaunchKernelGGL((chunk_scan<kTiles, 4>), dim3(g.heads, g.n / 16), block, 0, st, g);
-    } else {
+    if constexpr (KIND != CHUNK_DELTA) {
       const unsigned groups = g.heads * ((g.n + 63) / 64);
       if (segments > 1) {
         hipLaunchKernelGGL((segment_scan<kTiles * 4, false>), dim3(groups * (segments - 1)), block, 0, st, g);
@@ -661,6 +620,70 @@ void run_chunks(ChunkArgs g, hipStream_t st) {
     case 4: return run(std::integral_constant<int, 1>{});
     case 8: return run(std::integral_constant<int, 2>{});
     default: return run(std::integral_constant<int, 4>{});
+  }
+}
+
+// The delta rule's chunks one after the other.
+inline void launch_scan(const ChunkArgs& g, hipStream_t st) {
+  auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(g.heads, g.n / 16), dim3(kPfThreads), 0, st, g); };
+  switch (chunk_tiles(g.dim)) {
+    case 4: return run(chunk_scan<1, kChunkWaves>);
+    case 8: return run(chunk_scan<2, kChunkWaves>);
+    default: return run(chunk_scan<4, kChunkWaves>);
+  }
+}
+
+// rows: where the rotated part of a latent attention's keys is, behind the latent.  In fp32 two groups of waves share a workgroup's queries, except for
+// the largest heads, where they take 140 KB of LDS and more registers than there are (us a portion of one layer, 16 heads of 256 | 256, one group -> two:
+// 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508).  In bf16 the largest heads leave no registers for a second wave a SIMD, and take stages of 32 keys.
+// In bf16 heads of 128 and of 192 share a stage's work among the waves of 16 queries while such workgroups are all on the chip at once, two a CU of 128 and one of 192 (us, 16 heads behind
+// 400 keys, a wave's queries by themselves -> shared: 192 | 128, 43 tokens 16.2 -> 13.4, 200 tokens 19.3 -> 16.3, 500 tokens 25.6 -> 32.4; 128 | 128, 20 tokens 16.6 -> 11.8,
+// 200 tokens 19.0 -> 14.8, 500 tokens 25.4 -> 21.2, 1000 tokens 35.1 -> 46.9; behind 1000 keys 192 | 128, 43 tokens 28.2 -> 24.3, 250 tokens 32.0 -> 27.9; 128 | 128, 43 tokens 27.6 -> 22.2,
+// 250 tokens 31.2 -> 26.0, 500 tokens 35.9 -> 33.3; behind 4000 and 16000 keys 128 | 128, 260 tokens 81 -> 74 and 284 -> 262, 500 tokens 88 -> 84 and 291 -> 287; 192 | 128, 250 tokens 86 -> 80 and
+// 297 -> 281: keys are read four times as often, but out of the caches).
+// In fp32 the same heads take few_attention with one a CU (us, 16 heads, window_attention -> few_attention: 192 | 128, 43 tokens 16.1 -> 12.2, 200 tokens 30.0 -> 20.7, 400 tokens 50.2 -> 55.8;
+// behind 1000 keys 250 tokens 133 -> 83, behind 16000 1641 -> 1027; 128 | 128 behind 200 keys, 43 tokens 29.2 -> 19.0, 400 tokens 58.6 -> 63.2, behind 1000 keys 250 tokens 113 -> 72, behind
+// 16000 1294 -> 796).
+// `beside`: a delta rule whose chunks are prepared; they are walked in the same launch where a CU holds a workgroup of either, ahead of it where not (us, 2048 tokens of 16 heads, behind
+// nothing and behind 2048 keys, two launches -> one: XX).
+template <class T>
+void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
+                      const ChunkArgs* beside, hipStream_t st) {
+  if constexpr (sizeof(T) == 2) {
+    const AttentionArgs args{q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out.at};
+    auto workgroups = [&](int queries) { return static_cast<unsigned>((a->tokens + queries - 1) / queries * l.heads); };
+    if (beside != nullptr && l.q_stride <= 128 && l.v_dim <= 128 && chunk_tiles(beside->dim) <= 8) {
+      auto both = [&](auto one_tile, auto two_tiles, int queries) {
+        const dim3 grid(beside->heads * (beside->n / 16) + workgroups(queries));
+        if (chunk_tiles(beside->dim) == 4) hipLaunchKernelGGL(one_tile, grid, dim3(kPfThreads), 0, st, *beside, args);
+        else hipLaunchKernelGGL(two_tiles, grid, dim3(kPfThreads), 0, st, *beside, args);
+      };
+      if (l.v_dim <= 64) both(scan_and_attend<1, 4, 4, 64, 2, false>, scan_and_attend<2, 4, 4, 64, 2, false>, 64);
+      else if (workgroups(16) <= 512) both(scan_and_attend<1, 4, 8, 64, 2, true>, scan_and_attend<2, 4, 8, 64, 2, true>, 16);
+      else both(scan_and_attend<1, 4, 8, 64, 2, false>, scan_and_attend<2, 4, 8, 64, 2, false>, 64);
+      return;
+    }
+    if (beside != nullptr) launch_scan(*beside, st);
+    auto launch = [&](auto kernel, int queries) { hipLaunchKernelGGL(kernel, dim3(workgroups(queries)), dim3(kPfThreads), 0, st, args); };
+    auto rows_of = [&](auto shared, auto all, int a_cu) { workgroups(16) <= 256u * a_cu ? launch(shared, 16) : launch(all, 64); };
+    if (l.q_stride <= 128 && l.v_dim <= 64) launch(attention_rows<4, 4, 64, 2, 2>, 64);
+    else if (l.q_stride <= 128 && l.v_dim <= 128) rows_of(attention_rows<4, 8, 64, 2, 2, true>, attention_rows<4, 8, 64, 2, 2>, 2);
+    else if (l.q_stride <= 192 && l.v_dim <= 128) rows_of(attention_rows<6, 8, 64, 2, 1, true>, attention_rows<6, 8, 64, 2, 2>, 1);
+    else launch(attention_rows<8, 16, 32, 3, 1>, 64);
+  } else {
+    if (beside != nullptr) launch_scan(*beside, st);
+    const int few_runs = (a->tokens + 15) / 16;
+    auto launch_few = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(few_runs, l.heads), dim3(kPfThreads), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
+    };
+    auto launch = [&](auto kernel, int groups) {
+      hipLaunchKernelGGL(kernel, dim3((a->tokens + 63) / 64, l.heads), dim3(kPfThreads * groups), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
+    };
+    const bool few = few_runs * l.heads <= 256;
+    if (l.q_stride <= 128 && l.v_dim <= 64) launch(window_attention<4, 4, 2>, 2);
+    else if (l.q_stride <= 128 && l.v_dim <= 128) few ? launch_few(few_attention<4, 8>) : launch(window_attention<4, 8, 2>, 2);
+    else if (l.q_stride <= 192 && l.v_dim <= 128) few ? launch_few(few_attention<6, 8>) : launch(window_attention<6, 8, 2>, 2);
+    else launch(window_attention<8, 16, 1>, 1);
   }
 }
 
@@ -722,7 +745,7 @@ int prefill(const QmkHybridArgs* a) {
         launch_gemm<u16, T, T>(v, b.split, st);
       }
       const Keys<T> expanded{b.kn, l.heads * l.head_dim, l.head_dim, 1};
-      launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), st);
+      launch_attention<T>(a, l, b.p0, expanded, b.rows, b.vt, b.p1, first, cap, b.mix.of(W), nullptr, st);
     } else {
       const int N = W;
       hipLaunchKernelGGL(shift_mix<T>, dim3(M), block, 0, st, b.u, l, a->slot, a->flip, M, P, D, a->width_true, a->eps, b.h.of(D));
@@ -778,6 +801,69 @@ int prefill_plain(const QmkHybridArgs* a) {
     return g;
   };
   auto whole = [](T* rows) { return Operand<T>{rows, 0}; };
+  auto project_attention = [&](const QmkHybridLayer& l) {
+    GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_ATTENTION_IN);
+    g.out = b.q; g.out2 = b.gate;
+    launch_gemm<T, u16, T>(g, b.split, st);
+  };
+  auto attend = [&](const QmkHybridLayer& l, const ChunkArgs* beside) {
+    const int row = l.head_dim + l.v_dim, pitch = l.kv_heads * row, keys = a->position + M, cap = static_cast<int>(values_cap(a));
+    const T* cache = static_cast<const T*>(l.cache) + static_cast<size_t>(a->slot) * l.ring * pitch;
+    hipLaunchKernelGGL(transpose_values<T>, dim3((keys + 63) / 64, (l.v_dim + 63) / 64, l.kv_heads), block, 0, st, cache, pitch, row, l.head_dim, l.v_dim, keys, cap, b.vt);
+    launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix.of(l.mix_width), beside, st);
+  };
+  auto chunk_args = [&](const QmkHybridLayer& l) {
+    ChunkArgs c{};
+    c.layer = l; c.decay = b.decay; c.chunks = b.state.chunks; c.starts = b.state.starts; c.fades = b.state.fades; c.out = b.o;
+    c.M = M; c.heads = l.heads; c.dim = l.head_dim; c.n = l.v_dim; c.slot = a->slot; c.flip = a->flip;
+    return c;
+  };
+  auto decays = [&](const QmkHybridLayer& l, int ld, int epi) {
+    const int keys = l.heads * l.head_dim;
+    GemmArgs e = gemm_args(whole(b.low), l.mid_w, keys, l.rank, l, epi);
+    e.lda = ld; e.f0 = b.decay; e.ldo = keys;
+    launch_gemm<T, u16, T>(e, b.split, st);
+  };
+  // A delta rule up to its scan.  Writes nothing that an attention beside it reads: its output gate, which lies where the attention's does, comes behind.
+  auto prepare_delta = [&](const QmkHybridLayer& l) {
+    const int beta_ld = (l.heads + 15) / 16 * 16;
+    GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_DELTA_IN);
+    g.f1 = b.qkv; g.out2 = b.low; g.f0 = b.beta; g.ldo = beta_ld;
+    launch_gemm<T, u16, T>(g, b.split, st);
+    decays(l, l.rank + l.gate_rank, EPI_DELTA_DECAY);
+    ChunkArgs c = chunk_args(l);
+    c.q = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = l.mix_width;
+    run_chunks<T, CHUNK_DELTA>(c, st);
+    return c;
+  };
+  auto state_rows = [&](const QmkHybridLayer& l) {
+    hipLaunchKernelGGL(state_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.o, b.gate, l, M, a->eps, b.mix.of(l.mix_width));
+  };
+  auto finish_delta = [&](const QmkHybridLayer& l) {
+    const int channels = conv_channels(l), W = l.mix_width;
+    GemmArgs f = gemm_args(whole(b.low + l.rank), l.gate_w, W, l.gate_rank, l, EPI_SIGMOID);
+    f.lda = l.rank + l.gate_rank; f.out = b.gate; f.ldo = W;
+    launch_gemm<T, u16, T>(f, b.split, st);
+    if (l.taps > 1)
+      hipLaunchKernelGGL(keep_inputs, dim3((channels + kPfThreads - 1) / kPfThreads), block, 0, st, b.qkv, l, channels, a->slot, a->flip, M);
+    state_rows(l);
+  };
+  auto run_gla = [&](const QmkHybridLayer& l) {
+    const int W = l.mix_width, keys = l.heads * l.head_dim;
+    GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_GLA_IN);
+    g.f0 = b.qkv; g.out = b.gate; g.out2 = b.low;
+    launch_gemm<T, u16, T>(g, b.split, st);
+    decays(l, l.rank, EPI_GLA_DECAY);
+    ChunkArgs c = chunk_args(l);
+    c.q = b.qkv; c.k = b.qkv + keys; c.values = b.qkv; c.ld = c.value_ld = 2 * keys + W; c.value_at = 2 * keys;
+    run_chunks<T, CHUNK_GLA>(c, st);
+    state_rows(l);
+  };
+  auto project_out = [&](const QmkHybridLayer& l) {
+    GemmArgs o = gemm_args(b.mix.of(l.mix_width), l.o_w, D, l.mix_width, l, l.branches > 1 ? EPI_LOGITS : EPI_ADD);
+    o.f0 = l.branches > 1 ? b.branch + l.branch * rows : b.x;
+    launch_gemm<T, u16, T>(o, b.split, st);
+  };
   int runs_done = 0;
   // x as entry l reads it: its norm (or [x; embedding]) -> h; `want`: of those rows alone, x stays.
   auto residual = [&](const QmkHybridLayer& l, const int32_t* want, int count, bool added, float* dump) {
@@ -796,7 +882,6 @@ int prefill_plain(const QmkHybridArgs* a) {
   };
   for (int i = 0; i < a->num_layers; ++i) {
     const QmkHybridLayer& l = a->layers[i];
-    const int W = l.mix_width;
     if (l.type == QMK_ENTRY_FINAL) {
       float* dump = dump_of(l);
       if (dump != nullptr) residual(l, nullptr, M, true, dump);     // (and x is complete)
@@ -816,49 +901,18 @@ int prefill_plain(const QmkHybridArgs* a) {
       continue;
     }
     if (l.type == QMK_MIXER_ATTENTION) {
-      GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_ATTENTION_IN);
-      g.out = b.q; g.out2 = b.gate;
-      launch_gemm<T, u16, T>(g, b.split, st);
-      const int row = l.head_dim + l.v_dim, pitch = l.kv_heads * row, keys = a->position + M, cap = static_cast<int>(values_cap(a));
-      const T* cache = static_cast<const T*>(l.cache) + static_cast<size_t>(a->slot) * l.ring * pitch;
-      hipLaunchKernelGGL(transpose_values<T>, dim3((keys + 63) / 64, (l.v_dim + 63) / 64, l.kv_heads), block, 0, st, cache, pitch, row, l.head_dim, l.v_dim, keys, cap, b.vt);
-      launch_attention<T>(a, l, b.q, Keys<T>{cache, pitch, row, l.heads / l.kv_heads}, nullptr, b.vt, b.gate, 0, cap, b.mix.of(W), st);
+      project_attention(l);
+      // Beside a delta rule: its chunks are prepared first, since its scan leaves room on the chip for the attention.
+      const bool beside = l.branch + 1 < l.branches && a->layers[i + 1].type == QMK_MIXER_DELTA;
+      const ChunkArgs c = beside ? prepare_delta(a->layers[i + 1]) : ChunkArgs{};
+      attend(l, beside ? &c : nullptr);
+    } else if (l.type == QMK_MIXER_DELTA) {
+      if (l.branch == 0 || a->layers[i - 1].type != QMK_MIXER_ATTENTION) launch_scan(prepare_delta(l), st);
+      finish_delta(l);
     } else {
-      ChunkArgs c{};
-      c.layer = l; c.decay = b.decay; c.chunks = b.state.chunks; c.starts = b.state.starts; c.fades = b.state.fades; c.out = b.o;
-      c.M = M; c.heads = l.heads; c.dim = l.head_dim; c.n = l.v_dim; c.slot = a->slot; c.flip = a->flip;
-      if (l.type == QMK_MIXER_DELTA) {
-        const int channels = conv_channels(l), ranks = l.rank + l.gate_rank, beta_ld = (l.heads + 15) / 16 * 16;
-        GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_DELTA_IN);
-        g.f1 = b.qkv; g.out2 = b.low; g.f0 = b.beta; g.ldo = beta_ld;
-        launch_gemm<T, u16, T>(g, b.split, st);
-        const int keys = l.heads * l.head_dim;
-        GemmArgs e = gemm_args(whole(b.low), l.mid_w, keys, l.rank, l, EPI_DELTA_DECAY);
-        e.lda = ranks; e.f0 = b.decay; e.ldo = keys;
-        launch_gemm<T, u16, T>(e, b.split, st);
-        GemmArgs f = gemm_args(whole(b.low + l.rank), l.gate_w, W, l.gate_rank, l, EPI_SIGMOID);
-        f.lda = ranks; f.out = b.gate; f.ldo = W;
-        launch_gemm<T, u16, T>(f, b.split, st);
-        c.q = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = W;
-        run_chunks<T, CHUNK_DELTA>(c, st);
-        if (l.taps > 1)
-          hipLaunchKernelGGL(keep_inputs, dim3((channels + kPfThreads - 1) / kPfThreads), block, 0, st, b.qkv, l, channels, a->slot, a->flip, M);
-      } else {
-        const int keys = l.heads * l.head_dim;
-        GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_GLA_IN);
-        g.f0 = b.qkv; g.out = b.gate; g.out2 = b.low;
-        launch_gemm<T, u16, T>(g, b.split, st);
-        GemmArgs e = gemm_args(whole(b.low), l.mid_w, keys, l.rank, l, EPI_GLA_DECAY);
-        e.f0 = b.decay; e.ldo = keys;
-        launch_gemm<T, u16, T>(e, b.split, st);
-        c.q = b.qkv; c.k = b.qkv + keys; c.values = b.qkv; c.ld = c.value_ld = 2 * keys + W; c.value_at = 2 * keys;
-        run_chunks<T, CHUNK_GLA>(c, st);
-      }
-      hipLaunchKernelGGL(state_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.o, b.gate, l, M, a->eps, b.mix.of(W));
+      run_gla(l);
     }
-    GemmArgs o = gemm_args(b.mix.of(W), l.o_w, D, W, l, l.branches > 1 ? EPI_LOGITS : EPI_ADD);
-    o.f0 = l.branches > 1 ? b.branch + l.branch * rows : b.x;
-    launch_gemm<T, u16, T>(o, b.split, st);
+    project_out(l);
     if (l.branch + 1 == l.branches) {
       const QmkHybridLayer& head = a->layers[i - l.branch];
       if (head.has_mlp) {

@@ -39,22 +39,37 @@ __device__ __forceinline__ float max_of_quarters(float v) {
 // SHARED, for few workgroups: 16 queries a workgroup, its waves share a stage's work.  Each takes the scores of 16 of 64 keys, everybody the weights of all of them, and each
 // a quarter of a value's tiles: the same sums in the same order, a third of the fragments to read (us, 43 queries of 192 | 128 behind 400, 16 heads: 16.2 -> 13.4; with three stages
 // 13.9, so it is not the loads; three stages for 64 queries 18.7).
-template <int QT, int VT, int KEYS, int STAGES, int WAVES_PER_SIMD, bool SHARED = false>
-__global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(const u16* q, Keys<u16> keys, const u16* rows, const u16* v_t, const u16* gate, QmkHybridLayer l, int first,
-                                                                             int position, int M, int keys_cap, u16* out) {
+struct AttentionArgs {
+  const u16* q;
+  Keys<u16> keys;
+  const u16 *rows, *v_t, *gate;
+  QmkHybridLayer layer;
+  int first, position, M, keys_cap;
+  u16* out;
+};
+template <int QT, int VT, int KEYS, int STAGES, bool SHARED>
+constexpr int kAttentionLds = STAGES * (KEYS * QT * 4 + VT * 2 * KEYS) + (SHARED ? KEYS * 16 / 4 : 0);
+// Workgroup `block` of `blocks`.
+template <int QT, int VT, int KEYS, int STAGES, bool SHARED>
+__device__ __forceinline__ void attend_rows(const AttentionArgs& a, int block, int blocks, v4u* lds) {
+  const u16 *q = a.q, *rows = a.rows, *v_t = a.v_t, *gate = a.gate;
+  u16* out = a.out;
+  const Keys<u16>& keys = a.keys;
+  const QmkHybridLayer& l = a.layer;
+  const int first = a.first, position = a.position, M = a.M, keys_cap = a.keys_cap;
   constexpr int kRowK = QT * 4, kRowV = KEYS / 8;      // units of 16 bytes
   constexpr int kUnitsK = KEYS * kRowK, kUnits = kUnitsK + VT * 16 * kRowV;
   constexpr int kLoadsK = kUnitsK / kPfThreads, kLoads = kUnits / kPfThreads, kAhead = STAGES - 1, kSubs = KEYS / 32;
   constexpr int kWaves = kPfThreads / 64, kQueries = SHARED ? 16 : 64, kTiles = SHARED ? VT / kWaves : VT;      // tiles of a value: of this wave
   static_assert(kLoadsK * kPfThreads == kUnitsK && kLoads * kPfThreads == kUnits, "every thread stages the same number of units");
   static_assert(!SHARED || (KEYS == kWaves * 16 && VT % kWaves == 0), "a wave has 16 keys and whole tiles");
-  __shared__ __align__(16) v4u lds[STAGES * kUnits + (SHARED ? KEYS * 16 / 4 : 0)];
+  static_assert(kAttentionLds<QT, VT, KEYS, STAGES, SHARED> == STAGES * kUnits + (SHARED ? KEYS * 16 / 4 : 0), "its stages and shared scores");
   using Lds = __attribute__((address_space(3))) v4u;
   Lds* const buffers = (Lds*)lds;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, col = lane & 15;
   // The longest rows of keys first, and the workgroups of one key head on one XCD where there are eight of them, so that they share its keys.
-  const int kv_heads = l.heads / keys.heads_per, order = blockIdx.x % l.heads, kv = order % kv_heads, head = kv * keys.heads_per + order / kv_heads;
-  const int q0 = (gridDim.x / l.heads - 1 - blockIdx.x / l.heads) * kQueries;
+  const int kv_heads = l.heads / keys.heads_per, order = block % l.heads, kv = order % kv_heads, head = kv * keys.heads_per + order / kv_heads;
+  const int q0 = (blocks / l.heads - 1 - block / l.heads) * kQueries;
   const int dq = l.q_stride, width = l.rank + l.rot_dim;
   const int lo = max(first, position + q0 + 1 - l.window);      // the first key any of these queries sees
   const int hi = min(position + q0 + kQueries, position + M);          // behind the last one
@@ -242,6 +257,11 @@ __global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(con
     const int at = (own_tile + t) * 16 + g * 4;
     if (at < l.v_dim) store4(out + o + at, acc[t] * inv * read4(gate + o + at));
   }
+}
+template <int QT, int VT, int KEYS, int STAGES, int WAVES_PER_SIMD, bool SHARED = false>
+__global__ __launch_bounds__(kPfThreads, WAVES_PER_SIMD) void attention_rows(const AttentionArgs a) {
+  __shared__ __align__(16) v4u lds[kAttentionLds<QT, VT, KEYS, STAGES, SHARED>];
+  attend_rows<QT, VT, KEYS, STAGES, SHARED>(a, blockIdx.x, gridDim.x, lds);
 }
 
 }  // namespace hybrid

@@ -493,13 +493,14 @@ __global__ __launch_bounds__(kPfThreads) void segment_starts(const ChunkArgs g) 
 // A wave's instructions are on that chain too, one wave a SIMD: chunks are read and written by buffer accesses (places of 32 bits that stay, bases that move on by
 // one scalar addition, tokens behind the last one read as zero and not written).  us, 2048 tokens of 16 heads of 128 | 128, addresses of 64 bits worked out for every
 // access -> now 134 -> 120; lines of chunks further ahead asked for into L2: 141.
-template <int TILES, int WAVES>
-__global__ __launch_bounds__(WAVES * 64, 1) void chunk_scan(const ChunkArgs g) {
-  // Chunks in flight: what the registers hold (us, the shape above, with 2, 3 and 4 ahead: 131, 120, 123).
-  constexpr int kAhead = TILES == 1 ? 4 : TILES == 2 ? 3 : 2;
-  __shared__ f32x4 px[2][WAVES][64], po[2][WAVES][64];
+template <int WAVES>
+constexpr int kScanLds = 4 * WAVES * 64;
+// Chunks in flight: what the registers hold (us, the shape above, with 2, 3 and 4 ahead: 131, 120, 123).
+template <int TILES, int WAVES, int kAhead = TILES == 1 ? 4 : TILES == 2 ? 3 : 2>
+__device__ __forceinline__ void scan_chunks(const ChunkArgs& g, int head, int v0, f32x4* lds) {
+  auto px = reinterpret_cast<f32x4(*)[WAVES][64]>(lds), po = px + 2;
   const QmkHybridLayer& l = g.layer;
-  const int dim = g.dim, n = g.n, head = blockIdx.x, v0 = blockIdx.y * 16;
+  const int dim = g.dim, n = g.n;
   constexpr int tiles = TILES * WAVES;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, quad = lane >> 4;
   const int tile0 = wave * TILES, mine = min(max(dim / 16 - tile0, 0), TILES);
@@ -614,6 +615,28 @@ __global__ __launch_bounds__(WAVES * 64, 1) void chunk_scan(const ChunkArgs g) {
     if (j < mine)
 #pragma unroll
       for (int i = 0; i < 4; ++i) state[static_cast<size_t>((tile0 + j) * 16 + quad * 4 + i) * n] = s[j][i];
+}
+template <int TILES, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 1) void chunk_scan(const ChunkArgs g) {
+  __shared__ __align__(16) f32x4 lds[kScanLds<WAVES>];
+  scan_chunks<TILES, WAVES>(g, blockIdx.x, blockIdx.y * 16, lds);
+}
+
+// The two branches of a run need nothing of each other, and the delta rule's chunks are a chain of instructions on a part of the chip: its workgroups come first, and go first on their SIMDs, an
+// attention's fill what is left (us, 2048 tokens of 16 heads of 128 | 128 in either, behind nothing and behind 2048 keys, two launches -> one: 118 + 47 -> 129, 119 + 93 -> 150).  Registers
+// for two workgroups a CU leave room for two chunks in flight of two tiles a wave.
+template <int TILES, int QT, int VT, int KEYS, int STAGES, bool SHARED>
+__global__ __launch_bounds__(kPfThreads, 2) void scan_and_attend(const ChunkArgs c, const AttentionArgs a) {
+  constexpr int kUnits = kAttentionLds<QT, VT, KEYS, STAGES, SHARED>;
+  static_assert(kUnits >= kScanLds<kChunkWaves>, "one array for either");
+  __shared__ __align__(16) v4u lds[kUnits];
+  const int scans = c.heads * (c.n / 16), id = blockIdx.x;
+  if (id < scans) {
+    __builtin_amdgcn_s_setprio(3);
+    scan_chunks<TILES, kChunkWaves, TILES == 1 ? 4 : 2>(c, id % c.heads, id / c.heads * 16, reinterpret_cast<f32x4*>(lds));
+  } else {
+    attend_rows<QT, VT, KEYS, STAGES, SHARED>(a, id - scans, gridDim.x - scans, lds);
+  }
 }
 
 }  // namespace hybrid

@@ -168,6 +168,27 @@ def test_each_mechanism_alone(part, ff, loop):
     assert torch.all(out[:, :, shape.width:] == 0)
 
 
+@pytest.mark.parametrize("tokens", [2, 33, 530], ids=["one chunk", "few queries share", "64 queries a workgroup"])
+@pytest.mark.parametrize("v_dim", [40, 120], ids=["values up to 64", "values up to 128"])
+@pytest.mark.parametrize("delta_dim", [50, 100], ids=["one tile a wave", "two tiles a wave"])
+def test_both_branches_in_one_launch(delta_dim, v_dim, tokens):
+    """Every kind of launch that walks a delta rule's chunks beside an attention (bf16), at both lines of its choice."""
+    shape = synthetic.looped_shape("pp", width=64, vocab=70, ff={"p": 40}, heads=16, kv_heads=4, dim=72, v_dim=v_dim, rot_dim=16, delta_heads=3, delta_kv_heads=3,
+                                   delta_dim=delta_dim, delta_v_dim=40, taps=3, delta_rank=8, gate_rank=6)
+    w = synthetic.random_hybrid_weights(shape, 4)
+    layers, ids = [], tokens_of(shape, tokens)
+    want = O.forward(shape.to_config(), w, torch.tensor(ids), dtype=torch.float64, layer_outputs=layers)
+    g, mk = on_gpu(shape, w, torch.bfloat16, max_positions=540, portion_rows=540), mk_kernel.get_mk()
+    request = RequestTable(g).open("y")
+    g.slot, g.position_id, g.flip = request.slot, 0, 0
+    out = torch.zeros(shape.run_count, tokens, shape.width_s, device=DEVICE)
+    logits = mk.prefill(g, torch.tensor(ids, device=DEVICE), torch.arange(tokens, dtype=torch.int32, device=DEVICE), layer_out=out)
+    mk.check()
+    assert error(logits[:, : shape.vocab].double().cpu(), want) < TOL[torch.bfloat16]
+    for k, layer in enumerate(layers):
+        assert error(out[k, :, : shape.width].double().cpu(), layer) < TOL[torch.bfloat16]
+
+
 def pointed_model(heads=4, kv_heads=2):
     """One layer in whose attention token 1 asks and token 0 answers: the asker's score for the answerer stands far above all
     others, whatever lies between them."""
