@@ -416,7 +416,7 @@ size_t plain_buffers(const QmkHybridArgs* a, void* base, PlainBuffers<T>* b) {
     state.fit(P, l.heads, l.head_dim, l.v_dim, l.type == QMK_MIXER_GLA);
     if (l.type == QMK_MIXER_DELTA) {
       qkv = std::max(qkv, P * conv_channels(l));
-      values = std::max(values, P * l.mix_width);
+      values = std::max(values, static_cast<size_t>(chunks_of(static_cast<int>(P))) * kChunkTokens * l.mix_width);
       beta = std::max(beta, P * ((l.heads + 15) / 16 * 16));
     } else {
       qkv = std::max(qkv, P * (2 * l.heads * l.head_dim + l.mix_width));
@@ -832,7 +832,7 @@ int prefill_plain(const QmkHybridArgs* a) {
     launch_gemm<T, u16, T>(g, b.split, st);
     decays(l, l.rank + l.gate_rank, EPI_DELTA_DECAY);
     ChunkArgs c = chunk_args(l);
-    c.q = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values; c.value_ld = l.mix_width;
+    c.q = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values;
     run_chunks<T, CHUNK_DELTA>(c, st);
     return c;
   };

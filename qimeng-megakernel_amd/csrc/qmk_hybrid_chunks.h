@@ -5,7 +5,7 @@
 //   wkv: o_t = (S + diag(bonus) k_t v_t^T)^T r_t ahead of S <- g_t S + k_t v_t^T
 // Over a chunk that starts from S, with G_t = g_1 .. g_t and D_ts = g_{s+1} .. g_t (products, never quotients: a decay may
 // be small enough for its inverse to overflow):
-//   X_t = (G_t k_t)^T S           u = T (v - X),  T = (I + diag(beta) A)^-1 diag(beta),  A_ts = sum_i k_t D_ts k_s  (s < t)
+//   u = T v - W S,  W = T (G k)^T,  T = (I + diag(beta) A)^-1 diag(beta),  A_ts = sum_i k_t D_ts k_s  (s < t)
 //   o_t = (G_t q_t)^T S + sum_{s <= t} B_ts u_s,  B_ts = sum_i q_t D_ts k_s               (wkv: G_{t-1}, D_{t-1,s}, B_tt = sum_i r_t bonus k_t)
 //   S  <- G_16 S + sum_s (D_16,s k_s) u_s^T
 // chunk_prepare works out everything that no state enters, for all chunks at once.  Where u is v a chunk's state is a sum that may be cut anywhere: segments of
@@ -31,9 +31,9 @@ constexpr int kOwnStarts = 4;
 
 // Tiles of sixteen key channels of a head, the last ones zeros.
 __host__ __device__ constexpr int chunk_tiles(int head_dim) { return head_dim <= 64 ? 4 : head_dim <= 128 ? 8 : 16; }
-// Floats of one (chunk, head): per tile the fragments of G q, G k and D k and the decays G over the whole chunk, then B and
-// T.  A fragment is in the order the matrix instruction takes it: [lane][4].
-__host__ __device__ constexpr int chunk_floats(int head_dim) { return chunk_tiles(head_dim) * (3 * 256 + 16) + 2 * 256; }
+// Floats of one (chunk, head): per tile the fragments of G q, W and D k and the decays G over the whole chunk, then B.  A fragment is in the order the
+// matrix instruction takes it: [lane][4].
+__host__ __device__ constexpr int chunk_floats(int head_dim) { return chunk_tiles(head_dim) * (3 * 256 + 16) + 256; }
 __host__ __device__ constexpr int chunks_of(int tokens) { return (tokens + kChunkTokens - 1) / kChunkTokens; }
 __host__ __device__ constexpr int segments_of(int tokens, int chunks) { return (chunks_of(tokens) + chunks - 1) / chunks; }
 
@@ -44,7 +44,7 @@ struct ChunkArgs {
   const float* decay;    // [M][heads * dim]
   const float* beta;     // delta: [M][beta_ld]
   float* chunks;         // [chunk][head][chunk_floats]
-  float* values;         // [M][value_ld] at value_at; delta: written here
+  float* values;         // [M][value_ld] at value_at; delta: T v, [chunk][head][n / 16] fragments, written here
   float* out;            // [M][heads * n]
   float* starts;         // [segment][head][dim][n]: what the segment before leaves, then the state the segment starts from
   float* fades;          // [segment][head][dim]: decays over the segment before
@@ -64,6 +64,7 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
   __shared__ float norms[2][kChunkWaves][C], step[C];
   __shared__ __align__(16) float turned[kChunkWaves][C][C + 4];
   __shared__ __align__(16) float sa[C][C];
+  __shared__ f32x4 st[KIND == CHUNK_DELTA ? 64 : 1];      // T as a fragment
   const QmkHybridLayer& l = g.layer;
   const int head = blockIdx.y, chunk = blockIdx.x, m0 = chunk * C, count = min(C, g.M - m0);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), t = lane & 15, quad = lane >> 4;
@@ -71,40 +72,55 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
   const bool real = t < count;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
 
-  f32x4 q[TILES], k[TILES], w[TILES];
+  // One 16 x 16 matrix turned, through this wave's part of LDS: four columns of a row -> four rows of a column.
+  auto turn = [&](f32x4 v) {
+    store4(&turned[wave][t][quad * 4], v);
+    __builtin_amdgcn_wave_barrier();
+    const f32x4 out = {turned[wave][quad * 4][t], turned[wave][quad * 4 + 1][t], turned[wave][quad * 4 + 2][t], turned[wave][quad * 4 + 3][t]};
+    __builtin_amdgcn_wave_barrier();
+    return out;
+  };
+  // delta: four channels from `ch` on at this lane's token, behind convolution and silu.
+  auto convolved = [&](int ch) {
+    const int W = conv_channels(l), taps = l.taps;
+    const float* old = l.shift + (static_cast<size_t>(g.slot) * 2 + g.flip) * (taps - 1) * W;
+    constexpr int kFew = 4;
+    auto input = [&](int back) {      // tokens behind the portion are not used
+      const int at = min(m0 + t - back, g.M - 1);
+      return read4((at >= 0 ? g.q + static_cast<size_t>(at) * W : old + static_cast<size_t>(at + taps - 1) * W) + ch);
+    };
+    f32x4 v = zero;
+    if (taps <= kFew) {
+      f32x4 in[kFew], weight[kFew];
+#pragma unroll
+      for (int j = 0; j < kFew; ++j) {
+        const bool there = j >= kFew - taps;
+        in[j] = input(there ? kFew - 1 - j : 0);
+        weight[j] = there ? read4(l.vec2 + static_cast<size_t>(j - kFew + taps) * W + ch) : zero;
+      }
+#pragma unroll
+      for (int j = 0; j < kFew; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = j >= kFew - taps ? fmaf(weight[j][i], in[j][i], v[i]) : v[i];
+    } else {
+      for (int j = 0; j < taps; ++j) {
+        const f32x4 in = input(taps - 1 - j), weight = read4(l.vec2 + static_cast<size_t>(j) * W + ch);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = fmaf(weight[i], in[i], v[i]);
+      }
+    }
+    return each(v, [](float x) { return x * sigmoid(x); });
+  };
+  // Its values' tile `tile`, the head's last one again behind it.
+  auto value_tile = [&](int tile) {
+    const f32x4 v = convolved(2 * l.kv_heads * g.dim + head * g.n + min(tile * 16, g.n - 16) + quad * 4);
+    return real ? v : zero;
+  };
+  constexpr int kValues = 2;      // tiles of values that a wave holds until T is there
+  f32x4 q[TILES], k[TILES], w[TILES], held[KIND == CHUNK_DELTA ? kValues : 1];
   double dot = 0.;      // of this token's q and k: at a first token, or behind strong decays, it is all of an output, whose norm may leave little but its sign
   if constexpr (KIND == CHUNK_DELTA) {
-    const int kv = head / (l.heads / l.kv_heads), keys = l.kv_heads * g.dim, W = conv_channels(l), taps = l.taps;
-    const float* old = l.shift + (static_cast<size_t>(g.slot) * 2 + g.flip) * (taps - 1) * W;
-    // Four channels from `ch` on at this lane's token, behind silu.
-    auto convolved = [&](int ch) {
-      constexpr int kFew = 4;
-      auto input = [&](int back) {      // tokens behind the portion are not used
-        const int at = min(m0 + t - back, g.M - 1);
-        return read4((at >= 0 ? g.q + static_cast<size_t>(at) * W : old + static_cast<size_t>(at + taps - 1) * W) + ch);
-      };
-      f32x4 v = zero;
-      if (taps <= kFew) {
-        f32x4 in[kFew], weight[kFew];
-#pragma unroll
-        for (int j = 0; j < kFew; ++j) {
-          const bool there = j >= kFew - taps;
-          in[j] = input(there ? kFew - 1 - j : 0);
-          weight[j] = there ? read4(l.vec2 + static_cast<size_t>(j - kFew + taps) * W + ch) : zero;
-        }
-#pragma unroll
-        for (int j = 0; j < kFew; ++j)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = j >= kFew - taps ? fmaf(weight[j][i], in[j][i], v[i]) : v[i];
-      } else {
-        for (int j = 0; j < taps; ++j) {
-          const f32x4 in = input(taps - 1 - j), weight = read4(l.vec2 + static_cast<size_t>(j) * W + ch);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = fmaf(weight[i], in[i], v[i]);
-        }
-      }
-      return each(v, [](float x) { return x * sigmoid(x); });
-    };
+    const int kv = head / (l.heads / l.kv_heads), keys = l.kv_heads * g.dim;
     float nq = 0.f, nk = 0.f;
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
@@ -121,11 +137,8 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
         dot = fma(static_cast<double>(q[j][i]), static_cast<double>(k[j][i]), dot);
       }
     }
-    for (int tile = wave; tile * 16 < g.n; tile += kChunkWaves) {
-      const int c = head * g.n + tile * 16 + quad * 4;
-      const f32x4 v = convolved(2 * keys + c);
-      if (real) store4(g.values + row * g.value_ld + g.value_at + c, v);
-    }
+#pragma unroll
+    for (int j = 0; j < kValues; ++j) held[j] = value_tile(wave + j * kChunkWaves);
     if (tid < count) step[tid] = g.beta[static_cast<size_t>(m0 + tid) * g.beta_ld + head];
     nq += __shfl_xor(nq, 16);
     nk += __shfl_xor(nk, 16);
@@ -224,17 +237,18 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
 
   float* rec = g.chunks + (static_cast<size_t>(chunk) * g.heads + head) * chunk_floats(g.dim);
   constexpr int stored = TILES * kChunkWaves;
-  float *rq = rec, *rk = rq + stored * 256, *rd = rk + stored * 256, *rg = rd + stored * 256, *rb = rg + stored * 16, *rt = rb + 256;
+  float *rq = rec, *rk = rq + stored * 256, *rd = rk + stored * 256, *rg = rd + stored * 256, *rb = rg + stored * 16;
 #pragma unroll
   for (int j = 0; j < TILES; ++j) {
     const int tile = wave * TILES + j;
     store4(rq + tile * 256 + lane * 4, q[j] * ahead[j]);
-    if constexpr (KIND == CHUNK_DELTA) store4(rk + tile * 256 + lane * 4, key[j] * ahead[j]);
     if (t == 0) store4(rg + tile * 16 + quad * 4, all[j]);
-    store4(&turned[wave][t][quad * 4], k[j] * behind[j]);
-    __builtin_amdgcn_wave_barrier();
-    store4(rd + tile * 256 + lane * 4, f32x4{turned[wave][quad * 4][t], turned[wave][quad * 4 + 1][t], turned[wave][quad * 4 + 2][t], turned[wave][quad * 4 + 3][t]});
-    __builtin_amdgcn_wave_barrier();
+    store4(rd + tile * 256 + lane * 4, turn(k[j] * behind[j]));
+    if constexpr (KIND == CHUNK_DELTA) key[j] = turn(key[j] * ahead[j]);
+  }
+  if constexpr (KIND == CHUNK_DELTA) {
+#pragma unroll
+    for (int j = 0; j < kValues; ++j) held[j] = turn(held[j]);
   }
   __syncthreads();
   {
@@ -260,9 +274,29 @@ __global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
 #pragma unroll
         for (int j = 0; j < r; ++j) acc = fmaf(-sa[r][j], col[j], acc);
         col[r] = r < count ? acc * step[r] : 0.f;
-        rt[((tid >> 2) * 16 + r) * 4 + (tid & 3)] = col[r];
+        st[(tid >> 2) * 16 + r][tid & 3] = col[r];
       }
     }
+    __syncthreads();
+    // W and T v: what the scan's chain need not wait for.
+    const f32x4 T = st[lane];
+    auto product = [](f32x4 a, f32x4 b) {
+      f32x4 c = {};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+      return c;
+    };
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) store4(rk + (wave * TILES + j) * 256 + lane * 4, product(key[j], T));
+    float* values = g.values + (static_cast<size_t>(chunk) * g.heads + head) * (g.n * C) + lane * 4;
+#pragma unroll
+    for (int j = 0; j < kValues; ++j) {
+      const f32x4 v = product(T, held[j]);
+      const int tile = wave + j * kChunkWaves;
+      if (tile * 16 < g.n) store4(values + tile * 256, v);
+    }
+#pragma unroll 1
+    for (int tile = wave + kValues * kChunkWaves; tile * 16 < g.n; tile += kChunkWaves) store4(values + tile * 256, product(T, turn(value_tile(tile))));
   }
 }
 
@@ -485,19 +519,19 @@ __global__ __launch_bounds__(kPfThreads) void segment_starts(const ChunkArgs g) 
 // accumulators of the matrix instruction, which are also the second operand of the products that read it.  Tiles behind the
 // last one are zeros and take part: with a branch around each tile's products this compiler has left out the wait between a
 // tile's last product and the first use of its result on the path that skips the next tile.  Loads have no branches either,
-// so that kAhead chunks are in flight: a chunk, or token, behind the last one is the last one again, and its value is either
-// not used or multiplied by zero.
-// What bounds it is the chain of a chunk: products of the state with the keys (four dependent instructions of 32 cycles a tile), the
-// waves' sums through LDS, T (v - X), the state's update.  So what only the output needs is off the chain: G q S is taken while the sums are on their way, and a
-// chunk's outputs are added up and stored behind the next chunk's barrier.
-// A wave's instructions are on that chain too, one wave a SIMD: chunks are read and written by buffer accesses (places of 32 bits that stay, bases that move on by
-// one scalar addition, tokens behind the last one read as zero and not written).  us, 2048 tokens of 16 heads of 128 | 128, addresses of 64 bits worked out for every
-// access -> now 134 -> 120; lines of chunks further ahead asked for into L2: 141.
+// so that kAhead chunks are in flight: a chunk behind the last one is the last one again, and is not used; tokens behind the last one are zeros of the record.
+// What bounds it is the chain of a chunk: products of the state with W (four instructions of 32 cycles a tile), the waves' sums through LDS, the state's update.
+// What only the output needs fills the wait for the sums, is the same for every wave (of B u each takes the columns of one of the four instructions, of the sums the
+// tokens of one), and is added up behind the next chunk's barrier; W and T v come from chunk_prepare.  us, 2048 tokens of 16 heads of 128 | 128, beside an
+// attention behind nothing and behind 2048 keys, T (v - (Gk)^T S) on the chain and a chunk's outputs by one wave -> so: 132 -> 103, 147 -> 137 (the attention's own time there).  Error against
+// 64 bits in fp32, beside that: 1b shape, 150 tokens (40 models) states x 0.998 +- 0.001, logits x 1.008 +- 0.008, 331 tokens (30) x 0.998 +- 0.001, x 1.006 +- 0.009.  With B u's part in a sum
+// of its own the launch takes 136 where it takes 120.
 template <int WAVES>
 constexpr int kScanLds = 4 * WAVES * 64;
-// Chunks in flight: what the registers hold (us, the shape above, with 2, 3 and 4 ahead: 131, 120, 123).
-template <int TILES, int WAVES, int kAhead = TILES == 1 ? 4 : TILES == 2 ? 3 : 2>
+// kAhead: chunks in flight, what the registers hold.
+template <int TILES, int WAVES, int kAhead = TILES == 4 ? 2 : 3>
 __device__ __forceinline__ void scan_chunks(const ChunkArgs& g, int head, int v0, f32x4* lds) {
+  static_assert(WAVES == 4, "a wave takes one of four instructions, and four of sixteen tokens");
   auto px = reinterpret_cast<f32x4(*)[WAVES][64]>(lds), po = px + 2;
   const QmkHybridLayer& l = g.layer;
   const int dim = g.dim, n = g.n;
@@ -507,15 +541,9 @@ __device__ __forceinline__ void scan_chunks(const ChunkArgs& g, int head, int v0
   const int chunks = (g.M + kChunkTokens - 1) / kChunkTokens, out_ld = l.heads * n;
   float* state = l.state + (static_cast<size_t>(g.slot) * l.heads + head) * dim * n + v0 + col;
   auto buffer = [](const float* base, int bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000); };
-  // Bytes from a chunk's first value (output) to behind its last one, of rows of `ld`.
-  auto extent = [&](int chunk, int ld) { return ((min(g.M - chunk * kChunkTokens, kChunkTokens) - 1) * ld + 16) * 4; };
-  uint32_t value_at[4], out_at[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    value_at[i] = ((quad * 4 + i) * g.value_ld + col) * 4;
-    out_at[i] = ((quad * 4 + i) * out_ld + col) * 4;
-  }
-  const uint32_t fragment_at = tile0 * 1024 + lane * 16, decay_at = tile0 * 64 + quad * 16, shared_at = lane * 16;
+  // This lane's output of a chunk: token wave * 4 + quad, column col; rows behind the last token are not written.
+  const uint32_t out_at = ((wave * 4 + quad) * out_ld + col) * 4;
+  const uint32_t fragment_at = tile0 * 1024 + lane * 16, decay_at = tile0 * 64 + quad * 16, pairs_at = lane * 16 + wave * 4, value_at = lane * 16;
   f32x4 s[TILES];
 #pragma unroll
   for (int j = 0; j < TILES; ++j)
@@ -523,26 +551,25 @@ __device__ __forceinline__ void scan_chunks(const ChunkArgs& g, int head, int v0
     for (int i = 0; i < 4; ++i) s[j][i] = j < mine ? state[static_cast<size_t>((tile0 + j) * 16 + quad * 4 + i) * n] : 0.f;
 
   struct Fragments {
-    f32x4 q[TILES], k[TILES], d[TILES], g[TILES], b, t, v;
+    f32x4 q[TILES], w[TILES], d[TILES], g[TILES], v;
+    float b;
   };
   // Chunks are fetched in their order; behind the last one it is the last one again.
-  const size_t rec_step = static_cast<size_t>(l.heads) * chunk_floats(dim), value_step = static_cast<size_t>(kChunkTokens) * g.value_ld;
-  const float *rec = g.chunks + static_cast<size_t>(head) * chunk_floats(dim), *values = g.values + g.value_at + head * n + v0;
+  const size_t rec_step = static_cast<size_t>(l.heads) * chunk_floats(dim), value_step = static_cast<size_t>(l.heads) * n * kChunkTokens;
+  const float *rec = g.chunks + static_cast<size_t>(head) * chunk_floats(dim), *values = g.values + static_cast<size_t>(head) * n * kChunkTokens + v0 * kChunkTokens;
   int fetched = 0;
   auto fetch = [&](Fragments& f) {
-    const auto r = buffer(rec, chunk_floats(tiles * 16) * 4), v = buffer(values, extent(fetched, g.value_ld));
+    const auto r = buffer(rec, chunk_floats(tiles * 16) * 4), v = buffer(values, 1024);
     auto read = [&](uint32_t at, int first) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, first * 4, 0)); };
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
-      f.k[j] = read(fragment_at + j * 1024, tiles * 256);
+      f.w[j] = read(fragment_at + j * 1024, tiles * 256);
       f.q[j] = read(fragment_at + j * 1024, 0);
       f.d[j] = read(fragment_at + j * 1024, tiles * 512);
       f.g[j] = read(decay_at + j * 64, tiles * 768);
     }
-    f.b = read(shared_at, tiles * 784);
-    f.t = read(shared_at, tiles * 784 + 256);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) f.v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(v, value_at[i], 0, 0));
+    f.b = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, pairs_at, tiles * 784 * 4, 0));
+    f.v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(v, value_at, 0, 0));
     const bool more = fetched + 1 < chunks;
     rec += more ? rec_step : 0;
     values += more ? value_step : 0;
@@ -553,42 +580,41 @@ __device__ __forceinline__ void scan_chunks(const ChunkArgs& g, int head, int v0
     for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
     return c;
   };
-  // Ahead of a branch's end: this compiler (clang 22 of ROCm 7.2.0) has left out the wait between a product and the move of its result where paths meet; without
-  // this <1, 4> moves one two instructions behind its product.  The rule, for any kernel: an accumulator that lives across the end of a branch with a product in it is
-  // settled there if its built code has such a move (tests/test_matrix_waits.py walks every path of every kernel for it); none but these two places has.
+  // Ahead of a branch's end: this compiler (clang 22 of ROCm 7.2.0) has left out the wait between a product and the move of its result where paths meet.  The rule, for any
+  // kernel: an accumulator that lives across the end of a branch with a product in it is settled there if its built code has such a move (tests/test_matrix_waits.py walks every
+  // path of every kernel for it); none but this place has.
   auto settle = [](f32x4& v) { asm volatile("s_nop 15" : "+v"(v)); };
-  f32x4 inner = {};       // B u of the last chunk whose outputs are this wave's
-  auto outputs = [&](int chunk) {
-    if (chunk < 0 || wave != (chunk & (WAVES - 1))) return;
-    f32x4 o = inner;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) o += po[chunk & 1][w][lane];
-    const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, extent(chunk, out_ld));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[i]), to, out_at[i], 0, 0);
+  auto outputs = [&](int chunk) {      // of chunk 0 on: everybody's sums of its outputs are in LDS
+    const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, ((min(g.M - chunk * kChunkTokens, kChunkTokens) - 1) * out_ld + 16) * 4);
+    const float* from = reinterpret_cast<const float*>(po[chunk & 1][0]) + (wave * 16 + col) * 4 + quad;
+    const float o = (from[0] + from[256]) + (from[512] + from[768]);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), to, out_at, 0, 0);
   };
   auto advance = [&](const Fragments& f, int chunk) {
     const int buf = chunk & 1;
-    f32x4 x = {};
+    f32x4 x[2] = {}, o[2] = {};      // (two sums of every other tile: half as many roundings follow one another)
 #pragma unroll
-    for (int j = 0; j < TILES; ++j) x = product(f.k[j], s[j], x);
-    px[buf][wave][lane] = x;
-    __syncthreads();      // everybody's X; the chunk before's G q S
-    f32x4 u = f.v;
+    for (int j = 0; j < TILES; ++j) x[j & 1] = product(f.w[j], s[j], x[j & 1]);
+    px[buf][wave][lane] = TILES == 1 ? x[0] : x[0] + x[1];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) u -= px[buf][w][lane];
-    f32x4 o = {};
+    for (int j = 0; j < (TILES + 1) / 2; ++j) o[j & 1] = product(f.q[j], s[j], o[j & 1]);
+    wait_known<63>();
+    __builtin_amdgcn_s_barrier();      // everybody's W S; the outputs of the chunk before
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 part[WAVES];
 #pragma unroll
-    for (int j = 0; j < TILES; ++j) o = product(f.q[j], s[j], o);
-    po[buf][wave][lane] = o;
-    u = product(f.t, u, f32x4{0.f, 0.f, 0.f, 0.f});
+    for (int w = 0; w < WAVES; ++w) part[w] = px[buf][w][lane];
+#pragma unroll
+    for (int j = (TILES + 1) / 2; j < TILES; ++j) o[j & 1] = product(f.q[j], s[j], o[j & 1]);
+    const f32x4 u = f.v - ((part[0] + part[1]) + (part[2] + part[3]));
 #pragma unroll
     for (int j = 0; j < TILES; ++j) s[j] = product(f.d[j], u, s[j] * f.g[j]);
-    outputs(chunk - 1);
-    if (wave == (chunk & (WAVES - 1))) {
-      inner = product(f.b, u, f32x4{0.f, 0.f, 0.f, 0.f});
-      settle(inner);
-    }
+    const float own = wave == 0 ? u[0] : wave == 1 ? u[1] : wave == 2 ? u[2] : u[3];
+    o[TILES > 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.b, own, o[TILES > 1], 0, 0, 0);
+    po[buf][wave][lane] = TILES == 1 ? o[0] : o[0] + o[1];
+    if (chunk > 0) outputs(chunk - 1);
   };
   Fragments f[kAhead];
 #pragma unroll
@@ -623,8 +649,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void chunk_scan(const ChunkArgs g) {
 }
 
 // The two branches of a run need nothing of each other, and the delta rule's chunks are a chain of instructions on a part of the chip: its workgroups come first, and go first on their SIMDs, an
-// attention's fill what is left (us, 2048 tokens of 16 heads of 128 | 128 in either, behind nothing and behind 2048 keys, two launches -> one: 118 + 47 -> 129, 119 + 93 -> 150).  Registers
-// for two workgroups a CU leave room for two chunks in flight of two tiles a wave.
+// attention's fill what is left (us, 2048 tokens of 16 heads of 128 | 128 in either, behind nothing and behind 2048 keys, two launches -> one: 118 + 47 -> 132, 119 + 93 -> 147).
 template <int TILES, int QT, int VT, int KEYS, int STAGES, bool SHARED>
 __global__ __launch_bounds__(kPfThreads, 2) void scan_and_attend(const ChunkArgs c, const AttentionArgs a) {
   constexpr int kUnits = kAttentionLds<QT, VT, KEYS, STAGES, SHARED>;
@@ -633,7 +658,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void scan_and_attend(const ChunkArgs
   const int scans = c.heads * (c.n / 16), id = blockIdx.x;
   if (id < scans) {
     __builtin_amdgcn_s_setprio(3);
-    scan_chunks<TILES, kChunkWaves, TILES == 1 ? 4 : 2>(c, id % c.heads, id / c.heads * 16, reinterpret_cast<f32x4*>(lds));
+    scan_chunks<TILES, kChunkWaves>(c, id % c.heads, id / c.heads * 16, reinterpret_cast<f32x4*>(lds));
   } else {
     attend_rows<QT, VT, KEYS, STAGES, SHARED>(a, id - scans, gridDim.x - scans, lds);
   }
