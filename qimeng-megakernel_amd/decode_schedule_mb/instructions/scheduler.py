@@ -86,7 +86,8 @@ class BatchScheduler:
     split_kv_per_worker: float = 1.0   # split-KV instructions of a step per worker that the fan-out aims at (the reference: one)
     split_kv_cap: int = MAX_REDUCTION_LIST   # ... and never more slices per KV head than this
     lone_slice_tokens: int = 0         # where the rule gives two or three slices and the slices' tokens are at most this many: one slice
-                                       # (the only slice of its heads writes attn_out itself: no counted arrival, no merge)
+                                       # (the only slice of its heads writes attn_out itself: no counted arrival, no merge);
+                                       # heads of 128: one slice up to this many whatever the rule gives (0: the rule alone)
 
     def __post_init__(self) -> None:
         if not 1 <= self.batch_size <= MAX_BATCH:
@@ -156,10 +157,17 @@ class BatchScheduler:
         others = self.workers - self.batch_size
         blocks = _ceil_div(self.shape.qkv_out_dim, TILE_N_GRANULARITY)
         if start == 0 and 0 < others and blocks <= 2 * others:
-            # A block for every worker (Qwen3-1.7B shape: 256): the norm rows' workers still get none, a few of the others
-            # two — a second block costs 1 us, a block behind a norm row ends the phase 2.7 us late.
-            start = self.batch_size
-            plain = [QKVProj_GEMM_RoPE(layer, self.batch_size, 0, lo, hi) for lo, hi in _spans(blocks, others)]
+            # A block for every worker (Qwen3-1.7B shape: 256).  Where the split-KV round fits on the down projection's
+            # workers they go, two to a worker, to the others: those have both blocks' weights in registers before the layer in
+            # front ends, where a worker that has just run its down block asks for them only then and ends the phase 2.5 us
+            # later, and an attention worker starts its slice without a block in front (8 rows, context 500, two slices: 1294 ->
+            # 1199 us a step; context 130, one slice: 1157 -> 1097).  Above 8 rows also where it does not fit (16 rows, context 900,
+            # two slices: 1607 -> 1578), below that not (6 rows, 700, three: 1291 -> 1316): the norm rows' workers then get none,
+            # a few of the others two.
+            busy = min(self.workers, len(self.downproj(layer)))
+            beside = (slices <= busy or self.batch_size > 8) and blocks <= 2 * (self.workers - busy)
+            start = busy if beside else self.batch_size
+            plain = [QKVProj_GEMM_RoPE(layer, self.batch_size, 0, lo, hi) for lo, hi in _spans(blocks, self.workers - start)]
         return [NoOp()] * start + plain + [NoOp()] * (self.workers - start - len(plain))
 
     def oproj_round(self, layer: int, num_partials: int) -> list[Instruction]:
@@ -236,9 +244,17 @@ class BatchScheduler:
 
     def _fan_out(self, rows: int, blocks: int) -> int:
         p = min(self.split_kv_cap, partials_for_blocks(rows, blocks, self._split_kv_workers(), self.shape.num_key_value_heads))
-        if p in (2, 3) and self.merge_in_last and blocks * self.shape.attn_kv_block_size <= self.lone_slice_tokens:
-            return 1   # (three slices: 6 and 7 rows with heads of 64 — 45.5 -> 40.5 us per layer at context 300, 47 -> 45.5 at 900)
+        tokens, heads = blocks * self.shape.attn_kv_block_size, max(rows, 1) * self.shape.num_key_value_heads
+        beside = min(self.workers, _ceil_div(self.shape.hidden_size, self.down_tile)) // heads   # slices that the down projection's workers hold
+        if self.merge_in_last and (p in (2, 3) and tokens <= self.lone_slice_tokens or p > beside and rows < 8 and 2 * tokens <= self.lone_slice_tokens):
+            return 1   # (three slices: 6 and 7 rows with heads of 64 — 45.5 -> 40.5 us per layer at context 300, 47 -> 45.5 at 900;
+                       # four: 5 rows, 777 -> 698 us a step at 200, 805 -> 794 at 900, but 844 -> 907 at 1800)
         if self.merge_in_last:
+            if self.shape.head_dim > 64 and self.lone_slice_tokens:
+                if tokens <= self.lone_slice_tokens:
+                    return 1
+                if beside > 2 or beside == 2 and tokens <= 2 * self.lone_slice_tokens:
+                    p = min(p, beside)
             # The rule rounds up: 12 rows of 8 KV heads get 3 slices, 288 instructions for 256 workers — a second round of
             # 32 behind the first (Qwen3-1.7B shape, 12 rows: 1.83 ms per step against 1.64 at 16 rows).  Never more
             # instructions than workers.
@@ -320,7 +336,13 @@ def mi355x_scheduler(batch_size: int, shape: DecodeShape | None = None, *, merge
     what a slice saves in scores the merge by the last arrival (a counted arrival, a second read of the partials,
     a second hand-over) costs again: Llama shape, contexts 500 / 1000, step time with the reference's fan-out against
     half of it: B=2 938/947 -> 853/856 us, B=4 938/947 -> 881/905, B=8 1021/1048 -> 972/1009, B=16 1187/1233 ->
-    1108/1176.  With heads of 128 (Qwen3-1.7B shape, B=8: 1566/1636 us with 4 slices, 1591/1721 with 2) the rule stays.
+    1108/1176.  With heads of 128 (Qwen3-1.7B shape, B=8: 1566/1636 us with 4 slices, 1591/1721 with 2) the rule's number stays for long caches.
+    With heads of 128, from 5 rows on (fewer take the rows engine), a cache of up to 512 tokens has one slice, and a longer one as many as the down projection's workers
+    hold, where that is three, or two and at most 1024 tokens: the QKV blocks then keep off the slices' workers (8 rows, contexts
+    130 / 350 / 500 / 700 / 950 / 1500 with 1, 2 and 4 slices: 1097 / 1136 / 1206 / 1300 / 1412 / 1641, 1185 / 1192 / 1199 / 1245 / 1335 / 1475
+    and 1256 / 1273 / 1285 / 1314 / 1350 / 1400 us; 5 rows, 350 / 700 / 1500 with 1, 3 and 4: 1062 / 1224 / 1555, 1162 / 1170 / 1288 and
+    1208 / 1264 / 1348; 10 rows, 350 / 700 / 950 with 1, 2 and 3: 1217 / 1383 / 1494, 1339 / 1408 / 1494 and 1335 / 1384 / 1414; 16
+    rows, 180 / 350 / 700 with 1 and 2: 1283 / 1328 / 1535 and 1403 / 1443 / 1505).
     Never more than 4 slices (mean step time at contexts 250 / 500 / 1000 with 4 against 8 slices: Llama shape B=2
     843 against 856 us; Qwen3 shape B=2 1345 against 1362, B=4 1432 against 1433).  With heads of 64 and a cache of at
     most 2048 tokens one slice where the rule gives two: the only slice of its heads writes attn_out itself (Llama
@@ -330,4 +352,4 @@ def mi355x_scheduler(batch_size: int, shape: DecodeShape | None = None, *, merge
     shape = shape or LlamaConfig.shape()
     return BatchScheduler(shape, MI355X_WORKERS, batch_size, merge_in_last=merge_in_last, oproj_tile=residual_tile,
                           down_tile=residual_tile, skew_upgate=skew_upgate, split_kv_per_worker=0.5 if shape.head_dim <= 64 else 1.0,
-                          split_kv_cap=4, lone_slice_tokens=2048 if shape.head_dim <= 64 else 0)
+                          split_kv_cap=4, lone_slice_tokens=2048 if shape.head_dim <= 64 else 512 if batch_size > 4 else 0)

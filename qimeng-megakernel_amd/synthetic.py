@@ -135,12 +135,18 @@ def build_batch_globals(
 ) -> Any:
     """Buffers of the batch route for ``batch_size`` rows (allocation as the reference's
     `…/A100/fused_prefill.py:93-160` for batch sizes above one); all rows active, positions 0."""
+    from .decode_schedule_mb.mk_kernel import BatchMegaKernel
+    from .decode_schedule_mb.rows_kernel import MAX_ROWS
+
     if globals_cls is None:
         from .decode_schedule_mb.globs import Globals as globals_cls
     device = torch.device(device)
     bf16 = torch.bfloat16
     L, H, B = shape.num_hidden_layers, shape.hidden_size, batch_size
     nq, nkv, d = shape.num_attention_heads, shape.num_key_value_heads, shape.head_dim
+    # Where the tiles engine decodes, rows of at least the words that its counts per XCD need: without them 5..7 rows cost more
+    # than 8 (Qwen3-1.7B shape, 7 rows at context 180 1482 us a step, 8 rows 1268; Llama shape, 5 rows at 200 843, 6 rows 707).
+    spread = BatchMegaKernel.XCD_COUNTER_WORDS if B > MAX_ROWS else 0
 
     def zeros(*size: int, dtype: torch.dtype = bf16) -> torch.Tensor:
         return torch.zeros(*size, dtype=dtype, device=device)
@@ -148,7 +154,7 @@ def build_batch_globals(
     on_device = {k: v.to(device).contiguous() for k, v in weights.items()}
     g = globals_cls(
         position_id=0,
-        barriers=zeros(L, 10, (nq + 2 * nkv) * B, dtype=torch.int32),
+        barriers=zeros(L, 10, max((nq + 2 * nkv) * B, spread), dtype=torch.int32),
         k_cache=zeros(L, B, kv_capacity, nkv, d),
         v_cache=zeros(L, B, kv_capacity, nkv, d),
         hidden_states=zeros(B, H),
