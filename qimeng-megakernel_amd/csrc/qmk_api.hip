@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kThreads, 1) void decode_megakernel(const Params p_
       case OP_OPROJ_RESIDUAL:
         carried = M::CARRY_AFTER_ATTENTION || !after_attention;
         parked = !after_attention;   // a workgroup that has just run the attention has no wait to fill
-        [[clang::always_inline]] ok = op_oproj_residual<M>(params_for(kSegmentOproj), s, c, carry, carried, parked);
+        [[clang::always_inline]] ok = op_oproj_residual<M>(params_for(kSegmentOproj), s, c, carry, carried, parked, after_attention);
         break;
       case OP_RMS_UPGATE_SILU: [[clang::always_inline]] ok = op_rms_upgate_silu<M>(params_for(kSegmentUpGate), s, c, carry, carried, parked); forget(carry); break;
       case OP_DOWN_RESIDUAL: [[clang::always_inline]] ok = op_down_residual<M>(params_for(kSegmentDown), s, c); forget(carry); break;

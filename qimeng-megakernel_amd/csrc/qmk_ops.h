@@ -1095,7 +1095,8 @@ __device__ __forceinline__ void park_upgate_rows(const Params& p, Smem<M>& s, co
 // [4, layer, tile_M, n_start, n_end, reduction_block, tile_M_g, tile_N_g]
 // hidden[r] = bf16(hidden[r] + bf16(W_o[r] . attn_out))   (operations.py:251-262, 63-68)
 template <class M>
-__device__ bool op_oproj_residual(const Params& p, Smem<M>& s, const Ctx& c, Carried& carry, bool& carried, bool& parked) {
+__device__ bool op_oproj_residual(const Params& p, Smem<M>& s, const Ctx& c, Carried& carry, bool& carried, bool& parked,
+                                  bool after_attention = false) {
   constexpr int AW = M::AW;          // columns of W_o: all query heads side by side (= H for the dense models)
   constexpr int CH = AW / 512;
   static_assert(AW % (kThreads * 4) == 0 && AW <= M::F, "whole 8-byte pieces per thread; the vector fits the LDS buffer");
@@ -1126,6 +1127,14 @@ __device__ bool op_oproj_residual(const Params& p, Smem<M>& s, const Ctx& c, Car
   // The next instruction's rows, if it is the up/gate GEMV of this layer (see Carried).
   // (`carried` comes in as "may": a workgroup that has just run this layer's attention starts late,
   // and its requests would stand in front of its own reads of the partials.)
+  // Where the last slice merges, a workgroup whose slice was not the last has the merge to wait for, 4 us at 32 slices,
+  // and reads 4 KB behind it: it asks ahead as well (Llama shape, context 16384: 686 -> 671 us a step; rows in registers alone
+  // 678).  The Qwen3-1.7B shape carries behind attention anyway, and parks nothing there (context 16000: 1241, with it 1253).
+  const int self_merge = s.inst[5];  // reduction_block_idx: 0, or the split-KV fan-out P when this op merges
+  const bool merged = self_merge > 0 && self_merge <= min(kMaxSelfMerge, p.max_splits) && last_slice_merges<M>(p, self_merge);
+  if constexpr (!M::CARRY_AFTER_ATTENTION) {
+    if (after_attention && merged && !s.ctl[3]) carried = parked = true;
+  }
   carried = carried && s.next[0] == OP_RMS_UPGATE_SILU && s.next[1] == layer && upgate_check<M>(p, s.next) < 0;
   if (carried) {
     const int un = s.next[3], utile = s.next[5 + un];
@@ -1144,8 +1153,6 @@ __device__ bool op_oproj_residual(const Params& p, Smem<M>& s, const Ctx& c, Car
   // registers, measured 0.6 % slower).
   parked = parked && carried && M::PARK_ROWS > 0;
   if (parked) park_upgate_rows<M>(p, s, s.next, layer, lane, c.tid >> 6);
-  const int self_merge = s.inst[5];  // reduction_block_idx: 0, or the split-KV fan-out P when this op merges
-  const bool merged = self_merge > 0 && self_merge <= min(kMaxSelfMerge, p.max_splits) && last_slice_merges<M>(p, self_merge);
   if (__builtin_expect(self_merge == 0 || merged, 0)) {
     if (merged) {
       if (!wg_wait_all(p, s, c, layer, ROW_REDUCE, 0, M::NKV * self_merge)) return false;
