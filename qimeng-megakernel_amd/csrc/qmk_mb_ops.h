@@ -520,9 +520,15 @@ __device__ bool op_splitkv(const Params& p, Smem<M>& s, const Ctx& c) {
       for (int i = 0; i < NT / 2; ++i) tl.v[j][i] = src[i];
     }
   };
-  // A wave's next kDepth tiles are in flight at any time, the first of them from before the wait below: a tile
-  // costs a trip to memory and 16 tokens of arithmetic, so with one tile ahead every round paid most of the trip.
-  constexpr int kDepth = 2;   // (4 and 8 measured 0.2 % and 0.4 % slower)
+  // A wave's next `depth` tiles are in flight at any time, the first of them from before the wait below: a tile costs a trip
+  // to memory and 16 tokens of arithmetic, so with one tile ahead every round paid most of the trip.  Up to three slices a head the
+  // workgroup has nothing else to do in that wait, and four tiles pay (two -> four, Qwen3-1.7B shape, 8 rows, one slice, context 500 /
+  // 700 / 950: 1210 / 1296 / 1409 -> 1153 / 1225 / 1344 us a step; 16 rows, 900: 1631 -> 1533; Llama shape, 8 rows, 900: 820 -> 786;
+  // five spill).  With four slices it comes from a QKV block, a wave has three tiles at most up to 1500 tokens, and the other two's
+  // requests and code cost more than they give (1404 -> 1424 at 1500): two.
+  constexpr int kDepth = 4, kShort = 2;
+  const bool deep = P <= 3;   // uniform
+  const int depth = deep ? kDepth : kShort;
   int tb = t0 + wave * kTok;
   Tile ring[kDepth];
   static_for<0, kDepth>([&](auto i) {
@@ -532,7 +538,7 @@ __device__ bool op_splitkv(const Params& p, Smem<M>& s, const Ctx& c) {
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int e = 0; e < NT / 2; ++e) ring[i].v[j][e] = 0;
-    if (!empty && tb + i * kStep < t1) fetch(ring[i], tb + i * kStep);
+    if (!empty && (i < kShort || deep) && tb + i * kStep < t1) fetch(ring[i], tb + i * kStep);
   });
 
   if (!wait_counters(
@@ -723,12 +729,12 @@ __device__ bool op_splitkv(const Params& p, Smem<M>& s, const Ctx& c) {
       acc[tau] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(p_hi, vb, acc[tau], 0, 0, 0);
       acc[tau] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(p_lo, vb, acc[tau], 0, 0, 0);
     }
-    if (tb + kDepth * kStep < t1) fetch(cur, tb + kDepth * kStep);   // the tile that takes this one's place
+    if (tb + depth * kStep < t1) fetch(cur, tb + depth * kStep);   // the tile that takes this one's place
     tb += kStep;
   };
   while (tb < t1) {
     static_for<0, kDepth>([&](auto i) {
-      if (tb < t1) round(ring[i]);
+      if ((i < kShort || deep) && tb < t1) round(ring[i]);
     });
   }
   QMK_MB_STAMP(1);

@@ -253,7 +253,7 @@ class BatchScheduler:
             if self.shape.head_dim > 64 and self.lone_slice_tokens:
                 if tokens <= self.lone_slice_tokens:
                     return 1
-                if beside > 2 or beside == 2 and tokens <= 2 * self.lone_slice_tokens:
+                if beside > 2 or beside == 2 and tokens <= 1024:
                     p = min(p, beside)
             # The rule rounds up: 12 rows of 8 KV heads get 3 slices, 288 instructions for 256 workers — a second round of
             # 32 behind the first (Qwen3-1.7B shape, 12 rows: 1.83 ms per step against 1.64 at 16 rows).  Never more
@@ -337,12 +337,12 @@ def mi355x_scheduler(batch_size: int, shape: DecodeShape | None = None, *, merge
     a second hand-over) costs again: Llama shape, contexts 500 / 1000, step time with the reference's fan-out against
     half of it: B=2 938/947 -> 853/856 us, B=4 938/947 -> 881/905, B=8 1021/1048 -> 972/1009, B=16 1187/1233 ->
     1108/1176.  With heads of 128 (Qwen3-1.7B shape, B=8: 1566/1636 us with 4 slices, 1591/1721 with 2) the rule's number stays for long caches.
-    With heads of 128, from 5 rows on (fewer take the rows engine), a cache of up to 512 tokens has one slice, and a longer one as many as the down projection's workers
-    hold, where that is three, or two and at most 1024 tokens: the QKV blocks then keep off the slices' workers (8 rows, contexts
-    130 / 350 / 500 / 700 / 950 / 1500 with 1, 2 and 4 slices: 1097 / 1136 / 1206 / 1300 / 1412 / 1641, 1185 / 1192 / 1199 / 1245 / 1335 / 1475
-    and 1256 / 1273 / 1285 / 1314 / 1350 / 1400 us; 5 rows, 350 / 700 / 1500 with 1, 3 and 4: 1062 / 1224 / 1555, 1162 / 1170 / 1288 and
-    1208 / 1264 / 1348; 10 rows, 350 / 700 / 950 with 1, 2 and 3: 1217 / 1383 / 1494, 1339 / 1408 / 1494 and 1335 / 1384 / 1414; 16
-    rows, 180 / 350 / 700 with 1 and 2: 1283 / 1328 / 1535 and 1403 / 1443 / 1505).
+    With heads of 128, from 5 rows on (fewer take the rows engine), a cache of up to 640 tokens has one slice (above 8 rows: up to
+    1024), and a longer one as many as the down projection's workers hold, where that is three, or two and at most 1024 tokens: the
+    QKV blocks then keep off the slices' workers, and those ask for four tiles a wave ahead (8 rows, contexts 130 / 350 / 500 / 600 / 700 /
+    950 with 1 and 2 slices: 1092 / 1113 / 1153 / 1174 / 1225 / 1344, 1185 / 1188 / 1200 / 1200 / 1215 / 1270; with 4: 1256 / 1273 / 1285 /
+    - / 1314 / 1350 us; 5 rows, 600 / 800 / 1500 with 1, 3 and 4: 1114 / 1201 / -, 1161 / 1174 / 1242 and - / - / 1348; 10 rows, 800 with 1 and
+    3: 1329 and 1388; 16 rows, 400 / 980 with 1 and 2: 1308 / 1580 and 1443 / 1588).
     Never more than 4 slices (mean step time at contexts 250 / 500 / 1000 with 4 against 8 slices: Llama shape B=2
     843 against 856 us; Qwen3 shape B=2 1345 against 1362, B=4 1432 against 1433).  With heads of 64 and a cache of at
     most 2048 tokens one slice where the rule gives two: the only slice of its heads writes attn_out itself (Llama
@@ -352,4 +352,4 @@ def mi355x_scheduler(batch_size: int, shape: DecodeShape | None = None, *, merge
     shape = shape or LlamaConfig.shape()
     return BatchScheduler(shape, MI355X_WORKERS, batch_size, merge_in_last=merge_in_last, oproj_tile=residual_tile,
                           down_tile=residual_tile, skew_upgate=skew_upgate, split_kv_per_worker=0.5 if shape.head_dim <= 64 else 1.0,
-                          split_kv_cap=4, lone_slice_tokens=2048 if shape.head_dim <= 64 else 512 if batch_size > 4 else 0)
+                          split_kv_cap=4, lone_slice_tokens=2048 if shape.head_dim <= 64 else 0 if batch_size <= 4 else 640 if batch_size <= 8 else 1024)

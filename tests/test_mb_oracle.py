@@ -358,8 +358,8 @@ def test_two_stage_argmax_is_the_first_maximum():
 
 
 def test_slices_and_qkv_blocks_of_heads_of_128():
-    """MI355X template, a QKV block for every worker: one slice up to 512 tokens, then as many as the down projection's workers
-    hold, and where the slices fit there every QKV block on the other workers, two each; every block once."""
+    """MI355X template, a QKV block for every worker: one slice up to 640 tokens (1024 above 8 rows), then as many as the down projection's
+    workers hold, and where the slices fit there every QKV block on the other workers, two each; every block once."""
     from qimeng_megakernel_amd.decode_schedule.model_config import QWEN3_1_7B
 
     def plan(rows, capacity):
@@ -369,9 +369,10 @@ def test_slices_and_qkv_blocks_of_heads_of_128():
         blocks = [(i.tile_N_start_idx, i.tile_N_end_idx) for i in r if i.opcode() == 2]
         assert len(r) == 256 and [b for lo, hi in blocks for b in range(lo, hi)] == list(range(256))
         return p, next(k for k, i in enumerate(r) if i.opcode() == 2)
-    assert [plan(8, c) for c in (16, 512, 528, 1024, 1040, 4096)] == [(1, 128), (1, 128), (2, 128), (2, 128), (4, 8), (4, 8)]
-    assert [plan(5, c) for c in (512, 528, 2000)] == [(1, 128), (3, 128), (3, 128)]
-    assert [plan(6, c) for c in (1024, 1040)] == [(2, 128), (4, 6)] and plan(10, 700) == (3, 128) and plan(16, 700) == (2, 128)
+    assert [plan(8, c) for c in (16, 640, 656, 1024, 1040, 4096)] == [(1, 128), (1, 128), (2, 128), (2, 128), (4, 8), (4, 8)]
+    assert [plan(5, c) for c in (640, 656, 2000)] == [(1, 128), (3, 128), (3, 128)]
+    assert [plan(6, c) for c in (1024, 1040)] == [(2, 128), (4, 6)]
+    assert [plan(10, c) for c in (1024, 1040)] == [(1, 128), (3, 128)] and [plan(16, c) for c in (1024, 1040)] == [(1, 128), (2, 128)]
     assert plan(3, 300) == (4, 128)                       # the rows engine's range keeps the rule
     llama = [S.mi355x_scheduler(5, LLAMA_3_2_1B).partials_for_capacity(c) for c in (200, 1024, 1040)]
     assert llama == [1, 1, 4]
