@@ -592,39 +592,31 @@ using Factors = std::conditional_t<NORM, NormFactors<S::BM, S::kThreadCount, S::
 template <class S, bool NORM>
 constexpr int kFactorUnits = NORM ? (S::BM + 3) / 4 : 0;
 
-// Where a tile's quads of the residual lie: pass, then number -> token, column.
-template <class S>
-struct ResidualPlaces {
-  static constexpr int kPassM = S::WM / S::kPasses, kRowQuads = S::BN / 4, kRows = S::BM / S::kPasses, kTotal = kRows * kRowQuads;
-  const GemmArgs& g;
-  const int m0, n0, N, pass;
-  __device__ __forceinline__ bool operator()(int id, int& m, int& n) const {
-    const int r = id / kRowQuads;
-    m = m0 + r / kPassM * S::WM + pass * kPassM + r % kPassM;
-    n = n0 + id % kRowQuads * 4;
-    return m < g.M && n < N;
-  }
-};
-template <class T, class S, int BATCH>
-using TileStreams = ResidualQuads<T, S, BATCH, BATCH == 1 ? kMaxStreams : 4>;
 // A wave's accumulators -> epilogue, through its own part of LDS (quads of a row exchanged by its number): a lane then has eight neighbouring outputs of one
 // token, the same eight of every token it takes, and the lanes of a token write side by side (us, four outputs at a time with their columns worked out for each, by the whole
 // workgroup -> so: 2048 x 16384 x 2048 with gate and up 151 -> 141, 1531 x 16384 x 2048 129 -> 119).  Unit LDS of the array is one word beside it, behind that lie the factors of the tokens' norms.  (A kernel has one LDS
 // array: with two, this compiler waits for all requests before every read of the main loop, which costs half of the rate.)
-// `early`: the residual's streams; `begun`: they are asked for.
-template <class T, class S, int LDS, int BATCH, bool NORM>
-__device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int tile, int part, int m0, int n0, int N, v4u* lds, f32x4 (&acc)[S::kTn][S::kTm], TileStreams<T, S, BATCH>& early, bool begun) {
+template <class T, class S, int LDS, int BATCH = 1, bool NORM = false>
+__device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int tile, int part, int m0, int n0, int N, v4u* lds, f32x4 (&acc)[S::kTn][S::kTm]) {
   constexpr int kQuads = S::WN / 4, kPassM = S::WM / S::kPasses, kTm = S::kTm, kGroups = S::WN / 8;
   const float* factors = reinterpret_cast<const float*>(lds + LDS + 1);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
   f32x4 sums[S::kTn * kTm];
   constexpr int kRowQuads = S::BN / 4, kRows = S::BM / S::kPasses, kFewStreams = BATCH == 1 ? kMaxStreams : 4;
-  auto residual_at = [&](int pass) { return ResidualPlaces<S>{g, m0, n0, N, pass}; };
+  auto residual_at = [&](int pass) {
+    return [=, &g](int id, int& m, int& n) {
+      const int r = id / kRowQuads;
+      m = m0 + r / kPassM * S::WM + pass * kPassM + r % kPassM;
+      n = n0 + id % kRowQuads * 4;
+      return m < g.M && n < N;
+    };
+  };
   // (The first batch ahead of the sums, where registers allow.)
   constexpr bool kEarly = BATCH >= 4;
+  ResidualQuads<T, S, BATCH, kFewStreams> early{g};
   const bool few_streams = g.epi == EPI_RESIDUAL && g.streams <= kFewStreams;
-  if (kEarly && few_streams && !begun) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(0));
+  if (kEarly && few_streams) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(0));
   const bool multiplies = S::kLoaders == 0 || wave < S::kWavesM * S::kWavesN;
   __syncthreads();
 #pragma unroll
@@ -679,8 +671,14 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
         };
         __syncthreads();
         if (few_streams) {
-          if ((!kEarly || pass > 0) && !begun) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
-          early.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
+          if constexpr (kEarly) {
+            if (pass > 0) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
+            early.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
+          } else {
+            ResidualQuads<T, S, BATCH, kFewStreams> few{g};
+            few.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
+            few.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
+          }
         } else if constexpr (kFewStreams < kMaxStreams) {
           ResidualQuads<T, S, 1, kMaxStreams> many{g};
           many.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
@@ -711,12 +709,6 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
 #undef QMK_EPILOGUE
     __builtin_amdgcn_wave_barrier();
   }
-}
-
-template <class T, class S, int LDS, int BATCH = 1, bool NORM = false>
-__device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int tile, int part, int m0, int n0, int N, v4u* lds, f32x4 (&acc)[S::kTn][S::kTm]) {
-  TileStreams<T, S, BATCH> early{g};
-  finish_tile<T, S, LDS, BATCH, NORM>(g, group, tile, part, m0, n0, N, lds, acc, early, false);
 }
 
 // Which part of the product a workgroup takes.
@@ -939,13 +931,6 @@ __device__ __forceinline__ void few_tile(const GemmArgs& g, v4u* lds) {
       if (s < p.steps) stages.issue(s);
   }
   norm.put(g, lds + S::kLds + 1);
-  // The waves that multiply ask for nothing else: they hold the residual's streams from the start (us, the mean above: 10.8 -> 10.4).  In gemm_pipe, whose waves all wait for stages in the order
-  // of their requests, streams asked for a quad a step, or as few as one request a step, take longer than they save (96 x 128, 1531 x 2048 x 2048 with the streams 39.8 -> 41.6).
-  constexpr int kQuads = ResidualPlaces<S>::kTotal / (kMultipliers * 64);
-  static_assert(S::kPasses == 1 && kQuads == 1, "a quad a lane of the waves that multiply");
-  TileStreams<T, S, 2> streams{g};
-  const bool early = !NORM && g.epi == EPI_RESIDUAL && g.streams <= 4;
-  if (early && wave < kMultipliers) streams.begin(threadIdx.x, ResidualPlaces<S>::kTotal, S::kThreadCount, ResidualPlaces<S>{g, p.m0, p.n0, p.N, 0});
   if (wave >= kMultipliers) {
     int buf = S::kStages - 1;
     for (int s = 0; s < p.steps; ++s) {
@@ -972,7 +957,7 @@ __device__ __forceinline__ void few_tile(const GemmArgs& g, v4u* lds) {
       buf = buf + 1 == S::kStages ? 0 : buf + 1;
     }
   }
-  finish_tile<T, S, S::kLds, 2, NORM>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc, streams, early);
+  finish_tile<T, S, S::kLds, 2, NORM>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
 template <class T, class S, bool NORM = false>
 __global__ __launch_bounds__(S::kThreadCount, 1) void gemm_few(const GemmArgs g) {
