@@ -177,7 +177,6 @@ __device__ __forceinline__ float dpp_f32(float identity, float v) {
 constexpr int kDppQuadXor1 = 0xB1;       // quad_perm:[1,0,3,2]
 constexpr int kDppQuadXor2 = 0x4E;       // quad_perm:[2,3,0,1]
 constexpr int kDppHalfMirror = 0x141;    // row_half_mirror: lane i <-> 7-i within 8 lanes
-constexpr int kDppRowMirror = 0x140;     // row_mirror: lane i <-> 15-i within 16 lanes
 constexpr int kDppRowShr = 0x110;        // row_shr:n = 0x110 + n
 constexpr int kDppRowBcast15 = 0x142;    // lane 15 of a row -> every lane of the next row
 constexpr int kDppRowBcast31 = 0x143;    // lane 31 -> every lane of rows 2 and 3

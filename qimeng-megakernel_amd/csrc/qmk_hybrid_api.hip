@@ -449,7 +449,7 @@ inline int keys_cap(const QmkHybridArgs* a, const QmkHybridLayer& l) { return (s
 template <class T>
 struct PrefillBuffers {
   SplitBuffers split;
-  float *x, *u, *squares, *fa, *fb, *raw;
+  float *x, *u, *fa, *fb, *raw;
   ChunkBuffers state;
   T *p0, *p1, *p2, *rows, *kn, *vt;
   OperandRows<T> h, mix;
@@ -492,7 +492,6 @@ size_t prefill_buffers(const QmkHybridArgs* a, void* base, PrefillBuffers<T>* b)
   b->split = split_buffers(c);
   b->x = c.take<float>(P * a->streams * D);
   b->u = c.take<float>(P * D);
-  b->squares = c.take<float>(P * square_room(static_cast<int>(D)));
   b->fa = c.take<float>(fa);
   b->fb = c.take<float>(fb);
   b->raw = c.take<float>(raw);
@@ -517,38 +516,21 @@ template <class S, int KIND>
 constexpr bool priced_as_parts = kPartCosts[KIND].bm == S::BM && kPartCosts[KIND].bn == S::BN && S::kSplits;
 static_assert(priced_as_parts<Parts32, 0> && priced_as_parts<Parts64, 1> && priced_as_parts<PartsWide, 2>, "tiles of operands in parts and their prices");
 
-inline void cut_tokens(GemmArgs& g, int bm) {
-  g.tiles_m = static_cast<uint32_t>((g.M + bm - 1) / bm);
-  g.tiles_m_inverse = 0xffffffffu / g.tiles_m;
-}
-
-// Columns of the sums of squares that a product into the residual, M x width x K, leaves for the norm of the product behind it, M x N x width: 128, an eighth of the
-// values to read, where that one's tiles are of many tokens and the first one's as wide, else 16.  0: the norm is a launch of its own, which must not depend on M (a token's bits do not).  So it is
-// in fp32, where the rows are left in parts: the one workgroup that finishes a tile takes 2 us longer for them, and the launch saved is 5 (200 tokens, the whole portion the same).
-template <class T>
-int square_columns(int M, int width, int K, int N) {
-  if (sizeof(T) == 4 || width > kFactorWidth || width % 64 != 0 || K % 64 != 0) return 0;
-  const TileCost &first = kTileCosts[choose_tiles(M, width, K, 1, true)], &second = kTileCosts[choose_tiles(M, N, width, 1, false)];
-  return second.bm > kFewTokens && first.bn % 128 == 0 ? 128 : 16;
-}
-
-// NORM: of rows whose factors are still to come (GemmArgs::squares).
-template <class TA, class TW, class T, bool NORM = false>
+template <class TA, class TW, class T>
 void launch_gemm(GemmArgs g, const SplitBuffers& split, hipStream_t st) {
   const int n = std::max(g.N, g.last_n);
   g.tickets = split.tickets;
   g.partial = reinterpret_cast<float*>(split.partial);
   auto launch = [&](auto kernel, int bm, int bn, int threads) {
-    cut_tokens(g, bm);
-    hipLaunchKernelGGL(kernel, dim3((n + bn - 1) / bn * g.tiles_m * g.splits, 1, g.groups), dim3(threads), 0, st, g);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((n + bn - 1) / bn * ((g.M + bm - 1) / bm) * g.splits), 1, g.groups), dim3(threads), 0, st, g);
   };
   g.splits = 1;
   if constexpr (sizeof(TA) == 2 && sizeof(TW) == 2) {
     if (g.K % 64 == 0) {
-      auto direct = [&](auto s) { using S = decltype(s); launch(gemm_direct<T, S, NORM>, S::BM, S::BN, S::kThreadCount); };
-      auto pipe = [&](auto s) { using S = decltype(s); launch(gemm_pipe<T, S, 1, NORM>, S::BM, S::BN, S::kThreadCount); };
-      auto few = [&](auto s) { using S = decltype(s); launch(gemm_few<T, S, NORM>, S::BM, S::BN, S::kThreadCount); };
-      auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S, NORM>, S::BM, S::BN, S::kThreadCount); };
+      auto direct = [&](auto s) { using S = decltype(s); launch(gemm_direct<T, S>, S::BM, S::BN, S::kThreadCount); };
+      auto pipe = [&](auto s) { using S = decltype(s); launch(gemm_pipe<T, S>, S::BM, S::BN, S::kThreadCount); };
+      auto few = [&](auto s) { using S = decltype(s); launch(gemm_few<T, S>, S::BM, S::BN, S::kThreadCount); };
+      auto turns = [&](auto s) { using S = decltype(s); launch(gemm_turns<T, S>, S::BM, S::BN, S::kThreadCount); };
       switch (choose_tiles(g.M, n, g.K, g.groups, g.epi == EPI_RESIDUAL)) {
         case 0: pipe(Tiles64{}); break;
         case 1: pipe(Wide256{}); break;
@@ -605,8 +587,7 @@ void launch_gemm_pair(GemmPair pair, const SplitBuffers& split, hipStream_t st) 
   unsigned tiles = 0;
   for (GemmArgs& g : pair.g) {
     g.splits = 1;
-    cut_tokens(g, S::BM);
-    tiles = std::max(tiles, (g.N + S::BN - 1) / S::BN * g.tiles_m);
+    tiles = std::max(tiles, static_cast<unsigned>((g.N + S::BN - 1) / S::BN * ((g.M + S::BM - 1) / S::BM)));
   }
   hipLaunchKernelGGL((gemm_pipe_pair<T, S>), dim3(tiles, 2), dim3(S::kThreadCount), 0, st, pair);
 }
@@ -726,38 +707,20 @@ int prefill(const QmkHybridArgs* a) {
     return g;
   };
   auto whole = [](T* rows) { return Operand<T>{rows, 0}; };
-  // Behind it a sublayer whose first product has N rows and the norm `norm` (NULL: none of a kind that takes factors, or the last norm).  us, whole calls, a norm a launch (3.6 at 43 tokens, 5.5 at
-  // 1531) -> factors behind the product (up to 1 and 4 more for that one: 12288 x 2048 15.1 -> 15.5, 16384 x 2048 in three rounds of 256 x 128 98.4 -> 102.6), with fewer divisions in all products:
-  // 28 layers, 43 tokens behind 400, 2294 -> 2188; 16 layers, 1531 tokens 5034 -> 4946.
-  int columns = 0;      // of the sums of squares beside the rows in b.h (0: they are still to be normed, from b.u)
-  auto residual = [&](const u16* w, int K, const QmkHybridLayer& l, bool down, const float* norm, int N) {
+  auto residual = [&](const u16* w, int K, const QmkHybridLayer& l, bool down) {
     GemmArgs g = gemm_args(b.mix.of(K), K, w, D, K, l, EPI_RESIDUAL);
     g.f0 = b.x; g.f1 = b.u; g.down = down; g.next = down ? l.next2 : l.next1;
-    columns = norm != nullptr ? square_columns<T>(M, D, K, N) : 0;
-    if (columns > 0) {
-      g.norm = norm; g.h = b.h.at; g.squares = b.squares; g.square_columns = columns;
-    }
     launch_gemm<T, u16, T>(g, b.split, st);
-  };
-  // The first product of a sublayer, behind its norm.
-  auto norm_product = [&](const float* norm, const u16* w, int N, const QmkHybridLayer& l, int epi, T* out, T* out2, float* raw) {
-    GemmArgs g = gemm_args(b.h.of(D), D, w, N, D, l, epi);
-    g.out = out; g.out2 = out2; g.f0 = raw;
-    if (epi == EPI_GEGLU) g.out_part = b.mix.of(l.ff).part;
-    if (columns > 0) {
-      g.squares = b.squares; g.square_columns = columns; g.norm_width = a->width_true; g.norm_eps = a->eps;
-      if constexpr (sizeof(T) == 2) launch_gemm<T, u16, T, true>(g, b.split, st);
-    } else {
-      hipLaunchKernelGGL(norm_rows<T>, dim3(M), block, 0, st, b.u, norm, nullptr, M, D, a->width_true, a->eps, b.h.of(D));
-      launch_gemm<T, u16, T>(g, b.split, st);
-    }
   };
   for (int i = 0; i < a->num_layers; ++i) {
     const QmkHybridLayer& l = a->layers[i];
     const int W = l.mix_width;
-    const QmkHybridLayer* next = i + 1 < a->num_layers && a->layers[i + 1].type != QMK_MIXER_WKV ? a->layers + i + 1 : nullptr;
+    if (l.type != QMK_MIXER_WKV)
+      hipLaunchKernelGGL(norm_rows<T>, dim3(M), block, 0, st, b.u, l.norm1, nullptr, M, D, a->width_true, a->eps, b.h.of(D));
     if (l.type == QMK_MIXER_RGLRU) {
-      norm_product(l.norm1, l.in_w, l.in_rows, l, EPI_RGLRU_IN, b.p0, b.p1, nullptr);
+      GemmArgs g = gemm_args(b.h.of(D), D, l.in_w, l.in_rows, D, l, EPI_RGLRU_IN);
+      g.out = b.p0; g.out2 = b.p1;
+      launch_gemm<T, u16, T>(g, b.split, st);
       const long long quads = static_cast<long long>(M) * (W / 4);
       hipLaunchKernelGGL(causal_conv<T>, dim3(static_cast<unsigned>((quads + kPfThreads - 1) / kPfThreads)), block, 0, st, b.p1, l, a->slot, a->flip, M, b.p2);
       GemmArgs e = gemm_args(whole(b.p2), W, l.mid_w, 2 * l.block_dim, l.block_dim, l, EPI_LRU_GATES);
@@ -766,7 +729,9 @@ int prefill(const QmkHybridArgs* a) {
       launch_gemm<T, u16, T>(e, b.split, st);
       hipLaunchKernelGGL(lru_scan<T>, dim3(W / kScanChannels), dim3(kScanChannels * kScanRuns), 0, st, b.fa, b.fb, b.p0, l, a->slot, M, b.mix.of(W));
     } else if (l.type == QMK_MIXER_LATENT) {
-      norm_product(l.norm1, l.in_w, l.in_rows, l, EPI_LATENT_IN, b.p0, b.p1, b.raw);
+      GemmArgs g = gemm_args(b.h.of(D), D, l.in_w, l.in_rows, D, l, EPI_LATENT_IN);
+      g.out = b.p0; g.out2 = b.p1; g.f0 = b.raw;
+      launch_gemm<T, u16, T>(g, b.split, st);
       const int first = std::max(0, a->position + 1 - l.window), keys = a->position + M - first, cap = keys_cap(a, l), width = l.rank + l.rot_dim;
       hipLaunchKernelGGL(latent_rows<T>, dim3(keys), block, 0, st, b.raw, l, a->slot, first, a->position, a->eps, b.rows);
       GemmArgs k = gemm_args(whole(b.rows), width, l.uk_w, l.heads * l.head_dim, l.rank, l, EPI_STORE);
@@ -799,14 +764,13 @@ int prefill(const QmkHybridArgs* a) {
       run_chunks<T, CHUNK_WKV>(c, st);
       hipLaunchKernelGGL(wkv_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.raw, b.p0, l, M, a->eps, b.mix.of(W));
     }
-    const float* next_norm = next != nullptr ? next->norm1 : nullptr;
-    const int next_rows = next != nullptr ? next->in_rows : 0;
+    residual(l.o_w, W, l, false);
     if (l.has_mlp) {
-      residual(l.o_w, W, l, false, l.norm2, 2 * l.ff);
-      norm_product(l.norm2, l.mlp_w, 2 * l.ff, l, EPI_GEGLU, b.mix.at, nullptr, nullptr);
-      residual(l.down_w, l.ff, l, true, next_norm, next_rows);
-    } else {
-      residual(l.o_w, W, l, false, next_norm, next_rows);
+      hipLaunchKernelGGL(norm_rows<T>, dim3(M), block, 0, st, b.u, l.norm2, nullptr, M, D, a->width_true, a->eps, b.h.of(D));
+      GemmArgs g = gemm_args(b.h.of(D), D, l.mlp_w, 2 * l.ff, D, l, EPI_GEGLU);
+      g.out = b.mix.at; g.out_part = b.mix.of(l.ff).part;
+      launch_gemm<T, u16, T>(g, b.split, st);
+      residual(l.down_w, l.ff, l, true);
     }
     if (a->layer_out != nullptr)
       hipLaunchKernelGGL(sum_streams, dim3(M), block, 0, st, b.x, S, D, a->layer_out + static_cast<size_t>(i) * M * D);

@@ -139,22 +139,9 @@ struct GemmArgs {
   float* partial;        // sums of the parts of a product that is cut along K, and a zero per tile
   int32_t* tickets;
   int splits;
-  uint32_t tiles_m, tiles_m_inverse;       // tiles of tokens, (2^32 - 1) / tiles_m
   size_t a_part;         // Operand::part of a (last: the bf16 mode reads neither, and its first cache lines stay as they are)
   size_t out_part;       // EPI_GEGLU: Operand::part of out
-  // bf16: a norm's factor is one number a token, so it need not be applied to a product's rows but to its outputs.  Where `norm` is given, EPI_RESIDUAL leaves the next sublayer's input times
-  // its norm's weights as the next product's rows (`h`) and sums of its squares over `square_columns` columns, from which that product (NORM) takes the factors.
-  const float* norm;
-  void* h;
-  float* squares;        // [M][square_room(width)]
-  int square_columns, norm_width;
-  float norm_eps;
 };
-
-// Squares are added as a tree over the columns, whatever part of it a workgroup adds up: in one order for every kind of tile.
-constexpr int kFactorWidth = 2048;      // most columns of a token whose norm is a factor: sixteen runs of 128
-__host__ __device__ constexpr int square_room(int width) { return (width + 127) / 128 * 8; }
-constexpr int kFewTokens = 64;      // of a tile that takes sums over 16 columns
 
 template <class T>
 __device__ __forceinline__ void store4(T* at, f32x4 v) {
@@ -430,13 +417,10 @@ __global__ __launch_bounds__(kPfThreads) void clear_tickets(int32_t* tickets, in
 // All streams of the residual for quads id, id + step, .. of a tile, `BATCH` at a time: the next batch's streams are asked for before this one's are mixed, the first
 // one's (`begin`) ahead of the products' exchange where registers allow.  Few workgroups make it a chain of trips to memory, many are bound by its bytes (us, one
 // quad at a time with coefficients read among the stores -> now: 200 x 2048 x 64 on tiles of 64 x 128 in fp32 22.5 -> 14.9; 1531 x 2048 x 2048 on Turns96 45 -> 34).
-template <class T, class S_, int BATCH, int STREAMS>
+template <int BATCH, int STREAMS>
 struct ResidualQuads {
-  static constexpr int BN = S_::BN;
-  static constexpr bool kSameColumns = S_::kThreadCount % (BN / 4) == 0;      // a thread's quads lie under one another
-  static constexpr bool kFolds = sizeof(T) == 2;
   const GemmArgs& g;
-  f32x4 old[BATCH][STREAMS], weight;
+  f32x4 old[BATCH][STREAMS];
 
   template <class At>
   __device__ __forceinline__ void load(f32x4 (&to)[BATCH][STREAMS], int id, int total, int step, At&& at) const {
@@ -452,25 +436,7 @@ struct ResidualQuads {
     }
   }
   template <class At>
-  __device__ __forceinline__ void begin(int id, int total, int step, At&& at) {
-    load(old, id, total, step, at);
-    if (kFolds && kSameColumns && g.norm != nullptr) {
-      int m, n;
-      at(id, m, n);
-      weight = read4(g.norm + min(n, g.width - 4));
-    }
-  }
-  // Over the lanes that hold neighbouring quads of a token's columns.
-  __device__ __forceinline__ float sum_of_columns(float v) const {
-    v += dpp_f32<kDppQuadXor1>(0.f, v);
-    v += dpp_f32<kDppQuadXor2>(0.f, v);
-    if (BN % 128 == 0 && g.square_columns == 128) {
-      v += dpp_f32<kDppHalfMirror>(0.f, v);
-      v += dpp_f32<kDppRowMirror>(0.f, v);
-      v += __shfl_xor(v, 16);
-    }
-    return v;
-  }
+  __device__ __forceinline__ void begin(int id, int total, int step, At&& at) { load(old, id, total, step, at); }
   template <class At, class Value>
   __device__ __forceinline__ void run(int id, int total, int step, At&& at, Value&& value) {
     const QmkHybridLayer& l = g.layer;
@@ -483,11 +449,8 @@ struct ResidualQuads {
       load(ahead, id + BATCH * step, total, step, at);
 #pragma unroll
       for (int b = 0; b < BATCH; ++b) {
-        if (id + b * step >= total) continue;      // (all lanes of a wave)
         int m, n;
-        const bool there = at(id + b * step, m, n);
-        float square = 0.f;
-        if (there) {
+        if (id + b * step < total && at(id + b * step, m, n)) {
           const f32x4 v = value(id + b * step);
           float* x = g.f0 + static_cast<size_t>(m) * S * D + n;
           f32x4 u = {};
@@ -502,18 +465,7 @@ struct ResidualQuads {
               u += now * next[t];
             }
           }
-          const size_t place = static_cast<size_t>(m) * D + n;
-          if (!kFolds || g.norm == nullptr) {
-            store4(g.f1 + place, u);
-          } else {
-            if (!kSameColumns) weight = read4(g.norm + n);
-            store4(static_cast<T*>(g.h) + place, u * weight);
-            square = (u[0] * u[0] + u[1] * u[1]) + (u[2] * u[2] + u[3] * u[3]);
-          }
-        }
-        if (kFolds && g.norm != nullptr) {
-          square = sum_of_columns(square);
-          if (there && n % g.square_columns == 0) g.squares[static_cast<size_t>(m) * square_room(D) + n / g.square_columns] = square;
+          store4(g.f1 + static_cast<size_t>(m) * D + n, u);
         }
       }
 #pragma unroll
@@ -524,82 +476,13 @@ struct ResidualQuads {
   }
 };
 
-// The factors of a tile's tokens' norms -> LDS.  Asked for ahead of a product's first stages, all at once, and put there ahead of its first barrier.  FEW: from sums over 16 columns always,
-// sixteen lanes a token; otherwise four lanes a token, and such sums are added up on the spot (a product of few tokens left them to one of larger tiles).
-template <int BM, int THREADS, bool FEW>
-struct NormFactors {
-  static constexpr int kLanes = FEW ? 16 : 4, kEach = THREADS / kLanes, kPasses = (BM + kEach - 1) / kEach;
-  static_assert(kPasses <= kLanes, "a lane a pass");
-  f32x4 held[kPasses][FEW ? 2 : 1];
-  __device__ __forceinline__ NormFactors(const GemmArgs& g, int m0) {
-    const int lane = threadIdx.x % kLanes, row0 = m0 + threadIdx.x / kLanes, room = square_room(g.K);
-    auto row = [&](int pass) { return g.squares + static_cast<size_t>(min(row0 + pass * kEach, g.M - 1)) * room; };
-    if constexpr (FEW) {
-#pragma unroll
-      for (int pass = 0; pass < kPasses; ++pass)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) held[pass][i] = read4(row(pass) + min(lane * 8 + i * 4, room - 4));
-    } else if (g.square_columns == 128) {
-#pragma unroll
-      for (int pass = 0; pass < kPasses; ++pass) held[pass][0] = read4(row(pass) + min(lane * 4, room - 4));
-    } else {
-#pragma unroll
-      for (int pass = 0; pass < kPasses; ++pass)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float* from = row(pass) + min((lane * 4 + i) * 8, room - 8);
-          held[pass][0][i] = tree(g, lane * 4 + i, read4(from), read4(from + 4));
-        }
-    }
-  }
-  static __device__ __forceinline__ float tree(const GemmArgs& g, int run, f32x4 lo, f32x4 hi) {      // of a run of 128 columns, absent ones zeros
-    auto there = [&](float v, int i) { return run * 8 + i < g.K / 16 ? v : 0.f; };
-    return ((there(lo[0], 0) + there(lo[1], 1)) + (there(lo[2], 2) + there(lo[3], 3))) + ((there(hi[0], 4) + there(hi[1], 5)) + (there(hi[2], 6) + there(hi[3], 7)));
-  }
-  // (Written by hand: ahead of the compiler's own write it would wait for all stages under way.)
-  __device__ __forceinline__ void put(const GemmArgs& g, v4u* factors) const {
-    const int lane = threadIdx.x % kLanes, runs = (g.K + 127) / 128;
-    float sum = 0.f;      // lane p: of pass p's token
-#pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass) {
-      float v;
-      if constexpr (FEW) {
-        v = tree(g, lane, held[pass][0], held[pass][1]);
-      } else {
-        auto there = [&](int i) { return lane * 4 + i < runs ? held[pass][0][i] : 0.f; };
-        v = (there(0) + there(1)) + (there(2) + there(3));
-      }
-      v += dpp_f32<kDppQuadXor1>(0.f, v);
-      v += dpp_f32<kDppQuadXor2>(0.f, v);
-      if constexpr (FEW) {
-        v += dpp_f32<kDppHalfMirror>(0.f, v);
-        v += dpp_f32<kDppRowMirror>(0.f, v);
-      }
-      sum = lane == pass ? v : sum;
-    }
-    const uint32_t r = lane * kEach + threadIdx.x / kLanes, to = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) v4u*)factors)) + r * 4;
-    const float factor = 1.f / sqrtf(sum / g.norm_width + g.norm_eps);
-    if (lane < kPasses && r < BM) asm volatile("ds_write_b32 %0, %1" ::"v"(to), "v"(factor) : "memory");
-  }
-};
-// Nothing of it.
-struct NoFactors {
-  __device__ __forceinline__ NoFactors(const GemmArgs&, int) {}
-  __device__ __forceinline__ void put(const GemmArgs&, v4u*) const {}
-};
-template <class S, bool NORM>
-using Factors = std::conditional_t<NORM, NormFactors<S::BM, S::kThreadCount, S::BM <= kFewTokens>, NoFactors>;
-template <class S, bool NORM>
-constexpr int kFactorUnits = NORM ? (S::BM + 3) / 4 : 0;
-
 // A wave's accumulators -> epilogue, through its own part of LDS (quads of a row exchanged by its number): a lane then has eight neighbouring outputs of one
 // token, the same eight of every token it takes, and the lanes of a token write side by side (us, four outputs at a time with their columns worked out for each, by the whole
-// workgroup -> so: 2048 x 16384 x 2048 with gate and up 151 -> 141, 1531 x 16384 x 2048 129 -> 119).  Unit LDS of the array is one word beside it, behind that lie the factors of the tokens' norms.  (A kernel has one LDS
+// workgroup -> so: 2048 x 16384 x 2048 with gate and up 151 -> 141, 1531 x 16384 x 2048 129 -> 119).  Unit LDS of the array is one word beside it.  (A kernel has one LDS
 // array: with two, this compiler waits for all requests before every read of the main loop, which costs half of the rate.)
-template <class T, class S, int LDS, int BATCH = 1, bool NORM = false>
+template <class T, class S, int LDS, int BATCH = 1>
 __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int tile, int part, int m0, int n0, int N, v4u* lds, f32x4 (&acc)[S::kTn][S::kTm]) {
   constexpr int kQuads = S::WN / 4, kPassM = S::WM / S::kPasses, kTm = S::kTm, kGroups = S::WN / 8;
-  const float* factors = reinterpret_cast<const float*>(lds + LDS + 1);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
   f32x4 sums[S::kTn * kTm];
@@ -614,7 +497,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
   };
   // (The first batch ahead of the sums, where registers allow.)
   constexpr bool kEarly = BATCH >= 4;
-  ResidualQuads<T, S, BATCH, kFewStreams> early{g};
+  ResidualQuads<BATCH, kFewStreams> early{g};
   const bool few_streams = g.epi == EPI_RESIDUAL && g.streams <= kFewStreams;
   if (kEarly && few_streams) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(0));
   const bool multiplies = S::kLoaders == 0 || wave < S::kWavesM * S::kWavesN;
@@ -646,23 +529,8 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
       const Epilogue<T, decltype(epi)::value> put(g, group, n);
       const int end = min(kPassM, g.M - first);
 #pragma unroll 2
-      for (int r = lane / kGroups; r < end; r += kEachTime) {
-        f32x4 lo = out[place(r, lane % kGroups * 2)], hi = out[place(r, lane % kGroups * 2 + 1)];
-        if constexpr (NORM) {
-          lo *= factors[first - m0 + r];
-          hi *= factors[first - m0 + r];
-        }
-        put(first + r, lo, hi);
-      }
+      for (int r = lane / kGroups; r < end; r += kEachTime) put(first + r, out[place(r, lane % kGroups * 2)], out[place(r, lane % kGroups * 2 + 1)]);
     };
-#define QMK_EPILOGUE(EPI) case EPI: rows(std::integral_constant<int, EPI>{}); break;
-    if constexpr (NORM) {
-      switch (g.epi) {
-        QMK_EPILOGUE(EPI_RGLRU_IN)
-        QMK_EPILOGUE(EPI_LATENT_IN)
-        QMK_EPILOGUE(EPI_GEGLU)
-      }
-    } else {
     switch (g.epi) {
       case EPI_RESIDUAL: {      // the streams of a token are long runs: all waves take rows of the whole tile
         auto product = [&](int id) {
@@ -675,18 +543,19 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
             if (pass > 0) early.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
             early.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
           } else {
-            ResidualQuads<T, S, BATCH, kFewStreams> few{g};
+            ResidualQuads<BATCH, kFewStreams> few{g};
             few.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
             few.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
           }
         } else if constexpr (kFewStreams < kMaxStreams) {
-          ResidualQuads<T, S, 1, kMaxStreams> many{g};
+          ResidualQuads<1, kMaxStreams> many{g};
           many.begin(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass));
           many.run(tid, kRows * kRowQuads, S::kThreadCount, residual_at(pass), product);
         }
         __syncthreads();
         break;
       }
+#define QMK_EPILOGUE(EPI) case EPI: rows(std::integral_constant<int, EPI>{}); break;
       QMK_EPILOGUE(EPI_STORE)
       QMK_EPILOGUE(EPI_STORE_VALUES)
       QMK_EPILOGUE(EPI_RGLRU_IN)
@@ -704,9 +573,8 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
       QMK_EPILOGUE(EPI_SIGMOID)
       QMK_EPILOGUE(EPI_GLA_IN)
       QMK_EPILOGUE(EPI_GLA_DECAY)
-    }
-    }
 #undef QMK_EPILOGUE
+    }
     __builtin_amdgcn_wave_barrier();
   }
 }
@@ -715,25 +583,19 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& g, int group, int ti
 struct Place {
   int group, tile, part, m0, n0, N, first, steps;
 };
-// T: of the activations; in bf16 no product is cut.  (A division is some forty instructions ahead of a workgroup's first request.)
-template <class T, class S>
+template <class S>
 __device__ __forceinline__ Place place_of(const GemmArgs& g) {
-  constexpr bool CUT = sizeof(T) == 4;
   Place p;
   p.group = blockIdx.z;
   p.N = p.group == g.groups - 1 ? g.last_n : g.N;
-  const int id = xcd_order(blockIdx.x, gridDim.x), tile = CUT ? id / g.splits : id, all = (g.K + S::BK - 1) / S::BK;
-  uint32_t n = __umulhi(static_cast<uint32_t>(tile), g.tiles_m_inverse), m = tile - n * g.tiles_m;      // at most one too few
-  if (m >= g.tiles_m) {
-    ++n;
-    m -= g.tiles_m;
-  }
-  p.part = CUT ? id % g.splits : 0;
-  p.m0 = static_cast<int>(m) * S::BM;
-  p.n0 = static_cast<int>(n) * S::BN;
-  p.tile = CUT ? p.group * (gridDim.x / g.splits) + tile : 0;
-  p.first = CUT ? all * p.part / g.splits : 0;
-  p.steps = CUT ? all * (p.part + 1) / g.splits - p.first : all;
+  const int id = xcd_order(blockIdx.x, gridDim.x), tiles_m = (g.M + S::BM - 1) / S::BM, tile = id / g.splits;
+  p.part = id % g.splits;
+  p.m0 = tile % tiles_m * S::BM;
+  p.n0 = tile / tiles_m * S::BN;
+  p.tile = p.group * (gridDim.x / g.splits) + tile;
+  const int all = (g.K + S::BK - 1) / S::BK;
+  p.first = all * p.part / g.splits;
+  p.steps = all * (p.part + 1) / g.splits - p.first;
   return p;
 }
 
@@ -869,19 +731,18 @@ __device__ __forceinline__ void resolve_undefined(const GemmArgs& g, const Place
 
 // out[m][n] = sum_k a[m][k] w[n][k], bf16 x bf16, K a multiple of BK.  The weights are the matrix instruction's first operand,
 // so a lane ends up with four consecutive outputs of one token.  Two to eight waves; several workgroups share a CU where LDS has room.
-template <class T, class S, bool NORM>
-__device__ __forceinline__ void direct_tile(const GemmArgs& g, v4u* lds) {
+template <class T, class S>
+__global__ __launch_bounds__(S::kThreadCount, S::kThreadCount == 512 ? 4 : 1) void gemm_direct(const GemmArgs g) {
   constexpr int kAhead = S::kStages - 1;
+  __shared__ __align__(16) v4u lds[S::kLds + 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % S::kWavesM, wn = wave / S::kWavesM;
-  const Place p = place_of<T, S>(g);
+  const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
   Stages<S> stages(g, p, lds, wave);
-  const Factors<S, NORM> norm(g, p.m0);
   f32x4 acc[S::kTn][S::kTm] = {};
 #pragma unroll
   for (int s = 0; s < kAhead; ++s)
     if (s < p.steps) stages.issue(s);
-  norm.put(g, lds + S::kLds + 1);
   int buf = 0;
   for (int s = 0; s < p.steps; ++s) {
     // Everything up to this step's stage has landed; the barrier makes that true of every wave's part, and says that the
@@ -899,23 +760,19 @@ __device__ __forceinline__ void direct_tile(const GemmArgs& g, v4u* lds) {
     }
     buf = buf + 1 == S::kStages ? 0 : buf + 1;
   }
-  finish_tile<T, S, S::kLds, 2, NORM>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
-}
-template <class T, class S, bool NORM = false>
-__global__ __launch_bounds__(S::kThreadCount, S::kThreadCount == 512 ? 4 : 1) void gemm_direct(const GemmArgs g) {
-  __shared__ __align__(16) v4u lds[S::kLds + 1 + kFactorUnits<S, NORM>];
-  direct_tile<T, S, NORM>(g, lds);
+  finish_tile<T, S, S::kLds, 2>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
 
 // The same for the fewest tokens, whose workgroups have few waves that multiply: on their chain of products, fragments and barriers requests for stages take as long
 // as the products, so other waves make them.  A stage has landed for everybody behind the barrier that its loaders reach when it has landed for them; fragments of 32
 // columns are read while the 32 before are multiplied (us, the mean of 43 x 2048 x 2048 and x 6144 with the residual's streams, inside a portion: 12.0 with two waves that do both -> 10.8; four
 // loaders 10.9, three or six stages 11.5 and 11.1; the same with all weights in the last cache, so what is left is not memory's rate).
-template <class T, class S, bool NORM>
-__device__ __forceinline__ void few_tile(const GemmArgs& g, v4u* lds) {
+template <class T, class S>
+__global__ __launch_bounds__(S::kThreadCount, 1) void gemm_few(const GemmArgs g) {
   constexpr int kAhead = S::kStages - 1, kMultipliers = S::kWavesM * S::kWavesN;
+  __shared__ __align__(16) v4u lds[S::kLds + 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % S::kWavesM, wn = wave / S::kWavesM % S::kWavesN;
-  const Place p = place_of<T, S>(g);
+  const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
   Stages<S, 1, S::kLoaders * 64> stages(g, p, lds, wave - kMultipliers);
   f32x4 acc[S::kTn][S::kTm] = {};
@@ -924,14 +781,10 @@ __device__ __forceinline__ void few_tile(const GemmArgs& g, v4u* lds) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  const Factors<S, NORM> norm(g, p.m0);
   if (wave >= kMultipliers) {
 #pragma unroll
     for (int s = 0; s < kAhead; ++s)
       if (s < p.steps) stages.issue(s);
-  }
-  norm.put(g, lds + S::kLds + 1);
-  if (wave >= kMultipliers) {
     int buf = S::kStages - 1;
     for (int s = 0; s < p.steps; ++s) {
       if (s + kAhead - 1 < p.steps) stages.template wait<kAhead - 1>();
@@ -957,12 +810,7 @@ __device__ __forceinline__ void few_tile(const GemmArgs& g, v4u* lds) {
       buf = buf + 1 == S::kStages ? 0 : buf + 1;
     }
   }
-  finish_tile<T, S, S::kLds, 2, NORM>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
-}
-template <class T, class S, bool NORM = false>
-__global__ __launch_bounds__(S::kThreadCount, 1) void gemm_few(const GemmArgs g) {
-  __shared__ __align__(16) v4u lds[S::kLds + 1 + kFactorUnits<S, NORM>];
-  few_tile<T, S, NORM>(g, lds);
+  finish_tile<T, S, S::kLds, 2>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
 
 // Scheduling of a block of matrix instructions: one LDS read ahead of each of the first, the requests for a stage among the rest.
@@ -988,13 +836,13 @@ __device__ __forceinline__ void interleave() {
 // accumulators in the other half of the file and moves them at every step.)
 template <class S, int PARTS>
 constexpr int kPipeLds = S::kStages * Stages<S, PARTS>::kUnits > S::kLds ? S::kStages * Stages<S, PARTS>::kUnits : S::kLds;
-template <class T, class S, int PARTS, bool NORM>
+template <class T, class S, int PARTS>
 __device__ __forceinline__ void pipe_tile(const GemmArgs& g, v4u* lds) {
   static_assert(S::kSteps % 2 == 0 && S::kStages >= 2, "pairs of matrix steps a stage");
   constexpr int kDeep = S::kStages, kProducts = PARTS * S::kTm * S::kTn, kReads = PARTS * S::kTm + S::kTn, kRequests = Stages<S, PARTS>::kLoads, kLds = kPipeLds<S, PARTS>;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
-  const Place p = place_of<T, S>(g);
+  const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
   Stages<S, PARTS> stages(g, p, lds, wave);
   auto barrier = [] {
@@ -1009,11 +857,9 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, v4u* lds) {
   struct Fragments {
     Frag<u16> a[PARTS][S::kTm], w[S::kTn];
   } f[2];
-  const Factors<S, NORM> norm(g, p.m0);
 #pragma unroll
   for (int s = 0; s < kDeep; ++s)
     if (s < p.steps) stages.issue(s);
-  norm.put(g, lds + kLds + 1);
   if (kDeep <= p.steps) stages.template wait<kDeep - 1>();
   else wait_known<0>();
   barrier();
@@ -1057,12 +903,12 @@ __device__ __forceinline__ void pipe_tile(const GemmArgs& g, v4u* lds) {
       for (int i = 0; i < S::kTm; ++i) acc[j][i] += sums[kSums - 1][j][i];
     resolve_undefined<S>(g, p, wm, wn, acc);
   }
-  finish_tile<T, S, kLds, 4, NORM>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
+  finish_tile<T, S, kLds, 4>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
-template <class T, class S, int PARTS = 1, bool NORM = false>
+template <class T, class S, int PARTS = 1>
 __global__ __launch_bounds__(512, 2) void gemm_pipe(const GemmArgs g) {
-  __shared__ __align__(16) v4u lds[kPipeLds<S, PARTS> + 1 + kFactorUnits<S, NORM>];
-  pipe_tile<T, S, PARTS, NORM>(g, lds);
+  __shared__ __align__(16) v4u lds[kPipeLds<S, PARTS> + 1];
+  pipe_tile<T, S, PARTS>(g, lds);
 }
 // Two products that need nothing of each other.
 struct GemmPair {
@@ -1071,19 +917,20 @@ struct GemmPair {
 template <class T, class S>
 __global__ __launch_bounds__(512, 2) void gemm_pipe_pair(const GemmPair pair) {
   __shared__ __align__(16) v4u lds[kPipeLds<S, 1> + 1];
-  pipe_tile<T, S, 1, false>(pair.g[blockIdx.y], lds);
+  pipe_tile<T, S, 1>(pair.g[blockIdx.y], lds);
 }
 
 // The same with eight waves, one workgroup a CU.  Two waves share a SIMD's matrix unit, and the halves of the workgroup take
 // turns: while one multiplies, the other reads its next fragments; a barrier ends each turn, and the second half starts one
 // turn late.
-template <class T, class S, bool NORM>
-__device__ __forceinline__ void turns_tile(const GemmArgs& g, v4u* lds) {
+template <class T, class S>
+__global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
   static_assert(S::kThreadCount == 512 && S::kStages >= 3, "one turn a step, the next stage has landed before it");
   constexpr int kAhead = S::kStages - 1;
+  __shared__ __align__(16) v4u lds[S::kLds + 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave % S::kWavesM, wn = wave / S::kWavesM;
-  const Place p = place_of<T, S>(g);
+  const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
   Stages<S> stages(g, p, lds, wave);
   auto barrier = [] {
@@ -1092,12 +939,10 @@ __device__ __forceinline__ void turns_tile(const GemmArgs& g, v4u* lds) {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
   };
-  const Factors<S, NORM> norm(g, p.m0);
   f32x4 acc[S::kTn][S::kTm] = {};
 #pragma unroll
   for (int s = 0; s < kAhead; ++s)
     if (s < p.steps) stages.issue(s);
-  norm.put(g, lds + S::kLds + 1);
   if (kAhead - 1 < p.steps) stages.template wait<kAhead - 1>();
   else wait_outstanding<0>();
   barrier();                       // stage 0 is there
@@ -1121,12 +966,7 @@ __device__ __forceinline__ void turns_tile(const GemmArgs& g, v4u* lds) {
     buf = buf + 1 == S::kStages ? 0 : buf + 1;
   }
   if (wave < 4) barrier();
-  finish_tile<T, S, S::kLds, 1, NORM>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
-}
-template <class T, class S, bool NORM = false>
-__global__ __launch_bounds__(512, 2) void gemm_turns(const GemmArgs g) {
-  __shared__ __align__(16) v4u lds[S::kLds + 1 + kFactorUnits<S, NORM>];
-  turns_tile<T, S, NORM>(g, lds);
+  finish_tile<T, S, S::kLds>(g, p.group, p.tile, p.part, p.m0, p.n0, p.N, lds, acc);
 }
 
 // ---- products with an fp32 side, and bf16 ones of any K ----
@@ -1144,7 +984,7 @@ __global__ __launch_bounds__(kPfThreads) void gemm(const GemmArgs g) {
   constexpr int kStage = kPa * kUnitsA + kPw * kUnitsW, kLds = BUFFERS * kStage > S::kOutUnits ? BUFFERS * kStage : S::kOutUnits;
   __shared__ __align__(16) v4u lds[kLds + 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
-  const Place p = place_of<T, S>(g);
+  const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
   const TA* a = static_cast<const TA*>(g.a) + p.group * g.a_step;
   const TW* w = static_cast<const TW*>(g.w) + p.group * g.w_step;
@@ -1276,7 +1116,7 @@ __global__ __launch_bounds__(kPfThreads) void gemm_short(const GemmArgs g) {
   static_assert(64 * (kRowA + kRowW) <= S::kLds, "both tiles");
   v4u *la = lds, *lw = lds + 64 * kRowA;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
-  const Place p = place_of<T, S>(g);
+  const Place p = place_of<S>(g);
   if (p.n0 >= p.N) return;
   auto place = [](int r, int unit, int row_units) { return r * row_units + (unit ^ ((r & 7) * (row_units / 8))); };
   auto stage = [&](auto* from, v4u* to, int row_units, int unit, int row0, int rows, long long ld) {
