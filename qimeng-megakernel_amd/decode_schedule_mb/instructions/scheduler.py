@@ -342,7 +342,7 @@ def mi355x_scheduler(batch_size: int, shape: DecodeShape | None = None, *, merge
     QKV blocks then keep off the slices' workers, and those ask for four tiles a wave ahead (8 rows, contexts 130 / 350 / 500 / 600 / 700 /
     950 with 1 and 2 slices: 1092 / 1113 / 1153 / 1174 / 1225 / 1344, 1185 / 1188 / 1200 / 1200 / 1215 / 1270; with 4: 1256 / 1273 / 1285 /
     - / 1314 / 1350 us; 5 rows, 600 / 800 / 1500 with 1, 3 and 4: 1114 / 1201 / -, 1161 / 1174 / 1242 and - / - / 1348; 10 rows, 800 with 1 and
-    3: 1329 and 1388; 16 rows, 400 / 980 with 1 and 2: 1308 / 1580 and 1443 / 1588).
+    3: 1329 and 1388; 16 rows, 980 with 1 and 2: 1580 and 1588).
     Never more than 4 slices (mean step time at contexts 250 / 500 / 1000 with 4 against 8 slices: Llama shape B=2
     843 against 856 us; Qwen3 shape B=2 1345 against 1362, B=4 1432 against 1433).  With heads of 64 and a cache of at
     most 2048 tokens one slice where the rule gives two: the only slice of its heads writes attn_out itself (Llama
