@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kThreads, 1) void decode_megakernel(const Params p_
 // The batch route's interpreter: same queue walk, the ten opcodes of qmk_mb_ops.h, the reference's
 // counter protocol per batch row (…/A100/multi_batch/decode_kernel/mk.cu).  Per-row positions and
 // activity are read once per launch.
-template <class M>
+template <class M, int kTilesAhead>
 __global__ __launch_bounds__(kThreads, 1) void decode_megakernel_batch(const Params p) {
   __shared__ mb::Smem<M> s;
   if (threadIdx.x < 8) s.ctl[threadIdx.x] = 0;
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(kThreads, 1) void decode_megakernel_batch(const Par
       case mb::OP_MLP_RMS:
       case mb::OP_LM_RMS: [[clang::always_inline]] ok = mb::op_rms_row<M>(p, s, c); break;
       case mb::OP_QKV: [[clang::always_inline]] ok = mb::op_qkv<M>(p, s, c); break;
-      case mb::OP_SPLITKV: [[clang::always_inline]] ok = mb::op_splitkv<M>(p, s, c); break;
+      case mb::OP_SPLITKV: [[clang::always_inline]] ok = mb::op_splitkv<M, kTilesAhead>(p, s, c); break;
       case mb::OP_REDUCE: [[clang::always_inline]] ok = mb::op_reduce<M>(p, s, c); break;
       case mb::OP_OPROJ: [[clang::always_inline]] ok = mb::op_oproj<M>(p, s, c); break;
       case mb::OP_UPGATE: [[clang::always_inline]] ok = mb::op_upgate<M>(p, s, c); break;
@@ -642,11 +642,13 @@ int device_info(DeviceInfo** out) {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decode_megakernel<Llama1B>, kThreads, 0) != hipSuccess)
       return QMK_ERR_NO_DEVICE;
-    int per_cu_batch = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_batch, decode_megakernel_batch<Llama1B>, kThreads, 0) != hipSuccess)
+    int per_cu_batch = 0, per_cu_ahead = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_batch, decode_megakernel_batch<Llama1B, 2>, kThreads, 0) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_ahead, decode_megakernel_batch<Llama1B, 4>, kThreads, 0) != hipSuccess)
       return QMK_ERR_NO_DEVICE;
+    per_cu_batch = per_cu_ahead < per_cu_batch ? per_cu_ahead : per_cu_batch;
     int per_cu_batch3 = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_batch3, decode_megakernel_batch<Qwen3_1p7B>, kThreads, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_batch3, decode_megakernel_batch<Qwen3_1p7B, 4>, kThreads, 0) != hipSuccess)
       return QMK_ERR_NO_DEVICE;
     int per_cu_moe = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_moe, decode_megakernel_moe<QwenMoeA2_7B>, kThreads, 0) != hipSuccess)
@@ -901,7 +903,15 @@ static int decode_step_batch(const QmkBatchArgs* a) {
   p.q_norm = static_cast<const u16*>(a->q_norm_weights);
   p.k_norm = static_cast<const u16*>(a->k_norm_weights);
 
-  hipLaunchKernelGGL(decode_megakernel_batch<M>, dim3(a->num_queues), dim3(kThreads), 0, static_cast<hipStream_t>(a->stream), p);
+  // Four tiles of keys a wave ahead, or two in a kernel of their own.  Heads of 64 take four for 5 to 8 rows of at most 2048 positions, most of
+  // which the requests ahead of the attention's wait hold (two -> four, us a step of 8 rows, context 330 / 600 / 900 / 1500 / 2000: 748 / 777 /
+  // 817 / 899 / 967 -> 736 / 750 / 784 / 879 / 957).  Elsewhere the longer loop's code costs them more than it gives, at four slices too
+  // (8 rows, 2030 / 16000: 927 / 1890 -> 938 / 1956; 16 rows, 1000 / 2000 / 16000: 988 / 1118 / 2979 -> 1003 / 1148 / 3120; 12 rows, 16000:
+  // 2016 -> 2132; 4 rows, 16000: 1354 -> 1391), and both loops in one kernel are slower in either (8 rows, 600 / 16000: 758 / 1989).
+  const bool ahead = M::D > 64 || (a->batch_size > 4 && a->batch_size <= 8 && a->max_seq_len <= 2048);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(a->num_queues), dim3(kThreads), 0, static_cast<hipStream_t>(a->stream), p); };
+  if (ahead) launch(decode_megakernel_batch<M, 4>);
+  else if constexpr (M::D <= 64) launch(decode_megakernel_batch<M, 2>);
   return hipGetLastError() == hipSuccess ? QMK_OK : QMK_ERR_LAUNCH;
 }
 

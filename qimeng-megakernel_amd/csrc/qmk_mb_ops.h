@@ -470,7 +470,7 @@ __device__ __forceinline__ void zero_heads(const Params& p, const Ctx& c, int b,
 // merge_in_last (an extension; 0 in streams built by the reference scheduler): the workgroup whose
 // arrival completes the head group's counters merges all partials itself (or zeroes the heads of an
 // inactive row) and counts on the reduction row, so no reduction instruction and no second wait is needed.
-template <class M>
+template <class M, int kDepth>
 __device__ bool op_splitkv(const Params& p, Smem<M>& s, const Ctx& c) {
   constexpr int D = M::D, GQA = M::GQA;
   static_assert(D % 64 == 0 && GQA <= 4 && GQA * D <= kThreads, "a lane owns whole 16-byte vectors of K; one thread per merged output");
@@ -521,13 +521,15 @@ __device__ bool op_splitkv(const Params& p, Smem<M>& s, const Ctx& c) {
     }
   };
   // A wave's next `depth` tiles are in flight at any time, the first of them from before the wait below: a tile costs a trip
-  // to memory and 16 tokens of arithmetic, so with one tile ahead every round paid most of the trip.  Up to three slices a head the
-  // workgroup has nothing else to do in that wait, and four tiles pay (two -> four, Qwen3-1.7B shape, 8 rows, one slice, context 500 /
-  // 700 / 950: 1210 / 1296 / 1409 -> 1153 / 1225 / 1344 us a step; 16 rows, 900: 1631 -> 1533; Llama shape, 8 rows, 900: 820 -> 786;
-  // five spill).  With four slices it comes from a QKV block, a wave has three tiles at most up to 1500 tokens, and the other two's
-  // requests and code cost more than they give (1404 -> 1424 at 1500): two.
-  constexpr int kDepth = 4, kShort = 2;
-  const bool deep = P <= 3;   // uniform
+  // to memory and 16 tokens of arithmetic, so with one tile ahead every round paid most of the trip.  Up to three slices a head
+  // four tiles pay, most where no QKV block stands in front of the slice (two -> four, Qwen3-1.7B shape, 8 rows, one slice, context 500 /
+  // 700 / 950: 1210 / 1296 / 1409 -> 1153 / 1225 / 1344 us a step; 16 rows, 900: 1631 -> 1533; five spill).  Where one does (9 and 10 rows of
+  // three slices, 12 to 16 rows of two, behind 1024 tokens) they gain from 5000 tokens on (10 rows, 8000: 2716 -> 2667; 14 rows, 8000: 3407 ->
+  // 3313) and are within 1.5 % either way before (9 rows, 2000: 1570 -> 1594; 14 rows, 2000: 1791 -> 1776).  With four slices a wave has three
+  // tiles at most up to 1500 tokens, and the other two's requests cost more than they give (1404 -> 1424 at 1500): two.
+  // kDepth 2 is a kernel without the longer loop (see the launch).
+  constexpr int kShort = 2;
+  const bool deep = kDepth > kShort && P <= 3;   // uniform
   const int depth = deep ? kDepth : kShort;
   int tb = t0 + wave * kTok;
   Tile ring[kDepth];

@@ -43,3 +43,26 @@ def test_tiles_ahead(full, slices, monkeypatch):
         mk.check()
         out.append(g.attn_out.cpu())
     bf16_close(out[1], out[0], ulps=1.0, name="attn_out")
+
+
+def test_both_kernels_of_heads_of_64():
+    """Caches of 2048 and 2064 positions take the kernels of four and of two tiles ahead: the same tiles in the same order, the same bits."""
+    shape, rows, out = dataclasses.replace(LLAMA_3_2_1B, num_hidden_layers=1, vocab_size=512), len(POSITIONS), []
+    LlamaConfig.set_shape(shape)
+    weights = synthetic.random_weights(shape, 3, max_positions=2064)
+    gen = torch.Generator().manual_seed(9)
+    hidden = (torch.randn(rows, shape.hidden_size, generator=gen) * 0.7).bfloat16()
+    past = [torch.randn(1, rows, 2048, shape.num_key_value_heads, shape.head_dim, generator=gen).bfloat16() for _ in range(2)]
+    for capacity in (2048, 2064):
+        print(f"capacity {capacity}", flush=True)
+        g = synthetic.build_batch_globals(weights, shape, capacity, rows, "cuda:0")
+        g.hidden_states.copy_(hidden)
+        g.k_cache[:, :, :2048].copy_(past[0])
+        g.v_cache[:, :, :2048].copy_(past[1])
+        g.position_ids.copy_(torch.tensor([*POSITIONS[:-1], 2047], dtype=torch.int32))
+        mk_kernel.build(g, 2048)                      # one slice in either
+        mk = mk_kernel.get_mk(spin_limit=1 << 18)
+        mk_kernel.call_mk(g, mk)
+        mk.check()
+        out.append((g.attn_out.cpu(), g.hidden_states.cpu(), g.logits.cpu()))
+    assert all(torch.equal(a, b) for a, b in zip(*out))

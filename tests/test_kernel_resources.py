@@ -10,6 +10,7 @@ import pytest
 from conftest import ROOT
 
 LIBRARY = ROOT / "qimeng-megakernel_amd" / "libqmk_hybrid.so"
+DECODE = ROOT / "qimeng-megakernel_amd" / "libqmk_hip.so"
 READELF = Path("/opt/rocm/llvm/bin/llvm-readelf")
 
 
@@ -28,19 +29,32 @@ def device_code(data):
                 yield data[found.start() + offset : found.start() + offset + size]
 
 
-def test_no_prefill_kernel_spills(tmp_path):
-    if not LIBRARY.is_file() or not READELF.is_file():
+def notes_of(library, tmp_path):
+    if not library.is_file() or not READELF.is_file():
         pytest.skip("needs the built library and llvm-readelf")
     kernels = {}
-    for i, code in enumerate(device_code(LIBRARY.read_bytes())):
+    for i, code in enumerate(device_code(library.read_bytes())):
         path = tmp_path / f"{i}.co"
         path.write_bytes(code)
         notes = subprocess.run([READELF, "--notes", path], capture_output=True, text=True, check=True).stdout
         for entry in notes.split(".agpr_count:")[1:]:
             field = dict(re.findall(r"\.(\w+):\s+(\S+)", entry))
             kernels[field["symbol"]] = field
+    return kernels
+
+
+def test_no_prefill_kernel_spills(tmp_path):
+    kernels = notes_of(LIBRARY, tmp_path)
     assert any("gemm_direct" in name for name in kernels) and any("window_attention" in name for name in kernels) and any("attention_rows" in name for name in kernels)
     prefill = {name: k for name, k in kernels.items() if "decode_megakernel" not in name}
     spilled = {name: k["vgpr_spill_count"] for name, k in prefill.items() if int(k["vgpr_spill_count"])}
     assert not spilled, spilled
     assert all(int(k["group_segment_fixed_size"]) <= 160 * 1024 for k in prefill.values())
+
+
+def test_tiles_engine_kernels(tmp_path):
+    """Two and four tiles of keys ahead are kernels of their own for heads of 64 (one for both is slower in either), and none keeps registers in memory."""
+    kernels = {name: k for name, k in notes_of(DECODE, tmp_path).items() if "decode_megakernel_batch" in name}
+    found = sorted(re.search(r"batchINS_\d+(\w+?)ELi(\d)EE", name).groups() for name in kernels)
+    assert found == [("Llama1B", "2"), ("Llama1B", "4"), ("Qwen3_1p7B", "4")]
+    assert not any(int(k["vgpr_spill_count"]) for k in kernels.values())
