@@ -163,9 +163,10 @@ class BatchScheduler:
             # later, and an attention worker starts its slice without a block in front (8 rows, context 500, two slices: 1294 ->
             # 1199 us a step; context 130, one slice: 1157 -> 1097).  Above 8 rows also where it does not fit (16 rows, context 900,
             # two slices: 1607 -> 1578), below that not (6 rows, 700, three: 1291 -> 1316): the norm rows' workers then get none,
-            # a few of the others two.
+            # a few of the others two.  Up to four rows, which the rows engine decodes unless a caller asks for this one, neither (four slices, 130 /
+            # 600 / 1100: 2 rows 1197 / 1226 / 1265 -> 1265 / 1266 / 1275, 3 rows 1278 / 1311 / 1341 -> 1350 / 1350 / 1366): few rows' QKV phase is short.
             busy = min(self.workers, len(self.downproj(layer)))
-            beside = (slices <= busy or self.batch_size > 8) and blocks <= 2 * (self.workers - busy)
+            beside = (4 < self.batch_size and slices <= busy or self.batch_size > 8) and blocks <= 2 * (self.workers - busy)
             start = busy if beside else self.batch_size
             plain = [QKVProj_GEMM_RoPE(layer, self.batch_size, 0, lo, hi) for lo, hi in _spans(blocks, self.workers - start)]
         return [NoOp()] * start + plain + [NoOp()] * (self.workers - start - len(plain))

@@ -373,6 +373,6 @@ def test_slices_and_qkv_blocks_of_heads_of_128():
     assert [plan(5, c) for c in (640, 656, 2000)] == [(1, 128), (3, 128), (3, 128)]
     assert [plan(6, c) for c in (1024, 1040)] == [(2, 128), (4, 6)]
     assert [plan(10, c) for c in (1024, 1040)] == [(1, 128), (3, 128)] and [plan(16, c) for c in (1024, 1040)] == [(1, 128), (2, 128)]
-    assert plan(3, 300) == (4, 128)                       # the rows engine's range keeps the rule
+    assert [plan(r, 300) for r in (2, 3, 4)] == [(4, 2), (4, 3), (4, 4)]                       # the rows engine's range keeps the rule, and its QKV blocks behind the norm rows
     llama = [S.mi355x_scheduler(5, LLAMA_3_2_1B).partials_for_capacity(c) for c in (200, 1024, 1040)]
     assert llama == [1, 1, 4]
