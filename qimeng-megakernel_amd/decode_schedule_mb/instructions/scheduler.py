@@ -86,7 +86,8 @@ class BatchScheduler:
     split_kv_per_worker: float = 1.0   # split-KV instructions of a step per worker that the fan-out aims at (the reference: one)
     split_kv_cap: int = MAX_REDUCTION_LIST   # ... and never more slices per KV head than this
     lone_slice_tokens: int = 0         # where the rule gives two or three slices and the slices' tokens are at most this many: one slice
-                                       # (the only slice of its heads writes attn_out itself: no counted arrival, no merge);
+                                       # (the only slice of its heads writes attn_out itself: no counted arrival, no merge); below 8 rows, up to
+                                       # half as many, also where it gives more than the down projection's workers hold;
                                        # heads of 128: one slice up to this many whatever the rule gives (0: the rule alone)
 
     def __post_init__(self) -> None:
@@ -254,7 +255,9 @@ class BatchScheduler:
             if self.shape.head_dim > 64 and self.lone_slice_tokens:
                 if tokens <= self.lone_slice_tokens:
                     return 1
-                if beside > 2 or beside == 2 and tokens <= 1024:
+                # (5 rows, three slices, which keep clear of the QKV blocks, and four, which are shorter: 3000 / 5000 / 6000 / 8000 / 16000
+                # 1488 / 1797 / 1958 / 2237 / 3384 and 1581 / 1840 / 1959 / 2197 / 3124 us a step)
+                if beside > 2 and tokens <= 6000 or beside == 2 and tokens <= 1024:
                     p = min(p, beside)
             # The rule rounds up: 12 rows of 8 KV heads get 3 slices, 288 instructions for 256 workers — a second round of
             # 32 behind the first (Qwen3-1.7B shape, 12 rows: 1.83 ms per step against 1.64 at 16 rows).  Never more
@@ -339,7 +342,7 @@ def mi355x_scheduler(batch_size: int, shape: DecodeShape | None = None, *, merge
     half of it: B=2 938/947 -> 853/856 us, B=4 938/947 -> 881/905, B=8 1021/1048 -> 972/1009, B=16 1187/1233 ->
     1108/1176.  With heads of 128 (Qwen3-1.7B shape, B=8: 1566/1636 us with 4 slices, 1591/1721 with 2) the rule's number stays for long caches.
     With heads of 128, from 5 rows on (fewer take the rows engine), a cache of up to 640 tokens has one slice (above 8 rows: up to
-    1024), and a longer one as many as the down projection's workers hold, where that is three, or two and at most 1024 tokens: the
+    1024), and a longer one as many as the down projection's workers hold, where that is three and at most 6000 tokens, or two and at most 1024: the
     QKV blocks then keep off the slices' workers, and those ask for four tiles a wave ahead (8 rows, contexts 130 / 350 / 500 / 600 / 700 /
     950 with 1 and 2 slices: 1092 / 1113 / 1153 / 1174 / 1225 / 1344, 1185 / 1188 / 1200 / 1200 / 1215 / 1270; with 4: 1256 / 1273 / 1285 /
     - / 1314 / 1350 us; 5 rows, 600 / 800 / 1500 with 1, 3 and 4: 1114 / 1201 / -, 1161 / 1174 / 1242 and - / - / 1348; 10 rows, 800 with 1 and

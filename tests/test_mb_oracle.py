@@ -371,6 +371,7 @@ def test_slices_and_qkv_blocks_of_heads_of_128():
         return p, next(k for k, i in enumerate(r) if i.opcode() == 2)
     assert [plan(8, c) for c in (16, 640, 656, 1024, 1040, 4096)] == [(1, 128), (1, 128), (2, 128), (2, 128), (4, 8), (4, 8)]
     assert [plan(5, c) for c in (640, 656, 2000)] == [(1, 128), (3, 128), (3, 128)]
+    assert [plan(5, c) for c in (6000, 6016, 16384)] == [(3, 128), (4, 5), (4, 5)]      # four shorter slices win from there on
     assert [plan(6, c) for c in (1024, 1040)] == [(2, 128), (4, 6)]
     assert [plan(10, c) for c in (1024, 1040)] == [(1, 128), (3, 128)] and [plan(16, c) for c in (1024, 1040)] == [(1, 128), (2, 128)]
     assert [plan(r, 300) for r in (2, 3, 4)] == [(4, 2), (4, 3), (4, 4)]                       # the rows engine's range keeps the rule, and its QKV blocks behind the norm rows
