@@ -172,7 +172,7 @@ def test_each_mechanism_alone(part, ff, loop):
 @pytest.mark.parametrize("v_dim", [40, 120], ids=["values up to 64", "values up to 128"])
 @pytest.mark.parametrize("delta_dim", [50, 100], ids=["one tile a wave", "two tiles a wave"])
 def test_both_branches_in_one_launch(delta_dim, v_dim, tokens):
-    """Every kind of launch that walks a delta rule's chunks beside an attention (bf16), at both lines of its choice."""
+    """Every kind of launch that walks a delta rule's chunks beside an attention (bf16); the lines between them are the next test's."""
     shape = synthetic.looped_shape("pp", width=64, vocab=70, ff={"p": 40}, heads=16, kv_heads=4, dim=72, v_dim=v_dim, rot_dim=16, delta_heads=3, delta_kv_heads=3,
                                    delta_dim=delta_dim, delta_v_dim=40, taps=3, delta_rank=8, gate_rank=6)
     w = synthetic.random_hybrid_weights(shape, 4)
@@ -187,6 +187,51 @@ def test_both_branches_in_one_launch(delta_dim, v_dim, tokens):
     assert error(logits[:, : shape.vocab].double().cpu(), want) < TOL[torch.bfloat16]
     for k, layer in enumerate(layers):
         assert error(out[k, :, : shape.width].double().cpu(), layer) < TOL[torch.bfloat16]
+
+
+def beside(tokens_kept, *, v_dim=66, delta_dim=66, pattern="pp"):
+    """16 heads of attention (up to 512 tokens 16 queries a workgroup, then 64) beside a small delta rule."""
+    shape = synthetic.looped_shape(pattern, width=64, vocab=70, ff={"p": 40}, heads=16, kv_heads=4, dim=72, v_dim=v_dim, rot_dim=16, delta_heads=3, delta_kv_heads=3,
+                                   delta_dim=delta_dim, delta_v_dim=40, taps=3, delta_rank=8, gate_rank=6)
+    return shape, dict(max_positions=tokens_kept, portion_rows=tokens_kept)
+
+
+@pytest.mark.parametrize("cuts", [[512, 30], [513, 30], [20, 513]], ids=str)
+@pytest.mark.parametrize("delta_dim,v_dim", [(64, 64), (64, 66), (66, 64), (66, 66)])
+def test_one_launch_continues_a_state(delta_dim, v_dim, cuts):
+    """At the lines of the launch's choice, and a second portion of either kind behind a first one: it reads the state that a launch of both branches left."""
+    shape, room = beside(544, v_dim=v_dim, delta_dim=delta_dim)
+    w, ids = synthetic.random_hybrid_weights(shape, 4), tokens_of(shape, sum(cuts))
+    want = O.forward(shape.to_config(), w, torch.tensor(ids), dtype=torch.float64)
+    got = run(on_gpu(shape, w, torch.bfloat16, **room), mk_kernel.get_mk(), ids, cuts)
+    assert error(got, want) < TOL[torch.bfloat16]
+    assert error(got[cuts[0]:], want[cuts[0]:]) < TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("tokens", [40, 513], ids=["16 queries a workgroup", "64 queries a workgroup"])
+@pytest.mark.parametrize("delta_dim", [64, 128])
+@pytest.mark.parametrize("v_dim", [64, 128])
+def test_one_launch_and_two_leave_the_same_bits(v_dim, delta_dim, tokens):
+    """A delta rule's state beside an attention that shares its launch and beside one too wide to, and an attention's output beside a delta rule of either kind
+    (which adds nothing: its norm's weights are zero).  Two portions, so that the second starts from a state."""
+    def outcome(left, right):      # value size of the attention, key size of the delta rule
+        shape, room = beside(2 * tokens, v_dim=left, delta_dim=right, pattern="p")
+        common, attention, delta = (synthetic.random_hybrid_weights(beside(1, v_dim=v, delta_dim=d, pattern="p")[0], 4) for v, d in ((64, 64), (left, 64), (64, right)))
+        w = {name: (attention if ".left." in name else delta if ".right." in name else common)[name] for name in common}
+        w["l0.mix.right.out"] = torch.zeros_like(w["l0.mix.right.out"])
+        g, mk = on_gpu(shape, w, torch.bfloat16, **room), mk_kernel.get_mk()
+        request, out = RequestTable(g).open("y"), torch.zeros(2, shape.run_count, tokens, shape.width_s, device=DEVICE)
+        ids = torch.tensor(tokens_of(shape, 2 * tokens), device=DEVICE)
+        for i in range(2):
+            g.slot, g.position_id, g.flip = request.slot, i * tokens, i
+            mk.prefill(g, ids[i * tokens:(i + 1) * tokens], torch.arange(tokens, dtype=torch.int32, device=DEVICE), layer_out=out[i])
+        mk.check()
+        (state,) = [s["state"][request.slot] for s in g.layer_state if "state" in s]
+        return out, state
+
+    together, wide_attention, large_delta = outcome(v_dim, delta_dim), outcome(136, delta_dim), outcome(v_dim, 136)
+    assert torch.equal(together[1], wide_attention[1]) and float(together[1].abs().max()) > 0
+    assert torch.equal(together[0], large_delta[0]) and float(together[0].abs().max()) > 0
 
 
 def pointed_model(heads=4, kv_heads=2):
