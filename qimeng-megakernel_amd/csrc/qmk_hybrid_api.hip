@@ -633,6 +633,14 @@ inline void launch_scan(const ChunkArgs& g, hipStream_t st) {
   }
 }
 
+// Whether a delta rule's chunks are walked in the launch of the attention beside it: where a CU holds a workgroup of either.  Elsewhere (fp32, larger heads) the branches follow one
+// another, each with its output gate ahead of its chunks: the order that one launch needs only costs there (us a call of the 1b shape in fp32, 64 tokens behind 500 1907 and so 1894, 200 behind 500
+// 2870 and 2846; two layers with heads of 256, 530 tokens 607 and 602).
+template <class T>
+bool one_launch(const QmkHybridLayer& attention, const QmkHybridLayer& delta) {
+  return sizeof(T) == 2 && attention.q_stride <= 128 && attention.v_dim <= 128 && chunk_tiles(delta.head_dim) <= 8;
+}
+
 // rows: where the rotated part of a latent attention's keys is, behind the latent.  In fp32 two groups of waves share a workgroup's queries, except for
 // the largest heads, where they take 140 KB of LDS and more registers than there are (us a portion of one layer, 16 heads of 256 | 256, one group -> two:
 // 4000 tokens 2963 -> 3416, 1025 tokens 453 -> 508).  In bf16 the largest heads leave no registers for a second wave a SIMD, and take stages of 32 keys.
@@ -644,15 +652,14 @@ inline void launch_scan(const ChunkArgs& g, hipStream_t st) {
 // In fp32 the same heads take few_attention with one a CU (us, 16 heads, window_attention -> few_attention: 192 | 128, 43 tokens 16.1 -> 12.2, 200 tokens 30.0 -> 20.7, 400 tokens 50.2 -> 55.8;
 // behind 1000 keys 250 tokens 133 -> 83, behind 16000 1641 -> 1027; 128 | 128 behind 200 keys, 43 tokens 29.2 -> 19.0, 400 tokens 58.6 -> 63.2, behind 1000 keys 250 tokens 113 -> 72, behind
 // 16000 1294 -> 796).
-// `beside`: a delta rule whose chunks are prepared; they are walked in the same launch where a CU holds a workgroup of either, ahead of it where not (us, 2048 tokens of 16 heads, behind
-// nothing and behind 2048 keys, two launches -> one: XX).
+// `beside`: a delta rule that shares the launch, its chunks prepared.
 template <class T>
 void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* q, Keys<T> keys, const T* rows, const T* vt, const T* gate, int first, int cap, Operand<T> out,
                       const ChunkArgs* beside, hipStream_t st) {
   if constexpr (sizeof(T) == 2) {
     const AttentionArgs args{q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out.at};
     auto workgroups = [&](int queries) { return static_cast<unsigned>((a->tokens + queries - 1) / queries * l.heads); };
-    if (beside != nullptr && l.q_stride <= 128 && l.v_dim <= 128 && chunk_tiles(beside->dim) <= 8) {
+    if (beside != nullptr) {
       auto both = [&](auto one_tile, auto two_tiles, int queries) {
         const dim3 grid(beside->heads * (beside->n / 16) + workgroups(queries));
         if (chunk_tiles(beside->dim) == 4) hipLaunchKernelGGL(one_tile, grid, dim3(kPfThreads), 0, st, *beside, args);
@@ -663,7 +670,6 @@ void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* 
       else both(scan_and_attend<1, 4, 8, 64, 2, false>, scan_and_attend<2, 4, 8, 64, 2, false>, 64);
       return;
     }
-    if (beside != nullptr) launch_scan(*beside, st);
     auto launch = [&](auto kernel, int queries) { hipLaunchKernelGGL(kernel, dim3(workgroups(queries)), dim3(kPfThreads), 0, st, args); };
     auto rows_of = [&](auto shared, auto all, int a_cu) { workgroups(16) <= 256u * a_cu ? launch(shared, 16) : launch(all, 64); };
     if (l.q_stride <= 128 && l.v_dim <= 64) launch(attention_rows<4, 4, 64, 2, 2>, 64);
@@ -671,7 +677,6 @@ void launch_attention(const QmkHybridArgs* a, const QmkHybridLayer& l, const T* 
     else if (l.q_stride <= 192 && l.v_dim <= 128) rows_of(attention_rows<6, 8, 64, 2, 1, true>, attention_rows<6, 8, 64, 2, 2>, 1);
     else launch(attention_rows<8, 16, 32, 3, 1>, 64);
   } else {
-    if (beside != nullptr) launch_scan(*beside, st);
     const int few_runs = (a->tokens + 15) / 16;
     auto launch_few = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(few_runs, l.heads), dim3(kPfThreads), 0, st, q, keys, rows, vt, gate, l, first, a->position, a->tokens, cap, out);
@@ -824,13 +829,19 @@ int prefill_plain(const QmkHybridArgs* a) {
     e.lda = ld; e.f0 = b.decay; e.ldo = keys;
     launch_gemm<T, u16, T>(e, b.split, st);
   };
-  // A delta rule up to its scan.  Writes nothing that an attention beside it reads: its output gate, which lies where the attention's does, comes behind.
-  auto prepare_delta = [&](const QmkHybridLayer& l) {
+  auto delta_gate = [&](const QmkHybridLayer& l) {
+    GemmArgs f = gemm_args(whole(b.low + l.rank), l.gate_w, l.mix_width, l.gate_rank, l, EPI_SIGMOID);
+    f.lda = l.rank + l.gate_rank; f.out = b.gate; f.ldo = l.mix_width;
+    launch_gemm<T, u16, T>(f, b.split, st);
+  };
+  // A delta rule up to its scan.  `gate`: with its output gate, which lies where that of an attention does; in one launch with that it comes behind.
+  auto prepare_delta = [&](const QmkHybridLayer& l, bool gate) {
     const int beta_ld = (l.heads + 15) / 16 * 16;
     GemmArgs g = gemm_args(b.h.of(D), l.in_w, l.in_rows, D, l, EPI_DELTA_IN);
     g.f1 = b.qkv; g.out2 = b.low; g.f0 = b.beta; g.ldo = beta_ld;
     launch_gemm<T, u16, T>(g, b.split, st);
     decays(l, l.rank + l.gate_rank, EPI_DELTA_DECAY);
+    if (gate) delta_gate(l);
     ChunkArgs c = chunk_args(l);
     c.q = b.qkv; c.beta = b.beta; c.beta_ld = beta_ld; c.values = b.values;
     run_chunks<T, CHUNK_DELTA>(c, st);
@@ -840,10 +851,7 @@ int prefill_plain(const QmkHybridArgs* a) {
     hipLaunchKernelGGL(state_out<T>, dim3((M * l.heads + 3) / 4), block, 0, st, b.o, b.gate, l, M, a->eps, b.mix.of(l.mix_width));
   };
   auto finish_delta = [&](const QmkHybridLayer& l) {
-    const int channels = conv_channels(l), W = l.mix_width;
-    GemmArgs f = gemm_args(whole(b.low + l.rank), l.gate_w, W, l.gate_rank, l, EPI_SIGMOID);
-    f.lda = l.rank + l.gate_rank; f.out = b.gate; f.ldo = W;
-    launch_gemm<T, u16, T>(f, b.split, st);
+    const int channels = conv_channels(l);
     if (l.taps > 1)
       hipLaunchKernelGGL(keep_inputs, dim3((channels + kPfThreads - 1) / kPfThreads), block, 0, st, b.qkv, l, channels, a->slot, a->flip, M);
     state_rows(l);
@@ -880,6 +888,7 @@ int prefill_plain(const QmkHybridArgs* a) {
   auto dump_of = [&](const QmkHybridLayer& l) {   // where the run before this entry is asked for
     return a->layer_out != nullptr && l.prev >= 0 ? a->layer_out + static_cast<size_t>(runs_done++) * M * D : nullptr;
   };
+  bool walked = false;      // the next entry's chunks, beside the attention of this one
   for (int i = 0; i < a->num_layers; ++i) {
     const QmkHybridLayer& l = a->layers[i];
     if (l.type == QMK_ENTRY_FINAL) {
@@ -902,12 +911,13 @@ int prefill_plain(const QmkHybridArgs* a) {
     }
     if (l.type == QMK_MIXER_ATTENTION) {
       project_attention(l);
-      // Beside a delta rule: its chunks are prepared first, since its scan leaves room on the chip for the attention.
-      const bool beside = l.branch + 1 < l.branches && a->layers[i + 1].type == QMK_MIXER_DELTA;
-      const ChunkArgs c = beside ? prepare_delta(a->layers[i + 1]) : ChunkArgs{};
-      attend(l, beside ? &c : nullptr);
+      walked = l.branch + 1 < l.branches && a->layers[i + 1].type == QMK_MIXER_DELTA && one_launch<T>(l, a->layers[i + 1]);
+      const ChunkArgs c = walked ? prepare_delta(a->layers[i + 1], false) : ChunkArgs{};
+      attend(l, walked ? &c : nullptr);
     } else if (l.type == QMK_MIXER_DELTA) {
-      if (l.branch == 0 || a->layers[i - 1].type != QMK_MIXER_ATTENTION) launch_scan(prepare_delta(l), st);
+      if (walked) delta_gate(l);
+      else launch_scan(prepare_delta(l, true), st);
+      walked = false;
       finish_delta(l);
     } else {
       run_gla(l);
