@@ -56,8 +56,9 @@ struct ChunkArgs {
 // multiple of h on and those behind s up to it, each of them at most one, all pairs of that bit are one matrix product over the channels; the products of decays
 // over blocks of h tokens become those of 2h by one exchange between lanes of a row.  So four levels of products replace sixteen running keys a pair of threads
 // (us, 2048 tokens: 8 heads of 128 of gated linear attention 29 -> 13, 16 of 128 | 128 of the delta rule 71 -> 54).  What is left is memory: it writes 27 KB a chunk and head of 128 channels.
+// Three workgroups a CU for the delta rule's largest heads: left alone the compiler takes 180 registers there, which hold two (us, 1531 tokens of 8 heads of 256 | 256: 54 -> 42).
 template <int KIND, int TILES>      // of a wave
-__global__ __launch_bounds__(kPfThreads) void chunk_prepare(const ChunkArgs g) {
+__global__ __launch_bounds__(kPfThreads, KIND == CHUNK_DELTA && TILES == 4 ? 3 : 1) void chunk_prepare(const ChunkArgs g) {
   constexpr int C = kChunkTokens, kSums = KIND == CHUNK_DELTA ? 2 : 1;
   __shared__ f32x4 sums[kSums][kChunkWaves][64];
   __shared__ double diagonal[kChunkWaves][C];

@@ -58,3 +58,9 @@ def test_tiles_engine_kernels(tmp_path):
     found = sorted(re.search(r"batchINS_\d+(\w+?)ELi(\d)EE", name).groups() for name in kernels)
     assert found == [("Llama1B", "2"), ("Llama1B", "4"), ("Qwen3_1p7B", "4")]
     assert not any(int(k["vgpr_spill_count"]) for k in kernels.values())
+
+
+def test_largest_heads_of_a_delta_rule(tmp_path):
+    """Of the preparation of its chunks three workgroups of four waves share a CU: 512 registers a SIMD."""
+    (kernel,) = [k for name, k in notes_of(LIBRARY, tmp_path).items() if "chunk_prepareILi1ELi4E" in name]
+    assert int(kernel["vgpr_count"]) <= 168 and 3 * int(kernel["group_segment_fixed_size"]) <= 160 * 1024
