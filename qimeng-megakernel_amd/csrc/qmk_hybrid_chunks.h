@@ -524,9 +524,9 @@ __global__ __launch_bounds__(kPfThreads) void segment_starts(const ChunkArgs g) 
 // What bounds it is the chain of a chunk: products of the state with W (four instructions of 32 cycles a tile), the waves' sums through LDS, the state's update.
 // What only the output needs fills the wait for the sums, is the same for every wave (of B u each takes the columns of one of the four instructions, of the sums the
 // tokens of one), and is added up behind the next chunk's barrier; W and T v come from chunk_prepare.  us, 2048 tokens of 16 heads of 128 | 128, beside an
-// attention behind nothing and behind 2048 keys, T (v - (Gk)^T S) on the chain and a chunk's outputs by one wave -> so: 132 -> 103, 147 -> 137 (the attention's own time there).  Error against
-// 64 bits in fp32, beside that: 1b shape, 150 tokens (40 models) states x 0.998 +- 0.001, logits x 1.008 +- 0.008, 331 tokens (30) x 0.998 +- 0.001, x 1.006 +- 0.009.  With B u's part in a sum
-// of its own the launch takes 136 where it takes 120.
+// attention behind nothing and behind 2048 keys, T (v - (Gk)^T S) on the chain and a chunk's outputs by one wave -> so: 140 -> 116, 158 -> 158 (the attention's own time there), for which
+// chunk_prepare takes 58 where it took 55.  Error against 64 bits in fp32, beside that: 1b shape, 150 tokens (56 models) states x 0.999 +- 0.001, logits x 1.012 +- 0.007, 331 tokens (30) x 0.998 +- 0.001,
+// x 1.006 +- 0.009; one token over and over (12), where v is nearly what the state returns, x 1.10 +- 0.06, x 1.07 +- 0.10.  With B u's part in a sum of its own the launch takes 136 where it takes 120.
 template <int WAVES>
 constexpr int kScanLds = 4 * WAVES * 64;
 // kAhead: chunks in flight, what the registers hold.
@@ -583,7 +583,7 @@ __device__ __forceinline__ void scan_chunks(const ChunkArgs& g, int head, int v0
   };
   // Ahead of a branch's end: this compiler (clang 22 of ROCm 7.2.0) has left out the wait between a product and the move of its result where paths meet.  The rule, for any
   // kernel: an accumulator that lives across the end of a branch with a product in it is settled there if its built code has such a move (tests/test_matrix_waits.py walks every
-  // path of every kernel for it); none but this place has.
+  // path of every kernel for it).  As built now none has, here neither: it stays for the next change of these loops.
   auto settle = [](f32x4& v) { asm volatile("s_nop 15" : "+v"(v)); };
   auto outputs = [&](int chunk) {      // of chunk 0 on: everybody's sums of its outputs are in LDS
     const auto to = buffer(g.out + static_cast<size_t>(chunk) * kChunkTokens * out_ld + head * n + v0, ((min(g.M - chunk * kChunkTokens, kChunkTokens) - 1) * out_ld + 16) * 4);
@@ -650,7 +650,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void chunk_scan(const ChunkArgs g) {
 }
 
 // The two branches of a run need nothing of each other, and the delta rule's chunks are a chain of instructions on a part of the chip: its workgroups come first, and go first on their SIMDs, an
-// attention's fill what is left (us, 2048 tokens of 16 heads of 128 | 128 in either, behind nothing and behind 2048 keys, two launches -> one: 118 + 47 -> 132, 119 + 93 -> 147).
+// attention's fill what is left (us, 2048 tokens of 16 heads of 128 | 128 in either, behind nothing and behind 2048 keys, two launches -> one: 122 + 51 -> 116, 122 + 99 -> 158;
+// 530 tokens 34 + 18 -> 31, 200 tokens 15 + 8 -> 14).
 template <int TILES, int QT, int VT, int KEYS, int STAGES, bool SHARED>
 __global__ __launch_bounds__(kPfThreads, 2) void scan_and_attend(const ChunkArgs c, const AttentionArgs a) {
   constexpr int kUnits = kAttentionLds<QT, VT, KEYS, STAGES, SHARED>;

@@ -110,8 +110,8 @@ class BatchMegaKernel:
     ``xcd_counters``: the blocks of the O-projection, the up/gate and the down projection are counted on eight
     sub-counters (words 0, 32, .. 224 of their counter row, one 128-byte line per XCD) instead of all on word 0, where
     hundreds of arrivals from eight XCDs queue on one line.  Taken when the kernel clears the counters itself and
-    a row has the 256 words (Llama shape: 6 rows and more, Qwen3-1.7B shape: 8 and more); a launch that keeps the counters
-    leaves the reference's words.
+    a row has the 256 words (``synthetic.build_batch_globals`` makes them from 5 rows on; a row of the reference's size has them
+    from 6 rows on with the Llama shape, from 8 with the Qwen3-1.7B shape); a launch that keeps the counters leaves the reference's words.
     """
 
     XCD_COUNTER_WORDS = 32 * 8

@@ -1,6 +1,6 @@
 """Every result of a matrix instruction in the built libraries is waited for before anything but the next product's sum touches it.  The hardware does
-not hold such an instruction back; the compiler counts instructions and inserts the rest as `s_nop`, and has left that out where paths meet: without `settle` in
-`chunk_scan` (csrc/qmk_hybrid_chunks.h) a product's result was moved two instructions behind it, at one number of tiles a wave.  So this walks all paths of every kernel
+not hold such an instruction back; the compiler counts instructions and inserts the rest as `s_nop`, and has left that out where paths meet: in an earlier form of
+the delta rule's scan (csrc/qmk_hybrid_chunks.h) a product's result was moved two instructions behind it, at one number of tiles a wave, unless `settle` held it.  So this walks all paths of every kernel
 with a matrix instruction, as built."""
 import re
 import subprocess
